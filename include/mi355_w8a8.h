@@ -91,9 +91,7 @@ typedef enum mi355_w8a8_status {
  * places that depend on (k, n, n_adapters, rank) only, so the earlier call may have had another m, other
  * adapter_indices or another tile geometry.  The caller vouches for it; calls that run as 32-row chunks
  * keep no such copies and ignore the flag. */
-/* For calls of at most 16 rows (rank <= 32) the flag covers something else: the per-row regrouped copy of B
- * the decode kernels keep in the workspace.  There it vouches that the earlier call was a decode call with
- * the same m and that lora_b and adapter_indices have the contents they had then. */
+/* Calls of at most 32 rows (the skinny-M kernels) read A and B as they are, keep nothing and ignore it too. */
 /* mi355_w8a8_grouped_v1 takes the flag too: its launch that lays out the slots then leaves the transposed A
  * and the packed B of an earlier grouped call on the same workspace with the same (k, n, n_groups, rank) as
  * they are. */
@@ -556,7 +554,7 @@ int mi355_w8a8_gq_linear_v1(const mi355_w8a8_gq_problem* problem, void* stream);
  * (no counterpart in the reference; for benchmarks and logs).  Returns an MI355_W8A8_PATH_* value or
  * a negative status.
  */
-#define MI355_W8A8_PATH_SKINNY 1         /* m <= 32: row quantizer + weight-streaming kernel */
+#define MI355_W8A8_PATH_SKINNY 1         /* m <= 32 (SwiGLU included): row quantizer + weight-streaming kernel */
 #define MI355_W8A8_PATH_SKINNY_CHUNKS 2  /* 33..128 rows: the same two kernels per chunk of 32 rows */
 #define MI355_W8A8_PATH_TILED_256X128 3  /* prologue + 256 x 128 tiles, two workgroups per CU */
 #define MI355_W8A8_PATH_TILED_256X256 4  /* prologue + 256 x 256 tiles, one workgroup per CU */

@@ -54,7 +54,7 @@ constexpr uint32_t kMaxN = 1u << 20;
 inline uint64_t align256(uint64_t v) { return (v + 255u) & ~uint64_t(255); }
 
 struct WsLayout {
-  uint64_t xq, sx, xn, zp, at, bp, src_row, dst_pos, slot_group, blk_range, tile_ctr, skinny, total;
+  uint64_t xq, sx, zp, at, bp, src_row, dst_pos, slot_group, blk_range, tile_ctr, skinny, total;
   uint32_t slots, nkk, K_pad, KB, n_steps, steps_per_wave;
   uint32_t rows_bound;  // the slots that can hold rows (a multiple of 32)
 };
@@ -121,11 +121,8 @@ WsLayout make_layout(uint32_t m, uint32_t k, uint32_t n, uint32_t n_groups, uint
   w.slot_group = off; off += align256((uint64_t)w.slots * 4u);
   w.blk_range = off; off += align256((uint64_t)(w.slots / 32u) * 4u);
   w.tile_ctr = off; off += 1024u;  // two sets of eight counters, 64 bytes apart
-  // normalized rows: only the decode path keeps them in memory (RMSNorm + LoRA, M <= 32)
-  w.xn = off;
-  off += (rank && m <= kSkinnyChunkedMaxRows) ? align256((uint64_t)(m < 32u ? m : 32u) * k * 2u) : 0u;
   w.zp = off; off += rank ? align256((uint64_t)(w.slots / 32u) * w.nkk * 3u * kBlockBytes) : 0u;
-  w.skinny = off; off += align256(skinny_workspace_bytes(m, n, rank));
+  w.skinny = off; off += align256(skinny_workspace_bytes());
   w.total = off;
   return w;
 }
@@ -231,12 +228,52 @@ int validate_common(uint32_t m, uint32_t k, uint32_t n) {
   return MI355_W8A8_OK;
 }
 
-// Skinny-M path: quantize -> stream (weight + LoRA-A units) -> epilogue.
-int launch_skinny(const mi355_w8a8_problem* p, unsigned char* xq, float* sx, uint16_t* xn, unsigned char* sws,
-                  uint32_t K_pad, uint32_t KB, hipStream_t s, bool allow_regroup = true) {
+template <int NS, int RB, int KP>
+int launch_skinny_stream_one(const SkinnyStreamArgs& a, uint32_t lds_bytes, hipStream_t s) {
+  if (hipFuncSetAttribute(reinterpret_cast<const void*>(&skinny_stream_kernel<NS, RB, KP>),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes) != hipSuccess)
+    return MI355_W8A8_ERR_LAUNCH;
+  // 8 / NS units per 128-column group; groups are dealt to the eight XCD residues of the block index
+  const dim3 grid(((a.n_groups + 7u) / 8u) * (64u / NS)), block(kSkinnyStreamThreads);
+  hipLaunchKernelGGL((skinny_stream_kernel<NS, RB, KP>), grid, block, lds_bytes, s, a);
+  return launch_status();
+}
+
+// The stream kernel's instantiation: KP covers a wave's share of K in one round where registers allow it
+// (KP * (NS + RB) operands of four registers), so that all of it is in flight at once.  Slices of 16 columns
+// while 32-column units would leave CUs idle (fewer than 512 units: two workgroups share a CU); SwiGLU and
+// residual decide for themselves (a gate/up pair is two slices; the residual's dword gather serves one column).
+int launch_skinny_stream(SkinnyStreamArgs& a, hipStream_t s) {
+  const bool pairs = a.swiglu || (!a.residual && (a.N & 1u) == 0 && a.n_groups * 4u >= 512u);
+  const uint32_t rb = a.M > 16u ? 2u : 1u, ns = pairs ? 2u : 1u, ppw = a.pairs_per_wave;
+  const SkinnyStreamLds L = skinny_stream_lds(a.M, a.lora_b ? a.r : 0u, a.z_chunks, ns, rb);
+  a.z_off = L.z_off; a.tail_off = L.tail_off;
+  if (ns == 1u && rb == 1u) {
+    if (ppw <= 4u) return launch_skinny_stream_one<1, 1, 4>(a, L.bytes, s);
+    if (ppw <= 8u) return launch_skinny_stream_one<1, 1, 8>(a, L.bytes, s);
+    if (ppw <= 12u) return launch_skinny_stream_one<1, 1, 12>(a, L.bytes, s);
+    return launch_skinny_stream_one<1, 1, 24>(a, L.bytes, s);
+  }
+  if (ns == 1u) {
+    if (ppw <= 4u) return launch_skinny_stream_one<1, 2, 4>(a, L.bytes, s);
+    if (ppw <= 8u) return launch_skinny_stream_one<1, 2, 8>(a, L.bytes, s);
+    return launch_skinny_stream_one<1, 2, 12>(a, L.bytes, s);
+  }
+  if (rb == 1u) {
+    if (ppw <= 4u) return launch_skinny_stream_one<2, 1, 4>(a, L.bytes, s);
+    if (ppw <= 8u) return launch_skinny_stream_one<2, 1, 8>(a, L.bytes, s);
+    return launch_skinny_stream_one<2, 1, 12>(a, L.bytes, s);
+  }
+  if (ppw <= 4u) return launch_skinny_stream_one<2, 2, 4>(a, L.bytes, s);
+  return launch_skinny_stream_one<2, 2, 8>(a, L.bytes, s);
+}
+
+// Skinny-M path: quantize (+ LoRA-A units) -> stream the weight and finish.
+int launch_skinny(const mi355_w8a8_problem* p, unsigned char* xq, float* sx, unsigned char* sws, uint32_t K_pad,
+                  uint32_t KB, hipStream_t s) {
   const bool rms = p->rms_gamma != nullptr;
   const bool lora = p->n_adapters > 0;
-  const SkinnyLayout L = skinny_layout(p->m, p->k, p->n, p->rank);
+  const SkinnyLayout L = skinny_layout(p->k);
   int st;
   if (!(p->flags & MI355_W8A8_FLAG_SKIP_PROLOGUE)) {
     SkinnyQuantArgs q{};
@@ -246,35 +283,18 @@ int launch_skinny(const mi355_w8a8_problem* p, unsigned char* xq, float* sx, uin
     q.M = p->m; q.K = p->k; q.K_pad = K_pad; q.KB = KB;
     q.xq = xq; q.sx = sx;
     q.codes_rm = p->aux_x_codes; q.scales_rm = p->aux_x_scales;
-    q.xn = (rms && lora) ? xn : nullptr;
     q.xn_aux = static_cast<uint16_t*>(p->aux_normalized);
-    // without RMSNorm the LoRA-A units depend on x only and ride along with the quantizer
     q.lora_a = static_cast<const uint16_t*>(p->lora_a);
     q.idx = p->adapter_indices;
     q.z_part = reinterpret_cast<float*>(sws + L.z_part);
     q.n_adapters = p->n_adapters; q.r = p->rank; q.z_chunks = L.z_chunks; q.z_chunk_k = L.z_chunk_k;
-    q.n_z_units = (lora && !rms) ? p->m * L.z_chunks : 0u;
-    const bool regroup = allow_regroup && lora && p->rank <= 32u && p->m <= 16u && (p->n % 8u) == 0;
-    // the caller may vouch that the regrouped B of an earlier call (same B, same adapter per row) is still
-    // in the workspace; a call in 32-row chunks shares one workspace between its chunks and never keeps it
-    const bool keep_regrouped = regroup && (p->flags & MI355_W8A8_FLAG_LORA_PACK_VALID);
-    q.lora_b = (regroup && !keep_regrouped) ? static_cast<const uint16_t*>(p->lora_b) : nullptr;
-    q.bsel = reinterpret_cast<uint16_t*>(sws + L.bsel);
-    q.N = p->n; q.n_groups = n_padded(p->n) / 128u;
+    q.n_z_units = lora ? p->m * L.z_chunks : 0u;
     q.lora_scaling = lora ? p->lora_scaling : nullptr;
     q.row_scaling = reinterpret_cast<float*>(sws + L.row_scaling);
-    const uint32_t n_regroup = (regroup && !keep_regrouped) ? (p->m * q.n_groups + 3u) / 4u : 0u;
-    if (rms) hipLaunchKernelGGL((skinny_quant_kernel<true>), dim3(p->m + n_regroup), dim3(1024), 0, s, q);
-    else hipLaunchKernelGGL((skinny_quant_kernel<false>), dim3(p->m + q.n_z_units + n_regroup), dim3(1024), 0, s, q);
+    const dim3 grid(p->m + q.n_z_units), block(1024);
+    if (rms) hipLaunchKernelGGL((skinny_quant_kernel<true>), grid, block, 0, s, q);
+    else hipLaunchKernelGGL((skinny_quant_kernel<false>), grid, block, 0, s, q);
     if ((st = launch_status())) return st;
-    if (lora && rms) {  // the LoRA-A units read the normalized rows the quantizer has just written
-      SkinnyLoraAArgs la{};
-      la.xsrc = xn; la.lora_a = static_cast<const uint16_t*>(p->lora_a); la.idx = p->adapter_indices;
-      la.z_part = q.z_part; la.K = p->k; la.n_adapters = p->n_adapters; la.r = p->rank;
-      la.z_chunks = L.z_chunks; la.z_chunk_k = L.z_chunk_k;
-      hipLaunchKernelGGL(skinny_lora_a_kernel, dim3(p->m * L.z_chunks), dim3(1024), 0, s, la);
-      if ((st = launch_status())) return st;
-    }
   }
   if (p->flags & MI355_W8A8_FLAG_SKIP_GEMM) return MI355_W8A8_OK;
   SkinnyStreamArgs a{};
@@ -283,22 +303,17 @@ int launch_skinny(const mi355_w8a8_problem* p, unsigned char* xq, float* sx, uin
   a.z_part = reinterpret_cast<const float*>(sws + L.z_part);
   a.sx = sx; a.sw = p->w_scales;
   a.lora_b = lora ? static_cast<const uint16_t*>(p->lora_b) : nullptr;
-  a.bsel = (allow_regroup && lora && p->rank <= 32u && p->m <= 16u && (p->n % 8u) == 0)
-               ? reinterpret_cast<const uint16_t*>(sws + L.bsel) : nullptr;
-  a.lora_scaling = p->lora_scaling; a.idx = p->adapter_indices;
+  a.idx = p->adapter_indices;
   a.row_scaling = reinterpret_cast<const float*>(sws + L.row_scaling);
   a.residual = static_cast<const uint16_t*>(p->residual);
   a.out = static_cast<uint16_t*>(p->out);
   a.aux_acc = p->aux_acc;
-  a.M = p->m; a.N = p->n; a.N_pad = n_padded(p->n); a.K = p->k; a.KB = KB;
+  a.M = p->m; a.N = p->n; a.K = p->k; a.KB = KB;
   a.pairs_per_wave = L.pairs_per_wave;
-  a.n_adapters = p->n_adapters; a.r = p->rank; a.z_chunks = L.z_chunks;
-  a.n_groups = a.N_pad / 128u;
-  // eight units per 128-column group; groups are dealt to the eight XCD residues of the block index
-  const dim3 grid(((a.n_groups + 7u) / 8u) * 64u), block(kSkinnyStreamThreads);
-  if (p->m > 16u) hipLaunchKernelGGL((skinny_stream_kernel<true>), grid, block, 0, s, a);
-  else hipLaunchKernelGGL((skinny_stream_kernel<false>), grid, block, 0, s, a);
-  return launch_status();
+  a.n_adapters = p->n_adapters; a.r = lora ? p->rank : 0u; a.z_chunks = L.z_chunks;
+  a.n_groups = n_padded(p->n) / 128u;
+  a.swiglu = (p->flags & MI355_W8A8_FLAG_SWIGLU) ? 1u : 0u;
+  return launch_skinny_stream(a, s);
 }
 
 enum Required { kReqNone = 0, kReqLinear = 1, kReqGateUp = 2, kReqResidual = 3 };
@@ -307,9 +322,9 @@ enum Required { kReqNone = 0, kReqLinear = 1, kReqGateUp = 2, kReqResidual = 3 }
 // status for a contradictory request.  The choice depends on the dimensions and the flags only.
 int choose_forward_path(uint32_t m, uint32_t k, uint32_t n, uint32_t flags) {
   const bool swiglu = (flags & MI355_W8A8_FLAG_SWIGLU) != 0;
-  bool skinny = m <= (uint32_t)kSkinnyMaxRows && !(flags & MI355_W8A8_FLAG_FORCE_TILED) && !swiglu;
+  bool skinny = m <= (uint32_t)kSkinnyMaxRows && !(flags & MI355_W8A8_FLAG_FORCE_TILED);
   if (flags & MI355_W8A8_FLAG_FORCE_SKINNY) {
-    if (m > (uint32_t)kSkinnyMaxRows || swiglu) return MI355_W8A8_ERR_UNSUPPORTED;
+    if (m > (uint32_t)kSkinnyMaxRows) return MI355_W8A8_ERR_UNSUPPORTED;
     skinny = true;
   }
   if (!skinny_supported()) skinny = false;
@@ -402,8 +417,7 @@ int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
 
   const bool skinny = path == MI355_W8A8_PATH_SKINNY;
   if (skinny) {
-    return launch_skinny(p, ws + w.xq, reinterpret_cast<float*>(ws + w.sx),
-                         reinterpret_cast<uint16_t*>(ws + w.xn), ws + w.skinny, w.K_pad, w.KB, s);
+    return launch_skinny(p, ws + w.xq, reinterpret_cast<float*>(ws + w.sx), ws + w.skinny, w.K_pad, w.KB, s);
   }
   if (path == MI355_W8A8_PATH_SKINNY_CHUNKS) {
     // The chunks overwrite each other's prologue results, so there is no GEMM-only or prologue-only
@@ -423,8 +437,7 @@ int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
       if (p->aux_normalized)
         sub.aux_normalized = static_cast<unsigned char*>(p->aux_normalized) + (size_t)row0 * p->k * 2u;
       // the chunks share the workspace: they run one after the other on the stream
-      if ((st = launch_skinny(&sub, ws + w.xq, reinterpret_cast<float*>(ws + w.sx),
-                              reinterpret_cast<uint16_t*>(ws + w.xn), ws + w.skinny, w.K_pad, w.KB, s, false)))
+      if ((st = launch_skinny(&sub, ws + w.xq, reinterpret_cast<float*>(ws + w.sx), ws + w.skinny, w.K_pad, w.KB, s)))
         return st;
     }
     return MI355_W8A8_OK;

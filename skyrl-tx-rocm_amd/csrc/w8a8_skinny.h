@@ -2,18 +2,19 @@
 //   1. skinny_quant_kernel   one workgroup per row: (RMSNorm,) absmax, scale, int8 codes in
 //                            MFMA operand order.
 //                            LoRA-A units ride along: z_part[chunk][m][:] = x[m, chunk] @
-//                            A[idx[m]][chunk, :] in float32 (a launch of their own when they
-//                            need the normalized rows).
-//   2. skinny_stream_kernel  every workgroup owns 16 weight columns for all of K: its eight waves
+//                            A[idx[m]][chunk, :] in float32 (with RMSNorm every unit forms the row's
+//                            inverse RMS for itself: a few KiB from the L2 against a launch of its own).
+//   2. skinny_stream_kernel  every workgroup owns 16 or 32 weight columns for all of K: its eight waves
 //                            stream the weight once from HBM straight into MFMA operands (no LDS:
 //                            every byte is used once), are reduced through LDS, and the workgroup
 //                            finishes its columns: (float(acc) * sx) * sw + s * (z @ B[idx[m]])
-//                            + residual, one bf16 cast.
+//                            + residual, one bf16 cast, or the SwiGLU of the (gate, up) column pairs.
 // Integer sums are exact and the float32 sums have a fixed order: results are bit-identical
 // from run to run.  No atomics, no data crosses workgroups inside a launch.
 #pragma once
 #include "../../include/mi355_w8a8.h"
 #include "w8a8_device.h"
+#include "w8a8_gemm.h"
 
 namespace w8a8 {
 
@@ -22,11 +23,11 @@ constexpr uint32_t kSkinnyMaxZChunks = 16;
 constexpr uint32_t kSkinnyZChunkK = 1024;  // K elements per LoRA-A work unit (per row)
 
 struct SkinnyLayout {
-  uint64_t z_part, row_scaling, bsel, total;
+  uint64_t z_part, row_scaling, total;
   uint32_t pairs_per_wave, z_chunks, z_chunk_k;
 };
 
-inline SkinnyLayout skinny_layout(uint32_t m, uint32_t k, uint32_t n, uint32_t rank) {
+inline SkinnyLayout skinny_layout(uint32_t k) {
   SkinnyLayout L{};
   const uint32_t n_pairs = k_padded(k) / 64u;
   L.pairs_per_wave = (n_pairs + 7u) / 8u;
@@ -37,17 +38,11 @@ inline SkinnyLayout skinny_layout(uint32_t m, uint32_t k, uint32_t n, uint32_t r
   L.z_chunk_k = zk;
   L.z_part = 0;
   L.row_scaling = (uint64_t)kSkinnyMaxZChunks * kSkinnyMaxRows * kMaxRank * 4u;
-  L.bsel = L.row_scaling + 256u;
-  // LoRA B regrouped for the stream kernel's finish step (skinny_regroup_b): [unit][row][rank half]
-  // [column][16 ranks] bf16, for M <= 16 and rank <= 32
-  const bool regroup = rank > 0 && rank <= 32u && m <= 16u;
-  L.total = L.bsel + (regroup ? (uint64_t)(n_padded(n) / 16u) * m * 2u * 16u * 32u : 0u);
+  L.total = L.row_scaling + 256u;
   return L;
 }
 
-inline uint64_t skinny_workspace_bytes(uint32_t m, uint32_t n, uint32_t rank) {
-  return skinny_layout(m, 128u, n, rank).total;
-}
+inline uint64_t skinny_workspace_bytes() { return skinny_layout(128u).total; }
 inline bool skinny_supported() { return true; }
 
 // ---------------------------------------------------------------------------------------
@@ -60,62 +55,54 @@ struct SkinnyQuantArgs {
   float* sx;             // f32 [32]
   int8_t* codes_rm;      // optional row-major copy
   float* scales_rm;      // optional
-  uint16_t* xn;          // bf16 [M, K] normalized rows (RMSNorm only) or null
-  uint16_t* xn_aux;      // optional copy for the caller
-  // LoRA-A work units that share the launch (they need only x, not the codes); with RMSNorm they
-  // need the normalized rows and run as a launch of their own
+  uint16_t* xn_aux;      // bf16 [M, K] normalized rows for the caller (RMSNorm only) or null
+  // LoRA-A work units that share the launch (they need only x, not the codes)
   const uint16_t* lora_a;  // bf16 [n_adapters, K, r] or null
   const int32_t* idx;      // adapter per row or null
   float* z_part;           // f32 [z_chunks][32][kMaxRank]
   uint32_t n_adapters, r, z_chunks, z_chunk_k, n_z_units;
-  // LoRA-B regrouping items that share the launch (M <= 16, rank <= 32, N % 8 == 0), four per block
-  const uint16_t* lora_b;  // bf16 [n_adapters, r, N] or null
-  uint16_t* bsel;          // bf16 [N_pad/16 units][M][2][16][16]
-  uint32_t N, n_groups;    // n_groups = N_pad / 128
   const float* lora_scaling;  // f32 [n_adapters] or null
   float* row_scaling;      // f32 [32]: lora_scaling[idx[m]], written here for the stream kernel
 };
 
-// The stream kernel's unit u = 8 G + 2 j + h owns the original columns 128 G + 4 (16 h + c) + j,
-// c = 0..15, and its finish step needs, per row m and column c, the ranks of one parity:
-//   bsel[u][m][p][c][t] = B[idx[m]][p + 2 t][128 G + 4 (16 h + c) + j],  t = 0..15
-// so that a thread reads its 16 values as one 32-byte piece instead of 16 two-byte values that each
-// cost a 128-byte line.  One item = (row m, column group G): its r x 128 tile of B goes through LDS.
-__device__ inline void skinny_regroup_b(const SkinnyQuantArgs& a, uint32_t block, uint16_t (*tile)[32][128]) {
-  const uint32_t team = threadIdx.x >> 8, t256 = threadIdx.x & 255u;
-  const uint32_t item = block * 4u + team;
-  const bool live = item < a.M * a.n_groups;
-  const uint32_t m = live ? item / a.n_groups : 0u, G = live ? item % a.n_groups : 0u;
-  int ad = a.idx ? a.idx[m] : 0;
-  ad = ad < 0 ? 0 : (ad >= (int)a.n_adapters ? (int)a.n_adapters - 1 : ad);
-  const uint16_t* Bsrc = a.lora_b + (size_t)ad * a.r * a.N + G * 128u;
+// Inverse RMS of row xr by a workgroup of 1024 threads (float64 sum, IEEE division and square root), the
+// same value in every workgroup that forms it: v holds the thread's 2 x 8 values of the row.
+__device__ inline float skinny_inverse_rms(const float (&v)[2][8], uint32_t K, float eps, double* red_sum) {
+  double ss = 0.0;
 #pragma unroll
-  for (uint32_t u = 0; u < 2; ++u) {  // 32 ranks x 16 pieces of 8 columns
-    const uint32_t piece = t256 + 256u * u, rr = piece >> 4, c8 = (piece & 15u) * 8u;
-    v8us v = {0, 0, 0, 0, 0, 0, 0, 0};
-    if (live && rr < a.r && G * 128u + c8 < a.N) v = *reinterpret_cast<const v8us*>(Bsrc + (size_t)rr * a.N + c8);
-    *reinterpret_cast<v8us*>(&tile[team][rr][c8]) = v;
-  }
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) ss += (double)v[j][e] * (double)v[j][e];
+  ss = wave_sum(ss);
+  if ((threadIdx.x & 63u) == 0) red_sum[threadIdx.x >> 6] = ss;
   __syncthreads();
-  if (!live) return;
-  const uint32_t u8 = t256 >> 5, par = (t256 >> 4) & 1u, c = t256 & 15u;
-  const uint32_t col = 4u * (16u * (u8 & 1u) + c) + (u8 >> 1);
-  v8us lo, hi;
+  double tot = 0.0;
 #pragma unroll
-  for (uint32_t t = 0; t < 8; ++t) {
-    lo[t] = tile[team][par + 2u * t][col];
-    hi[t] = tile[team][par + 2u * (t + 8u)][col];
+  for (int w = 0; w < 16; ++w) tot += red_sum[w];
+  const float var = (float)(tot / (double)K);
+  return 1.0f / sqrtf(var + eps);
+}
+__device__ inline void skinny_row_values(const uint16_t* __restrict__ xr, uint32_t K, float (&v)[2][8]) {
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const uint32_t k0 = (j * 1024u + threadIdx.x) * 8u;
+    uint4 raw = make_uint4(0, 0, 0, 0);
+    if (k0 < K) raw = *reinterpret_cast<const uint4*>(xr + k0);
+    const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      v[j][2 * e] = __uint_as_float(w[e] << 16);
+      v[j][2 * e + 1] = __uint_as_float(w[e] & 0xffff0000u);
+    }
   }
-  uint16_t* dst = a.bsel + (((((size_t)G * 8u + u8) * a.M + m) * 2u + par) * 16u + c) * 16u;
-  *reinterpret_cast<v8us*>(dst) = lo;
-  *reinterpret_cast<v8us*>(dst + 8) = hi;
 }
 
 // z_part[ch][m][:] = x[m, chunk ch] @ A[idx[m]][chunk ch, :] in float32.  Thread (kl, q)
 // accumulates rank columns 8q..8q+7 over the rows k = k_begin + kl + kpt*j; lanes with equal q are
-// reduced by a fixed butterfly and the waves are added in wave order.
-template <int THREADS>
-__device__ inline void skinny_lora_a_unit(const uint16_t* __restrict__ xsrc, const uint16_t* __restrict__ lora_a,
+// reduced by a fixed butterfly and the waves are added in wave order.  With RMS the row's values are the
+// normalized ones, bf16((x * inv) * gamma), formed here as the quantizer forms them.
+template <int THREADS, bool RMS>
+__device__ inline void skinny_lora_a_unit(const uint16_t* __restrict__ xsrc, const float* __restrict__ gamma, float inv, const uint16_t* __restrict__ lora_a,
                                           const int32_t* __restrict__ idx, float* __restrict__ z_part,
                                           uint32_t unit, uint32_t K, uint32_t n_adapters, uint32_t r,
                                           uint32_t z_chunks, uint32_t z_chunk_k, float (*zw)[64]) {
@@ -139,7 +126,7 @@ __device__ inline void skinny_lora_a_unit(const uint16_t* __restrict__ xsrc, con
       // four rows of A per round, their loads issued together (same order of additions as a plain loop)
       for (uint32_t k = k_begin + kl; k < k_end; k += 4u * kpt) {
         v8us w[4];
-        float xv[4];
+        float xv[4], gv[4];
 #pragma unroll
         for (uint32_t u = 0; u < 4; ++u) {
           const uint32_t ku = k + u * kpt;
@@ -147,6 +134,11 @@ __device__ inline void skinny_lora_a_unit(const uint16_t* __restrict__ xsrc, con
           const v8us zero = {0, 0, 0, 0, 0, 0, 0, 0};
           w[u] = in ? *reinterpret_cast<const v8us*>(Ar + (size_t)ku * r + q * 8u) : zero;
           xv[u] = in ? bf16_bits_to_f32(xr[ku]) : 0.f;
+          gv[u] = (RMS && in) ? gamma[ku] : 0.f;
+        }
+        if (RMS) {
+#pragma unroll
+          for (uint32_t u = 0; u < 4; ++u) xv[u] = bf16_round_f32((xv[u] * inv) * gv[u]);
         }
 #pragma unroll
         for (uint32_t u = 0; u < 4; ++u) {
@@ -158,7 +150,8 @@ __device__ inline void skinny_lora_a_unit(const uint16_t* __restrict__ xsrc, con
       }
     } else {
       for (uint32_t k = k_begin + kl; k < k_end; k += kpt) {
-        const float xv = bf16_bits_to_f32(xr[k]);
+        float xv = bf16_bits_to_f32(xr[k]);
+        if (RMS) xv = bf16_round_f32((xv * inv) * gamma[k]);
         const uint16_t* src = Ar + (size_t)k * r + q * 8u;
 #pragma unroll
         for (int e = 0; e < 8; ++e)
@@ -188,47 +181,25 @@ __global__ __launch_bounds__(1024) void skinny_quant_kernel(SkinnyQuantArgs a) {
   __shared__ float red_max[16];
   __shared__ double red_sum[16];
   __shared__ float zw[16][64];
-  if (blockIdx.x >= a.M + a.n_z_units) {
-    __shared__ __attribute__((aligned(16))) uint16_t tile[4][32][128];  // 32 KiB
-    skinny_regroup_b(a, blockIdx.x - a.M - a.n_z_units, tile);
-    return;
-  }
   if (blockIdx.x >= a.M) {
     const uint32_t unit = blockIdx.x - a.M;
-    skinny_lora_a_unit<1024>(a.x, a.lora_a, a.idx, a.z_part, unit, a.K, a.n_adapters, a.r, a.z_chunks,
-                             a.z_chunk_k, zw);
+    float inv = 1.0f;
+    if (RMS) {
+      float v[2][8];
+      skinny_row_values(a.x + (size_t)(unit / a.z_chunks) * a.K, a.K, v);
+      inv = skinny_inverse_rms(v, a.K, a.eps, red_sum);
+    }
+    skinny_lora_a_unit<1024, RMS>(a.x, a.gamma, inv, a.lora_a, a.idx, a.z_part, unit, a.K, a.n_adapters, a.r, a.z_chunks,
+                                  a.z_chunk_k, zw);
     return;
   }
   const uint32_t m = blockIdx.x;
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
   const uint16_t* xr = a.x + (size_t)m * a.K;
   float v[2][8];
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const uint32_t k0 = (j * 1024u + tid) * 8u;
-    uint4 raw = make_uint4(0, 0, 0, 0);
-    if (k0 < a.K) raw = *reinterpret_cast<const uint4*>(xr + k0);
-    const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      v[j][2 * e] = __uint_as_float(w[e] << 16);
-      v[j][2 * e + 1] = __uint_as_float(w[e] & 0xffff0000u);
-    }
-  }
+  skinny_row_values(xr, a.K, v);
   if (RMS) {
-    double ss = 0.0;
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) ss += (double)v[j][e] * (double)v[j][e];
-    ss = wave_sum(ss);
-    if (lane == 0) red_sum[wave] = ss;
-    __syncthreads();
-    double tot = 0.0;
-#pragma unroll
-    for (int w = 0; w < 16; ++w) tot += red_sum[w];
-    const float var = (float)(tot / (double)a.K);
-    const float inv = 1.0f / sqrtf(var + a.eps);
+    const float inv = skinny_inverse_rms(v, a.K, a.eps, red_sum);
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const uint32_t k0 = (j * 1024u + tid) * 8u;
@@ -246,7 +217,6 @@ __global__ __launch_bounds__(1024) void skinny_quant_kernel(SkinnyQuantArgs a) {
           if (e & 1) packed[e >> 1] |= b << 16; else packed[e >> 1] = b;
         }
         const uint4 o = make_uint4(packed[0], packed[1], packed[2], packed[3]);
-        if (a.xn) *reinterpret_cast<uint4*>(a.xn + (size_t)m * a.K + k0) = o;
         if (a.xn_aux) *reinterpret_cast<uint4*>(a.xn_aux + (size_t)m * a.K + k0) = o;
       }
     }
@@ -292,19 +262,6 @@ __global__ __launch_bounds__(1024) void skinny_quant_kernel(SkinnyQuantArgs a) {
 }
 
 // ---------------------------------------------------------------------------------------
-// LoRA-A units as a launch of their own (only when they need the normalized rows of the
-// quantizer launch; otherwise they ride along with it).
-struct SkinnyLoraAArgs {
-  const uint16_t* xsrc; const uint16_t* lora_a; const int32_t* idx; float* z_part;
-  uint32_t K, n_adapters, r, z_chunks, z_chunk_k;
-};
-__global__ __launch_bounds__(1024) void skinny_lora_a_kernel(SkinnyLoraAArgs a) {
-  __shared__ float zw[16][64];
-  skinny_lora_a_unit<1024>(a.xsrc, a.lora_a, a.idx, a.z_part, blockIdx.x, a.K, a.n_adapters, a.r, a.z_chunks,
-                           a.z_chunk_k, zw);
-}
-
-// ---------------------------------------------------------------------------------------
 constexpr uint32_t kSkinnyStreamWaves = 8;   // waves of a stream workgroup; they split K
 constexpr uint32_t kSkinnyStreamThreads = kSkinnyStreamWaves * 64u;
 
@@ -315,316 +272,341 @@ struct SkinnyStreamArgs {
   const float* sx;           // f32 [32]
   const float* sw;           // f32 [N]
   const uint16_t* lora_b;    // bf16 [n_adapters, r, N] or null
-  const uint16_t* bsel;      // B regrouped per unit (skinny_regroup_b) or null: then B is gathered directly
-  const float* lora_scaling;
   const float* row_scaling;  // f32 [32]: lora_scaling[idx[m]] (from the quantizer launch)
   const int32_t* idx;        // adapter per row or null
   const uint16_t* residual;  // bf16 [M, N] or null
-  uint16_t* out;             // bf16 [M, N]
+  uint16_t* out;             // bf16 [M, N], or [M, N / 2] with swiglu
   int32_t* aux_acc;          // int32 [M, N] or null
-  uint32_t M, N, N_pad, K, KB, pairs_per_wave, n_adapters, r, z_chunks, n_groups;
+  uint32_t M, N, K, KB, pairs_per_wave, n_adapters, r, z_chunks, n_groups;
+  uint32_t swiglu;
+  uint32_t z_off;            // bytes of the staged B in front of the staged z partials (skinny_stream_lds)
+  uint32_t tail_off;         // ... of both (or of the accumulators that take their place), in front of the rest
 };
 
-// Every workgroup owns 16 packed weight columns for all of K and finishes them itself; nothing
-// crosses workgroups.
+// LDS of a stream workgroup: [staged B rows | staged z partials], the same bytes later the waves'
+// accumulators; behind them z, the per-output scales and the odd-rank sums.
+struct SkinnyStreamLds { uint32_t z_off, tail_off, bytes; };
+constexpr uint32_t kSkinnyZlStride = 65;  // floats between two rows of z: four rows a wave reads at a time in four banks
+constexpr uint32_t kSkinnyTailBytes = 16u * kSkinnyZlStride * 4u + 5u * 2048u + 2u * 1024u + 64u;
+inline SkinnyStreamLds skinny_stream_lds(uint32_t m, uint32_t r, uint32_t z_chunks, uint32_t ns, uint32_t rb) {
+  SkinnyStreamLds L{};
+  const uint32_t rows = m < 16u ? m : 16u, rpad = round_up(r, 4u);
+  const uint32_t per_piece = r <= 32u ? 8u : 4u;  // rows of z per KiB
+  L.z_off = r ? round_up(rows * rpad * 64u + 4u * 64u, 1024u) : 0u;
+  const uint32_t staged = L.z_off + (r ? z_chunks * ((rows + per_piece - 1u) / per_piece) * 1024u : 0u);
+  const uint32_t red = kSkinnyStreamWaves * ns * rb * 1024u;
+  L.tail_off = staged > red ? staged : red;
+  L.bytes = L.tail_off + kSkinnyTailBytes;
+  return L;
+}
+
+// Every workgroup owns NS slices of 16 packed weight columns for all of K and finishes them itself;
+// nothing crosses workgroups.
 //  * Its eight waves each stream a K range of the weight from HBM straight into
 //    v_mfma_i32_16x16x64_i8 operands (a lane loads its 16 bytes from the 1 KiB fragment blocks:
-//    column c of a block pair's four 16-wide k chunks) and are reduced through LDS.
-//  * Finish: (float(acc) * sx) * sw + s * (z @ B) + residual, one bf16 cast.  z[m][r] is the
-//    fixed-order sum of the LoRA-A partials; the rank sum runs in two fixed halves.
-// Packed column pc of block nb is original column 128*(nb/4) + 4*pc + nb%4, so the eight units of
-// a 128-column group read the same stretches of B; they are given workgroup ids that land on one
-// XCD (ids are dealt round-robin to the XCDs) so that those stretches come from HBM once.
-template <bool ROWS2>  // more than 16 rows: a second MFMA per step for rows 16..31
-__global__ __launch_bounds__(kSkinnyStreamThreads) void skinny_stream_kernel(SkinnyStreamArgs a) {
-  // 64-wide k steps a wave keeps in flight (1 KiB of weight each): 192 KiB per workgroup, one
-  // workgroup per CU
-  constexpr uint32_t kInFlight = ROWS2 ? 16 : 24;
-  constexpr uint32_t kRankSplit = ROWS2 ? 1 : 2;  // threads per output in the finish step
-  __shared__ __attribute__((aligned(16))) int red[kSkinnyStreamWaves][2][4][64];  // 16 KiB
-  __shared__ float zl[kSkinnyMaxRows][kMaxRank];                                 // 8 KiB
-  __shared__ float low_odd[256];
-  // one-round form: the finish step's LoRA operands, staged by direct-to-LDS loads behind the weight stream
-  __shared__ __attribute__((aligned(1024))) float zst[ROWS2 ? 1 : kSkinnyMaxZChunks][16][32];  // z partials [chunk][row][rank], 32 KiB
-  __shared__ __attribute__((aligned(1024))) uint16_t bst[ROWS2 ? 8 : 16 * 2 * 16 * 16];         // the unit's regrouped B, 16 KiB
-  __shared__ __attribute__((aligned(1024))) uint32_t fst[4][256];  // per output thread: sx, sw, the row's LoRA scaling, the residual's dword
+//    column c of a block pair's four 16-wide k chunks) and are reduced through LDS.  KP is what a wave
+//    keeps in flight: KP 64-wide k steps of every slice; a longer share of K takes further rounds.
+//  * Finish: (float(acc) * sx) * sw + s * (z @ B) + residual, one bf16 cast, or SwiGLU.  z[m][r] is the
+//    fixed-order sum of the LoRA-A partials; the rank sum runs as an even and an odd chain.
+// Slice (nb, half) is the original columns 128 G + 4 (16 half + c) + j, c = 0..15, of column block
+// nb = 4 G + j.  NS = 2 takes j = 2 p and 2 p + 1: adjacent column pairs, so a dword of B (or of the output)
+// is both columns, and a fused gate/up projection's (gate, up) pair ends in one thread.  The units of a
+// 128-column group share stretches of B and of memory pages; they get workgroup ids that land on one XCD
+// (ids are dealt round-robin to the XCDs).
+//
+// Bound by HBM, and for short weights by the latency of the launch.  What the finish step works with (the
+// rows' B, the z partials, scales, residual) takes no registers -- the MFMA operands take all there are --
+// the waves copy it into the LDS with direct-to-LDS loads, the first loads they issue (a wave's loads return
+// in order), and form the low-rank term from there while the weight is on its way.  B is gathered as dwords
+// (64 per instruction: four ranks x sixteen columns) straight from its [rank, N] rows: half or all of every
+// 64 bytes fetched is used, and no regrouped copy of it is written and read back, which cost 2 x 25 MB for
+// sixteen adapters of a 24576-wide projection whenever an adapter had changed.
+// Measured: 4096 x 24576 with SwiGLU, 16 rows, 16 adapters of rank 32: 22.9 us for 126 MB (5.5 TB/s), the whole
+// call 29 us against 139 us on 128 x 128 tiles behind the tiled quantizer (which such a call took before);
+// 2560 x 6144, one row, rank 64: 8.1 us against 18.3 us with B's loads behind the weight's; 12288 x 4096,
+// 16 rows: 14.1 us (12.6 us from a regrouped B already in memory, 15.2 us with the regrouping).
+// Rows 16..31 (RB = 2) share the weight operands; their B is staged in a second step behind the stream.
+template <int NS, int RB, int KP>
+__global__ __launch_bounds__(kSkinnyStreamThreads, (NS + RB) * KP <= 24 ? 4 : 2)
+void skinny_stream_kernel(SkinnyStreamArgs a) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char sk_lds[];
   const uint32_t tid = threadIdx.x, lane = tid & 63u;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  constexpr uint32_t kUnits = 8u / NS;  // of a 128-column group
   const uint32_t slot = blockIdx.x >> 3;
-  const uint32_t grp = (slot >> 3) * 8u + (blockIdx.x & 7u);
+  const uint32_t grp = (slot / kUnits) * 8u + (blockIdx.x & 7u), unit = slot % kUnits;
   if (grp >= a.n_groups) return;
-  const uint32_t nb = grp * 4u + ((slot & 7u) >> 1), chalf = slot & 1u;
+  const uint32_t j0 = NS == 2 ? (unit >> 1) * 2u : unit >> 1, chalf = unit & 1u;
   const uint32_t c16 = lane & 15u, q = lane >> 4;        // MFMA operand: column / row c16, k chunk q
-  const uint32_t pc = 16u * chalf + c16;                 // packed column inside block nb
+  const uint32_t pc = 16u * chalf + c16;                 // packed column inside its block
   // byte offsets inside a pair of 1 KiB blocks: chunk q sits in block q/2, k half q%2
   const uint32_t w_lane_off = (q >> 1) * kBlockBytes + (pc + 32u * (q & 1u)) * 16u;
-  const uint32_t x_lane_off = (q >> 1) * kBlockBytes + (c16 + 32u * (q & 1u)) * 16u;
-  const unsigned char* wsrc = a.wp + (size_t)nb * a.KB * kBlockBytes + w_lane_off;
-  const unsigned char* xsrc = a.xq + x_lane_off;
+  // (rows beyond M repeat the last one: fewer cache lines, and their results are dropped)
+  const uint32_t xrow0 = c16 < a.M ? c16 : a.M - 1u, xrow1 = c16 + 16u < a.M ? c16 + 16u : a.M - 1u;
+  const uint32_t x_chunk = (q >> 1) * kBlockBytes + 512u * (q & 1u);
   const uint32_t n_pairs = a.KB >> 1;
   uint32_t p0 = wave * a.pairs_per_wave, p1 = p0 + a.pairs_per_wave;
   if (p0 > n_pairs) p0 = n_pairs;
   if (p1 > n_pairs) p1 = n_pairs;
+  // Buffer resources that end with the wave's share of K: a step beyond it reads zeros without touching
+  // memory, so the loads need no clamps and the MFMAs no conditions (and no 64-bit address per load).
+  __amdgpu_buffer_rsrc_t wrsrc[NS];
+#pragma unroll
+  for (int s = 0; s < NS; ++s)
+    wrsrc[s] = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(a.wp) + (size_t)(grp * 4u + j0 + s) * a.KB * kBlockBytes,
+                                                 0, (int)(p1 * 2u * kBlockBytes), 0x00020000);
+  const __amdgpu_buffer_rsrc_t xrsrc =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(a.xq), 0, (int)(p1 * 2u * kBlockBytes), 0x00020000);
+  const uint32_t x_lane_off0 = x_chunk + xrow0 * 16u, x_lane_off1 = x_chunk + xrow1 * 16u;
 
-  // ---- finish step mapping: thread -> output (row frow, packed column pc) and a rank share
-  const uint32_t fe = (tid >> 6) & 3u;
-  const uint32_t frow = (ROWS2 ? 16u * (tid >> 8) : 0u) + 4u * q + fe;
-  const uint32_t rsel = ROWS2 ? 0u : (tid >> 8);  // ranks rsel, rsel + kRankSplit, ...
-  const uint32_t fn = 128u * (nb >> 2) + 4u * pc + (nb & 3u);
-  const bool fvalid = frow < a.M && fn < a.N;
+  // ---- finish step mapping: thread -> output row, columns fn .. fn + NS - 1, and (RB = 1) a rank parity.
+  // Each use derives it anew from the thread id behind an opaque copy: kept across the stream it would take
+  // registers that the operands in flight need.
+  struct Finish {
+    uint32_t t8, t256, lane, fe, frow16, frow, c16, fn, srow, scol;
+    bool valid;
+  };
+  auto finish_map = [&]() -> Finish {
+    uint32_t t = threadIdx.x;
+    asm volatile("" : "+v"(t));
+    Finish f;
+    f.t8 = t >> 8; f.t256 = t & 255u; f.lane = t & 63u;
+    f.fe = (t >> 6) & 3u;
+    f.c16 = t & 15u;
+    f.frow16 = 4u * (f.lane >> 4) + f.fe;                  // row inside its half
+    f.frow = (RB == 2 ? 16u * f.t8 : 0u) + f.frow16;
+    f.fn = 128u * grp + 4u * (16u * chalf + f.c16) + j0;
+    f.valid = f.frow < a.M && f.fn < a.N;                  // (NS = 2 needs an even N: both columns exist or none)
+    // Lanes without an output read element 0 instead of selecting on the loaded value.
+    f.srow = f.valid ? f.frow : 0u;
+    f.scol = f.valid ? f.fn : 0u;
+    return f;
+  };
   const bool lora = a.lora_b != nullptr;
-  // Lanes without an output read element 0 instead of selecting on the loaded value.
-  const uint32_t srow = fvalid ? frow : 0u, scol = fvalid ? fn : 0u;
-  // z[m][r] share of this thread: value index tid (and tid + 512, ...) of the M x rpad values
-  const uint32_t rpad = (a.r + 7u) & ~7u;
-  const uint32_t n_zval = lora ? a.M * rpad : 0u;
-  // With B regrouped per unit the low-rank term needs three independent, coalesced requests per
-  // thread: its 16 ranks of B, its z partials, its row's scaling.
-  const bool early = !ROWS2 && lora && a.bsel != nullptr && n_zval <= kSkinnyStreamThreads;  // workgroup-uniform
-  float low = 0.f, f_s = 0.f, f_sx, f_sw;
-  uint16_t res_raw = 0;
-  v4i acc0 = {0, 0, 0, 0}, acc1 = {0, 0, 0, 0};
+  const uint32_t rpad = (a.r + 3u) & ~3u;
+  const uint32_t rp = a.r <= 32u ? 32u : 64u;            // ranks of a staged z row
+  uint32_t* const bst = reinterpret_cast<uint32_t*>(sk_lds);
+  const float* const zst = reinterpret_cast<const float*>(sk_lds + a.z_off);
+  int* const red = reinterpret_cast<int*>(sk_lds);       // [wave][slice][row half][4][64], once the staged data is spent
+  float* const zl = reinterpret_cast<float*>(sk_lds + a.tail_off);
+  uint32_t* const fst = reinterpret_cast<uint32_t*>(zl + 16u * kSkinnyZlStride);  // [5][512]: sx, sw, scaling, residual, sw of the second column
+  float* const low_odd = reinterpret_cast<float*>(fst + 5u * 512u);               // [NS][256]
+  uint32_t* const odd_base = reinterpret_cast<uint32_t*>(low_odd + 512u);          // [16]
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(lptr_t)sk_lds;
+  const uint32_t fst_addr = lds0 + a.tail_off + 16u * kSkinnyZlStride * 4u + wave * 256u;
 
-  // ---- One round: every wave's share of K is exactly what it keeps in flight (K = 512 * kInFlight: the
-  // Qwen3-8B down projection), and the low-rank term, if any, has its regrouped B.
-  //  * What the finish step works with (the unit's regrouped B, the z partials of all rows, every output's
-  //    scales and residual) takes no registers -- the operands of the MFMAs take all there are, and a
-  //    value loaded beside them is spilled behind a wait for the whole stream -- the waves copy it into
-  //    the LDS with direct-to-LDS loads, the first loads they issue.
-  //  * Then the code and the weight loads go out, nothing waited for, spilled or converted in front of
-  //    them.
-  //  * While the weight is on its way the low-rank term is formed from the LDS (a wave's loads return in
-  //    order: a wait that leaves only the code and weight loads outstanding has the staged pieces).
-  //  * The MFMAs run as their operands arrive, and what is left behind them is the sum over the waves and
-  //    one line of float32 arithmetic per output.
-  const bool one_round = !ROWS2 && n_pairs == kSkinnyStreamWaves * kInFlight && (!lora || early);  // workgroup-uniform
-  if (one_round) {
-    // the staged operands first: a handful of instructions, and their data is then in the LDS long before
-    // the weight is in the registers
-    const uint32_t res_elem = srow * a.N + scol;  // (M * N is below 2^32)
-    if (lora) {  // kernel-uniform
-      const uint32_t unit = grp * 8u + (slot & 7u);
-      const unsigned char* bsrc = reinterpret_cast<const unsigned char*>(a.bsel) + (size_t)unit * a.M * 1024u;  // M KiB, contiguous
-      const uint32_t bst_addr = (uint32_t)(uintptr_t)(lptr_t)bst, zst_addr = (uint32_t)(uintptr_t)(lptr_t)zst;
-      for (uint32_t i = wave; i < a.M; i += kSkinnyStreamWaves) lds_load_1k(bsrc, i * 1024u + lane * 16u, bst_addr + i * 1024u);
-      // z partials: per chunk the first 32 ranks of rows 0..15, two pieces of eight rows x 128 bytes
-      for (uint32_t i = wave; i < 2u * a.z_chunks; i += kSkinnyStreamWaves) {
-        const uint32_t ch = i >> 1, h = i & 1u;
-        const uint32_t voff = ((ch * (uint32_t)kSkinnyMaxRows + 8u * h + (lane >> 3)) * (uint32_t)kMaxRank) * 4u + (lane & 7u) * 16u;
-        lds_load_1k(reinterpret_cast<const unsigned char*>(a.z_part), voff, zst_addr + i * 1024u);
+  // adapters of the rows this wave stages (wave, wave + 8, ...)
+  int ads[2 * RB];
+#pragma unroll
+  for (uint32_t i = 0; i < 2u * RB; ++i) {
+    const uint32_t m = wave + 8u * i;
+    int ad = (lora && a.idx && m < a.M) ? a.idx[m] : 0;
+    ad = ad < 0 ? 0 : (ad >= (int)a.n_adapters ? (int)a.n_adapters - 1 : ad);
+    ads[i] = __builtin_amdgcn_readfirstlane(ad);
+  }
+  // B rows and z partials of rows 16 hf .. 16 hf + 15 on their way into the LDS
+  auto stage_half = [&](uint32_t hf) {
+    const uint32_t rows = a.M - 16u * hf < 16u ? a.M - 16u * hf : 16u;
+#pragma unroll
+    for (uint32_t mi = 0; mi < 2u; ++mi) {
+      const uint32_t m = wave + 8u * mi;
+      if (m >= rows) break;
+      const int ad = (RB == 2 && hf) ? ads[RB == 2 ? 2 + mi : mi] : ads[mi];
+      // (the gathers are dwords on 4-byte boundaries: an adapter that starts in the middle of one -- odd N and
+      // rank -- is addressed from the boundary in front of it)
+      const size_t e0 = (size_t)ad * a.r * a.N;
+      const uint32_t odd0 = (uint32_t)(e0 & 1u);
+      if (lane == 0) odd_base[m] = odd0;
+      const uint16_t* brow = a.lora_b + (e0 - odd0);
+      const uint32_t dst = lds0 + m * rpad * 64u + (m >> 2) * 64u;
+      uint32_t col = 128u * grp + 4u * pc + j0;
+      if (col + NS > a.N) col = 0u;
+      for (uint32_t i = 0; i < rpad / 4u; ++i) {
+        uint32_t rr = 4u * i + q;
+        rr = rr < a.r ? rr : a.r - 1u;
+        lds_gather_dword(brow, ((rr * a.N + col + odd0) * 2u) & ~3u, dst + i * 256u);
       }
-      // the chunk slots no unit has written count as zeros, so that the sum below needs no conditions
-      for (uint32_t i = a.z_chunks * 128u + tid; i < kSkinnyMaxZChunks * 128u; i += kSkinnyStreamThreads)
-        reinterpret_cast<float4*>(&zst[0][0][0])[i] = make_float4(0.f, 0.f, 0.f, 0.f);
     }
-    if (wave < 4u) {  // the output threads: thread tid finds its four values at fst[.][tid]
-      const uint32_t fst_addr = (uint32_t)(uintptr_t)(lptr_t)fst + wave * 256u;
-      lds_gather_dword(a.sx, srow * 4u, fst_addr);
-      lds_gather_dword(a.sw, scol * 4u, fst_addr + 1024u);
-      if (lora) lds_gather_dword(a.row_scaling, srow * 4u, fst_addr + 2048u);
-      if (a.residual) lds_gather_dword(a.residual, (res_elem * 2u) & ~3u, fst_addr + 3072u);
+    const uint32_t per_piece = 1024u / (rp * 4u), pieces = (rows + per_piece - 1u) / per_piece;
+    const uint32_t lanes_row = rp / 4u;  // lanes of 16 bytes per row
+    for (uint32_t i = wave; i < pieces * a.z_chunks; i += kSkinnyStreamWaves) {
+      const uint32_t ch = i / pieces, pi = i % pieces;
+      const uint32_t row = 16u * hf + pi * per_piece + lane / lanes_row;
+      const uint32_t voff = ((ch * (uint32_t)kSkinnyMaxRows + row) * (uint32_t)kMaxRank) * 4u + (lane % lanes_row) * 16u;
+      lds_load_1k(reinterpret_cast<const unsigned char*>(a.z_part), voff, lds0 + a.z_off + i * 1024u);
     }
-    v4i wf[kInFlight], xf[kInFlight];
-    const unsigned char* wb = wsrc + (size_t)p0 * 2u * kBlockBytes;
-    const unsigned char* xb = xsrc + (size_t)p0 * 2u * kBlockBytes;
+  };
+  // z of the staged rows, then the thread's share of the low-rank term (every wave has its pieces: a
+  // barrier stands in front)
+  auto low_rank = [&](uint32_t hf, float (&low)[NS]) {
+    const Finish f = finish_map();
+    const uint32_t rows = a.M - 16u * hf < 16u ? a.M - 16u * hf : 16u;
+    const uint32_t per_piece = 1024u / (rp * 4u), chunk_stride = (rows + per_piece - 1u) / per_piece * 256u;
+    for (uint32_t zi = tid; zi < rows * rp; zi += kSkinnyStreamThreads) {
+      float s4[4] = {0.f, 0.f, 0.f, 0.f};  // four interleaved partial sums, combined in a fixed order
+      for (uint32_t ch = 0; ch < a.z_chunks; ch += 4u) {
+#pragma unroll
+        for (uint32_t u = 0; u < 4u; ++u)
+          if (ch + u < a.z_chunks) s4[u] += zst[(ch + u) * chunk_stride + zi];
+      }
+      zl[(zi / rp) * kSkinnyZlStride + zi % rp] = ((s4[0] + s4[1]) + s4[2]) + s4[3];
+    }
+    __syncthreads();
+    if ((RB == 1 || f.t8 == hf) && f.frow < a.M) {
+      const uint32_t* bl = bst + f.frow16 * rpad * 16u + (f.frow16 >> 2) * 16u + f.c16;
+      const float* zr = zl + f.frow16 * kSkinnyZlStride;
+      const uint32_t odd_row = NS == 1 ? odd_base[f.frow16] : 0u;
+      const uint32_t r0 = RB == 2 ? 0u : f.t8, step = RB == 2 ? 1u : 2u;
+#pragma unroll 2
+      for (uint32_t r = r0; r < a.r; r += step) {
+        const uint32_t w = bl[r * 16u];
+        const float z = zr[r];
+        if constexpr (NS == 2) {
+          low[0] = fmaf(z, __uint_as_float(w << 16), low[0]);
+          low[1] = fmaf(z, __uint_as_float(w & 0xffff0000u), low[1]);
+        } else {
+          const bool odd = ((r * a.N + f.scol + odd_row) & 1u) != 0;  // which half of the dword holds the column
+          low[0] = fmaf(z, __uint_as_float(odd ? w & 0xffff0000u : w << 16), low[0]);
+        }
+      }
+    }
+    if constexpr (RB == 1) {  // the two rank parities of an output, added in a fixed order
+      if (f.t8 == 1u) {
+#pragma unroll
+        for (int s = 0; s < NS; ++s) low_odd[s * 256 + f.t256] = low[s];
+      }
+      __syncthreads();
+      if (f.t8 == 0u) {
+#pragma unroll
+        for (int s = 0; s < NS; ++s) low[s] = low[s] + low_odd[s * 256 + f.t256];
+      }
+    }
+  };
+
+  if (lora) stage_half(0);  // kernel-uniform
+  if (RB == 2 || wave < 4u) {  // the output threads: thread tid finds its values at fst[.][tid]
+    const Finish f = finish_map();
+    const uint32_t srow = f.srow, scol = f.scol, res_elem = srow * a.N + scol;  // (M * N is below 2^32)
+    lds_gather_dword(a.sx, srow * 4u, fst_addr);
+    lds_gather_dword(a.sw, scol * 4u, fst_addr + 2048u);
+    if (lora) lds_gather_dword(a.row_scaling, srow * 4u, fst_addr + 4096u);
+    if (a.residual) lds_gather_dword(a.residual, (res_elem * 2u) & ~3u, fst_addr + 6144u);
+    if constexpr (NS == 2) lds_gather_dword(a.sw, (scol + 1u < a.N ? scol + 1u : scol) * 4u, fst_addr + 8192u);
+  }
+
+  // accumulators take turns, so that no MFMA waits for the one before it (integer sums: any order)
+  constexpr int kTurns = NS * RB >= 4 ? 1 : 4 / (NS * RB);
+  v4i acc[kTurns][NS][RB];
+  float low[NS];
+#pragma unroll
+  for (int s = 0; s < NS; ++s) low[s] = 0.f;
+
+  // One round: KP steps of every slice requested, then multiplied.  The first one forms the low-rank term in
+  // between (and starts the accumulators, which so take no registers while it does).
+  auto round = [&](uint32_t base, auto first) {
+    v4i wf[KP][NS], xf[KP][RB];
     // (the codes first: they come from the L2 and are in the registers long before the weight, whose
     // requests the memory takes at its own pace)
 #pragma unroll
-    for (uint32_t t = 0; t < kInFlight; ++t) xf[t] = *reinterpret_cast<const v4i*>(xb + t * 2u * kBlockBytes);
+    for (uint32_t t = 0; t < (uint32_t)KP; ++t)
+#pragma unroll
+      for (int b = 0; b < RB; ++b)
+        xf[t][b] = __builtin_amdgcn_raw_buffer_load_b128(xrsrc, (b ? x_lane_off1 : x_lane_off0) + (base + t) * 2u * kBlockBytes, 0, 0);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (uint32_t t = 0; t < kInFlight; ++t)
-      wf[t] = __builtin_nontemporal_load(reinterpret_cast<const v4i*>(wb + t * 2u * kBlockBytes));
+    for (uint32_t t = 0; t < (uint32_t)KP; ++t)
+#pragma unroll
+      for (int s = 0; s < NS; ++s)  // (non-temporal)
+        wf[t][s] = __builtin_amdgcn_raw_buffer_load_b128(wrsrc[s], w_lane_off + (base + t) * 2u * kBlockBytes, 0, 2);
     __builtin_amdgcn_sched_barrier(0);
-    // ---- the low-rank term, while the weight is on its way: the staged operands are the wave's oldest
-    // loads, so a wait that leaves the code and weight loads outstanding has them
+    if constexpr (decltype(first)::value) {
+      if (lora) {  // kernel-uniform: the low-rank term, while the weight is on its way
+        // the staged operands are the wave's oldest loads: a wait that leaves the code and weight loads
+        // outstanding has them
+        asm volatile("s_waitcnt vmcnt(%0)" :: "n"(KP * (NS + RB)) : "memory");
+        __syncthreads();  // ... and the other waves' pieces
+        low_rank(0u, low);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int u = 0; u < kTurns; ++u)
+#pragma unroll
+        for (int s = 0; s < NS; ++s)
+#pragma unroll
+          for (int b = 0; b < RB; ++b) acc[u][s][b] = v4i{0, 0, 0, 0};
+    }
+#pragma unroll
+    for (uint32_t t = 0; t < (uint32_t)KP; ++t)
+#pragma unroll
+      for (int s = 0; s < NS; ++s)
+#pragma unroll
+        for (int b = 0; b < RB; ++b)
+          acc[t % kTurns][s][b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(xf[t][b], wf[t][s], acc[t % kTurns][s][b], 0, 0, 0);
+  };
+  round(p0, std::true_type{});
+#pragma unroll 1
+  for (uint32_t base = p0 + (uint32_t)KP; base < p1; base += (uint32_t)KP) round(base, std::false_type{});
+  if constexpr (RB == 2) {
+    if (lora) {  // rows 16..31: their B and z into the same bytes
+      __syncthreads();
+      stage_half(1);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+      low_rank(1u, low);
+    }
+  }
+  __syncthreads();  // the staged operands are spent
+#pragma unroll
+  for (int s = 0; s < NS; ++s)
+#pragma unroll
+    for (int b = 0; b < RB; ++b)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        int v = acc[0][s][b][e];
+#pragma unroll
+        for (int u = 1; u < kTurns; ++u) v += acc[u][s][b][e];
+        red[(((wave * NS + s) * RB + b) * 4u + e) * 64u + lane] = v;
+      }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (without LoRA nothing has waited for the staged scales yet)
+  __syncthreads();
+  const Finish f = finish_map();
+  if ((RB == 1 && f.t8 == 1u) || !f.valid) return;
+  const float f_sx = __uint_as_float(fst[tid]);
+  const float f_s = lora ? __uint_as_float(fst[1024u + tid]) : 0.f;
+  float y[NS];
+  int sum[NS];
+#pragma unroll
+  for (int s = 0; s < NS; ++s) {
+    sum[s] = 0;
+#pragma unroll
+    for (uint32_t w = 0; w < kSkinnyStreamWaves; ++w)
+      sum[s] += red[(((w * NS + s) * RB + (RB == 2 ? f.t8 : 0u)) * 4u + f.fe) * 64u + f.lane];
+    y[s] = ((float)sum[s] * f_sx) * __uint_as_float(fst[(s == 0 ? 512u : 2048u) + tid]);
     if (lora) {
-      asm volatile("s_waitcnt vmcnt(%0)" :: "n"(2 * kInFlight) : "memory");
-      __syncthreads();  // ... and the other waves' pieces
-      {  // z[m][r] for 16 rows x 32 ranks, one per thread: four interleaved partial sums, combined in a fixed order
-        const uint32_t zr = tid >> 5, zc = tid & 31u;
-        float zv[kSkinnyMaxZChunks];
-#pragma unroll
-        for (uint32_t ch = 0; ch < kSkinnyMaxZChunks; ++ch) zv[ch] = zst[ch][zr][zc];
-        float s4[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (uint32_t ch = 0; ch < kSkinnyMaxZChunks; ++ch) s4[ch & 3u] += zv[ch];
-        zl[zr][zc] = ((s4[0] + s4[1]) + s4[2]) + s4[3];
-      }
-      __syncthreads();
-      if (wave < 4u) {  // the output threads
-        // the even and the odd ranks as two chains, added at the end: the order of the two-thread form.
-        // (Ranks beyond the rank are zeros in z and in the regrouped B alike: they add nothing.)
-        float zrow[32];
-#pragma unroll
-        for (uint32_t i = 0; i < 8; ++i) {
-          const float4 z4 = *reinterpret_cast<const float4*>(&zl[srow][4u * i]);
-          zrow[4 * i] = z4.x; zrow[4 * i + 1] = z4.y; zrow[4 * i + 2] = z4.z; zrow[4 * i + 3] = z4.w;
-        }
-        float lo2[2] = {0.f, 0.f};
-#pragma unroll
-        for (uint32_t par = 0; par < 2; ++par) {
-          const uint16_t* bl = bst + ((srow * 2u + par) * 16u + c16) * 16u;
-          const v8us blo = *reinterpret_cast<const v8us*>(bl), bhi = *reinterpret_cast<const v8us*>(bl + 8);
-#pragma unroll
-          for (uint32_t t = 0; t < 16; ++t) {
-            const uint16_t bv = t < 8u ? blo[t & 7u] : bhi[t & 7u];
-            lo2[par] = fmaf(zrow[par + 2u * t], bf16_bits_to_f32(bv), lo2[par]);
-          }
-        }
-        low = lo2[0] + lo2[1];
-      }
+      const float l = low[s] * f_s;
+      y[s] = y[s] + l;
     }
-    __builtin_amdgcn_sched_barrier(0);
-    // four accumulators take turns, so that no MFMA waits for the one before it (integer sums: any order)
-    v4i part[4] = {{0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}};
-#pragma unroll
-    for (uint32_t t = 0; t < kInFlight; ++t) part[t & 3u] = __builtin_amdgcn_mfma_i32_16x16x64_i8(xf[t], wf[t], part[t & 3u], 0, 0, 0);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) red[wave][0][e][lane] = (part[0][e] + part[1][e]) + (part[2][e] + part[3][e]);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (without LoRA nothing has waited for the staged scales yet)
-    __syncthreads();  // the accumulators of every wave
-    if (wave >= 4u) return;  // one thread per output from here on
-    f_sx = __uint_as_float(fst[0][tid]);
-    f_sw = __uint_as_float(fst[1][tid]);
-    if (a.residual) res_raw = (uint16_t)((res_elem & 1u) ? fst[3][tid] >> 16 : fst[3][tid] & 0xffffu);
-    if (lora) f_s = __uint_as_float(fst[2][tid]);
-  } else {
-  f_sx = a.sx[srow];
-  f_sw = a.sw[scol];
-  int ad_raw = 0;
-  if (lora && a.idx) ad_raw = a.idx[srow];
-  // The low-rank term's requests go out ahead of the weight loads: a wave's loads return in order, so they
-  // are back while the weight is still streaming, and the term is computed under the stream.
-  v8us blo = {0, 0, 0, 0, 0, 0, 0, 0}, bhi = {0, 0, 0, 0, 0, 0, 0, 0};
-  float zv[kSkinnyMaxZChunks];
-  if (early) {
-    if (a.residual) res_raw = a.residual[(size_t)srow * a.N + scol];
-    f_s = a.row_scaling[srow];
-    const uint32_t unit = grp * 8u + (slot & 7u);
-    const uint16_t* bs = a.bsel + (((((size_t)unit * a.M + srow) * 2u + rsel) * 16u + c16) * 16u);
-    blo = *reinterpret_cast<const v8us*>(bs);
-    bhi = *reinterpret_cast<const v8us*>(bs + 8);
-    const uint32_t zi = tid < n_zval ? tid : 0u;
-    const float* zp = a.z_part + (size_t)(zi / rpad) * kMaxRank + zi % rpad;
-#pragma unroll
-    for (uint32_t ch = 0; ch < kSkinnyMaxZChunks; ++ch)
-      zv[ch] = ch < a.z_chunks ? zp[(size_t)ch * kSkinnyMaxRows * kMaxRank] : 0.f;
   }
-  __builtin_amdgcn_sched_barrier(0);  // the weight loads below are issued after the requests above
-  uint32_t base = p0;
-  do {
-    v4i wf[kInFlight], xf[kInFlight], xg[ROWS2 ? kInFlight : 1];
+  const size_t o = (size_t)f.frow * a.N + f.fn;
+  if (a.aux_acc) {
 #pragma unroll
-    for (uint32_t t = 0; t < kInFlight; ++t) {
-      const uint32_t pr = base + t < p1 ? base + t : (p1 ? p1 - 1u : 0u);  // clamped: repeats are skipped below
-      wf[t] = __builtin_nontemporal_load(reinterpret_cast<const v4i*>(wsrc + (size_t)pr * 2u * kBlockBytes));
-    }
-#pragma unroll
-    for (uint32_t t = 0; t < kInFlight; ++t) {
-      const uint32_t pr = base + t < p1 ? base + t : (p1 ? p1 - 1u : 0u);
-      xf[t] = *reinterpret_cast<const v4i*>(xsrc + (size_t)pr * 2u * kBlockBytes);
-      if constexpr (ROWS2) xg[t] = *reinterpret_cast<const v4i*>(xsrc + (size_t)pr * 2u * kBlockBytes + 256u);
-    }
-    if (early && base == p0) {  // workgroup-uniform: the low-rank term, under the first round's loads
-      __builtin_amdgcn_sched_barrier(0);
-      if (tid < n_zval) {  // z[m][r]: four interleaved partial sums, combined in a fixed order
-        float s4[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (uint32_t ch = 0; ch < kSkinnyMaxZChunks; ++ch) s4[ch & 3u] += zv[ch];
-        zl[tid / rpad][tid % rpad] = ((s4[0] + s4[1]) + s4[2]) + s4[3];
-      }
-      __syncthreads();
-#pragma unroll
-      for (uint32_t t = 0; t < 16; ++t) {
-        const uint32_t r = rsel + kRankSplit * t;
-        const uint16_t bv = t < 8u ? blo[t & 7u] : bhi[t & 7u];
-        if (r < a.r) low = fmaf(zl[srow][r], bf16_bits_to_f32(bv), low);
-      }
-      if (rsel == 1u) low_odd[tid & 255u] = low;  // the two rank halves of an output, added in a fixed order
-      __syncthreads();
-      if (rsel == 0u) low = low + low_odd[tid];
-      __builtin_amdgcn_sched_barrier(0);
-    }
-#pragma unroll
-    for (uint32_t t = 0; t < kInFlight; ++t) {
-      if (base + t < p1) {  // wave-uniform
-        acc0 = __builtin_amdgcn_mfma_i32_16x16x64_i8(xf[t], wf[t], acc0, 0, 0, 0);
-        if constexpr (ROWS2) acc1 = __builtin_amdgcn_mfma_i32_16x16x64_i8(xg[t], wf[t], acc1, 0, 0, 0);
-      }
-    }
-    base += kInFlight;
-  } while (base < p1);
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    red[wave][0][e][lane] = acc0[e];
-    red[wave][1][e][lane] = acc1[e];
+    for (int s = 0; s < NS; ++s) a.aux_acc[o + s] = sum[s];
   }
-  if (!early) {
-    // Without the regrouped B the term's loads start only now: issued while the weight stream is in
-    // flight they would be served after it anyway, and here they cost one trip to an idle memory.
-    if (a.residual) res_raw = a.residual[(size_t)srow * a.N + scol];
-    const int ad = ad_raw < 0 ? 0 : (ad_raw >= (int)a.n_adapters ? (int)a.n_adapters - 1 : ad_raw);
-    f_s = (fvalid && lora) ? a.lora_scaling[ad] : 0.f;
-    // Every B value of the thread (ranks rsel, rsel + kRankSplit, ... below 64) is requested before the
-    // first is used: one trip to memory instead of one per value.
-    // The loads are unconditional (a load under a lane condition gets a branch and a wait of its own):
-    // lanes without an output read column 0, ranks beyond the rank read the last one; both are skipped
-    // when the values are used.
-    constexpr uint32_t kBValues = (uint32_t)kMaxRank / kRankSplit;
-    uint32_t bq[kBValues];
-    if (lora) {  // kernel-uniform
-      const uint16_t* Bs = a.lora_b + (size_t)ad * a.r * a.N + scol;
-#pragma unroll
-      for (uint32_t t = 0; t < kBValues; ++t) {
-        uint32_t r = rsel + kRankSplit * t;
-        r = r < a.r ? r : a.r - 1u;
-        bq[t] = (uint32_t)Bs[(size_t)r * a.N];
-      }
-    }
-    for (uint32_t zi = tid; zi < n_zval; zi += kSkinnyStreamThreads) {
-      const float* zp = a.z_part + (size_t)(zi / rpad) * kMaxRank + zi % rpad;
-      float zw4[kSkinnyMaxZChunks];
-#pragma unroll
-      for (uint32_t ch = 0; ch < kSkinnyMaxZChunks; ++ch)
-        zw4[ch] = ch < a.z_chunks ? zp[(size_t)ch * kSkinnyMaxRows * kMaxRank] : 0.f;
-      float s4[4] = {0.f, 0.f, 0.f, 0.f};  // four interleaved partial sums, combined in a fixed order
-#pragma unroll
-      for (uint32_t ch = 0; ch < kSkinnyMaxZChunks; ++ch) s4[ch & 3u] += zw4[ch];
-      zl[zi / rpad][zi % rpad] = ((s4[0] + s4[1]) + s4[2]) + s4[3];
-    }
-    __syncthreads();
-    if (fvalid && lora) {
-#pragma unroll
-      for (uint32_t t = 0; t < kBValues; ++t) {
-        const uint32_t r = rsel + kRankSplit * t;
-        if (r < a.r) low = fmaf(zl[frow][r], bf16_bits_to_f32(bq[t]), low);
-      }
-    }
-    if (!ROWS2) {
-      if (rsel == 1u) low_odd[tid & 255u] = low;
-      __syncthreads();
-      if (rsel == 0u) low = low + low_odd[tid];
+  if constexpr (NS == 2) {
+    const uint32_t pair = pack_bf16x2(y[0], y[1]);
+    if (a.swiglu) {  // kernel-uniform: gate and up are rounded to bf16 first
+      a.out[(size_t)f.frow * (a.N >> 1) + (f.fn >> 1)] =
+          (uint16_t)f32_to_bf16_bits(swiglu_f32(__uint_as_float(pair << 16), __uint_as_float(pair & 0xffff0000u)));
+    } else {
+      *reinterpret_cast<uint32_t*>(a.out + o) = pair;
     }
   } else {
-    __syncthreads();  // the accumulators in `red`
+    if (a.residual) {
+      const uint32_t w = fst[1536u + tid];
+      y[0] = y[0] + __uint_as_float((o & 1u) ? w & 0xffff0000u : w << 16);
+    }
+    a.out[o] = (uint16_t)f32_to_bf16_bits(y[0]);
   }
-  }
-  if (!ROWS2 && rsel == 1u) return;  // (only the multi-round form gets here with rsel == 1)
-  if (!fvalid) return;
-  int sum = 0;
-#pragma unroll
-  for (uint32_t w = 0; w < kSkinnyStreamWaves; ++w) sum += red[w][ROWS2 ? (tid >> 8) : 0u][fe][lane];
-  float y = ((float)sum * f_sx) * f_sw;
-  if (lora) {
-    const float l = low * f_s;
-    y = y + l;
-  }
-  const size_t o = (size_t)frow * a.N + fn;
-  if (a.residual) y = y + bf16_bits_to_f32(res_raw);
-  a.out[o] = (uint16_t)f32_to_bf16_bits(y);
-  if (a.aux_acc) a.aux_acc[o] = sum;
 }
 
 }  // namespace w8a8

@@ -40,6 +40,7 @@ MAX_IN_FEATURES = 16384
 MAX_OUT_FEATURES = 1 << 20
 MAX_LORA_RANK = 64
 MAX_ADAPTERS = 64
+SKINNY_MAX_ROWS = 32  # up to here a forward call runs the weight-streaming kernels
 _SUPPORTED_BLOCK_SIZES = frozenset((16, 32, 64, 128))
 
 
@@ -361,7 +362,7 @@ class ForwardPlan:
     def run(self, extra_flags: int = 0) -> torch.Tensor:
         """Enqueue the call on torch's current stream; returns the (reused) output tensor.
 
-        The transposed LoRA A and packed LoRA B (for a decode-sized call: B regrouped per row by its adapter)
+        The transposed LoRA A and packed LoRA B (a decode-sized call keeps neither)
         live in the plan's workspace: while neither tensor nor the adapter indices have been
         written since the last full run (``Tensor._version``), the call is told to keep them
         (``FLAG_LORA_PACK_VALID``) instead of packing 2 * n * r * (K + N) bytes again.  A training step
@@ -371,8 +372,8 @@ class ForwardPlan:
         # (a captured call is replayed later, when the adapters may have changed: it always packs)
         capturing = torch.cuda.is_current_stream_capturing()
         if self._lora is not None and not capturing and self.keep_lora_pack:
-            # (what the workspace holds also depends on the path the flags choose: decode kernels keep B
-            # regrouped per row, the tiled kernels A and B in operand order)
+            # (what the workspace holds also depends on the path the flags choose: the decode kernels keep
+            # nothing, the tiled kernels A and B in operand order)
             versions = (_version_of(self._lora[0]), _version_of(self._lora[1]),
                         0 if self.adapter_indices is None else _version_of(self.adapter_indices))
             if None not in versions:  # (a tensor torch keeps no version of may have been written: pack)
@@ -711,10 +712,12 @@ class _RmsGateUpFunction(torch.autograd.Function):
         ctx.eps = eps
         ctx.saved_projection = bool(save_projection) and prepare_weight(weight).out_features % 8 == 0
         if ctx.saved_projection:
-            # the tiled kernel, as the fused call takes it (the streaming kernels for few rows have no
-            # SwiGLU epilogue and add the LoRA term in another order): the product is then bit-identical
+            # the kernels the fused call takes, so that the product is bit-identical: the streaming ones up to
+            # 32 rows, the tiled one beyond (a call without SwiGLU may run as 32-row chunks there)
+            rows = math.prod(x.shape[:-1])
             plan = ForwardPlan(x, weight, lora_a, lora_b, lora_scaling, adapter_indices=adapter_indices,
-                               rms_gamma=gamma, eps=eps, want_normalized=True, flags=_native.FLAG_FORCE_TILED)
+                               rms_gamma=gamma, eps=eps, want_normalized=True,
+                               flags=0 if rows <= SKINNY_MAX_ROWS else _native.FLAG_FORCE_TILED)
             fused = plan.run()
             ctx.save_for_backward(x, lora_a, lora_b, lora_scaling, gamma, fused, plan.aux["normalized"])
             return swiglu(fused)
