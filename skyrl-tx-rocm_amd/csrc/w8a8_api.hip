@@ -54,7 +54,7 @@ constexpr uint32_t kMaxN = 1u << 20;
 inline uint64_t align256(uint64_t v) { return (v + 255u) & ~uint64_t(255); }
 
 struct WsLayout {
-  uint64_t xq, sx, zp, at, bp, src_row, dst_pos, slot_group, blk_range, tile_ctr, skinny, total;
+  uint64_t xq, sx, zp, at, bp, row_scale, row_inv, src_row, dst_pos, slot_group, blk_range, tile_ctr, skinny, total;
   uint32_t slots, nkk, K_pad, KB, n_steps, steps_per_wave;
   uint32_t rows_bound;  // the slots that can hold rows (a multiple of 32)
 };
@@ -86,7 +86,7 @@ inline uint32_t padded_rows_bound(uint32_t m, uint32_t n_groups) {
 // the GEMM's tiles (512 resident tiles of 128 x 128, 256 of 256 x 256) need another round on the chip
 // than the packed layout does.
 inline bool padded_groups_fit(uint32_t m, uint32_t n, uint32_t n_groups, bool wide_tiles = false) {
-  if (n_groups < 2u || m > kInlineRouteMaxRows) return false;
+  if (n_groups < 2u || m > kPaddedRouteMaxRows) return false;
   const uint32_t rows = padded_rows_bound(m, n_groups), base = round_up(m, 32u);
   auto rounds = [](uint64_t items, uint64_t resident) { return (items + resident - 1u) / resident; };
   if (rounds(rows / 16u, 256u) != rounds(base / 16u, 256u)) return false;
@@ -116,6 +116,8 @@ WsLayout make_layout(uint32_t m, uint32_t k, uint32_t n, uint32_t n_groups, uint
   w.bp = off; off += rank ? align256((uint64_t)n_groups * (n_padded(n) / 32u) * w.nkk * kBlockBytes) : 0u;
   w.xq = off; off += align256((uint64_t)w.slots * w.K_pad);
   w.sx = off; off += align256((uint64_t)w.slots * 4u);
+  w.row_scale = off; off += align256((uint64_t)m * 4u);
+  w.row_inv = off; off += align256((uint64_t)m * 4u);
   w.src_row = off; off += align256((uint64_t)w.slots * 4u);
   w.dst_pos = off; off += align256((uint64_t)m * 4u);
   w.slot_group = off; off += align256((uint64_t)w.slots * 4u);
@@ -445,13 +447,8 @@ int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
 
   const bool skip_prologue = (p->flags & MI355_W8A8_FLAG_SKIP_PROLOGUE) != 0;
   const bool skip_gemm = (p->flags & MI355_W8A8_FLAG_SKIP_GEMM) != 0;
-  // Up to 8192 rows the quantizer's workgroups sort the adapter indices themselves (one launch less) --
-  // unless the launch that lays out the LoRA operands runs anyway (adapters that changed since the last
-  // call, as in every training step): then its first block sorts, beside the others, and the quantizer
-  // reads the tables (4-6 us less in each of its workgroups).
-  const bool pack_launch = lora && !skip_prologue && !(p->flags & MI355_W8A8_FLAG_LORA_PACK_VALID);
-  const bool route_inline = routed && p->m <= kInlineRouteMaxRows && !pack_launch;
-  if ((routed || lora) && !skip_prologue) {
+  // launch 1: adapter routing, the rows' statistics and (unless the workspace holds them) the LoRA operands
+  if (!skip_prologue) {
     LoraPrepArgs pa{};
     pa.idx = routed ? p->adapter_indices : nullptr;
     pa.src_row = src_row; pa.dst_pos = dst_pos; pa.slot_group = slot_group; pa.blk_range = blk_range;
@@ -461,25 +458,35 @@ int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
     pa.bp = ws + w.bp;
     pa.M = p->m; pa.K = p->k; pa.N = p->n; pa.n_groups = p->n_adapters; pa.r = p->rank; pa.nkk = w.nkk;
     pa.ncb = n_padded(p->n) / 32u; pa.slots = w.slots;
-    pa.route_blocks = (routed && !route_inline) ? 1u : 0u;
+    pa.route_blocks = routed ? 1u : 0u;
     pa.route_pad = pad_groups ? 32u : 1u;
     pa.a_operand_kb = w.KB;  // the quantizer reads A in MFMA operand order
-    const uint64_t a_items = (uint64_t)p->n_adapters * w.KB * w.nkk * 64u;
-    const uint64_t b_items = (uint64_t)p->n_adapters * pa.ncb * w.nkk * 64u;
-    const bool pack = !(p->flags & MI355_W8A8_FLAG_LORA_PACK_VALID);  // else the workspace holds both already
+    pa.stat_blocks = (p->m + 15u) / 16u;
+    pa.x = static_cast<const uint16_t*>(p->x);
+    pa.gamma = p->rms_gamma; pa.eps = p->rms_eps;
+    pa.row_scale = reinterpret_cast<float*>(ws + w.row_scale);
+    pa.row_inv = reinterpret_cast<float*>(ws + w.row_inv);
+    pa.scales_rm = p->aux_x_scales;
+    pa.xn_aux = static_cast<uint16_t*>(p->aux_normalized);
+    const uint64_t a_items = (uint64_t)p->n_adapters * w.KB * w.nkk * (p->rank % 4u ? 64u : 16u);
+    const uint64_t b_items = (uint64_t)p->n_adapters * pa.ncb * w.nkk * (p->n % 4u ? 64u : 16u);
+    const bool pack = lora && !(p->flags & MI355_W8A8_FLAG_LORA_PACK_VALID);
     pa.a_blocks = pack ? (uint32_t)((a_items + 1023u) / 1024u) : 0u;
     const uint32_t b_blocks = pack ? (uint32_t)((b_items + 1023u) / 1024u) : 0u;
-    if (pa.route_blocks + pa.a_blocks + b_blocks) {
-      hipLaunchKernelGGL(lora_prep_kernel, dim3(pa.route_blocks + pa.a_blocks + b_blocks), dim3(1024), 0, s, pa);
-      if ((st = launch_status())) return st;
-    }
+    const dim3 grid(pa.route_blocks + pa.stat_blocks + pa.a_blocks + b_blocks), block(1024);
+    if (rms) hipLaunchKernelGGL((lora_prep_kernel<2>), grid, block, 0, s, pa);
+    else hipLaunchKernelGGL((lora_prep_kernel<1>), grid, block, 0, s, pa);
+    if ((st = launch_status())) return st;
   }
 
-  // quantizer and LoRA-A projection: one pass over x
+  // launch 2: codes and LoRA-A projection
   QuantLoraArgs q{};
-  q.x = static_cast<const uint16_t*>(p->x);
+  // (normalized rows that the statistics launch has written for the caller are read as they are)
+  const bool normalize = rms && !p->aux_normalized;
+  q.x = static_cast<const uint16_t*>(rms && !normalize ? p->aux_normalized : p->x);
   q.gamma = p->rms_gamma;
-  q.eps = p->rms_eps;
+  q.row_scale = reinterpret_cast<const float*>(ws + w.row_scale);
+  q.row_inv = reinterpret_cast<const float*>(ws + w.row_inv);
   q.M = p->m; q.K = p->k; q.K_pad = w.K_pad; q.KB = w.KB;
   q.n_half_blocks = w.rows_bound / 16u;
   q.src_row = routed ? src_row : nullptr;
@@ -487,34 +494,17 @@ int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
   q.blk_range = routed ? blk_range : nullptr;
   q.xq_packed = ws + w.xq;
   q.sx_slots = reinterpret_cast<float*>(ws + w.sx);
-  q.codes_rm = p->aux_x_codes;
-  q.scales_rm = p->aux_x_scales;
-  q.xn_aux = static_cast<uint16_t*>(p->aux_normalized);
   q.at = lora ? reinterpret_cast<const uint16_t*>(ws + w.at) : nullptr;
   q.zp = ws + w.zp;
   q.r = p->rank; q.nkk = w.nkk;
   q.nterms = (p->flags & MI355_W8A8_FLAG_LORA_SPLIT2) ? 2u : 3u;
   q.tile_ctr = reinterpret_cast<uint32_t*>(ws + w.tile_ctr);
   q.group_pad = pad_groups ? 32u : 1u;
-  q.rows_per_wg = quant_lora_rows_per_wg(p->k);
-  q.row_stride = quant_lora_row_stride(p->k);
-  if (route_inline) {
-    q.route_idx = p->adapter_indices; q.n_groups = p->n_adapters; q.slots = w.slots;
-    q.src_row = src_row; q.slot_group = slot_group; q.blk_range = blk_range;
-  }
   if (!skip_prologue) {
-    const dim3 grid(q.n_half_blocks * (16u / q.rows_per_wg)), block(1024);
-    const uint32_t ql_lds = quant_lora_lds_bytes(p->k, lora ? w.nkk : 0u);
-#define W8A8_QL1(CB, RMS)                                                                                   \
-  {                                                                                                         \
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&quant_lora_kernel<CB, RMS>),                     \
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)ql_lds) != hipSuccess)         \
-      return MI355_W8A8_ERR_LAUNCH;                                                                         \
-    hipLaunchKernelGGL((quant_lora_kernel<CB, RMS>), grid, block, ql_lds, s, q);                            \
-  }
-#define W8A8_QL(CB)                \
-  if (rms) W8A8_QL1(CB, true)      \
-  else W8A8_QL1(CB, false)
+    const dim3 grid(q.n_half_blocks), block(1024);
+#define W8A8_QL(CB)                                                                              \
+  if (normalize) hipLaunchKernelGGL((quant_lora_kernel<CB, true>), grid, block, 0, s, q);        \
+  else hipLaunchKernelGGL((quant_lora_kernel<CB, false>), grid, block, 0, s, q)
     switch (lora ? w.nkk : 0u) {
       case 0: W8A8_QL(0); break;
       case 1: W8A8_QL(1); break;
@@ -522,8 +512,12 @@ int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
       default: W8A8_QL(4); break;
     }
 #undef W8A8_QL
-#undef W8A8_QL1
     if ((st = launch_status())) return st;
+    if (p->aux_x_codes) {
+      hipLaunchKernelGGL(codes_row_major_kernel, dim3(w.rows_bound), dim3(256), 0, s, q.xq_packed, q.src_row, p->aux_x_codes,
+                         p->m, p->k, w.KB);
+      if ((st = launch_status())) return st;
+    }
   } else if (!skip_gemm && path != MI355_W8A8_PATH_TILED_256X256) {
     // measurement calls: the tile counters of the 256 x 128 geometry's dynamic schedule still have to
     // start at zero (the 256 x 256 kernel has a static schedule and no counters)
@@ -681,11 +675,11 @@ int run_grouped(const mi355_w8a8_grouped_problem* p, hipStream_t s) {
     // launch then only lays out the slots)
     if (lora && !(p->flags & MI355_W8A8_FLAG_LORA_PACK_VALID)) {
       const uint64_t a_items = (uint64_t)p->n_groups * p->k * ((p->rank + 7u) / 8u);
-      const uint64_t b_items = (uint64_t)p->n_groups * pa.ncb * w.nkk * 64u;
+      const uint64_t b_items = (uint64_t)p->n_groups * pa.ncb * w.nkk * (p->n % 4u ? 64u : 16u);
       pa.a_blocks = (uint32_t)((a_items + 1023u) / 1024u);
       b_blocks = (uint32_t)((b_items + 1023u) / 1024u);
     }
-    hipLaunchKernelGGL(lora_prep_kernel, dim3(pa.route_blocks + pa.a_blocks + b_blocks), dim3(1024), 0, s, pa);
+    hipLaunchKernelGGL((lora_prep_kernel<0>), dim3(pa.route_blocks + pa.a_blocks + b_blocks), dim3(1024), 0, s, pa);
     if ((st = launch_status())) return st;
   }
 
@@ -1741,7 +1735,7 @@ int run_gq_linear(const mi355_w8a8_gq_problem* p, hipStream_t s) {
     pa.a_operand_steps = (p->k + 63u) / 64u; pa.a_operand_rb = rank_chunks(p->rank) > 2u ? 2u : 1u;  // lora_a_kernel's operand order
     const uint64_t a_items = (uint64_t)p->n_adapters * pa.a_operand_steps * pa.a_operand_rb * 256u;
     pa.a_blocks = (uint32_t)((a_items + 1023u) / 1024u);
-    hipLaunchKernelGGL(lora_prep_kernel, dim3(pa.route_blocks + pa.a_blocks), dim3(1024), 0, s, pa);
+    hipLaunchKernelGGL((lora_prep_kernel<0>), dim3(pa.route_blocks + pa.a_blocks), dim3(1024), 0, s, pa);
     if ((st = launch_status())) return st;
     LoraAArgs la{};
     la.xsrc = q.x;

@@ -197,12 +197,19 @@ __device__ inline void lora_a_operand_item(const uint16_t* __restrict__ a, unsig
   const uint64_t gc = rest / nkk;
   const uint32_t kb = (uint32_t)(gc % kb32), grp = (uint32_t)(gc / kb32);
   const uint32_t k = kb * 32u + (l & 31u);
-  v8us o = {0, 0, 0, 0, 0, 0, 0, 0};
-  if (k < K) {
+  v8us o;
+  const uint32_t row0 = 16u * kk + 8u * (l >> 5);
+  if ((r & 7u) == 0) {  // kernel-uniform: one 16-byte load (unconditional, like the ones below: a load under a lane
+    const bool in = k < K && row0 < r;  // condition becomes a branch with a wait of its own)
+    const v8us zero = {0, 0, 0, 0, 0, 0, 0, 0};
+    const v8us v = *reinterpret_cast<const v8us*>(a + (in ? ((size_t)grp * K + k) * r + row0 : 0u));
+    o = in ? v : zero;
+  } else {
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      const uint32_t row = 16u * kk + 8u * (l >> 5) + e;
-      if (row < r) o[e] = a[((size_t)grp * K + k) * r + row];
+      const bool in = k < K && row0 + e < r;
+      const uint16_t v = a[in ? ((size_t)grp * K + k) * r + row0 + e : 0u];
+      o[e] = in ? v : (uint16_t)0;
     }
   }
   *reinterpret_cast<v8us*>(ap + idx * 16u) = o;
@@ -222,7 +229,7 @@ __global__ __launch_bounds__(1024) void bwd_prep_kernel(BwdPrepArgs p) {
   uint32_t b = blockIdx.x;
   if (b < p.route_blocks) {
     if (p.idx) {
-      route_rows_block(p.idx, p.M, p.n_groups, p.slots, p.src_row, p.dst_pos, p.slot_group, p.blk_range, p.group_off, true);
+      route_rows_block(p.idx, p.M, p.n_groups, p.slots, p.src_row, p.dst_pos, p.slot_group, p.blk_range, p.group_off);
     } else {  // one adapter for every row: identity order, everything in group 0
       for (uint32_t g = threadIdx.x; g <= p.n_groups; g += 1024u) p.group_off[g] = g == 0 ? 0 : (int)p.M;
     }

@@ -1,6 +1,8 @@
 // Prologue kernels: weight (un)packing, adapter routing, per-token quantization with the
 // optional fused RMSNorm, and the LoRA-A projection z = n @ A[adapter].
 #pragma once
+#include <type_traits>
+
 #include "w8a8_device.h"
 
 namespace w8a8 {
@@ -51,100 +53,105 @@ __global__ __launch_bounds__(256) void unpack_weight_kernel(const unsigned char*
 //   blk_range[b]  = first adapter | last adapter << 16 of the 32-row block b
 //   group_off[a]  = first grouped slot of adapter a (optional; entry n_groups = M)
 // Out-of-range adapter indices are clamped into range (XLA gather semantics).
-// One workgroup.  The order of rows inside a group does not influence any forward result; the
-// backward asks for the stable order because it sums over a group's rows.
 // ---------------------------------------------------------------------------------------
-// With group_pad = 32 every group starts on a 32-slot boundary (see route_rows_inline): the slots between
+// With group_pad = 32 every group starts on a 32-slot boundary, so that no 32-slot block holds rows of two
+// groups (neither the quantizer nor the GEMM's epilogue then runs a block once per group): the slots between
 // a group's last row and the next group's first stay empty.
+// One workgroup of sixteen waves, each with a contiguous range of the rows: a wave counts its rows per group
+// (lanes with the same group find each other with one ballot per bit of the index, so a group costs a wave one
+// LDS atomic per 64 rows), wave 0 turns the counts into first slots, and the waves place their rows in order.
+// Rows so keep their order inside a group: reductions over a group's rows have a fixed order.  Bound by the
+// latency of its few steps: 14 us for
+// 4096 rows with an atomic per row and a search per slot.
 __device__ inline void route_rows_block(const int32_t* __restrict__ idx, uint32_t M, uint32_t n_groups,
                                         uint32_t slots, int32_t* __restrict__ src_row,
                                         int32_t* __restrict__ dst_pos, int32_t* __restrict__ slot_group,
                                         int32_t* __restrict__ blk_range, int32_t* __restrict__ group_off = nullptr,
-                                        bool stable = false, uint32_t group_pad = 1u) {
+                                        uint32_t group_pad = 1u) {
+  static_assert(kMaxAdapters == 64, "a lane per group");
+  __shared__ int wcnt[16][kMaxAdapters];  // rows of group g in wave w; then the wave's next slot in the group
   __shared__ int cnt[kMaxAdapters];
   __shared__ int start[kMaxAdapters + 1];
-  __shared__ int cursor[kMaxAdapters];
-  const uint32_t tid = threadIdx.x;
-  if (tid < kMaxAdapters) { cnt[tid] = 0; cursor[tid] = 0; }
-  __syncthreads();
-  for (uint32_t i = tid; i < M; i += 1024) {
-    int a = idx[i];
-    a = a < 0 ? 0 : (a >= (int)n_groups ? (int)n_groups - 1 : a);
-    atomicAdd(&cnt[a], 1);
-  }
-  __syncthreads();
-  if (tid == 0) {
-    int pos = 0;
-    for (uint32_t a = 0; a < n_groups; ++a) {
-      start[a] = pos;
-      pos += (int)round_up((uint32_t)cnt[a], group_pad);
+  __shared__ int last_group;
+  const uint32_t tid = threadIdx.x, lane = tid & 63u;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t per = (M + 1024u - 1u) / (1024u);  // 64-row steps of a wave
+  auto group_at = [&](uint32_t it) -> int {
+    const uint32_t i = (wave * per + it) * 64u + lane;
+    const int a = idx[i < M ? i : M - 1u];
+    return i < M ? (a < 0 ? 0 : (a >= (int)n_groups ? (int)n_groups - 1 : a)) : -1;
+  };
+  auto peers_of = [&](int a) -> unsigned long long {  // lanes with this lane's group
+    unsigned long long mask = __builtin_amdgcn_ballot_w64(a >= 0);
+#pragma unroll
+    for (int bit = 0; bit < 6; ++bit) {
+      const unsigned long long set = __builtin_amdgcn_ballot_w64((a >> bit) & 1);
+      mask &= ((a >> bit) & 1) ? set : ~set;
     }
-    start[n_groups] = pos;
+    return mask;
+  };
+  wcnt[wave][lane] = 0;
+  auto count = [&](int a) {
+    const unsigned long long peers = peers_of(a);
+    if (a >= 0 && (int)lane == __builtin_ctzll(peers)) atomicAdd(&wcnt[wave][a], __builtin_popcountll(peers));
+  };
+#pragma unroll 4
+  for (uint32_t it = 0; it < per; ++it) count(group_at(it));
+  __syncthreads();
+  if (wave == 0) {  // lane g: group g
+    int total = 0;
+#pragma unroll
+    for (uint32_t w = 0; w < 16; ++w) total += wcnt[w][lane];  // (groups that do not exist: zeros)
+    const int padded = (int)round_up((uint32_t)total, group_pad);
+    int incl = padded;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int up = __shfl_up(incl, off, 64);
+      if ((int)lane >= off) incl += up;
+    }
+    int pos = incl - padded;
+    cnt[lane] = total;
+    start[lane] = pos;  // (groups that do not exist: empty, behind the last one)
+    if (lane == 63u) start[64] = incl;
+#pragma unroll
+    for (uint32_t w = 0; w < 16; ++w) {
+      const int c = wcnt[w][lane];
+      wcnt[w][lane] = pos;
+      pos += c;
+    }
+    const unsigned long long nonempty = __builtin_amdgcn_ballot_w64(total > 0);
+    if (lane == 0) last_group = nonempty ? 63 - __builtin_clzll(nonempty) : 0;
   }
   __syncthreads();
   const uint32_t E = (uint32_t)start[n_groups];  // first slot behind the last group (M when the groups are packed)
-  if (group_pad > 1u)
-    for (uint32_t p = tid; p < E && p < slots; p += 1024) src_row[p] = -1;  // the empty slots between groups
-  __syncthreads();
-  if (group_off && tid <= n_groups) group_off[tid] = start[tid];  // first slot of every group, then M
-  if (stable) {
-    // rows keep their order inside a group (reductions over a group's rows then have a fixed order):
-    // rank = rows of the same group before this one, counted per wave with ballots, per 1024-row
-    // chunk with the waves' counts, and across chunks with the running count in cursor[]
-    __shared__ int wave_cnt[16][kMaxAdapters];
-    const uint32_t lane = tid & 63u, wave = tid >> 6;
-    for (uint32_t base = 0; base < M; base += 1024) {
-      const uint32_t i = base + tid;
-      int a = -1;
-      if (i < M) {
-        a = idx[i];
-        a = a < 0 ? 0 : (a >= (int)n_groups ? (int)n_groups - 1 : a);
-      }
-      int rank = 0;
-      for (uint32_t g = 0; g < n_groups; ++g) {
-        const unsigned long long mask = __builtin_amdgcn_ballot_w64(a == (int)g);
-        if (a == (int)g) rank = __builtin_popcountll(mask & ((1ull << lane) - 1ull));
-        if (lane == 0) wave_cnt[wave][g] = __builtin_popcountll(mask);
-      }
-      __syncthreads();
-      if (a >= 0) {
-        int off = cursor[a];
-        for (uint32_t w = 0; w < wave; ++w) off += wave_cnt[w][a];
-        const int p = start[a] + off + rank;
-        src_row[p] = (int)i;
-        dst_pos[i] = p;
-      }
-      __syncthreads();
-      if (tid < n_groups) {
-        int t = 0;
-        for (uint32_t w = 0; w < 16; ++w) t += wave_cnt[w][tid];
-        cursor[tid] += t;
-      }
-      __syncthreads();
-    }
-  } else {
-    for (uint32_t i = tid; i < M; i += 1024) {
-      int a = idx[i];
-      a = a < 0 ? 0 : (a >= (int)n_groups ? (int)n_groups - 1 : a);
-      const int p = start[a] + atomicAdd(&cursor[a], 1);
-      src_row[p] = (int)i;
+  auto place = [&](int a, uint32_t it) {
+    const unsigned long long peers = peers_of(a);
+    const int leader = peers ? __builtin_ctzll(peers) : 0;
+    int p = 0;
+    if (a >= 0 && (int)lane == leader) p = atomicAdd(&wcnt[wave][a], __builtin_popcountll(peers));
+    p = __builtin_amdgcn_ds_bpermute(4 * leader, p) + __builtin_popcountll(peers & ((1ull << lane) - 1ull));
+    if (a >= 0) {
+      const int i = (int)((wave * per + it) * 64u + lane);
+      src_row[p] = i;
       dst_pos[i] = p;
+      slot_group[p] = a;
     }
+  };
+#pragma unroll 4
+  for (uint32_t it = 0; it < per; ++it) place(group_at(it), it);
+  if (group_off && tid <= n_groups) group_off[tid] = start[tid];  // first slot of every group, then E
+  if (group_pad > 1u) {  // the empty slots between groups (fewer than group_pad <= 32 behind each)
+    for (uint32_t t = tid; t < n_groups * 32u; t += 1024u) {
+      const uint32_t g = t >> 5, p = (uint32_t)(start[g] + cnt[g]) + (t & 31u);
+      if (p < (uint32_t)start[g + 1u] && p < slots) { src_row[p] = -1; slot_group[p] = (int)g; }
+    }
+  }
+  for (uint32_t p = E + tid; p < slots; p += 1024u) {  // padding slots follow the last non-empty group
+    src_row[p] = -1;
+    slot_group[p] = last_group;
   }
   // group of a slot = the group whose [start, next start) range holds it
-  for (uint32_t p = tid; p < slots; p += 1024) {
-    int g = 0;
-    if (p < E) {
-      for (uint32_t a = 0; a < n_groups; ++a)
-        if ((int)p >= start[a] && (int)p < start[a + 1]) g = (int)a;
-    } else {
-      src_row[p] = -1;
-      for (uint32_t a = 0; a < n_groups; ++a)
-        if (cnt[a] > 0) g = (int)a;  // padding slots follow the last non-empty group
-    }
-    slot_group[p] = g;
-  }
-  for (uint32_t b = tid; b < slots / 32u; b += 1024) {
+  for (uint32_t b = tid; b < slots / 32u; b += 1024u) {
     const int p0 = (int)b * 32, p1 = (p0 + 31 < (int)E) ? p0 + 31 : (int)E - 1;
     int g0 = 0, g1 = 0;
     for (uint32_t a = 0; a < n_groups; ++a) {
@@ -440,16 +447,46 @@ __device__ inline void lora_b_pack_item(const uint16_t* __restrict__ b, unsigned
   const uint64_t gc = rest / nkk;
   const uint32_t cb = (uint32_t)(gc % ncb), grp = (uint32_t)(gc / ncb);
   const uint32_t col = packed_to_orig_col(cb * 32u + (l & 31u));
-  v8us o = {0, 0, 0, 0, 0, 0, 0, 0};
-  if (col < N) {
+  v8us o;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const uint32_t row = 16u * kk + 8u * (l >> 5) + e;
-      if (row < r) o[e] = b[((size_t)grp * r + row) * N + col];
-    }
+  for (int e = 0; e < 8; ++e) {
+    const uint32_t row = 16u * kk + 8u * (l >> 5) + e;
+    const bool in = col < N && row < r;
+    const uint16_t v = b[in ? ((size_t)grp * r + row) * N + col : 0u];
+    o[e] = in ? v : (uint16_t)0;
   }
   *reinterpret_cast<v8us*>(bp + idx * 16u) = o;
 }
+// Four operands per thread where a row's columns come in aligned fours (N % 4 == 0): the lane's column of each
+// of a group's four column blocks, four adjacent columns of B, so a quarter of the loads.  The packing is
+// bound by the loads it issues: 8 adapters of rank 32 at 4096 -> 24576 take 6 us where one two-byte load per
+// value takes 20.
+__device__ inline void lora_b_pack4_item(const uint16_t* __restrict__ b, unsigned char* __restrict__ bp,
+                                         uint32_t n_groups, uint32_t r, uint32_t N, uint32_t ncb, uint32_t nkk,
+                                         uint64_t idx) {
+  const uint64_t total = (uint64_t)n_groups * (ncb / 4u) * nkk * 64u;
+  if (idx >= total) return;
+  const uint32_t l = (uint32_t)(idx & 63u);
+  const uint64_t rest = idx >> 6;
+  const uint32_t kk = (uint32_t)(rest % nkk);
+  const uint64_t gc = rest / nkk;
+  const uint32_t G = (uint32_t)(gc % (ncb / 4u)), grp = (uint32_t)(gc / (ncb / 4u));
+  const uint32_t col = 128u * G + 4u * (l & 31u), row0 = 16u * kk + 8u * (l >> 5);
+  v8us o[4];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const bool in = col < N && row0 + e < r;
+    // (loaded whatever the condition: a load under a lane condition becomes a branch with a wait of its own)
+    const uint2 v = *reinterpret_cast<const uint2*>(b + (in ? ((size_t)grp * r + row0 + e) * N + col : 0u));
+    const uint32_t vx = in ? v.x : 0u, vy = in ? v.y : 0u;
+    o[0][e] = (uint16_t)vx; o[1][e] = (uint16_t)(vx >> 16);
+    o[2][e] = (uint16_t)vy; o[3][e] = (uint16_t)(vy >> 16);
+  }
+#pragma unroll
+  for (uint32_t j = 0; j < 4; ++j)
+    *reinterpret_cast<v8us*>(bp + ((((size_t)grp * ncb + 4u * G + j) * nkk + kk) * 64u + l) * 16u) = o[j];
+}
+
 
 // ---------------------------------------------------------------------------------------
 // LoRA A re-layout for the dense path's quantizer: A [n, K, r] -> the B-operand order of
@@ -470,15 +507,41 @@ __device__ inline void lora_a_pack_item(const uint16_t* __restrict__ a, unsigned
   const uint64_t gk = rest / nkk;
   const uint32_t kb = (uint32_t)(gk % KB), grp = (uint32_t)(gk / KB);
   const uint32_t col = 16u * b + (l & 15u);
-  v8us o = {0, 0, 0, 0, 0, 0, 0, 0};
-  if (col < r) {
+  v8us o;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const uint32_t k = 32u * kb + 8u * (l >> 4) + e;
-      if (k < K) o[e] = a[((size_t)grp * K + k) * r + col];
-    }
+  for (int e = 0; e < 8; ++e) {
+    const uint32_t k = 32u * kb + 8u * (l >> 4) + e;
+    const bool in = col < r && k < K;
+    const uint16_t v = a[in ? ((size_t)grp * K + k) * r + col : 0u];
+    o[e] = in ? v : (uint16_t)0;
   }
   *reinterpret_cast<v8us*>(ap + idx * 16u) = o;
+}
+
+// Four operands per thread (r % 4 == 0): four adjacent rank columns of the same eight k.
+__device__ inline void lora_a_pack4_item(const uint16_t* __restrict__ a, unsigned char* __restrict__ ap,
+                                         uint32_t n_groups, uint32_t K, uint32_t r, uint32_t KB, uint32_t nkk,
+                                         uint64_t idx) {
+  const uint64_t total = (uint64_t)n_groups * KB * nkk * 16u;
+  if (idx >= total) return;
+  const uint32_t i4 = (uint32_t)(idx & 3u), q = (uint32_t)(idx >> 2) & 3u;
+  const uint64_t rest = idx >> 4;
+  const uint32_t b = (uint32_t)(rest % nkk);
+  const uint64_t gk = rest / nkk;
+  const uint32_t kb = (uint32_t)(gk % KB), grp = (uint32_t)(gk / KB);
+  const uint32_t col = 16u * b + 4u * i4, k0 = 32u * kb + 8u * q;
+  v8us o[4];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const bool in = col < r && k0 + e < K;
+    const uint2 v = *reinterpret_cast<const uint2*>(a + (in ? ((size_t)grp * K + k0 + e) * r + col : 0u));
+    const uint32_t vx = in ? v.x : 0u, vy = in ? v.y : 0u;
+    o[0][e] = (uint16_t)vx; o[1][e] = (uint16_t)(vx >> 16);
+    o[2][e] = (uint16_t)vy; o[3][e] = (uint16_t)(vy >> 16);
+  }
+  v8us* dst = reinterpret_cast<v8us*>(ap) + (rest * 64u + 16u * q + 4u * i4);
+#pragma unroll
+  for (uint32_t j = 0; j < 4; ++j) dst[j] = o[j];
 }
 
 // The same for lora_a_kernel (v_mfma_f32_32x32x16_bf16, 64-wide k steps), whose operand loads of the
@@ -497,13 +560,13 @@ __device__ inline void lora_a_pack32_item(const uint16_t* __restrict__ a, unsign
   const uint64_t gs = rest / rb;
   const uint32_t st = (uint32_t)(gs % n_steps), grp = (uint32_t)(gs / n_steps);
   const uint32_t col = 32u * b + (l & 31u);
-  v8us o = {0, 0, 0, 0, 0, 0, 0, 0};
-  if (col < r) {
+  v8us o;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const uint32_t k = 64u * st + 32u * (l >> 5) + 8u * t + e;
-      if (k < K) o[e] = a[((size_t)grp * K + k) * r + col];
-    }
+  for (int e = 0; e < 8; ++e) {
+    const uint32_t k = 64u * st + 32u * (l >> 5) + 8u * t + e;
+    const bool in = col < r && k < K;
+    const uint16_t v = a[in ? ((size_t)grp * K + k) * r + col : 0u];
+    o[e] = in ? v : (uint16_t)0;
   }
   *reinterpret_cast<v8us*>(ap + idx * 16u) = o;
 }
@@ -514,8 +577,9 @@ __global__ __launch_bounds__(256) void zero_words_kernel(uint32_t* p, uint32_t c
 }
 
 // ---------------------------------------------------------------------------------------
-// One launch for the three independent preparation jobs of a call: adapter routing (block 0
-// when `idx` is given), LoRA A transposition and LoRA B operand packing (the other blocks).
+// One launch for the independent preparation jobs of a call: adapter routing (block 0
+// when `idx` is given), the rows' statistics (dense calls), LoRA A transposition and LoRA B operand packing
+// (the other blocks).
 // ---------------------------------------------------------------------------------------
 struct LoraPrepArgs {
   const int32_t* idx;        // adapter per row, or null (no routing block)
@@ -533,24 +597,152 @@ struct LoraPrepArgs {
   uint32_t group_pad;          // slots every group is padded to
   uint16_t* zero_out;          // bf16 [M, zero_cols]: rows beyond the groups are cleared, or null
   uint32_t zero_cols;
+  // row statistics of the dense call (STATS != 0): sixteen rows per block, behind the routing block
+  uint32_t stat_blocks;
+  const uint16_t* x;           // bf16 [M, K]
+  const float* gamma;          // f32 [K] (STATS == 2)
+  float eps;
+  float* row_scale;            // f32 [M]: absmax / 127 of the (normalized) row, 1 where that is not positive
+  float* row_inv;              // f32 [M]: 1 / sqrt(mean square + eps) (STATS == 2)
+  float* scales_rm;            // f32 [M] for the caller, or null
+  uint16_t* xn_aux;            // bf16 [M, K] normalized rows for the caller, or null (STATS == 2)
 };
 
-__global__ __launch_bounds__(1024) void lora_prep_kernel(LoraPrepArgs p) {
+// Largest |value| of eight bf16 values against a running maximum of pairs: |bf16| compares like its 15
+// magnitude bits as an integer (a NaN ends above every number and the scale then falls back to 1, as the
+// reference's comparison amax > 0 does).
+__device__ inline uint32_t bf16_absmax_pairs(uint32_t amax_bits, const uint4& raw) {
+  typedef unsigned short us2 __attribute__((ext_vector_type(2)));
+  us2 mx = __builtin_bit_cast(us2, amax_bits);
+  mx = __builtin_elementwise_max(mx, __builtin_bit_cast(us2, raw.x & 0x7fff7fffu));
+  mx = __builtin_elementwise_max(mx, __builtin_bit_cast(us2, raw.y & 0x7fff7fffu));
+  mx = __builtin_elementwise_max(mx, __builtin_bit_cast(us2, raw.z & 0x7fff7fffu));
+  mx = __builtin_elementwise_max(mx, __builtin_bit_cast(us2, raw.w & 0x7fff7fffu));
+  return __builtin_bit_cast(uint32_t, mx);
+}
+// (x * inv) * gamma, one bf16 rounding, of eight values
+__device__ inline uint4 rms_normalize8(const uint4& raw, float inv, const float4& g0, const float4& g1) {
+  const float g[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
+  uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    float t0 = __uint_as_float(w[e] << 16) * inv, t1 = __uint_as_float(w[e] & 0xffff0000u) * inv;
+    t0 = t0 * g[2 * e];
+    t1 = t1 * g[2 * e + 1];
+    w[e] = pack_bf16x2(t0, t1);
+  }
+  return make_uint4(w[0], w[1], w[2], w[3]);
+}
+
+// Statistics of row m by one wave: kPieces 1 KiB pieces of the row in flight at a time.  With RMSNorm the row
+// is read a second time for the normalized maximum (from the L2: its wave has just read it); holding it took
+// registers that cost the launch its second workgroup per CU.
+template <bool RMS>
+__device__ inline void row_stats(const LoraPrepArgs& p, uint32_t m) {
+  constexpr uint32_t kPieces = RMS ? 4 : 8;
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t row_bytes = 2u * p.K;
+  // (the row and the norm weights through buffer resources that end with them: a load under a lane condition
+  // becomes a branch with a wait of its own, and the loads then run one after the other)
+  const __amdgpu_buffer_rsrc_t xrsrc =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p.x) + (size_t)m * p.K, 0, (int)row_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t grsrc =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.gamma), 0, RMS ? (int)(p.K * 4u) : 0, 0x00020000);
+  uint32_t amax_bits = 0;
+  uint4 r[kPieces];
+  auto fetch = [&](uint32_t base) {
+#pragma unroll
+    for (uint32_t j = 0; j < kPieces; ++j)
+      r[j] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(xrsrc, base + j * 1024u + lane * 16u, 0, 0));
+  };
+  if constexpr (!RMS) {
+#pragma unroll 1
+    for (uint32_t base = 0; base < row_bytes; base += kPieces * 1024u) {
+      fetch(base);
+#pragma unroll
+      for (uint32_t j = 0; j < kPieces; ++j) amax_bits = bf16_absmax_pairs(amax_bits, r[j]);
+    }
+  } else {
+    double ss = 0.0;
+#pragma unroll 1
+    for (uint32_t base = 0; base < row_bytes; base += kPieces * 1024u) {
+      fetch(base);
+#pragma unroll
+      for (uint32_t j = 0; j < kPieces; ++j) {
+        const uint32_t w[4] = {r[j].x, r[j].y, r[j].z, r[j].w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          // the square of a bf16 value is exact in double, so the fused form rounds like mul + add
+          const double lo = (double)__uint_as_float(w[e] << 16), hi = (double)__uint_as_float(w[e] & 0xffff0000u);
+          ss = __builtin_fma(lo, lo, ss);
+          ss = __builtin_fma(hi, hi, ss);
+        }
+      }
+    }
+    ss = wave_sum(ss);
+    const float var = (float)(ss / (double)p.K);
+    const float inv = 1.0f / sqrtf(var + p.eps);
+    if (lane == 0) p.row_inv[m] = inv;
+#pragma unroll 1
+    for (uint32_t base = 0; base < row_bytes; base += kPieces * 1024u) {
+      fetch(base);
+#pragma unroll
+      for (uint32_t j = 0; j < kPieces; ++j) {
+        const uint32_t off = base + j * 1024u + lane * 16u;
+        if ((j & 1u) == 0) __builtin_amdgcn_sched_barrier(0);  // (norm weights of two pieces at a time: registers)
+        const float4 g0 = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(grsrc, 2u * off, 0, 0));
+        const float4 g1 = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(grsrc, 2u * off + 16u, 0, 0));
+        const uint4 n = rms_normalize8(r[j], inv, g0, g1);  // (zeros beyond the row)
+        if (p.xn_aux && off < row_bytes) *reinterpret_cast<uint4*>(reinterpret_cast<unsigned char*>(p.xn_aux) + (size_t)m * row_bytes + off) = n;
+        amax_bits = bf16_absmax_pairs(amax_bits, n);
+      }
+    }
+  }
+  uint32_t top = (amax_bits >> 16) > (amax_bits & 0xffffu) ? (amax_bits >> 16) : (amax_bits & 0xffffu);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    const uint32_t other = (uint32_t)__shfl_xor((int)top, o, 64);
+    top = other > top ? other : top;
+  }
+  const float amax = __uint_as_float(top << 16);
+  const float scale = amax > 0.0f ? amax / 127.0f : 1.0f;
+  if (lane == 0) {
+    p.row_scale[m] = scale;
+    if (p.scales_rm) p.scales_rm[m] = scale;
+  }
+}
+
+// (Two workgroups per CU: 4096 rows are 256 blocks of statistics, and the routing block beside them must not
+// put one of them into a second round.)
+template <int STATS>  // 0: no row statistics, 1: of x, 2: of the normalized rows
+__global__ __launch_bounds__(1024, 8) void lora_prep_kernel(LoraPrepArgs p) {
   uint32_t b = blockIdx.x;
   if (b < p.route_blocks) {
+    __builtin_amdgcn_s_setprio(3);  // a chain of short steps beside waves that wait for memory
     if (p.group_sizes)
       route_groups_block(p.group_sizes, p.M, p.n_groups, p.slots, p.src_row, p.dst_pos, p.blk_range, p.group_pad,
                          p.zero_out, p.zero_cols, b, p.route_blocks);
     else
-      route_rows_block(p.idx, p.M, p.n_groups, p.slots, p.src_row, p.dst_pos, p.slot_group, p.blk_range, nullptr, false,
+      route_rows_block(p.idx, p.M, p.n_groups, p.slots, p.src_row, p.dst_pos, p.slot_group, p.blk_range, nullptr,
                        p.route_pad > 1u ? p.route_pad : 1u);
     return;
   }
   b -= p.route_blocks;
+  if constexpr (STATS != 0) {
+    if (b < p.stat_blocks) {
+      const uint32_t m = b * 16u + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+      if (m < p.M) row_stats<STATS == 2>(p, m);
+      return;
+    }
+    b -= p.stat_blocks;
+  }
   if (b < p.a_blocks) {
     if (p.a_operand_steps)
       lora_a_pack32_item(p.lora_a, reinterpret_cast<unsigned char*>(p.at), p.n_groups, p.K, p.r, p.a_operand_steps,
                          p.a_operand_rb, (uint64_t)b * 1024u + threadIdx.x);
+    else if (p.a_operand_kb && (p.r & 3u) == 0)
+      lora_a_pack4_item(p.lora_a, reinterpret_cast<unsigned char*>(p.at), p.n_groups, p.K, p.r, p.a_operand_kb, p.nkk,
+                        (uint64_t)b * 1024u + threadIdx.x);
     else if (p.a_operand_kb)
       lora_a_pack_item(p.lora_a, reinterpret_cast<unsigned char*>(p.at), p.n_groups, p.K, p.r, p.a_operand_kb, p.nkk,
                        (uint64_t)b * 1024u + threadIdx.x);
@@ -559,7 +751,10 @@ __global__ __launch_bounds__(1024) void lora_prep_kernel(LoraPrepArgs p) {
     return;
   }
   b -= p.a_blocks;
-  lora_b_pack_item(p.lora_b, p.bp, p.n_groups, p.r, p.N, p.ncb, p.nkk, (uint64_t)b * 1024u + threadIdx.x);
+  if ((p.N & 3u) == 0)
+    lora_b_pack4_item(p.lora_b, p.bp, p.n_groups, p.r, p.N, p.ncb, p.nkk, (uint64_t)b * 1024u + threadIdx.x);
+  else
+    lora_b_pack_item(p.lora_b, p.bp, p.n_groups, p.r, p.N, p.ncb, p.nkk, (uint64_t)b * 1024u + threadIdx.x);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -794,376 +989,123 @@ __global__ __launch_bounds__(1024) void lora_a_kernel(LoraAArgs a) {
 }
 
 // ---------------------------------------------------------------------------------------
-// Quantizer and LoRA-A projection in one pass over x (the dense path's prologue).
-// One workgroup of 16 waves per R grouped slots (R = 16, or 8 / 4 / 2 when longer rows would not fit the
-// LDS: half a 32-row block or a part of one):
-//   1. wave w < R copies slot row w from memory into the LDS with direct-to-LDS loads -- the only
-//      time x is read -- and takes its statistics from there: (RMSNorm sum of squares, the row normalized
-//      in place,) absmax -> scale;
-//   2. the waves split K in 32-wide blocks; lane (i = lane % 16, q = lane / 16) takes the 8 (normalized)
-//      values k = 32 kb + 8 q .. +7 of row i from the LDS and uses them twice: as int8 codes written into
-//      the activation's 1 KiB fragment block, and as the A operand of v_mfma_f32_16x16x32_bf16 against the
-//      LoRA A of the row's group in that instruction's operand order, so the normalized rows never travel
-//      through memory;
-//   3. the waves' z tiles are added in a fixed order, split exactly into three bf16 terms and
-//      stored in the operand order the GEMM epilogue reads (see lora_a_kernel).
+// Codes and LoRA-A projection of the dense path's prologue, behind the launch that took the rows'
+// statistics (row_stats, beside the routing and the LoRA operand layouts).
+// One workgroup of 16 waves per half of a 32-slot block: the waves split K in 32-wide blocks; lane
+// (i = lane % 16, q = lane / 16) takes the 8 (normalized) values k = 32 kb + 8 q .. +7 of slot row i and
+// uses them twice: as int8 codes written into the activation's 1 KiB fragment block, and as the A operand
+// of v_mfma_f32_16x16x32_bf16 against the LoRA A of the row's group in that instruction's operand order.
+// The waves' z tiles are added in a fixed order, split exactly into three bf16 terms and stored in the
+// operand order the GEMM epilogue reads (see lora_a_kernel).
 // Arithmetic follows quant_rows_kernel (skyrl/tx/kernels/quantized_lora.py:199-212 and the
 // RMSNorm of bf16_rms_gate_up_lora_swiglu.py:299-303) operation for operation.
+// Bound by memory for long rows and by latency for few of them.  Splitting the statistics off reads x twice,
+// the second time largely from the caches, and in return nothing has to be held: rows that had to wait in the
+// LDS for their scale gave a workgroup 16 of them only up to K = 4608 and four at K = 12288, where every
+// workgroup fetched the whole LoRA A for four rows.  Measured: 4096 x 12288, 8 adapters of rank 32: 22 us
+// (statistics, routing, operand layouts) + 54 us against 14 us (layouts, routing) + 120 us; 333 x 4096, 4 adapters
+// of rank 64: 7 + 16 us against 6 + 20 us; 4096 x 4096 with RMSNorm, where sixteen rows did fit the LDS:
+// 20 + 28 us against 14 + 32 us.
 // ---------------------------------------------------------------------------------------
 struct QuantLoraArgs {
-  const uint16_t* x;        // bf16 [M, K]
+  const uint16_t* x;        // bf16 [M, K]: the rows, or (RMS false) rows that are normalized already
   const float* gamma;       // f32 [K] (RMS only)
-  float eps;
-  uint32_t M, K, K_pad, KB, n_half_blocks;  // n_half_blocks = ceil(M / 16)
+  const float* row_scale;   // f32 [M] from row_stats
+  const float* row_inv;     // f32 [M] from row_stats (RMS only)
+  uint32_t M, K, K_pad, KB, n_half_blocks;  // n_half_blocks = ceil(slots that can hold rows / 16)
   const int32_t* src_row;   // original row of a slot, or null (identity)
   const int32_t* slot_group;// or null
   const int32_t* blk_range; // per 32-slot block, or null (group 0)
   unsigned char* xq_packed; // packed codes [slots/32][KB][1 KiB]
   float* sx_slots;          // f32 [slots]
-  int8_t* codes_rm;         // row-major codes [M, K] or null
-  float* scales_rm;         // f32 [M] or null
-  uint16_t* xn_aux;         // bf16 [M, K] normalized rows for the caller, or null
   const uint16_t* at;       // LoRA A in MFMA operand order [n_groups][KB][CB][64 lanes][8 bf16] (lora_a_pack_item) or null (CB == 0)
   unsigned char* zp;        // packed z fragments
   uint32_t r, nkk, nterms;
   uint32_t* tile_ctr;       // 256 words cleared for the GEMM launches' tile counters, or null
-  // Routing inside this launch (route_idx != null; M <= kInlineRouteMaxRows): every workgroup sorts the
-  // adapter indices for itself and WRITES its slots' entries of src_row / slot_group / blk_range
-  // (then non-const outputs, read later by the GEMM) instead of reading them.
-  const int32_t* route_idx; // adapter per row
-  uint32_t n_groups, slots;
-  uint32_t group_pad;       // every group's first slot is a multiple of this (1: groups packed; 32: no block holds two groups)
-  uint32_t rows_per_wg;     // R: 16, 8, 4 or 2 slots per workgroup (quant_lora_rows_per_wg)
-  uint32_t row_stride;      // bytes between two rows in the LDS (quant_lora_row_stride)
+  uint32_t group_pad;       // > 1: whole half blocks may be empty
 };
 
-constexpr uint32_t kInlineRouteMaxRows = 8192;  // eight rows per thread of a 1024-thread workgroup
-
-// LDS bytes of a row: its 2 K bytes rounded up to the 1 KiB a wave's direct-to-LDS load moves, plus 16 so
-// that the sixteen rows a wave reads side by side in step 2 (16 bytes each) fall on sixteen different
-// bank groups.
-__host__ __device__ inline uint32_t quant_lora_row_stride(uint32_t k) { return round_up(2u * k, 1024u) + 16u; }
-constexpr uint32_t kQuantLoraLdsBudget = 150u * 1024u;  // rows + reduction tiles; the rest of the 160 KiB is static
-__host__ __device__ inline uint32_t quant_lora_rows_per_wg(uint32_t k) {
-  uint32_t r = 16u;
-  while (r > 2u && r * quant_lora_row_stride(k) > kQuantLoraLdsBudget) r >>= 1;
-  return r;
-}
-// dynamic LDS of a launch: the rows, or the reduction tiles that reuse the same bytes once the rows are spent
-__host__ __device__ inline uint32_t quant_lora_lds_bytes(uint32_t k, uint32_t cb) {
-  const uint32_t rows = quant_lora_rows_per_wg(k) * quant_lora_row_stride(k);
-  const uint32_t red = 8u * (cb ? cb : 1u) * 4u * 64u * 4u;
-  return rows > red ? rows : red;
+// Row-major copy of the packed codes for a caller that asks for them (one workgroup per slot).
+__global__ __launch_bounds__(256) void codes_row_major_kernel(const unsigned char* __restrict__ xq, const int32_t* __restrict__ src_row,
+                                                              int8_t* __restrict__ codes, uint32_t M, uint32_t K, uint32_t KB) {
+  const uint32_t p = blockIdx.x;
+  const int src = src_row ? src_row[p] : (int)p;
+  if (src < 0 || src >= (int)M) return;
+  for (uint32_t k = threadIdx.x * 8u; k < K; k += 2048u)
+    *reinterpret_cast<uint2*>(codes + (size_t)src * K + k) = *reinterpret_cast<const uint2*>(xq + packed_offset(p, k, KB));
 }
 
-// The routing tables of route_rows_block for the 16 slots [16 hb, 16 hb + 16), computed by the
-// workgroup itself: rows keep their order inside a group (slot start[g] + j holds the j-th row of group
-// g), which every workgroup derives alike from the adapter indices alone.  Returns through LDS:
-// out_src[16], out_grp[16], out_range (the group range of the 32-slot block that holds the slots).
-// With group_pad = 32 every group starts on a block boundary (the slots between a group's last row and
-// the next group's first stay empty, src -1), so no 32-slot block holds rows of two groups: neither
-// this kernel nor the GEMM's epilogue then runs a block once per group.  The slots in use end at
-// sum(round_up(count, group_pad)) <= M + (group_pad - 1) * min(n_groups, M).
-// Steps: every wave counts its rows per group (LDS atomics on its own counters: with 16 waves on a CU
-// the vector ALU's share per wave makes a ballot per group and row several times dearer); wave 0 turns
-// the counts into per-wave prefixes, the groups' first slots and the groups of the sixteen slots; the
-// waves that hold the wanted ranks of a group pick their rows.  Three barriers.
-__device__ inline void route_rows_inline(const int32_t* __restrict__ idx, uint32_t M, uint32_t n_groups,
-                                         uint32_t slots, uint32_t group_pad, uint32_t hb, int* out_src, int* out_grp,
-                                         uint32_t* out_range, int* out_last_group) {
-  __shared__ int wcnt[kMaxAdapters][17];  // rows of group g in wave w; then the exclusive prefix over the waves
-  __shared__ int start[kMaxAdapters + 1];
-  __shared__ int cnt[kMaxAdapters];
-  __shared__ uint32_t used_end;  // first slot behind the last group
-  __shared__ int g_first_s, g_last_s;
-  const uint32_t tid = threadIdx.x, lane = tid & 63u;
-  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const uint32_t per = (M + 1023u) / 1024u;  // consecutive rows per thread (<= 8)
-  int mine[8];
-#pragma unroll
-  for (uint32_t j = 0; j < 8; ++j) {
-    const uint32_t i = tid * per + j;
-    int a = -1;
-    if (j < per && i < M) {
-      a = idx[i];
-      a = a < 0 ? 0 : (a >= (int)n_groups ? (int)n_groups - 1 : a);
-    }
-    mine[j] = a;
-  }
-  if (lane < n_groups) wcnt[lane][wave] = 0;  // (the loads above are still in flight)
-  __builtin_amdgcn_wave_barrier();
-#pragma unroll
-  for (uint32_t j = 0; j < 8; ++j)
-    if (j < per && mine[j] >= 0) atomicAdd(&wcnt[mine[j]][wave], 1);  // integer counts of one wave: any order
-  __syncthreads();
-  const uint32_t p0 = hb * 16u;
-  if (wave == 0) {  // lane g: group g (n_groups <= 64)
-    int total = 0;
-    if (lane < n_groups) {
-      int c[16];
-#pragma unroll
-      for (uint32_t w = 0; w < 16; ++w) c[w] = wcnt[lane][w];  // all reads first: one round trip
-#pragma unroll
-      for (uint32_t w = 0; w < 16; ++w) {
-        wcnt[lane][w] = total;
-        total += c[w];
-      }
-    }
-    const int padded = (int)round_up((uint32_t)total, group_pad);
-    int incl = padded;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const int up = __shfl_up(incl, off, 64);
-      if ((int)lane >= off) incl += up;
-    }
-    const int st = incl - padded;  // first slot of group `lane`
-    const uint32_t E = (uint32_t)__shfl(incl, 63, 64);
-    const unsigned long long nonempty = __builtin_amdgcn_ballot_w64(total > 0);
-    const int last_ne = nonempty ? 63 - __builtin_clzll(nonempty) : 0;
-    if (lane < n_groups) { start[lane] = st; cnt[lane] = total; }
-    if (lane == 0) { start[n_groups] = (int)E; used_end = E; *out_last_group = last_ne; }
-    // group of a slot: the last group whose first slot is not behind it (empty groups share their
-    // successor's first slot, so the last one is the one that holds the slot); slots behind the last
-    // group follow the last non-empty one
-    auto group_of = [&](uint32_t p) -> int {
-      if (p >= E) return last_ne;
-      const unsigned long long m = __builtin_amdgcn_ballot_w64(lane < n_groups && (uint32_t)st <= p);
-      return m ? 63 - __builtin_clzll(m) : 0;
-    };
-    const uint32_t p_end = (p0 + 16u < E) ? p0 + 16u : E;
-    const int gf = group_of(p0), gl = group_of(p_end ? p_end - 1u : 0u);
-    int my_grp = group_of(p0 + 15u);  // (the slots behind the last group follow the last non-empty one)
-    if (my_grp != gf) {  // wave-uniform: the sixteen slots hold a group boundary (or the end)
-#pragma unroll
-      for (uint32_t s16 = 0; s16 < 16; ++s16) {
-        const int g = group_of(p0 + s16);
-        if (lane == s16) my_grp = g;
-      }
-    }
-    if (lane < 16u) { out_grp[lane] = my_grp; out_src[lane] = -1; }
-    const uint32_t b0 = (p0 / 32u) * 32u;
-    const uint32_t b1 = (b0 + 31u < E) ? b0 + 31u : (E ? E - 1u : 0u);
-    const int gb0 = group_of(b0), gb1 = group_of(b1);
-    if (lane == 0) {
-      *out_range = b0 >= E ? 0u : ((uint32_t)gb0 | ((uint32_t)gb1 << 16));
-      g_first_s = p0 < E ? gf : 1;  // an empty range when the slots lie behind the last group
-      g_last_s = p0 < E ? gl : 0;
-    }
-  }
-  __syncthreads();
-  // the rows of the slots in use, group by group (a workgroup's 16 slots usually lie in one group)
-  const uint32_t E = used_end;
-  const uint32_t p_end = (p0 + 16u < E) ? p0 + 16u : E;
-  const int g_first = g_first_s, g_last = g_last_s;
-  for (int g = g_first; g <= g_last; ++g) {  // workgroup-uniform
-    const int cg = cnt[g], sg = start[g];
-    if (cg == 0) continue;
-    // slots of group g among mine: ranks [lo, hi)
-    const int lo = ((int)p0 > sg ? (int)p0 : sg) - sg;
-    const int hi = ((int)p_end < sg + cg ? (int)p_end : sg + cg) - sg;
-    const int wbefore = wcnt[g][wave];
-    const int wafter = wave < 15u ? wcnt[g][wave + 1u] : cg;
-    if (hi <= lo || wafter <= lo || wbefore >= hi) continue;  // wave-uniform: none of the wanted ranks is in this wave
-    int c = 0;
-#pragma unroll
-    for (uint32_t j = 0; j < 8; ++j) c += (mine[j] == g) ? 1 : 0;
-    int incl = c;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const int up = __shfl_up(incl, off, 64);
-      if ((int)lane >= off) incl += up;
-    }
-    int rank = wbefore + incl - c;
-#pragma unroll
-    for (uint32_t j = 0; j < 8; ++j) {
-      if (mine[j] == g) {
-        if (rank >= lo && rank < hi) out_src[sg + rank - (int)p0] = (int)(tid * per + j);
-        ++rank;
-      }
-    }
-  }
-  __syncthreads();
-}
+constexpr uint32_t kPaddedRouteMaxRows = 8192;  // groups start on block boundaries up to here (padded_groups_fit)
 
 template <int CB, bool RMS>  // CB: 16-wide rank blocks (0 = no LoRA, 1, 2, 4)
 __global__ __launch_bounds__(1024) void quant_lora_kernel(QuantLoraArgs a) {
   constexpr int kCB = CB > 0 ? CB : 1;
-  extern __shared__ __attribute__((aligned(1024))) unsigned char ql_lds[];  // the rows; later the wave tiles of z
-  __shared__ float row_scale[16];
-  __shared__ int row_src[16];
+  constexpr uint32_t kRing = CB == 4 || (CB == 2 && RMS) ? 2 : 4;  // operand sets (what 128 registers per lane hold)
+  constexpr uint32_t kAhead = 4;  // k-blocks of x a wave has in flight; a multiple of kRing
+  __shared__ float red[CB > 0 ? 8 : 1][kCB][4][64];  // wave tiles on their way to waves 0..7, then 0..3
   __shared__ float zs[16][kCB * 16 + 1];
-  typedef float red_t[kCB][4][64];  // wave tiles on their way to waves 0..7, then 0..3
-  red_t* const red = reinterpret_cast<red_t*>(ql_lds);
   const uint32_t tid = threadIdx.x, lane = tid & 63u;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const uint32_t R = a.rows_per_wg, per_hb = 16u / R;
-  const uint32_t hb = blockIdx.x / per_hb;           // half block: slots 16 hb .. 16 hb + 15
-  const uint32_t r0 = (blockIdx.x % per_hb) * R;     // this workgroup's slots inside it: r0 .. r0 + R - 1
+  const uint32_t hb = blockIdx.x;                    // half block: slots 16 hb .. 16 hb + 15
   if (a.tile_ctr && blockIdx.x == 0 && tid < 256u) a.tile_ctr[tid] = 0u;
   if (hb >= a.n_half_blocks) return;
   const uint32_t pb = hb >> 1, half16 = hb & 1u;
-  __shared__ int route_src[16], route_grp[16], route_last_group;
-  __shared__ uint32_t route_range;
-  const bool route_here = a.route_idx != nullptr;  // workgroup-uniform
-  if (route_here) {
-    route_rows_inline(a.route_idx, a.M, a.n_groups, a.slots, a.group_pad, hb, route_src, route_grp, &route_range,
-                      &route_last_group);
-    // the tables the GEMM reads later (every workgroup of a half block derives the same values)
-    if (tid >= r0 && tid < r0 + R) {
-      const_cast<int32_t*>(a.src_row)[hb * 16u + tid] = route_src[tid];
-      const_cast<int32_t*>(a.slot_group)[hb * 16u + tid] = route_grp[tid];
-    }
-    if (tid == 16u) const_cast<int32_t*>(a.blk_range)[pb] = (int32_t)route_range;  // (the same value from each)
-    if (blockIdx.x + 1u == gridDim.x) {  // the padding slots behind the last 32-row block, up to the GEMM's tile rows
-      for (uint32_t p = a.n_half_blocks * 16u + tid; p < a.slots; p += 1024u) {
-        const_cast<int32_t*>(a.src_row)[p] = -1;
-        const_cast<int32_t*>(a.slot_group)[p] = route_last_group;
-        if ((p & 31u) == 0) const_cast<int32_t*>(a.blk_range)[p / 32u] = 0;
-      }
-    }
-  }
-  if (a.group_pad > 1u && (route_here || a.src_row)) {
-    // padded groups leave whole stretches of slots empty: nothing reads their codes, scales or z
-    int any = 0;
-    for (uint32_t j = r0; j < r0 + R; ++j) any |= ((route_here ? route_src[j] : a.src_row[hb * 16u + j]) >= 0) ? 1 : 0;
-    if (!any) return;  // workgroup-uniform
-  }
-  // ---- 1. the rows into the LDS and their statistics: wave w, slot row r0 + w
-  const uint32_t lds_addr = (uint32_t)(uintptr_t)(lptr_t)ql_lds;
-  const uint32_t row_bytes = 2u * a.K;
-  const uint32_t n_chunks = (row_bytes + 1023u) / 1024u;  // 1 KiB pieces of a row (the last one may be partial)
-  if (wave < R) {
-    const uint32_t sl = r0 + wave;
-    const uint32_t p = hb * 16u + sl;
-    int src = route_here ? route_src[sl] : (a.src_row ? a.src_row[p] : (int)p);
-    if (src < 0 || src >= (int)a.M) src = -1;
-    src = __builtin_amdgcn_readfirstlane(src);
-    unsigned char* const rowl = ql_lds + wave * a.row_stride;
-    float inv = 1.0f;
-    uint32_t amax_bits = 0;  // largest |value| as bf16 bits in both halves
-    if (src >= 0) {
-      const unsigned char* xr = reinterpret_cast<const unsigned char*>(a.x) + (size_t)src * row_bytes;
-      const uint32_t row_lds = lds_addr + wave * a.row_stride;
-      for (uint32_t u = 0; u < n_chunks; ++u) {
-        const uint32_t voff = u * 1024u + lane * 16u;
-        if (voff < row_bytes) lds_load_1k(xr, voff, row_lds + u * 1024u);
-      }
-      // (the first chunk's norm weights travel with the row)
-      float4 gn0 = make_float4(0.f, 0.f, 0.f, 0.f), gn1 = gn0;
-      if (RMS && lane * 16u < row_bytes) {
-        gn0 = *reinterpret_cast<const float4*>(a.gamma + lane * 8u);
-        gn1 = *reinterpret_cast<const float4*>(a.gamma + lane * 8u + 4);
-      }
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      if (RMS) {
-        double ss = 0.0;
-        for (uint32_t u = 0; u < n_chunks; ++u) {
-          const uint32_t off = u * 1024u + lane * 16u;
-          const uint4 raw = off < row_bytes ? *reinterpret_cast<const uint4*>(rowl + off) : make_uint4(0, 0, 0, 0);
-          const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            // the square of a bf16 value is exact in double, so the fused form rounds like mul + add
-            const double lo = (double)__uint_as_float(w[e] << 16), hi = (double)__uint_as_float(w[e] & 0xffff0000u);
-            ss = __builtin_fma(lo, lo, ss);
-            ss = __builtin_fma(hi, hi, ss);
-          }
-        }
-        ss = wave_sum(ss);
-        const float var = (float)(ss / (double)a.K);
-        inv = 1.0f / sqrtf(var + a.eps);
-      }
-      for (uint32_t u = 0; u < n_chunks; ++u) {
-        const uint32_t off = u * 1024u + lane * 16u;
-        float4 g0 = gn0, g1 = gn1;
-        if (RMS) {  // the norm weights of the next chunk are requested before this one is worked on
-          const uint32_t offn = off + 1024u;
-          if (offn < row_bytes) {
-            gn0 = *reinterpret_cast<const float4*>(a.gamma + (offn >> 1));
-            gn1 = *reinterpret_cast<const float4*>(a.gamma + (offn >> 1) + 4);
-          }
-        }
-        if (off >= row_bytes) continue;
-        uint4 raw = *reinterpret_cast<const uint4*>(rowl + off);
-        if (RMS) {
-          const float g[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
-          uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            float t0 = __uint_as_float(w[e] << 16) * inv, t1 = __uint_as_float(w[e] & 0xffff0000u) * inv;
-            t0 = t0 * g[2 * e];
-            t1 = t1 * g[2 * e + 1];
-            w[e] = pack_bf16x2(t0, t1);
-          }
-          raw = make_uint4(w[0], w[1], w[2], w[3]);
-          *reinterpret_cast<uint4*>(rowl + off) = raw;  // the normalized row replaces the row
-          if (a.xn_aux) *reinterpret_cast<uint4*>(reinterpret_cast<unsigned char*>(a.xn_aux) + (size_t)src * row_bytes + off) = raw;
-        }
-        // |bf16| compares like its 15 magnitude bits as an integer (a NaN ends above every number and the
-        // scale then falls back to 1, as the reference's comparison amax > 0 does)
-        const uint32_t m0 = raw.x & 0x7fff7fffu, m1 = raw.y & 0x7fff7fffu, m2 = raw.z & 0x7fff7fffu, m3 = raw.w & 0x7fff7fffu;
-        typedef unsigned short us2 __attribute__((ext_vector_type(2)));
-        us2 mx = __builtin_bit_cast(us2, amax_bits);
-        mx = __builtin_elementwise_max(mx, __builtin_bit_cast(us2, m0));
-        mx = __builtin_elementwise_max(mx, __builtin_bit_cast(us2, m1));
-        mx = __builtin_elementwise_max(mx, __builtin_bit_cast(us2, m2));
-        mx = __builtin_elementwise_max(mx, __builtin_bit_cast(us2, m3));
-        amax_bits = __builtin_bit_cast(uint32_t, mx);
-      }
-    }
-    uint32_t top = (amax_bits >> 16) > (amax_bits & 0xffffu) ? (amax_bits >> 16) : (amax_bits & 0xffffu);
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      const uint32_t other = (uint32_t)__shfl_xor((int)top, o, 64);
-      top = other > top ? other : top;
-    }
-    const float amax = __uint_as_float(top << 16);
-    const float scale = amax > 0.0f ? amax / 127.0f : 1.0f;
-    if (lane == 0) {
-      row_scale[sl] = scale;
-      row_src[sl] = src;
-      a.sx_slots[p] = scale;
-      if (a.scales_rm && src >= 0) a.scales_rm[src] = scale;
-    }
-  }
-  __syncthreads();
-
-  // ---- 2. codes and z
   const uint32_t i = lane & 15u, q = lane >> 4;
-  const bool mine_row = i >= r0 && i < r0 + R;  // slot row i belongs to this workgroup
-  const int src = mine_row ? row_src[i] : -1;
-  const float scale = mine_row ? row_scale[i] : 1.0f;
+  int src = a.src_row ? a.src_row[hb * 16u + i] : (int)(hb * 16u + i);
+  if (src < 0 || src >= (int)a.M) src = -1;
+  if (a.group_pad > 1u && __builtin_amdgcn_ballot_w64(src >= 0) == 0)
+    return;  // workgroup-uniform: padded groups leave whole stretches of slots empty: nothing reads their codes, scales or z
+  // (a slot without a row works on row 0: nothing reads what it leaves, and no load sits under a lane condition)
+  const uint32_t row = src < 0 ? 0u : (uint32_t)src;
+  const float scale = a.row_scale[row];
+  const float inv = RMS ? a.row_inv[row] : 1.0f;
+  if (wave == 0 && lane < 16u) a.sx_slots[hb * 16u + i] = scale;
   const float rscale = __builtin_amdgcn_rcpf(scale);
-  const unsigned char* const rowl = ql_lds + (mine_row ? i - r0 : 0u) * a.row_stride;
-  const uint32_t range = CB == 0 ? 0u : (route_here ? route_range : (a.blk_range ? (uint32_t)a.blk_range[pb] : 0u));
+  const unsigned char* const xr = reinterpret_cast<const unsigned char*>(a.x) + (size_t)row * 2u * a.K;
+  const uint32_t range = (CB > 0 && a.blk_range) ? (uint32_t)a.blk_range[pb] : 0u;
   const uint32_t glo = range & 0xffffu, ghi = range >> 16;
-  const uint32_t rowgrp = (CB > 0 && ghi > glo)
-                              ? (route_here ? (uint32_t)route_grp[i] : (a.slot_group ? (uint32_t)a.slot_group[hb * 16u + i] : glo))
-                              : glo;
+  const uint32_t rowgrp = (CB > 0 && ghi > glo && a.slot_group) ? (uint32_t)a.slot_group[hb * 16u + i] : glo;
   v4f acc[kCB];
 #pragma unroll
   for (int b = 0; b < kCB; ++b) acc[b] = v4f{0.f, 0.f, 0.f, 0.f};
-  // fragment block byte offset of this lane's 8 codes: row 16*half16 + i, k half q/2, byte 8*(q%2)
-  const uint32_t code_off = (16u * half16 + i + 32u * (q >> 1)) * 16u + 8u * (q & 1u);
-  // One pass over the k-blocks per group present among the slots (one, except at a group boundary): the
-  // first pass also forms the codes; a later pass only adds the rows of its group to z (the rows are still
-  // in the LDS).  The loop is kept rolled, two k-blocks per trip with their operands requested one trip
-  // ahead and no load inside the work on a k-block, so that the compiler's waits count loads instead of
-  // draining them.
-  auto request = [&](uint32_t grp, uint32_t kb, v4i (&w)[kCB], uint4& raw) {
-    if constexpr (CB > 0) {
-      // operands of group grp, k-block kb: CB consecutive 1 KiB pieces (zero beyond K and the rank)
-      const v4i* ap = reinterpret_cast<const v4i*>(a.at) + (((size_t)grp * a.KB + kb) * CB) * 64u + lane;
-#pragma unroll
-      for (int b = 0; b < CB; ++b) w[b] = kb < a.KB ? ap[b * 64] : v4i{0, 0, 0, 0};
-    }
-    const uint32_t k0 = kb * 32u + q * 8u;
-    raw = (kb < a.KB && k0 < a.K && src >= 0) ? *reinterpret_cast<const uint4*>(rowl + 2u * k0) : make_uint4(0, 0, 0, 0);
+  // this lane's 8 codes of a fragment block: row 16*half16 + i, k half q/2, byte 8*(q%2)
+  unsigned char* const xq_dst =
+      a.xq_packed + (size_t)pb * a.KB * kBlockBytes + (16u * half16 + i + 32u * (q >> 1)) * 16u + 8u * (q & 1u);
+
+  // The wave's j-th k-block is wave + 16 j.  Everything beyond the last block is read as zeros without a
+  // condition: A and the norm weights through buffer resources that end with the data, x from the row's start.
+  const __amdgpu_buffer_rsrc_t grsrc =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.gamma), 0, RMS ? (int)(a.K * 4u) : 0, 0x00020000);
+  const uint32_t at_bytes = a.KB * (uint32_t)kCB * kBlockBytes;  // of one group
+  const uint32_t kq = wave * 32u + q * 8u;                       // the lane's k in its wave's first k-block
+  auto fetch_x = [&](uint32_t j) -> uint4 {
+    const uint32_t k0 = kq + 512u * j;
+    return *reinterpret_cast<const uint4*>(xr + 2u * (k0 < a.K ? k0 : 0u));  // (beyond K: zeroed where it is used)
   };
-  auto work = [&](bool first, bool in_group, uint32_t kb, const v4i (&w)[kCB], const uint4& raw) {
-    if (first) {  // wave-uniform
-      const uint32_t k0 = kb * 32u + q * 8u;
-      const bool live = src >= 0 && k0 < a.K;  // K is a multiple of 8
+  struct Operands { v4i w[kCB]; v4f g0, g1; };
+  auto fetch_operands = [&](const __amdgpu_buffer_rsrc_t& arsrc, uint32_t j, Operands& o) {
+    if constexpr (CB > 0) {  // CB consecutive 1 KiB pieces (zero beyond K and the rank)
+      const uint32_t off = (wave + 16u * j) * (uint32_t)(kCB * kBlockBytes) + lane * 16u;
+#pragma unroll
+      for (int b = 0; b < CB; ++b) o.w[b] = __builtin_amdgcn_raw_buffer_load_b128(arsrc, off + b * kBlockBytes, 0, 0);
+    }
+    if constexpr (RMS) {
+      const uint32_t off = (kq + 512u * j) * 4u;
+      o.g0 = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(grsrc, off, 0, 0));
+      o.g1 = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(grsrc, off + 16u, 0, 0));
+    }
+  };
+  const bool scale_safe = scale > 1e-30f && scale < 1e30f;
+  auto work = [&](auto codes, bool in_group, uint32_t j, const uint4& rawx, const Operands& o) {
+    const uint32_t kb = wave + 16u * j;
+    uint4 raw = rawx;
+    if constexpr (RMS)
+      raw = rms_normalize8(rawx, inv, make_float4(o.g0[0], o.g0[1], o.g0[2], o.g0[3]), make_float4(o.g1[0], o.g1[1], o.g1[2], o.g1[3]));
+    if (kb * 32u + 32u > a.K) {  // wave-uniform: the last k-block of an odd K, and the padding behind it
+      const bool live = kq + 512u * j < a.K;
+      raw.x = live ? raw.x : 0u; raw.y = live ? raw.y : 0u; raw.z = live ? raw.z : 0u; raw.w = live ? raw.w : 0u;
+    }
+    if constexpr (decltype(codes)::value) {
       const uint32_t nb[4] = {raw.x, raw.y, raw.z, raw.w};  // the (normalized) values as bf16 pairs
       float v[8];
 #pragma unroll
@@ -1185,7 +1127,7 @@ __global__ __launch_bounds__(1024) void quant_lora_kernel(QuantLoraArgs a) {
         c[e] = rintf(t);
         off_integer = fmaxf(off_integer, fabsf(t - c[e]));
       }
-      const bool redo = !(scale > 1e-30f && scale < 1e30f) || off_integer > 0.49996f;  // margin 4e-5 > 2.3e-5 + 2^-17
+      const bool redo = !scale_safe || off_integer > 0.49996f;  // margin 4e-5 > 2.3e-5 + 2^-17
       if (__builtin_amdgcn_ballot_w64(redo) != 0) {  // wave-uniform
 #pragma unroll
         for (int e = 0; e < 8; ++e) c[e] = rintf(v[e] / scale) + 128.0f;
@@ -1198,54 +1140,71 @@ __global__ __launch_bounds__(1024) void quant_lora_kernel(QuantLoraArgs a) {
       }
       lo ^= 0x80808080u;  // (a lane without a value holds zeros: 0 -> 128 -> code 0)
       hi ^= 0x80808080u;
-      if (live && a.codes_rm) *reinterpret_cast<uint2*>(a.codes_rm + (size_t)src * a.K + k0) = make_uint2(lo, hi);
-      if (mine_row) *reinterpret_cast<uint2*>(a.xq_packed + ((size_t)pb * a.KB + kb) * kBlockBytes + code_off) = make_uint2(lo, hi);
+      *reinterpret_cast<uint2*>(xq_dst + (size_t)kb * kBlockBytes) = make_uint2(lo, hi);
     }
     if constexpr (CB > 0) {
       // (zeros where the lane has no value; at a group boundary the rows of the other groups are zeroed)
       const v4i xa = in_group ? v4i{(int)raw.x, (int)raw.y, (int)raw.z, (int)raw.w} : v4i{0, 0, 0, 0};
 #pragma unroll
       for (int b = 0; b < CB; ++b)
-        acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, xa), __builtin_bit_cast(v8bf, w[b]),
+        acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, xa), __builtin_bit_cast(v8bf, o.w[b]),
                                                          acc[b], 0, 0, 0);
     }
   };
+  // A pass over the k-blocks, kAhead per trip: the x of kAhead k-blocks and the other operands of kRing - 1
+  // are in flight beside the one at work.  (With few workgroups on the chip the loop is a chain of those
+  // loads' latencies; no load or store in it is conditional, so the compiler's waits can count.)
+  const uint32_t n_j = wave < a.KB ? (a.KB - wave + 15u) / 16u : 0u;
+  auto pass = [&](auto codes, uint32_t grp, bool in_group) {
+    const __amdgpu_buffer_rsrc_t arsrc = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint16_t*>(a.at) + (size_t)grp * (at_bytes / 2u), 0, CB > 0 ? (int)at_bytes : 0, 0x00020000);
+    uint4 xc[kAhead];
+    Operands o[kRing];
+#pragma unroll
+    for (uint32_t u = 0; u < kAhead; ++u) xc[u] = fetch_x(u);
+#pragma unroll
+    for (uint32_t u = 0; u + 1u < kRing; ++u) fetch_operands(arsrc, u, o[u]);
+    uint32_t j = 0;
 #pragma unroll 1
-  for (uint32_t grp = glo; grp <= ghi; ++grp) {  // workgroup-uniform: one trip except at a group boundary
-    const bool first = grp == glo;
-    const bool in_group = ghi == glo || rowgrp == grp;
-    v4i wa[kCB], wb2[kCB];
-    uint4 ra, rb;
-    request(grp, wave, wa, ra);
-    request(grp, wave + 16u, wb2, rb);
-#pragma unroll 1
-    for (uint32_t kb = wave; kb < a.KB; kb += 32u) {
-      work(first, in_group, kb, wa, ra);
-      request(grp, kb + 32u, wa, ra);
-      if (kb + 16u >= a.KB) break;  // wave-uniform
-      work(first, in_group, kb + 16u, wb2, rb);
-      request(grp, kb + 48u, wb2, rb);
+    for (; j + kAhead <= n_j; j += kAhead) {
+#pragma unroll
+      for (uint32_t u = 0; u < kAhead; ++u) {
+        fetch_operands(arsrc, j + u + kRing - 1u, o[(u + kRing - 1u) % kRing]);
+        work(codes, in_group, j + u, xc[u], o[u % kRing]);
+        xc[u] = fetch_x(j + u + kAhead);
+      }
     }
-    if constexpr (CB == 0) break;
+#pragma unroll
+    for (uint32_t u = 0; u + 1u < kAhead; ++u) {  // the rest, fewer than kAhead
+      if (j + u >= n_j) break;  // wave-uniform
+      fetch_operands(arsrc, j + u + kRing - 1u, o[(u + kRing - 1u) % kRing]);
+      work(codes, in_group, j + u, xc[u], o[u % kRing]);
+    }
+  };
+  // one pass per group present among the slots (one, except at a group boundary): the first also forms the
+  // codes, a later one only adds the rows of its group to z
+  pass(std::true_type{}, glo, ghi == glo || rowgrp == glo);
+  if constexpr (CB > 0) {
+#pragma unroll 1
+    for (uint32_t grp = glo + 1u; grp <= ghi; ++grp) pass(std::false_type{}, grp, rowgrp == grp);
   }
   if constexpr (CB == 0) return;
 
-  // ---- 3. fixed-order sum of the 16 wave tiles: 8..15 onto 0..7, 4..7 onto 0..3, then 0+1+2+3
-  __syncthreads();  // the rows are spent: their bytes take the wave tiles
+  // ---- fixed-order sum of the 16 wave tiles: 8..15 onto 0..7, 4..7 onto 0..3, then 0+1+2+3
 #pragma unroll 1
   for (uint32_t half = 8u; half >= 4u; half >>= 1) {
     if (wave >= half && wave < 2u * half) {
 #pragma unroll
       for (int b = 0; b < kCB; ++b)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) red[wave - half][b][e][lane] = acc[b][e];
+        for (int e = 0; e < 4; ++e) red[CB > 0 ? wave - half : 0u][b][e][lane] = acc[b][e];
     }
     __syncthreads();
     if (wave < half) {
 #pragma unroll
       for (int b = 0; b < kCB; ++b)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc[b][e] = acc[b][e] + red[wave][b][e][lane];
+        for (int e = 0; e < 4; ++e) acc[b][e] = acc[b][e] + red[CB > 0 ? wave : 0u][b][e][lane];
     }
     __syncthreads();
   }
@@ -1253,20 +1212,19 @@ __global__ __launch_bounds__(1024) void quant_lora_kernel(QuantLoraArgs a) {
 #pragma unroll
     for (int b = 0; b < kCB; ++b)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) red[wave][b][e][lane] = acc[b][e];
+      for (int e = 0; e < 4; ++e) red[CB > 0 ? wave : 0u][b][e][lane] = acc[b][e];
   }
   __syncthreads();
   // MFMA result layout: lane l holds column l % 16 and rows 4 * (l / 16) + e
   for (uint32_t t = tid; t < (uint32_t)kCB * 256u; t += 1024u) {
     const uint32_t l = t & 63u, e = (t >> 6) & 3u, b = t >> 8;
-    const float sum = ((red[0][b][e][l] + red[1][b][e][l]) + red[2][b][e][l]) + red[3][b][e][l];
+    const float sum = ((red[0][b][e][l] + red[CB > 0 ? 1 : 0][b][e][l]) + red[CB > 0 ? 2 : 0][b][e][l]) + red[CB > 0 ? 3 : 0][b][e][l];
     zs[4u * (l >> 4) + e][b * 16u + (l & 15u)] = sum;
   }
   __syncthreads();
   // zp[pb][kk][term][lane64][8]: lane = row % 32 + 32 * hh holds rank columns 16 kk + 8 hh + 0..7
   for (uint32_t t = tid; t < a.nkk * 3u * 32u; t += 1024u) {
     const uint32_t row = t & 15u, hh = (t >> 4) & 1u, term = (t >> 5) % 3u, kk = t / 96u;
-    if (row < r0 || row >= r0 + R) continue;
     v8us o;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
