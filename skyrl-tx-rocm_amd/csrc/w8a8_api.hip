@@ -755,7 +755,37 @@ int run_grouped(const mi355_w8a8_grouped_problem* p, hipStream_t s) {
 // ---------------------------------------------------------------------------------------
 // backward
 // ---------------------------------------------------------------------------------------
+// How the pull-back's tiles of 256 x 256 are spread over the chip: whole tiles while they come in full rounds of
+// 256 workgroups, the rest split along the contraction so that the last round takes its share of the time
+// and not all of it (sk_wgs workgroups of sk_q stages each; 0: no split).
+struct BwdDxSplit { uint32_t direct_tiles, sk_q, sk_wgs; };
+
+// Costs in stage times (about 1.05 us): a split adds the partial tiles' way through memory, 256 KiB written
+// and read again for every workgroup and split tile (about 0.11 each at 4.7 TB/s), and a launch.  Measured: 2048 x 2560,
+// N = 10240 (80 tiles of 320 stages) 339 us whole, 135 + 22 us split; 3003 x 4096, N = 24576 (192 of 768) 800 us and 657 + 29 us.
+// Calls of fewer than 64 stages (N < 2048) stay whole: little to gain, and a grouped call over the same rows
+// then gives the same bits.
+BwdDxSplit bwd_dx_split(uint32_t tiles_m, uint32_t tiles_k, uint32_t NB) {
+  const uint32_t ntile = tiles_m * tiles_k, rem = ntile % 256u;
+  BwdDxSplit best{ntile, 0u, 0u};
+  if (rem == 0u || NB < 64u) return best;
+  double cost = 0.9 * NB;
+  for (uint32_t wgs = 64u; wgs <= 256u; wgs += 64u) {
+    uint32_t q = (rem * NB + wgs - 1u) / wgs;
+    q = round_up(q < 16u ? 16u : q, 2u);
+    const double c = q + 0.11 * (wgs + rem) + 8.0;
+    if (c < cost) {
+      cost = c;
+      best.direct_tiles = ntile - rem; best.sk_q = q;
+      best.sk_wgs = round_up((rem * NB + q - 1u) / q, 8u);
+    }
+  }
+  return best;
+}
+
 struct BwdLayout {
+  BwdDxSplit split;
+  uint64_t part;
   uint64_t dyp, swp, at, ap, rp, z, r_raw, rs, rpart, src_row, dst_pos, slot_group, blk_range, group_off, partA, partB, total;
   uint32_t slots, nkk, K_pad, KB, N_pad, NB, tiles_m, tiles_k, max_chunks, R, n_slices, groups_per_slice;
 };
@@ -775,7 +805,9 @@ BwdLayout make_bwd_layout(uint32_t m, uint32_t k, uint32_t n, uint32_t n_groups,
     w.n_slices = (ng + 3u) / 4u < 8u ? (ng + 3u) / 4u : 8u;
     w.groups_per_slice = (ng + w.n_slices - 1u) / w.n_slices;
   }
+  w.split = bwd_dx_split(w.tiles_m, w.tiles_k, w.NB);
   uint64_t off = 0;
+  w.part = off; off += (uint64_t)w.split.sk_wgs * 2u * kBwdPartFloats * 4u;
   w.dyp = off; off += align256((uint64_t)w.slots * w.N_pad * 2u);
   w.swp = off; off += align256((uint64_t)(w.N_pad + kBwdScalePad) * 4u);  // a stage fetches 1 KiB of scales starting at its own 32
   w.src_row = off; off += align256((uint64_t)w.slots * 4u);
@@ -810,13 +842,17 @@ int validate_bwd_dims(uint32_t m, uint32_t k, uint32_t n, uint32_t n_adapters, u
 
 template <int NKK, bool ROWS128>
 int launch_bwd_dx_geometry(const BwdDxArgs& g, hipStream_t s) {
-  const uint32_t ntile = g.tiles_m * g.tiles_k;
-  const uint32_t want = ((ntile + 7u) / 8u) * 8u;
+  uint32_t want = ((g.direct_tiles + 7u) / 8u) * 8u;
+  if (g.sk_wgs > want) want = g.sk_wgs;
   const dim3 grid(want < 256u ? want : 256u), block(512);
   if (hipFuncSetAttribute(reinterpret_cast<const void*>(&bwd_dx_kernel<NKK, ROWS128>),
                           hipFuncAttributeMaxDynamicSharedMemorySize, kBwdLdsBytes) != hipSuccess)
     return MI355_W8A8_ERR_LAUNCH;
   hipLaunchKernelGGL((bwd_dx_kernel<NKK, ROWS128>), grid, block, kBwdLdsBytes, s, g);
+  if (!g.sk_wgs) return launch_status();
+  if (const int st = launch_status()) return st;
+  const uint32_t split_tiles = g.tiles_m * g.tiles_k - g.direct_tiles;
+  hipLaunchKernelGGL((bwd_dx_finish_kernel<NKK>), dim3(split_tiles * 8u), dim3(256), 0, s, g);
   return launch_status();
 }
 
@@ -842,6 +878,7 @@ struct BwdBody {
   const int32_t* group_end;
   size_t w_stride; uint32_t sw_stride;
   bool rows128;  // the pull-back runs 128-row x 512-k tiles (the tables are padded to match)
+  BwdDxSplit split; uint64_t part;  // dense calls
 };
 
 template <class Layout>
@@ -921,6 +958,9 @@ int launch_bwd_body(const BwdBody& b, const Layout& w, unsigned char* ws, hipStr
     g.dx = static_cast<uint16_t*>(b.dx);
     g.M = b.m; g.K = b.k; g.KB = w.KB; g.NB = w.NB; g.tiles_m = w.tiles_m; g.tiles_k = w.tiles_k;
     g.tile_weight = b.tile_weight; g.w_stride = b.w_stride; g.sw_stride = b.sw_stride;
+    g.direct_tiles = b.split.sk_wgs ? b.split.direct_tiles : w.tiles_m * w.tiles_k;
+    g.sk_q = b.split.sk_q; g.sk_wgs = b.split.sk_wgs;
+    g.part = b.split.sk_wgs ? reinterpret_cast<float*>(ws + b.part) : nullptr;
     switch (b.lora ? w.nkk : 0u) {
       case 0: st = launch_bwd_dx<0>(g, b.rows128, s); break;
       case 1: st = launch_bwd_dx<1>(g, b.rows128, s); break;
@@ -1044,6 +1084,7 @@ int run_backward(const mi355_w8a8_bwd_problem* p, hipStream_t s) {
   b.slot_group = routed ? slot_group : nullptr;
   b.blk_range = routed ? blk_range : nullptr;
   b.group_off = group_off;
+  b.split = w.split; b.part = w.part;
   return launch_bwd_body(b, w, ws, s);
 }
 

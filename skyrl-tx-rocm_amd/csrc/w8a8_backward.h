@@ -433,7 +433,74 @@ struct BwdDxArgs {
   const int32_t* tile_weight;
   size_t w_stride;
   uint32_t sw_stride;
+  // dense calls: the tiles from direct_tiles on are split (bwd_dx_split): sk_wgs workgroups take sk_q
+  // consecutive stages each of their joint stage sequence and leave float32 partial tiles in part
+  uint32_t direct_tiles, sk_q, sk_wgs;
+  float* part;   // [2 * sk_wgs slots][8 waves][4 row blocks][2 k blocks][4][64 lanes][4]
 };
+constexpr uint32_t kBwdPartFloats = 65536;  // of a slot
+
+// (row tile, k tile) of position t in the band-major tile order: 4 row tiles x all k tiles to a band
+__device__ inline void bwd_dx_tile_at(const BwdDxArgs& g, uint32_t t, uint32_t& tm, uint32_t& tk) {
+  const uint32_t band_tiles = 4u * g.tiles_k, band = t / band_tiles, in_band = t - band * band_tiles;
+  const uint32_t band_rows = (g.tiles_m - band * 4u) < 4u ? (g.tiles_m - band * 4u) : 4u;
+  tm = band * 4u + in_band % band_rows;
+  tk = in_band / band_rows;
+}
+
+// A wave's 32 x 64 block of dx: + rs @ A.T, one cast, rows back to their original positions.  pbase: first
+// slot of the block's 32; kbw: first of its two k blocks.
+template <int NKK>
+__device__ inline void bwd_dx_store_block(const BwdDxArgs& g, uint32_t pbase, uint32_t kbw, const v16f (&acc)[2]) {
+  const int lane = threadIdx.x & 63, c = lane & 31, h = lane >> 5;
+  const uint32_t blk = pbase / 32u;
+  const int src_lane = g.src_row ? g.src_row[pbase + c] : (int)(pbase + c);
+  const bool row_ok = src_lane >= 0 && src_lane < (int)g.M;
+  const uint32_t off_lane = row_ok ? (uint32_t)src_lane * g.K : 0xffffffffu;
+  if (__builtin_amdgcn_ballot_w64(row_ok) == 0) return;  // wave-uniform: no row of this block exists
+  const uint32_t range = (NKK > 0 && g.blk_range) ? (uint32_t)g.blk_range[blk] : 0u;
+  const int glo = (int)(range & 0xffffu), ghi = (int)(range >> 16);
+  const int grp_lane = (NKK > 0 && g.slot_group && ghi > glo) ? g.slot_group[pbase + c] : glo;
+  const int row_addr = 16 * h;
+  for (int gi = glo; gi <= ghi; ++gi) {  // a block at a group boundary runs once per group
+#pragma unroll
+    for (int cb = 0; cb < 2; ++cb) {
+      const uint32_t kb = kbw + cb;
+      if (kb >= g.KB) continue;  // wave-uniform
+      const uint32_t kcol = kb * 32u + c;
+      v16f y = acc[cb];
+      if constexpr (NKK > 0) {
+        const unsigned char* rb0 = g.rp + (size_t)blk * NKK * 3u * kBlockBytes + lane * 16;
+        const unsigned char* ab0 = g.ap + ((size_t)gi * g.KB + kb) * NKK * kBlockBytes + lane * 16;
+        v16f low;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) low[e] = 0.0f;
+#pragma unroll
+        for (int kk = 0; kk < NKK; ++kk) {
+          const v8bf ab = __builtin_bit_cast(v8bf, *reinterpret_cast<const v8us*>(ab0 + kk * kBlockBytes));
+#pragma unroll
+          for (int t3 = 2; t3 >= 0; --t3) {
+            const v8bf rf = __builtin_bit_cast(v8bf, *reinterpret_cast<const v8us*>(rb0 + (kk * 3 + t3) * kBlockBytes));
+            low = __builtin_amdgcn_mfma_f32_32x32x16_bf16(rf, ab, low, 0, 0, 0);
+          }
+        }
+#pragma unroll
+        for (int e = 0; e < 16; ++e) y[e] = y[e] + low[e];
+      }
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int src_lane_addr = row_addr + 4 * (8 * (v >> 2) + (v & 3));
+        const uint32_t rowoff = (uint32_t)__builtin_amdgcn_ds_bpermute(src_lane_addr, (int)off_lane);
+        // every lane takes part in the cross-lane reads: a lane that is switched off (a column
+        // beyond K) would hand zeros to the lanes that read from it
+        int row_grp = gi;
+        if (NKK > 0 && ghi > glo) row_grp = __builtin_amdgcn_ds_bpermute(src_lane_addr, grp_lane);
+        const bool ok = (rowoff != 0xffffffffu) & (kcol < g.K) & (row_grp == gi);
+        if (ok) g.dx[(size_t)rowoff + kcol] = (uint16_t)f32_to_bf16_bits(y[v]);
+      }
+    }
+  }
+}
 
 // ROWS128: the tile is 128 rows x 512 k (the eight waves side by side along k, the same 128 x 64 wave
 // tile): a stage then holds half the dy panel and twice the weight blocks, the same bytes and the same
@@ -460,36 +527,15 @@ __global__ __launch_bounds__(512, 1) void bwd_dx_kernel(BwdDxArgs g) {
     ident[2] = wi == 2 ? word : 0; ident[3] = wi == 3 ? word : 0;
   }
 
-  const uint32_t ntile = g.tiles_m * g.tiles_k;
-  const uint32_t wgs_per_xcd = gridDim.x >> 3, xcd = blockIdx.x & 7u;
-  // band-major tile order: 4 row tiles x all k tiles, so an XCD's workgroups share panels.  One weight:
-  // every XCD walks a contiguous range of bands.  Grouped calls: the bands are dealt round-robin to the
-  // XCDs, because the slots in use end before the last bands and a contiguous split would leave the
-  // last XCDs without work.
-  const uint32_t band_tiles = 4u * g.tiles_k, n_bands = (g.tiles_m + 3u) / 4u;
-  const uint32_t per_xcd = g.tile_weight ? ((n_bands + 7u) / 8u) * band_tiles : (ntile + 7u) / 8u;
-  for (uint32_t ti = blockIdx.x >> 3; ti < per_xcd; ti += wgs_per_xcd) {
-    uint32_t band, in_band;
-    if (g.tile_weight) {
-      band = xcd + 8u * (ti / band_tiles);
-      in_band = ti % band_tiles;
-      if (band >= n_bands) break;
-    } else {
-      const uint32_t t = xcd * per_xcd + ti;
-      if (t >= ntile) break;
-      band = t / band_tiles;
-      in_band = t - band * band_tiles;
-    }
-    const uint32_t band_rows = (g.tiles_m - band * 4u) < 4u ? (g.tiles_m - band * 4u) : 4u;
-    if (in_band >= band_rows * g.tiles_k) continue;  // a last band with fewer than 4 row tiles (grouped order only)
-    const uint32_t tm = band * 4u + in_band % band_rows, tk = in_band / band_rows;
+  // One tile, or the stages nb0 .. nb0 + L - 1 (an even number) of one whose partial sums go to slot `slot`.
+  auto segment = [&](uint32_t tm, uint32_t tk, int nb0, int L, bool whole, uint32_t slot) {
     int tw = 0;
     int n_act = 4;  // 32-row blocks of this wave that hold rows: the others skip their matrix-core work
     // row block whose dy panel this wave fetches: both 1 KiB halves, or one half of it in a 128-row tile
     uint32_t load_rb = ROWS128 ? (uint32_t)wave >> 1 : (uint32_t)wave;
     if (g.tile_weight) {
       const int tv = g.tile_weight[tm];
-      if (tv < 0) continue;  // workgroup-uniform: no row lives in this tile
+      if (tv < 0) return;  // workgroup-uniform: no row lives in this tile
       tw = tv & 0xffff;
       const int live_blocks = ((tv >> 16) + 31) / 32;
       const int live = live_blocks - wrow * 4;
@@ -497,6 +543,9 @@ __global__ __launch_bounds__(512, 1) void bwd_dx_kernel(BwdDxArgs g) {
       // a block without rows is never multiplied: its slot is filled from block 0 of the tile, which
       // is in the caches anyway, instead of streaming unused memory (the load count stays the same)
       if ((int)load_rb >= live_blocks) load_rb = 0u;
+    } else {  // (the rows of a dense call fill the slots from the first)
+      const int live = ((int)(g.M - tm * (uint32_t)(kRowBlocks * 32)) + 31) / 32 - wrow * 4;
+      n_act = live < 0 ? 0 : (live > 4 ? 4 : live);
     }
     n_act = __builtin_amdgcn_readfirstlane(n_act);
     const float* swp_t = g.swp + (size_t)tw * g.sw_stride;
@@ -513,8 +562,9 @@ __global__ __launch_bounds__(512, 1) void bwd_dx_kernel(BwdDxArgs g) {
     const unsigned char* Bg1 = g.wp + (size_t)tw * g.w_stride + (size_t)kbl1 * kBlockBytes + lane * 16;
     const size_t nb_stride = (size_t)g.KB * kBlockBytes;
 
-    auto issue = [&](int nb) {
-      unsigned char* St = lds + (nb % kBwdStages) * kBwdStageBytes;
+    auto issue = [&](int i) {  // stage i of the segment
+      unsigned char* St = lds + (i % kBwdStages) * kBwdStageBytes;
+      const int nb = nb0 + i;
       const unsigned char* src = Ag + (size_t)nb * 2048u;
       if constexpr (ROWS128) {
         load_1k_to_lds(src, St + wave * kBlockBytes);
@@ -624,12 +674,13 @@ __global__ __launch_bounds__(512, 1) void bwd_dx_kernel(BwdDxArgs g) {
       }
     };
 
-    // ---- main loop.  Stage nb issues the loads of stage nb + 5.
+    // ---- main loop.  Stage i issues the loads of stage i + 5.
     v8bf bqA[2][2], bqB[2][2];
     wait_vmcnt<0>();  // stores of the previous tile
     lds_barrier();
 #pragma unroll
-    for (int i = 0; i < kBwdAhead; ++i) issue(i);  // NB >= 8
+    for (int i = 0; i < kBwdAhead; ++i)
+      if (i < L) issue(i);
     wait_vmcnt<0>();
     lds_barrier();
     if (n_act > 0) {  // operands of stage 0
@@ -645,91 +696,138 @@ __global__ __launch_bounds__(512, 1) void bwd_dx_kernel(BwdDxArgs g) {
         to_operands(pk, bqA[cb]);
       }
     }
-    const int NB_main = NBi - kBwdAhead;  // stages that still have loads to issue; odd
-    int nb = 0;
-    for (; nb + 1 < NB_main; nb += 2) {
-      // stage nb + 1 (and so stage nb) is older than the loads of the last three stages
+    const int L_main = L - kBwdAhead;  // stages that still have loads to issue
+    int i = 0;
+    for (; i + 1 < L_main; i += 2) {
+      // stage i + 1 (and so stage i) is older than the loads of the last three stages
       wait_vmcnt<(kBwdAhead - 2) * kBwdLoadsPerStage>();
       lds_barrier();
       __builtin_amdgcn_sched_barrier(0);
-      issue(nb + kBwdAhead);
-      stage(nb, bqA, bqB, true);
+      issue(i + kBwdAhead);
+      stage(i, bqA, bqB, true);
       __builtin_amdgcn_sched_barrier(0);
       wait_vmcnt<(kBwdAhead - 2) * kBwdLoadsPerStage>();
       lds_barrier();
       __builtin_amdgcn_sched_barrier(0);
-      issue(nb + 1 + kBwdAhead);
-      stage(nb + 1, bqB, bqA, true);
+      issue(i + 1 + kBwdAhead);
+      stage(i + 1, bqB, bqA, true);
       __builtin_amdgcn_sched_barrier(0);
     }
-    for (; nb < NBi; nb += 2) {  // drain: fewer loads in flight than the count above assumes
+    for (; i < L; i += 2) {  // drain: fewer loads in flight than the count above assumes
       wait_vmcnt<0>();
       lds_barrier();
       __builtin_amdgcn_sched_barrier(0);
-      if (nb + kBwdAhead < NBi) issue(nb + kBwdAhead);
-      stage(nb, bqA, bqB, true);
+      if (i + kBwdAhead < L) issue(i + kBwdAhead);
+      stage(i, bqA, bqB, true);
       __builtin_amdgcn_sched_barrier(0);
       wait_vmcnt<0>();
       lds_barrier();
       __builtin_amdgcn_sched_barrier(0);
-      if (nb + 1 + kBwdAhead < NBi) issue(nb + 1 + kBwdAhead);
-      stage(nb + 1, bqB, bqA, nb + 2 < NBi);
+      if (i + 1 + kBwdAhead < L) issue(i + 1 + kBwdAhead);
+      stage(i + 1, bqB, bqA, i + 2 < L);
       __builtin_amdgcn_sched_barrier(0);
     }
 
-    // ---- epilogue: + rs @ A.T, one cast, rows back to their original positions
+    if (whole) {
 #pragma unroll
-    for (int rb = 0; rb < 4; ++rb) {
-      const uint32_t pbase = tm * (uint32_t)(kRowBlocks * 32) + (uint32_t)wrow * 128u + rb * 32u;
-      const uint32_t blk = pbase / 32u;
-      const int src_lane = g.src_row ? g.src_row[pbase + c] : (int)(pbase + c);
-      const bool row_ok = src_lane >= 0 && src_lane < (int)g.M;
-      const uint32_t off_lane = row_ok ? (uint32_t)src_lane * g.K : 0xffffffffu;
-      if (__builtin_amdgcn_ballot_w64(row_ok) == 0) continue;  // wave-uniform: no row of this block exists
-      const uint32_t range = (NKK > 0 && g.blk_range) ? (uint32_t)g.blk_range[blk] : 0u;
-      const int glo = (int)(range & 0xffffu), ghi = (int)(range >> 16);
-      const int grp_lane = (NKK > 0 && g.slot_group && ghi > glo) ? g.slot_group[pbase + c] : glo;
-      const int row_addr = 16 * h;
-      for (int gi = glo; gi <= ghi; ++gi) {  // a block at a group boundary runs once per group
+      for (int rb = 0; rb < 4; ++rb)
+        if (rb < n_act)
+          bwd_dx_store_block<NKK>(g, tm * (uint32_t)(kRowBlocks * 32) + (uint32_t)wrow * 128u + rb * 32u, kbw, acc[rb]);
+    } else {
+      float4* dst = reinterpret_cast<float4*>(g.part + (size_t)slot * kBwdPartFloats) + (uint32_t)wave * 2048u + lane;
 #pragma unroll
-        for (int cb = 0; cb < 2; ++cb) {
-          const uint32_t kb = kbw + cb;
-          if (kb >= g.KB) continue;  // wave-uniform
-          const uint32_t kcol = kb * 32u + c;
-          v16f y = acc[rb][cb];
-          if constexpr (NKK > 0) {
-            const unsigned char* rb0 = g.rp + (size_t)blk * NKK * 3u * kBlockBytes + lane * 16;
-            const unsigned char* ab0 = g.ap + ((size_t)gi * g.KB + kb) * NKK * kBlockBytes + lane * 16;
-            v16f low;
+      for (int rb = 0; rb < 4; ++rb)
+        if (rb < n_act)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) low[e] = 0.0f;
+          for (int cb = 0; cb < 2; ++cb)
 #pragma unroll
-            for (int kk = 0; kk < NKK; ++kk) {
-              const v8bf ab = __builtin_bit_cast(v8bf, *reinterpret_cast<const v8us*>(ab0 + kk * kBlockBytes));
-#pragma unroll
-              for (int t3 = 2; t3 >= 0; --t3) {
-                const v8bf rf = __builtin_bit_cast(v8bf, *reinterpret_cast<const v8us*>(rb0 + (kk * 3 + t3) * kBlockBytes));
-                low = __builtin_amdgcn_mfma_f32_32x32x16_bf16(rf, ab, low, 0, 0, 0);
-              }
-            }
-#pragma unroll
-            for (int e = 0; e < 16; ++e) y[e] = y[e] + low[e];
-          }
-#pragma unroll
-          for (int v = 0; v < 16; ++v) {
-            const int src_lane_addr = row_addr + 4 * (8 * (v >> 2) + (v & 3));
-            const uint32_t rowoff = (uint32_t)__builtin_amdgcn_ds_bpermute(src_lane_addr, (int)off_lane);
-            // every lane takes part in the cross-lane reads: a lane that is switched off (a column
-            // beyond K) would hand zeros to the lanes that read from it
-            int row_grp = gi;
-            if (NKK > 0 && ghi > glo) row_grp = __builtin_amdgcn_ds_bpermute(src_lane_addr, grp_lane);
-            const bool ok = (rowoff != 0xffffffffu) & (kcol < g.K) & (row_grp == gi);
-            if (ok) g.dx[(size_t)rowoff + kcol] = (uint16_t)f32_to_bf16_bits(y[v]);
-          }
-        }
-      }
+            for (int e = 0; e < 4; ++e)
+              dst[((rb * 2 + cb) * 4 + e) * 64] = make_float4(acc[rb][cb][4 * e], acc[rb][cb][4 * e + 1], acc[rb][cb][4 * e + 2], acc[rb][cb][4 * e + 3]);
     }
+  };
+
+  const uint32_t ntile = g.direct_tiles;
+  const uint32_t wgs_per_xcd = gridDim.x >> 3, xcd = blockIdx.x & 7u;
+  // band-major tile order, so an XCD's workgroups share panels.  One weight:
+  // every XCD walks a contiguous range of bands.  Grouped calls: the bands are dealt round-robin to the
+  // XCDs, because the slots in use end before the last bands and a contiguous split would leave the
+  // last XCDs without work.
+  const uint32_t band_tiles = 4u * g.tiles_k, n_bands = (g.tiles_m + 3u) / 4u;
+  const uint32_t per_xcd = g.tile_weight ? ((n_bands + 7u) / 8u) * band_tiles : (ntile + 7u) / 8u;
+  uint32_t ti = blockIdx.x >> 3;
+  // behind the whole tiles: this workgroup's stages of the split tiles' joint sequence (an XCD's workgroups are
+  // neighbours)
+  const uint32_t sw8 = g.sk_wgs >> 3, sk_w = xcd * sw8 + (blockIdx.x >> 3);
+  uint32_t s0 = 0, s1 = 0;
+  if (!ROWS128 && (blockIdx.x >> 3) < sw8) {
+    const uint32_t total = (g.tiles_m * g.tiles_k - ntile) * g.NB;
+    s0 = sk_w * g.sk_q < total ? sk_w * g.sk_q : total;
+    s1 = s0 + g.sk_q < total ? s0 + g.sk_q : total;
   }
+  const uint32_t sk_t0 = s0 / g.NB;
+#pragma unroll 1
+  for (;;) {
+    uint32_t t, nb0 = 0, len = g.NB, slot = 0;
+    if (ti < per_xcd) {
+      const uint32_t pos = ti;
+      ti += wgs_per_xcd;
+      if (g.tile_weight) {
+        const uint32_t band = xcd + 8u * (pos / band_tiles), in_band = pos % band_tiles;
+        if (band >= n_bands) { ti = per_xcd; continue; }
+        const uint32_t band_rows = (g.tiles_m - band * 4u) < 4u ? (g.tiles_m - band * 4u) : 4u;
+        if (in_band >= band_rows * g.tiles_k) continue;  // a last band with fewer than 4 row tiles
+        t = band * band_tiles + in_band;
+      } else {
+        t = xcd * per_xcd + pos;
+        if (t >= ntile) { ti = per_xcd; continue; }
+      }
+    } else if (s0 < s1) {
+      const uint32_t u = s0 / g.NB;
+      nb0 = s0 - u * g.NB;
+      len = s1 - s0 < g.NB - nb0 ? s1 - s0 : g.NB - nb0;
+      t = ntile + u;
+      slot = 2u * sk_w + (u == sk_t0 ? 0u : 1u);
+      s0 += len;
+    } else {
+      break;
+    }
+    uint32_t tm, tk;
+    bwd_dx_tile_at(g, t, tm, tk);
+    segment(tm, tk, (int)nb0, (int)len, len == g.NB, slot);
+  }
+}
+
+// The split tiles of bwd_dx_kernel: the partial sums of a tile added in the order of its stages, then the
+// kernel's own epilogue.  A wave per 32 x 64 block.
+template <int NKK>
+__global__ __launch_bounds__(256) void bwd_dx_finish_kernel(BwdDxArgs g) {
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t item = blockIdx.x * 4u + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t u = item >> 5, wave = (item >> 2) & 7u, rb = item & 3u;
+  const uint32_t first = u * g.NB / g.sk_q, last = ((u + 1u) * g.NB - 1u) / g.sk_q;
+  if (first == last) return;  // one workgroup had all its stages and has stored it
+  uint32_t tm, tk;
+  bwd_dx_tile_at(g, g.direct_tiles + u, tm, tk);
+  const uint32_t pbase = tm * 256u + (wave >> 2) * 128u + rb * 32u;
+  const uint32_t kbw = tk * 8u + (wave & 3u) * 2u;
+  if (pbase >= g.M || kbw >= g.KB) return;
+  v16f y[2];
+#pragma unroll
+  for (int cb = 0; cb < 2; ++cb)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) y[cb][e] = 0.0f;
+  for (uint32_t w = first; w <= last; ++w) {
+    const uint32_t slot = 2u * w + (w * g.sk_q / g.NB == u ? 0u : 1u);
+    const float4* src = reinterpret_cast<const float4*>(g.part + (size_t)slot * kBwdPartFloats) + wave * 2048u + rb * 512u + lane;
+#pragma unroll
+    for (int cb = 0; cb < 2; ++cb)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float4 v = src[(cb * 4 + e) * 64];
+        y[cb][4 * e] += v.x; y[cb][4 * e + 1] += v.y; y[cb][4 * e + 2] += v.z; y[cb][4 * e + 3] += v.w;
+      }
+  }
+  bwd_dx_store_block<NKK>(g, pbase, kbw, y);
 }
 
 // ---------------------------------------------------------------------------------------
