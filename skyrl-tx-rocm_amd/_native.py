@@ -27,6 +27,7 @@ FLAG_LORA_PACK_VALID = 1024
 FLAG_TILE_128X128 = 2048
 FLAG_TILE_256X128_PAIR = 4096
 FLAG_GQ_DIRECT = 1  # mi355_w8a8_gq_problem.flags
+FLAG_GQ_BF16_SCALES = 2  # mi355_w8a8_gq_bwd_problem.flags
 STATIC_WORKSPACE_BYTES = 32 << 20
 PATH_NAMES = {1: "skinny", 2: "skinny-chunks", 3: "tiled-256x128", 4: "tiled-256x256", 5: "tiled-128x128",
               6: "tiled-256x128-pair"}
@@ -51,7 +52,7 @@ EXPORTS = (
     "mi355_w8a8_moe_route_v1", "mi355_w8a8_moe_route_bwd_v1", "mi355_w8a8_moe_dispatch_workspace_bytes", "mi355_w8a8_moe_dispatch_v1",
     "mi355_w8a8_moe_combine_v1", "mi355_w8a8_moe_combine_bwd_v1",
     "mi355_w8a8_gq_packed_weight_bytes", "mi355_w8a8_gq_pack_weight_v1", "mi355_w8a8_gq_workspace_bytes",
-    "mi355_w8a8_gq_linear_v1",
+    "mi355_w8a8_gq_linear_v1", "mi355_w8a8_gq_bwd_workspace_bytes", "mi355_w8a8_gq_linear_bwd_v1",
     "mi355_w8a8_forward_path", "mi355_w8a8_calibrate_operand_bytes", "mi355_w8a8_calibrate_mfma_ops", "mi355_w8a8_calibrate_mfma_v1",
     "mi355_w8a8_calibrate_read_v1", "mi355_w8a8_calibrate_copy_v1",
 )
@@ -157,6 +158,18 @@ class GqProblem(ctypes.Structure):
     ]
 
 
+class GqBwdProblem(ctypes.Structure):
+    """struct mi355_w8a8_gq_bwd_problem"""
+
+    _fields_ = [
+        ("struct_size", _u32), ("flags", _u32), ("m", _u32), ("k", _u32), ("k_pad", _u32), ("n", _u32),
+        ("group_size", _u32), ("weight_bits", _u32), ("rank", _u32), ("reserved", _u32),
+        ("x", _vp), ("dy", _vp), ("w_packed", _vp), ("w_scales", _vp), ("lora_a", _vp), ("lora_b", _vp),
+        ("lora_scaling", _vp), ("dx", _vp), ("d_lora_a", _vp), ("d_lora_b", _vp), ("d_lora_scaling", _vp),
+        ("workspace", _vp), ("workspace_bytes", _u64),
+    ]
+
+
 class NativeError(RuntimeError):
     def __init__(self, fn: str, status: int, detail: str):
         super().__init__(f"{fn} failed: {STATUS.get(status, status)} ({detail})")
@@ -228,6 +241,10 @@ def _bind(lib: ctypes.CDLL) -> None:
     lib.mi355_w8a8_gq_workspace_bytes.argtypes = (_u32, _u32, _u32, _u32, _u32)
     lib.mi355_w8a8_gq_linear_v1.restype = ctypes.c_int
     lib.mi355_w8a8_gq_linear_v1.argtypes = (ctypes.POINTER(GqProblem), _vp)
+    lib.mi355_w8a8_gq_bwd_workspace_bytes.restype = _u64
+    lib.mi355_w8a8_gq_bwd_workspace_bytes.argtypes = (_u32,) * 6
+    lib.mi355_w8a8_gq_linear_bwd_v1.restype = ctypes.c_int
+    lib.mi355_w8a8_gq_linear_bwd_v1.argtypes = (ctypes.POINTER(GqBwdProblem), _vp)
     lib.mi355_w8a8_forward_path.restype = ctypes.c_int
     lib.mi355_w8a8_forward_path.argtypes = (_u32, _u32, _u32, _u32)
     lib.mi355_w8a8_calibrate_operand_bytes.restype = _u64

@@ -17,6 +17,7 @@
 #include "w8a8_fused_bwd.h"
 #include "w8a8_moe.h"
 #include "w8a8_gq.h"
+#include "w8a8_gq_bwd.h"
 
 using namespace w8a8;
 
@@ -765,7 +766,8 @@ struct BwdDxSplit { uint32_t direct_tiles, sk_q, sk_wgs; };
 // N = 10240 (80 tiles of 320 stages) 339 us whole, 135 + 22 us split; 3003 x 4096, N = 24576 (192 of 768) 800 us and 657 + 29 us.
 // Calls of fewer than 64 stages (N < 2048) stay whole: little to gain, and a grouped call over the same rows
 // then gives the same bits.
-BwdDxSplit bwd_dx_split(uint32_t tiles_m, uint32_t tiles_k, uint32_t NB) {
+// k_blocks: k blocks of a wave's tile (2; 1 in the group-scaled kernel, whose partial tiles are half the size).
+BwdDxSplit bwd_dx_split(uint32_t tiles_m, uint32_t tiles_k, uint32_t NB, uint32_t k_blocks = 2u) {
   const uint32_t ntile = tiles_m * tiles_k, rem = ntile % 256u;
   BwdDxSplit best{ntile, 0u, 0u};
   if (rem == 0u || NB < 64u) return best;
@@ -773,7 +775,7 @@ BwdDxSplit bwd_dx_split(uint32_t tiles_m, uint32_t tiles_k, uint32_t NB) {
   for (uint32_t wgs = 64u; wgs <= 256u; wgs += 64u) {
     uint32_t q = (rem * NB + wgs - 1u) / wgs;
     q = round_up(q < 16u ? 16u : q, 2u);
-    const double c = q + 0.11 * (wgs + rem) + 8.0;
+    const double c = q + 0.055 * k_blocks * (wgs + rem) + 8.0;
     if (c < cost) {
       cost = c;
       best.direct_tiles = ntile - rem; best.sk_q = q;
@@ -790,13 +792,14 @@ struct BwdLayout {
   uint32_t slots, nkk, K_pad, KB, N_pad, NB, tiles_m, tiles_k, max_chunks, R, n_slices, groups_per_slice;
 };
 
-BwdLayout make_bwd_layout(uint32_t m, uint32_t k, uint32_t n, uint32_t n_groups, uint32_t rank) {
+// gq_k_pad: padded K of a group-scaled weight (its own k blocks, tiles of 128 k), or 0
+BwdLayout make_bwd_layout(uint32_t m, uint32_t k, uint32_t n, uint32_t n_groups, uint32_t rank, uint32_t gq_k_pad = 0u) {
   BwdLayout w{};
-  w.K_pad = k_padded(k); w.KB = w.K_pad / 32u;
+  w.K_pad = gq_k_pad ? gq_k_pad : k_padded(k); w.KB = w.K_pad / 32u;
   w.N_pad = n_padded(n); w.NB = w.N_pad / 32u;
   w.slots = round_up(m, kTileM);
   w.tiles_m = w.slots / 256u;
-  w.tiles_k = (w.K_pad + 255u) / 256u;
+  w.tiles_k = gq_k_pad ? (w.K_pad + 127u) / 128u : (w.K_pad + 255u) / 256u;
   w.nkk = rank_chunks(rank);
   w.R = w.nkk > 2u ? 64u : 32u;  // rank rows of a partial (32-wide rank blocks)
   w.max_chunks = (m + kBwdChunkRows - 1u) / kBwdChunkRows + n_groups;
@@ -805,9 +808,9 @@ BwdLayout make_bwd_layout(uint32_t m, uint32_t k, uint32_t n, uint32_t n_groups,
     w.n_slices = (ng + 3u) / 4u < 8u ? (ng + 3u) / 4u : 8u;
     w.groups_per_slice = (ng + w.n_slices - 1u) / w.n_slices;
   }
-  w.split = bwd_dx_split(w.tiles_m, w.tiles_k, w.NB);
+  w.split = bwd_dx_split(w.tiles_m, w.tiles_k, w.NB, gq_k_pad ? 1u : 2u);
   uint64_t off = 0;
-  w.part = off; off += (uint64_t)w.split.sk_wgs * 2u * kBwdPartFloats * 4u;
+  w.part = off; off += (uint64_t)w.split.sk_wgs * 2u * kBwdPartFloats * 2u * 4u;
   w.dyp = off; off += align256((uint64_t)w.slots * w.N_pad * 2u);
   w.swp = off; off += align256((uint64_t)(w.N_pad + kBwdScalePad) * 4u);  // a stage fetches 1 KiB of scales starting at its own 32
   w.src_row = off; off += align256((uint64_t)w.slots * 4u);
@@ -852,7 +855,7 @@ int launch_bwd_dx_geometry(const BwdDxArgs& g, hipStream_t s) {
   if (!g.sk_wgs) return launch_status();
   if (const int st = launch_status()) return st;
   const uint32_t split_tiles = g.tiles_m * g.tiles_k - g.direct_tiles;
-  hipLaunchKernelGGL((bwd_dx_finish_kernel<NKK>), dim3(split_tiles * 8u), dim3(256), 0, s, g);
+  hipLaunchKernelGGL((bwd_dx_finish_kernel<NKK, 2>), dim3(split_tiles * 8u), dim3(256), 0, s, g);
   return launch_status();
 }
 
@@ -879,7 +882,30 @@ struct BwdBody {
   size_t w_stride; uint32_t sw_stride;
   bool rows128;  // the pull-back runs 128-row x 512-k tiles (the tables are padded to match)
   BwdDxSplit split; uint64_t part;  // dense calls
+  // group-scaled weights: their format (weight_bits 0: per-channel)
+  uint32_t weight_bits, group, terms; const float* w_scales;
 };
+
+template <bool W4, int TERMS, int NKK>
+int launch_gq_bwd_dx_one(const GqBwdDxArgs& a, hipStream_t s) {
+  const BwdDxArgs& g = a.g;
+  uint32_t want = ((g.direct_tiles + 7u) / 8u) * 8u;
+  if (g.sk_wgs > want) want = g.sk_wgs;
+  const dim3 grid(want < 256u ? want : 256u), block(512);
+  if (hipFuncSetAttribute(reinterpret_cast<const void*>(&gq_bwd_dx_kernel<W4, TERMS, NKK>),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, kGqBwdLdsBytes) != hipSuccess)
+    return MI355_W8A8_ERR_LAUNCH;
+  hipLaunchKernelGGL((gq_bwd_dx_kernel<W4, TERMS, NKK>), grid, block, kGqBwdLdsBytes, s, a);
+  if (!g.sk_wgs) return launch_status();
+  if (const int st = launch_status()) return st;
+  hipLaunchKernelGGL((bwd_dx_finish_kernel<NKK, 1>), dim3((g.tiles_m * g.tiles_k - g.direct_tiles) * 8u), dim3(256), 0, s, g);
+  return launch_status();
+}
+template <int NKK>
+int launch_gq_bwd_dx(const GqBwdDxArgs& a, uint32_t bits, uint32_t terms, hipStream_t s) {
+  if (bits == 4u) return terms == 2u ? launch_gq_bwd_dx_one<true, 2, NKK>(a, s) : launch_gq_bwd_dx_one<true, 3, NKK>(a, s);
+  return terms == 2u ? launch_gq_bwd_dx_one<false, 2, NKK>(a, s) : launch_gq_bwd_dx_one<false, 3, NKK>(a, s);
+}
 
 template <class Layout>
 int launch_bwd_body(const BwdBody& b, const Layout& w, unsigned char* ws, hipStream_t s) {
@@ -894,7 +920,11 @@ int launch_bwd_body(const BwdBody& b, const Layout& w, unsigned char* ws, hipStr
     d.M = b.m; d.N = b.n; d.NB = w.NB; d.n_row_blocks = w.slots / 32u; d.n_col_groups = w.N_pad / 128u;
     d.n_slices = w.n_slices; d.groups_per_slice = w.groups_per_slice; d.r = b.rank; d.slots = w.slots;
     const dim3 grid(d.n_row_blocks * d.n_slices), block(256);
-    if (!b.lora) hipLaunchKernelGGL((bwd_pack_dy_kernel<0>), grid, block, 0, s, d);
+    if (b.weight_bits) {
+      if (!b.lora) hipLaunchKernelGGL((gq_bwd_pack_dy_kernel<0>), grid, block, 0, s, d);
+      else if (w.nkk > 2u) hipLaunchKernelGGL((gq_bwd_pack_dy_kernel<2>), grid, block, 0, s, d);
+      else hipLaunchKernelGGL((gq_bwd_pack_dy_kernel<1>), grid, block, 0, s, d);
+    } else if (!b.lora) hipLaunchKernelGGL((bwd_pack_dy_kernel<0>), grid, block, 0, s, d);
     else if (w.nkk > 2u) hipLaunchKernelGGL((bwd_pack_dy_kernel<2>), grid, block, 0, s, d);
     else hipLaunchKernelGGL((bwd_pack_dy_kernel<1>), grid, block, 0, s, d);
     if ((st = launch_status())) return st;
@@ -961,7 +991,17 @@ int launch_bwd_body(const BwdBody& b, const Layout& w, unsigned char* ws, hipStr
     g.direct_tiles = b.split.sk_wgs ? b.split.direct_tiles : w.tiles_m * w.tiles_k;
     g.sk_q = b.split.sk_q; g.sk_wgs = b.split.sk_wgs;
     g.part = b.split.sk_wgs ? reinterpret_cast<float*>(ws + b.part) : nullptr;
-    switch (b.lora ? w.nkk : 0u) {
+    if (b.weight_bits) {
+      GqBwdDxArgs a{};
+      a.g = g;
+      a.ws = b.w_scales; a.N = b.n; a.group = b.group; a.weight_nb = (b.n + 31u) / 32u;
+      switch (b.lora ? w.nkk : 0u) {
+        case 0: st = launch_gq_bwd_dx<0>(a, b.weight_bits, b.terms, s); break;
+        case 1: st = launch_gq_bwd_dx<1>(a, b.weight_bits, b.terms, s); break;
+        case 2: st = launch_gq_bwd_dx<2>(a, b.weight_bits, b.terms, s); break;
+        default: st = launch_gq_bwd_dx<4>(a, b.weight_bits, b.terms, s); break;
+      }
+    } else switch (b.lora ? w.nkk : 0u) {
       case 0: st = launch_bwd_dx<0>(g, b.rows128, s); break;
       case 1: st = launch_bwd_dx<1>(g, b.rows128, s); break;
       case 2: st = launch_bwd_dx<2>(g, b.rows128, s); break;
@@ -1085,6 +1125,71 @@ int run_backward(const mi355_w8a8_bwd_problem* p, hipStream_t s) {
   b.blk_range = routed ? blk_range : nullptr;
   b.group_off = group_off;
   b.split = w.split; b.part = w.part;
+  return launch_bwd_body(b, w, ws, s);
+}
+
+// group-scaled weights: the same stages around the group-scaled pull-back, one adapter
+int validate_gq_bwd_dims(uint32_t m, uint32_t k, uint32_t k_pad, uint32_t n, uint32_t group, uint32_t rank) {
+  if (m == 0 || k == 0 || n == 0 || k > k_pad) return MI355_W8A8_ERR_SHAPE;
+  if (group == 0 || group % 32u || k_pad % group) return MI355_W8A8_ERR_SHAPE;
+  if (m > kMaxRows || n > kMaxN || k_pad > kMaxK || k % 8u || n % 8u || rank > (uint32_t)kMaxRank) return MI355_W8A8_ERR_UNSUPPORTED;
+  const uint64_t limit = (1ull << 32) - (1ull << 20);  // 32-bit offsets
+  if ((uint64_t)m * k >= limit || (uint64_t)m * n >= limit) return MI355_W8A8_ERR_UNSUPPORTED;
+  return MI355_W8A8_OK;
+}
+
+int run_gq_backward(const mi355_w8a8_gq_bwd_problem* p, hipStream_t s) {
+  if (!p) return MI355_W8A8_ERR_NULL;
+  if (p->struct_size != sizeof(mi355_w8a8_gq_bwd_problem)) return MI355_W8A8_ERR_STRUCT;
+  int st = validate_gq_bwd_dims(p->m, p->k, p->k_pad, p->n, p->group_size, p->rank);
+  if (st) return st;
+  if (p->flags & ~(MI355_W8A8_FLAG_SKIP_GEMM | MI355_W8A8_FLAG_GQ_BF16_SCALES)) return MI355_W8A8_ERR_SHAPE;
+  if (p->weight_bits != 4u && p->weight_bits != 8u) return MI355_W8A8_ERR_SHAPE;
+  const bool no_dx = (p->flags & MI355_W8A8_FLAG_SKIP_GEMM) != 0;
+  if (!p->dy || !p->w_packed || !p->w_scales || (!p->dx && !no_dx)) return MI355_W8A8_ERR_NULL;
+  const bool lora = p->rank > 0;
+  const bool want_grads = p->d_lora_a || p->d_lora_b || p->d_lora_scaling;
+  if (lora) {
+    if (!p->lora_a || !p->lora_b || !p->lora_scaling) return MI355_W8A8_ERR_NULL;
+    if (want_grads && !p->x) return MI355_W8A8_ERR_NULL;
+  } else if (want_grads) {
+    return MI355_W8A8_ERR_SHAPE;
+  }
+  if (!aligned16(p->x) || !aligned16(p->dy) || !aligned16(p->w_packed) || !aligned16(p->w_scales) ||
+      !aligned16(p->lora_a) || !aligned16(p->lora_b) || !aligned16(p->dx) || !aligned16(p->d_lora_a) || !aligned16(p->d_lora_b))
+    return MI355_W8A8_ERR_ALIGN;
+  const uint64_t dx_bytes = (uint64_t)p->m * p->k * 2u;
+  if (!no_dx && (overlaps(p->dx, dx_bytes, p->dy, (uint64_t)p->m * p->n * 2u) || overlaps(p->dx, dx_bytes, p->x, dx_bytes) ||
+                 overlaps(p->dx, dx_bytes, p->workspace, p->workspace_bytes)))
+    return MI355_W8A8_ERR_ALIAS;
+  const BwdLayout w = make_bwd_layout(p->m, p->k, p->n, lora ? 1u : 0u, p->rank, p->k_pad);
+  if (!p->workspace || p->workspace_bytes < w.total) return MI355_W8A8_ERR_WORKSPACE;
+  if (reinterpret_cast<uintptr_t>(p->workspace) & 255u) return MI355_W8A8_ERR_ALIGN;
+  unsigned char* ws = static_cast<unsigned char*>(p->workspace);
+  (void)hipGetLastError();
+  if (lora) {  // A transposed and in operand order, the group table
+    BwdPrepArgs pa{};
+    pa.group_off = reinterpret_cast<int32_t*>(ws + w.group_off);
+    pa.lora_a = static_cast<const uint16_t*>(p->lora_a);
+    pa.at = reinterpret_cast<uint16_t*>(ws + w.at);
+    pa.ap = ws + w.ap;
+    pa.M = p->m; pa.K = p->k; pa.n_groups = 1u; pa.r = p->rank;
+    pa.nkk = w.nkk; pa.kb32 = w.KB; pa.slots = w.slots;
+    pa.route_blocks = 1u;
+    pa.a_blocks = (uint32_t)(((uint64_t)p->k * ((p->rank + 7u) / 8u) + 1023u) / 1024u);
+    pa.ap_blocks = (uint32_t)(((uint64_t)w.KB * w.nkk * 64u + 1023u) / 1024u);
+    hipLaunchKernelGGL(bwd_prep_kernel, dim3(pa.route_blocks + pa.a_blocks + pa.ap_blocks), dim3(1024), 0, s, pa);
+    if ((st = launch_status())) return st;
+  }
+  BwdBody b{};
+  b.m = p->m; b.k = p->k; b.n = p->n; b.n_groups = lora ? 1u : 0u; b.rank = p->rank;
+  b.x = p->x; b.dy = p->dy; b.w_packed = p->w_packed; b.lora_b = p->lora_b; b.lora_scaling = p->lora_scaling;
+  b.dx = p->dx; b.d_lora_a = p->d_lora_a; b.d_lora_b = p->d_lora_b; b.d_lora_scaling = p->d_lora_scaling;
+  b.lora = lora; b.want_grads = want_grads; b.skip_gemm = no_dx;
+  b.group_off = reinterpret_cast<int32_t*>(ws + w.group_off);
+  b.split = w.split; b.part = w.part;
+  b.weight_bits = p->weight_bits; b.group = p->group_size; b.w_scales = p->w_scales;
+  b.terms = (p->flags & MI355_W8A8_FLAG_GQ_BF16_SCALES) ? 2u : 3u;
   return launch_bwd_body(b, w, ws, s);
 }
 
@@ -2100,6 +2205,16 @@ uint64_t mi355_w8a8_gq_workspace_bytes(uint32_t m, uint32_t k_pad, uint32_t grou
 
 int mi355_w8a8_gq_linear_v1(const mi355_w8a8_gq_problem* p, void* stream) {
   return run_gq_linear(p, static_cast<hipStream_t>(stream));
+}
+
+uint64_t mi355_w8a8_gq_bwd_workspace_bytes(uint32_t m, uint32_t k, uint32_t k_pad, uint32_t n, uint32_t group_size,
+                                           uint32_t rank) {
+  if (validate_gq_bwd_dims(m, k, k_pad, n, group_size, rank)) return 0;
+  return make_bwd_layout(m, k, n, rank ? 1u : 0u, rank, k_pad).total;
+}
+
+int mi355_w8a8_gq_linear_bwd_v1(const mi355_w8a8_gq_bwd_problem* p, void* stream) {
+  return run_gq_backward(p, static_cast<hipStream_t>(stream));
 }
 
 int mi355_w8a8_forward_path(uint32_t m, uint32_t k, uint32_t n, uint32_t flags) {

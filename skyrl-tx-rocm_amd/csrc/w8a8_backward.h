@@ -436,9 +436,9 @@ struct BwdDxArgs {
   // dense calls: the tiles from direct_tiles on are split (bwd_dx_split): sk_wgs workgroups take sk_q
   // consecutive stages each of their joint stage sequence and leave float32 partial tiles in part
   uint32_t direct_tiles, sk_q, sk_wgs;
-  float* part;   // [2 * sk_wgs slots][8 waves][4 row blocks][2 k blocks][4][64 lanes][4]
+  float* part;   // [2 * sk_wgs slots][8 waves][4 row blocks][k blocks of a wave][4][64 lanes][4]
 };
-constexpr uint32_t kBwdPartFloats = 65536;  // of a slot
+constexpr uint32_t kBwdPartFloats = 32768;  // of a slot, per k block of a wave
 
 // (row tile, k tile) of position t in the band-major tile order: 4 row tiles x all k tiles to a band
 __device__ inline void bwd_dx_tile_at(const BwdDxArgs& g, uint32_t t, uint32_t& tm, uint32_t& tk) {
@@ -448,10 +448,10 @@ __device__ inline void bwd_dx_tile_at(const BwdDxArgs& g, uint32_t t, uint32_t& 
   tk = in_band / band_rows;
 }
 
-// A wave's 32 x 64 block of dx: + rs @ A.T, one cast, rows back to their original positions.  pbase: first
-// slot of the block's 32; kbw: first of its two k blocks.
-template <int NKK>
-__device__ inline void bwd_dx_store_block(const BwdDxArgs& g, uint32_t pbase, uint32_t kbw, const v16f (&acc)[2]) {
+// A wave's block of dx, 32 rows x CBN k blocks: + rs @ A.T, one cast, rows back to their original positions.
+// pbase: first slot of the block's 32; kbw: first of its k blocks.
+template <int NKK, int CBN>
+__device__ inline void bwd_dx_store_block(const BwdDxArgs& g, uint32_t pbase, uint32_t kbw, const v16f (&acc)[CBN]) {
   const int lane = threadIdx.x & 63, c = lane & 31, h = lane >> 5;
   const uint32_t blk = pbase / 32u;
   const int src_lane = g.src_row ? g.src_row[pbase + c] : (int)(pbase + c);
@@ -464,7 +464,7 @@ __device__ inline void bwd_dx_store_block(const BwdDxArgs& g, uint32_t pbase, ui
   const int row_addr = 16 * h;
   for (int gi = glo; gi <= ghi; ++gi) {  // a block at a group boundary runs once per group
 #pragma unroll
-    for (int cb = 0; cb < 2; ++cb) {
+    for (int cb = 0; cb < CBN; ++cb) {
       const uint32_t kb = kbw + cb;
       if (kb >= g.KB) continue;  // wave-uniform
       const uint32_t kcol = kb * 32u + c;
@@ -732,9 +732,9 @@ __global__ __launch_bounds__(512, 1) void bwd_dx_kernel(BwdDxArgs g) {
 #pragma unroll
       for (int rb = 0; rb < 4; ++rb)
         if (rb < n_act)
-          bwd_dx_store_block<NKK>(g, tm * (uint32_t)(kRowBlocks * 32) + (uint32_t)wrow * 128u + rb * 32u, kbw, acc[rb]);
+          bwd_dx_store_block<NKK, 2>(g, tm * (uint32_t)(kRowBlocks * 32) + (uint32_t)wrow * 128u + rb * 32u, kbw, acc[rb]);
     } else {
-      float4* dst = reinterpret_cast<float4*>(g.part + (size_t)slot * kBwdPartFloats) + (uint32_t)wave * 2048u + lane;
+      float4* dst = reinterpret_cast<float4*>(g.part + (size_t)slot * (2u * kBwdPartFloats)) + (uint32_t)wave * 2048u + lane;
 #pragma unroll
       for (int rb = 0; rb < 4; ++rb)
         if (rb < n_act)
@@ -797,9 +797,9 @@ __global__ __launch_bounds__(512, 1) void bwd_dx_kernel(BwdDxArgs g) {
   }
 }
 
-// The split tiles of bwd_dx_kernel: the partial sums of a tile added in the order of its stages, then the
-// kernel's own epilogue.  A wave per 32 x 64 block.
-template <int NKK>
+// The split tiles of a pull-back kernel: the partial sums of a tile added in the order of its stages, then the
+// kernel's own epilogue.  A wave per block of 32 rows x CBN k blocks (CBN: k blocks of a wave's tile).
+template <int NKK, int CBN>
 __global__ __launch_bounds__(256) void bwd_dx_finish_kernel(BwdDxArgs g) {
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t item = blockIdx.x * 4u + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -809,25 +809,25 @@ __global__ __launch_bounds__(256) void bwd_dx_finish_kernel(BwdDxArgs g) {
   uint32_t tm, tk;
   bwd_dx_tile_at(g, g.direct_tiles + u, tm, tk);
   const uint32_t pbase = tm * 256u + (wave >> 2) * 128u + rb * 32u;
-  const uint32_t kbw = tk * 8u + (wave & 3u) * 2u;
+  const uint32_t kbw = (tk * 4u + (wave & 3u)) * (uint32_t)CBN;
   if (pbase >= g.M || kbw >= g.KB) return;
-  v16f y[2];
+  v16f y[CBN];
 #pragma unroll
-  for (int cb = 0; cb < 2; ++cb)
+  for (int cb = 0; cb < CBN; ++cb)
 #pragma unroll
     for (int e = 0; e < 16; ++e) y[cb][e] = 0.0f;
   for (uint32_t w = first; w <= last; ++w) {
     const uint32_t slot = 2u * w + (w * g.sk_q / g.NB == u ? 0u : 1u);
-    const float4* src = reinterpret_cast<const float4*>(g.part + (size_t)slot * kBwdPartFloats) + wave * 2048u + rb * 512u + lane;
+    const float4* src = reinterpret_cast<const float4*>(g.part) + ((size_t)slot * 32u + wave * 4u + rb) * (256u * CBN) + lane;
 #pragma unroll
-    for (int cb = 0; cb < 2; ++cb)
+    for (int cb = 0; cb < CBN; ++cb)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const float4 v = src[(cb * 4 + e) * 64];
         y[cb][4 * e] += v.x; y[cb][4 * e + 1] += v.y; y[cb][4 * e + 2] += v.z; y[cb][4 * e + 3] += v.w;
       }
   }
-  bwd_dx_store_block<NKK>(g, pbase, kbw, y);
+  bwd_dx_store_block<NKK, CBN>(g, pbase, kbw, y);
 }
 
 // ---------------------------------------------------------------------------------------

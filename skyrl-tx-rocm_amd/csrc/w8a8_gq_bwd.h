@@ -1,0 +1,369 @@
+// Backward of the group-scaled linear (W4 or W8 codes, one scale per K group and output):
+//   dx = dy @ deq(W).T + rs @ A.T    rs = (dy @ B.T) * s      deq(W)[k, n] = float32(code * scale[g(k), n])
+// and the LoRA cotangents of w8a8_backward.h (skyrl/tx/kernels/quantized_lora.py:337-394).  The rule there is
+// float32 throughout; on the matrix core a float32 weight value is carried as its exact split into bf16
+// terms, so that every product dy * deq(W) is exact and only float32 sums round, as in a float32 GEMM:
+//   two terms when the scales are bf16 values (a code of at most 8 bits times 8 bits), three otherwise.
+//
+//   gq_bwd_pack_dy_kernel  dy in operand order, and the partial sums of r = dy @ B.T
+//   gq_bwd_dx_kernel       the pull-back
+// The rest (tables, r / z finish, LoRA cotangents) is the per-channel backward's.
+#pragma once
+#include "w8a8_backward.h"
+#include "w8a8_gq.h"
+
+namespace w8a8 {
+
+// dy in MFMA A-operand order: dyp[row block][n block][q][64 lanes][8 bf16]: lane (i = l % 32, h = l / 32) element e
+// of (n block nb, q) holds column 32 nb + 16 q + 8 (e / 4) + 4 h + e % 4, the n that the transposing MFMA
+// leaves in contraction slot 8 h + e of its q-th half.  (bwd_pack_dy_kernel without the packed weight's column
+// permutation.)  A lane loads 8 consecutive columns of its row, h of its 16, and the two halves of the wave
+// exchange four of them.
+template <int RB>  // 32-wide rank blocks (0 = packing only)
+__global__ __launch_bounds__(256) void gq_bwd_pack_dy_kernel(BwdPackDyArgs a) {
+  constexpr int kRB = RB > 0 ? RB : 1;
+  __shared__ float red[4][kRB][16][64];
+  const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t mb = blockIdx.x / a.n_slices, sl = blockIdx.x % a.n_slices;
+  if (mb >= a.n_row_blocks) return;
+  const uint32_t i = lane & 31u, h = lane >> 5;
+  const uint32_t row = mb * 32u + i;
+  v16f acc[kRB];
+#pragma unroll
+  for (int b = 0; b < kRB; ++b)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[b][e] = 0.0f;
+  const uint32_t per = (a.NB + a.n_slices - 1u) / a.n_slices;
+  const uint32_t nb1 = (sl + 1u) * per < a.NB ? (sl + 1u) * per : a.NB;
+  const uint16_t* const dyr = a.dy + (size_t)(row < a.M ? row : 0u) * a.N;
+  // 16 columns in operand order; loads whatever the condition (a load under one becomes a branch with a wait)
+  auto fetch = [&](const uint16_t* r, bool live, uint32_t col) -> v8us {
+    const bool in = live && col < a.N;
+    const v4i raw = *reinterpret_cast<const v4i*>(r + (col < a.N ? col : 0u));
+    const v4i z = in ? raw : v4i{0, 0, 0, 0};
+    const auto s0 = __builtin_amdgcn_permlane32_swap(z[0], z[2], false, false);
+    const auto s1 = __builtin_amdgcn_permlane32_swap(z[1], z[3], false, false);
+    return __builtin_bit_cast(v8us, v4i{(int)s0[0], (int)s1[0], (int)s0[1], (int)s1[1]});
+  };
+  for (uint32_t nb = sl * per + wave; nb < nb1; nb += 4u) {
+    v8us pc[2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) pc[q] = fetch(dyr, row < a.M, 32u * nb + 16u * q + 8u * h);
+    v8us wb[kRB][2];
+    if constexpr (RB > 0) {
+#pragma unroll
+      for (int b = 0; b < RB; ++b) {
+        const uint32_t j = b * 32u + i;
+#pragma unroll
+        for (int q = 0; q < 2; ++q) wb[b][q] = fetch(a.lora_b + (size_t)(j < a.r ? j : 0u) * a.N, j < a.r, 32u * nb + 16u * q + 8u * h);
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      *reinterpret_cast<v8us*>(a.dyp + ((((size_t)mb * a.NB + nb) * 2u + q) * 64u + lane) * 16u) = pc[q];
+      if constexpr (RB > 0) {
+#pragma unroll
+        for (int b = 0; b < RB; ++b)
+          acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, pc[q]), __builtin_bit_cast(v8bf, wb[b][q]), acc[b], 0, 0, 0);
+      }
+    }
+  }
+  if constexpr (RB > 0) {
+#pragma unroll
+    for (int b = 0; b < RB; ++b)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) red[wave][b][e][lane] = acc[b][e];
+    __syncthreads();
+    for (uint32_t q = threadIdx.x; q < RB * 1024u; q += 256u) {
+      const uint32_t l = q & 63u, e = (q >> 6) & 15u, b = q >> 10;
+      const float sum = ((red[0][b][e][l] + red[1][b][e][l]) + red[2][b][e][l]) + red[3][b][e][l];
+      const uint32_t r = 8u * (e >> 2) + 4u * (l >> 5) + (e & 3u), col = b * 32u + (l & 31u);
+      a.rpart[((size_t)sl * a.slots + mb * 32u + r) * kBwdRankStride + col] = sum;
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------------------
+// The pull-back.  Workgroup = 8 waves (2 along rows x 4 along k), tile 256 rows x 128 k, wave tile 128 x 32
+// (4 accumulator blocks of v_mfma_f32_32x32x16_bf16), contraction in stages of one 32-wide n block.  A stage's
+// dy panel (16 KiB), its four weight blocks (4 KiB, half that in 4-bit codes) and their scales (128 bytes a block)
+// travel L2 -> LDS with direct-to-LDS loads six stages ahead, three per wave.  While the matrix core works on
+// a stage, each wave prepares its weight block of the next: transposed by the identity MFMA, scaled in float32,
+// split into TERMS bf16 operands.  The schedule is bwd_dx_kernel's; half its k per wave leaves the registers for
+// the terms, and a stage has as many MFMAs (TERMS = 2) for half the tile.
+// Bound by the matrix core and the term arithmetic beside it: 1536 rows, K = 12288, N = 4096, 8-bit codes, groups of
+// 64: 352 us (0.88 PFLOP/s of bf16 products in two terms) where the float32 library GEMM took 1096 us and the
+// dequantization and casts before it 250.
+// ---------------------------------------------------------------------------------------
+constexpr int kGqBwdStages = 7;
+constexpr int kGqBwdAhead = kGqBwdStages - 1;
+constexpr int kGqBwdPanel = 16384, kGqBwdWeight = 4096;
+constexpr int kGqBwdStageBytes = kGqBwdPanel + kGqBwdWeight + 1024;
+constexpr int kGqBwdLdsBytes = kGqBwdStages * kGqBwdStageBytes;
+constexpr int kGqBwdLoads = 3;  // per wave and stage: 2 panel chunks, and weight blocks or scales
+
+struct GqBwdDxArgs {
+  BwdDxArgs g;          // wp: packed codes; KB: k blocks (k_pad / 32); NB: n blocks of dyp (even)
+  const float* ws;      // f32 [k_pad / group, N]
+  uint32_t N, group, weight_nb;  // weight_nb: n blocks of the packed weight
+};
+
+template <bool W4, int TERMS, int NKK>
+__global__ __launch_bounds__(512, 1) void gq_bwd_dx_kernel(GqBwdDxArgs a) {
+  const BwdDxArgs& g = a.g;
+  extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wrow = wave >> 2, wcol = wave & 3;
+  const int c = lane & 31, h = lane >> 5;
+  const uint32_t lds_base = (uint32_t)(uintptr_t)(lptr_t)lds;
+  constexpr uint32_t kBlk8 = W4 ? 512u : 1024u;  // bytes of a weight block
+
+  // identity operand of the transposing MFMA: lane (column c, k half h) holds byte 1 at k == c
+  v4i ident = {0, 0, 0, 0};
+  {
+    const int word = ((c >> 4) == h) ? (int)(1u << (8 * (c & 3))) : 0;
+    const int wi = (c & 15) >> 2;
+    ident[0] = wi == 0 ? word : 0; ident[1] = wi == 1 ? word : 0;
+    ident[2] = wi == 2 ? word : 0; ident[3] = wi == 3 ? word : 0;
+  }
+
+  auto segment = [&](uint32_t tm, uint32_t tk, int nb0, int L, bool whole, uint32_t slot) {
+    int n_act = ((int)(g.M - tm * 256u) + 31) / 32 - wrow * 4;  // the wave's row blocks with rows
+    n_act = __builtin_amdgcn_readfirstlane(n_act < 0 ? 0 : (n_act > 4 ? 4 : n_act));
+    const unsigned char* panel = g.dyp + ((size_t)(tm * 8u + (uint32_t)wave) * g.NB) * 2048u + lane * 16;
+    const uint32_t kb0 = tk * 4u;
+    auto clamp_kb = [&](uint32_t kb) { return kb < g.KB ? kb : g.KB - 1u; };
+    // what this wave fetches beside the panel: waves 0..3 the weight blocks (one each, or in 4-bit codes two
+    // of 512 bytes, waves 2 and 3 repeating 0 and 1), waves 4..7 the four blocks' scales (each all of them, to
+    // the same place)
+    uint32_t w_off, w_dst;  // of waves 0..3: byte offset inside an n block's row of blocks
+    if (W4) {
+      w_off = clamp_kb(kb0 + 2u * (wave & 1) + (uint32_t)h) * 512u + (lane & 31) * 16u;
+      w_dst = (wave & 1) * 1024u;
+    } else {
+      w_off = clamp_kb(kb0 + (wave & 3)) * 1024u + lane * 16u;
+      w_dst = (wave & 3) * 1024u;
+    }
+    const uint32_t s_piece = (lane & 7) * 4u;
+    const float* s_row = a.ws + (size_t)(clamp_kb(kb0 + ((lane >> 3) & 3)) * 32u / a.group) * a.N;
+    auto issue = [&](int i) {  // stage i of the segment
+      const uint32_t st = lds_base + (i % kGqBwdStages) * kGqBwdStageBytes;
+      const uint32_t nb = (uint32_t)(nb0 + i);
+      unsigned char* St = lds + (i % kGqBwdStages) * kGqBwdStageBytes;
+      (void)st;
+      load_1k_to_lds(panel + (size_t)nb * 2048u, St + (wave * 2) * kBlockBytes);
+      load_1k_to_lds(panel + (size_t)nb * 2048u + 1024u, St + (wave * 2 + 1) * kBlockBytes);
+      if (wave < 4) {
+        const uint32_t nbw = nb < a.weight_nb ? nb : a.weight_nb - 1u;  // (dy is zero beyond the last column)
+        load_1k_to_lds(g.wp + (size_t)nbw * g.KB * kBlk8 + w_off, St + kGqBwdPanel + w_dst);
+      } else {
+        const uint32_t n = nb * 32u + s_piece;
+        load_1k_to_lds(reinterpret_cast<const unsigned char*>(s_row + (n < a.N ? n : 0u)), St + kGqBwdPanel + kGqBwdWeight);
+      }
+    };
+
+    v16f acc[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][e] = 0.0f;
+
+    // explicit LDS reads: a compiler-visible one of memory that direct-to-LDS loads write would drain every
+    // load in flight first; the values are valid after next_wait()
+    struct NextRegs { v4i raw; v4f s4[4]; };
+    auto next_read = [&](int i, NextRegs& r) {
+      const uint32_t st = lds_base + (i % kGqBwdStages) * kGqBwdStageBytes + kGqBwdPanel;
+      const uint32_t sa = st + kGqBwdWeight + wcol * 128 + 16 * h;
+      if constexpr (W4) {
+        const uint32_t wa = st + wcol * 512 + lane * 8;
+        uint2 raw;
+        asm volatile("ds_read_b64 %0, %5\n\tds_read_b128 %1, %6\n\tds_read_b128 %2, %6 offset:32\n\t"
+                     "ds_read_b128 %3, %6 offset:64\n\tds_read_b128 %4, %6 offset:96"
+                     : "=&v"(raw), "=&v"(r.s4[0]), "=&v"(r.s4[1]), "=&v"(r.s4[2]), "=&v"(r.s4[3])
+                     : "v"(wa), "v"(sa) : "memory");
+        asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(raw), "+v"(r.s4[0]), "+v"(r.s4[1]), "+v"(r.s4[2]), "+v"(r.s4[3]) : : "memory");
+        GqRawFragment<true> f;
+        f.v = make_uint4(raw.x, raw.y, 0u, 0u);
+        r.raw = gq_expand<true>(f);  // 16 * code; the scale takes the exact 1 / 16
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) r.s4[q][e] = r.s4[q][e] * 0.0625f;
+      } else {
+        const uint32_t wa = st + wcol * 1024 + lane * 16;
+        asm volatile("ds_read_b128 %0, %5\n\tds_read_b128 %1, %6\n\tds_read_b128 %2, %6 offset:32\n\t"
+                     "ds_read_b128 %3, %6 offset:64\n\tds_read_b128 %4, %6 offset:96"
+                     : "=&v"(r.raw), "=&v"(r.s4[0]), "=&v"(r.s4[1]), "=&v"(r.s4[2]), "=&v"(r.s4[3])
+                     : "v"(wa), "v"(sa) : "memory");
+        asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(r.raw), "+v"(r.s4[0]), "+v"(r.s4[1]), "+v"(r.s4[2]), "+v"(r.s4[3]) : : "memory");
+      }
+    };
+    auto transpose_block = [&](const v4i& rawb) -> v16i {
+      v16i z16;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) z16[e] = 0;
+      return __builtin_amdgcn_mfma_i32_32x32x32_i8(rawb, ident, z16, 0, 0, 0);
+    };
+    // rows 8 gq + 4 h + 0..3 of a transposed block: code * scale in float32, split into TERMS bf16 values
+    auto convert4 = [&](const v16i& tr, const v4f& s4, int gq, uint32_t (&pk)[TERMS][8]) {
+      float f[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) f[e] = (float)tr[4 * gq + e] * s4[e];
+#pragma unroll
+      for (int t = 0; t < TERMS; ++t)
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+          const uint32_t w = pack_bf16x2(f[2 * p], f[2 * p + 1]);
+          pk[t][2 * gq + p] = w;
+          if (t + 1 < TERMS) {
+            f[2 * p] = f[2 * p] - __uint_as_float(w << 16);
+            f[2 * p + 1] = f[2 * p + 1] - __uint_as_float(w & 0xffff0000u);
+          }
+        }
+    };
+    auto to_operands = [&](const uint32_t (&pk)[TERMS][8], v8bf (&bq)[2][TERMS]) {
+#pragma unroll
+      for (int t = 0; t < TERMS; ++t)
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+          bq[q][t] = __builtin_bit_cast(v8bf, v4i{(int)pk[t][4 * q], (int)pk[t][4 * q + 1], (int)pk[t][4 * q + 2], (int)pk[t][4 * q + 3]});
+    };
+    auto panel_frag = [&](int i, int pair) -> v8bf {  // pair = 4 q + row block
+      const unsigned char* St = lds + (i % kGqBwdStages) * kGqBwdStageBytes;
+      return __builtin_bit_cast(
+          v8bf, *reinterpret_cast<const v4i*>(St + ((wrow * 4 + (pair & 3)) * 2 + (pair >> 2)) * kBlockBytes + lane * 16));
+    };
+    auto stage = [&](int i, const v8bf (&bqC)[2][TERMS], v8bf (&bqN)[2][TERMS], bool convert_next) {
+      if (n_act == 0) return;  // wave-uniform: a wave without rows only feeds the pipeline
+      NextRegs nx;
+      v16i tr;
+      uint32_t pk[TERMS][8];
+      if (convert_next) {
+        next_read(i + 1, nx);
+        tr = transpose_block(nx.raw);
+      }
+      v8bf af = panel_frag(i, 0);
+#pragma unroll
+      for (int pair = 0; pair < 8; ++pair) {
+        const int q = pair >> 2, rb = pair & 3;
+        v8bf af_next = af;
+        if (pair < 7) af_next = panel_frag(i, pair + 1);
+        if (rb < n_act) {
+#pragma unroll
+          for (int t = TERMS - 1; t >= 0; --t)  // small terms first
+            acc[rb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af, bqC[q][t], acc[rb], 0, 0, 0);
+        }
+        if (convert_next && pair >= 2 && pair < 6) convert4(tr, nx.s4[pair - 2], pair - 2, pk);
+        __builtin_amdgcn_sched_barrier(0);
+        af = af_next;
+      }
+      if (convert_next) to_operands(pk, bqN);
+    };
+
+    // ---- main loop.  Stage i issues the loads of stage i + 6.
+    v8bf bqA[2][TERMS], bqB[2][TERMS];
+    wait_vmcnt<0>();  // stores of the previous tile
+    lds_barrier();
+#pragma unroll
+    for (int i = 0; i < kGqBwdAhead; ++i)
+      if (i < L) issue(i);
+    wait_vmcnt<0>();
+    lds_barrier();
+    if (n_act > 0) {  // operands of stage 0
+      NextRegs nx;
+      next_read(0, nx);
+      uint32_t pk[TERMS][8];
+      const v16i tr = transpose_block(nx.raw);
+#pragma unroll
+      for (int gq = 0; gq < 4; ++gq) convert4(tr, nx.s4[gq], gq, pk);
+      to_operands(pk, bqA);
+    }
+    const int L_main = L - kGqBwdAhead;  // stages that still have loads to issue
+    int i = 0;
+    for (; i + 1 < L_main; i += 2) {
+      // stage i + 1 (and so stage i) is older than the loads of the last four stages
+      wait_vmcnt<(kGqBwdAhead - 2) * kGqBwdLoads>();
+      lds_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+      issue(i + kGqBwdAhead);
+      stage(i, bqA, bqB, true);
+      __builtin_amdgcn_sched_barrier(0);
+      wait_vmcnt<(kGqBwdAhead - 2) * kGqBwdLoads>();
+      lds_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+      issue(i + 1 + kGqBwdAhead);
+      stage(i + 1, bqB, bqA, true);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    for (; i < L; i += 2) {  // drain: fewer loads in flight than the count above assumes
+      wait_vmcnt<0>();
+      lds_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+      if (i + kGqBwdAhead < L) issue(i + kGqBwdAhead);
+      stage(i, bqA, bqB, true);
+      __builtin_amdgcn_sched_barrier(0);
+      wait_vmcnt<0>();
+      lds_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+      if (i + 1 + kGqBwdAhead < L) issue(i + 1 + kGqBwdAhead);
+      stage(i + 1, bqB, bqA, i + 2 < L);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+
+    const uint32_t kbw = kb0 + (uint32_t)wcol;
+    if (whole) {
+#pragma unroll
+      for (int rb = 0; rb < 4; ++rb)
+        if (rb < n_act) {
+          const v16f one[1] = {acc[rb]};
+          bwd_dx_store_block<NKK, 1>(g, tm * 256u + (uint32_t)wrow * 128u + rb * 32u, kbw, one);
+        }
+    } else {
+      float4* dst = reinterpret_cast<float4*>(g.part + (size_t)slot * kBwdPartFloats) + (uint32_t)wave * 1024u + lane;
+#pragma unroll
+      for (int rb = 0; rb < 4; ++rb)
+        if (rb < n_act)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            dst[(rb * 4 + e) * 64] = make_float4(acc[rb][4 * e], acc[rb][4 * e + 1], acc[rb][4 * e + 2], acc[rb][4 * e + 3]);
+    }
+  };
+
+  // ---- whole tiles (an XCD walks a contiguous range of the band-major order), then the split ones
+  const uint32_t ntile = g.direct_tiles;
+  const uint32_t wgs_per_xcd = gridDim.x >> 3, xcd = blockIdx.x & 7u;
+  const uint32_t per_xcd = (ntile + 7u) / 8u;
+  uint32_t ti = blockIdx.x >> 3;
+  const uint32_t sw8 = g.sk_wgs >> 3, sk_w = xcd * sw8 + (blockIdx.x >> 3);
+  uint32_t s0 = 0, s1 = 0;
+  if ((blockIdx.x >> 3) < sw8) {
+    const uint32_t total = (g.tiles_m * g.tiles_k - ntile) * g.NB;
+    s0 = sk_w * g.sk_q < total ? sk_w * g.sk_q : total;
+    s1 = s0 + g.sk_q < total ? s0 + g.sk_q : total;
+  }
+  const uint32_t sk_t0 = s0 / g.NB;
+#pragma unroll 1
+  for (;;) {
+    uint32_t t, nb0 = 0, len = g.NB, slot = 0;
+    if (ti < per_xcd) {
+      t = xcd * per_xcd + ti;
+      ti += wgs_per_xcd;
+      if (t >= ntile) { ti = per_xcd; continue; }
+    } else if (s0 < s1) {
+      const uint32_t u = s0 / g.NB;
+      nb0 = s0 - u * g.NB;
+      len = s1 - s0 < g.NB - nb0 ? s1 - s0 : g.NB - nb0;
+      t = ntile + u;
+      slot = 2u * sk_w + (u == sk_t0 ? 0u : 1u);
+      s0 += len;
+    } else {
+      break;
+    }
+    uint32_t tm, tk;
+    bwd_dx_tile_at(g, t, tm, tk);
+    segment(tm, tk, (int)nb0, (int)len, len == g.NB, slot);
+  }
+}
+
+}  // namespace w8a8

@@ -8,7 +8,7 @@ gfx950 HIP kernels: the per-token / per-channel geometry (``bits == 8``,
 ``group_size == K``, ``activation_bits == 8``) takes the tiled / streaming W8A8
 kernels, every other geometry of the format (W4 codes, scales per K group, A4
 activations, any group size) the group-scaled kernels of ``rocm/gq_linear.py``; under
-autograd that path carries the reference's pullback on float32 library GEMMs.
+autograd that path carries the reference's pullback.
 The weight quantizer is an offline, one-time torch computation.
 """
 
@@ -159,8 +159,9 @@ def _group_scaled_input_pullback(dy: torch.Tensor, weight: GroupQuantizedWeight)
 class _GroupScaledLoraFunction(torch.autograd.Function):
     """The group-scaled forward with the reference's pullback (quantized_lora.py:337-394): straight through
     the quantizers, ``dx = dy @ deq(W).T + r @ A.T`` with ``r = (dy @ B.T) * s``, ``dA = x.T @ r``,
-    ``dB = ((x @ A).T @ dy) * s``, ``ds = sum(dy * ((x @ A) @ B))``, all in float32 on the library GEMMs and
-    cast once.  The frozen weight gets no gradient."""
+    ``dB = ((x @ A).T @ dy) * s``, ``ds = sum(dy * ((x @ A) @ B))``, all in float32 and cast once.  The kernels
+    of ``gq_linear.backward`` do it; groups that the packing had to embed and K or N off a multiple of 8 go
+    through float32 library GEMMs on the dequantized weight.  The frozen weight gets no gradient."""
 
     @staticmethod
     def forward(ctx, x, lora_a, lora_b, scaling, weight, activation_bits):
@@ -174,6 +175,14 @@ class _GroupScaledLoraFunction(torch.autograd.Function):
     def backward(ctx, dy):
         x, lora_a, lora_b, scaling = ctx.saved_tensors
         weight = ctx.weight
+        from .rocm import gq_linear
+
+        if gq_linear.has_native_backward(weight) and dy.dtype == torch.bfloat16:
+            dx, da, db, ds = gq_linear.backward(x, dy, weight, lora_a, lora_b, scaling, need_dx=ctx.needs_input_grad[0],
+                                                need_lora_grads=any(ctx.needs_input_grad[1:4]))
+            if ds is not None:
+                ds = ds.reshape(scaling.shape).to(device=scaling.device, dtype=scaling.dtype)
+            return dx, da, db, ds, None, None
         xf = x.reshape(-1, x.shape[-1]).to(torch.float32)
         dyf = dy.reshape(-1, dy.shape[-1]).to(torch.float32)
         a, b = lora_a.to(torch.float32), lora_b.to(torch.float32)
@@ -223,13 +232,18 @@ def quantized_lora_linear(x: torch.Tensor, weight: GroupQuantizedWeight, lora_a:
             f"weight K={weight.original_in_features}")
     if lora_b.shape[1] != weight.codes.shape[-1]:
         raise ValueError(f"LoRA output N={lora_b.shape[1]} does not match weight N={weight.codes.shape[-1]}")
-    scaling = torch.as_tensor(lora_scaling, dtype=torch.float32)
-    if scaling.ndim != 0:
+    # (a Python number stays one: the kernels' side keeps a constant vector per value, where a scalar tensor
+    # would be copied to the device, and waited for, at every call)
+    scaling = lora_scaling if isinstance(lora_scaling, float) else torch.as_tensor(lora_scaling, dtype=torch.float32)
+    if not isinstance(scaling, float) and scaling.ndim != 0:
         raise ValueError(f"lora_scaling must be scalar, got {tuple(scaling.shape)}")
     if per_channel:
         return w8a8_lora.w8a8_lora_linear(x, weight, lora_a, lora_b, scaling, enabled=True)
     if torch.is_grad_enabled() and any(isinstance(t, torch.Tensor) and t.requires_grad
                                        for t in (x, lora_a, lora_b, lora_scaling)):
-        s_arg = lora_scaling if isinstance(lora_scaling, torch.Tensor) and lora_scaling.requires_grad else scaling
+        if isinstance(scaling, float):
+            s_arg = w8a8_lora._scaling_scalar(scaling, x.device)
+        else:
+            s_arg = lora_scaling if isinstance(lora_scaling, torch.Tensor) and lora_scaling.requires_grad else scaling
         return _GroupScaledLoraFunction.apply(x, lora_a, lora_b, s_arg, weight, activation_bits)
     return gq_linear.forward(x, weight, lora_a, lora_b, scaling, activation_bits=activation_bits)

@@ -18,7 +18,7 @@ import torch
 
 from ... import _native
 from .. import quantized_lora as ql
-from .w8a8_lora import MAX_LORA_RANK, _require_cuda, _stream_ptr, _version_of
+from .w8a8_lora import MAX_LORA_RANK, _require_cuda, _scaling_vector, _stream_ptr, _version_of
 
 
 @dataclass(frozen=True)
@@ -37,6 +37,7 @@ class PackedGroupWeight:
     # by zeros at the same places), which changes no maximum, no code of a real element and no integer sum.
     source_group_size: int = 0
     source_padded_in_features: int = 0
+    bf16_scales: bool = False  # every scale is a bf16 value
 
 
 _pack_cache: dict = {}
@@ -83,7 +84,7 @@ def prepare_group_weight(weight) -> PackedGroupWeight:
                                                   _stream_ptr(codes.device))
     _native.check("mi355_w8a8_gq_pack_weight_v1", status)
     out = PackedGroupWeight(packed, weight.scales.to(torch.float32).contiguous(), weight.original_in_features, k_pad,
-                            n, weight.bits, group, src_group, src_k_pad)
+                            n, weight.bits, group, src_group, src_k_pad, weight.scales.dtype == torch.bfloat16)
     with _pack_lock:
         if len(_pack_cache) > 4096:
             _pack_cache.clear()
@@ -136,7 +137,7 @@ def forward(x: torch.Tensor, weight, lora_a=None, lora_b=None, lora_scaling=None
         if r < 1 or r > MAX_LORA_RANK:
             raise ValueError(f"LoRA rank must be in [1, {MAX_LORA_RANK}], got {r}")
         a3, b3 = (embed(a3, 1) if embedded else a3).contiguous(), b3.contiguous()
-        s1 = torch.as_tensor(lora_scaling, dtype=torch.float32, device=dev).reshape(-1)
+        s1 = _scaling_vector(lora_scaling, n_ad, dev).reshape(-1)
         s1 = (s1.expand(n_ad) if s1.numel() == 1 else s1).contiguous()
         if s1.numel() != n_ad:
             raise ValueError(f"lora_scaling must be a scalar or have {n_ad} entries")
@@ -189,4 +190,56 @@ def forward(x: torch.Tensor, weight, lora_a=None, lora_b=None, lora_scaling=None
     return (result, aux) if return_aux else result
 
 
-__all__ = ("PackedGroupWeight", "prepare_group_weight", "forward")
+def has_native_backward(weight) -> bool:
+    """True where ``backward`` covers the geometry: groups that needed no embedding, K and N multiples of 8."""
+    pw = prepare_group_weight(weight)
+    return pw.source_group_size == 0 and pw.in_features % 8 == 0 and pw.out_features % 8 == 0
+
+
+def backward(x: torch.Tensor, dy: torch.Tensor, weight, lora_a: torch.Tensor, lora_b: torch.Tensor,
+             lora_scaling, *, need_dx: bool = True, need_lora_grads: bool = True):
+    """Cotangents ``(dx, d_lora_a, d_lora_b, d_lora_scaling)`` of ``forward`` with one adapter
+    (skyrl/tx/kernels/quantized_lora.py:337-394), float32 throughout and cast once; entries that are not
+    asked for are ``None``."""
+    pw = prepare_group_weight(weight)
+    k, n = pw.in_features, pw.out_features
+    dev = dy.device
+    for t, name in ((x, "x"), (dy, "dy"), (lora_a, "lora_a"), (lora_b, "lora_b")):
+        if t.dtype != torch.bfloat16:
+            raise TypeError(f"{name} must be BF16, got {t.dtype}")
+        _require_cuda(t, name)
+    r = lora_b.shape[0]
+    if tuple(lora_a.shape) != (k, r) or tuple(lora_b.shape) != (r, n) or dy.shape[-1] != n or x.shape != (*dy.shape[:-1], k):
+        raise ValueError(f"incompatible shapes: x={tuple(x.shape)}, dy={tuple(dy.shape)}, A={tuple(lora_a.shape)}, "
+                         f"B={tuple(lora_b.shape)}, weight K={k}, N={n}")
+    xf, dyf = x.reshape(-1, k).contiguous(), dy.reshape(-1, n).contiguous()
+    m = dyf.shape[0]
+    a, b = lora_a.contiguous(), lora_b.contiguous()
+    s1 = _scaling_vector(lora_scaling, 1, dev)
+    lib = _native.load()
+    ws_bytes = int(lib.mi355_w8a8_gq_bwd_workspace_bytes(m, k, pw.padded_in_features, n, pw.group_size, r))
+    if ws_bytes == 0 or pw.source_group_size:
+        raise ValueError(f"geometry M={m}, K={k}, N={n}, group={pw.group_size}, rank={r} is outside the native backward")
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+    dx = torch.empty((m, k), dtype=torch.bfloat16, device=dev) if need_dx else None
+    da = torch.empty_like(a) if need_lora_grads else None
+    db = torch.empty_like(b) if need_lora_grads else None
+    ds = torch.empty((1,), dtype=torch.float32, device=dev) if need_lora_grads else None
+    p = _native.GqBwdProblem()
+    p.struct_size = ctypes.sizeof(_native.GqBwdProblem)
+    p.flags = (_native.FLAG_GQ_BF16_SCALES if pw.bf16_scales else 0) | (0 if need_dx else _native.FLAG_SKIP_GEMM)
+    p.m, p.k, p.k_pad, p.n = m, k, pw.padded_in_features, n
+    p.group_size, p.weight_bits, p.rank = pw.group_size, pw.bits, r
+    p.x, p.dy, p.w_packed, p.w_scales = xf.data_ptr(), dyf.data_ptr(), pw.packed.data_ptr(), pw.scales.data_ptr()
+    p.lora_a, p.lora_b, p.lora_scaling = a.data_ptr(), b.data_ptr(), s1.data_ptr()
+    p.dx = dx.data_ptr() if need_dx else None
+    if need_lora_grads:
+        p.d_lora_a, p.d_lora_b, p.d_lora_scaling = da.data_ptr(), db.data_ptr(), ds.data_ptr()
+    p.workspace, p.workspace_bytes = ws.data_ptr(), ws_bytes
+    with torch.cuda.device(dev):
+        status = lib.mi355_w8a8_gq_linear_bwd_v1(ctypes.byref(p), _stream_ptr(dev))
+    _native.check("mi355_w8a8_gq_linear_bwd_v1", status)
+    return (dx.reshape(x.shape) if need_dx else None), da, db, ds
+
+
+__all__ = ("PackedGroupWeight", "prepare_group_weight", "forward", "has_native_backward", "backward")

@@ -193,7 +193,12 @@ def _new_constant(value: float, count: int, device: str) -> torch.Tensor:
         return torch.full((count,), value, dtype=torch.float32, device=torch.device(device))
 
 
-_cached_constant = functools.lru_cache(maxsize=256)(_new_constant)
+@functools.lru_cache(maxsize=256)
+def _cached_constant(value: float, count: int, device: str) -> torch.Tensor:
+    out = _new_constant(value, count, device)
+    if out.is_cuda:  # filled before another stream or thread can find it
+        torch.cuda.current_stream(out.device).synchronize()
+    return out
 
 
 def _constant_scaling(value: float, count: int, device: str) -> torch.Tensor:
