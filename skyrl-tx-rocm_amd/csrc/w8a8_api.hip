@@ -1853,13 +1853,17 @@ int run_gq_linear(const mi355_w8a8_gq_problem* p, hipStream_t s) {
   // few rows: a row's groups are dealt to several waves so that the launch still fills the chip
   const uint32_t q_slices = L.m_pad >= 1024u ? 1u : (L.G < 16u ? L.G : 16u);
   q.groups_per_slice = (L.G + q_slices - 1u) / q_slices;
-  hipLaunchKernelGGL(gq_quant_kernel, dim3(L.m_pad / 4u, (L.G + q.groups_per_slice - 1u) / q.groups_per_slice), dim3(256),
-                     0, s, q);
-  if ((st = launch_status())) return st;
+  const uint32_t q_grid_y = (L.G + q.groups_per_slice - 1u) / q.groups_per_slice;
+  const bool decode = L.m_pad == 32u;  // few rows: z in K slices instead of row blocks
+  // one adapter's z shares the quantizer's launch (rows of 16-byte pieces; several adapters: a wave per row)
+  const bool decode_z = decode && p->n_adapters == 1u && (p->k & 7u) == 0 && aligned16(p->x);
+  if (!decode_z) {
+    hipLaunchKernelGGL(gq_quant_kernel, dim3(L.m_pad / 4u, q_grid_y), dim3(256), 0, s, q);
+    if ((st = launch_status())) return st;
+  }
 
   // z = x @ A[idx]: rows routed by adapter and multiplied on the matrix core (the kernels of the
   // per-channel path) when the adapter count and K allow it, else one wave per row
-  const bool decode = L.m_pad == 32u;  // few rows: a wave per (row, k slice) instead of one row block
   const bool fast_z = lora && !decode && p->n_adapters <= (uint32_t)kMaxAdapters && (p->k & 7u) == 0 &&
                       aligned16(p->x) && aligned16(p->lora_a);
   const bool routed = fast_z && p->adapter_indices && p->n_adapters > 1u;
@@ -1910,15 +1914,24 @@ int run_gq_linear(const mi355_w8a8_gq_problem* p, hipStream_t s) {
     z.idx = p->adapter_indices;
     z.z = reinterpret_cast<float*>(ws + L.z);
     z.M = p->m; z.K = p->k; z.r = p->rank; z.n_adapters = p->n_adapters;
-    z.k_split = decode ? (p->k + 255u) / 256u : 1u;
-    if (z.k_split > kGqZSlices) z.k_split = kGqZSlices;
-    z.k_chunk = round_up((p->k + z.k_split - 1u) / z.k_split, 64u);
+    const uint32_t most = decode_z ? kGqDecodeZSlices : kGqZSlices, per = decode_z ? kGqDecodeZChunk : 256u;
+    z.k_split = decode ? (p->k + per - 1u) / per : 1u;
+    if (z.k_split > most) z.k_split = most;
+    z.k_chunk = round_up((p->k + z.k_split - 1u) / z.k_split, decode_z ? 128u : 64u);
     z_slices = z.k_split;
-    const dim3 zgrid((p->m + 3u) / 4u, z.k_split), zblock(256);
-    if (p->rank <= 8u) hipLaunchKernelGGL((gq_lora_z_kernel<1>), zgrid, zblock, 0, s, z);
-    else if (p->rank <= 16u) hipLaunchKernelGGL((gq_lora_z_kernel<2>), zgrid, zblock, 0, s, z);
-    else if (p->rank <= 32u) hipLaunchKernelGGL((gq_lora_z_kernel<4>), zgrid, zblock, 0, s, z);
-    else hipLaunchKernelGGL((gq_lora_z_kernel<8>), zgrid, zblock, 0, s, z);
+    if (decode_z) {
+      GqDecodePrologueArgs d{};
+      d.q = q; d.z = z;
+      d.z_units = z.k_split * ((p->rank + 15u) / 16u) * ((p->m + 15u) / 16u);
+      d.row_quads = L.m_pad / 4u;
+      hipLaunchKernelGGL(gq_decode_prologue_kernel, dim3(d.z_units + d.row_quads * q_grid_y), dim3(256), 0, s, d);
+    } else {
+      const dim3 zgrid((p->m + 3u) / 4u, z.k_split), zblock(256);
+      if (p->rank <= 8u) hipLaunchKernelGGL((gq_lora_z_kernel<1>), zgrid, zblock, 0, s, z);
+      else if (p->rank <= 16u) hipLaunchKernelGGL((gq_lora_z_kernel<2>), zgrid, zblock, 0, s, z);
+      else if (p->rank <= 32u) hipLaunchKernelGGL((gq_lora_z_kernel<4>), zgrid, zblock, 0, s, z);
+      else hipLaunchKernelGGL((gq_lora_z_kernel<8>), zgrid, zblock, 0, s, z);
+    }
     if ((st = launch_status())) return st;
   }
 
@@ -1938,7 +1951,18 @@ int run_gq_linear(const mi355_w8a8_gq_problem* p, hipStream_t s) {
   g.bits = p->weight_bits;
   g.r = p->rank; g.n_adapters = p->n_adapters;
   g.n_col_blocks = (p->n + 31u) / 32u;
-  if (L.m_pad == 32u) {  // decode: split the groups over the waves of a workgroup per column block
+  if (decode && p->group_size % 64u == 0) {  // the groups split over the waves of a workgroup per 16 columns
+    const dim3 sgrid((p->n + 15u) / 16u), sblock(1024);
+    if (p->weight_bits == 4u) {
+      if (p->m <= 16u) hipLaunchKernelGGL((gq_stream_kernel<true, 1>), sgrid, sblock, 0, s, g);
+      else hipLaunchKernelGGL((gq_stream_kernel<true, 2>), sgrid, sblock, 0, s, g);
+    } else {
+      if (p->m <= 16u) hipLaunchKernelGGL((gq_stream_kernel<false, 1>), sgrid, sblock, 0, s, g);
+      else hipLaunchKernelGGL((gq_stream_kernel<false, 2>), sgrid, sblock, 0, s, g);
+    }
+    return launch_status();
+  }
+  if (decode) {  // groups that are no multiple of 64: per 32-column block
     const dim3 sgrid(g.n_col_blocks), sblock(kGqSkinnyWaves * 64u);
     if (p->weight_bits == 4u) hipLaunchKernelGGL((gq_skinny_kernel<true>), sgrid, sblock, 0, s, g);
     else hipLaunchKernelGGL((gq_skinny_kernel<false>), sgrid, sblock, 0, s, g);

@@ -14,7 +14,9 @@
 //   gq_quant_kernel        per (row, group): amax, scale, codes (row-major int8, rows padded to 32)
 //   gq_lora_z_kernel       z = x @ A[idx] in float32
 //   gq_gemm_kernel         one wave per 64 x 64 output tile over all groups, epilogue, store
-//   gq_skinny_kernel       up to 32 rows: the groups dealt to the eight waves of a column block
+//   gq_stream_kernel       up to 32 rows: the groups dealt to the sixteen waves of a 16-column unit
+//   gq_skinny_kernel       the same for groups that are no multiple of 64 k, on 32-column units
+//   gq_decode_prologue_kernel  up to 32 rows, one adapter: the quantizer and z in one launch
 #pragma once
 #include "w8a8_device.h"
 
@@ -97,18 +99,18 @@ __device__ inline void gq_load_piece(const GqQuantArgs& a, const uint16_t* xr, b
   }
 }
 
-__global__ __launch_bounds__(256) void gq_quant_kernel(GqQuantArgs a) {
+__device__ inline void gq_quant_rows(const GqQuantArgs& a, uint32_t row_quad, uint32_t slice) {
   __shared__ float piece_max[4][kGqMaxPieces];
   __shared__ float group_scale[4][kGqMaxGroups];
   __shared__ float group_rscale[4][kGqMaxGroups];  // 1 / scale, or -1: divide
   const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-  const uint32_t row = blockIdx.x * 4u + wave;
+  const uint32_t row = row_quad * 4u + wave;
   if (row >= a.M_pad) return;
   const bool live = row < a.M;
   const uint16_t* xr = a.x + (size_t)(live ? row : 0u) * a.K;
   int8_t* cblk = a.codes + (size_t)(row >> 5) * (a.K_pad / 32u) * 1024u + (row & 31u) * 16u;
   const uint32_t pieces_per_group = a.group / 8u;
-  const uint32_t g_lo = blockIdx.y * a.groups_per_slice;
+  const uint32_t g_lo = slice * a.groups_per_slice;
   const uint32_t g_hi = g_lo + a.groups_per_slice < a.G ? g_lo + a.groups_per_slice : a.G;
   if (g_lo >= g_hi) return;
   const uint32_t p_lo = g_lo * pieces_per_group, n_pieces = (g_hi - g_lo) * pieces_per_group;
@@ -220,6 +222,8 @@ __global__ __launch_bounds__(256) void gq_quant_kernel(GqQuantArgs a) {
   }
 }
 
+__global__ __launch_bounds__(256) void gq_quant_kernel(GqQuantArgs a) { gq_quant_rows(a, blockIdx.x, blockIdx.y); }
+
 // ---------------------------------------------------------------------------------------
 struct GqLoraZArgs {
   const uint16_t* x;       // bf16 [M, K]
@@ -276,6 +280,80 @@ __global__ __launch_bounds__(256) void gq_lora_z_kernel(GqLoraZArgs a) {
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
     if (lane == 0 && j < a.r) zout[j] = v;
+  }
+}
+
+// The prologue of a decode call (up to 32 rows) with one adapter: the quantizer and z = x @ A in one launch.
+// Units of 16 rows x 16 ranks x one K slice take the first workgroups, their four waves a quarter of the slice
+// each, on v_mfma_f32_16x16x32_bf16 (products of bf16 exact, float32 sums); the waves are added in order through
+// the LDS, the slices by the consumer.  A's rows are read as they lie: a lane gathers its eight k of one rank,
+// four steps ahead.  Bound by the latency of one such round: 768 KB of A spread over 32 workgroups (K = 12288,
+// rank 32, 16 rows).  A wave per (row, K slice) with a butterfly per rank took 16.8 us there beside 5.1 us of
+// the quantizer; this launch takes 5.4 us for both.  Needs K % 8 == 0 and x aligned to 16 bytes.
+constexpr uint32_t kGqDecodeZSlices = 16, kGqDecodeZChunk = 512;  // most slices; k per slice while there are fewer
+struct GqDecodePrologueArgs {
+  GqQuantArgs q;
+  GqLoraZArgs z;       // k_chunk a multiple of 128
+  uint32_t z_units;    // k_split * rank tiles * row tiles
+  uint32_t row_quads;  // M_pad / 4
+};
+
+__device__ inline void gq_decode_z_unit(const GqLoraZArgs& a, uint32_t unit) {
+  __shared__ float red[3][4][64];
+  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+  const uint32_t c16 = lane & 15u, q = lane >> 4;
+  const uint32_t slice = unit % a.k_split, tile = unit / a.k_split, n_rt = (a.r + 15u) / 16u;
+  const uint32_t row0 = tile / n_rt * 16u, rank0 = tile % n_rt * 16u;
+  const bool row_ok = row0 + c16 < a.M, rank_ok = rank0 + c16 < a.r;
+  const uint16_t* xr = a.x + (size_t)(row_ok ? row0 + c16 : 0u) * a.K;
+  const uint16_t* ar = a.lora_a + (rank_ok ? rank0 + c16 : 0u);
+  const uint32_t quarter = a.k_chunk / 4u, k_lo = slice * a.k_chunk + wave * quarter;
+  uint32_t k_hi = k_lo + quarter;
+  if (k_hi > a.K) k_hi = a.K;
+  v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
+  for (uint32_t base = k_lo; base < k_hi; base += 128u) {
+    v4i xf[4];
+    uint32_t af[4][8];
+#pragma unroll
+    for (uint32_t u = 0; u < 4; ++u) {
+      const uint32_t k = base + u * 32u + 8u * q;
+      const uint32_t kc = k < k_hi ? k : 0u;  // (loads without a condition; what lies beyond is dropped below)
+      xf[u] = *reinterpret_cast<const v4i*>(xr + kc);
+#pragma unroll
+      for (uint32_t j = 0; j < 8; ++j) af[u][j] = ar[(size_t)(kc + j) * a.r];
+    }
+#pragma unroll
+    for (uint32_t u = 0; u < 4; ++u) {
+      const bool in = base + u * 32u + 8u * q < k_hi;
+      v4i af4;
+#pragma unroll
+      for (int d = 0; d < 4; ++d) {
+        xf[u][d] = in && row_ok ? xf[u][d] : 0;
+        af4[d] = in && rank_ok ? (int)(af[u][2 * d] | (af[u][2 * d + 1] << 16)) : 0;
+      }
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, xf[u]), __builtin_bit_cast(v8bf, af4), acc, 0, 0, 0);
+    }
+  }
+  if (wave > 0) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) red[wave - 1u][v][lane] = acc[v];
+  }
+  __syncthreads();
+  if (wave > 0 || !rank_ok) return;
+#pragma unroll
+  for (uint32_t v = 0; v < 4; ++v) {
+    const uint32_t row = row0 + 4u * q + v;
+    const float sum = ((acc[v] + red[0][v][lane]) + red[1][v][lane]) + red[2][v][lane];
+    if (row < a.M) a.z[((size_t)slice * a.M + row) * 64u + rank0 + c16] = sum;
+  }
+}
+
+__global__ __launch_bounds__(256) void gq_decode_prologue_kernel(GqDecodePrologueArgs p) {
+  if (blockIdx.x < p.z_units) {
+    gq_decode_z_unit(p.z, blockIdx.x);
+  } else {
+    const uint32_t b = blockIdx.x - p.z_units;
+    gq_quant_rows(p.q, b % p.row_quads, b / p.row_quads);
   }
 }
 
@@ -928,7 +1006,151 @@ __global__ __launch_bounds__(256, 2) void gq_gemm_lds_kernel(GqGemmArgs a) {
 }
 
 // ---------------------------------------------------------------------------------------
-// Up to 32 rows (decode): a workgroup of eight waves owns one 32-column block for all of K.  Wave w
+// Up to 32 rows (decode), groups of whole 64-wide k steps: a workgroup of sixteen waves owns 16 columns for all
+// of K.  Wave w takes a contiguous range of groups and multiplies on v_mfma_i32_16x16x64_i8 (RB row halves share
+// the weight operand; a lane picks column c of a block pair's four 16-wide k chunks, 128 or 256 consecutive
+// bytes per chunk); U steps stay in flight per wave in registers, each slot asked for again as soon as it is
+// spent.  The buffer resources end with the wave's share of K, and a group's scales are asked for with its last
+// step only (the other steps point beyond the resource), so the stream has neither clamps nor conditions.
+// A wave adds its groups in order, the waves are added in wave order through the LDS (not the strictly
+// sequential sum of the reference: inside the tolerance, the same from run to run).  z and B are staged while
+// the first steps are under way.
+// Bound by the latency of the stream more than by HBM: 12288 x 4096, 16 rows, 4-bit codes (25 MB), groups of
+// 128, rank 32: 14.9 us.  The eight-wave units of 32 columns below (128 of 256 CUs, four dependent B loads per
+// output behind the stream) took 38.2 us there.
+template <bool W4, int RB>
+__global__ __launch_bounds__(1024) void gq_stream_kernel(GqGemmArgs a) {
+  constexpr uint32_t kWaves = 16u, U = RB == 2 ? 4u : (W4 ? 8u : 6u);
+  constexpr uint32_t kBlk = W4 ? 512u : 1024u, kLane = W4 ? 8u : 16u, kBeyond = 0xfffffff0u;
+  typedef int v2i __attribute__((ext_vector_type(2)));
+  __shared__ float red[kWaves][RB * 4][64];
+  __shared__ float zst[RB * 16][64];
+  __shared__ float bst[64][16];
+  const uint32_t tid = threadIdx.x, lane = tid & 63u;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t c16 = lane & 15u, q = lane >> 4;
+  const uint32_t cb = blockIdx.x >> 1, half = blockIdx.x & 1u;
+  const uint32_t col = cb * 32u + half * 16u + c16;
+  const uint32_t kbs = a.K_pad / 32u, spg = a.group / 64u;  // k steps per group
+  const uint32_t g_lo = (wave * a.G) / kWaves, g_hi = ((wave + 1u) * a.G) / kWaves;
+  const uint32_t s_lo = g_lo * spg, s_hi = g_hi * spg;
+  const __amdgpu_buffer_rsrc_t wrsrc = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<unsigned char*>(a.wp) + (size_t)cb * kbs * kBlk, 0, (int)(s_hi * 2u * kBlk), 0x00020000);
+  const __amdgpu_buffer_rsrc_t xrsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(a.codes), 0, (int)(s_hi * 2048u), 0x00020000);
+  const __amdgpu_buffer_rsrc_t swrsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.ws), 0, (int)(a.G * a.N * 4u), 0x00020000);
+  const __amdgpu_buffer_rsrc_t sxrsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.xs), 0, (int)(a.G * a.M_pad * 4u), 0x00020000);
+  const uint32_t w_lane = (q >> 1) * kBlk + (half * 16u + c16 + 32u * (q & 1u)) * kLane;
+  const uint32_t x_lane = (q >> 1) * 1024u + 512u * (q & 1u) + c16 * 16u;
+  struct Step { v4i w, x[RB]; float sw; v4f sx[RB]; } st[U];
+  uint32_t next = s_lo, next_in_group = 0, next_g = g_lo;  // the step to ask for
+  auto fetch = [&](Step& f) {
+    const bool closes = next_in_group + 1u == spg && next < s_hi;
+    if (W4) {
+      const v2i t = __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(wrsrc, w_lane + next * 2u * kBlk, 0, 0));
+      f.w[0] = t[0]; f.w[1] = t[1];
+    } else {
+      f.w = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wrsrc, w_lane + next * 2u * kBlk, 0, 0));
+    }
+#pragma unroll
+    for (int b = 0; b < RB; ++b)
+      f.x[b] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(xrsrc, x_lane + (uint32_t)b * 256u + next * 2048u, 0, 0));
+    f.sw = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(swrsrc, closes ? (next_g * a.N + col) * 4u : kBeyond, 0, 0));
+#pragma unroll
+    for (int b = 0; b < RB; ++b)
+      f.sx[b] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(
+                                            sxrsrc, closes ? (next_g * a.M_pad + 16u * (uint32_t)b + 4u * q) * 4u : kBeyond, 0, 0));
+    ++next;
+    if (++next_in_group == spg) { next_in_group = 0; ++next_g; }
+  };
+#pragma unroll
+  for (uint32_t u = 0; u < U; ++u) fetch(st[u]);
+
+  const bool lora = a.z != nullptr, one_adapter = a.n_adapters == 1u;
+  if (lora) {
+#pragma unroll
+    for (uint32_t b = 0; b < (uint32_t)RB; ++b) {
+      const uint32_t row = 16u * b + (tid >> 6), r = tid & 63u;
+      if (row < a.M && r < a.r) {
+        const float* zp = a.z + (size_t)(a.z_slot ? (uint32_t)a.z_slot[row] : row) * 64u + r;
+        float zv = zp[0];
+#pragma unroll 8
+        for (uint32_t sl = 1; sl < a.z_slices; ++sl) zv = zv + zp[(size_t)sl * a.z_slice_stride];
+        zst[row][r] = zv;
+      }
+    }
+    const uint32_t rank = tid >> 4, bcol = cb * 32u + half * 16u + (tid & 15u);
+    if (one_adapter && rank < a.r && bcol < a.N) bst[rank][tid & 15u] = bf16_bits_to_f32(a.lora_b[(size_t)rank * a.N + bcol]);
+  }
+
+  v4i acc[RB];
+  float part[RB][4];
+#pragma unroll
+  for (int b = 0; b < RB; ++b)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) { acc[b][v] = 0; part[b][v] = -0.0f; }  // (-0 + t is t for every t)
+  uint32_t in_group = 0;
+  for (uint32_t base = s_lo; base < s_hi; base += U) {
+#pragma unroll
+    for (uint32_t u = 0; u < U; ++u) {
+      Step& f = st[u];
+      v4i w = f.w;
+      if (W4) {
+        const uint32_t x0 = (uint32_t)f.w[0], x1 = (uint32_t)f.w[1];
+        w[0] = (int)((x0 << 4) & 0xf0f0f0f0u); w[1] = (int)(x0 & 0xf0f0f0f0u);
+        w[2] = (int)((x1 << 4) & 0xf0f0f0f0u); w[3] = (int)(x1 & 0xf0f0f0f0u);
+      }
+#pragma unroll
+      for (int b = 0; b < RB; ++b) acc[b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(f.x[b], w, acc[b], 0, 0, 0);
+      if (++in_group == spg) {  // the group is complete (the shares are whole groups; steps beyond them are zeros)
+        in_group = 0;
+        const float sw = W4 ? f.sw * 0.0625f : f.sw;
+        if (base + u < s_hi) {
+#pragma unroll
+          for (int b = 0; b < RB; ++b)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+              float t = (float)acc[b][v] * f.sx[b][v];
+              t = t * sw;
+              part[b][v] = part[b][v] + t;
+              acc[b][v] = 0;
+            }
+        }
+      }
+      fetch(f);
+    }
+  }
+#pragma unroll
+  for (int b = 0; b < RB; ++b)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) red[wave][b * 4 + v][lane] = part[b][v];
+  __syncthreads();
+  const uint32_t v = tid >> 6;
+  if (v >= RB * 4u) return;
+  const uint32_t row = 16u * (v >> 2) + 4u * q + (v & 3u);
+  if (row >= a.M || col >= a.N) return;
+  float y = -0.0f;
+#pragma unroll
+  for (uint32_t w = 0; w < kWaves; ++w) y = y + red[w][v][lane];
+  if (a.aux_base) a.aux_base[(size_t)row * a.N + col] = y;
+  if (lora) {
+    int ad = a.idx ? a.idx[row] : 0;
+    ad = ad < 0 ? 0 : (ad >= (int)a.n_adapters ? (int)a.n_adapters - 1 : ad);
+    float low = 0.0f;
+    if (one_adapter) {
+#pragma unroll 8
+      for (uint32_t r = 0; r < a.r; ++r) low = fmaf(zst[row][r], bst[r][c16], low);
+    } else {
+      const uint16_t* bp = a.lora_b + (size_t)ad * a.r * a.N + col;
+#pragma unroll 8
+      for (uint32_t r = 0; r < a.r; ++r) low = fmaf(zst[row][r], bf16_bits_to_f32(bp[(size_t)r * a.N]), low);
+    }
+    y = y + low * a.lora_scaling[ad];
+  }
+  a.out[(size_t)row * a.N + col] = (uint16_t)f32_to_bf16_bits(y);
+}
+
+// ---------------------------------------------------------------------------------------
+// Up to 32 rows, groups that are no multiple of 64 k: a workgroup of eight waves owns one 32-column block for all of K.  Wave w
 // takes a contiguous range of groups, streams its weight fragments eight k blocks ahead, forms its
 // groups' float32 terms in group order, and the eight partial sums are added in wave order through
 // LDS -- the groups are summed in order inside a wave and the waves in order, which differs from
