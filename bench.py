@@ -94,8 +94,8 @@ PROFILE_TRAFFIC = {
     "qwen3-8b-down-m16-decode": ("skinny_stream_kernel__qwen3-8b-down-m16-decode.txt",
                                  [r"skinny_quant_kernel<", r"skinny_stream_kernel<"]),
     "qwen3-8b-gate_up-m4096-backward": ("bwd_dx_kernel__qwen3-8b-gate_up-m4096-backward.txt", [r"bwd_dx_kernel<"]),
-    "qwen3-30b-a3b-moe-mlp-t2048": ("w8a8_gemm_kernel_grouped__qwen3-30b-a3b-moe-mlp-t2048.txt",
-                                    [r"w8a8_gemm_kernel<1, 1, "]),  # grouped gate/up with the SwiGLU epilogue
+    "qwen3-30b-a3b-moe-mlp-t2048": ("w8a8_grouped_kernel__qwen3-30b-a3b-moe-mlp-t2048.txt",
+                                    [r"w8a8_grouped_kernel<1, 1, "]),  # grouped gate/up with the SwiGLU epilogue
     "qwen3-30b-a3b-moe-experts-t2048-backward": ("bwd_dx_kernel_grouped__qwen3-30b-a3b-moe-experts-t2048-backward.txt",
                                                  [r"bwd_pack_dy_kernel<0>", r"bwd_dx_kernel<0, true>"]),
     "qwen3-8b-gate_up-m4096-fused-backward": ("swiglu_bwd_kernel__qwen3-8b-gate_up-m4096-fused-backward.txt",
@@ -683,7 +683,7 @@ def bench_moe_mlp(args, cfg, pkg, dev):
         "config": {"workload": args.workload, **{kk: v for kk, v in cfg.items() if kk != "seed"}},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS, "traffic": measured_traffic_bytes(args.workload),
-                     "kernel": "w8a8_gemm_kernel in grouped mode, gate/up projection with the SwiGLU epilogue",
+                     "kernel": "w8a8_grouped_kernel, gate/up projection with the SwiGLU epilogue",
                      "kernel_avg_ms": gemm_ms, "algorithmic_bytes": gemm_bytes, "algorithmic_ops": gu_ops,
                      "frac_of_int8_mfma_peak": gu_ops / (gemm_ms * 1e-3) / 1e12 / INT8_PEAK_TOPS},
         "stages": stages,

@@ -80,8 +80,9 @@ typedef enum mi355_w8a8_status {
 #define MI355_W8A8_FLAG_TILE_256X256 128u
 #define MI355_W8A8_FLAG_TILE_128X128 2048u
 #define MI355_W8A8_FLAG_TILE_256X128_PAIR 4096u
-/* tile rows of the grouped call (and the slots every group is padded to); default: 128 once the
- * groups average at least 96 rows, else 64.  Pass the same flags to the workspace query. */
+/* row tiles of the grouped call: the first forces tiles of at most 128 rows, the second of at most 256 (K > 128;
+ * shorter K keeps 128); default: by the groups' average size, the rank and how many tiles result.  The results are
+ * the same bits.  Pass the same flags to the workspace query. */
 #define MI355_W8A8_FLAG_GROUPED_TILE64 256u
 #define MI355_W8A8_FLAG_GROUPED_TILE128 512u
 /* The workspace still holds the LoRA A and B in operand order that an earlier call of the tiled path

@@ -8,6 +8,7 @@
 
 #include "w8a8_device.h"
 #include "w8a8_gemm.h"
+#include "w8a8_grouped.h"
 #include "w8a8_gemm16.h"
 #include "w8a8_calibration.h"
 #include "w8a8_prologue.h"
@@ -169,15 +170,11 @@ int launch_lora_a(const LoraAArgs& la, uint32_t nkk, dim3 grid, hipStream_t s) {
 
 template <int EPI, int NKK, int MODE>
 int launch_gemm_one(const GemmArgs& g, hipStream_t s) {
-  // persistent grid: one workgroup slot per CU (two in the 256 x 128 geometry), a multiple of 8
+  // persistent grid: two workgroups per CU, a multiple of 8
   const uint32_t ntile = g.tiles_m * g.tiles_n;
-  const uint32_t slots = (MODE == kModeDense || MODE == kModeDense128) ? 512u : 256u;
   const uint32_t want = ((ntile + 7u) / 8u) * 8u;
-  const dim3 grid(want < slots ? want : slots), block(MODE == kModeGrouped128 ? 512 : 256);
-  constexpr uint32_t lds_bytes =
-      MODE == kModeGrouped128 ? kGrouped128LdsBytes
-                              : (MODE == kModeGrouped ? kGroupedLdsBytes
-                                                      : (MODE == kModeDense128 ? kGemmStages * kGemm128StageBytes : kGemmLdsBytes));
+  const dim3 grid(want < 512u ? want : 512u), block(256);
+  constexpr uint32_t lds_bytes = MODE == kModeDense128 ? kGemmStages * kGemm128StageBytes : kGemmLdsBytes;
   if (hipFuncSetAttribute(reinterpret_cast<const void*>(&w8a8_gemm_kernel<EPI, NKK, MODE>),
                           hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes) != hipSuccess)
     return MI355_W8A8_ERR_LAUNCH;
@@ -192,6 +189,29 @@ int launch_gemm(const GemmArgs& g, uint32_t nkk, hipStream_t s) {
     case 1: return launch_gemm_one<EPI, 1, MODE>(g, s);
     case 2: return launch_gemm_one<EPI, 2, MODE>(g, s);
     case 4: return launch_gemm_one<EPI, 4, MODE>(g, s);
+    default: return MI355_W8A8_ERR_UNSUPPORTED;
+  }
+}
+
+template <int EPI, int NKK, int RB>
+int launch_grouped_one(const GemmArgs& g, hipStream_t s) {
+  // one workgroup per CU; how many tiles there are stands in the tile table
+  const uint32_t want = round_up(g.tiles_m * g.tiles_n, 8u);
+  constexpr uint32_t lds_bytes = grouped_lds_bytes(RB);
+  if (hipFuncSetAttribute(reinterpret_cast<const void*>(&w8a8_grouped_kernel<EPI, NKK, RB>),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes) != hipSuccess)
+    return MI355_W8A8_ERR_LAUNCH;
+  hipLaunchKernelGGL((w8a8_grouped_kernel<EPI, NKK, RB>), dim3(want < 256u ? want : 256u), dim3(kGroupedThreads), lds_bytes, s, g);
+  return launch_status();
+}
+
+template <int EPI, int RB>
+int launch_grouped(const GemmArgs& g, uint32_t nkk, hipStream_t s) {
+  switch (nkk) {
+    case 0: return launch_grouped_one<EPI, 0, RB>(g, s);
+    case 1: return launch_grouped_one<EPI, 1, RB>(g, s);
+    case 2: return launch_grouped_one<EPI, 2, RB>(g, s);
+    case 4: return launch_grouped_one<EPI, 4, RB>(g, s);
     default: return MI355_W8A8_ERR_UNSUPPORTED;
   }
 }
@@ -570,16 +590,22 @@ int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
 }
 
 struct GroupedLayout {
-  uint64_t xq, sx, zp, at, bp, src_row, dst_pos, blk_range, total;
-  uint32_t slots, nkk, K_pad, KB, n_steps, steps_per_wave, pad;
+  uint64_t xq, sx, zp, at, bp, src_row, dst_pos, blk_range, tile_tab, total;
+  uint32_t slots, nkk, K_pad, KB, n_steps, steps_per_wave, tile_blocks, max_tiles;
 };
 
-// Rows of padding per group = rows of a GEMM tile: 128 once the groups average at least 96 rows (the
-// weight panel then travels L2 -> LDS once per 128 rows), else 64; the flags force either.
-uint32_t grouped_pad(uint32_t m, uint32_t n_groups, uint32_t flags) {
-  if (flags & MI355_W8A8_FLAG_GROUPED_TILE64) return 64u;
-  if (flags & MI355_W8A8_FLAG_GROUPED_TILE128) return 128u;
-  return (uint64_t)m >= 96ull * n_groups ? 128u : 64u;
+// 32-row blocks that a GEMM tile holds at most, 4 or 8; the flags force either (8 only where K has the steps it
+// needs).  8 once the groups average at least 96 rows, so that nearly every group is one tile, while those tiles
+// still fill three quarters of the CUs and the epilogue's operands fit the ring (rank <= 16; beyond it the
+// tall tile's registers spill).  Grouped call, 4 / 8, sizes rows x K x N: 48 groups of 200 x 1024 x 1024, rank 16:
+// 63 / 59 us; 32 of 256 x 1024 x 1024 (128 tall tiles): 47 / 56; 128 of 128 x 2048 x 1536, rank 64: 240 / 273;
+// 128 of 64 x 2048 x 1536, rank 16: 112 / 116.
+uint32_t grouped_tile_blocks(uint32_t m, uint32_t k, uint32_t n, uint32_t n_groups, uint32_t rank, uint32_t flags) {
+  if (k_padded(k) < kGroupedTallMinK) return 4u;
+  if (flags & MI355_W8A8_FLAG_GROUPED_TILE64) return 4u;
+  if (flags & MI355_W8A8_FLAG_GROUPED_TILE128) return 8u;
+  const uint64_t tall_tiles = (uint64_t)(n_groups > m / 256u ? n_groups : m / 256u) * (n_padded(n) / kGroupedTileN);
+  return (uint64_t)m >= 96ull * n_groups && rank <= 16u && tall_tiles >= 192u ? 8u : 4u;
 }
 
 GroupedLayout make_grouped_layout(uint32_t m, uint32_t k, uint32_t n, uint32_t n_groups, uint32_t rank,
@@ -587,10 +613,10 @@ GroupedLayout make_grouped_layout(uint32_t m, uint32_t k, uint32_t n, uint32_t n
   GroupedLayout w{};
   w.K_pad = k_padded(k);
   w.KB = w.K_pad / 32u;
-  w.pad = grouped_pad(m, n_groups, flags);
-  // every group is padded to a multiple of pad slots: at most pad - 1 padding slots per group
-  const uint64_t worst = (uint64_t)m + (uint64_t)(w.pad - 1u) * n_groups;
-  w.slots = (uint32_t)((worst + w.pad - 1u) / w.pad * w.pad);
+  w.tile_blocks = grouped_tile_blocks(m, k, n, n_groups, rank, flags);
+  // every group is padded to a multiple of 32 slots: at most 31 padding slots per group
+  w.slots = (uint32_t)(((uint64_t)m + 31u * (uint64_t)n_groups + 31u) / 32u * 32u);
+  w.max_tiles = w.slots / 32u / w.tile_blocks + n_groups;
   w.nkk = rank_chunks(rank);
   w.n_steps = (k + 63u) / 64u;
   w.steps_per_wave = (w.n_steps + 15u) / 16u;
@@ -604,6 +630,7 @@ GroupedLayout make_grouped_layout(uint32_t m, uint32_t k, uint32_t n, uint32_t n
   w.src_row = off; off += align256((uint64_t)w.slots * 4u);
   w.dst_pos = off; off += align256((uint64_t)m * 4u);
   w.blk_range = off; off += align256((uint64_t)(w.slots / 32u) * 4u);
+  w.tile_tab = off; off += align256(((uint64_t)w.max_tiles + 1u) * 8u);
   w.zp = off; off += rank ? align256((uint64_t)(w.slots / 32u) * w.nkk * 3u * kBlockBytes) : 0u;
   w.total = off;
   return w;
@@ -662,7 +689,8 @@ int run_grouped(const mi355_w8a8_grouped_problem* p, hipStream_t s) {
   if (!skip_prologue) {
     LoraPrepArgs pa{};
     pa.src_row = src_row; pa.dst_pos = dst_pos; pa.blk_range = blk_range;
-    pa.group_sizes = p->group_sizes; pa.group_pad = w.pad;
+    pa.group_sizes = p->group_sizes;
+    pa.tile_tab = reinterpret_cast<uint64_t*>(ws + w.tile_tab); pa.tile_blocks = w.tile_blocks;
     pa.lora_a = static_cast<const uint16_t*>(p->lora_a);
     pa.lora_b = static_cast<const uint16_t*>(p->lora_b);
     pa.at = reinterpret_cast<uint16_t*>(ws + w.at);
@@ -736,21 +764,19 @@ int run_grouped(const mi355_w8a8_grouped_problem* p, hipStream_t s) {
   g.w_group_stride = mi355_w8a8_packed_weight_bytes(p->k, p->n);
   g.M = p->m; g.N = p->n; g.K_pad = w.K_pad; g.KB = w.KB; g.slots = w.slots;
   g.total_rows = w.slots;
-  g.tiles_m = w.slots / w.pad;
-  g.tiles_n = (n_padded(p->n) + kGroupedTileN - 1u) / kGroupedTileN;
+  g.tiles_m = w.max_tiles;
+  g.tiles_n = n_padded(p->n) / kGroupedTileN;
+  g.tile_tab = reinterpret_cast<const uint64_t*>(ws + w.tile_tab);
   g.rank = p->rank;
   g.groups_per_weight = gpw;
+  const bool tall = w.tile_blocks == 8u;
   if (p->aux_acc) {
     GemmArgs ga = g;
     ga.out = p->aux_acc;
-    if ((st = w.pad == 128u ? launch_gemm<kEpiAcc, kModeGrouped128>(ga, 0u, s)
-                            : launch_gemm<kEpiAcc, kModeGrouped>(ga, 0u, s)))
-      return st;
+    if ((st = tall ? launch_grouped<kEpiAcc, 8>(ga, 0u, s) : launch_grouped<kEpiAcc, 4>(ga, 0u, s))) return st;
   }
-  if (w.pad == 128u)
-    return swiglu ? launch_gemm<kEpiSwiglu, kModeGrouped128>(g, w.nkk, s)
-                  : launch_gemm<kEpiPlain, kModeGrouped128>(g, w.nkk, s);
-  return swiglu ? launch_gemm<kEpiSwiglu, kModeGrouped>(g, w.nkk, s) : launch_gemm<kEpiPlain, kModeGrouped>(g, w.nkk, s);
+  if (tall) return swiglu ? launch_grouped<kEpiSwiglu, 8>(g, w.nkk, s) : launch_grouped<kEpiPlain, 8>(g, w.nkk, s);
+  return swiglu ? launch_grouped<kEpiSwiglu, 4>(g, w.nkk, s) : launch_grouped<kEpiPlain, 4>(g, w.nkk, s);
 }
 
 // ---------------------------------------------------------------------------------------

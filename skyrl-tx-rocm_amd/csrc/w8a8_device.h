@@ -110,5 +110,10 @@ __device__ inline void lds_load_1k(const unsigned char* base_uniform, uint32_t v
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
                :: "v"(voff), "s"(base_uniform), "s"(lds_addr_uniform) : "memory", "m0");
 }
+// ... for data that is read once (non-temporal)
+__device__ inline void lds_load_1k_once(const unsigned char* base_uniform, uint32_t voff, uint32_t lds_addr_uniform) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt"
+               :: "v"(voff), "s"(base_uniform), "s"(lds_addr_uniform) : "memory", "m0");
+}
 
 }  // namespace w8a8

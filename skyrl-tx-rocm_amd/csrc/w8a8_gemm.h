@@ -31,10 +31,11 @@ struct GemmArgs {
   const int32_t* blk_range;  // per 32-row block: first group | last group << 16, or null
   const uint16_t* residual;  // bf16 [M, n_out] or null
   void* out;                 // bf16 [M, n_out] or int32 [M, N]
-  uint64_t w_group_stride;   // grouped mode: bytes between the packed weights of two experts
+  uint64_t w_group_stride;   // grouped call: bytes between the packed weights of two experts
   uint32_t M, N, K_pad, KB, slots, total_rows;
   uint32_t tiles_m, tiles_n, rank;
-  uint32_t groups_per_weight; // grouped mode: weight index = group / groups_per_weight
+  uint32_t groups_per_weight; // grouped call: weight index = group / groups_per_weight
+  const uint64_t* tile_tab;   // grouped call: number of row tiles, then first 32-slot block | blocks << 32 | group << 48 of each
   uint32_t* tile_ctr;         // 8 zeroed counters, 64 bytes apart (one per XCD), or null: static schedule
 };
 
@@ -50,26 +51,187 @@ constexpr int kGemmTileN = 128;
 constexpr int kGemmStages = 3;
 constexpr int kGemmStageBytes = 24576;  // A: 8 row blocks x 2 k blocks, B: 4 column blocks x 2 k blocks
 constexpr int kGemmLdsBytes = kGemmStages * kGemmStageBytes;
-// Grouped (ragged, per-expert weight) mode: tile 64 x 512, the four waves sit side by side along
-// N (64 x 128 each) and share the 64-row activation panel; every 64-row tile belongs to one group.
-constexpr int kGroupedTileM = 64;
-constexpr int kGroupedTileN = 512;
-constexpr int kGroupedStages = 4;
-constexpr int kGroupedStageBytes = 36864;  // A: 2 row blocks x 2 k blocks, B: 16 column blocks x 2 k blocks
-constexpr int kGroupedLdsBytes = kGroupedStages * kGroupedStageBytes;
-// grouped geometry for experts with many rows: 128 x 512 tile, 8 waves (2 x 4), the weight panel
-// travels L2 -> LDS once per 128 rows instead of once per 64
-constexpr int kGrouped128TileM = 128;
-constexpr int kGrouped128Stages = 3;
-constexpr int kGrouped128StageBytes = 40960;  // A: 4 row blocks x 2 k blocks, B: 16 column blocks x 2 k blocks
-constexpr int kGrouped128LdsBytes = kGrouped128Stages * kGrouped128StageBytes;
-
 // (The 256 x 256 geometry for large problems is a kernel of its own: w8a8_gemm16.h.)
 // Dense geometry for calls whose 256 x 128 tiles would leave most CUs idle: 128 x 128 tiles, the four
 // waves stacked along M with 32 x 128 each, so a wave carries half the MFMAs and half the epilogue.
 constexpr int kGemm128TileM = 128;
 constexpr int kGemm128StageBytes = 16384;  // A: 4 row blocks x 2 k blocks, B: 4 column blocks x 2 k blocks
-enum { kModeDense = 0, kModeGrouped = 1, kModeGrouped128 = 2, kModeDense128 = 3 };
+enum { kModeDense = 0, kModeDense128 = 1 };
+
+// Where the epilogue of one 32-row block finds its operands: in memory.  (The grouped kernel has a form that finds them in the LDS.)
+struct EpilogueFromMemory {
+  const GemmArgs& g;
+  uint32_t pbase, tcol0, ncb_total;
+  __device__ float sx(int c) const { return g.sx[pbase + c]; }
+  __device__ int src_row(int c) const { return g.src_row ? g.src_row[pbase + c] : (int)(pbase + c); }
+  __device__ uint32_t range() const { return g.blk_range ? (uint32_t)g.blk_range[pbase / 32u] : 0u; }
+  __device__ int slot_group(int c, int first) const { return g.slot_group ? g.slot_group[pbase + c] : first; }
+  __device__ float scaling(int gi) const { return g.lora_scaling[gi]; }
+  template <int NKK>
+  __device__ v8us z(int kk, int term, int lane) const {
+    return *reinterpret_cast<const v8us*>(g.zp + ((size_t)(pbase / 32u) * NKK * 3u + kk * 3 + term) * kBlockBytes + lane * 16);
+  }
+  // operand of the wave's packed column block j: rows 16 kk + 8 h + 0..7 of column 4 c + j
+  template <int NKK>
+  __device__ v8us b(int gi, int j, int kk, int lane) const {
+    return *reinterpret_cast<const v8us*>(g.bp + (((size_t)gi * ncb_total + tcol0 / 32u + j) * NKK + kk) * kBlockBytes + lane * 16);
+  }
+};
+
+// Epilogue of one 32-row block of a wave's 128 columns from tcol0 on: accumulators acc[j] of the packed column
+// blocks j.  Lane (c = lane % 32, h = lane / 32) owns the four consecutive original columns ncol .. ncol + 3
+// (ncol = tcol0 + 4 c) of the 16 rows 8*(v/4) + 4*h + v%4; sw holds their scales.
+template <int EPI, int NKK, class Source>
+__device__ inline __attribute__((always_inline)) void gemm_epilogue_block(const GemmArgs& g, const Source& from, const v16i (&acc)[4],
+                                                                          const float (&sw)[4], uint32_t tcol0, bool full_n,
+                                                                          uint32_t n_out) {
+  constexpr bool kLora = (NKK > 0) && (EPI != kEpiAcc);
+  const int lane = threadIdx.x & 63;
+  const int c = lane & 31, h = lane >> 5;
+  const uint32_t ncol = tcol0 + 4u * c;
+  __builtin_amdgcn_sched_barrier(0);  // keep the blocks' register lifetimes apart
+
+  // Per-row scale and output offset of the block's 32 rows live in one register each (lane l
+  // holds row l % 32); a lane's 16 rows 8*(v/4) + 4*h + v%4 are fetched across lanes below.
+  const float sx_lane = (EPI != kEpiAcc) ? from.sx(c) : 0.0f;
+  const int src_lane = from.src_row(c);
+  const bool row_ok = src_lane >= 0 && src_lane < (int)g.M;
+  const uint32_t off_lane = row_ok ? (uint32_t)src_lane * ((EPI == kEpiAcc) ? g.N : n_out) : 0xffffffffu;
+  const bool fast = full_n && (__builtin_amdgcn_ballot_w64(!row_ok) == 0);  // wave-uniform
+  const int row_addr = 16 * h;  // byte address (4 * lane) of the lane holding row 4*h
+
+  if (EPI == kEpiAcc) {
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      const uint32_t rowoff =
+          (uint32_t)__builtin_amdgcn_ds_bpermute(row_addr + 4 * (8 * (v >> 2) + (v & 3)), (int)off_lane);
+      if (!fast && rowoff == 0xffffffffu) continue;
+      int32_t* o = reinterpret_cast<int32_t*>(g.out) + rowoff + ncol;
+      if (fast) {
+        *reinterpret_cast<int4*>(o) = make_int4(acc[0][v], acc[1][v], acc[2][v], acc[3][v]);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (ncol + j < g.N) o[j] = acc[j][v];
+      }
+    }
+    return;
+  }
+
+  // Groups (adapters) present in this 32-row block: one, except at a group boundary.  A
+  // boundary block is simply processed once per group; each pass stores only its own rows.
+  const uint32_t range = kLora ? from.range() : 0u;
+  const int glo = (int)(range & 0xffffu), ghi = (int)(range >> 16);
+  const int grp_lane = (kLora && ghi > glo) ? from.slot_group(c, glo) : glo;
+  for (int gi = glo; gi <= ghi; ++gi) {  // wave-uniform
+  // The lane's four columns are processed as two pairs (jp): LoRA MFMAs of the pair (section A),
+  // then dequantize + add + activate per row (section B).  The first pair's packed result waits
+  // in `hold` so that every row is written with one 4- or 8-byte store.
+  uint32_t hold[16];
+#pragma unroll
+  for (int jp = 0; jp < 2; ++jp) {
+    // ---- section A: lowS[j][v] = s_g * (z @ B_g) for the column pair
+    v16f lowS[2];
+    if constexpr (kLora) {
+#pragma unroll
+      for (int kk = 0; kk < NKK; ++kk) {
+        v8us zf[3];
+#pragma unroll
+        for (int t3 = 0; t3 < 3; ++t3) zf[t3] = from.template z<NKK>(kk, t3, lane);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const v8bf bb = __builtin_bit_cast(v8bf, from.template b<NKK>(gi, 2 * jp + j, kk, lane));
+          v16f cur;
+          if (kk == 0) {
+#pragma unroll
+            for (int e = 0; e < 16; ++e) cur[e] = 0.0f;
+          } else {
+            cur = lowS[j];
+          }
+          cur = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, zf[2]), bb, cur, 0, 0, 0);
+          cur = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, zf[1]), bb, cur, 0, 0, 0);
+          cur = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, zf[0]), bb, cur, 0, 0, 0);
+          lowS[j] = cur;
+        }
+      }
+      const float sgrp = from.scaling(gi);
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) lowS[j][e] = lowS[j][e] * sgrp;
+    }
+
+    // ---- section B
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      // row 8*(v/4) + 4*h + v%4 of the block: its data sits in that lane (cross-lane read on
+      // the LDS crossbar, which is idle here; no vector-ALU work)
+      const int src_lane_addr = row_addr + 4 * (8 * (v >> 2) + (v & 3));
+      const uint32_t rowoff = (uint32_t)__builtin_amdgcn_ds_bpermute(src_lane_addr, (int)off_lane);
+      const float sxv =
+          __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(src_lane_addr, __builtin_bit_cast(int, sx_lane)));
+      const float t0 = (float)acc[2 * jp][v] * sxv;
+      const float t1 = (float)acc[2 * jp + 1][v] * sxv;
+      // same f32 operations, in the same order, as the reference epilogue: a fused
+      // multiply-add here would flip rare bf16 roundings that SwiGLU then amplifies
+      float y0 = t0 * sw[2 * jp];
+      float y1 = t1 * sw[2 * jp + 1];
+      if constexpr (kLora) {
+        y0 = y0 + lowS[0][v];
+        y1 = y1 + lowS[1][v];
+      }
+      bool row_valid = fast || rowoff != 0xffffffffu;
+      if (kLora && ghi > glo)  // boundary block: this pass owns only the rows of group gi
+        row_valid = row_valid && (__builtin_amdgcn_ds_bpermute(src_lane_addr, grp_lane) == gi);
+      uint32_t mine_bits;
+      if (EPI == kEpiSwiglu) {
+        // (y0, y1) = (gate, up) of the product column ncol/2 + jp
+        const uint32_t f = pack_bf16x2(y0, y1);
+        mine_bits = __float_as_uint(swiglu_f32(__uint_as_float(f << 16), __uint_as_float(f & 0xffff0000u)));
+      } else {
+        if (g.residual && row_valid) {
+          uint32_t rr;
+          if (fast) {
+            rr = *reinterpret_cast<const uint32_t*>(g.residual + rowoff + ncol + 2u * jp);
+          } else {
+            rr = 0;
+            if (ncol + 2u * jp < g.N) rr |= (uint32_t)g.residual[rowoff + ncol + 2u * jp];
+            if (ncol + 2u * jp + 1u < g.N) rr |= (uint32_t)g.residual[rowoff + ncol + 2u * jp + 1u] << 16;
+          }
+          y0 = y0 + __uint_as_float(rr << 16);
+          y1 = y1 + __uint_as_float(rr & 0xffff0000u);
+        }
+        mine_bits = pack_bf16x2(y0, y1);
+      }
+      if (jp == 0) {
+        hold[v] = mine_bits;
+        continue;
+      }
+      if (!row_valid) continue;
+      if (EPI == kEpiSwiglu) {
+        const uint32_t pk = pack_bf16x2(__uint_as_float(hold[v]), __uint_as_float(mine_bits));
+        uint16_t* o = reinterpret_cast<uint16_t*>(g.out) + rowoff + (ncol >> 1);
+        if (fast) {
+          *reinterpret_cast<uint32_t*>(o) = pk;
+        } else {
+          if ((ncol >> 1) < n_out) o[0] = (uint16_t)(pk & 0xffffu);
+          if ((ncol >> 1) + 1u < n_out) o[1] = (uint16_t)(pk >> 16);
+        }
+      } else {
+        uint16_t* o = reinterpret_cast<uint16_t*>(g.out) + rowoff + ncol;
+        if (fast) {
+          *reinterpret_cast<uint2*>(o) = make_uint2(hold[v], mine_bits);
+        } else {
+          if (ncol + 0u < g.N) o[0] = (uint16_t)(hold[v] & 0xffffu);
+          if (ncol + 1u < g.N) o[1] = (uint16_t)(hold[v] >> 16);
+          if (ncol + 2u < g.N) o[2] = (uint16_t)(mine_bits & 0xffffu);
+          if (ncol + 3u < g.N) o[3] = (uint16_t)(mine_bits >> 16);
+        }
+      }
+    }
+  }
+  }  // groups of the block
+}
 
 // One tile of the persistent loop.
 struct GemmTile {
@@ -81,29 +243,24 @@ struct GemmTile {
 };
 
 template <int EPI, int NKK, int MODE = kModeDense>
-__global__ __launch_bounds__(MODE == kModeGrouped128 ? 512 : 256, (MODE == kModeDense || MODE == kModeDense128) ? 2 : 1)
+__global__ __launch_bounds__(256, 2)
 void w8a8_gemm_kernel(GemmArgs g) {
-  constexpr bool G128 = MODE == kModeGrouped128;
   constexpr bool D128 = MODE == kModeDense128;
-  constexpr bool GROUPED = MODE == kModeGrouped || G128;
-  constexpr int kWaves = G128 ? 8 : 4;
+  constexpr int kWaves = 4;
   constexpr int kWR = D128 ? 1 : 2;                                  // 32-row blocks of a wave's tile
-  constexpr uint32_t kRowBlocks = (G128 || D128) ? 4 : (GROUPED ? 2 : 8);  // 32-row blocks of the activation panel
-  constexpr uint32_t kColBlocks = GROUPED ? 16 : 4;                 // 32-column blocks of the weight panel
-  constexpr int kStages = G128 ? kGrouped128Stages : (GROUPED ? kGroupedStages : kGemmStages);
-  constexpr int kStageBytes =
-      G128 ? kGrouped128StageBytes : (GROUPED ? kGroupedStageBytes : (D128 ? kGemm128StageBytes : kGemmStageBytes));
+  constexpr uint32_t kRowBlocks = D128 ? 4 : 8;                     // 32-row blocks of the activation panel
+  constexpr uint32_t kColBlocks = 4;                                // 32-column blocks of the weight panel
+  constexpr int kStages = kGemmStages;
+  constexpr int kStageBytes = D128 ? kGemm128StageBytes : kGemmStageBytes;
   constexpr int kAChunks = kRowBlocks * 2;                              // 1 KiB chunks of A per stage
   constexpr int kLoadsPerTile = (kAChunks + kColBlocks * 2) / kWaves;   // direct-to-LDS loads per wave per k-tile
-  constexpr bool kLora = (NKK > 0) && (EPI != kEpiAcc);
 
   extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wrow = G128 ? (wave >> 2) : (GROUPED ? 0 : wave);  // wave position along M (32 * kWR rows each)
-  const int wcol = G128 ? (wave & 3) : (GROUPED ? wave : 0);    // wave position along N (128 columns each)
-  const int c = lane & 31, h = lane >> 5;
+  const int wrow = wave;  // wave position along M (32 * kWR rows each)
+  const int c = lane & 31;
 
   const uint32_t total_rows = g.total_rows;
   const uint32_t ntile = g.tiles_m * g.tiles_n;
@@ -121,21 +278,15 @@ void w8a8_gemm_kernel(GemmArgs g) {
     GemmTile T{};
     const uint32_t t = i < per_xcd ? (blockIdx.x & 7u) * per_xcd + i : ntile;
     if (t >= ntile) return T;
-    constexpr uint32_t GM = GROUPED ? 1 : 4;
+    constexpr uint32_t GM = 4;
     const uint32_t band = t / (GM * g.tiles_n);
     const uint32_t band_rows = (g.tiles_m - band * GM) < GM ? (g.tiles_m - band * GM) : GM;
     const uint32_t in_band = t - band * GM * g.tiles_n;
     T.tm = band * GM + in_band % band_rows;
     T.tn = in_band / band_rows;
-    uint32_t widx = 0;
-    if (GROUPED) {
-      const int32_t range = g.blk_range[T.tm * kRowBlocks];
-      if (range < 0) return T;  // tile beyond the rows in use: nothing to do, but later tiles may exist
-      widx = ((uint32_t)range & 0xffffu) / g.groups_per_weight;
-    }
     T.Ag = g.xq + (size_t)T.tm * kRowBlocks * g.KB * kBlockBytes;
-    T.Bg = g.wp + (size_t)widx * g.w_group_stride;
-    T.swp = g.sw + (size_t)widx * (GROUPED ? g.N : 0u);
+    T.Bg = g.wp;
+    T.swp = g.sw;
     T.valid = true;
     return T;
   };
@@ -143,7 +294,7 @@ void w8a8_gemm_kernel(GemmArgs g) {
   // Dynamic schedule (two workgroups per CU): positions come from the XCD's counter, because the
   // hardware favours the older workgroup of a CU and a static split would leave the younger one
   // to finish alone.  The result does not depend on which workgroup computes which tile.
-  const bool dyn = !GROUPED && g.tile_ctr != nullptr;
+  const bool dyn = g.tile_ctr != nullptr;
   uint32_t* const ctr = g.tile_ctr + (blockIdx.x & 7u) * 16u;
   __shared__ uint32_t dyn_slot[2];
   uint32_t cur_i = blockIdx.x >> 3, nxt_i = 0;
@@ -174,14 +325,14 @@ void w8a8_gemm_kernel(GemmArgs g) {
       af[i] = *reinterpret_cast<const v4i*>(As + ((wrow * kWR + i) * 2 + ks) * kBlockBytes + lane * 16);
 #pragma unroll
     for (int j = 0; j < 4; ++j)
-      bf[j] = *reinterpret_cast<const v4i*>(Bs + ((wcol * 4 + j) * 2 + ks) * kBlockBytes + lane * 16);
+      bf[j] = *reinterpret_cast<const v4i*>(Bs + (j * 2 + ks) * kBlockBytes + lane * 16);
   };
 
   bool prefetched = false;  // the first kStages-1 k-tiles of the current tile are already in flight
   for (uint32_t step = 0; cur_i < per_xcd; ++step, cur_i = nxt_i) {
     const GemmTile T = tile_at(cur_i);
     nxt_i = cur_i + wgs_per_xcd;
-    if (!T.valid) { prefetched = false; continue; }  // static schedules only (empty grouped tile, range end)
+    if (!T.valid) { prefetched = false; continue; }  // static schedules only (range end)
 
     v16i acc[kWR][4];
 #pragma unroll
@@ -288,11 +439,8 @@ void w8a8_gemm_kernel(GemmArgs g) {
     }
 
     // ---------------------------------------------------------------- epilogue
-    // Lane (c = lane % 32, h = lane / 32) owns, in each of its wave's two 32 x 128 strips, the four
-    // consecutive original columns ncol .. ncol+3 (accumulator blocks j = 0..3) of the 16 rows
-    // 8*(v/4) + 4*h + v%4.
     const uint32_t m0 = T.tm * (kRowBlocks * 32u) + wrow * (32u * kWR);
-    const uint32_t tcol0 = T.tn * (kColBlocks * 32u) + wcol * 128u;  // first column of the wave
+    const uint32_t tcol0 = T.tn * (kColBlocks * 32u);  // first column of the wave
     const uint32_t ncol = tcol0 + 4u * c;
     const bool full_n = (tcol0 + 128u <= g.N) && ((g.N & 3u) == 0);  // wave-uniform
     if (tcol0 >= g.N) continue;  // wave beyond the last column; it still takes part in the next tile
@@ -307,162 +455,13 @@ void w8a8_gemm_kernel(GemmArgs g) {
           if (ncol + j < g.N) sw[j] = T.swp[ncol + j];
       }
     }
-    auto epilogue_block = [&](auto BI) {
-      constexpr int bi = decltype(BI)::value;
+    const auto epilogue_block = [&](int bi) {
       const uint32_t pbase = m0 + bi * 32u;
       if (pbase >= total_rows) return;  // wave-uniform
-      const uint32_t blk = pbase / 32u;
-      if (GROUPED && g.blk_range[blk] < 0) return;  // block beyond the rows in use
-      __builtin_amdgcn_sched_barrier(0);  // keep the blocks' register lifetimes apart
-
-      // Per-row scale and output offset of the block's 32 rows live in one register each (lane l
-      // holds row l % 32); a lane's 16 rows 8*(v/4) + 4*h + v%4 are fetched across lanes below.
-      const float sx_lane = (EPI != kEpiAcc) ? g.sx[pbase + c] : 0.0f;
-      const int src_lane = g.src_row ? g.src_row[pbase + c] : (int)(pbase + c);
-      const bool row_ok = src_lane >= 0 && src_lane < (int)g.M;
-      const uint32_t off_lane = row_ok ? (uint32_t)src_lane * ((EPI == kEpiAcc) ? g.N : n_out) : 0xffffffffu;
-      const bool fast = full_n && (__builtin_amdgcn_ballot_w64(!row_ok) == 0);  // wave-uniform
-      const int row_addr = 16 * h;  // byte address (4 * lane) of the lane holding row 4*h
-
-      if (EPI == kEpiAcc) {
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const uint32_t rowoff =
-              (uint32_t)__builtin_amdgcn_ds_bpermute(row_addr + 4 * (8 * (v >> 2) + (v & 3)), (int)off_lane);
-          if (!fast && rowoff == 0xffffffffu) continue;
-          int32_t* o = reinterpret_cast<int32_t*>(g.out) + rowoff + ncol;
-          if (fast) {
-            *reinterpret_cast<int4*>(o) = make_int4(acc[bi][0][v], acc[bi][1][v], acc[bi][2][v], acc[bi][3][v]);
-          } else {
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-              if (ncol + j < g.N) o[j] = acc[bi][j][v];
-          }
-        }
-        return;
-      }
-
-      // Groups (adapters) present in this 32-row block: one, except at a group boundary.  A
-      // boundary block is simply processed once per group; each pass stores only its own rows.
-      const uint32_t range = (kLora && g.blk_range) ? (uint32_t)g.blk_range[blk] : 0u;
-      const int glo = (int)(range & 0xffffu), ghi = (int)(range >> 16);
-      const int grp_lane = (kLora && g.slot_group && ghi > glo) ? g.slot_group[pbase + c] : glo;
-      for (int gi = glo; gi <= ghi; ++gi) {  // wave-uniform
-      // The lane's four columns are processed as two pairs (jp): LoRA MFMAs of the pair (section A),
-      // then dequantize + add + activate per row (section B).  The first pair's packed result waits
-      // in `hold` so that every row is written with one 4- or 8-byte store.
-      uint32_t hold[16];
-#pragma unroll
-      for (int jp = 0; jp < 2; ++jp) {
-        // ---- section A: lowS[j][v] = s_g * (z @ B_g) for the column pair
-        v16f lowS[2];
-        if constexpr (kLora) {
-          const unsigned char* zb = g.zp + (size_t)blk * NKK * 3u * kBlockBytes + lane * 16;
-          // operand of packed column block cb = tcol0/32 + j: rows 16kk + 8h + 0..7 of column 4c + j
-          const unsigned char* bb0 =
-              g.bp + ((size_t)gi * ncb_total + tcol0 / 32u + 2u * jp) * NKK * kBlockBytes + lane * 16;
-#pragma unroll
-          for (int kk = 0; kk < NKK; ++kk) {
-            v8us zf[3];
-#pragma unroll
-            for (int t3 = 0; t3 < 3; ++t3) zf[t3] = *reinterpret_cast<const v8us*>(zb + (kk * 3 + t3) * kBlockBytes);
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-              const v8bf bb = __builtin_bit_cast(
-                  v8bf, *reinterpret_cast<const v8us*>(bb0 + ((size_t)j * NKK + kk) * kBlockBytes));
-              v16f cur;
-              if (kk == 0) {
-#pragma unroll
-                for (int e = 0; e < 16; ++e) cur[e] = 0.0f;
-              } else {
-                cur = lowS[j];
-              }
-              cur = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, zf[2]), bb, cur, 0, 0, 0);
-              cur = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, zf[1]), bb, cur, 0, 0, 0);
-              cur = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, zf[0]), bb, cur, 0, 0, 0);
-              lowS[j] = cur;
-            }
-          }
-          const float sgrp = g.lora_scaling[gi];
-#pragma unroll
-          for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) lowS[j][e] = lowS[j][e] * sgrp;
-        }
-
-        // ---- section B
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          // row 8*(v/4) + 4*h + v%4 of the block: its data sits in that lane (cross-lane read on
-          // the LDS crossbar, which is idle here; no vector-ALU work)
-          const int src_lane_addr = row_addr + 4 * (8 * (v >> 2) + (v & 3));
-          const uint32_t rowoff = (uint32_t)__builtin_amdgcn_ds_bpermute(src_lane_addr, (int)off_lane);
-          const float sxv =
-              __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(src_lane_addr, __builtin_bit_cast(int, sx_lane)));
-          const float t0 = (float)acc[bi][2 * jp][v] * sxv;
-          const float t1 = (float)acc[bi][2 * jp + 1][v] * sxv;
-          // same f32 operations, in the same order, as the reference epilogue: a fused
-          // multiply-add here would flip rare bf16 roundings that SwiGLU then amplifies
-          float y0 = t0 * sw[2 * jp];
-          float y1 = t1 * sw[2 * jp + 1];
-          if constexpr (kLora) {
-            y0 = y0 + lowS[0][v];
-            y1 = y1 + lowS[1][v];
-          }
-          bool row_valid = fast || rowoff != 0xffffffffu;
-          if (kLora && ghi > glo)  // boundary block: this pass owns only the rows of group gi
-            row_valid = row_valid && (__builtin_amdgcn_ds_bpermute(src_lane_addr, grp_lane) == gi);
-          uint32_t mine_bits;
-          if (EPI == kEpiSwiglu) {
-            // (y0, y1) = (gate, up) of the product column ncol/2 + jp
-            const uint32_t f = pack_bf16x2(y0, y1);
-            mine_bits = __float_as_uint(swiglu_f32(__uint_as_float(f << 16), __uint_as_float(f & 0xffff0000u)));
-          } else {
-            if (g.residual && row_valid) {
-              uint32_t rr;
-              if (fast) {
-                rr = *reinterpret_cast<const uint32_t*>(g.residual + rowoff + ncol + 2u * jp);
-              } else {
-                rr = 0;
-                if (ncol + 2u * jp < g.N) rr |= (uint32_t)g.residual[rowoff + ncol + 2u * jp];
-                if (ncol + 2u * jp + 1u < g.N) rr |= (uint32_t)g.residual[rowoff + ncol + 2u * jp + 1u] << 16;
-              }
-              y0 = y0 + __uint_as_float(rr << 16);
-              y1 = y1 + __uint_as_float(rr & 0xffff0000u);
-            }
-            mine_bits = pack_bf16x2(y0, y1);
-          }
-          if (jp == 0) {
-            hold[v] = mine_bits;
-            continue;
-          }
-          if (!row_valid) continue;
-          if (EPI == kEpiSwiglu) {
-            const uint32_t pk = pack_bf16x2(__uint_as_float(hold[v]), __uint_as_float(mine_bits));
-            uint16_t* o = reinterpret_cast<uint16_t*>(g.out) + rowoff + (ncol >> 1);
-            if (fast) {
-              *reinterpret_cast<uint32_t*>(o) = pk;
-            } else {
-              if ((ncol >> 1) < n_out) o[0] = (uint16_t)(pk & 0xffffu);
-              if ((ncol >> 1) + 1u < n_out) o[1] = (uint16_t)(pk >> 16);
-            }
-          } else {
-            uint16_t* o = reinterpret_cast<uint16_t*>(g.out) + rowoff + ncol;
-            if (fast) {
-              *reinterpret_cast<uint2*>(o) = make_uint2(hold[v], mine_bits);
-            } else {
-              if (ncol + 0u < g.N) o[0] = (uint16_t)(hold[v] & 0xffffu);
-              if (ncol + 1u < g.N) o[1] = (uint16_t)(hold[v] >> 16);
-              if (ncol + 2u < g.N) o[2] = (uint16_t)(mine_bits & 0xffffu);
-              if (ncol + 3u < g.N) o[3] = (uint16_t)(mine_bits >> 16);
-            }
-          }
-        }
-      }
-      }  // groups of the block
+      gemm_epilogue_block<EPI, NKK>(g, EpilogueFromMemory{g, pbase, tcol0, ncb_total}, acc[bi], sw, tcol0, full_n, n_out);
     };
-    epilogue_block(std::integral_constant<int, 0>{});
-    if constexpr (kWR == 2) epilogue_block(std::integral_constant<int, 1>{});
+    epilogue_block(0);
+    if constexpr (kWR == 2) epilogue_block(1);
   }
 }
 

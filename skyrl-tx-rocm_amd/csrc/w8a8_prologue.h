@@ -166,10 +166,12 @@ __device__ inline void route_rows_block(const int32_t* __restrict__ idx, uint32_
 // ---------------------------------------------------------------------------------------
 // Tables for rows that arrive already grouped (ragged groups of an expert layer,
 // skyrl/tx/layers/util.py:8-59): group g owns group_sizes[g] consecutive rows and is padded
-// to a multiple of `pad` (64 or 128) grouped slots so that a GEMM tile never mixes two weights.
+// to a multiple of 32 grouped slots so that a 32-row block never mixes two weights.
 //   src_row[p]   = original row of slot p, -1 for padding
 //   dst_pos[m]   = slot of row m, -1 for rows beyond sum(group_sizes) (their output is zero)
 //   blk_range[b] = g | g << 16 for the 32-row blocks in use, -1 beyond
+//   tile_tab     = number of row tiles, then first block | blocks << 32 | group << 48 of each: a group's blocks
+//                  in the fewest tiles of at most tile_blocks, of heights that differ by one at most
 // ---------------------------------------------------------------------------------------
 constexpr int kMaxGroups = 1024;
 // Exclusive prefix sums of one value per thread over a workgroup of 1024 threads, every partial sum capped
@@ -211,7 +213,7 @@ __device__ inline uint32_t block_prefix_capped(uint32_t v, uint32_t limit, uint3
 __device__ inline void route_groups_block(const int32_t* __restrict__ group_sizes, uint32_t M, uint32_t n_groups,
                                           uint32_t slots, int32_t* __restrict__ src_row,
                                           int32_t* __restrict__ dst_pos, int32_t* __restrict__ blk_range,
-                                          uint32_t pad, uint16_t* __restrict__ zero_out, uint32_t zero_cols,
+                                          uint64_t* __restrict__ tile_tab, uint32_t tile_blocks, uint16_t* __restrict__ zero_out, uint32_t zero_cols,
                                           uint32_t part, uint32_t n_parts) {
   __shared__ uint32_t row_start[kMaxGroups + 1];
   __shared__ uint32_t slot_start[kMaxGroups + 1];
@@ -222,8 +224,17 @@ __device__ inline void route_groups_block(const int32_t* __restrict__ group_size
   const uint32_t r0 = block_prefix_capped((uint32_t)sz, M, &rows_total);
   // the group's rows after the cap: up to the next group's start
   const uint32_t r1 = (uint64_t)r0 + (uint32_t)sz > M ? M : r0 + (uint32_t)sz;
-  const uint32_t padded = (r1 - r0 + pad - 1u) & ~(pad - 1u);
-  const uint32_t p0 = block_prefix_capped(padded, 0xffffffffu, &slots_total);
+  const uint32_t nblk = (r1 - r0 + 31u) / 32u;
+  const uint32_t p0 = block_prefix_capped(nblk * 32u, 0xffffffffu, &slots_total);
+  const uint32_t n_tiles = (nblk + tile_blocks - 1u) / tile_blocks;
+  uint32_t tiles_total;
+  const uint32_t t0 = block_prefix_capped(n_tiles, 0xffffffffu, &tiles_total);
+  if (part == 0 && tid == 0) tile_tab[0] = tiles_total;
+  for (uint32_t i = part; i < n_tiles; i += n_parts) {
+    const uint32_t low = nblk / n_tiles, high = nblk % n_tiles;  // the first `high` tiles have a block more
+    const uint32_t first = i * low + (i < high ? i : high), count = low + (i < high ? 1u : 0u);
+    tile_tab[1u + t0 + i] = (uint64_t)(p0 / 32u + first) | (uint64_t)count << 32 | (uint64_t)tid << 48;
+  }
   if (tid < n_groups) { row_start[tid] = r0; slot_start[tid] = p0; }
   if (tid == 0) { row_start[n_groups] = rows_total; slot_start[n_groups] = slots_total; }
   __syncthreads();
@@ -594,7 +605,8 @@ struct LoraPrepArgs {
   uint32_t a_operand_steps, a_operand_rb;  // or: ceil(K / 64) and the 32-wide rank blocks of lora_a_kernel's operand order
   // grouped (ragged) call: the routing block lays the groups out from their sizes instead
   const int32_t* group_sizes;  // int32 [n_groups] or null
-  uint32_t group_pad;          // slots every group is padded to
+  uint64_t* tile_tab;          // row tiles of the grouped GEMM ...
+  uint32_t tile_blocks;        // ... and the 32-row blocks they hold at most
   uint16_t* zero_out;          // bf16 [M, zero_cols]: rows beyond the groups are cleared, or null
   uint32_t zero_cols;
   // row statistics of the dense call (STATS != 0): sixteen rows per block, behind the routing block
@@ -720,8 +732,8 @@ __global__ __launch_bounds__(1024, 8) void lora_prep_kernel(LoraPrepArgs p) {
   if (b < p.route_blocks) {
     __builtin_amdgcn_s_setprio(3);  // a chain of short steps beside waves that wait for memory
     if (p.group_sizes)
-      route_groups_block(p.group_sizes, p.M, p.n_groups, p.slots, p.src_row, p.dst_pos, p.blk_range, p.group_pad,
-                         p.zero_out, p.zero_cols, b, p.route_blocks);
+      route_groups_block(p.group_sizes, p.M, p.n_groups, p.slots, p.src_row, p.dst_pos, p.blk_range, p.tile_tab,
+                         p.tile_blocks, p.zero_out, p.zero_cols, b, p.route_blocks);
     else
       route_rows_block(p.idx, p.M, p.n_groups, p.slots, p.src_row, p.dst_pos, p.slot_group, p.blk_range, nullptr,
                        p.route_pad > 1u ? p.route_pad : 1u);
