@@ -483,6 +483,7 @@ int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
     pa.route_pad = pad_groups ? 32u : 1u;
     pa.a_operand_kb = w.KB;  // the quantizer reads A in MFMA operand order
     pa.stat_blocks = (p->m + 15u) / 16u;
+    pa.stat_rows = p->m;
     pa.x = static_cast<const uint16_t*>(p->x);
     pa.gamma = p->rms_gamma; pa.eps = p->rms_eps;
     pa.row_scale = reinterpret_cast<float*>(ws + w.row_scale);
@@ -590,8 +591,8 @@ int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
 }
 
 struct GroupedLayout {
-  uint64_t xq, sx, zp, at, bp, src_row, dst_pos, blk_range, tile_tab, total;
-  uint32_t slots, nkk, K_pad, KB, n_steps, steps_per_wave, tile_blocks, max_tiles;
+  uint64_t xq, sx, zp, at, bp, row_scale, src_row, dst_pos, blk_range, tile_tab, total;
+  uint32_t slots, nkk, K_pad, KB, tile_blocks, max_tiles;
 };
 
 // 32-row blocks that a GEMM tile holds at most, 4 or 8; the flags force either (8 only where K has the steps it
@@ -618,15 +619,14 @@ GroupedLayout make_grouped_layout(uint32_t m, uint32_t k, uint32_t n, uint32_t n
   w.slots = (uint32_t)(((uint64_t)m + 31u * (uint64_t)n_groups + 31u) / 32u * 32u);
   w.max_tiles = w.slots / 32u / w.tile_blocks + n_groups;
   w.nkk = rank_chunks(rank);
-  w.n_steps = (k + 63u) / 64u;
-  w.steps_per_wave = (w.n_steps + 15u) / 16u;
   uint64_t off = 0;
   // (the LoRA operands a caller may vouch for come first, as in make_layout: their places depend on
   // (k, n, n_groups, rank) only, not on the row count)
-  w.at = off; off += rank ? align256((uint64_t)n_groups * rank * k * 2u) : 0u;
+  w.at = off; off += rank ? align256((uint64_t)n_groups * w.KB * w.nkk * kBlockBytes) : 0u;
   w.bp = off; off += rank ? align256((uint64_t)n_groups * (n_padded(n) / 32u) * w.nkk * kBlockBytes) : 0u;
   w.xq = off; off += align256((uint64_t)w.slots * w.K_pad);
   w.sx = off; off += align256((uint64_t)w.slots * 4u);
+  w.row_scale = off; off += align256((uint64_t)m * 4u);
   w.src_row = off; off += align256((uint64_t)w.slots * 4u);
   w.dst_pos = off; off += align256((uint64_t)m * 4u);
   w.blk_range = off; off += align256((uint64_t)(w.slots / 32u) * 4u);
@@ -634,6 +634,25 @@ GroupedLayout make_grouped_layout(uint32_t m, uint32_t k, uint32_t n, uint32_t n
   w.zp = off; off += rank ? align256((uint64_t)(w.slots / 32u) * w.nkk * 3u * kBlockBytes) : 0u;
   w.total = off;
   return w;
+}
+
+// Four waves per half block once the half blocks fill the chip several times over (a wave then has more of K to itself and
+// the sum over the waves costs less), else sixteen (the pass is a chain of latencies).  Measured, 16 / 4 waves, 128 groups, rank 16:
+// 16384 gathered rows of 2048: 44 / 31 us, 8168: 25 / 20, 128 (256 half blocks at most): 8.2 / 9.8; 16384 rows of 768: 22 / 14.5.
+int launch_grouped_quant(const QuantLoraArgs& q, uint32_t nkk, hipStream_t s) {
+  const bool few_waves = q.M >= 4096u;
+  const dim3 grid(q.n_half_blocks);
+#define W8A8_GQL(CB)                                                                                          \
+  if (few_waves) hipLaunchKernelGGL((quant_lora_kernel<CB, false, 4u>), grid, dim3(256), 0, s, q);            \
+  else hipLaunchKernelGGL((quant_lora_kernel<CB, false, 16u>), grid, dim3(1024), 0, s, q)
+  switch (nkk) {
+    case 0: W8A8_GQL(0); break;
+    case 1: W8A8_GQL(1); break;
+    case 2: W8A8_GQL(2); break;
+    default: W8A8_GQL(4); break;
+  }
+#undef W8A8_GQL
+  return launch_status();
 }
 
 int run_grouped(const mi355_w8a8_grouped_problem* p, hipStream_t s) {
@@ -685,12 +704,15 @@ int run_grouped(const mi355_w8a8_grouped_problem* p, hipStream_t s) {
   const bool skip_gemm = (p->flags & MI355_W8A8_FLAG_SKIP_GEMM) != 0;
   if (skip_prologue && (p->aux_x_codes || p->aux_x_scales)) return MI355_W8A8_ERR_UNSUPPORTED;
 
-  // launch 1: the slot layout of the groups next to the LoRA operand re-layouts
+  // Launch 1: the slot layout of the groups next to the rows' statistics and the LoRA operand layouts.  With a row map the
+  // statistics are the source rows' (a token's row is read once, not once per expert), unless there are more of those than rows.
+  const bool by_source = p->x_row_map && x_rows <= p->m;
   if (!skip_prologue) {
     LoraPrepArgs pa{};
     pa.src_row = src_row; pa.dst_pos = dst_pos; pa.blk_range = blk_range;
     pa.group_sizes = p->group_sizes;
     pa.tile_tab = reinterpret_cast<uint64_t*>(ws + w.tile_tab); pa.tile_blocks = w.tile_blocks;
+    pa.zero_out = static_cast<uint16_t*>(p->out); pa.zero_cols = n_out;
     pa.lora_a = static_cast<const uint16_t*>(p->lora_a);
     pa.lora_b = static_cast<const uint16_t*>(p->lora_b);
     pa.at = reinterpret_cast<uint16_t*>(ws + w.at);
@@ -699,52 +721,50 @@ int run_grouped(const mi355_w8a8_grouped_problem* p, hipStream_t s) {
     pa.ncb = n_padded(p->n) / 32u; pa.slots = w.slots;
     // (the layout is filled slot by slot: a few workgroups, each with the prefix sums of its own)
     pa.route_blocks = (w.slots + 2047u) / 2048u < 16u ? (w.slots + 2047u) / 2048u : 16u;
+    pa.a_operand_kb = w.KB;
+    pa.stat_rows = by_source ? x_rows : p->m;
+    pa.stat_blocks = (pa.stat_rows + 15u) / 16u;
+    pa.x = static_cast<const uint16_t*>(p->x);
+    if (p->x_row_map && !by_source) { pa.stat_map = p->x_row_map; pa.stat_div = x_repeat; pa.stat_limit = x_rows; }
+    pa.row_scale = reinterpret_cast<float*>(ws + w.row_scale);
     uint32_t b_blocks = 0;
-    // (a caller that vouches for the operand packs of an earlier call on this workspace keeps them: the
-    // launch then only lays out the slots)
+    // (a caller that vouches for the operand packs of an earlier call on this workspace keeps them)
     if (lora && !(p->flags & MI355_W8A8_FLAG_LORA_PACK_VALID)) {
-      const uint64_t a_items = (uint64_t)p->n_groups * p->k * ((p->rank + 7u) / 8u);
+      const uint64_t a_items = (uint64_t)p->n_groups * w.KB * w.nkk * (p->rank % 4u ? 64u : 16u);
       const uint64_t b_items = (uint64_t)p->n_groups * pa.ncb * w.nkk * (p->n % 4u ? 64u : 16u);
       pa.a_blocks = (uint32_t)((a_items + 1023u) / 1024u);
       b_blocks = (uint32_t)((b_items + 1023u) / 1024u);
     }
-    hipLaunchKernelGGL((lora_prep_kernel<0>), dim3(pa.route_blocks + pa.a_blocks + b_blocks), dim3(1024), 0, s, pa);
+    hipLaunchKernelGGL((lora_prep_kernel<1>), dim3(pa.route_blocks + pa.stat_blocks + pa.a_blocks + b_blocks), dim3(1024), 0, s, pa);
     if ((st = launch_status())) return st;
   }
 
-  // launch 2: the quantizer, a wave per row (measured faster here than the fused quantizer + LoRA-A
-  // kernel of the dense path, whose 16-slot workgroups are sized for longer rows)
+  // launch 2: codes and LoRA-A projection in one pass over the gathered rows
   if (!skip_prologue) {
-  QuantArgs q{};
-  q.x = static_cast<const uint16_t*>(p->x);
-  q.M = p->m; q.K = p->k; q.K_pad = w.K_pad; q.KB = w.KB;
-  q.dst_pos = dst_pos;
-  q.xq_packed = ws + w.xq;
-  q.sx_slots = reinterpret_cast<float*>(ws + w.sx);
-  q.codes_rm = p->aux_x_codes;
-  q.scales_rm = p->aux_x_scales;
-  q.zero_out = static_cast<uint16_t*>(p->out);
-  q.zero_cols = n_out;
-  q.row_map = p->x_row_map; q.row_div = x_repeat; q.row_limit = x_rows;
-  if ((st = launch_quant<false>(q, s))) return st;
-  }
-
-  // launch 3: LoRA-A projection per 32-slot block
-  if (lora && !skip_prologue) {
-    LoraAArgs la{};
-    la.xsrc = static_cast<const uint16_t*>(p->x);
-    la.at = reinterpret_cast<const uint16_t*>(ws + w.at);
-    la.src_row = src_row;
-    la.slot_group = nullptr;
-    la.blk_range = blk_range;
-    la.row_map = p->x_row_map; la.row_div = x_repeat; la.row_limit = x_rows;
-    la.zp = ws + w.zp;
-    la.M = p->m; la.K = p->k; la.r = p->rank; la.nkk = w.nkk;
-    la.steps_per_wave = w.steps_per_wave; la.n_steps = w.n_steps;
-    la.nterms = (p->flags & MI355_W8A8_FLAG_LORA_SPLIT2) ? 2u : 3u;
-    la.n_blocks = w.slots / 32u;
-    const dim3 grid(w.slots / 32u);
-    if ((st = launch_lora_a(la, w.nkk, grid, s))) return st;
+    QuantLoraArgs q{};
+    q.x = static_cast<const uint16_t*>(p->x);
+    q.row_scale = reinterpret_cast<const float*>(ws + w.row_scale);
+    q.M = p->m; q.K = p->k; q.K_pad = w.K_pad; q.KB = w.KB;
+    q.n_half_blocks = w.slots / 16u;
+    q.src_row = src_row; q.blk_range = blk_range;
+    q.xq_packed = ws + w.xq;
+    q.sx_slots = reinterpret_cast<float*>(ws + w.sx);
+    q.at = lora ? reinterpret_cast<const uint16_t*>(ws + w.at) : nullptr;
+    q.zp = ws + w.zp;
+    q.r = p->rank; q.nkk = w.nkk;
+    q.nterms = (p->flags & MI355_W8A8_FLAG_LORA_SPLIT2) ? 2u : 3u;
+    q.group_pad = 32u;
+    q.row_map = p->x_row_map; q.row_div = x_repeat; q.row_limit = x_rows; q.scale_by_source = by_source ? 1u : 0u;
+    if ((st = launch_grouped_quant(q, lora ? w.nkk : 0u, s))) return st;
+    if (p->aux_x_codes || p->aux_x_scales) {  // the caller's copies, row by row (rows without a slot among them)
+      QuantArgs c{};
+      c.x = static_cast<const uint16_t*>(p->x);
+      c.M = p->m; c.K = p->k; c.K_pad = w.K_pad; c.KB = w.KB;
+      c.codes_rm = p->aux_x_codes;
+      c.scales_rm = p->aux_x_scales;
+      c.row_map = p->x_row_map; c.row_div = x_repeat; c.row_limit = x_rows;
+      if ((st = launch_quant<false>(c, s))) return st;
+    }
   }
   if (skip_gemm) return MI355_W8A8_OK;
 

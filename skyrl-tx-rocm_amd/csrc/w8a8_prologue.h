@@ -609,8 +609,10 @@ struct LoraPrepArgs {
   uint32_t tile_blocks;        // ... and the 32-row blocks they hold at most
   uint16_t* zero_out;          // bf16 [M, zero_cols]: rows beyond the groups are cleared, or null
   uint32_t zero_cols;
-  // row statistics of the dense call (STATS != 0): sixteen rows per block, behind the routing block
-  uint32_t stat_blocks;
+  // row statistics (STATS != 0): sixteen rows per block, behind the routing block
+  uint32_t stat_blocks, stat_rows;
+  const int32_t* stat_map;     // statistics of row m are those of source row mapped_row(stat_map[m], ...), or null
+  uint32_t stat_div, stat_limit;
   const uint16_t* x;           // bf16 [M, K]
   const float* gamma;          // f32 [K] (STATS == 2)
   float eps;
@@ -654,10 +656,11 @@ __device__ inline void row_stats(const LoraPrepArgs& p, uint32_t m) {
   constexpr uint32_t kPieces = RMS ? 4 : 8;
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t row_bytes = 2u * p.K;
+  const uint32_t xrow = p.stat_map ? mapped_row(p.stat_map[m], p.stat_div, p.stat_limit) : m;
   // (the row and the norm weights through buffer resources that end with them: a load under a lane condition
   // becomes a branch with a wait of its own, and the loads then run one after the other)
   const __amdgpu_buffer_rsrc_t xrsrc =
-      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p.x) + (size_t)m * p.K, 0, (int)row_bytes, 0x00020000);
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p.x) + (size_t)xrow * p.K, 0, (int)row_bytes, 0x00020000);
   const __amdgpu_buffer_rsrc_t grsrc =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.gamma), 0, RMS ? (int)(p.K * 4u) : 0, 0x00020000);
   uint32_t amax_bits = 0;
@@ -743,7 +746,7 @@ __global__ __launch_bounds__(1024, 8) void lora_prep_kernel(LoraPrepArgs p) {
   if constexpr (STATS != 0) {
     if (b < p.stat_blocks) {
       const uint32_t m = b * 16u + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-      if (m < p.M) row_stats<STATS == 2>(p, m);
+      if (m < p.stat_rows) row_stats<STATS == 2>(p, m);
       return;
     }
     b -= p.stat_blocks;
@@ -1018,6 +1021,9 @@ __global__ __launch_bounds__(1024) void lora_a_kernel(LoraAArgs a) {
 // (statistics, routing, operand layouts) + 54 us against 14 us (layouts, routing) + 120 us; 333 x 4096, 4 adapters
 // of rank 64: 7 + 16 us against 6 + 20 us; 4096 x 4096 with RMSNorm, where sixteen rows did fit the LDS:
 // 20 + 28 us against 14 + 32 us.
+// The grouped (per-expert) call takes the same pass, its rows gathered through a row map and their statistics taken once
+// per source row; as a quantizer and a LoRA-A launch over the gathered rows, 16384 of 2048, top 8 of 2048 tokens, it took
+// 7 + 26 + 30 us, now 7 + 31.
 // ---------------------------------------------------------------------------------------
 struct QuantLoraArgs {
   const uint16_t* x;        // bf16 [M, K]: the rows, or (RMS false) rows that are normalized already
@@ -1035,6 +1041,10 @@ struct QuantLoraArgs {
   uint32_t r, nkk, nterms;
   uint32_t* tile_ctr;       // 256 words cleared for the GEMM launches' tile counters, or null
   uint32_t group_pad;       // > 1: whole half blocks may be empty
+  // Optional gather on the way in (see QuantArgs): source row = row_map[row] / row_div, clamped to row_limit;
+  // row_scale then holds a value per source row (scale_by_source) or per row
+  const int32_t* row_map;
+  uint32_t row_div, row_limit, scale_by_source;
 };
 
 // Row-major copy of the packed codes for a caller that asks for them (one workgroup per slot).
@@ -1049,12 +1059,13 @@ __global__ __launch_bounds__(256) void codes_row_major_kernel(const unsigned cha
 
 constexpr uint32_t kPaddedRouteMaxRows = 8192;  // groups start on block boundaries up to here (padded_groups_fit)
 
-template <int CB, bool RMS>  // CB: 16-wide rank blocks (0 = no LoRA, 1, 2, 4)
-__global__ __launch_bounds__(1024) void quant_lora_kernel(QuantLoraArgs a) {
+template <int CB, bool RMS, uint32_t WAVES = 16>  // CB: 16-wide rank blocks (0 = no LoRA, 1, 2, 4)
+__global__ __launch_bounds__(WAVES * 64, 4) void quant_lora_kernel(QuantLoraArgs a) {
   constexpr int kCB = CB > 0 ? CB : 1;
   constexpr uint32_t kRing = CB == 4 || (CB == 2 && RMS) ? 2 : 4;  // operand sets (what 128 registers per lane hold)
   constexpr uint32_t kAhead = 4;  // k-blocks of x a wave has in flight; a multiple of kRing
-  __shared__ float red[CB > 0 ? 8 : 1][kCB][4][64];  // wave tiles on their way to waves 0..7, then 0..3
+  static_assert(WAVES == 4 || WAVES == 16, "the reduction ends in four waves");
+  __shared__ float red[CB > 0 ? (WAVES == 16 ? 8 : 4) : 1][kCB][4][64];  // wave tiles on their way to waves 0..7, then 0..3
   __shared__ float zs[16][kCB * 16 + 1];
   const uint32_t tid = threadIdx.x, lane = tid & 63u;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1069,11 +1080,12 @@ __global__ __launch_bounds__(1024) void quant_lora_kernel(QuantLoraArgs a) {
     return;  // workgroup-uniform: padded groups leave whole stretches of slots empty: nothing reads their codes, scales or z
   // (a slot without a row works on row 0: nothing reads what it leaves, and no load sits under a lane condition)
   const uint32_t row = src < 0 ? 0u : (uint32_t)src;
-  const float scale = a.row_scale[row];
+  const uint32_t xrow = a.row_map ? mapped_row(a.row_map[row], a.row_div, a.row_limit) : row;
+  const float scale = a.row_scale[a.scale_by_source ? xrow : row];
   const float inv = RMS ? a.row_inv[row] : 1.0f;
   if (wave == 0 && lane < 16u) a.sx_slots[hb * 16u + i] = scale;
   const float rscale = __builtin_amdgcn_rcpf(scale);
-  const unsigned char* const xr = reinterpret_cast<const unsigned char*>(a.x) + (size_t)row * 2u * a.K;
+  const unsigned char* const xr = reinterpret_cast<const unsigned char*>(a.x) + (size_t)xrow * 2u * a.K;
   const uint32_t range = (CB > 0 && a.blk_range) ? (uint32_t)a.blk_range[pb] : 0u;
   const uint32_t glo = range & 0xffffu, ghi = range >> 16;
   const uint32_t rowgrp = (CB > 0 && ghi > glo && a.slot_group) ? (uint32_t)a.slot_group[hb * 16u + i] : glo;
@@ -1084,37 +1096,37 @@ __global__ __launch_bounds__(1024) void quant_lora_kernel(QuantLoraArgs a) {
   unsigned char* const xq_dst =
       a.xq_packed + (size_t)pb * a.KB * kBlockBytes + (16u * half16 + i + 32u * (q >> 1)) * 16u + 8u * (q & 1u);
 
-  // The wave's j-th k-block is wave + 16 j.  Everything beyond the last block is read as zeros without a
+  // The wave's j-th k-block is wave + WAVES j.  Everything beyond the last block is read as zeros without a
   // condition: A and the norm weights through buffer resources that end with the data, x from the row's start.
   const __amdgpu_buffer_rsrc_t grsrc =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.gamma), 0, RMS ? (int)(a.K * 4u) : 0, 0x00020000);
   const uint32_t at_bytes = a.KB * (uint32_t)kCB * kBlockBytes;  // of one group
   const uint32_t kq = wave * 32u + q * 8u;                       // the lane's k in its wave's first k-block
   auto fetch_x = [&](uint32_t j) -> uint4 {
-    const uint32_t k0 = kq + 512u * j;
+    const uint32_t k0 = kq + WAVES * 32u * j;
     return *reinterpret_cast<const uint4*>(xr + 2u * (k0 < a.K ? k0 : 0u));  // (beyond K: zeroed where it is used)
   };
   struct Operands { v4i w[kCB]; v4f g0, g1; };
   auto fetch_operands = [&](const __amdgpu_buffer_rsrc_t& arsrc, uint32_t j, Operands& o) {
     if constexpr (CB > 0) {  // CB consecutive 1 KiB pieces (zero beyond K and the rank)
-      const uint32_t off = (wave + 16u * j) * (uint32_t)(kCB * kBlockBytes) + lane * 16u;
+      const uint32_t off = (wave + WAVES * j) * (uint32_t)(kCB * kBlockBytes) + lane * 16u;
 #pragma unroll
       for (int b = 0; b < CB; ++b) o.w[b] = __builtin_amdgcn_raw_buffer_load_b128(arsrc, off + b * kBlockBytes, 0, 0);
     }
     if constexpr (RMS) {
-      const uint32_t off = (kq + 512u * j) * 4u;
+      const uint32_t off = (kq + WAVES * 32u * j) * 4u;
       o.g0 = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(grsrc, off, 0, 0));
       o.g1 = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(grsrc, off + 16u, 0, 0));
     }
   };
   const bool scale_safe = scale > 1e-30f && scale < 1e30f;
   auto work = [&](auto codes, bool in_group, uint32_t j, const uint4& rawx, const Operands& o) {
-    const uint32_t kb = wave + 16u * j;
+    const uint32_t kb = wave + WAVES * j;
     uint4 raw = rawx;
     if constexpr (RMS)
       raw = rms_normalize8(rawx, inv, make_float4(o.g0[0], o.g0[1], o.g0[2], o.g0[3]), make_float4(o.g1[0], o.g1[1], o.g1[2], o.g1[3]));
     if (kb * 32u + 32u > a.K) {  // wave-uniform: the last k-block of an odd K, and the padding behind it
-      const bool live = kq + 512u * j < a.K;
+      const bool live = kq + WAVES * 32u * j < a.K;
       raw.x = live ? raw.x : 0u; raw.y = live ? raw.y : 0u; raw.z = live ? raw.z : 0u; raw.w = live ? raw.w : 0u;
     }
     if constexpr (decltype(codes)::value) {
@@ -1166,7 +1178,7 @@ __global__ __launch_bounds__(1024) void quant_lora_kernel(QuantLoraArgs a) {
   // A pass over the k-blocks, kAhead per trip: the x of kAhead k-blocks and the other operands of kRing - 1
   // are in flight beside the one at work.  (With few workgroups on the chip the loop is a chain of those
   // loads' latencies; no load or store in it is conditional, so the compiler's waits can count.)
-  const uint32_t n_j = wave < a.KB ? (a.KB - wave + 15u) / 16u : 0u;
+  const uint32_t n_j = wave < a.KB ? (a.KB - wave + WAVES - 1u) / WAVES : 0u;
   auto pass = [&](auto codes, uint32_t grp, bool in_group) {
     const __amdgpu_buffer_rsrc_t arsrc = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<uint16_t*>(a.at) + (size_t)grp * (at_bytes / 2u), 0, CB > 0 ? (int)at_bytes : 0, 0x00020000);
@@ -1202,9 +1214,9 @@ __global__ __launch_bounds__(1024) void quant_lora_kernel(QuantLoraArgs a) {
   }
   if constexpr (CB == 0) return;
 
-  // ---- fixed-order sum of the 16 wave tiles: 8..15 onto 0..7, 4..7 onto 0..3, then 0+1+2+3
+  // ---- fixed-order sum of the wave tiles: of 16, 8..15 onto 0..7, 4..7 onto 0..3; then 0+1+2+3
 #pragma unroll 1
-  for (uint32_t half = 8u; half >= 4u; half >>= 1) {
+  for (uint32_t half = WAVES / 2u; half >= 4u; half >>= 1) {
     if (wave >= half && wave < 2u * half) {
 #pragma unroll
       for (int b = 0; b < kCB; ++b)
@@ -1228,14 +1240,14 @@ __global__ __launch_bounds__(1024) void quant_lora_kernel(QuantLoraArgs a) {
   }
   __syncthreads();
   // MFMA result layout: lane l holds column l % 16 and rows 4 * (l / 16) + e
-  for (uint32_t t = tid; t < (uint32_t)kCB * 256u; t += 1024u) {
+  for (uint32_t t = tid; t < (uint32_t)kCB * 256u; t += WAVES * 64u) {
     const uint32_t l = t & 63u, e = (t >> 6) & 3u, b = t >> 8;
     const float sum = ((red[0][b][e][l] + red[CB > 0 ? 1 : 0][b][e][l]) + red[CB > 0 ? 2 : 0][b][e][l]) + red[CB > 0 ? 3 : 0][b][e][l];
     zs[4u * (l >> 4) + e][b * 16u + (l & 15u)] = sum;
   }
   __syncthreads();
   // zp[pb][kk][term][lane64][8]: lane = row % 32 + 32 * hh holds rank columns 16 kk + 8 hh + 0..7
-  for (uint32_t t = tid; t < a.nkk * 3u * 32u; t += 1024u) {
+  for (uint32_t t = tid; t < a.nkk * 3u * 32u; t += WAVES * 64u) {
     const uint32_t row = t & 15u, hh = (t >> 4) & 1u, term = (t >> 5) % 3u, kk = t / 96u;
     v8us o;
 #pragma unroll

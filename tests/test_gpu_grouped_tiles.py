@@ -59,3 +59,30 @@ def test_row_tiles(sizes, k, n, rank, swiglu):
     assert np.all(got[sum(sizes):] == 0)
     ok = o.within_tolerance(got, want)
     assert ok.all(), int((~ok).sum())
+
+
+@pytest.mark.parametrize("m,x_rows,repeat,k,rank", [
+    (40, 5, 8, 136, 16), (300, 700, 1, 512, 24), (4100, 513, 8, 320, 8), (4097, 5000, 1, 256, 0), (24, 24, 3, 1032, 40),
+])
+def test_mapped_rows_equal_gathered_rows(m, x_rows, repeat, k, rank):
+    """Rows read through a map -- fewer source rows than rows (their statistics are taken per source row) and more,
+    repeated and out of range entries, both workgroup sizes of the quantizer -- against the same rows gathered."""
+    import torch
+
+    w8 = load_package().w8a8_lora
+    dev, e, n = torch.device("cuda:0"), 5, 264
+    gen = torch.Generator(device=dev).manual_seed(m + k)
+    x = torch.randn(x_rows, k, device=dev, generator=gen).to(torch.bfloat16)
+    rmap = torch.randint(-3, x_rows * repeat + 9, (m,), device=dev, generator=gen, dtype=torch.int32)
+    gw = w8.prepare_grouped_weight(torch.randint(-127, 128, (e, k, n), device=dev, generator=gen, dtype=torch.int8),
+                                   torch.rand(e, n, device=dev, generator=gen) * 0.01)
+    a = (torch.randn(e, k, rank, device=dev, generator=gen) * 0.02).to(torch.bfloat16) if rank else None
+    b = (torch.randn(e, rank, n, device=dev, generator=gen) * 0.02).to(torch.bfloat16) if rank else None
+    sizes = torch.tensor([m // 3, 0, m // 4, 7, m // 5], dtype=torch.int32)
+    src = torch.div(rmap.clamp(min=0), repeat, rounding_mode="floor").clamp(max=x_rows - 1).long()
+    print(f"[case] mapped rows m={m} x_rows={x_rows} repeat={repeat} k={k} rank={rank}", flush=True)
+    want, want_aux = w8.grouped_forward(x[src], sizes, gw, a, b, 1.0 if rank else None, return_aux=True)
+    got, aux = w8.grouped_forward(x, sizes, gw, a, b, 1.0 if rank else None, row_map=rmap, row_repeat=repeat, return_aux=True)
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+    for name in ("x_codes", "x_scales", "acc"):
+        assert torch.equal(aux[name], want_aux[name])
