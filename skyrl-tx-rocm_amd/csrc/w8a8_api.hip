@@ -1379,8 +1379,10 @@ int run_grouped_backward(const mi355_w8a8_grouped_bwd_problem* p, hipStream_t s)
     pa.a_blocks = lora ? (uint32_t)(((uint64_t)p->n_groups * p->k * ((p->rank + 7u) / 8u) + 1023u) / 1024u) : 0u;
     pa.ap_blocks = lora ? (uint32_t)(((uint64_t)p->n_groups * w.KB * w.nkk * 64u + 1023u) / 1024u) : 0u;
     pa.sw_blocks_per_weight = (w.N_pad + 1023u) / 1024u;
+    // (the tables are filled slot by slot: a few workgroups, each with the prefix sums of its own)
+    pa.route_blocks = (w.slots + 2047u) / 2048u < 16u ? (w.slots + 2047u) / 2048u : 16u;
     hipLaunchKernelGGL(bwd_grouped_prep_kernel,
-                       dim3(1u + pa.a_blocks + pa.ap_blocks + pa.sw_blocks_per_weight * w.n_weights), dim3(1024), 0, s, pa);
+                       dim3(pa.route_blocks + pa.a_blocks + pa.ap_blocks + pa.sw_blocks_per_weight * w.n_weights), dim3(1024), 0, s, pa);
     if ((st = launch_status())) return st;
   }
   BwdBody b{};

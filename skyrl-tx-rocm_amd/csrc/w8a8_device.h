@@ -96,6 +96,10 @@ typedef __attribute__((address_space(3))) void* lptr_t;
 __device__ inline void load_1k_to_lds(const unsigned char* src_lane, unsigned char* lds_dst_uniform) {
   __builtin_amdgcn_global_load_lds((gptr_t)src_lane, (lptr_t)lds_dst_uniform, 16, 0, 0);
 }
+// ... for data that is read once (non-temporal)
+__device__ inline void load_1k_to_lds_once(const unsigned char* src_lane, unsigned char* lds_dst_uniform) {
+  __builtin_amdgcn_global_load_lds((gptr_t)src_lane, (lptr_t)lds_dst_uniform, 16, 0, 2);
+}
 // The same as an assembly statement the compiler keeps no books on (it treats the builtin as an access
 // that may touch the LDS and then drains every counter at its next wait): lane l moves 16 bytes
 // global[base + voff] -> LDS[lds_addr_uniform + 16 l]; inactive lanes move nothing.  The caller waits
@@ -110,7 +114,6 @@ __device__ inline void lds_load_1k(const unsigned char* base_uniform, uint32_t v
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
                :: "v"(voff), "s"(base_uniform), "s"(lds_addr_uniform) : "memory", "m0");
 }
-// ... for data that is read once (non-temporal)
 __device__ inline void lds_load_1k_once(const unsigned char* base_uniform, uint32_t voff, uint32_t lds_addr_uniform) {
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt"
                :: "v"(voff), "s"(base_uniform), "s"(lds_addr_uniform) : "memory", "m0");
