@@ -268,6 +268,8 @@ def _bind(lib: ctypes.CDLL) -> None:
 def load() -> ctypes.CDLL:
     """Load (once) and return the native library; raises if it was not built."""
     global _lib
+    if _lib is not None:
+        return _lib
     with _lock:
         if _lib is None:
             if not LIB_PATH.exists():

@@ -18,7 +18,7 @@ import torch
 
 from ... import _native
 from .. import quantized_lora as ql
-from .w8a8_lora import MAX_LORA_RANK, _require_cuda, _scaling_vector, _stream_ptr, _version_of
+from .w8a8_lora import MAX_LORA_RANK, _on, _require_cuda, _scaling_vector, _stream_ptr, _version_of
 
 
 @dataclass(frozen=True)
@@ -79,7 +79,7 @@ def prepare_group_weight(weight) -> PackedGroupWeight:
         raise ValueError(f"geometry K_pad={k_pad}, N={n}, bits={weight.bits} is outside the native path")
     src = codes.contiguous()
     packed = torch.empty(nbytes, dtype=torch.uint8, device=codes.device)
-    with torch.cuda.device(codes.device):
+    with _on(codes.device):
         status = lib.mi355_w8a8_gq_pack_weight_v1(src.data_ptr(), packed.data_ptr(), k_pad, n, weight.bits,
                                                   _stream_ptr(codes.device))
     _native.check("mi355_w8a8_gq_pack_weight_v1", status)
@@ -179,7 +179,7 @@ def forward(x: torch.Tensor, weight, lora_a=None, lora_b=None, lora_scaling=None
     p.aux_x_codes = aux["x_codes"].data_ptr() if return_aux else None
     p.aux_x_scales = aux["x_scales"].data_ptr() if return_aux else None
     p.aux_base = aux["base"].data_ptr() if return_aux else None
-    with torch.cuda.device(dev):
+    with _on(dev):
         status = lib.mi355_w8a8_gq_linear_v1(ctypes.byref(p), _stream_ptr(dev))
     _native.check("mi355_w8a8_gq_linear_v1", status)
     result = out.reshape(*x.shape[:-1], n)
@@ -236,7 +236,7 @@ def backward(x: torch.Tensor, dy: torch.Tensor, weight, lora_a: torch.Tensor, lo
     if need_lora_grads:
         p.d_lora_a, p.d_lora_b, p.d_lora_scaling = da.data_ptr(), db.data_ptr(), ds.data_ptr()
     p.workspace, p.workspace_bytes = ws.data_ptr(), ws_bytes
-    with torch.cuda.device(dev):
+    with _on(dev):
         status = lib.mi355_w8a8_gq_linear_bwd_v1(ctypes.byref(p), _stream_ptr(dev))
     _native.check("mi355_w8a8_gq_linear_bwd_v1", status)
     return (dx.reshape(x.shape) if need_dx else None), da, db, ds

@@ -18,6 +18,7 @@ stream.  There is no CPU or eager fallback.
 
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import functools
 import math
@@ -77,7 +78,16 @@ def _validate_row_superblock(value, block_m: int) -> None:
 
 
 def _stream_ptr(device) -> int:
-    return int(torch.cuda.current_stream(device).cuda_stream)
+    # (the raw handle: a Stream object per call costs a microsecond that a decode step waits for)
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if device.index is None else device.index)
+
+
+_here = contextlib.nullcontext()
+
+
+def _on(device):
+    """``torch.cuda.device(device)``, without its two device switches where that is the current device already."""
+    return _here if torch.cuda.current_device() == device.index else torch.cuda.device(device)
 
 
 def _version_of(t: torch.Tensor):
@@ -136,7 +146,7 @@ def prepare_weight(weight) -> PackedW8Weight:
     codes = weight.codes.contiguous()
     nbytes = int(lib.mi355_w8a8_packed_weight_bytes(k, n))
     packed = torch.empty(nbytes, dtype=torch.uint8, device=codes.device)
-    with torch.cuda.device(codes.device):
+    with _on(codes.device):
         _native.check("mi355_w8a8_pack_weight_v1",
                       lib.mi355_w8a8_pack_weight_v1(codes.data_ptr(), packed.data_ptr(), k, n,
                                                     _stream_ptr(codes.device)))
@@ -153,7 +163,7 @@ def unpack_weight(packed: PackedW8Weight) -> torch.Tensor:
     """Inverse of the fragment-order packing: int8 [K, N] row-major."""
     lib = _native.load()
     out = torch.empty((packed.in_features, packed.out_features), dtype=torch.int8, device=packed.packed.device)
-    with torch.cuda.device(out.device):
+    with _on(out.device):
         _native.check("mi355_w8a8_unpack_weight_v1",
                       lib.mi355_w8a8_unpack_weight_v1(packed.packed.data_ptr(), out.data_ptr(),
                                                       packed.in_features, packed.out_features,
@@ -175,7 +185,7 @@ def dynamic_quantize_rows(x: torch.Tensor):
         raise ValueError(f"K must be a multiple of 8 not exceeding {MAX_IN_FEATURES}, got {k}")
     codes = torch.empty((m, k), dtype=torch.int8, device=x.device)
     scales = torch.empty((m,), dtype=torch.float32, device=x.device)
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         _native.check("mi355_w8a8_quantize_rows_v1",
                       lib.mi355_w8a8_quantize_rows_v1(flat.data_ptr(), codes.data_ptr(), scales.data_ptr(),
                                                       m, k, _stream_ptr(x.device)))
@@ -205,7 +215,7 @@ def _constant_scaling(value: float, count: int, device: str) -> torch.Tensor:
     """One constant vector per (value, count, device).  During a stream capture the cache is bypassed:
     a tensor created there lives in the graph's private pool, is only filled at replay and dangles once
     the graph is gone."""
-    if torch.cuda.is_available() and torch.cuda.is_current_stream_capturing():
+    if torch.cuda.is_initialized() and torch.cuda.is_current_stream_capturing():
         return _new_constant(value, count, device)
     return _cached_constant(value, count, device)
 
@@ -216,7 +226,9 @@ def _scaling_vector(lora_scaling, count: int, device) -> torch.Tensor:
     front of every native call.  The cached vectors are inputs only; nothing writes them."""
     if isinstance(lora_scaling, (int, float)) and not isinstance(lora_scaling, bool):
         return _constant_scaling(float(lora_scaling), count, str(device))
-    s = torch.as_tensor(lora_scaling, dtype=torch.float32, device=device)
+    s = lora_scaling
+    if not (isinstance(s, torch.Tensor) and s.dtype == torch.float32 and s.device == device):
+        s = torch.as_tensor(s, dtype=torch.float32, device=device)
     if s.ndim == 0:
         s = s.reshape(1).expand(count)
     return s.contiguous()
@@ -291,7 +303,9 @@ class ForwardPlan:
                 if idx.shape[0] == 0 or m % idx.shape[0]:
                     raise ValueError(f"adapter_indices of length {idx.shape[0]} do not divide {m} rows")
                 idx = idx.repeat_interleave(m // idx.shape[0])  # one entry per example (lora.py:142)
-            idx = idx.to(device=dev, dtype=torch.int32).contiguous()
+            if idx.dtype != torch.int32 or idx.device != dev:
+                idx = idx.to(device=dev, dtype=torch.int32)
+            idx = idx.contiguous()
         gamma = None
         if rms_gamma is not None:
             if tuple(rms_gamma.shape) != (k,):
@@ -375,7 +389,7 @@ class ForwardPlan:
         flags = self.flags | extra_flags
         key = None
         # (a captured call is replayed later, when the adapters may have changed: it always packs)
-        capturing = torch.cuda.is_current_stream_capturing()
+        capturing = self.keep_lora_pack and torch.cuda.is_current_stream_capturing()
         if self._lora is not None and not capturing and self.keep_lora_pack:
             # (what the workspace holds also depends on the path the flags choose: the decode kernels keep
             # nothing, the tiled kernels A and B in operand order)
@@ -387,7 +401,7 @@ class ForwardPlan:
             if key is not None and key == self._packed_lora_key:
                 flags |= _native.FLAG_LORA_PACK_VALID
         self.problem.flags = flags
-        with torch.cuda.device(self.device):
+        with _on(self.device):
             status = self._fn(ctypes.byref(self.problem), _stream_ptr(self.device))
         self.problem.flags = self.flags
         _native.check(f"mi355_w8a8_{self.entry}", status)
@@ -404,6 +418,7 @@ def forward(x: torch.Tensor, weight, lora_a=None, lora_b=None, lora_scaling=None
     plan = ForwardPlan(x, weight, lora_a, lora_b, lora_scaling, adapter_indices=adapter_indices,
                        rms_gamma=rms_gamma, eps=eps, residual=residual, swiglu=swiglu, flags=flags,
                        return_aux=return_aux, entry=entry)
+    plan.keep_lora_pack = False  # (run once: nothing to compare versions with)
     result = plan.run()
     # Everything the kernels touch was allocated for torch's current stream, the one they were
     # enqueued on, so the caching allocator orders any reuse after them.
@@ -491,7 +506,7 @@ class BackwardPlan:
     def run(self, flags: int = 0):
         """Enqueue the call; returns ``(dx, d_lora_a, d_lora_b, d_lora_scaling)`` (reused tensors)."""
         self.problem.flags = flags
-        with torch.cuda.device(self.device):
+        with _on(self.device):
             status = self._fn(ctypes.byref(self.problem), _stream_ptr(self.device))
         self.problem.flags = 0
         _native.check("mi355_w8a8_lora_linear_bwd_v1", status)
@@ -574,7 +589,7 @@ def swiglu_backward(fused: torch.Tensor, d_product: torch.Tensor, *, in_place: b
     f2 = fused.reshape(-1, n).contiguous()
     d2 = d_product.reshape(-1, n // 2).contiguous()
     out = f2 if in_place else torch.empty_like(f2)
-    with torch.cuda.device(fused.device):
+    with _on(fused.device):
         status = _native.load().mi355_w8a8_swiglu_bwd_v1(f2.data_ptr(), d2.data_ptr(), out.data_ptr(), f2.shape[0], n,
                                                          _stream_ptr(fused.device))
     _native.check("mi355_w8a8_swiglu_bwd_v1", status)
@@ -602,7 +617,7 @@ def rms_norm_backward(x: torch.Tensor, gamma: torch.Tensor, d_normalized: torch.
     d2 = d_normalized.reshape(-1, k).contiguous()
     g = gamma.to(device=x.device, dtype=torch.float32).contiguous()
     out = d2 if in_place else torch.empty_like(d2)
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         status = _native.load().mi355_w8a8_rms_norm_bwd_v1(x2.data_ptr(), g.data_ptr(), d2.data_ptr(), out.data_ptr(),
                                                            x2.shape[0], k, eps, _stream_ptr(x.device))
     _native.check("mi355_w8a8_rms_norm_bwd_v1", status)
@@ -649,7 +664,7 @@ class FusedBackwardPlan:
 
     def run_swiglu_stage(self) -> None:
         d = self.dims
-        with torch.cuda.device(self.device):
+        with _on(self.device):
             status = self._lib.mi355_w8a8_swiglu_bwd_v1(self.fwd.out.data_ptr(), self.d_product.data_ptr(),
                                                         self.fwd.out.data_ptr(), d["m"], d["n"],
                                                         _stream_ptr(self.device))
@@ -657,7 +672,7 @@ class FusedBackwardPlan:
 
     def run_rms_stage(self) -> None:
         d = self.dims
-        with torch.cuda.device(self.device):
+        with _on(self.device):
             status = self._lib.mi355_w8a8_rms_norm_bwd_v1(self.x.data_ptr(), self.gamma.data_ptr(),
                                                           self.bwd.dx.data_ptr(), self.bwd.dx.data_ptr(), d["m"],
                                                           d["k"], self.eps, _stream_ptr(self.device))
@@ -692,7 +707,7 @@ def swiglu(fused: torch.Tensor) -> torch.Tensor:
         raise ValueError(f"need fused [..., N] with N % 8 == 0, got {tuple(fused.shape)}")
     f2 = fused.reshape(-1, n).contiguous()
     out = torch.empty((f2.shape[0], n // 2), dtype=torch.bfloat16, device=fused.device)
-    with torch.cuda.device(fused.device):
+    with _on(fused.device):
         status = _native.load().mi355_w8a8_swiglu_v1(f2.data_ptr(), out.data_ptr(), f2.shape[0], n,
                                                      _stream_ptr(fused.device))
     _native.check("mi355_w8a8_swiglu_v1", status)
@@ -801,7 +816,7 @@ def prepare_grouped_weight(codes: torch.Tensor, scales: torch.Tensor) -> PackedG
     each = int(lib.mi355_w8a8_packed_weight_bytes(k, n))
     packed = torch.empty(e * each, dtype=torch.uint8, device=codes.device)
     codes = codes.contiguous()
-    with torch.cuda.device(codes.device):
+    with _on(codes.device):
         for i in range(e):
             _native.check("mi355_w8a8_pack_weight_v1",
                           lib.mi355_w8a8_pack_weight_v1(codes[i].data_ptr(), packed.data_ptr() + i * each, k, n,
@@ -938,7 +953,7 @@ class GroupedForwardPlan:
             if key is not None and key == self._packed_lora_key:
                 flags |= _native.FLAG_LORA_PACK_VALID
         self.problem.flags = flags
-        with torch.cuda.device(self.device):
+        with _on(self.device):
             status = self._lib.mi355_w8a8_grouped_v1(ctypes.byref(self.problem), _stream_ptr(self.device))
         self.problem.flags = self.flags
         _native.check("mi355_w8a8_grouped_v1", status)
@@ -1037,7 +1052,7 @@ class GroupedBackwardPlan:
 
     def run(self):
         """Enqueue the call; returns ``(dx, d_lora_a, d_lora_b, d_lora_scaling)`` (reused tensors)."""
-        with torch.cuda.device(self.device):
+        with _on(self.device):
             status = self._fn(ctypes.byref(self.problem), _stream_ptr(self.device))
         _native.check("mi355_w8a8_grouped_bwd_v1", status)
         return self.dx, self.d_lora_a, self.d_lora_b, self.d_lora_scaling
@@ -1168,7 +1183,7 @@ def moe_route(router_logits: torch.Tensor, top_k: int, norm_topk_prob: bool = Tr
     dev = logits.device
     weights = torch.empty((t, top_k), dtype=torch.float32, device=dev)
     selected = torch.empty((t, top_k), dtype=torch.int32, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         status = _native.load().mi355_w8a8_moe_route_v1(logits.data_ptr(), t, e, top_k, int(norm_topk_prob),
                                                         weights.data_ptr(), selected.data_ptr(), _stream_ptr(dev))
     _native.check("mi355_w8a8_moe_route_v1", status)
@@ -1191,7 +1206,7 @@ def moe_route_backward(router_logits: torch.Tensor, selected: torch.Tensor, d_we
     dw = d_weights.detach().to(device=dev, dtype=torch.float32).contiguous()
     t, e = logits.shape
     out = torch.empty_like(logits)
-    with torch.cuda.device(dev):
+    with _on(dev):
         status = _native.load().mi355_w8a8_moe_route_bwd_v1(logits.data_ptr(), sel.data_ptr(), dw.data_ptr(), t, e,
                                                             sel.shape[1], int(norm_topk_prob), out.data_ptr(),
                                                             _stream_ptr(dev))
@@ -1280,7 +1295,7 @@ def moe_dispatch(tokens: torch.Tensor | None, indices: torch.Tensor, num_groups:
     p.sorted_adapters = sorted_adapters.data_ptr() if ad is not None else None
     p.workspace = ws.data_ptr()
     p.workspace_bytes = ws_bytes
-    with torch.cuda.device(dev):
+    with _on(dev):
         status = lib.mi355_w8a8_moe_dispatch_v1(ctypes.byref(p), _stream_ptr(dev))
     _native.check("mi355_w8a8_moe_dispatch_v1", status)
     return sorted_tokens, group_sizes, sort_indices, unsort_indices, sorted_adapters
@@ -1312,7 +1327,7 @@ def moe_combine(expert_out: torch.Tensor, unsort_indices: torch.Tensor, weights:
     un = unsort_indices.reshape(-1).to(device=dev, dtype=torch.int32).contiguous()
     w = weights.detach().to(device=dev, dtype=torch.float32).contiguous()
     out = torch.empty((t, eo.shape[1]), dtype=torch.bfloat16, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         status = _native.load().mi355_w8a8_moe_combine_v1(eo.data_ptr(), un.data_ptr(), w.data_ptr(), out.data_ptr(),
                                                           t, top_k, eo.shape[1], _stream_ptr(dev))
     _native.check("mi355_w8a8_moe_combine_v1", status)
@@ -1346,7 +1361,7 @@ def moe_combine_backward(d_out: torch.Tensor, expert_out: torch.Tensor | None, s
         eo = expert_out.contiguous()
     d_eo = torch.empty((t * top_k, width), dtype=torch.bfloat16, device=dev)
     d_w = torch.empty((t, top_k), dtype=torch.float32, device=dev) if need_weight_grads else None
-    with torch.cuda.device(dev):
+    with _on(dev):
         status = _native.load().mi355_w8a8_moe_combine_bwd_v1(
             do.data_ptr(), eo.data_ptr() if eo is not None else None, so.data_ptr(), w.data_ptr(), d_eo.data_ptr(),
             d_w.data_ptr() if d_w is not None else None, t, top_k, width, _stream_ptr(dev))
@@ -1663,7 +1678,7 @@ class QkvPostPlan:
         self._keep = (flat, qw, kw, pos)
 
     def run(self):
-        with torch.cuda.device(self.device):
+        with _on(self.device):
             status = self._fn(ctypes.byref(self.problem), _stream_ptr(self.device))
         _native.check("mi355_w8a8_qkv_split_norm_rope_v1", status)
         c, lead = self.config, self.lead
@@ -1729,7 +1744,7 @@ def qkv_split_norm_rope_backward(fused: torch.Tensor, q_norm_weight: torch.Tenso
         ws = torch.empty(int(lib.mi355_w8a8_qkv_bwd_workspace_bytes(m, d)), dtype=torch.uint8, device=dev)
         p.d_q_norm_weight, p.d_k_norm_weight = dqw.data_ptr(), dkw.data_ptr()
         p.workspace, p.workspace_bytes = ws.data_ptr(), ws.numel()
-    with torch.cuda.device(dev):
+    with _on(dev):
         status = lib.mi355_w8a8_qkv_split_norm_rope_bwd_v1(ctypes.byref(p), _stream_ptr(dev))
     _native.check("mi355_w8a8_qkv_split_norm_rope_bwd_v1", status)
     return d_fused.reshape(fused.shape), dqw, dkw
@@ -1767,7 +1782,7 @@ def delta_rms_norm_backward(x: torch.Tensor, gamma: torch.Tensor, d_normalized: 
         ws = torch.empty(int(lib.mi355_w8a8_delta_rms_norm_bwd_workspace_bytes(x2.shape[0], k)), dtype=torch.uint8,
                          device=x.device)
         dw_ptr, ws_ptr, ws_bytes = dw.data_ptr(), ws.data_ptr(), ws.numel()
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         status = lib.mi355_w8a8_delta_rms_norm_bwd_v1(x2.data_ptr(), g.data_ptr(), d2.data_ptr(), out.data_ptr(), dw_ptr,
                                                       ws_ptr, ws_bytes, x2.shape[0], k, eps, _stream_ptr(x.device))
     _native.check("mi355_w8a8_delta_rms_norm_bwd_v1", status)
@@ -1837,14 +1852,14 @@ class QkvStageBackwardPlan:
         self._keep = (flat, normalized, cots, qw, kw, pos)
 
     def run_post_stage(self) -> None:
-        with torch.cuda.device(self.device):
+        with _on(self.device):
             status = self._lib.mi355_w8a8_qkv_split_norm_rope_bwd_v1(ctypes.byref(self.post_problem),
                                                                      _stream_ptr(self.device))
         _native.check("mi355_w8a8_qkv_split_norm_rope_bwd_v1", status)
 
     def run_rms_stage(self) -> None:
         dx = self.bwd.dx
-        with torch.cuda.device(self.device):
+        with _on(self.device):
             status = self._lib.mi355_w8a8_delta_rms_norm_bwd_v1(self.x.data_ptr(), self.gamma.data_ptr(), dx.data_ptr(),
                                                                 dx.data_ptr(), None, None, 0, self.m, self.k, self.eps,
                                                                 _stream_ptr(self.device))
