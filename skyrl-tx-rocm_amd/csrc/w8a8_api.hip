@@ -1741,11 +1741,15 @@ int run_moe_dispatch(const mi355_w8a8_moe_dispatch_problem* p, hipStream_t s) {
   a.group_start = reinterpret_cast<int32_t*>(ws + L.group_start);
   a.P = p->n_pairs; a.G = p->n_groups; a.repeat = p->repeat; a.width = p->width; a.n_chunks = L.n_chunks;
   (void)hipGetLastError();
-  hipLaunchKernelGGL(moe_hist_kernel, dim3(L.n_chunks), dim3(1024), 0, s, a);
-  if ((st = launch_status())) return st;
-  hipLaunchKernelGGL(moe_scan_kernel, dim3(1), dim3(1024), 0, s, a);
-  if ((st = launch_status())) return st;
-  hipLaunchKernelGGL(moe_scatter_kernel, dim3(L.n_chunks), dim3(1024), 0, s, a);
+  if (L.n_chunks <= kMoeSortChunks) {
+    hipLaunchKernelGGL(moe_sort_kernel, dim3(L.n_chunks), dim3(1024), 0, s, a);
+  } else {
+    hipLaunchKernelGGL(moe_hist_kernel, dim3(L.n_chunks), dim3(1024), 0, s, a);
+    if ((st = launch_status())) return st;
+    hipLaunchKernelGGL(moe_scan_kernel, dim3(1), dim3(1024), 0, s, a);
+    if ((st = launch_status())) return st;
+    hipLaunchKernelGGL(moe_scatter_kernel, dim3(L.n_chunks), dim3(1024), 0, s, a);
+  }
   if ((st = launch_status()) || !a.tokens) return st;
   if (p->repeat > 1u)
     hipLaunchKernelGGL(moe_spread_kernel, dim3((p->n_pairs / p->repeat + 3u) / 4u), dim3(256), 0, s, a);

@@ -5,6 +5,7 @@
 //
 //   moe_route_kernel           one wave per token: probabilities, top-k (ties: lower expert), weights
 //   moe_route_bwd_kernel       one wave per token: the weights' cotangent back to the logits
+//   moe_sort_kernel            up to kMoeSortChunks chunks: the next three in one launch
 //   moe_hist_kernel            per 1024-pair chunk: pairs per group
 //   moe_scan_kernel            one workgroup: group sizes, group starts, per-chunk offsets
 //   moe_scatter_kernel         per chunk: stable position of every pair, the index arrays
@@ -14,6 +15,7 @@
 //   moe_combine_bwd_kernel     a wave per sorted row: the cotangents of expert_out and of w
 #pragma once
 #include "w8a8_device.h"
+#include "w8a8_prologue.h"
 
 namespace w8a8 {
 
@@ -235,9 +237,11 @@ __global__ __launch_bounds__(1024) void moe_scan_kernel(MoeSortArgs a) {
 
 // Position of pair p = start of its group + pairs of the group in earlier chunks + pairs of the
 // group earlier in this chunk (earlier waves, then earlier lanes of its wave): a stable sort.
-__global__ __launch_bounds__(1024) void moe_scatter_kernel(MoeSortArgs a) {
+// first_of(g): the first two of these.
+template <class FirstOf>
+__device__ inline void moe_scatter_chunk(const MoeSortArgs& a, uint32_t chunk, FirstOf first_of) {
   __shared__ uint16_t wave_cnt[16][kMoeMaxExperts];
-  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, chunk = blockIdx.x;
+  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
   for (uint32_t i = tid; i < 16u * a.G; i += 1024u) wave_cnt[i / a.G][i % a.G] = 0;
   __syncthreads();
   const uint32_t p = chunk * kMoeChunk + tid;
@@ -257,11 +261,44 @@ __global__ __launch_bounds__(1024) void moe_scatter_kernel(MoeSortArgs a) {
   if (valid) {
     uint32_t before = 0;
     for (uint32_t w = 0; w < wave; ++w) before += wave_cnt[w][g];
-    const int pos = a.group_start[g] + a.chunk_cnt[(size_t)chunk * a.G + g] + (int)before + (int)rank;
+    const int pos = first_of(g) + (int)before + (int)rank;
     a.sort_indices[pos] = (int)p;
     a.unsort_indices[p] = pos;
     if (a.sorted_adapters) a.sorted_adapters[pos] = a.adapters[p / a.repeat];
   }
+}
+
+__global__ __launch_bounds__(1024) void moe_scatter_kernel(MoeSortArgs a) {
+  const uint32_t chunk = blockIdx.x;
+  moe_scatter_chunk(a, chunk, [&](uint32_t g) { return a.group_start[g] + a.chunk_cnt[(size_t)chunk * a.G + g]; });
+}
+
+// The whole sort in one launch: every chunk's workgroup counts all pairs for itself, those of earlier chunks apart.
+// Bound by the launches (three dependent ones of 3-5 us otherwise); the repeated counting grows with the square of
+// the chunks, hence the limit.  Measured, 128 groups: 128 pairs 9 -> 4.4 us, 16384 pairs (16 chunks) 14.5 -> 10.4.
+constexpr uint32_t kMoeSortChunks = 16;
+__global__ __launch_bounds__(1024) void moe_sort_kernel(MoeSortArgs a) {
+  __shared__ uint32_t all[kMoeMaxExperts];   // pairs per group; then first position of this chunk's pairs of a group
+  __shared__ uint32_t earlier[kMoeMaxExperts];
+  const uint32_t tid = threadIdx.x, chunk = blockIdx.x;
+  all[tid] = 0; earlier[tid] = 0;
+  __syncthreads();
+#pragma unroll 4
+  for (uint32_t c = 0; c < a.n_chunks; ++c) {
+    const uint32_t p = c * kMoeChunk + tid;
+    const uint32_t g = moe_group_of(a, p < a.P ? p : a.P - 1u);
+    if (p < a.P) {
+      atomicAdd(&all[g], 1u);
+      if (c < chunk) atomicAdd(&earlier[g], 1u);
+    }
+  }
+  __syncthreads();
+  const uint32_t n = all[tid];
+  uint32_t total;
+  const uint32_t start = block_prefix_capped(n, 0xffffffffu, &total);
+  if (chunk == 0 && tid < a.G) a.group_sizes[tid] = (int)n;
+  all[tid] = start + earlier[tid];  // (read again behind a barrier)
+  moe_scatter_chunk(a, chunk, [&](uint32_t g) { return (int)all[g]; });
 }
 
 // sorted_tokens[pos] = tokens[sort_indices[pos] / repeat]: a wave per row, two rows a wave.
