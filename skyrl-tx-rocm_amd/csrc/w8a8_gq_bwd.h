@@ -170,7 +170,7 @@ __global__ __launch_bounds__(512, 1) void gq_bwd_dx_kernel(GqBwdDxArgs a) {
       for (int e = 0; e < 16; ++e) acc[i][e] = 0.0f;
 
     // explicit LDS reads: a compiler-visible one of memory that direct-to-LDS loads write would drain every
-    // load in flight first; the values are valid after next_wait()
+    // load in flight first; the wait stands in the same block, so no register is handed out before it is filled
     struct NextRegs { v4i raw; v4f s4[4]; };
     auto next_read = [&](int i, NextRegs& r) {
       const uint32_t st = lds_base + (i % kGqBwdStages) * kGqBwdStageBytes + kGqBwdPanel;
@@ -179,10 +179,9 @@ __global__ __launch_bounds__(512, 1) void gq_bwd_dx_kernel(GqBwdDxArgs a) {
         const uint32_t wa = st + wcol * 512 + lane * 8;
         uint2 raw;
         asm volatile("ds_read_b64 %0, %5\n\tds_read_b128 %1, %6\n\tds_read_b128 %2, %6 offset:32\n\t"
-                     "ds_read_b128 %3, %6 offset:64\n\tds_read_b128 %4, %6 offset:96"
+                     "ds_read_b128 %3, %6 offset:64\n\tds_read_b128 %4, %6 offset:96\n\ts_waitcnt lgkmcnt(0)"
                      : "=&v"(raw), "=&v"(r.s4[0]), "=&v"(r.s4[1]), "=&v"(r.s4[2]), "=&v"(r.s4[3])
                      : "v"(wa), "v"(sa) : "memory");
-        asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(raw), "+v"(r.s4[0]), "+v"(r.s4[1]), "+v"(r.s4[2]), "+v"(r.s4[3]) : : "memory");
         GqRawFragment<true> f;
         f.v = make_uint4(raw.x, raw.y, 0u, 0u);
         r.raw = gq_expand<true>(f);  // 16 * code; the scale takes the exact 1 / 16
@@ -193,10 +192,9 @@ __global__ __launch_bounds__(512, 1) void gq_bwd_dx_kernel(GqBwdDxArgs a) {
       } else {
         const uint32_t wa = st + wcol * 1024 + lane * 16;
         asm volatile("ds_read_b128 %0, %5\n\tds_read_b128 %1, %6\n\tds_read_b128 %2, %6 offset:32\n\t"
-                     "ds_read_b128 %3, %6 offset:64\n\tds_read_b128 %4, %6 offset:96"
+                     "ds_read_b128 %3, %6 offset:64\n\tds_read_b128 %4, %6 offset:96\n\ts_waitcnt lgkmcnt(0)"
                      : "=&v"(r.raw), "=&v"(r.s4[0]), "=&v"(r.s4[1]), "=&v"(r.s4[2]), "=&v"(r.s4[3])
                      : "v"(wa), "v"(sa) : "memory");
-        asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(r.raw), "+v"(r.s4[0]), "+v"(r.s4[1]), "+v"(r.s4[2]), "+v"(r.s4[3]) : : "memory");
       }
     };
     auto transpose_block = [&](const v4i& rawb) -> v16i {
