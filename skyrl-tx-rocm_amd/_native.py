@@ -52,10 +52,12 @@ EXPORTS = (
     "mi355_w8a8_moe_route_v1", "mi355_w8a8_moe_route_bwd_v1", "mi355_w8a8_moe_dispatch_workspace_bytes", "mi355_w8a8_moe_dispatch_v1",
     "mi355_w8a8_moe_combine_v1", "mi355_w8a8_moe_combine_bwd_v1",
     "mi355_w8a8_gq_packed_weight_bytes", "mi355_w8a8_gq_pack_weight_v1", "mi355_w8a8_gq_workspace_bytes",
-    "mi355_w8a8_gq_linear_v1", "mi355_w8a8_gq_bwd_workspace_bytes", "mi355_w8a8_gq_linear_bwd_v1",
+    "mi355_w8a8_gq_linear_v1",
     "mi355_w8a8_forward_path", "mi355_w8a8_calibrate_operand_bytes", "mi355_w8a8_calibrate_mfma_ops", "mi355_w8a8_calibrate_mfma_v1",
     "mi355_w8a8_calibrate_read_v1", "mi355_w8a8_calibrate_copy_v1",
 )
+# called by the torch mirror alone (csrc/w8a8_gq_bwd_api.h)
+PRIVATE_EXPORTS = ("mi355_w8a8_gq_bwd_workspace_bytes", "mi355_w8a8_gq_linear_bwd_v1")
 
 _u32, _u64, _vp, _f32 = ctypes.c_uint32, ctypes.c_uint64, ctypes.c_void_p, ctypes.c_float
 
@@ -277,7 +279,7 @@ def load() -> ctypes.CDLL:
                     f"{LIB_PATH} is missing: build it with skyrl-tx-rocm_amd/build.py "
                     "(there is no CPU fallback for the W8A8 path)")
             lib = ctypes.CDLL(str(LIB_PATH), mode=ctypes.RTLD_LOCAL)
-            for name in EXPORTS:
+            for name in EXPORTS + PRIVATE_EXPORTS:
                 if not hasattr(lib, name):
                     raise RuntimeError(f"{LIB_PATH} does not export {name}")
             _bind(lib)

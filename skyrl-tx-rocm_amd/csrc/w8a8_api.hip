@@ -1,6 +1,7 @@
 // C ABI of the MI355X W8A8 LoRA linear forward path: argument validation, workspace
 // carving and kernel launches.  Nothing here synchronises, allocates or keeps state.
 #include "../../include/mi355_w8a8.h"
+#include "w8a8_gq_bwd_api.h"
 
 #include <hip/hip_runtime.h>
 
