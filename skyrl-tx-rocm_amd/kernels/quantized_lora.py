@@ -161,7 +161,8 @@ class _GroupScaledLoraFunction(torch.autograd.Function):
     the quantizers, ``dx = dy @ deq(W).T + r @ A.T`` with ``r = (dy @ B.T) * s``, ``dA = x.T @ r``,
     ``dB = ((x @ A).T @ dy) * s``, ``ds = sum(dy * ((x @ A) @ B))``, all in float32 and cast once.  The kernels
     of ``gq_linear.backward`` do it; groups that the packing had to embed and K or N off a multiple of 8 go
-    through float32 library GEMMs on the dequantized weight.  The frozen weight gets no gradient."""
+    through float32 library GEMMs on the dequantized weight, as does a backward that autograd records
+    (``create_graph``): what the kernels return has no graph.  The frozen weight gets no gradient."""
 
     @staticmethod
     def forward(ctx, x, lora_a, lora_b, scaling, weight, activation_bits):
@@ -177,7 +178,8 @@ class _GroupScaledLoraFunction(torch.autograd.Function):
         weight = ctx.weight
         from .rocm import gq_linear
 
-        if gq_linear.has_native_backward(weight) and dy.dtype == torch.bfloat16:
+        recorded = torch.is_grad_enabled()
+        if not recorded and dy.dtype == torch.bfloat16 and gq_linear.has_native_backward(weight):
             dx, da, db, ds = gq_linear.backward(x, dy, weight, lora_a, lora_b, scaling, need_dx=ctx.needs_input_grad[0],
                                                 need_lora_grads=any(ctx.needs_input_grad[1:4]))
             if ds is not None:
