@@ -196,6 +196,12 @@ def has_native_backward(weight) -> bool:
     return pw.source_group_size == 0 and pw.in_features % 8 == 0 and pw.out_features % 8 == 0
 
 
+def _aligned(t: torch.Tensor) -> torch.Tensor:
+    """The contiguous tensor itself, or a copy where it starts off a 16-byte boundary (a view into a flat buffer):
+    the backward kernels load 16 bytes at a time."""
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
 def backward(x: torch.Tensor, dy: torch.Tensor, weight, lora_a: torch.Tensor, lora_b: torch.Tensor,
              lora_scaling, *, need_dx: bool = True, need_lora_grads: bool = True):
     """Cotangents ``(dx, d_lora_a, d_lora_b, d_lora_scaling)`` of ``forward`` with one adapter
@@ -212,9 +218,9 @@ def backward(x: torch.Tensor, dy: torch.Tensor, weight, lora_a: torch.Tensor, lo
     if tuple(lora_a.shape) != (k, r) or tuple(lora_b.shape) != (r, n) or dy.shape[-1] != n or x.shape != (*dy.shape[:-1], k):
         raise ValueError(f"incompatible shapes: x={tuple(x.shape)}, dy={tuple(dy.shape)}, A={tuple(lora_a.shape)}, "
                          f"B={tuple(lora_b.shape)}, weight K={k}, N={n}")
-    xf, dyf = x.reshape(-1, k).contiguous(), dy.reshape(-1, n).contiguous()
+    xf, dyf = _aligned(x.reshape(-1, k).contiguous()), _aligned(dy.reshape(-1, n).contiguous())
     m = dyf.shape[0]
-    a, b = lora_a.contiguous(), lora_b.contiguous()
+    a, b, w_scales = _aligned(lora_a.contiguous()), _aligned(lora_b.contiguous()), _aligned(pw.scales)
     s1 = _scaling_vector(lora_scaling, 1, dev)
     lib = _native.load()
     ws_bytes = int(lib.mi355_w8a8_gq_bwd_workspace_bytes(m, k, pw.padded_in_features, n, pw.group_size, r))
@@ -230,7 +236,7 @@ def backward(x: torch.Tensor, dy: torch.Tensor, weight, lora_a: torch.Tensor, lo
     p.flags = (_native.FLAG_GQ_BF16_SCALES if pw.bf16_scales else 0) | (0 if need_dx else _native.FLAG_SKIP_GEMM)
     p.m, p.k, p.k_pad, p.n = m, k, pw.padded_in_features, n
     p.group_size, p.weight_bits, p.rank = pw.group_size, pw.bits, r
-    p.x, p.dy, p.w_packed, p.w_scales = xf.data_ptr(), dyf.data_ptr(), pw.packed.data_ptr(), pw.scales.data_ptr()
+    p.x, p.dy, p.w_packed, p.w_scales = xf.data_ptr(), dyf.data_ptr(), pw.packed.data_ptr(), w_scales.data_ptr()
     p.lora_a, p.lora_b, p.lora_scaling = a.data_ptr(), b.data_ptr(), s1.data_ptr()
     p.dx = dx.data_ptr() if need_dx else None
     if need_lora_grads:

@@ -2,6 +2,9 @@
 graph, so a backward that is itself recorded (create_graph) has to run as torch operations.  On the CPU the
 native calls are replaced by stand-ins without a graph; the GPU test runs the real ones."""
 
+import contextlib
+import types
+
 import pytest
 import torch
 
@@ -84,3 +87,44 @@ def test_second_derivatives_on_the_gpu():
     w, x, a, b = _setup("cuda:0", m=40, k=128, n=72)
     y = ql.quantized_lora_linear(x, w, a, b, 0.5)
     _close(_penalised(w, x, a, b, y), _reference(w, x, a, b, 0.5))
+
+
+def _shifted(t, by=1):
+    """The same values as a contiguous view that starts `by` elements into its storage (a flat parameter buffer)."""
+    flat = torch.zeros(t.numel() + by, dtype=t.dtype, device=t.device)
+    flat[by:] = t.detach().reshape(-1)
+    return flat[by:].reshape(t.shape)
+
+
+def test_operands_reach_the_kernels_aligned(monkeypatch):
+    """The entry point refuses operands off a 16-byte boundary; the forward takes them, so the backward has to."""
+    w, x, a, b = _setup("cpu")
+    seen = {}
+
+    def entry(ref, stream):
+        p = ref._obj
+        seen.update({f: getattr(p, f) for f in ("x", "dy", "w_packed", "w_scales", "lora_a", "lora_b", "dx", "d_lora_a", "d_lora_b")})
+        return 0
+
+    lib = types.SimpleNamespace(mi355_w8a8_gq_bwd_workspace_bytes=lambda *dims: 256, mi355_w8a8_gq_linear_bwd_v1=entry)
+    monkeypatch.setattr(gq._native, "load", lambda: lib)
+    monkeypatch.setattr(gq, "_require_cuda", lambda *args: None)
+    monkeypatch.setattr(gq, "_on", lambda dev: contextlib.nullcontext())
+    monkeypatch.setattr(gq, "_stream_ptr", lambda dev: 0)
+    pw = gq.PackedGroupWeight(torch.zeros(64 * 24, dtype=torch.uint8), _shifted(w.scales.float()), 64, 64, 24, 8, 32)
+    gq.backward(_shifted(x), _shifted(torch.zeros(5, 24, dtype=torch.bfloat16)), pw, _shifted(a, 3), _shifted(b), torch.tensor(0.5))
+    assert seen and all(ptr % 16 == 0 for ptr in seen.values()), seen
+
+
+@pytest.mark.gpu
+def test_operands_at_odd_offsets():
+    w, x, a, b = _setup("cuda:0", m=40, k=128, n=72)
+    w = ql.GroupQuantizedWeight(w.codes, _shifted(w.scales.float()), w.original_in_features, w.padded_in_features, w.bits,
+                                w.group_size)
+    dy = torch.randn(40, 72, device="cuda:0").to(torch.bfloat16)
+    grads = []
+    for shift in (lambda t: t.detach().clone(), _shifted):
+        leaves = [shift(t).requires_grad_() for t in (x, a, b)]
+        y = ql.quantized_lora_linear(leaves[0], w, leaves[1], leaves[2], 0.5)
+        grads.append(torch.autograd.grad(y, leaves, shift(dy)))
+    assert all(torch.equal(p, q) for p, q in zip(*grads))
