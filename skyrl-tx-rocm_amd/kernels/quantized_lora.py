@@ -160,9 +160,9 @@ class _GroupScaledLoraFunction(torch.autograd.Function):
     """The group-scaled forward with the reference's pullback (quantized_lora.py:337-394): straight through
     the quantizers, ``dx = dy @ deq(W).T + r @ A.T`` with ``r = (dy @ B.T) * s``, ``dA = x.T @ r``,
     ``dB = ((x @ A).T @ dy) * s``, ``ds = sum(dy * ((x @ A) @ B))``, all in float32 and cast once.  The kernels
-    of ``gq_linear.backward`` do it; groups that the packing had to embed and K or N off a multiple of 8 go
-    through float32 library GEMMs on the dequantized weight, as does a backward that autograd records
-    (``create_graph``): what the kernels return has no graph.  The frozen weight gets no gradient."""
+    of ``gq_linear.backward`` do it; calls beyond them (``has_native_backward``) go through float32 library GEMMs on
+    the dequantized weight, as does a backward that autograd records (``create_graph``): what the kernels return
+    has no graph.  The frozen weight gets no gradient."""
 
     @staticmethod
     def forward(ctx, x, lora_a, lora_b, scaling, weight, activation_bits):
@@ -179,7 +179,8 @@ class _GroupScaledLoraFunction(torch.autograd.Function):
         from .rocm import gq_linear
 
         recorded = torch.is_grad_enabled()
-        if not recorded and dy.dtype == torch.bfloat16 and gq_linear.has_native_backward(weight):
+        if not recorded and dy.dtype == torch.bfloat16 and gq_linear.has_native_backward(
+                weight, x.numel() // x.shape[-1], lora_b.shape[0]):
             dx, da, db, ds = gq_linear.backward(x, dy, weight, lora_a, lora_b, scaling, need_dx=ctx.needs_input_grad[0],
                                                 need_lora_grads=any(ctx.needs_input_grad[1:4]))
             if ds is not None:

@@ -190,10 +190,12 @@ def forward(x: torch.Tensor, weight, lora_a=None, lora_b=None, lora_scaling=None
     return (result, aux) if return_aux else result
 
 
-def has_native_backward(weight) -> bool:
-    """True where ``backward`` covers the geometry: groups that needed no embedding, K and N multiples of 8."""
+def has_native_backward(weight, rows: int = 1, rank: int = 1) -> bool:
+    """True where ``backward`` covers a call: groups that needed no embedding, and dimensions that the kernels take
+    (K and N multiples of 8, rows * K and rows * N inside 32-bit offsets)."""
     pw = prepare_group_weight(weight)
-    return pw.source_group_size == 0 and pw.in_features % 8 == 0 and pw.out_features % 8 == 0
+    return pw.source_group_size == 0 and _native.load().mi355_w8a8_gq_bwd_workspace_bytes(
+        rows, pw.in_features, pw.padded_in_features, pw.out_features, pw.group_size, rank) != 0
 
 
 def _aligned(t: torch.Tensor) -> torch.Tensor:

@@ -128,3 +128,30 @@ def test_operands_at_odd_offsets():
         y = ql.quantized_lora_linear(leaves[0], w, leaves[1], leaves[2], 0.5)
         grads.append(torch.autograd.grad(y, leaves, shift(dy)))
     assert all(torch.equal(p, q) for p, q in zip(*grads))
+
+
+@pytest.mark.parametrize("m,k,n,group,rank,covered", [
+    (4096, 12288, 4096, 128, 32, True),
+    (350_000, 12288, 512, 128, 32, False),   # m * k beyond 32-bit offsets
+    (350_000, 512, 12288, 128, 32, False),   # m * n
+    (3, 60, 24, 32, 8, False), (3, 64, 20, 32, 8, False),  # K, N off a multiple of 8
+    (0, 64, 24, 32, 8, False),
+])
+def test_which_calls_the_kernels_cover(m, k, n, group, rank, covered):
+    if not pkg._native.LIB_PATH.exists():
+        pytest.skip("libmi355_w8a8.so not built (run __graft_entry__.build())")
+    k_pad = -(-k // group) * group
+    pw = gq.PackedGroupWeight(torch.empty(0), torch.empty(0), k, k_pad, n, 8, group)
+    assert gq.has_native_backward(pw, m, rank) is covered
+
+
+def test_calls_beyond_the_kernels_take_the_library(stand_ins, monkeypatch):
+    """The rule decides on the call at hand, rows and rank included."""
+    asked = []
+    monkeypatch.setattr(gq, "has_native_backward", lambda weight, rows, rank: asked.append((rows, rank)))
+    w, x, a, b = _setup("cpu", m=6)
+    y = ql.quantized_lora_linear(x.reshape(2, 3, 64), w, a, b, 0.5)
+    got = torch.autograd.grad(y.float().sum(), (a, b))
+    leaves = [t.detach().double().requires_grad_() for t in (x, a, b)]
+    _close(got, torch.autograd.grad(_rule(w, *leaves, 0.5).sum(), leaves[1:]))
+    assert asked == [(6, 8)] and not stand_ins
