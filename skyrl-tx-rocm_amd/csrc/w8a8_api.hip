@@ -836,8 +836,12 @@ struct BwdLayout {
   BwdDxSplit split;
   uint64_t part;
   uint64_t dyp, swp, at, ap, rp, z, r_raw, rs, rpart, src_row, dst_pos, slot_group, blk_range, group_off, partA, partB, total;
+  uint64_t beyond;  // group-scaled calls
   uint32_t slots, nkk, K_pad, KB, N_pad, NB, tiles_m, tiles_k, max_chunks, R, n_slices, groups_per_slice;
 };
+
+// Workgroups of the preparation that lay out A for the pull-back's epilogue.
+uint32_t bwd_ap_blocks(uint32_t n_groups, uint32_t KB, uint32_t nkk) { return (uint32_t)(((uint64_t)n_groups * KB * nkk * 64u + 1023u) / 1024u); }
 
 // gq_k_pad: padded K of a group-scaled weight (its own k blocks, tiles of 128 k), or 0
 BwdLayout make_bwd_layout(uint32_t m, uint32_t k, uint32_t n, uint32_t n_groups, uint32_t rank, uint32_t gq_k_pad = 0u) {
@@ -875,6 +879,7 @@ BwdLayout make_bwd_layout(uint32_t m, uint32_t k, uint32_t n, uint32_t n_groups,
     w.rpart = off; off += align256((uint64_t)w.n_slices * w.slots * kBwdRankStride * 4u);  // also the K slices of z
     w.partA = off; off += align256((uint64_t)w.max_chunks * w.R * k * 4u);
     w.partB = off; off += align256((uint64_t)w.max_chunks * w.R * n * 4u);
+    w.beyond = off; off += gq_k_pad ? align256((1u + bwd_ap_blocks(n_groups, w.KB, w.nkk)) * 4u) : 0u;
   }
   w.total = off;
   return w;
@@ -929,8 +934,9 @@ struct BwdBody {
   size_t w_stride; uint32_t sw_stride;
   bool rows128;  // the pull-back runs 128-row x 512-k tiles (the tables are padded to match)
   BwdDxSplit split; uint64_t part;  // dense calls
-  // group-scaled weights: their format (weight_bits 0: per-channel)
+  // group-scaled weights: their format (weight_bits 0: per-channel), A itself and the notes of non-finite operands
   uint32_t weight_bits, group, terms; const float* w_scales;
+  const void* lora_a; uint64_t beyond;
 };
 
 template <bool W4, int TERMS, int NKK>
@@ -957,6 +963,7 @@ int launch_gq_bwd_dx(const GqBwdDxArgs& a, uint32_t bits, uint32_t terms, hipStr
 template <class Layout>
 int launch_bwd_body(const BwdBody& b, const Layout& w, unsigned char* ws, hipStream_t s) {
   int st;
+  uint32_t* const beyond = b.lora && b.weight_bits ? reinterpret_cast<uint32_t*>(ws + b.beyond) : nullptr;
   if (!b.skip_prologue) {  // dy into operand order; the same pass leaves the partial sums of r = dy @ B.T
     BwdPackDyArgs d{};
     d.dy = static_cast<const uint16_t*>(b.dy);
@@ -987,10 +994,12 @@ int launch_bwd_body(const BwdBody& b, const Layout& w, unsigned char* ws, hipStr
       f.rs = reinterpret_cast<float*>(ws + w.rs);
       f.rp = ws + w.rp;
       f.n_slices = w.n_slices; f.slots = w.slots; f.nkk = w.nkk; f.cols = w.nkk > 2u ? 64u : 32u;
+      f.beyond = beyond;
       hipLaunchKernelGGL(bwd_r_finish_kernel, dim3(w.slots / 32u), dim3(256), 0, s, f);
       if ((st = launch_status())) return st;
     }
-    if (b.d_lora_b || b.d_lora_scaling) {  // z = x @ A, recomputed rather than saved by the forward
+    // z = x @ A, recomputed rather than saved by the forward (and, of a group-scaled call, looked at for x)
+    if (b.d_lora_b || b.d_lora_scaling || (beyond && b.d_lora_a)) {
       LoraAArgs lz{};
       lz.xsrc = static_cast<const uint16_t*>(b.x);
       lz.at = reinterpret_cast<const uint16_t*>(ws + w.at);
@@ -1020,6 +1029,7 @@ int launch_bwd_body(const BwdBody& b, const Layout& w, unsigned char* ws, hipStr
       f.blk_range = b.skip_range;
       f.r_raw = reinterpret_cast<float*>(ws + w.z);
       f.n_slices = nks; f.slots = w.slots; f.nkk = w.nkk; f.cols = w.nkk > 2u ? 64u : 32u;
+      f.beyond = beyond;
       hipLaunchKernelGGL(bwd_r_finish_kernel, dim3(w.slots / 32u), dim3(256), 0, s, f);
       if ((st = launch_status())) return st;
     }
@@ -1056,6 +1066,7 @@ int launch_bwd_body(const BwdBody& b, const Layout& w, unsigned char* ws, hipStr
     }
     if (st) return st;
   }
+  BwdReduceArgs r{};
   if (b.lora && b.want_grads) {
     BwdDloraArgs d{};
     d.x = static_cast<const uint16_t*>(b.x);
@@ -1083,7 +1094,6 @@ int launch_bwd_body(const BwdBody& b, const Layout& w, unsigned char* ws, hipStr
       }
       if ((st = launch_status())) return st;
     }
-    BwdReduceArgs r{};
     r.partA = d.partA; r.partB = d.partB;
     r.r_raw = reinterpret_cast<const float*>(ws + w.r_raw);
     r.z = d.z;
@@ -1096,8 +1106,22 @@ int launch_bwd_body(const BwdBody& b, const Layout& w, unsigned char* ws, hipStr
     r.K = b.k; r.N = b.n; r.r = b.rank; r.R = w.R; r.n_groups = b.n_groups;
     r.blocks_a = b.d_lora_a ? (uint32_t)(((uint64_t)b.n_groups * b.rank * b.k + 255u) / 256u) : 0u;
     r.blocks_b = b.d_lora_b ? (uint32_t)(((uint64_t)b.n_groups * b.rank * b.n / 4u + 255u) / 256u) : 0u;
-    const uint32_t s_blocks = b.d_lora_scaling ? b.n_groups : 0u;
-    hipLaunchKernelGGL(bwd_dlora_reduce_kernel, dim3(r.blocks_a + r.blocks_b + s_blocks), dim3(256), 0, s, r);
+  }
+  if (b.lora && (b.want_grads || (beyond && !b.skip_gemm))) {
+    const uint32_t blocks = r.blocks_a + r.blocks_b + (b.d_lora_scaling ? b.n_groups : 0u);
+    if (beyond) {
+      GqBwdPlain q{};
+      q.beyond = beyond; q.n_beyond = 1u + bwd_ap_blocks(b.n_groups, w.KB, w.nkk);
+      q.x = static_cast<const uint16_t*>(b.x); q.dy = static_cast<const uint16_t*>(b.dy);
+      q.lora_a = static_cast<const uint16_t*>(b.lora_a); q.lora_b = static_cast<const uint16_t*>(b.lora_b);
+      q.rs = reinterpret_cast<const float*>(ws + w.rs);
+      q.dx = b.skip_gemm ? nullptr : static_cast<uint16_t*>(b.dx);
+      q.wp = static_cast<const unsigned char*>(b.w_packed); q.ws = b.w_scales;
+      q.M = b.m; q.K = b.k; q.N = b.n; q.r = b.rank; q.KB = w.KB; q.group = b.group; q.bits = b.weight_bits;
+      hipLaunchKernelGGL((bwd_dlora_reduce_kernel<GqBwdPlain>), dim3(blocks + (q.dx ? kGqPlainDxBlocks : 0u)), dim3(256), 0, s, r, q);
+    } else {
+      hipLaunchKernelGGL((bwd_dlora_reduce_kernel<BwdNoPlain>), dim3(blocks), dim3(256), 0, s, r, BwdNoPlain{});
+    }
     if ((st = launch_status())) return st;
   }
   return MI355_W8A8_OK;
@@ -1157,7 +1181,7 @@ int run_backward(const mi355_w8a8_bwd_problem* p, hipStream_t s) {
     pa.nkk = w.nkk; pa.kb32 = w.KB; pa.slots = w.slots;
     pa.route_blocks = lora ? 1u : 0u;
     pa.a_blocks = lora ? (uint32_t)(((uint64_t)p->n_adapters * p->k * ((p->rank + 7u) / 8u) + 1023u) / 1024u) : 0u;
-    pa.ap_blocks = lora ? (uint32_t)(((uint64_t)p->n_adapters * w.KB * w.nkk * 64u + 1023u) / 1024u) : 0u;
+    pa.ap_blocks = lora ? bwd_ap_blocks(p->n_adapters, w.KB, w.nkk) : 0u;
     const uint32_t sw_blocks = (w.N_pad + 1023u) / 1024u;
     hipLaunchKernelGGL(bwd_prep_kernel, dim3(pa.route_blocks + pa.a_blocks + pa.ap_blocks + sw_blocks), dim3(1024), 0, s, pa);
     if ((st = launch_status())) return st;
@@ -1224,7 +1248,8 @@ int run_gq_backward(const mi355_w8a8_gq_bwd_problem* p, hipStream_t s) {
     pa.nkk = w.nkk; pa.kb32 = w.KB; pa.slots = w.slots;
     pa.route_blocks = 1u;
     pa.a_blocks = (uint32_t)(((uint64_t)p->k * ((p->rank + 7u) / 8u) + 1023u) / 1024u);
-    pa.ap_blocks = (uint32_t)(((uint64_t)w.KB * w.nkk * 64u + 1023u) / 1024u);
+    pa.ap_blocks = bwd_ap_blocks(1u, w.KB, w.nkk);
+    pa.beyond = reinterpret_cast<uint32_t*>(ws + w.beyond);
     hipLaunchKernelGGL(bwd_prep_kernel, dim3(pa.route_blocks + pa.a_blocks + pa.ap_blocks), dim3(1024), 0, s, pa);
     if ((st = launch_status())) return st;
   }
@@ -1236,6 +1261,7 @@ int run_gq_backward(const mi355_w8a8_gq_bwd_problem* p, hipStream_t s) {
   b.group_off = reinterpret_cast<int32_t*>(ws + w.group_off);
   b.split = w.split; b.part = w.part;
   b.weight_bits = p->weight_bits; b.group = p->group_size; b.w_scales = p->w_scales;
+  b.lora_a = p->lora_a; b.beyond = w.beyond;
   b.terms = (p->flags & MI355_W8A8_FLAG_GQ_BF16_SCALES) ? 2u : 3u;
   return launch_bwd_body(b, w, ws, s);
 }
@@ -1378,7 +1404,7 @@ int run_grouped_backward(const mi355_w8a8_grouped_bwd_problem* p, hipStream_t s)
     pa.n_weights = w.n_weights; pa.r = p->rank; pa.nkk = w.nkk; pa.kb32 = w.KB; pa.slots = w.slots;
     pa.max_chunks = w.max_chunks; pa.sw_stride = w.sw_stride; pa.tile_rows = w.tile_rows;
     pa.a_blocks = lora ? (uint32_t)(((uint64_t)p->n_groups * p->k * ((p->rank + 7u) / 8u) + 1023u) / 1024u) : 0u;
-    pa.ap_blocks = lora ? (uint32_t)(((uint64_t)p->n_groups * w.KB * w.nkk * 64u + 1023u) / 1024u) : 0u;
+    pa.ap_blocks = lora ? bwd_ap_blocks(p->n_groups, w.KB, w.nkk) : 0u;
     pa.sw_blocks_per_weight = (w.N_pad + 1023u) / 1024u;
     // (the tables are filled slot by slot: a few workgroups, each with the prefix sums of its own)
     pa.route_blocks = (w.slots + 2047u) / 2048u < 16u ? (w.slots + 2047u) / 2048u : 16u;

@@ -144,7 +144,11 @@ struct BwdRFinishArgs {
   const float* rpart; const int32_t* slot_group; const int32_t* blk_range; const float* lora_scaling;
   float* r_raw; float* rs; unsigned char* rp;
   uint32_t n_slices, slots, nkk, cols;  // cols = 16 * nkk rounded up to 32
+  uint32_t* beyond;  // set where a value is beyond what bf16 terms can carry, or null
 };
+
+// A float32 value that is no sum of bf16 terms: not finite, or rounded to infinity by the first of them.
+__device__ inline bool beyond_bf16_terms(float v) { return (__float_as_uint(v) & 0x7fffffffu) >= 0x7f7f8000u; }
 
 __global__ __launch_bounds__(256) void bwd_r_finish_kernel(BwdRFinishArgs a) {
   __shared__ float zs[32][kBwdRankStride + 1];
@@ -155,9 +159,11 @@ __global__ __launch_bounds__(256) void bwd_r_finish_kernel(BwdRFinishArgs a) {
     float raw = 0.0f;
     for (uint32_t sl = 0; sl < a.n_slices; ++sl) raw += a.rpart[((size_t)sl * a.slots + slot) * kBwdRankStride + col];
     a.r_raw[(size_t)slot * kBwdRankStride + col] = raw;
+    if (a.beyond && beyond_bf16_terms(raw)) *a.beyond = 1u;
     if (!a.rp) continue;  // plain sum of the slices (the z table)
     const uint32_t gr = a.slot_group ? (uint32_t)a.slot_group[slot] : 0u;
     const float scaled = raw * a.lora_scaling[gr];
+    if (a.beyond && beyond_bf16_terms(scaled)) *a.beyond = 1u;
     a.rs[(size_t)slot * kBwdRankStride + col] = scaled;
     zs[row][col] = scaled;
   }
@@ -186,11 +192,11 @@ __global__ __launch_bounds__(256) void bwd_r_finish_kernel(BwdRFinishArgs a) {
 //   ap[group][k block][kk][64 lanes][8]: lane (c, h) holds A[group][32 kb + c][16 kk + 8 h + 0..7],
 // and the per-channel scales in packed column order, swp[p] = sw[packed_to_orig_col(p)].
 // ---------------------------------------------------------------------------------------
-__device__ inline void lora_a_operand_item(const uint16_t* __restrict__ a, unsigned char* __restrict__ ap,
+__device__ inline v8us lora_a_operand_item(const uint16_t* __restrict__ a, unsigned char* __restrict__ ap,
                                            uint32_t n_groups, uint32_t K, uint32_t r, uint32_t kb32, uint32_t nkk,
                                            uint64_t idx) {
   const uint64_t total = (uint64_t)n_groups * kb32 * nkk * 64u;
-  if (idx >= total) return;
+  if (idx >= total) return v8us{0, 0, 0, 0, 0, 0, 0, 0};
   const uint32_t l = (uint32_t)(idx & 63u);
   const uint64_t rest = idx >> 6;
   const uint32_t kk = (uint32_t)(rest % nkk);
@@ -213,6 +219,7 @@ __device__ inline void lora_a_operand_item(const uint16_t* __restrict__ a, unsig
     }
   }
   *reinterpret_cast<v8us*>(ap + idx * 16u) = o;
+  return o;
 }
 
 struct BwdPrepArgs {
@@ -223,11 +230,13 @@ struct BwdPrepArgs {
   unsigned char* ap;
   const float* sw; float* swp;
   uint32_t M, K, N, N_pad, n_groups, r, nkk, kb32, slots, route_blocks, a_blocks, ap_blocks;
+  uint32_t* beyond;          // word 0 cleared, words 1 .. ap_blocks: A not finite somewhere in that block; or null
 };
 
 __global__ __launch_bounds__(1024) void bwd_prep_kernel(BwdPrepArgs p) {
   uint32_t b = blockIdx.x;
   if (b < p.route_blocks) {
+    if (p.beyond && threadIdx.x == 0) p.beyond[0] = 0u;
     if (p.idx) {
       route_rows_block(p.idx, p.M, p.n_groups, p.slots, p.src_row, p.dst_pos, p.slot_group, p.blk_range, p.group_off);
     } else {  // one adapter for every row: identity order, everything in group 0
@@ -242,7 +251,14 @@ __global__ __launch_bounds__(1024) void bwd_prep_kernel(BwdPrepArgs p) {
   }
   b -= p.a_blocks;
   if (b < p.ap_blocks) {
-    lora_a_operand_item(p.lora_a, p.ap, p.n_groups, p.K, p.r, p.kb32, p.nkk, (uint64_t)b * 1024u + threadIdx.x);
+    const v8us o = lora_a_operand_item(p.lora_a, p.ap, p.n_groups, p.K, p.r, p.kb32, p.nkk, (uint64_t)b * 1024u + threadIdx.x);
+    if (p.beyond) {  // kernel-uniform
+      int bad = 0;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) bad |= (o[e] & 0x7f80u) == 0x7f80u;
+      bad = __syncthreads_or(bad);
+      if (threadIdx.x == 0) p.beyond[1u + b] = bad ? 1u : 0u;
+    }
     return;
   }
   b -= p.ap_blocks;
@@ -1027,10 +1043,16 @@ struct BwdReduceArgs {
   uint32_t K, N, r, R, n_groups, blocks_a, blocks_b;
 };
 
-__global__ __launch_bounds__(256) void bwd_dlora_reduce_kernel(BwdReduceArgs a) {
+struct BwdNoPlain { static constexpr bool kAny = false; };
+
+// Plain: what replaces the sums of the partials where an operand is not finite (group-scaled calls), or BwdNoPlain.
+template <class Plain>
+__global__ __launch_bounds__(256) void bwd_dlora_reduce_kernel(BwdReduceArgs a, Plain plain) {
   __shared__ uint32_t chunk0_lds[kMaxAdapters + 1];
   __shared__ double red[256];
   const uint32_t tid = threadIdx.x;
+  bool use_plain = false;  // kernel-uniform
+  if constexpr (Plain::kAny) use_plain = plain.wanted();
   if (!a.chunk0_tab && tid < 64u) {
     // first chunk of every group: the dense tables hold at most 64 groups, so one wave loads all the
     // offsets at once and scans the chunk counts (a serial loop over dependent loads in front of every
@@ -1057,7 +1079,9 @@ __global__ __launch_bounds__(256) void bwd_dlora_reduce_kernel(BwdReduceArgs a) 
     // four rows, longer than the rest of the launch takes
     double sum = 0.0;
     const uint32_t j = tid & 63u;
-    if (j < a.r) {
+    if (use_plain) {
+      if constexpr (Plain::kAny) sum = plain.d_s(a.r_raw, a.z);
+    } else if (j < a.r) {
       uint32_t slot = o0 + (tid >> 6);
       for (; slot + 28u < o1; slot += 32u) {
         float rv[8], zv[8];
@@ -1097,7 +1121,11 @@ __global__ __launch_bounds__(256) void bwd_dlora_reduce_kernel(BwdReduceArgs a) 
     if (e >= (uint64_t)a.n_groups * a.K * a.r || !a.d_a) return;
     const uint32_t j = (uint32_t)(e % a.r), col = (uint32_t)((e / a.r) % a.K), grp = (uint32_t)(e / ((uint64_t)a.r * a.K));
     float sum = 0.0f;
-    for (uint32_t ch = chunk0(grp), ce = chunk0(grp + 1u); ch < ce; ++ch) sum += a.partA[((size_t)ch * a.R + j) * a.K + col];
+    if (use_plain) {
+      if constexpr (Plain::kAny) sum = plain.d_a(col, j);
+    } else {
+      for (uint32_t ch = chunk0(grp), ce = chunk0(grp + 1u); ch < ce; ++ch) sum += a.partA[((size_t)ch * a.R + j) * a.K + col];
+    }
     a.d_a[e] = (uint16_t)f32_to_bf16_bits(sum);
     return;
   }
@@ -1107,13 +1135,21 @@ __global__ __launch_bounds__(256) void bwd_dlora_reduce_kernel(BwdReduceArgs a) 
     if (e >= (uint64_t)a.n_groups * a.r * a.N || !a.d_b) return;
     const uint32_t col = (uint32_t)(e % a.N), j = (uint32_t)((e / a.N) % a.r), grp = (uint32_t)(e / ((uint64_t)a.N * a.r));
     float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (uint32_t ch = chunk0(grp), ce = chunk0(grp + 1u); ch < ce; ++ch) {
-      const float4 v = *reinterpret_cast<const float4*>(a.partB + ((size_t)ch * a.R + j) * a.N + col);
-      sum.x += v.x; sum.y += v.y; sum.z += v.z; sum.w += v.w;
+    if (use_plain) {
+      if constexpr (Plain::kAny)
+        sum = make_float4(plain.d_b(a.z, col, j), plain.d_b(a.z, col + 1u, j), plain.d_b(a.z, col + 2u, j), plain.d_b(a.z, col + 3u, j));
+    } else {
+      for (uint32_t ch = chunk0(grp), ce = chunk0(grp + 1u); ch < ce; ++ch) {
+        const float4 v = *reinterpret_cast<const float4*>(a.partB + ((size_t)ch * a.R + j) * a.N + col);
+        sum.x += v.x; sum.y += v.y; sum.z += v.z; sum.w += v.w;
+      }
     }
     const float sc = a.lora_scaling[grp];
     *reinterpret_cast<uint2*>(a.d_b + e) = make_uint2(pack_bf16x2(sum.x * sc, sum.y * sc), pack_bf16x2(sum.z * sc, sum.w * sc));
     return;
+  }
+  if constexpr (Plain::kAny) {
+    if (use_plain) plain.d_x(b - a.blocks_a - a.blocks_b);
   }
 }
 

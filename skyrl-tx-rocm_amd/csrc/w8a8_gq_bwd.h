@@ -364,4 +364,116 @@ __global__ __launch_bounds__(512, 1) void gq_bwd_dx_kernel(GqBwdDxArgs a) {
   }
 }
 
+// ---------------------------------------------------------------------------------------
+// Operands that are not finite.  A sum of bf16 terms does not carry an infinity (inf * 0 and inf - inf are NaN where
+// the float32 product is a signed infinity), nor does a transposition on the matrix core keep one to its
+// column.  The preparation and the tables of r and z note such values (BwdRFinishArgs::beyond); the last launch
+// then forms the LoRA cotangents as plain sums and rewrites the entries of dx that are infinite or NaN, as
+// the rule in float32 gives them.  A finite call pays the look at the notes.
+// ---------------------------------------------------------------------------------------
+constexpr uint32_t kGqPlainDxBlocks = 256;
+struct GqBwdPlain {
+  static constexpr bool kAny = true;
+  const uint32_t* beyond; uint32_t n_beyond;
+  const uint16_t* x; const uint16_t* dy;          // bf16 [M, K], [M, N]
+  const uint16_t* lora_a; const uint16_t* lora_b; // bf16 [K, r], [r, N]
+  const float* rs;                                // f32 [M][64]
+  uint16_t* dx;                                   // or null
+  const unsigned char* wp; const float* ws;       // packed codes, scales [K_pad / group, N]
+  uint32_t M, K, N, r, KB, group, bits;
+
+  __device__ bool wanted() const {
+    uint32_t any = 0;
+    for (uint32_t i = threadIdx.x & 63u; i < n_beyond; i += 64u) any |= beyond[i];
+    return __builtin_amdgcn_ballot_w64(any != 0) != 0;
+  }
+  __device__ static bool is_nan(double v) { return v != v; }
+  __device__ float d_a(uint32_t k, uint32_t j) const {
+    double sum = 0.0;
+    for (uint32_t m = 0; m < M && !is_nan(sum); ++m)
+      sum += (double)(bf16_bits_to_f32(x[(size_t)m * K + k]) * rs[(size_t)m * kBwdRankStride + j]);
+    return (float)sum;
+  }
+  __device__ float d_b(const float* z, uint32_t n, uint32_t j) const {
+    double sum = 0.0;
+    for (uint32_t m = 0; m < M && !is_nan(sum); ++m)
+      sum += (double)(z[(size_t)m * kBwdRankStride + j] * bf16_bits_to_f32(dy[(size_t)m * N + n]));
+    return (float)sum;
+  }
+  // This thread's share of sum(dy * (z @ B)).  By rows: r . z, or the products themselves where either is infinite.
+  __device__ double d_s(const float* r_raw, const float* z) const {
+    double sum = 0.0;
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    for (uint32_t m = 0; m < M && __builtin_amdgcn_ballot_w64(is_nan(sum)) == 0; ++m) {
+      const size_t row = (size_t)m * kBwdRankStride;
+      const float rv = lane < r ? r_raw[row + lane] : 0.0f, zv = lane < r ? z[row + lane] : 0.0f;
+      if (__builtin_amdgcn_ballot_w64(beyond_bf16_terms(rv) || beyond_bf16_terms(zv)) == 0) {
+        if (wave == (m & 3u)) sum += (double)rv * (double)zv;
+        continue;
+      }
+      for (uint32_t n = threadIdx.x; n < N; n += 256u) {
+        float zb = 0.0f;
+        for (uint32_t j = 0; j < r; ++j) zb += z[row + j] * bf16_bits_to_f32(lora_b[(size_t)j * N + n]);
+        sum += (double)(bf16_bits_to_f32(dy[(size_t)m * N + n]) * zb);
+      }
+    }
+    return sum;
+  }
+  __device__ float weight(uint32_t k, uint32_t n) const {
+    const size_t blk = (size_t)(n >> 5) * KB + (k >> 5);
+    const uint32_t lane = (n & 31u) + 32u * ((k >> 4) & 1u), j = k & 15u;
+    int code;
+    if (bits == 8u) {
+      code = (int8_t)wp[blk * 1024u + lane * 16u + j];
+    } else {
+      const uint32_t byte = wp[blk * 512u + lane * 8u + 4u * (j >> 3) + (j & 3u)];
+      code = (int8_t)((j & 4u) ? byte & 0xf0u : byte << 4) / 16;
+    }
+    return (float)code * ws[(size_t)(k / group) * N + n];
+  }
+  // Entries of dx that are not finite: all of a row whose r is not, and a column's whose row of A is not.  Their finite
+  // terms do not matter.
+  __device__ void d_x(uint32_t block) const {
+    if (!dx) return;
+    __shared__ uint16_t list[256];
+    __shared__ uint32_t count;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    for (uint32_t m = block; m < M; m += kGqPlainDxBlocks) {
+      const float* const rsm = rs + (size_t)m * kBwdRankStride;
+      const bool bad_row = __builtin_amdgcn_ballot_w64(lane < r && beyond_bf16_terms(rsm[lane < r ? lane : 0u])) != 0;
+      for (uint32_t k0 = 0; k0 < K; k0 += 256u) {
+        const uint32_t k = k0 + tid;
+        bool redo = bad_row && k < K;
+        float v = 0.0f;
+        if (k < K) {
+          for (uint32_t j = 0; j < r; ++j) {
+            const float av = bf16_bits_to_f32(lora_a[(size_t)k * r + j]);
+            redo = redo || beyond_bf16_terms(av);
+            v += rsm[j] * av;
+          }
+        }
+        if (__syncthreads_or(redo && v == v)) {  // (what is NaN stays NaN)
+          for (uint32_t n0 = 0; n0 < N; n0 += 256u) {
+            if (tid == 0) count = 0;
+            __syncthreads();
+            if (n0 + tid < N && (dy[(size_t)m * N + n0 + tid] & 0x7f80u) == 0x7f80u) list[atomicAdd(&count, 1u)] = (uint16_t)tid;
+            __syncthreads();
+            if (redo) {
+              for (uint32_t i = 0; i < count && v == v; ++i) {
+                const uint32_t n = n0 + list[i];
+                v += bf16_bits_to_f32(dy[(size_t)m * N + n]) * weight(k, n);
+              }
+            }
+            __syncthreads();
+          }
+        }
+        if (!redo) continue;
+        if (!(v != v || __builtin_isinf(v)))  // (r of nearly the largest float: finite, but not a sum of bf16 terms)
+          for (uint32_t n = 0; n < N; ++n) v += bf16_bits_to_f32(dy[(size_t)m * N + n]) * weight(k, n);
+        dx[(size_t)m * K + k] = (uint16_t)f32_to_bf16_bits(v);
+      }
+    }
+  }
+};
+
 }  // namespace w8a8
