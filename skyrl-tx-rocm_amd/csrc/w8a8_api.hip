@@ -84,7 +84,7 @@ inline bool skinny_chunked_pays(uint32_t m, uint32_t k, uint32_t n) {
 inline uint32_t padded_rows_bound(uint32_t m, uint32_t n_groups) {
   return round_up(m + 31u * (n_groups < m ? n_groups : m), 32u);
 }
-// Whether a routed call may lay its groups out that way: the quantizer sorts the rows itself, and the
+// Whether a routed call may lay its groups out that way: the
 // empty slots cost no time -- neither the quantizer's workgroups (16 slots each, one resident per CU) nor
 // the GEMM's tiles (512 resident tiles of 128 x 128, 256 of 256 x 256) need another round on the chip
 // than the packed layout does.
@@ -380,6 +380,48 @@ int choose_forward_path(uint32_t m, uint32_t k, uint32_t n, uint32_t flags) {
   return wide ? MI355_W8A8_PATH_TILED_256X256 : MI355_W8A8_PATH_TILED_256X128;
 }
 
+template <int CB, bool RMS>
+int launch_quant_rows_one(const QuantLoraRowsArgs& a, hipStream_t s) {
+  const uint32_t lds_bytes = quant_lora_rows_lds_bytes(a.q.K, CB);
+  if (hipFuncSetAttribute(reinterpret_cast<const void*>(&quant_lora_rows_kernel<CB, RMS>),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes) != hipSuccess)
+    return MI355_W8A8_ERR_LAUNCH;
+  hipLaunchKernelGGL((quant_lora_rows_kernel<CB, RMS>), dim3(a.q.n_half_blocks * (16u / a.rows_per_wg)), dim3(1024), lds_bytes, s, a);
+  return launch_status();
+}
+
+template <bool RMS>
+int launch_quant_rows(const QuantLoraRowsArgs& a, uint32_t nkk, hipStream_t s) {
+  switch (nkk) {
+    case 0: return launch_quant_rows_one<0, RMS>(a, s);
+    case 1: return launch_quant_rows_one<1, RMS>(a, s);
+    case 2: return launch_quant_rows_one<2, RMS>(a, s);
+    default: return launch_quant_rows_one<4, RMS>(a, s);
+  }
+}
+
+// Which of the two prologues a tiled call takes: quant_lora_rows_kernel (the rows held in the LDS: no launch for their statistics,
+// and a second group among sixteen rows costs little) or quant_lora_kernel (x read twice, two workgroups per CU,
+// A fetched once per sixteen rows whatever K is).  `boundaries`: the groups follow each other without padding, so
+// that sixteen rows may belong to several.  Prologue in us, rows held / read twice, back to back:
+//   no LoRA: 4096 x 4096 RMSNorm 20.8 / 23.4, 184 x 12288 RMSNorm 36 / 48, 1024 x 12288 34 / 35; 2048 x 12288 63 / 38.
+//   boundaries: 48 x 4096, 8 adapters of rank 32, RMSNorm 32 / 52; 4096 x 4096 34 / 40; 8192 x 4096 62 / 68;
+//     48 x 12288 72 / 155, 512 x 12288 (128 workgroups) 65 / 73, 1024 x 12288 72 / 59.
+//   operands kept: 4096 x 2560, rank 16 21 / 28, 333 x 4096 level; 6000 x 4096, rank 64, groups padded 54 / 51;
+//     184 x 12288 RMSNorm 46 / 51, without the norm 40 / 36.
+//   operands laid out by this call, groups padded: 1024 x 4096, rank 32 29 / 26, 333 x 4096, rank 64 25 / 23.
+// (Packed groups that happen to meet on block boundaries take the second form 1-2 % of a call faster, 4096 x 2560 -> 6144
+// 92 / 94; the layout is not known here.)
+bool prologue_keeps_rows(uint32_t rows_bound, uint32_t k, bool rms, bool lora, bool pack, bool boundaries) {
+  const uint32_t per_wg = quant_lora_rows_per_wg(k), wgs = (rows_bound + per_wg - 1u) / per_wg;
+  if (per_wg < 16u) {  // K > 4608: A fetched for fewer rows
+    if (!lora) return wgs <= 256u;
+    return wgs <= 128u && (boundaries || (rms && !pack));
+  }
+  if (!lora || boundaries) return true;
+  return !pack && (wgs <= 256u || k <= 2304u);  // (two workgroups of up to 2304 k share a CU)
+}
+
 int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
   if (!p) return MI355_W8A8_ERR_NULL;
   if (p->struct_size != sizeof(mi355_w8a8_problem)) return MI355_W8A8_ERR_STRUCT;
@@ -426,7 +468,7 @@ int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
   if (reinterpret_cast<uintptr_t>(p->workspace) & 255u) return MI355_W8A8_ERR_ALIGN;
   const int path = choose_forward_path(p->m, p->k, p->n, p->flags);
   if (path < 0) return path;
-  // groups on block boundaries: only where the quantizer sorts the rows itself and the tiles stay resident
+  // groups on block boundaries: only where the empty slots cost no round on the chip
   const bool pad_groups =
       routed && ((path == MI355_W8A8_PATH_TILED_128X128 && padded_groups_fit(p->m, p->n, p->n_adapters)) ||
                  (path == MI355_W8A8_PATH_TILED_256X256 && padded_groups_fit(p->m, p->n, p->n_adapters, true)));
@@ -469,8 +511,14 @@ int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
 
   const bool skip_prologue = (p->flags & MI355_W8A8_FLAG_SKIP_PROLOGUE) != 0;
   const bool skip_gemm = (p->flags & MI355_W8A8_FLAG_SKIP_GEMM) != 0;
+  // Rows held in the LDS, or read twice behind a launch that takes their statistics (quant_lora_rows_kernel,
+  // quant_lora_kernel).
+  const bool pack = lora && !(p->flags & MI355_W8A8_FLAG_LORA_PACK_VALID);
+  const bool rows_in_lds = prologue_keeps_rows(w.rows_bound, p->k, rms, lora, pack, routed && !pad_groups);
+  const bool route_inline = rows_in_lds && routed && !pack && p->m <= kInlineRouteMaxRows;
   // launch 1: adapter routing, the rows' statistics and (unless the workspace holds them) the LoRA operands
-  if (!skip_prologue) {
+  const uint32_t route_blocks = routed && !route_inline ? 1u : 0u, stat_blocks = rows_in_lds ? 0u : (p->m + 15u) / 16u;
+  if (!skip_prologue && (route_blocks || stat_blocks || pack)) {
     LoraPrepArgs pa{};
     pa.idx = routed ? p->adapter_indices : nullptr;
     pa.src_row = src_row; pa.dst_pos = dst_pos; pa.slot_group = slot_group; pa.blk_range = blk_range;
@@ -480,10 +528,10 @@ int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
     pa.bp = ws + w.bp;
     pa.M = p->m; pa.K = p->k; pa.N = p->n; pa.n_groups = p->n_adapters; pa.r = p->rank; pa.nkk = w.nkk;
     pa.ncb = n_padded(p->n) / 32u; pa.slots = w.slots;
-    pa.route_blocks = routed ? 1u : 0u;
+    pa.route_blocks = route_blocks;
     pa.route_pad = pad_groups ? 32u : 1u;
     pa.a_operand_kb = w.KB;  // the quantizer reads A in MFMA operand order
-    pa.stat_blocks = (p->m + 15u) / 16u;
+    pa.stat_blocks = stat_blocks;
     pa.stat_rows = p->m;
     pa.x = static_cast<const uint16_t*>(p->x);
     pa.gamma = p->rms_gamma; pa.eps = p->rms_eps;
@@ -493,11 +541,11 @@ int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
     pa.xn_aux = static_cast<uint16_t*>(p->aux_normalized);
     const uint64_t a_items = (uint64_t)p->n_adapters * w.KB * w.nkk * (p->rank % 4u ? 64u : 16u);
     const uint64_t b_items = (uint64_t)p->n_adapters * pa.ncb * w.nkk * (p->n % 4u ? 64u : 16u);
-    const bool pack = lora && !(p->flags & MI355_W8A8_FLAG_LORA_PACK_VALID);
     pa.a_blocks = pack ? (uint32_t)((a_items + 1023u) / 1024u) : 0u;
     const uint32_t b_blocks = pack ? (uint32_t)((b_items + 1023u) / 1024u) : 0u;
     const dim3 grid(pa.route_blocks + pa.stat_blocks + pa.a_blocks + b_blocks), block(1024);
-    if (rms) hipLaunchKernelGGL((lora_prep_kernel<2>), grid, block, 0, s, pa);
+    if (rows_in_lds) hipLaunchKernelGGL((lora_prep_kernel<0>), grid, block, 0, s, pa);
+    else if (rms) hipLaunchKernelGGL((lora_prep_kernel<2>), grid, block, 0, s, pa);
     else hipLaunchKernelGGL((lora_prep_kernel<1>), grid, block, 0, s, pa);
     if ((st = launch_status())) return st;
   }
@@ -505,7 +553,7 @@ int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
   // launch 2: codes and LoRA-A projection
   QuantLoraArgs q{};
   // (normalized rows that the statistics launch has written for the caller are read as they are)
-  const bool normalize = rms && !p->aux_normalized;
+  const bool normalize = rms && (rows_in_lds || !p->aux_normalized);
   q.x = static_cast<const uint16_t*>(rms && !normalize ? p->aux_normalized : p->x);
   q.gamma = p->rms_gamma;
   q.row_scale = reinterpret_cast<const float*>(ws + w.row_scale);
@@ -525,17 +573,27 @@ int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
   q.group_pad = pad_groups ? 32u : 1u;
   if (!skip_prologue) {
     const dim3 grid(q.n_half_blocks), block(1024);
+    if (rows_in_lds) {
+      QuantLoraRowsArgs qr{};
+      qr.q = q;
+      qr.eps = p->rms_eps; qr.scales_rm = p->aux_x_scales; qr.xn_aux = static_cast<uint16_t*>(p->aux_normalized);
+      if (route_inline) qr.route_idx = p->adapter_indices;
+      qr.src_row = src_row; qr.slot_group = slot_group; qr.blk_range = blk_range;
+      qr.n_groups = p->n_adapters; qr.slots = w.slots; qr.rows_per_wg = quant_lora_rows_per_wg(p->k); qr.row_stride = quant_lora_row_stride(p->k);
+      if ((st = rms ? launch_quant_rows<true>(qr, lora ? w.nkk : 0u, s) : launch_quant_rows<false>(qr, lora ? w.nkk : 0u, s))) return st;
+    } else {
 #define W8A8_QL(CB)                                                                              \
   if (normalize) hipLaunchKernelGGL((quant_lora_kernel<CB, true>), grid, block, 0, s, q);        \
   else hipLaunchKernelGGL((quant_lora_kernel<CB, false>), grid, block, 0, s, q)
-    switch (lora ? w.nkk : 0u) {
-      case 0: W8A8_QL(0); break;
-      case 1: W8A8_QL(1); break;
-      case 2: W8A8_QL(2); break;
-      default: W8A8_QL(4); break;
-    }
+      switch (lora ? w.nkk : 0u) {
+        case 0: W8A8_QL(0); break;
+        case 1: W8A8_QL(1); break;
+        case 2: W8A8_QL(2); break;
+        default: W8A8_QL(4); break;
+      }
 #undef W8A8_QL
-    if ((st = launch_status())) return st;
+      if ((st = launch_status())) return st;
+    }
     if (p->aux_x_codes) {
       hipLaunchKernelGGL(codes_row_major_kernel, dim3(w.rows_bound), dim3(256), 0, s, q.xq_packed, q.src_row, p->aux_x_codes,
                          p->m, p->k, w.KB);

@@ -648,6 +648,18 @@ __device__ inline uint4 rms_normalize8(const uint4& raw, float inv, const float4
   return make_uint4(w[0], w[1], w[2], w[3]);
 }
 
+// The scale of a row from its wave's running maxima.
+__device__ inline float row_scale_of(uint32_t amax_bits) {
+  uint32_t top = (amax_bits >> 16) > (amax_bits & 0xffffu) ? (amax_bits >> 16) : (amax_bits & 0xffffu);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    const uint32_t other = (uint32_t)__shfl_xor((int)top, o, 64);
+    top = other > top ? other : top;
+  }
+  const float amax = __uint_as_float(top << 16);
+  return amax > 0.0f ? amax / 127.0f : 1.0f;
+}
+
 // Statistics of row m by one wave: kPieces 1 KiB pieces of the row in flight at a time.  With RMSNorm the row
 // is read a second time for the normalized maximum (from the L2: its wave has just read it); holding it took
 // registers that cost the launch its second workgroup per CU.
@@ -713,14 +725,7 @@ __device__ inline void row_stats(const LoraPrepArgs& p, uint32_t m) {
       }
     }
   }
-  uint32_t top = (amax_bits >> 16) > (amax_bits & 0xffffu) ? (amax_bits >> 16) : (amax_bits & 0xffffu);
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    const uint32_t other = (uint32_t)__shfl_xor((int)top, o, 64);
-    top = other > top ? other : top;
-  }
-  const float amax = __uint_as_float(top << 16);
-  const float scale = amax > 0.0f ? amax / 127.0f : 1.0f;
+  const float scale = row_scale_of(amax_bits);
   if (lane == 0) {
     p.row_scale[m] = scale;
     if (p.scales_rm) p.scales_rm[m] = scale;
@@ -1019,8 +1024,8 @@ __global__ __launch_bounds__(1024) void lora_a_kernel(LoraAArgs a) {
 // LDS for their scale gave a workgroup 16 of them only up to K = 4608 and four at K = 12288, where every
 // workgroup fetched the whole LoRA A for four rows.  Measured: 4096 x 12288, 8 adapters of rank 32: 22 us
 // (statistics, routing, operand layouts) + 54 us against 14 us (layouts, routing) + 120 us; 333 x 4096, 4 adapters
-// of rank 64: 7 + 16 us against 6 + 20 us; 4096 x 4096 with RMSNorm, where sixteen rows did fit the LDS:
-// 20 + 28 us against 14 + 32 us.
+// of rank 64: 7 + 16 us against 6 + 20 us.  Where the rows fit the LDS and the call has no operands to lay out, or
+// sixteen slots hold several groups, quant_lora_rows_kernel below is the faster one (prologue_keeps_rows).
 // The grouped (per-expert) call takes the same pass, its rows gathered through a row map and their statistics taken once
 // per source row; as a quantizer and a LoRA-A launch over the gathered rows, 16384 of 2048, top 8 of 2048 tokens, it took
 // 7 + 26 + 30 us, now 7 + 31.
@@ -1058,6 +1063,106 @@ __global__ __launch_bounds__(256) void codes_row_major_kernel(const unsigned cha
 }
 
 constexpr uint32_t kPaddedRouteMaxRows = 8192;  // groups start on block boundaries up to here (padded_groups_fit)
+
+// The int8 codes of eight (normalized) bf16 values.
+__device__ inline uint2 quant_codes8(const uint4& raw, float scale, float rscale, bool scale_safe) {
+  const uint32_t nb[4] = {raw.x, raw.y, raw.z, raw.w};  // the (normalized) values as bf16 pairs
+  float v[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e)
+    v[e] = (e & 1) ? __uint_as_float(nb[e >> 1] & 0xffff0000u) : __uint_as_float(nb[e >> 1] << 16);
+  // codes = rint(v / scale) with the correctly rounded quotient.  v * (1 / scale) with the
+  // hardware reciprocal is within 3 * 2^-24 * 128 < 2.3e-5 of it, so both round to the same
+  // integer unless the product lies that close to a tie; those cases (and scales outside the
+  // reciprocal's safe range) are redone with the division.
+  // The codes are formed biased by 128 (the fused v * (1 / scale) + 128 adds at most another 2^-17 to
+  // the distance above, still far inside the tie margin): c is then an integer in [1, 255] (|v| <= the
+  // row's absmax, so the clip of the reference never acts), lands in its byte with one
+  // v_cvt_pk_u8_f32, and flipping bit 7 of every byte turns the biased value into two's complement.
+  float c[8];
+  float off_integer = 0.0f;  // largest distance of a quotient from its rounded value
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float t = __builtin_fmaf(v[e], rscale, 128.0f);
+    c[e] = rintf(t);
+    off_integer = fmaxf(off_integer, fabsf(t - c[e]));
+  }
+  const bool redo = !scale_safe || off_integer > 0.49996f;  // margin 4e-5 > 2.3e-5 + 2^-17
+  if (__builtin_amdgcn_ballot_w64(redo) != 0) {  // wave-uniform
+#pragma unroll
+    for (int e = 0; e < 8; ++e) c[e] = rintf(v[e] / scale) + 128.0f;
+  }
+  uint32_t lo = 0, hi = 0;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    lo = __builtin_amdgcn_cvt_pk_u8_f32(c[e], (uint32_t)e, lo);
+    hi = __builtin_amdgcn_cvt_pk_u8_f32(c[e + 4], (uint32_t)e, hi);
+  }
+  lo ^= 0x80808080u;  // (a lane without a value holds zeros: 0 -> 128 -> code 0)
+  hi ^= 0x80808080u;
+  return make_uint2(lo, hi);
+}
+
+// z of a half block: the waves' tiles added in a fixed order, split into three bf16 terms and stored as the GEMM
+// epilogue reads them (its rows first_row .. end_row - 1).  red: a wave tile each for waves 0..7 (of 16) or 0..3; zs: the
+// sixteen rows of z.
+template <int kCB, uint32_t WAVES>
+__device__ inline void quant_lora_store_z(const QuantLoraArgs& a, v4f (&acc)[kCB], float (*red)[kCB][4][64], float (*zs)[kCB * 16 + 1],
+                                          uint32_t pb, uint32_t half16, uint32_t first_row = 0u, uint32_t end_row = 16u) {
+  const uint32_t tid = threadIdx.x, lane = tid & 63u;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // of 16 waves, 8..15 onto 0..7, 4..7 onto 0..3; then 0+1+2+3
+#pragma unroll 1
+  for (uint32_t half = WAVES / 2u; half >= 4u; half >>= 1) {
+    if (wave >= half && wave < 2u * half) {
+#pragma unroll
+      for (int b = 0; b < kCB; ++b)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) red[wave - half][b][e][lane] = acc[b][e];
+    }
+    __syncthreads();
+    if (wave < half) {
+#pragma unroll
+      for (int b = 0; b < kCB; ++b)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[b][e] = acc[b][e] + red[wave][b][e][lane];
+    }
+    __syncthreads();
+  }
+  if (wave < 4u) {
+#pragma unroll
+    for (int b = 0; b < kCB; ++b)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) red[wave][b][e][lane] = acc[b][e];
+  }
+  __syncthreads();
+  // MFMA result layout: lane l holds column l % 16 and rows 4 * (l / 16) + e
+  for (uint32_t t = tid; t < (uint32_t)kCB * 256u; t += WAVES * 64u) {
+    const uint32_t l = t & 63u, e = (t >> 6) & 3u, b = t >> 8;
+    const float sum = ((red[0][b][e][l] + red[1][b][e][l]) + red[2][b][e][l]) + red[3][b][e][l];
+    zs[4u * (l >> 4) + e][b * 16u + (l & 15u)] = sum;
+  }
+  __syncthreads();
+  // zp[pb][kk][term][lane64][8]: lane = row % 32 + 32 * hh holds rank columns 16 kk + 8 hh + 0..7
+  for (uint32_t t = tid; t < a.nkk * 3u * 32u; t += WAVES * 64u) {
+    const uint32_t row = t & 15u, hh = (t >> 4) & 1u, term = (t >> 5) % 3u, kk = t / 96u;
+    if (row < first_row || row >= end_row) continue;
+    v8us o;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const uint32_t col = 16u * kk + 8u * hh + e;
+      const float z = col < (uint32_t)kCB * 16u ? zs[row][col] : 0.0f;
+      const uint32_t b0 = f32_to_bf16_bits(z);
+      const float r1 = z - bf16_bits_to_f32(b0);
+      const uint32_t b1 = f32_to_bf16_bits(r1);
+      const float r2 = r1 - bf16_bits_to_f32(b1);
+      const uint32_t b2 = f32_to_bf16_bits(r2);
+      o[e] = (unsigned short)(term == 0 ? b0 : (term == 1 ? b1 : (a.nterms >= 3u ? b2 : 0u)));
+    }
+    const uint32_t l64 = 16u * half16 + row + 32u * hh;
+    *reinterpret_cast<v8us*>(a.zp + (((size_t)pb * a.nkk + kk) * 3u + term) * kBlockBytes + l64 * 16u) = o;
+  }
+}
 
 template <int CB, bool RMS, uint32_t WAVES = 16>  // CB: 16-wide rank blocks (0 = no LoRA, 1, 2, 4)
 __global__ __launch_bounds__(WAVES * 64, 4) void quant_lora_kernel(QuantLoraArgs a) {
@@ -1130,41 +1235,7 @@ __global__ __launch_bounds__(WAVES * 64, 4) void quant_lora_kernel(QuantLoraArgs
       raw.x = live ? raw.x : 0u; raw.y = live ? raw.y : 0u; raw.z = live ? raw.z : 0u; raw.w = live ? raw.w : 0u;
     }
     if constexpr (decltype(codes)::value) {
-      const uint32_t nb[4] = {raw.x, raw.y, raw.z, raw.w};  // the (normalized) values as bf16 pairs
-      float v[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e)
-        v[e] = (e & 1) ? __uint_as_float(nb[e >> 1] & 0xffff0000u) : __uint_as_float(nb[e >> 1] << 16);
-      // codes = rint(v / scale) with the correctly rounded quotient.  v * (1 / scale) with the
-      // hardware reciprocal is within 3 * 2^-24 * 128 < 2.3e-5 of it, so both round to the same
-      // integer unless the product lies that close to a tie; those cases (and scales outside the
-      // reciprocal's safe range) are redone with the division.
-      // The codes are formed biased by 128 (the fused v * (1 / scale) + 128 adds at most another 2^-17 to
-      // the distance above, still far inside the tie margin): c is then an integer in [1, 255] (|v| <= the
-      // row's absmax, so the clip of the reference never acts), lands in its byte with one
-      // v_cvt_pk_u8_f32, and flipping bit 7 of every byte turns the biased value into two's complement.
-      float c[8];
-      float off_integer = 0.0f;  // largest distance of a quotient from its rounded value
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float t = __builtin_fmaf(v[e], rscale, 128.0f);
-        c[e] = rintf(t);
-        off_integer = fmaxf(off_integer, fabsf(t - c[e]));
-      }
-      const bool redo = !scale_safe || off_integer > 0.49996f;  // margin 4e-5 > 2.3e-5 + 2^-17
-      if (__builtin_amdgcn_ballot_w64(redo) != 0) {  // wave-uniform
-#pragma unroll
-        for (int e = 0; e < 8; ++e) c[e] = rintf(v[e] / scale) + 128.0f;
-      }
-      uint32_t lo = 0, hi = 0;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        lo = __builtin_amdgcn_cvt_pk_u8_f32(c[e], (uint32_t)e, lo);
-        hi = __builtin_amdgcn_cvt_pk_u8_f32(c[e + 4], (uint32_t)e, hi);
-      }
-      lo ^= 0x80808080u;  // (a lane without a value holds zeros: 0 -> 128 -> code 0)
-      hi ^= 0x80808080u;
-      *reinterpret_cast<uint2*>(xq_dst + (size_t)kb * kBlockBytes) = make_uint2(lo, hi);
+      *reinterpret_cast<uint2*>(xq_dst + (size_t)kb * kBlockBytes) = quant_codes8(raw, scale, rscale, scale_safe);
     }
     if constexpr (CB > 0) {
       // (zeros where the lane has no value; at a group boundary the rows of the other groups are zeroed)
@@ -1212,57 +1283,347 @@ __global__ __launch_bounds__(WAVES * 64, 4) void quant_lora_kernel(QuantLoraArgs
 #pragma unroll 1
     for (uint32_t grp = glo + 1u; grp <= ghi; ++grp) pass(std::false_type{}, grp, rowgrp == grp);
   }
-  if constexpr (CB == 0) return;
+  if constexpr (CB > 0) quant_lora_store_z<kCB, WAVES>(a, acc, red, zs, pb, half16);
+}
 
-  // ---- fixed-order sum of the wave tiles: of 16, 8..15 onto 0..7, 4..7 onto 0..3; then 0+1+2+3
+// ---------------------------------------------------------------------------------------
+// The same with the rows in the LDS: a wave brings one row in with direct-to-LDS loads, takes its statistics there
+// (RMSNorm: and leaves it normalized), and the pass then reads the workgroup's R rows.  No launch takes statistics
+// in front of it, x is read once and normalized once, and a further group among the rows costs a pass over the LDS; in return
+// a workgroup has a CU to itself, starts the pass behind its own chain of statistics, and fetches the whole of A
+// for as few rows as fit.
+// With route_idx the workgroup sorts the adapter indices for its own slots, too, so that a call whose LoRA operands lie
+// in the workspace already has this launch alone in front of the GEMM.
+// ---------------------------------------------------------------------------------------
+// LDS bytes of a row: its 2 K bytes rounded up to the 1 KiB a wave's direct-to-LDS load moves, plus 16 so
+// that the sixteen rows a wave reads side by side (16 bytes each) fall on sixteen different bank groups.
+__host__ __device__ inline uint32_t quant_lora_row_stride(uint32_t k) { return round_up(2u * k, 1024u) + 16u; }
+inline uint32_t quant_lora_rows_per_wg(uint32_t k) {  // 16 up to K = 4608, then 8, from 9728 on 4
+  uint32_t r = 16u;
+  while (r > 4u && r * quant_lora_row_stride(k) > 150u * 1024u) r >>= 1;
+  return r;
+}
+// dynamic LDS of a launch: the rows, or the reduction tiles that reuse the same bytes once the rows are spent
+inline uint32_t quant_lora_rows_lds_bytes(uint32_t k, uint32_t cb) {
+  const uint32_t rows = quant_lora_rows_per_wg(k) * quant_lora_row_stride(k), red = 8u * (cb ? cb : 1u) * 4u * 64u * 4u;
+  return rows > red ? rows : red;
+}
+
+struct QuantLoraRowsArgs {
+  QuantLoraArgs q;           // row_scale, row_inv unused
+  float eps;
+  float* scales_rm;          // f32 [M] for the caller, or null
+  uint16_t* xn_aux;          // bf16 [M, K] normalized rows for the caller, or null (RMS only)
+  // Routing inside this launch (M <= kInlineRouteMaxRows): every workgroup sorts the indices for itself and writes
+  // its slots' entries of the tables, which the GEMM reads.
+  const int32_t* route_idx;  // adapter per row, or null: the tables of an earlier launch, or none
+  int32_t* src_row; int32_t* slot_group; int32_t* blk_range;
+  uint32_t n_groups, slots;
+  uint32_t rows_per_wg, row_stride;
+};
+constexpr uint32_t kInlineRouteMaxRows = 8192;  // eight rows per thread of a 1024-thread workgroup
+
+// The routing tables of route_rows_block for the 16 slots [16 hb, 16 hb + 16), computed by the
+// workgroup itself: rows keep their order inside a group (slot start[g] + j holds the j-th row of group
+// g), which every workgroup derives alike from the adapter indices alone.  Returns through LDS:
+// out_src[16], out_grp[16], out_range (the group range of the 32-slot block that holds the slots).
+// With group_pad = 32 every group starts on a block boundary (the slots between a group's last row and
+// the next group's first stay empty, src -1), so no 32-slot block holds rows of two groups: neither
+// this kernel nor the GEMM's epilogue then runs a block once per group.  The slots in use end at
+// sum(round_up(count, group_pad)) <= M + (group_pad - 1) * min(n_groups, M).
+// Steps: every wave counts its rows per group (LDS atomics on its own counters: with 16 waves on a CU
+// the vector ALU's share per wave makes a ballot per group and row several times dearer); wave 0 turns
+// the counts into per-wave prefixes, the groups' first slots and the groups of the sixteen slots; the
+// waves that hold the wanted ranks of a group pick their rows.  Three barriers.
+__device__ inline void route_rows_inline(const int32_t* __restrict__ idx, uint32_t M, uint32_t n_groups,
+                                         uint32_t slots, uint32_t group_pad, uint32_t hb, int* out_src, int* out_grp,
+                                         uint32_t* out_range, int* out_last_group) {
+  __shared__ int wcnt[kMaxAdapters][17];  // rows of group g in wave w; then the exclusive prefix over the waves
+  __shared__ int start[kMaxAdapters + 1];
+  __shared__ int cnt[kMaxAdapters];
+  __shared__ uint32_t used_end;  // first slot behind the last group
+  __shared__ int g_first_s, g_last_s;
+  const uint32_t tid = threadIdx.x, lane = tid & 63u;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t per = (M + 1023u) / 1024u;  // consecutive rows per thread (<= 8)
+  int mine[8];
+#pragma unroll
+  for (uint32_t j = 0; j < 8; ++j) {
+    const uint32_t i = tid * per + j;
+    int a = -1;
+    if (j < per && i < M) {
+      a = idx[i];
+      a = a < 0 ? 0 : (a >= (int)n_groups ? (int)n_groups - 1 : a);
+    }
+    mine[j] = a;
+  }
+  if (lane < n_groups) wcnt[lane][wave] = 0;  // (the loads above are still in flight)
+  __builtin_amdgcn_wave_barrier();
+#pragma unroll
+  for (uint32_t j = 0; j < 8; ++j)
+    if (j < per && mine[j] >= 0) atomicAdd(&wcnt[mine[j]][wave], 1);  // integer counts of one wave: any order
+  __syncthreads();
+  const uint32_t p0 = hb * 16u;
+  if (wave == 0) {  // lane g: group g (n_groups <= 64)
+    int total = 0;
+    if (lane < n_groups) {
+      int c[16];
+#pragma unroll
+      for (uint32_t w = 0; w < 16; ++w) c[w] = wcnt[lane][w];  // all reads first: one round trip
+#pragma unroll
+      for (uint32_t w = 0; w < 16; ++w) {
+        wcnt[lane][w] = total;
+        total += c[w];
+      }
+    }
+    const int padded = (int)round_up((uint32_t)total, group_pad);
+    int incl = padded;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int up = __shfl_up(incl, off, 64);
+      if ((int)lane >= off) incl += up;
+    }
+    const int st = incl - padded;  // first slot of group `lane`
+    const uint32_t E = (uint32_t)__shfl(incl, 63, 64);
+    const unsigned long long nonempty = __builtin_amdgcn_ballot_w64(total > 0);
+    const int last_ne = nonempty ? 63 - __builtin_clzll(nonempty) : 0;
+    if (lane < n_groups) { start[lane] = st; cnt[lane] = total; }
+    if (lane == 0) { start[n_groups] = (int)E; used_end = E; *out_last_group = last_ne; }
+    // group of a slot: the last group whose first slot is not behind it (empty groups share their
+    // successor's first slot, so the last one is the one that holds the slot); slots behind the last
+    // group follow the last non-empty one
+    auto group_of = [&](uint32_t p) -> int {
+      if (p >= E) return last_ne;
+      const unsigned long long m = __builtin_amdgcn_ballot_w64(lane < n_groups && (uint32_t)st <= p);
+      return m ? 63 - __builtin_clzll(m) : 0;
+    };
+    const uint32_t p_end = (p0 + 16u < E) ? p0 + 16u : E;
+    const int gf = group_of(p0), gl = group_of(p_end ? p_end - 1u : 0u);
+    int my_grp = group_of(p0 + 15u);  // (the slots behind the last group follow the last non-empty one)
+    if (my_grp != gf) {  // wave-uniform: the sixteen slots hold a group boundary (or the end)
+#pragma unroll
+      for (uint32_t s16 = 0; s16 < 16; ++s16) {
+        const int g = group_of(p0 + s16);
+        if (lane == s16) my_grp = g;
+      }
+    }
+    if (lane < 16u) { out_grp[lane] = my_grp; out_src[lane] = -1; }
+    const uint32_t b0 = (p0 / 32u) * 32u;
+    const uint32_t b1 = (b0 + 31u < E) ? b0 + 31u : (E ? E - 1u : 0u);
+    const int gb0 = group_of(b0), gb1 = group_of(b1);
+    if (lane == 0) {
+      *out_range = b0 >= E ? 0u : ((uint32_t)gb0 | ((uint32_t)gb1 << 16));
+      g_first_s = p0 < E ? gf : 1;  // an empty range when the slots lie behind the last group
+      g_last_s = p0 < E ? gl : 0;
+    }
+  }
+  __syncthreads();
+  // the rows of the slots in use, group by group (a workgroup's 16 slots usually lie in one group)
+  const uint32_t E = used_end;
+  const uint32_t p_end = (p0 + 16u < E) ? p0 + 16u : E;
+  const int g_first = g_first_s, g_last = g_last_s;
+  for (int g = g_first; g <= g_last; ++g) {  // workgroup-uniform
+    const int cg = cnt[g], sg = start[g];
+    if (cg == 0) continue;
+    // slots of group g among mine: ranks [lo, hi)
+    const int lo = ((int)p0 > sg ? (int)p0 : sg) - sg;
+    const int hi = ((int)p_end < sg + cg ? (int)p_end : sg + cg) - sg;
+    const int wbefore = wcnt[g][wave];
+    const int wafter = wave < 15u ? wcnt[g][wave + 1u] : cg;
+    if (hi <= lo || wafter <= lo || wbefore >= hi) continue;  // wave-uniform: none of the wanted ranks is in this wave
+    int c = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < 8; ++j) c += (mine[j] == g) ? 1 : 0;
+    int incl = c;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int up = __shfl_up(incl, off, 64);
+      if ((int)lane >= off) incl += up;
+    }
+    int rank = wbefore + incl - c;
+#pragma unroll
+    for (uint32_t j = 0; j < 8; ++j) {
+      if (mine[j] == g) {
+        if (rank >= lo && rank < hi) out_src[sg + rank - (int)p0] = (int)(tid * per + j);
+        ++rank;
+      }
+    }
+  }
+  __syncthreads();
+}
+
+template <int CB, bool RMS>  // CB: 16-wide rank blocks (0 = no LoRA, 1, 2, 4)
+__global__ __launch_bounds__(1024) void quant_lora_rows_kernel(QuantLoraRowsArgs p) {
+  const QuantLoraArgs& a = p.q;
+  constexpr int kCB = CB > 0 ? CB : 1;
+  extern __shared__ __attribute__((aligned(1024))) unsigned char ql_lds[];  // the rows; later the wave tiles of z
+  __shared__ float row_scale[16];
+  __shared__ int row_src[16];
+  __shared__ float zs[16][kCB * 16 + 1];
+  const uint32_t tid = threadIdx.x, lane = tid & 63u;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t R = p.rows_per_wg, per_hb = 16u / R;
+  const uint32_t hb = blockIdx.x / per_hb;           // half block: slots 16 hb .. 16 hb + 15
+  const uint32_t r0 = (blockIdx.x % per_hb) * R;     // this workgroup's slots inside it: r0 .. r0 + R - 1
+  if (a.tile_ctr && blockIdx.x == 0 && tid < 256u) a.tile_ctr[tid] = 0u;
+  if (hb >= a.n_half_blocks) return;
+  const uint32_t pb = hb >> 1, half16 = hb & 1u;
+  __shared__ int route_src[16], route_grp[16], route_last_group;
+  __shared__ uint32_t route_range;
+  const bool route_here = p.route_idx != nullptr;  // kernel-uniform
+  if (route_here) {
+    route_rows_inline(p.route_idx, a.M, p.n_groups, p.slots, a.group_pad, hb, route_src, route_grp, &route_range,
+                      &route_last_group);
+    // the tables the GEMM reads later (every workgroup of a block derives the same range)
+    if (tid >= r0 && tid < r0 + R) {
+      p.src_row[hb * 16u + tid] = route_src[tid];
+      p.slot_group[hb * 16u + tid] = route_grp[tid];
+    }
+    if (tid == 16u) p.blk_range[pb] = (int32_t)route_range;
+    if (blockIdx.x + 1u == gridDim.x) {  // the padding slots behind the last 32-row block, up to the GEMM's tile rows
+      for (uint32_t s = a.n_half_blocks * 16u + tid; s < p.slots; s += 1024u) {
+        p.src_row[s] = -1;
+        p.slot_group[s] = route_last_group;
+        if ((s & 31u) == 0) p.blk_range[s / 32u] = 0;
+      }
+    }
+  }
+  // ---- 1. the rows into the LDS and their statistics: wave w < R, slot row r0 + w
+  const uint32_t slot = hb * 16u + r0 + wave;
+  int wsrc = -1;
+  if (wave < R) wsrc = route_here ? route_src[r0 + wave] : (a.src_row ? a.src_row[slot] : (int)slot);
+  if (wsrc < 0 || wsrc >= (int)a.M) wsrc = -1;
+  wsrc = __builtin_amdgcn_readfirstlane(wsrc);
+  if (a.group_pad > 1u) {  // padded groups leave whole stretches of slots empty: nothing reads their codes, scales or z
+    if (__syncthreads_or(wsrc >= 0) == 0) return;
+  }
+  const uint32_t lds_addr = (uint32_t)(uintptr_t)(lptr_t)ql_lds;
+  const uint32_t row_bytes = 2u * a.K;
+  if (wave < R) {
+    unsigned char* const rowl = ql_lds + wave * p.row_stride;
+    float inv = 1.0f;
+    uint32_t amax_bits = 0;  // largest |value| as bf16 bits in both halves
+    if (wsrc >= 0) {
+      const unsigned char* xr = reinterpret_cast<const unsigned char*>(a.x) + (size_t)wsrc * row_bytes;
+      for (uint32_t off = 0; off < row_bytes; off += 1024u) {
+        const uint32_t voff = off + lane * 16u;
+        if (voff < row_bytes) lds_load_1k(xr, voff, lds_addr + wave * p.row_stride + off);
+      }
+      // (the first piece's norm weights travel with the row)
+      float4 gn0 = make_float4(0.f, 0.f, 0.f, 0.f), gn1 = gn0;
+      if (RMS && lane * 16u < row_bytes) {
+        gn0 = *reinterpret_cast<const float4*>(a.gamma + lane * 8u);
+        gn1 = *reinterpret_cast<const float4*>(a.gamma + lane * 8u + 4);
+      }
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      if (RMS) {
+        double ss = 0.0;
+        for (uint32_t off = lane * 16u; off < row_bytes; off += 1024u) {
+          const uint4 raw = *reinterpret_cast<const uint4*>(rowl + off);
+          const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {  // (exact squares, as in row_stats)
+            const double lo = (double)__uint_as_float(w[e] << 16), hi = (double)__uint_as_float(w[e] & 0xffff0000u);
+            ss = __builtin_fma(lo, lo, ss);
+            ss = __builtin_fma(hi, hi, ss);
+          }
+        }
+        ss = wave_sum(ss);
+        const float var = (float)(ss / (double)a.K);
+        inv = 1.0f / sqrtf(var + p.eps);
+      }
+      for (uint32_t off = lane * 16u; off < row_bytes; off += 1024u) {
+        const float4 g0 = gn0, g1 = gn1;
+        if (RMS && off + 1024u < row_bytes) {  // the norm weights of the next piece are requested before this one is worked on
+          gn0 = *reinterpret_cast<const float4*>(a.gamma + ((off + 1024u) >> 1));
+          gn1 = *reinterpret_cast<const float4*>(a.gamma + ((off + 1024u) >> 1) + 4);
+        }
+        uint4 raw = *reinterpret_cast<const uint4*>(rowl + off);
+        if (RMS) {
+          raw = rms_normalize8(raw, inv, g0, g1);
+          *reinterpret_cast<uint4*>(rowl + off) = raw;  // the normalized row replaces the row
+          if (p.xn_aux) *reinterpret_cast<uint4*>(reinterpret_cast<unsigned char*>(p.xn_aux) + (size_t)wsrc * row_bytes + off) = raw;
+        }
+        amax_bits = bf16_absmax_pairs(amax_bits, raw);
+      }
+    }
+    const float scale = row_scale_of(amax_bits);
+    if (lane == 0) {
+      row_scale[r0 + wave] = scale;
+      row_src[r0 + wave] = wsrc;
+      a.sx_slots[slot] = scale;
+      if (p.scales_rm && wsrc >= 0) p.scales_rm[wsrc] = scale;
+    }
+  }
+  __syncthreads();
+
+  // ---- 2. codes and z: lane (i, q) takes k = 32 kb + 8 q .. + 7 of slot row i, wave w the k-blocks w + 16 j
+  const uint32_t i = lane & 15u, q = lane >> 4;
+  const bool mine_row = i >= r0 && i < r0 + R;  // slot row i belongs to this workgroup
+  const int src = mine_row ? row_src[i] : -1;
+  const float scale = mine_row ? row_scale[i] : 1.0f;
+  const float rscale = __builtin_amdgcn_rcpf(scale);
+  const bool scale_safe = scale > 1e-30f && scale < 1e30f;
+  const unsigned char* const rowl = ql_lds + (mine_row ? i - r0 : 0u) * p.row_stride;
+  const uint32_t range = CB == 0 ? 0u : (route_here ? route_range : (a.blk_range ? (uint32_t)a.blk_range[pb] : 0u));
+  const uint32_t glo = range & 0xffffu, ghi = range >> 16;
+  const uint32_t rowgrp = (CB > 0 && ghi > glo)
+                              ? (route_here ? (uint32_t)route_grp[i] : (a.slot_group ? (uint32_t)a.slot_group[hb * 16u + i] : glo))
+                              : glo;
+  v4f acc[kCB];
+#pragma unroll
+  for (int b = 0; b < kCB; ++b) acc[b] = v4f{0.f, 0.f, 0.f, 0.f};
+  unsigned char* const xq_dst =
+      a.xq_packed + (size_t)pb * a.KB * kBlockBytes + (16u * half16 + i + 32u * (q >> 1)) * 16u + 8u * (q & 1u);
+  // One pass over the k-blocks per group present among the slots (one, except at a group boundary): the
+  // first pass also forms the codes; a later pass only adds the rows of its group to z.  The loop is kept rolled, two
+  // k-blocks per trip with their operands requested one trip ahead and no load inside the work on a
+  // k-block, so that the compiler's waits count loads instead of draining them.
+  auto request = [&](uint32_t grp, uint32_t kb, v4i (&w)[kCB], uint4& raw) {
+    if constexpr (CB > 0) {
+      // operands of group grp, k-block kb: CB consecutive 1 KiB pieces (zero beyond K and the rank)
+      const v4i* ap = reinterpret_cast<const v4i*>(a.at) + (((size_t)grp * a.KB + kb) * CB) * 64u + lane;
+#pragma unroll
+      for (int b = 0; b < CB; ++b) w[b] = kb < a.KB ? ap[b * 64] : v4i{0, 0, 0, 0};
+    }
+    const uint32_t k0 = kb * 32u + q * 8u;
+    raw = (kb < a.KB && k0 < a.K && src >= 0) ? *reinterpret_cast<const uint4*>(rowl + 2u * k0) : make_uint4(0, 0, 0, 0);
+  };
+  auto work = [&](bool first, bool in_group, uint32_t kb, const v4i (&w)[kCB], const uint4& raw) {
+    if (first) {  // wave-uniform
+      const uint2 codes = quant_codes8(raw, scale, rscale, scale_safe);
+      if (mine_row) *reinterpret_cast<uint2*>(xq_dst + (size_t)kb * kBlockBytes) = codes;
+    }
+    if constexpr (CB > 0) {
+      // (zeros where the lane has no value; at a group boundary the rows of the other groups are zeroed)
+      const v4i xa = in_group ? v4i{(int)raw.x, (int)raw.y, (int)raw.z, (int)raw.w} : v4i{0, 0, 0, 0};
+#pragma unroll
+      for (int b = 0; b < CB; ++b)
+        acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, xa), __builtin_bit_cast(v8bf, w[b]),
+                                                         acc[b], 0, 0, 0);
+    }
+  };
 #pragma unroll 1
-  for (uint32_t half = WAVES / 2u; half >= 4u; half >>= 1) {
-    if (wave >= half && wave < 2u * half) {
-#pragma unroll
-      for (int b = 0; b < kCB; ++b)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) red[CB > 0 ? wave - half : 0u][b][e][lane] = acc[b][e];
+  for (uint32_t grp = glo; grp <= ghi; ++grp) {  // workgroup-uniform: one trip except at a group boundary
+    const bool first = grp == glo;
+    const bool in_group = ghi == glo || rowgrp == grp;
+    v4i wa[kCB], wb2[kCB];
+    uint4 ra, rb;
+    request(grp, wave, wa, ra);
+    request(grp, wave + 16u, wb2, rb);
+#pragma unroll 1
+    for (uint32_t kb = wave; kb < a.KB; kb += 32u) {
+      work(first, in_group, kb, wa, ra);
+      request(grp, kb + 32u, wa, ra);
+      if (kb + 16u >= a.KB) break;  // wave-uniform
+      work(first, in_group, kb + 16u, wb2, rb);
+      request(grp, kb + 48u, wb2, rb);
     }
-    __syncthreads();
-    if (wave < half) {
-#pragma unroll
-      for (int b = 0; b < kCB; ++b)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) acc[b][e] = acc[b][e] + red[CB > 0 ? wave : 0u][b][e][lane];
-    }
-    __syncthreads();
+    if constexpr (CB == 0) break;
   }
-  if (wave < 4u) {
-#pragma unroll
-    for (int b = 0; b < kCB; ++b)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) red[CB > 0 ? wave : 0u][b][e][lane] = acc[b][e];
-  }
-  __syncthreads();
-  // MFMA result layout: lane l holds column l % 16 and rows 4 * (l / 16) + e
-  for (uint32_t t = tid; t < (uint32_t)kCB * 256u; t += WAVES * 64u) {
-    const uint32_t l = t & 63u, e = (t >> 6) & 3u, b = t >> 8;
-    const float sum = ((red[0][b][e][l] + red[CB > 0 ? 1 : 0][b][e][l]) + red[CB > 0 ? 2 : 0][b][e][l]) + red[CB > 0 ? 3 : 0][b][e][l];
-    zs[4u * (l >> 4) + e][b * 16u + (l & 15u)] = sum;
-  }
-  __syncthreads();
-  // zp[pb][kk][term][lane64][8]: lane = row % 32 + 32 * hh holds rank columns 16 kk + 8 hh + 0..7
-  for (uint32_t t = tid; t < a.nkk * 3u * 32u; t += WAVES * 64u) {
-    const uint32_t row = t & 15u, hh = (t >> 4) & 1u, term = (t >> 5) % 3u, kk = t / 96u;
-    v8us o;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const uint32_t col = 16u * kk + 8u * hh + e;
-      const float z = col < (uint32_t)kCB * 16u ? zs[row][col] : 0.0f;
-      const uint32_t b0 = f32_to_bf16_bits(z);
-      const float r1 = z - bf16_bits_to_f32(b0);
-      const uint32_t b1 = f32_to_bf16_bits(r1);
-      const float r2 = r1 - bf16_bits_to_f32(b1);
-      const uint32_t b2 = f32_to_bf16_bits(r2);
-      o[e] = (unsigned short)(term == 0 ? b0 : (term == 1 ? b1 : (a.nterms >= 3u ? b2 : 0u)));
-    }
-    const uint32_t l64 = 16u * half16 + row + 32u * hh;
-    *reinterpret_cast<v8us*>(a.zp + (((size_t)pb * a.nkk + kk) * 3u + term) * kBlockBytes + l64 * 16u) = o;
+  if constexpr (CB > 0) {
+    __syncthreads();  // the rows are spent: their bytes take the wave tiles
+    quant_lora_store_z<kCB, 16u>(a, acc, reinterpret_cast<float (*)[kCB][4][64]>(ql_lds), zs, pb, half16, r0, r0 + R);
   }
 }
 
