@@ -595,8 +595,8 @@ int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
       if ((st = launch_status())) return st;
     }
     if (p->aux_x_codes) {
-      hipLaunchKernelGGL(codes_row_major_kernel, dim3(w.rows_bound), dim3(256), 0, s, q.xq_packed, q.src_row, p->aux_x_codes,
-                         p->m, p->k, w.KB);
+      hipLaunchKernelGGL(codes_row_major_kernel, dim3(w.rows_bound), dim3(256), 0, s, q.xq_packed, nullptr, q.src_row,
+                         p->aux_x_codes, nullptr, p->m, p->k, w.KB);
       if ((st = launch_status())) return st;
     }
   } else if (!skip_gemm && path != MI355_W8A8_PATH_TILED_256X256) {
@@ -815,7 +815,7 @@ int run_grouped(const mi355_w8a8_grouped_problem* p, hipStream_t s) {
     q.group_pad = 32u;
     q.row_map = p->x_row_map; q.row_div = x_repeat; q.row_limit = x_rows; q.scale_by_source = by_source ? 1u : 0u;
     if ((st = launch_grouped_quant(q, lora ? w.nkk : 0u, s))) return st;
-    if (p->aux_x_codes || p->aux_x_scales) {  // the caller's copies, row by row (rows without a slot among them)
+    if (p->aux_x_codes || p->aux_x_scales) {  // the caller's copies: of every row (some have no slot), then what the GEMM reads
       QuantArgs c{};
       c.x = static_cast<const uint16_t*>(p->x);
       c.M = p->m; c.K = p->k; c.K_pad = w.K_pad; c.KB = w.KB;
@@ -823,6 +823,9 @@ int run_grouped(const mi355_w8a8_grouped_problem* p, hipStream_t s) {
       c.scales_rm = p->aux_x_scales;
       c.row_map = p->x_row_map; c.row_div = x_repeat; c.row_limit = x_rows;
       if ((st = launch_quant<false>(c, s))) return st;
+      hipLaunchKernelGGL(codes_row_major_kernel, dim3(w.slots), dim3(256), 0, s, q.xq_packed, q.sx_slots, src_row,
+                         p->aux_x_codes, p->aux_x_scales, p->m, p->k, w.KB);
+      if ((st = launch_status())) return st;
     }
   }
   if (skip_gemm) return MI355_W8A8_OK;

@@ -1052,12 +1052,16 @@ struct QuantLoraArgs {
   uint32_t row_div, row_limit, scale_by_source;
 };
 
-// Row-major copy of the packed codes for a caller that asks for them (one workgroup per slot).
-__global__ __launch_bounds__(256) void codes_row_major_kernel(const unsigned char* __restrict__ xq, const int32_t* __restrict__ src_row,
-                                                              int8_t* __restrict__ codes, uint32_t M, uint32_t K, uint32_t KB) {
+// Row-major copies of the packed codes and of the slots' scales for a caller that asks for them (one workgroup per slot;
+// either may be null).
+__global__ __launch_bounds__(256) void codes_row_major_kernel(const unsigned char* __restrict__ xq, const float* __restrict__ sx,
+                                                              const int32_t* __restrict__ src_row, int8_t* __restrict__ codes,
+                                                              float* __restrict__ scales, uint32_t M, uint32_t K, uint32_t KB) {
   const uint32_t p = blockIdx.x;
   const int src = src_row ? src_row[p] : (int)p;
   if (src < 0 || src >= (int)M) return;
+  if (scales && threadIdx.x == 0) scales[src] = sx[p];
+  if (!codes) return;
   for (uint32_t k = threadIdx.x * 8u; k < K; k += 2048u)
     *reinterpret_cast<uint2*>(codes + (size_t)src * K + k) = *reinterpret_cast<const uint2*>(xq + packed_offset(p, k, KB));
 }
