@@ -898,6 +898,7 @@ struct BwdLayout {
   uint64_t part;
   uint64_t dyp, swp, at, ap, rp, z, r_raw, rs, rpart, src_row, dst_pos, slot_group, blk_range, group_off, partA, partB, total;
   uint64_t beyond;  // group-scaled calls
+  uint32_t part_blocks;
   uint32_t slots, nkk, K_pad, KB, N_pad, NB, tiles_m, tiles_k, max_chunks, R, n_slices, groups_per_slice;
 };
 
@@ -920,9 +921,13 @@ BwdLayout make_bwd_layout(uint32_t m, uint32_t k, uint32_t n, uint32_t n_groups,
     w.n_slices = (ng + 3u) / 4u < 8u ? (ng + 3u) / 4u : 8u;
     w.groups_per_slice = (ng + w.n_slices - 1u) / w.n_slices;
   }
-  w.split = bwd_dx_split(w.tiles_m, w.tiles_k, w.NB, gq_k_pad ? 1u : 2u);
+  const uint32_t k_blocks = gq_k_pad ? 1u : 2u;  // of a wave's tile
+  w.split = bwd_dx_split(w.tiles_m, w.tiles_k, w.NB, k_blocks);
+  w.part_blocks = w.tiles_m > 1u ? 8u : (m + 31u) / 32u;
   uint64_t off = 0;
-  w.part = off; off += (uint64_t)w.split.sk_wgs * 2u * kBwdPartFloats * 2u * 4u;
+  w.part = off;
+  if (w.split.sk_wgs)  // a partial tile per workgroup, and another wherever a tile ends inside its stages
+    off += (uint64_t)(w.split.sk_wgs + w.tiles_m * w.tiles_k - w.split.direct_tiles) * w.part_blocks * kBwdPartBlockFloats * k_blocks * 4u;
   w.dyp = off; off += align256((uint64_t)w.slots * w.N_pad * 2u);
   w.swp = off; off += align256((uint64_t)(w.N_pad + kBwdScalePad) * 4u);  // a stage fetches 1 KiB of scales starting at its own 32
   w.src_row = off; off += align256((uint64_t)w.slots * 4u);
@@ -994,7 +999,7 @@ struct BwdBody {
   const int32_t* group_end;
   size_t w_stride; uint32_t sw_stride;
   bool rows128;  // the pull-back runs 128-row x 512-k tiles (the tables are padded to match)
-  BwdDxSplit split; uint64_t part;  // dense calls
+  BwdDxSplit split; uint64_t part; uint32_t part_blocks;  // dense calls
   // group-scaled weights: their format (weight_bits 0: per-channel), A itself and the notes of non-finite operands
   uint32_t weight_bits, group, terms; const float* w_scales;
   const void* lora_a; uint64_t beyond;
@@ -1109,6 +1114,7 @@ int launch_bwd_body(const BwdBody& b, const Layout& w, unsigned char* ws, hipStr
     g.direct_tiles = b.split.sk_wgs ? b.split.direct_tiles : w.tiles_m * w.tiles_k;
     g.sk_q = b.split.sk_q; g.sk_wgs = b.split.sk_wgs;
     g.part = b.split.sk_wgs ? reinterpret_cast<float*>(ws + b.part) : nullptr;
+    g.part_blocks = b.part_blocks;
     if (b.weight_bits) {
       GqBwdDxArgs a{};
       a.g = g;
@@ -1256,7 +1262,7 @@ int run_backward(const mi355_w8a8_bwd_problem* p, hipStream_t s) {
   b.slot_group = routed ? slot_group : nullptr;
   b.blk_range = routed ? blk_range : nullptr;
   b.group_off = group_off;
-  b.split = w.split; b.part = w.part;
+  b.split = w.split; b.part = w.part; b.part_blocks = w.part_blocks;
   return launch_bwd_body(b, w, ws, s);
 }
 
@@ -1320,7 +1326,7 @@ int run_gq_backward(const mi355_w8a8_gq_bwd_problem* p, hipStream_t s) {
   b.dx = p->dx; b.d_lora_a = p->d_lora_a; b.d_lora_b = p->d_lora_b; b.d_lora_scaling = p->d_lora_scaling;
   b.lora = lora; b.want_grads = want_grads; b.skip_gemm = no_dx;
   b.group_off = reinterpret_cast<int32_t*>(ws + w.group_off);
-  b.split = w.split; b.part = w.part;
+  b.split = w.split; b.part = w.part; b.part_blocks = w.part_blocks;
   b.weight_bits = p->weight_bits; b.group = p->group_size; b.w_scales = p->w_scales;
   b.lora_a = p->lora_a; b.beyond = w.beyond;
   b.terms = (p->flags & MI355_W8A8_FLAG_GQ_BF16_SCALES) ? 2u : 3u;

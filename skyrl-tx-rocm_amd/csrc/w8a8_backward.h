@@ -450,9 +450,17 @@ struct BwdDxArgs {
   // dense calls: the tiles from direct_tiles on are split (bwd_dx_split): sk_wgs workgroups take sk_q
   // consecutive stages each of their joint stage sequence and leave float32 partial tiles in part
   uint32_t direct_tiles, sk_q, sk_wgs;
-  float* part;   // [2 * sk_wgs slots][8 waves][4 row blocks][k blocks of a wave][4][64 lanes][4]
+  // [slot w + u of workgroup w's stages of split tile u][part_blocks row blocks][4 wave columns][k blocks of a wave][4][64 lanes][4]
+  float* part;
+  uint32_t part_blocks;  // 8, or the blocks that hold rows when there is one row tile
 };
-constexpr uint32_t kBwdPartFloats = 32768;  // of a slot, per k block of a wave
+constexpr uint32_t kBwdPartBlockFloats = 4096;  // of a row block of a slot, per k block of a wave
+
+// Where a wave keeps its block of a partial tile (CBN k blocks); row_block: of the tile's eight.
+template <int CBN>
+__device__ inline float4* bwd_dx_part(const BwdDxArgs& g, uint32_t slot, uint32_t row_block, uint32_t wcol) {
+  return reinterpret_cast<float4*>(g.part) + ((size_t)(slot * g.part_blocks + row_block) * 4u + wcol) * (256u * CBN) + (threadIdx.x & 63u);
+}
 
 // (row tile, k tile) of position t in the band-major tile order: 4 row tiles x all k tiles to a band
 __device__ inline void bwd_dx_tile_at(const BwdDxArgs& g, uint32_t t, uint32_t& tm, uint32_t& tk) {
@@ -749,15 +757,16 @@ __global__ __launch_bounds__(512, 1) void bwd_dx_kernel(BwdDxArgs g) {
         if (rb < n_act)
           bwd_dx_store_block<NKK, 2>(g, tm * (uint32_t)(kRowBlocks * 32) + (uint32_t)wrow * 128u + rb * 32u, kbw, acc[rb]);
     } else {
-      float4* dst = reinterpret_cast<float4*>(g.part + (size_t)slot * (2u * kBwdPartFloats)) + (uint32_t)wave * 2048u + lane;
 #pragma unroll
       for (int rb = 0; rb < 4; ++rb)
-        if (rb < n_act)
+        if (rb < n_act) {
+          float4* dst = bwd_dx_part<2>(g, slot, (uint32_t)(wrow * 4 + rb), (uint32_t)wcol);
 #pragma unroll
           for (int cb = 0; cb < 2; ++cb)
 #pragma unroll
             for (int e = 0; e < 4; ++e)
-              dst[((rb * 2 + cb) * 4 + e) * 64] = make_float4(acc[rb][cb][4 * e], acc[rb][cb][4 * e + 1], acc[rb][cb][4 * e + 2], acc[rb][cb][4 * e + 3]);
+              dst[(cb * 4 + e) * 64] = make_float4(acc[rb][cb][4 * e], acc[rb][cb][4 * e + 1], acc[rb][cb][4 * e + 2], acc[rb][cb][4 * e + 3]);
+        }
     }
   };
 
@@ -779,7 +788,6 @@ __global__ __launch_bounds__(512, 1) void bwd_dx_kernel(BwdDxArgs g) {
     s0 = sk_w * g.sk_q < total ? sk_w * g.sk_q : total;
     s1 = s0 + g.sk_q < total ? s0 + g.sk_q : total;
   }
-  const uint32_t sk_t0 = s0 / g.NB;
 #pragma unroll 1
   for (;;) {
     uint32_t t, nb0 = 0, len = g.NB, slot = 0;
@@ -801,7 +809,7 @@ __global__ __launch_bounds__(512, 1) void bwd_dx_kernel(BwdDxArgs g) {
       nb0 = s0 - u * g.NB;
       len = s1 - s0 < g.NB - nb0 ? s1 - s0 : g.NB - nb0;
       t = ntile + u;
-      slot = 2u * sk_w + (u == sk_t0 ? 0u : 1u);
+      slot = sk_w + u;
       s0 += len;
     } else {
       break;
@@ -816,7 +824,6 @@ __global__ __launch_bounds__(512, 1) void bwd_dx_kernel(BwdDxArgs g) {
 // kernel's own epilogue.  A wave per block of 32 rows x CBN k blocks (CBN: k blocks of a wave's tile).
 template <int NKK, int CBN>
 __global__ __launch_bounds__(256) void bwd_dx_finish_kernel(BwdDxArgs g) {
-  const uint32_t lane = threadIdx.x & 63u;
   const uint32_t item = blockIdx.x * 4u + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t u = item >> 5, wave = (item >> 2) & 7u, rb = item & 3u;
   const uint32_t first = u * g.NB / g.sk_q, last = ((u + 1u) * g.NB - 1u) / g.sk_q;
@@ -832,8 +839,7 @@ __global__ __launch_bounds__(256) void bwd_dx_finish_kernel(BwdDxArgs g) {
 #pragma unroll
     for (int e = 0; e < 16; ++e) y[cb][e] = 0.0f;
   for (uint32_t w = first; w <= last; ++w) {
-    const uint32_t slot = 2u * w + (w * g.sk_q / g.NB == u ? 0u : 1u);
-    const float4* src = reinterpret_cast<const float4*>(g.part) + ((size_t)slot * 32u + wave * 4u + rb) * (256u * CBN) + lane;
+    const float4* src = bwd_dx_part<CBN>(g, w + u, (wave >> 2) * 4u + rb, wave & 3u);
 #pragma unroll
     for (int cb = 0; cb < CBN; ++cb)
 #pragma unroll

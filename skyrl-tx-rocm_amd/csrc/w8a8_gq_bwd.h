@@ -318,13 +318,14 @@ __global__ __launch_bounds__(512, 1) void gq_bwd_dx_kernel(GqBwdDxArgs a) {
           bwd_dx_store_block<NKK, 1>(g, tm * 256u + (uint32_t)wrow * 128u + rb * 32u, kbw, one);
         }
     } else {
-      float4* dst = reinterpret_cast<float4*>(g.part + (size_t)slot * kBwdPartFloats) + (uint32_t)wave * 1024u + lane;
 #pragma unroll
       for (int rb = 0; rb < 4; ++rb)
-        if (rb < n_act)
+        if (rb < n_act) {
+          float4* dst = bwd_dx_part<1>(g, slot, (uint32_t)(wrow * 4 + rb), (uint32_t)wcol);
 #pragma unroll
           for (int e = 0; e < 4; ++e)
-            dst[(rb * 4 + e) * 64] = make_float4(acc[rb][4 * e], acc[rb][4 * e + 1], acc[rb][4 * e + 2], acc[rb][4 * e + 3]);
+            dst[e * 64] = make_float4(acc[rb][4 * e], acc[rb][4 * e + 1], acc[rb][4 * e + 2], acc[rb][4 * e + 3]);
+        }
     }
   };
 
@@ -340,7 +341,6 @@ __global__ __launch_bounds__(512, 1) void gq_bwd_dx_kernel(GqBwdDxArgs a) {
     s0 = sk_w * g.sk_q < total ? sk_w * g.sk_q : total;
     s1 = s0 + g.sk_q < total ? s0 + g.sk_q : total;
   }
-  const uint32_t sk_t0 = s0 / g.NB;
 #pragma unroll 1
   for (;;) {
     uint32_t t, nb0 = 0, len = g.NB, slot = 0;
@@ -353,7 +353,7 @@ __global__ __launch_bounds__(512, 1) void gq_bwd_dx_kernel(GqBwdDxArgs a) {
       nb0 = s0 - u * g.NB;
       len = s1 - s0 < g.NB - nb0 ? s1 - s0 : g.NB - nb0;
       t = ntile + u;
-      slot = 2u * sk_w + (u == sk_t0 ? 0u : 1u);
+      slot = sk_w + u;
       s0 += len;
     } else {
       break;
