@@ -383,6 +383,8 @@ void skinny_stream_kernel(SkinnyStreamArgs a) {
     return f;
   };
   const bool lora = a.lora_b != nullptr;
+  // an odd number of values in B: the dword gathers would read two bytes behind it (NS = 2: N is even)
+  const bool odd_b = NS == 1 && (a.n_adapters & a.r & a.N & 1u);
   const uint32_t rpad = (a.r + 3u) & ~3u;
   const uint32_t rp = a.r <= 32u ? 32u : 64u;            // ranks of a staged z row
   uint32_t* const bst = reinterpret_cast<uint32_t*>(sk_lds);
@@ -421,10 +423,19 @@ void skinny_stream_kernel(SkinnyStreamArgs a) {
       const uint32_t dst = lds0 + m * rpad * 64u + (m >> 2) * 64u;
       uint32_t col = 128u * grp + 4u * pc + j0;
       if (col + NS > a.N) col = 0u;
-      for (uint32_t i = 0; i < rpad / 4u; ++i) {
-        uint32_t rr = 4u * i + q;
-        rr = rr < a.r ? rr : a.r - 1u;
-        lds_gather_dword(brow, ((rr * a.N + col + odd0) * 2u) & ~3u, dst + i * 256u);
+      if (!(odd_b && ad + 1 == (int)a.n_adapters)) {
+        for (uint32_t i = 0; i < rpad / 4u; ++i) {
+          uint32_t rr = 4u * i + q;
+          rr = rr < a.r ? rr : a.r - 1u;
+          lds_gather_dword(brow, ((rr * a.N + col + odd0) * 2u) & ~3u, dst + i * 256u);
+        }
+      } else {  // B's last value has no whole dword: it is loaded by itself
+        for (uint32_t i = 0; i < rpad / 4u; ++i) {
+          uint32_t rr = 4u * i + q;
+          rr = rr < a.r ? rr : a.r - 1u;
+          if (rr + 1u == a.r && col + 1u == a.N) bst[(dst - lds0) / 4u + i * 64u + lane] = brow[rr * a.N + col + odd0];
+          else lds_gather_dword(brow, ((rr * a.N + col + odd0) * 2u) & ~3u, dst + i * 256u);
+        }
       }
     }
     const uint32_t per_piece = 1024u / (rp * 4u), pieces = (rows + per_piece - 1u) / per_piece;
@@ -490,7 +501,10 @@ void skinny_stream_kernel(SkinnyStreamArgs a) {
     lds_gather_dword(a.sx, srow * 4u, fst_addr);
     lds_gather_dword(a.sw, scol * 4u, fst_addr + 2048u);
     if (lora) lds_gather_dword(a.row_scaling, srow * 4u, fst_addr + 4096u);
-    if (a.residual) lds_gather_dword(a.residual, (res_elem * 2u) & ~3u, fst_addr + 6144u);
+    if (a.residual) {  // (the last of an odd number of values: as above)
+      if (NS == 1 && (a.M & a.N & 1u) && res_elem + 1u == a.M * a.N) fst[1536u + threadIdx.x] = a.residual[res_elem];
+      else lds_gather_dword(a.residual, (res_elem * 2u) & ~3u, fst_addr + 6144u);
+    }
     if constexpr (NS == 2) lds_gather_dword(a.sw, (scol + 1u < a.N ? scol + 1u : scol) * 4u, fst_addr + 8192u);
   }
 
