@@ -92,11 +92,19 @@ typedef enum mi355_w8a8_status {
  * places that depend on (k, n, n_adapters, rank) only, so the earlier call may have had another m, other
  * adapter_indices or another tile geometry.  The caller vouches for it; calls that run as 32-row chunks
  * keep no such copies and ignore the flag. */
-/* Calls of at most 32 rows (the skinny-M kernels) read A and B as they are, keep nothing and ignore it too. */
+/* Calls of at most 32 rows (the skinny-M kernels, with SwiGLU too) write no such copies and ignore it: a larger call
+ * may not rely on one of them.  What they can keep has flags of its own, MI355_W8A8_FLAG_DECODE_B_WRITE / _KEPT. */
 /* mi355_w8a8_grouped_v1 takes the flag too: its launch that lays out the slots then leaves the transposed A
  * and the packed B of an earlier grouped call on the same workspace with the same (k, n, n_groups, rank) as
  * they are. */
 #define MI355_W8A8_FLAG_LORA_PACK_VALID 1024u
+/* Calls of at most 16 rows, rank at most 32, m * rank at least 256, n a multiple of 4, without SwiGLU: B regrouped per row and adapter in the
+ * workspace (a loop over the same batch reads it faster than B itself).  WRITE: this call regroups B and uses it.  KEPT: the
+ * workspace holds what a call with WRITE left there, for the same m, k, n, n_adapters and rank and the same contents
+ * of lora_b and adapter_indices, and no other call has used the workspace with other dimensions since; the
+ * caller vouches for it.  Pass the flag to the workspace query.  Other calls ignore both. */
+#define MI355_W8A8_FLAG_DECODE_B_WRITE 8192u
+#define MI355_W8A8_FLAG_DECODE_B_KEPT 16384u
 
 /*
  * One forward call.  y = dequant(quant(n) @ W) + s[idx] * ((n @ A[idx]) @ B[idx]) (+ residual),

@@ -101,7 +101,7 @@ inline bool padded_groups_fit(uint32_t m, uint32_t n, uint32_t n_groups, bool wi
 }
 
 WsLayout make_layout(uint32_t m, uint32_t k, uint32_t n, uint32_t n_groups, uint32_t rank, bool routed,
-                     bool pad_groups = false) {
+                     bool pad_groups = false, bool keep_b = false) {
   WsLayout w{};
   w.K_pad = k_padded(k);
   w.KB = w.K_pad / 32u;
@@ -127,7 +127,7 @@ WsLayout make_layout(uint32_t m, uint32_t k, uint32_t n, uint32_t n_groups, uint
   w.blk_range = off; off += align256((uint64_t)(w.slots / 32u) * 4u);
   w.tile_ctr = off; off += 1024u;  // two sets of eight counters, 64 bytes apart
   w.zp = off; off += rank ? align256((uint64_t)(w.slots / 32u) * w.nkk * 3u * kBlockBytes) : 0u;
-  w.skinny = off; off += align256(skinny_workspace_bytes());
+  w.skinny = off; off += align256(skinny_layout(k, keep_b, m, n, rank).total);
   w.total = off;
   return w;
 }
@@ -264,13 +264,11 @@ int launch_skinny_stream_one(const SkinnyStreamArgs& a, uint32_t lds_bytes, hipS
 }
 
 // The stream kernel's instantiation: KP covers a wave's share of K in one round where registers allow it
-// (KP * (NS + RB) operands of four registers), so that all of it is in flight at once.  Slices of 16 columns
-// while 32-column units would leave CUs idle (fewer than 512 units: two workgroups share a CU); SwiGLU and
-// residual decide for themselves (a gate/up pair is two slices; the residual's dword gather serves one column).
+// (KP * (NS + RB) operands of four registers), so that all of it is in flight at once.
 int launch_skinny_stream(SkinnyStreamArgs& a, hipStream_t s) {
-  const bool pairs = a.swiglu || (!a.residual && (a.N & 1u) == 0 && a.n_groups * 4u >= 512u);
+  const bool pairs = skinny_pairs(a.N, a.swiglu != 0, a.residual != nullptr);
   const uint32_t rb = a.M > 16u ? 2u : 1u, ns = pairs ? 2u : 1u, ppw = a.pairs_per_wave;
-  const SkinnyStreamLds L = skinny_stream_lds(a.M, a.lora_b ? a.r : 0u, a.z_chunks, ns, rb);
+  const SkinnyStreamLds L = skinny_stream_lds(a.M, a.lora_b ? a.r : 0u, a.z_chunks, ns, rb, a.bsel != nullptr);
   a.z_off = L.z_off; a.tail_off = L.tail_off;
   if (ns == 1u && rb == 1u) {
     if (ppw <= 4u) return launch_skinny_stream_one<1, 1, 4>(a, L.bytes, s);
@@ -294,12 +292,18 @@ int launch_skinny_stream(SkinnyStreamArgs& a, hipStream_t s) {
 
 // Skinny-M path: quantize (+ LoRA-A units) -> stream the weight and finish.
 int launch_skinny(const mi355_w8a8_problem* p, unsigned char* xq, float* sx, unsigned char* sws, uint32_t K_pad,
-                  uint32_t KB, hipStream_t s) {
+                  uint32_t KB, hipStream_t s, bool allow_kept_b = true) {
   const bool rms = p->rms_gamma != nullptr;
   const bool lora = p->n_adapters > 0;
+  const bool skip_prologue = (p->flags & MI355_W8A8_FLAG_SKIP_PROLOGUE) != 0;
+  // B regrouped per unit: written by this call, or kept from an earlier one
+  const bool can_keep_b = allow_kept_b && lora && skinny_b_can_be_kept(p->m, p->n, p->rank, (p->flags & MI355_W8A8_FLAG_SWIGLU) != 0) &&
+                          !skinny_pairs(p->n, false, p->residual != nullptr);
+  const bool write_b = can_keep_b && !skip_prologue && (p->flags & MI355_W8A8_FLAG_DECODE_B_WRITE);
+  const bool use_b = write_b || (can_keep_b && (p->flags & MI355_W8A8_FLAG_DECODE_B_KEPT));
   const SkinnyLayout L = skinny_layout(p->k);
   int st;
-  if (!(p->flags & MI355_W8A8_FLAG_SKIP_PROLOGUE)) {
+  if (!skip_prologue) {
     SkinnyQuantArgs q{};
     q.x = static_cast<const uint16_t*>(p->x);
     q.gamma = p->rms_gamma;
@@ -315,7 +319,9 @@ int launch_skinny(const mi355_w8a8_problem* p, unsigned char* xq, float* sx, uns
     q.n_z_units = lora ? p->m * L.z_chunks : 0u;
     q.lora_scaling = lora ? p->lora_scaling : nullptr;
     q.row_scaling = reinterpret_cast<float*>(sws + L.row_scaling);
-    const dim3 grid(p->m + q.n_z_units), block(1024);
+    q.N = p->n; q.n_groups = n_padded(p->n) / 128u;
+    if (write_b) { q.lora_b = static_cast<const uint16_t*>(p->lora_b); q.bsel = reinterpret_cast<uint16_t*>(sws + L.bsel); }
+    const dim3 grid(p->m + q.n_z_units + (write_b ? (p->m * q.n_groups + 15u) / 16u : 0u)), block(1024);
     if (rms) hipLaunchKernelGGL((skinny_quant_kernel<true>), grid, block, 0, s, q);
     else hipLaunchKernelGGL((skinny_quant_kernel<false>), grid, block, 0, s, q);
     if ((st = launch_status())) return st;
@@ -327,6 +333,7 @@ int launch_skinny(const mi355_w8a8_problem* p, unsigned char* xq, float* sx, uns
   a.z_part = reinterpret_cast<const float*>(sws + L.z_part);
   a.sx = sx; a.sw = p->w_scales;
   a.lora_b = lora ? static_cast<const uint16_t*>(p->lora_b) : nullptr;
+  a.bsel = use_b ? reinterpret_cast<const uint16_t*>(sws + L.bsel) : nullptr;
   a.idx = p->adapter_indices;
   a.row_scaling = reinterpret_cast<const float*>(sws + L.row_scaling);
   a.residual = static_cast<const uint16_t*>(p->residual);
@@ -351,9 +358,8 @@ int choose_forward_path(uint32_t m, uint32_t k, uint32_t n, uint32_t flags) {
     if (m > (uint32_t)kSkinnyMaxRows) return MI355_W8A8_ERR_UNSUPPORTED;
     skinny = true;
   }
-  if (!skinny_supported()) skinny = false;
   if (skinny) return MI355_W8A8_PATH_SKINNY;
-  if (skinny_supported() && !swiglu && skinny_chunked_pays(m, k, n) &&
+  if (!swiglu && skinny_chunked_pays(m, k, n) &&
       !(flags & (MI355_W8A8_FLAG_FORCE_TILED | MI355_W8A8_FLAG_TILE_256X128 | MI355_W8A8_FLAG_TILE_256X256 |
                  MI355_W8A8_FLAG_TILE_128X128 | MI355_W8A8_FLAG_TILE_256X128_PAIR)))
     return MI355_W8A8_PATH_SKINNY_CHUNKS;
@@ -503,7 +509,7 @@ int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
       if (p->aux_normalized)
         sub.aux_normalized = static_cast<unsigned char*>(p->aux_normalized) + (size_t)row0 * p->k * 2u;
       // the chunks share the workspace: they run one after the other on the stream
-      if ((st = launch_skinny(&sub, ws + w.xq, reinterpret_cast<float*>(ws + w.sx), ws + w.skinny, w.K_pad, w.KB, s)))
+      if ((st = launch_skinny(&sub, ws + w.xq, reinterpret_cast<float*>(ws + w.sx), ws + w.skinny, w.K_pad, w.KB, s, false)))
         return st;
     }
     return MI355_W8A8_OK;
@@ -2213,12 +2219,13 @@ int mi355_w8a8_quantize_rows_v1(const void* x_bf16, int8_t* codes, float* scales
 
 uint64_t mi355_w8a8_workspace_bytes(uint32_t m, uint32_t k, uint32_t n, uint32_t n_adapters, uint32_t rank,
                                     uint32_t flags) {
-  (void)flags;
   if (validate_common(m, k, n)) return 0;
   if (n_adapters > (uint32_t)kMaxAdapters || rank > (uint32_t)kMaxRank) return 0;
   // (sized for groups on block boundaries wherever a call of these dimensions may lay them out so)
+  const bool keep_b = (flags & (MI355_W8A8_FLAG_DECODE_B_WRITE | MI355_W8A8_FLAG_DECODE_B_KEPT)) && n_adapters &&
+                      skinny_b_can_be_kept(m, n, rank, (flags & MI355_W8A8_FLAG_SWIGLU) != 0);
   return make_layout(m, k, n, n_adapters, n_adapters ? rank : 0u, n_adapters > 1,
-                     padded_groups_fit(m, n, n_adapters) || padded_groups_fit(m, n, n_adapters, true)).total;
+                     padded_groups_fit(m, n, n_adapters) || padded_groups_fit(m, n, n_adapters, true), keep_b).total;
 }
 
 int mi355_w8a8_lora_linear_v1(const mi355_w8a8_problem* p, void* stream) {
@@ -2241,7 +2248,8 @@ int mi355_w8a8_forward_static_ws_v1(const mi355_w8a8_problem* p, void* stream) {
   if (st) return st;
   // Every caller in the process shares the array: what an earlier call left in it may be another layer's,
   // so a call must not be told to keep it.
-  if (p->flags & (MI355_W8A8_FLAG_LORA_PACK_VALID | MI355_W8A8_FLAG_SKIP_PROLOGUE)) return MI355_W8A8_ERR_UNSUPPORTED;
+  if (p->flags & (MI355_W8A8_FLAG_LORA_PACK_VALID | MI355_W8A8_FLAG_SKIP_PROLOGUE | MI355_W8A8_FLAG_DECODE_B_KEPT))
+    return MI355_W8A8_ERR_UNSUPPORTED;
   const uint64_t need = mi355_w8a8_workspace_bytes(p->m, p->k, p->n, p->n_adapters, p->rank, p->flags);
   if (need == 0 || need > MI355_W8A8_STATIC_WORKSPACE_BYTES) return MI355_W8A8_ERR_WORKSPACE;
   void* ws = static_workspace();

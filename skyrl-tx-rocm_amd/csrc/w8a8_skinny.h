@@ -1,6 +1,6 @@
 // Skinny-M (decode) path, M <= 32 rows: the weight is streamed exactly once from HBM.
 //   1. skinny_quant_kernel   one workgroup per row: (RMSNorm,) absmax, scale, int8 codes in
-//                            MFMA operand order.
+//                            MFMA operand order; where a loop asks for it, B regrouped for the stream kernel.
 //                            LoRA-A units ride along: z_part[chunk][m][:] = x[m, chunk] @
 //                            A[idx[m]][chunk, :] in float32 (with RMSNorm every unit forms the row's
 //                            inverse RMS for itself: a few KiB from the L2 against a launch of its own).
@@ -22,12 +22,28 @@ constexpr int kSkinnyMaxRows = 32;
 constexpr uint32_t kSkinnyMaxZChunks = 16;
 constexpr uint32_t kSkinnyZChunkK = 1024;  // K elements per LoRA-A work unit (per row)
 
+// Ranks of a row of the regrouped B (skinny_regroup_b): 1 KiB holds whole rows.
+__host__ __device__ inline uint32_t skinny_b_ranks(uint32_t r) { return r <= 16u ? 16u : 32u; }
+// Two slices of 16 columns to a workgroup, or one: slices of 16 columns while 32-column units would leave CUs idle
+// (fewer than 512 units: two workgroups share a CU); SwiGLU and residual decide for themselves (a gate/up
+// pair is two slices; the residual's dword gather serves one column).
+inline bool skinny_pairs(uint32_t n, bool swiglu, bool residual) {
+  return swiglu || (!residual && (n & 1u) == 0 && n_padded(n) / 128u * 4u >= 512u);
+}
+// Calls that can keep B regrouped: one slice, one row half, whole column quads, and values enough.  Per call of a loop, B
+// gathered / regrouped: 12288 x 4096, 16 rows of rank 32 20.4 / 18.9 us, 8 rows 17.9 / 17.3; 2560 x 6144, 16 rows of
+// rank 32 16.2 / 13.8; with 4 rows of rank 16 or one row level (10.8 / 11.0, 11.5 / 11.9).
+inline bool skinny_b_can_be_kept(uint32_t m, uint32_t n, uint32_t r, bool swiglu) {
+  return !swiglu && m <= 16u && r <= 32u && m * r >= 256u && (n & 3u) == 0;
+}
+
 struct SkinnyLayout {
-  uint64_t z_part, row_scaling, total;
+  uint64_t z_part, row_scaling, bsel, total;
   uint32_t pairs_per_wave, z_chunks, z_chunk_k;
 };
 
-inline SkinnyLayout skinny_layout(uint32_t k) {
+// keep_b: with the regrouped B of m rows of rank r
+inline SkinnyLayout skinny_layout(uint32_t k, bool keep_b = false, uint32_t m = 0u, uint32_t n = 0u, uint32_t r = 0u) {
   SkinnyLayout L{};
   const uint32_t n_pairs = k_padded(k) / 64u;
   L.pairs_per_wave = (n_pairs + 7u) / 8u;
@@ -38,12 +54,10 @@ inline SkinnyLayout skinny_layout(uint32_t k) {
   L.z_chunk_k = zk;
   L.z_part = 0;
   L.row_scaling = (uint64_t)kSkinnyMaxZChunks * kSkinnyMaxRows * kMaxRank * 4u;
-  L.total = L.row_scaling + 256u;
+  L.bsel = L.row_scaling + 256u;
+  L.total = L.bsel + (keep_b ? (uint64_t)(n_padded(n) / 16u) * m * skinny_b_ranks(r) * 32u + 1024u : 0u);  // (whole KiBs are read)
   return L;
 }
-
-inline uint64_t skinny_workspace_bytes() { return skinny_layout(128u).total; }
-inline bool skinny_supported() { return true; }
 
 // ---------------------------------------------------------------------------------------
 struct SkinnyQuantArgs {
@@ -63,7 +77,33 @@ struct SkinnyQuantArgs {
   uint32_t n_adapters, r, z_chunks, z_chunk_k, n_z_units;
   const float* lora_scaling;  // f32 [n_adapters] or null
   float* row_scaling;      // f32 [32]: lora_scaling[idx[m]], written here for the stream kernel
+  // B regrouped for the stream kernel, by blocks behind the LoRA-A units (sixteen items of a row and 128 columns each)
+  const uint16_t* lora_b;  // bf16 [n_adapters, r, N]
+  uint16_t* bsel;          // or null
+  uint32_t N, n_groups;    // n_groups = N_pad / 128
 };
+
+// B of row m's adapter in the order in which the stream kernel's units of 16 columns read it, 128 columns of it:
+// bsel[8 G + u][m][p][c][t] = B[idx[m]][2 t + p][128 G + 4 (16 (u & 1) + c) + u / 2], zeros beyond the rank.  A wave; two
+// ranks at a time.
+__device__ inline void skinny_regroup_b(const SkinnyQuantArgs& a, uint32_t item) {
+  const uint32_t lane = threadIdx.x & 63u, m = item / a.n_groups, G = item % a.n_groups;
+  if (m >= a.M) return;
+  int ad = a.idx ? a.idx[m] : 0;
+  ad = ad < 0 ? 0 : (ad >= (int)a.n_adapters ? (int)a.n_adapters - 1 : ad);
+  const uint32_t quad = lane & 31u, p = lane >> 5, col = 128u * G + 4u * quad, ranks = skinny_b_ranks(a.r);
+  const uint16_t* src = a.lora_b + (size_t)ad * a.r * a.N + (col < a.N ? col : 0u);
+  uint16_t* dst = a.bsel + (((size_t)(8u * G + (quad >> 4)) * a.M + m) * 2u + p) * (8u * ranks) + (quad & 15u) * (ranks / 2u);
+  const size_t next = (size_t)2u * a.M * ranks * 16u;  // the next column of the quad: two units on
+#pragma unroll 4
+  for (uint32_t t = 0; t < ranks / 2u; ++t) {
+    const uint32_t r = 2u * t + p;
+    uint2 v = *reinterpret_cast<const uint2*>(src + (size_t)(r < a.r ? r : 0u) * a.N);
+    if (r >= a.r) v = make_uint2(0u, 0u);
+    dst[t] = (uint16_t)v.x; dst[next + t] = (uint16_t)(v.x >> 16);
+    dst[2u * next + t] = (uint16_t)v.y; dst[3u * next + t] = (uint16_t)(v.y >> 16);
+  }
+}
 
 // Inverse RMS of row xr by a workgroup of 1024 threads (float64 sum, IEEE division and square root), the
 // same value in every workgroup that forms it: v holds the thread's 2 x 8 values of the row.
@@ -181,6 +221,10 @@ __global__ __launch_bounds__(1024) void skinny_quant_kernel(SkinnyQuantArgs a) {
   __shared__ float red_max[16];
   __shared__ double red_sum[16];
   __shared__ float zw[16][64];
+  if (blockIdx.x >= a.M + a.n_z_units) {
+    skinny_regroup_b(a, (blockIdx.x - a.M - a.n_z_units) * 16u + (threadIdx.x >> 6));
+    return;
+  }
   if (blockIdx.x >= a.M) {
     const uint32_t unit = blockIdx.x - a.M;
     float inv = 1.0f;
@@ -272,6 +316,7 @@ struct SkinnyStreamArgs {
   const float* sx;           // f32 [32]
   const float* sw;           // f32 [N]
   const uint16_t* lora_b;    // bf16 [n_adapters, r, N] or null
+  const uint16_t* bsel;      // B regrouped (skinny_regroup_b; NS = 1, RB = 1), or null: gathered from lora_b
   const float* row_scaling;  // f32 [32]: lora_scaling[idx[m]] (from the quantizer launch)
   const int32_t* idx;        // adapter per row or null
   const uint16_t* residual;  // bf16 [M, N] or null
@@ -288,11 +333,12 @@ struct SkinnyStreamArgs {
 struct SkinnyStreamLds { uint32_t z_off, tail_off, bytes; };
 constexpr uint32_t kSkinnyZlStride = 65;  // floats between two rows of z: four rows a wave reads at a time in four banks
 constexpr uint32_t kSkinnyTailBytes = 16u * kSkinnyZlStride * 4u + 5u * 2048u + 2u * 1024u + 64u;
-inline SkinnyStreamLds skinny_stream_lds(uint32_t m, uint32_t r, uint32_t z_chunks, uint32_t ns, uint32_t rb) {
+inline SkinnyStreamLds skinny_stream_lds(uint32_t m, uint32_t r, uint32_t z_chunks, uint32_t ns, uint32_t rb, bool kept_b) {
   SkinnyStreamLds L{};
   const uint32_t rows = m < 16u ? m : 16u, rpad = round_up(r, 4u);
   const uint32_t per_piece = r <= 32u ? 8u : 4u;  // rows of z per KiB
-  L.z_off = r ? round_up(rows * rpad * 64u + 4u * 64u, 1024u) : 0u;
+  const uint32_t b_bytes = kept_b ? round_up(rows * skinny_b_ranks(r) * 32u, 1024u) : rows * rpad * 64u;
+  L.z_off = r ? round_up(b_bytes + 4u * 64u, 1024u) : 0u;
   const uint32_t staged = L.z_off + (r ? z_chunks * ((rows + per_piece - 1u) / per_piece) * 1024u : 0u);
   const uint32_t red = kSkinnyStreamWaves * ns * rb * 1024u;
   L.tail_off = staged > red ? staged : red;
@@ -320,11 +366,12 @@ inline SkinnyStreamLds skinny_stream_lds(uint32_t m, uint32_t r, uint32_t z_chun
 // in order), and form the low-rank term from there while the weight is on its way.  B is gathered as dwords
 // (64 per instruction: four ranks x sixteen columns) straight from its [rank, N] rows: half or all of every
 // 64 bytes fetched is used, and no regrouped copy of it is written and read back, which cost 2 x 25 MB for
-// sixteen adapters of a 24576-wide projection whenever an adapter had changed.
+// sixteen adapters of a 24576-wide projection whenever an adapter had changed.  A loop that keeps its adapters has B
+// regrouped once (skinny_regroup_b) and then finds a unit's in whole KiBs.
 // Measured: 4096 x 24576 with SwiGLU, 16 rows, 16 adapters of rank 32: 22.9 us for 126 MB (5.5 TB/s), the whole
 // call 29 us against 139 us on 128 x 128 tiles behind the tiled quantizer (which such a call took before);
 // 2560 x 6144, one row, rank 64: 8.1 us against 18.3 us with B's loads behind the weight's; 12288 x 4096,
-// 16 rows: 14.1 us (12.6 us from a regrouped B already in memory, 15.2 us with the regrouping).
+// 16 rows: 14.6 us, 13.0 us from the regrouped B.
 // Rows 16..31 (RB = 2) share the weight operands; their B is staged in a second step behind the stream.
 template <int NS, int RB, int KP>
 __global__ __launch_bounds__(kSkinnyStreamThreads, (NS + RB) * KP <= 24 ? 4 : 2)
@@ -383,6 +430,7 @@ void skinny_stream_kernel(SkinnyStreamArgs a) {
     return f;
   };
   const bool lora = a.lora_b != nullptr;
+  const bool kept_b = NS == 1 && RB == 1 && a.bsel != nullptr;  // kernel-uniform
   // an odd number of values in B: the dword gathers would read two bytes behind it (NS = 2: N is even)
   const bool odd_b = NS == 1 && (a.n_adapters & a.r & a.N & 1u);
   const uint32_t rpad = (a.r + 3u) & ~3u;
@@ -409,6 +457,12 @@ void skinny_stream_kernel(SkinnyStreamArgs a) {
   // B rows and z partials of rows 16 hf .. 16 hf + 15 on their way into the LDS
   auto stage_half = [&](uint32_t hf) {
     const uint32_t rows = a.M - 16u * hf < 16u ? a.M - 16u * hf : 16u;
+    if (kept_b) {  // 1 KiB at a time, whole rows of one row quad (the quads 64 bytes apart: bank groups of their own)
+      const uint32_t row_bytes = skinny_b_ranks(a.r) * 32u, pieces = (rows * row_bytes + 1023u) / 1024u, quad_bytes = 4u * row_bytes;
+      const unsigned char* src = reinterpret_cast<const unsigned char*>(a.bsel) + (size_t)(grp * 8u + unit) * a.M * row_bytes;
+      for (uint32_t i = wave; i < pieces; i += kSkinnyStreamWaves)
+        lds_load_1k(src, i * 1024u + lane * 16u, lds0 + i * 1024u + (i * 1024u / quad_bytes) * 64u);
+    } else
 #pragma unroll
     for (uint32_t mi = 0; mi < 2u; ++mi) {
       const uint32_t m = wave + 8u * mi;
@@ -468,6 +522,15 @@ void skinny_stream_kernel(SkinnyStreamArgs a) {
       const float* zr = zl + f.frow16 * kSkinnyZlStride;
       const uint32_t odd_row = NS == 1 ? odd_base[f.frow16] : 0u;
       const uint32_t r0 = RB == 2 ? 0u : f.t8, step = RB == 2 ? 1u : 2u;
+      if (kept_b) {
+        const uint32_t ranks = skinny_b_ranks(a.r);
+        const uint16_t* bk = reinterpret_cast<const uint16_t*>(sk_lds) + f.frow16 * ranks * 16u + (f.frow16 >> 2) * 32u + (f.t8 * 16u + f.c16) * (ranks / 2u);
+        for (uint32_t t0 = 0; t0 < ranks / 2u; t0 += 8u) {  // (z and B are zeros beyond the rank: they add nothing)
+          const v8us b8 = *reinterpret_cast<const v8us*>(bk + t0);
+#pragma unroll
+          for (uint32_t e = 0; e < 8u; ++e) low[0] = fmaf(zr[2u * (t0 + e) + f.t8], bf16_bits_to_f32(b8[e]), low[0]);
+        }
+      } else
 #pragma unroll 2
       for (uint32_t r = r0; r < a.r; r += step) {
         const uint32_t w = bl[r * 16u];

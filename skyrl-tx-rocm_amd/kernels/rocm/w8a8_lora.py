@@ -280,7 +280,7 @@ class ForwardPlan:
                  adapter_indices: torch.Tensor | None = None, rms_gamma: torch.Tensor | None = None,
                  eps: float = 1e-6, residual: torch.Tensor | None = None, swiglu: bool = False,
                  flags: int = 0, return_aux: bool = False, entry: str = "forward",
-                 want_normalized: bool = False):
+                 want_normalized: bool = False, keep_lora_pack: bool = True):
         if x.dtype != torch.bfloat16:
             raise TypeError(f"x must be BF16, got {x.dtype}")
         if x.ndim < 2 or math.prod(x.shape[:-1]) <= 0:
@@ -327,7 +327,8 @@ class ForwardPlan:
         if swiglu:
             flags |= _native.FLAG_SWIGLU
         out = torch.empty((m, n_out), dtype=torch.bfloat16, device=dev)
-        ws_bytes = int(lib.mi355_w8a8_workspace_bytes(m, k, n, n_ad, r, flags))
+        # (room for B regrouped where a decode loop may keep it: see run)
+        ws_bytes = int(lib.mi355_w8a8_workspace_bytes(m, k, n, n_ad, r, flags | (_native.FLAG_DECODE_B_WRITE if keep_lora_pack else 0)))
         if ws_bytes == 0:
             raise ValueError(
                 f"geometry M={m}, K={k}, N={n}, rank={r}, adapters={n_ad} is outside the native path")
@@ -376,23 +377,26 @@ class ForwardPlan:
         self._keep = (flat, pw, a3, b3, s1, idx, gamma, res, ws)
         self._lora = (a3, b3) if n_ad else None
         self._packed_lora_key = None  # versions of A / B whose transposed / packed copies sit in the workspace
-        self.keep_lora_pack = True    # False: pack on every run (what a caller that rewrites A / B behind torch's back needs)
+        self._decode_b_key = None     # ... and of those whose B, regrouped for the decode kernels, does
+        self._decode_room = bool(keep_lora_pack)
+        self.keep_lora_pack = keep_lora_pack  # False: pack on every run (what a caller that rewrites A / B behind torch's back needs)
 
     def run(self, extra_flags: int = 0) -> torch.Tensor:
         """Enqueue the call on torch's current stream; returns the (reused) output tensor.
 
-        The transposed LoRA A and packed LoRA B (a decode-sized call keeps neither)
-        live in the plan's workspace: while neither tensor nor the adapter indices have been
-        written since the last full run (``Tensor._version``), the call is told to keep them
+        The transposed LoRA A and packed LoRA B live in the plan's workspace: while neither tensor nor the
+        adapter indices have been written since the last full run (``Tensor._version``), the call is told to keep them
         (``FLAG_LORA_PACK_VALID``) instead of packing 2 * n * r * (K + N) bytes again.  A training step
-        updates the adapters, so its forward packs once per step as before."""
+        updates the adapters, so its forward packs once per step as before.  A decode-sized call reads A and B as they are;
+        from the second run with the same adapters on it keeps B regrouped (``FLAG_DECODE_B_WRITE``, then
+        ``FLAG_DECODE_B_KEPT``)."""
         flags = self.flags | extra_flags
         key = None
         # (a captured call is replayed later, when the adapters may have changed: it always packs)
         capturing = self.keep_lora_pack and torch.cuda.is_current_stream_capturing()
         if self._lora is not None and not capturing and self.keep_lora_pack:
             # (what the workspace holds also depends on the path the flags choose: the decode kernels keep
-            # nothing, the tiled kernels A and B in operand order)
+            # B regrouped, the tiled kernels A and B in operand order)
             versions = (_version_of(self._lora[0]), _version_of(self._lora[1]),
                         0 if self.adapter_indices is None else _version_of(self.adapter_indices))
             if None not in versions:  # (a tensor torch keeps no version of may have been written: pack)
@@ -400,6 +404,8 @@ class ForwardPlan:
                                             _native.FLAG_LORA_PACK_VALID),)
             if key is not None and key == self._packed_lora_key:
                 flags |= _native.FLAG_LORA_PACK_VALID
+                if self._decode_room and not flags & _native.FLAG_SKIP_PROLOGUE:
+                    flags |= _native.FLAG_DECODE_B_KEPT if key == self._decode_b_key else _native.FLAG_DECODE_B_WRITE
         self.problem.flags = flags
         with _on(self.device):
             status = self._fn(ctypes.byref(self.problem), _stream_ptr(self.device))
@@ -407,6 +413,8 @@ class ForwardPlan:
         _native.check(f"mi355_w8a8_{self.entry}", status)
         if not extra_flags & _native.FLAG_SKIP_PROLOGUE and not capturing:
             self._packed_lora_key = key
+            if flags & _native.FLAG_DECODE_B_WRITE:
+                self._decode_b_key = key
         return self.out.reshape(self.out_shape)
 
 
@@ -417,8 +425,7 @@ def forward(x: torch.Tensor, weight, lora_a=None, lora_b=None, lora_scaling=None
     """One W8A8 forward through the C ABI.  Returns bf16 [..., n_out] (and aux tensors)."""
     plan = ForwardPlan(x, weight, lora_a, lora_b, lora_scaling, adapter_indices=adapter_indices,
                        rms_gamma=rms_gamma, eps=eps, residual=residual, swiglu=swiglu, flags=flags,
-                       return_aux=return_aux, entry=entry)
-    plan.keep_lora_pack = False  # (run once: nothing to compare versions with)
+                       return_aux=return_aux, entry=entry, keep_lora_pack=False)  # (run once: nothing to compare versions with)
     result = plan.run()
     # Everything the kernels touch was allocated for torch's current stream, the one they were
     # enqueued on, so the caching allocator orders any reuse after them.
