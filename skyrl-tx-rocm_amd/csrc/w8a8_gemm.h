@@ -67,14 +67,14 @@ struct EpilogueFromMemory {
   __device__ uint32_t range() const { return g.blk_range ? (uint32_t)g.blk_range[pbase / 32u] : 0u; }
   __device__ int slot_group(int c, int first) const { return g.slot_group ? g.slot_group[pbase + c] : first; }
   __device__ float scaling(int gi) const { return g.lora_scaling[gi]; }
+  // (Bases from which the operands lie at constant distances: an address of its own for each took registers that
+  // the accumulators need.)  z: operand (kk, term) at kk * 3 + term blocks
   template <int NKK>
-  __device__ v8us z(int kk, int term, int lane) const {
-    return *reinterpret_cast<const v8us*>(g.zp + ((size_t)(pbase / 32u) * NKK * 3u + kk * 3 + term) * kBlockBytes + lane * 16);
-  }
-  // operand of the wave's packed column block j: rows 16 kk + 8 h + 0..7 of column 4 c + j
+  __device__ const unsigned char* z(int lane) const { return g.zp + (size_t)(pbase / 32u) * NKK * 3u * kBlockBytes + lane * 16; }
+  // of the wave's packed column block j, operand kk (rows 16 kk + 8 h + 0..7 of column 4 c + j) at kk blocks, block j + 1 at NKK
   template <int NKK>
-  __device__ v8us b(int gi, int j, int kk, int lane) const {
-    return *reinterpret_cast<const v8us*>(g.bp + (((size_t)gi * ncb_total + tcol0 / 32u + j) * NKK + kk) * kBlockBytes + lane * 16);
+  __device__ const unsigned char* b(int gi, int j, int lane) const {
+    return g.bp + ((size_t)gi * ncb_total + tcol0 / 32u + j) * NKK * kBlockBytes + lane * 16;
   }
 };
 
@@ -133,14 +133,16 @@ __device__ inline __attribute__((always_inline)) void gemm_epilogue_block(const 
     // ---- section A: lowS[j][v] = s_g * (z @ B_g) for the column pair
     v16f lowS[2];
     if constexpr (kLora) {
+      const unsigned char* const zb = from.template z<NKK>(lane);
+      const unsigned char* const bb0 = from.template b<NKK>(gi, 2 * jp, lane);
 #pragma unroll
       for (int kk = 0; kk < NKK; ++kk) {
         v8us zf[3];
 #pragma unroll
-        for (int t3 = 0; t3 < 3; ++t3) zf[t3] = from.template z<NKK>(kk, t3, lane);
+        for (int t3 = 0; t3 < 3; ++t3) zf[t3] = *reinterpret_cast<const v8us*>(zb + (kk * 3 + t3) * kBlockBytes);
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-          const v8bf bb = __builtin_bit_cast(v8bf, from.template b<NKK>(gi, 2 * jp + j, kk, lane));
+          const v8bf bb = __builtin_bit_cast(v8bf, *reinterpret_cast<const v8us*>(bb0 + (j * NKK + kk) * kBlockBytes));
           v16f cur;
           if (kk == 0) {
 #pragma unroll

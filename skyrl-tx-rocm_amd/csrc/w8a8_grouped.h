@@ -51,9 +51,9 @@ struct EpilogueFromLds {
   __device__ int slot_group(int, int first) const { return first; }
   __device__ float scaling(int) const { return s; }
   template <int NKK>
-  __device__ v8us z(int, int term, int lane) const { return *reinterpret_cast<const v8us*>(zs + term * kBlockBytes + lane * 16); }
+  __device__ const unsigned char* z(int lane) const { return zs + lane * 16; }
   template <int NKK>
-  __device__ v8us b(int, int j, int, int lane) const { return *reinterpret_cast<const v8us*>(bs + j * kBlockBytes + lane * 16); }
+  __device__ const unsigned char* b(int, int j, int lane) const { return bs + j * kBlockBytes + lane * 16; }
 };
 
 template <int EPI, int NKK, int kRB>
