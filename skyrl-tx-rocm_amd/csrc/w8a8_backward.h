@@ -474,7 +474,10 @@ __device__ inline void bwd_dx_tile_at(const BwdDxArgs& g, uint32_t t, uint32_t& 
 // pbase: first slot of the block's 32; kbw: first of its k blocks.
 template <int NKK, int CBN>
 __device__ inline void bwd_dx_store_block(const BwdDxArgs& g, uint32_t pbase, uint32_t kbw, const v16f (&acc)[CBN]) {
-  const int lane = threadIdx.x & 63, c = lane & 31, h = lane >> 5;
+  int lane = threadIdx.x & 63;
+  // (opaque: what the epilogue derives from it is formed here and not held in registers through the stages)
+  asm volatile("" : "+v"(lane));
+  const int c = lane & 31, h = lane >> 5;
   const uint32_t blk = pbase / 32u;
   const int src_lane = g.src_row ? g.src_row[pbase + c] : (int)(pbase + c);
   const bool row_ok = src_lane >= 0 && src_lane < (int)g.M;
@@ -528,6 +531,12 @@ __device__ inline void bwd_dx_store_block(const BwdDxArgs& g, uint32_t pbase, ui
 // tile): a stage then holds half the dy panel and twice the weight blocks, the same bytes and the same
 // four loads per wave.  For grouped calls whose weights own few rows each: half the padding per weight,
 // and every wave has rows.
+//
+// The 256 registers that two waves per SIMD leave are the kernel's limit: the loads' addresses are a scalar base plus the
+// lane's offset (issue), and the epilogue derives its lane constants for itself (bwd_dx_store_block).  Held in vector
+// registers through the stages both cost 44 bytes of scratch per lane (16 with ROWS128).  Spilling / as it is, pull-back and
+// what goes before it: 2048 x 2560, N = 10240, rank 64 211 / 205 us; 512 x 2560, N = 6144 78.0 / 74.9; 4096 x 4096,
+// N = 24576 947 / 946 (whole tiles: the reloads stand outside the stages); 8168 rows of 128 experts, 2048 <- 1536 207 / 204.
 template <int NKK, bool ROWS128 = false>
 __global__ __launch_bounds__(512, 1) void bwd_dx_kernel(BwdDxArgs g) {
   constexpr int kRowBlocks = ROWS128 ? 4 : 8, kKBlocks = ROWS128 ? 16 : 8;  // of a tile
@@ -539,6 +548,7 @@ __global__ __launch_bounds__(512, 1) void bwd_dx_kernel(BwdDxArgs g) {
   const int wrow = ROWS128 ? 0 : wave >> 2, wcol = ROWS128 ? wave : wave & 3;
   const int c = lane & 31, h = lane >> 5;
   const int NBi = (int)g.NB;  // a multiple of 8
+  const uint32_t lane16 = (uint32_t)lane * 16u;
 
   // identity operand of the transposing MFMA: lane (column c, k half h) holds byte 1 at k == c
   v4i ident = {0, 0, 0, 0};
@@ -574,32 +584,32 @@ __global__ __launch_bounds__(512, 1) void bwd_dx_kernel(BwdDxArgs g) {
 
     // this wave's two panel chunks of a stage (row block = wave, halves q = 0, 1) and its weight block
     const unsigned char* Ag = g.dyp + ((size_t)(tm * (uint32_t)kRowBlocks + load_rb) * g.NB) * 2048u +
-                              (ROWS128 ? (wave & 1) * 1024 : 0) + lane * 16;
+                              (ROWS128 ? (wave & 1) * 1024 : 0);
     const uint32_t kbw = tk * (uint32_t)kKBlocks + (uint32_t)wcol * 2u;  // first of the two k blocks this wave multiplies
     // the block(s) it loads: one of eight, or its own two of sixteen; blocks past the weight repeat the last
     const uint32_t kbl0 = tk * (uint32_t)kKBlocks + (ROWS128 ? 2u * (uint32_t)wave : (uint32_t)wave);
     const uint32_t kbl = kbl0 < g.KB ? kbl0 : g.KB - 1u;
     const uint32_t kbl1 = kbl0 + 1u < g.KB ? kbl0 + 1u : g.KB - 1u;
-    const unsigned char* Bg = g.wp + (size_t)tw * g.w_stride + (size_t)kbl * kBlockBytes + lane * 16;
-    const unsigned char* Bg1 = g.wp + (size_t)tw * g.w_stride + (size_t)kbl1 * kBlockBytes + lane * 16;
+    const unsigned char* Bg = g.wp + (size_t)tw * g.w_stride + (size_t)kbl * kBlockBytes;
+    const unsigned char* Bg1 = g.wp + (size_t)tw * g.w_stride + (size_t)kbl1 * kBlockBytes;
     const size_t nb_stride = (size_t)g.KB * kBlockBytes;
 
     auto issue = [&](int i) {  // stage i of the segment
       unsigned char* St = lds + (i % kBwdStages) * kBwdStageBytes;
       const int nb = nb0 + i;
-      const unsigned char* src = Ag + (size_t)nb * 2048u;
+      const unsigned char* src = Ag + (size_t)nb * 2048u + lane16;
       if constexpr (ROWS128) {
         load_1k_to_lds(src, St + wave * kBlockBytes);
         // (few rows per weight: most of its bytes are read by one workgroup only)
-        load_1k_to_lds_once(Bg + (size_t)nb * nb_stride, St + kPanel + (wave * 2) * kBlockBytes);
-        load_1k_to_lds_once(Bg1 + (size_t)nb * nb_stride, St + kPanel + (wave * 2 + 1) * kBlockBytes);
+        load_1k_to_lds_once(Bg + (size_t)nb * nb_stride + lane16, St + kPanel + (wave * 2) * kBlockBytes);
+        load_1k_to_lds_once(Bg1 + (size_t)nb * nb_stride + lane16, St + kPanel + (wave * 2 + 1) * kBlockBytes);
       } else {
         load_1k_to_lds(src, St + (wave * 2) * kBlockBytes);
         load_1k_to_lds(src + 1024, St + (wave * 2 + 1) * kBlockBytes);
-        load_1k_to_lds(Bg + (size_t)nb * nb_stride, St + kPanel + wave * kBlockBytes);
+        load_1k_to_lds(Bg + (size_t)nb * nb_stride + lane16, St + kPanel + wave * kBlockBytes);
       }
       // every wave fetches the same 1 KiB of scales (the stage's 32 lead it) to the same place
-      load_1k_to_lds(reinterpret_cast<const unsigned char*>(swp_t + 32 * nb) + lane * 16, St + kPanel + kWeight);
+      load_1k_to_lds(reinterpret_cast<const unsigned char*>(swp_t + 32 * nb) + lane16, St + kPanel + kWeight);
     };
 
     v16f acc[4][2];
