@@ -101,8 +101,8 @@ typedef enum mi355_w8a8_status {
 /* Calls of at most 16 rows, rank at most 32, m * rank at least 256, n a multiple of 4, without SwiGLU: B regrouped per row and adapter in the
  * workspace (a loop over the same batch reads it faster than B itself).  WRITE: this call regroups B and uses it.  KEPT: the
  * workspace holds what a call with WRITE left there, for the same m, k, n, n_adapters and rank and the same contents
- * of lora_b and adapter_indices, and no other call has used the workspace with other dimensions since; the
- * caller vouches for it.  Pass the flag to the workspace query.  Other calls ignore both. */
+ * of lora_b and adapter_indices, and no call of other dimensions, or with MI355_W8A8_FLAG_FORCE_TILED, has used the
+ * workspace since; the caller vouches for it.  Pass the flag to the workspace query.  Other calls ignore both. */
 #define MI355_W8A8_FLAG_DECODE_B_WRITE 8192u
 #define MI355_W8A8_FLAG_DECODE_B_KEPT 16384u
 

@@ -413,8 +413,8 @@ class ForwardPlan:
         _native.check(f"mi355_w8a8_{self.entry}", status)
         if not extra_flags & _native.FLAG_SKIP_PROLOGUE and not capturing:
             self._packed_lora_key = key
-            if flags & _native.FLAG_DECODE_B_WRITE:
-                self._decode_b_key = key
+            # (a run by another path lays the workspace out in another way and may write over it)
+            self._decode_b_key = key if flags & (_native.FLAG_DECODE_B_WRITE | _native.FLAG_DECODE_B_KEPT) else None
         return self.out.reshape(self.out_shape)
 
 

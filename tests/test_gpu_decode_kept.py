@@ -43,6 +43,22 @@ def test_kept_b(m, k, n, n_ad, rank, form):
     runs(dict(case, idx=idx, b=case["b"] * np.float32(-0.5)))
 
 
+def test_a_run_by_the_tiled_path_between():
+    """Sixteen adapters on block boundaries: the tiled path's codes then reach over the place of the regrouped B."""
+    import torch
+
+    p = load_package()
+    case = wc.make_case(16, 1024, 4096, n_adapters=16, rank=32, seed=5, residual=False)
+    case["idx"] = np.arange(16, dtype=np.int32)
+    t = wc.to_torch(case, "cuda:0")
+    plan = p.w8a8_lora.ForwardPlan(t["x"], t["weight"], t["a"], t["b"], t["s"], adapter_indices=t["idx"])
+    print("[case] kept B, tiled run between", flush=True)
+    want = [plan.run().clone() for _ in range(3)]
+    plan.run(p._native.FLAG_FORCE_TILED)
+    got = [plan.run().clone() for _ in range(3)]
+    assert all(torch.equal(want[0].view(torch.int16), g.view(torch.int16)) for g in want[1:] + got)
+
+
 def test_one_run_reserves_no_room():
     native = load_package()._native
     size = native.load().mi355_w8a8_workspace_bytes
