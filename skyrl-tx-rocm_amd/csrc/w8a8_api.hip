@@ -57,7 +57,7 @@ constexpr uint32_t kMaxN = 1u << 20;
 inline uint64_t align256(uint64_t v) { return (v + 255u) & ~uint64_t(255); }
 
 struct WsLayout {
-  uint64_t xq, sx, zp, at, bp, row_scale, row_inv, src_row, dst_pos, slot_group, blk_range, tile_ctr, skinny, total;
+  uint64_t xq, sx, zp, at, bp, row_scale, row_inv, src_row, slot_group, blk_range, tile_ctr, skinny, total;
   uint32_t slots, nkk, K_pad, KB, n_steps, steps_per_wave;
   uint32_t rows_bound;  // the slots that can hold rows (a multiple of 32)
 };
@@ -122,7 +122,6 @@ WsLayout make_layout(uint32_t m, uint32_t k, uint32_t n, uint32_t n_groups, uint
   w.row_scale = off; off += align256((uint64_t)m * 4u);
   w.row_inv = off; off += align256((uint64_t)m * 4u);
   w.src_row = off; off += align256((uint64_t)w.slots * 4u);
-  w.dst_pos = off; off += align256((uint64_t)m * 4u);
   w.slot_group = off; off += align256((uint64_t)w.slots * 4u);
   w.blk_range = off; off += align256((uint64_t)(w.slots / 32u) * 4u);
   w.tile_ctr = off; off += 1024u;  // two sets of eight counters, 64 bytes apart
@@ -141,13 +140,12 @@ inline bool overlaps(const void* a, uint64_t an, const void* b, uint64_t bn) {
 
 inline int launch_status() { return hipGetLastError() == hipSuccess ? MI355_W8A8_OK : MI355_W8A8_ERR_LAUNCH; }
 
-template <bool RMS>
 int launch_quant(const QuantArgs& a, hipStream_t s) {
-  const uint32_t need = (a.K_pad + 511u) / 512u;
+  const uint32_t need = (a.K + 511u) / 512u;
   const dim3 grid((a.M + 3u) / 4u), block(256);
 #define W8A8_Q(NCH)                                                              \
   if (need <= NCH) {                                                             \
-    hipLaunchKernelGGL((quant_rows_kernel<NCH, RMS>), grid, block, 0, s, a);     \
+    hipLaunchKernelGGL((quant_rows_kernel<NCH>), grid, block, 0, s, a);          \
     return launch_status();                                                      \
   }
   W8A8_Q(1) W8A8_Q(2) W8A8_Q(4) W8A8_Q(8) W8A8_Q(16) W8A8_Q(24) W8A8_Q(32)
@@ -155,7 +153,7 @@ int launch_quant(const QuantArgs& a, hipStream_t s) {
   return MI355_W8A8_ERR_UNSUPPORTED;
 }
 
-// LoRA-A projection on the transposed A.  Up to 32 ranks the operands travel through LDS in whole
+// LoRA-A projection.  Up to 32 ranks (nkk: 16-wide rank chunks) the operands travel through LDS in whole
 // cache lines (the staged form of the kernel); beyond, two rank blocks per wave leave no room for that.
 int launch_lora_a(const LoraAArgs& la, uint32_t nkk, dim3 grid, hipStream_t s) {
   if (nkk > 2u) {
@@ -481,7 +479,6 @@ int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
   const WsLayout w = make_layout(p->m, p->k, p->n, p->n_adapters, lora ? p->rank : 0u, routed, pad_groups);
   unsigned char* ws = static_cast<unsigned char*>(p->workspace);
   int32_t* src_row = reinterpret_cast<int32_t*>(ws + w.src_row);
-  int32_t* dst_pos = reinterpret_cast<int32_t*>(ws + w.dst_pos);
   int32_t* slot_group = reinterpret_cast<int32_t*>(ws + w.slot_group);
   int32_t* blk_range = reinterpret_cast<int32_t*>(ws + w.blk_range);
 
@@ -527,7 +524,7 @@ int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
   if (!skip_prologue && (route_blocks || stat_blocks || pack)) {
     LoraPrepArgs pa{};
     pa.idx = routed ? p->adapter_indices : nullptr;
-    pa.src_row = src_row; pa.dst_pos = dst_pos; pa.slot_group = slot_group; pa.blk_range = blk_range;
+    pa.src_row = src_row; pa.slot_group = slot_group; pa.blk_range = blk_range;
     pa.lora_a = static_cast<const uint16_t*>(p->lora_a);
     pa.lora_b = static_cast<const uint16_t*>(p->lora_b);
     pa.at = reinterpret_cast<uint16_t*>(ws + w.at);
@@ -644,7 +641,7 @@ int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
     ga.residual = nullptr;
     if ((st = wide ? launch_gemm16_one<kEpiAcc, 0>(ga, s)
                    : (pair ? launch_gemm16_one<kEpiAcc, 0, 2>(ga, s)
-                           : (small ? launch_gemm<kEpiAcc, kModeDense128>(ga, 0u, s) : launch_gemm<kEpiAcc>(ga, 0u, s)))))
+                           : (small ? launch_gemm_one<kEpiAcc, 0, kModeDense128>(ga, s) : launch_gemm_one<kEpiAcc, 0, kModeDense>(ga, s)))))
       return st;
     g.tile_ctr += 128;  // the second counter set
   }
@@ -656,7 +653,7 @@ int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
 }
 
 struct GroupedLayout {
-  uint64_t xq, sx, zp, at, bp, row_scale, src_row, dst_pos, blk_range, tile_tab, total;
+  uint64_t xq, sx, zp, at, bp, row_scale, src_row, blk_range, tile_tab, total;
   uint32_t slots, nkk, K_pad, KB, tile_blocks, max_tiles;
 };
 
@@ -693,7 +690,6 @@ GroupedLayout make_grouped_layout(uint32_t m, uint32_t k, uint32_t n, uint32_t n
   w.sx = off; off += align256((uint64_t)w.slots * 4u);
   w.row_scale = off; off += align256((uint64_t)m * 4u);
   w.src_row = off; off += align256((uint64_t)w.slots * 4u);
-  w.dst_pos = off; off += align256((uint64_t)m * 4u);
   w.blk_range = off; off += align256((uint64_t)(w.slots / 32u) * 4u);
   w.tile_tab = off; off += align256(((uint64_t)w.max_tiles + 1u) * 8u);
   w.zp = off; off += rank ? align256((uint64_t)(w.slots / 32u) * w.nkk * 3u * kBlockBytes) : 0u;
@@ -759,7 +755,6 @@ int run_grouped(const mi355_w8a8_grouped_problem* p, hipStream_t s) {
   if (reinterpret_cast<uintptr_t>(p->workspace) & 255u) return MI355_W8A8_ERR_ALIGN;
   unsigned char* ws = static_cast<unsigned char*>(p->workspace);
   int32_t* src_row = reinterpret_cast<int32_t*>(ws + w.src_row);
-  int32_t* dst_pos = reinterpret_cast<int32_t*>(ws + w.dst_pos);
   int32_t* blk_range = reinterpret_cast<int32_t*>(ws + w.blk_range);
   (void)hipGetLastError();
 
@@ -774,7 +769,7 @@ int run_grouped(const mi355_w8a8_grouped_problem* p, hipStream_t s) {
   const bool by_source = p->x_row_map && x_rows <= p->m;
   if (!skip_prologue) {
     LoraPrepArgs pa{};
-    pa.src_row = src_row; pa.dst_pos = dst_pos; pa.blk_range = blk_range;
+    pa.src_row = src_row; pa.blk_range = blk_range;
     pa.group_sizes = p->group_sizes;
     pa.tile_tab = reinterpret_cast<uint64_t*>(ws + w.tile_tab); pa.tile_blocks = w.tile_blocks;
     pa.zero_out = static_cast<uint16_t*>(p->out); pa.zero_cols = n_out;
@@ -824,11 +819,11 @@ int run_grouped(const mi355_w8a8_grouped_problem* p, hipStream_t s) {
     if (p->aux_x_codes || p->aux_x_scales) {  // the caller's copies: of every row (some have no slot), then what the GEMM reads
       QuantArgs c{};
       c.x = static_cast<const uint16_t*>(p->x);
-      c.M = p->m; c.K = p->k; c.K_pad = w.K_pad; c.KB = w.KB;
+      c.M = p->m; c.K = p->k;
       c.codes_rm = p->aux_x_codes;
       c.scales_rm = p->aux_x_scales;
       c.row_map = p->x_row_map; c.row_div = x_repeat; c.row_limit = x_rows;
-      if ((st = launch_quant<false>(c, s))) return st;
+      if ((st = launch_quant(c, s))) return st;
       hipLaunchKernelGGL(codes_row_major_kernel, dim3(w.slots), dim3(256), 0, s, q.xq_packed, q.sx_slots, src_row,
                          p->aux_x_codes, p->aux_x_scales, p->m, p->k, w.KB);
       if ((st = launch_status())) return st;
@@ -861,7 +856,7 @@ int run_grouped(const mi355_w8a8_grouped_problem* p, hipStream_t s) {
   if (p->aux_acc) {
     GemmArgs ga = g;
     ga.out = p->aux_acc;
-    if ((st = tall ? launch_grouped<kEpiAcc, 8>(ga, 0u, s) : launch_grouped<kEpiAcc, 4>(ga, 0u, s))) return st;
+    if ((st = tall ? launch_grouped_one<kEpiAcc, 0, 8>(ga, s) : launch_grouped_one<kEpiAcc, 0, 4>(ga, s))) return st;
   }
   if (tall) return swiglu ? launch_grouped<kEpiSwiglu, 8>(g, w.nkk, s) : launch_grouped<kEpiPlain, 8>(g, w.nkk, s);
   return swiglu ? launch_grouped<kEpiSwiglu, 4>(g, w.nkk, s) : launch_grouped<kEpiPlain, 4>(g, w.nkk, s);
@@ -902,7 +897,7 @@ BwdDxSplit bwd_dx_split(uint32_t tiles_m, uint32_t tiles_k, uint32_t NB, uint32_
 struct BwdLayout {
   BwdDxSplit split;
   uint64_t part;
-  uint64_t dyp, swp, at, ap, rp, z, r_raw, rs, rpart, src_row, dst_pos, slot_group, blk_range, group_off, partA, partB, total;
+  uint64_t dyp, swp, at, ap, rp, z, r_raw, rs, rpart, src_row, slot_group, blk_range, group_off, partA, partB, total;
   uint64_t beyond;  // group-scaled calls
   uint32_t part_blocks;
   uint32_t slots, nkk, K_pad, KB, N_pad, NB, tiles_m, tiles_k, max_chunks, R, n_slices, groups_per_slice;
@@ -937,7 +932,6 @@ BwdLayout make_bwd_layout(uint32_t m, uint32_t k, uint32_t n, uint32_t n_groups,
   w.dyp = off; off += align256((uint64_t)w.slots * w.N_pad * 2u);
   w.swp = off; off += align256((uint64_t)(w.N_pad + kBwdScalePad) * 4u);  // a stage fetches 1 KiB of scales starting at its own 32
   w.src_row = off; off += align256((uint64_t)w.slots * 4u);
-  w.dst_pos = off; off += align256((uint64_t)m * 4u);
   w.slot_group = off; off += align256((uint64_t)w.slots * 4u);
   w.blk_range = off; off += align256((uint64_t)(w.slots / 32u) * 4u);
   w.group_off = off; off += align256((uint64_t)(kMaxAdapters + 1) * 4u);
@@ -1076,10 +1070,8 @@ int launch_bwd_body(const BwdBody& b, const Layout& w, unsigned char* ws, hipStr
       lz.xsrc = static_cast<const uint16_t*>(b.x);
       lz.at = reinterpret_cast<const uint16_t*>(ws + w.at);
       lz.src_row = b.src_row; lz.slot_group = b.slot_group; lz.blk_range = b.blk_range;
-      lz.zp = nullptr;
-      lz.M = b.m; lz.K = b.k; lz.r = b.rank; lz.nkk = w.nkk;
+      lz.M = b.m; lz.K = b.k; lz.r = b.rank;
       lz.n_steps = (b.k + 63u) / 64u;
-      lz.nterms = 3u;
       lz.n_blocks = w.slots / 32u;
       // K is cut into slices so that a call of few row blocks still fills the chip; the slices land
       // in the partial table (r's partials have been consumed, it holds n_slices of them) and are
@@ -1093,8 +1085,7 @@ int launch_bwd_body(const BwdBody& b, const Layout& w, unsigned char* ws, hipStr
       lz.zf = reinterpret_cast<float*>(ws + w.rpart);
       lz.zf_stride = kBwdRankStride;
       lz.zf_slice = w.slots * kBwdRankStride;
-      const dim3 grid(lz.n_blocks * nks), block(1024);
-      (void)block;
+      const dim3 grid(lz.n_blocks * nks);
       if ((st = launch_lora_a(lz, w.nkk, grid, s))) return st;
       BwdRFinishArgs f{};
       f.rpart = reinterpret_cast<const float*>(ws + w.rpart);
@@ -1244,7 +1235,7 @@ int run_backward(const mi355_w8a8_bwd_problem* p, hipStream_t s) {
   if (!skip_prologue) {  // tables: routing, A transposed / in operand order, scales in packed column order
     BwdPrepArgs pa{};
     pa.idx = routed ? p->adapter_indices : nullptr;
-    pa.src_row = src_row; pa.dst_pos = reinterpret_cast<int32_t*>(ws + w.dst_pos);
+    pa.src_row = src_row;
     pa.slot_group = slot_group; pa.blk_range = blk_range; pa.group_off = group_off;
     pa.lora_a = static_cast<const uint16_t*>(p->lora_a);
     pa.at = lora ? reinterpret_cast<uint16_t*>(ws + w.at) : nullptr;
@@ -1343,7 +1334,7 @@ int run_gq_backward(const mi355_w8a8_gq_bwd_problem* p, hipStream_t s) {
 // grouped (per-expert) backward
 // ---------------------------------------------------------------------------------------
 struct BwdGroupedLayout {
-  uint64_t dyp, swp, src_row, dst_pos, slot_group, blk_range, group_beg, group_end, tile_weight, chunk_tab, chunk0,
+  uint64_t dyp, swp, src_row, slot_group, blk_range, group_beg, group_end, tile_weight, chunk_tab, chunk0,
       at, ap, rp, z, r_raw, rs, rpart, partA, partB, total;
   uint32_t slots, nkk, K_pad, KB, N_pad, NB, tiles_m, tiles_k, max_chunks, R, n_slices, groups_per_slice, n_weights,
       gpw, sw_stride, tile_rows;
@@ -1383,7 +1374,6 @@ BwdGroupedLayout make_bwd_grouped_layout(uint32_t m, uint32_t k, uint32_t n, uin
   w.dyp = off; off += align256((uint64_t)w.slots * w.N_pad * 2u);
   w.swp = off; off += align256((uint64_t)w.n_weights * w.sw_stride * 4u);
   w.src_row = off; off += align256((uint64_t)w.slots * 4u);
-  w.dst_pos = off; off += align256((uint64_t)m * 4u);
   w.slot_group = off; off += align256((uint64_t)w.slots * 4u);
   w.blk_range = off; off += align256((uint64_t)(w.slots / 32u) * 4u);
   w.group_beg = off; off += align256((uint64_t)n_groups * 4u);
@@ -1454,7 +1444,6 @@ int run_grouped_backward(const mi355_w8a8_grouped_bwd_problem* p, hipStream_t s)
   unsigned char* ws = static_cast<unsigned char*>(p->workspace);
   BwdGroupTables tab{};
   tab.src_row = reinterpret_cast<int32_t*>(ws + w.src_row);
-  tab.dst_pos = reinterpret_cast<int32_t*>(ws + w.dst_pos);
   tab.slot_group = reinterpret_cast<int32_t*>(ws + w.slot_group);
   tab.blk_range = reinterpret_cast<int32_t*>(ws + w.blk_range);
   tab.group_beg = reinterpret_cast<int32_t*>(ws + w.group_beg);
@@ -2046,19 +2035,16 @@ int run_gq_linear(const mi355_w8a8_gq_problem* p, hipStream_t s) {
     la.src_row = routed ? src_row : nullptr;
     la.slot_group = routed ? slot_group : nullptr;
     la.blk_range = routed ? blk_range : nullptr;
-    la.zp = nullptr;
     la.zf = reinterpret_cast<float*>(ws + L.z);
     la.zf_stride = 64u;
-    la.M = p->m; la.K = p->k; la.r = p->rank; la.nkk = rank_chunks(p->rank);
+    la.M = p->m; la.K = p->k; la.r = p->rank;
     const uint32_t nks = gq_z_ksplit(L.m_pad, p->k);
     la.n_steps = (p->k + 63u) / 64u; la.steps_per_wave = ((la.n_steps + nks - 1u) / nks + 15u) / 16u;
     la.n_ksplit = nks; la.zf_slice = L.m_pad * 64u;
     z_slices = nks; z_slice_stride = L.m_pad * 64u;
-    la.nterms = 3u;
     la.n_blocks = L.m_pad / 32u;
-    const dim3 zgrid(L.m_pad / 32u * nks), zblock(1024);
-    (void)zblock;
-    if ((st = launch_lora_a(la, la.nkk, zgrid, s))) return st;
+    const dim3 zgrid(L.m_pad / 32u * nks);
+    if ((st = launch_lora_a(la, rank_chunks(p->rank), zgrid, s))) return st;
   } else if (lora) {
     GqLoraZArgs z{};
     z.x = q.x;
@@ -2210,11 +2196,11 @@ int mi355_w8a8_quantize_rows_v1(const void* x_bf16, int8_t* codes, float* scales
     return MI355_W8A8_ERR_ALIAS;
   QuantArgs q{};
   q.x = static_cast<const uint16_t*>(x_bf16);
-  q.M = m; q.K = k; q.K_pad = k_padded(k); q.KB = q.K_pad / 32u;
+  q.M = m; q.K = k;
   q.codes_rm = codes;
   q.scales_rm = scales;
   (void)hipGetLastError();
-  return launch_quant<false>(q, static_cast<hipStream_t>(stream));
+  return launch_quant(q, static_cast<hipStream_t>(stream));
 }
 
 uint64_t mi355_w8a8_workspace_bytes(uint32_t m, uint32_t k, uint32_t n, uint32_t n_adapters, uint32_t rank,

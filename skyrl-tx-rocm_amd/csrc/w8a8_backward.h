@@ -224,7 +224,7 @@ __device__ inline v8us lora_a_operand_item(const uint16_t* __restrict__ a, unsig
 
 struct BwdPrepArgs {
   const int32_t* idx;        // adapter per row, or null
-  int32_t* src_row; int32_t* dst_pos; int32_t* slot_group; int32_t* blk_range; int32_t* group_off;
+  int32_t* src_row; int32_t* slot_group; int32_t* blk_range; int32_t* group_off;
   const uint16_t* lora_a;    // bf16 [n_groups, K, r]
   uint16_t* at;              // bf16 [n_groups, r, K]
   unsigned char* ap;
@@ -238,7 +238,7 @@ __global__ __launch_bounds__(1024) void bwd_prep_kernel(BwdPrepArgs p) {
   if (b < p.route_blocks) {
     if (p.beyond && threadIdx.x == 0) p.beyond[0] = 0u;
     if (p.idx) {
-      route_rows_block(p.idx, p.M, p.n_groups, p.slots, p.src_row, p.dst_pos, p.slot_group, p.blk_range, p.group_off);
+      route_rows_block(p.idx, p.M, p.n_groups, p.slots, p.src_row, nullptr, p.slot_group, p.blk_range, p.group_off);
     } else {  // one adapter for every row: identity order, everything in group 0
       for (uint32_t g = threadIdx.x; g <= p.n_groups; g += 1024u) p.group_off[g] = g == 0 ? 0 : (int)p.M;
     }
@@ -276,7 +276,7 @@ __global__ __launch_bounds__(1024) void bwd_prep_kernel(BwdPrepArgs p) {
 // (256 slots, or 128 when the weights average few rows), so that
 // a pull-back tile never mixes two weights; inside a weight the groups follow each other without
 // gaps, exactly as the adapters of a dense call over that weight's rows would.
-//   src_row / dst_pos / slot_group / blk_range   as in the dense call; blk_range -1 for 32-slot blocks without a
+//   src_row / slot_group / blk_range             as in the dense call; blk_range -1 for 32-slot blocks without a
 //                                                row: no kernel prepares or consumes their operands
 //   group_beg[g], group_end[g]                   slots of group g
 //   tile_weight[t]                               weight of tile t | its rows << 16, -1 beyond the slots in use
@@ -288,7 +288,7 @@ __global__ __launch_bounds__(1024) void bwd_prep_kernel(BwdPrepArgs p) {
 // groups of 8168 rows.)
 // ---------------------------------------------------------------------------------------
 struct BwdGroupTables {
-  int32_t* src_row; int32_t* dst_pos; int32_t* slot_group; int32_t* blk_range;
+  int32_t* src_row; int32_t* slot_group; int32_t* blk_range;
   int32_t* group_beg; int32_t* group_end; int32_t* tile_weight; int32_t* chunk_tab; int32_t* chunk0;
 };
 
@@ -354,7 +354,6 @@ __device__ inline void route_weight_groups_block(const int32_t* __restrict__ gro
       grp = last_group[w0];  // (padding slots name the weight's last group that has rows)
       if (p < end) {
         src = (int)(row_start[g] + (p - slot_beg[g]));
-        t.dst_pos[src] = (int)p;
         grp = (int)g;
         // blocks behind the weight's rows stay at -1
         if ((p & 31u) == 0) range = (int)(g | group_at(p + 31u < end ? p + 31u : end - 1u) << 16);
@@ -367,7 +366,6 @@ __device__ inline void route_weight_groups_block(const int32_t* __restrict__ gro
     if ((p & 31u) == 0) t.blk_range[p >> 5] = range;
     if (p % tile_rows == 0) t.tile_weight[p / tile_rows] = tile;  // (a weight's tiles start at its first slot)
   }
-  for (uint32_t i = rows_total + first; i < M; i += stride) t.dst_pos[i] = -1;
   if (dx) {
     const size_t begin = (size_t)rows_total * K, end = (size_t)M * K;
     for (size_t i = begin + first; i < end; i += stride) dx[i] = 0;
@@ -547,7 +545,6 @@ __global__ __launch_bounds__(512, 1) void bwd_dx_kernel(BwdDxArgs g) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wrow = ROWS128 ? 0 : wave >> 2, wcol = ROWS128 ? wave : wave & 3;
   const int c = lane & 31, h = lane >> 5;
-  const int NBi = (int)g.NB;  // a multiple of 8
   const uint32_t lane16 = (uint32_t)lane * 16u;
 
   // identity operand of the transposing MFMA: lane (column c, k half h) holds byte 1 at k == c

@@ -148,10 +148,8 @@ __global__ __launch_bounds__(512, 1) void gq_bwd_dx_kernel(GqBwdDxArgs a) {
     const uint32_t s_piece = (lane & 7) * 4u;
     const float* s_row = a.ws + (size_t)(clamp_kb(kb0 + ((lane >> 3) & 3)) * 32u / a.group) * a.N;
     auto issue = [&](int i) {  // stage i of the segment
-      const uint32_t st = lds_base + (i % kGqBwdStages) * kGqBwdStageBytes;
       const uint32_t nb = (uint32_t)(nb0 + i);
       unsigned char* St = lds + (i % kGqBwdStages) * kGqBwdStageBytes;
-      (void)st;
       load_1k_to_lds(panel + (size_t)nb * 2048u, St + (wave * 2) * kBlockBytes);
       load_1k_to_lds(panel + (size_t)nb * 2048u + 1024u, St + (wave * 2 + 1) * kBlockBytes);
       if (wave < 4) {

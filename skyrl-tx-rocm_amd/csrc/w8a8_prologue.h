@@ -48,7 +48,7 @@ __global__ __launch_bounds__(256) void unpack_weight_kernel(const unsigned char*
 // Adapter routing: rows are grouped by adapter with no padding between groups (the
 // counterpart of prepare_routing, skyrl/tx/layers/util.py:66-87).
 //   src_row[p]    = original row of grouped slot p (p < M), -1 for the slots beyond M
-//   dst_pos[m]    = grouped slot of original row m
+//   dst_pos[m]    = grouped slot of original row m (optional)
 //   slot_group[p] = adapter of grouped slot p
 //   blk_range[b]  = first adapter | last adapter << 16 of the 32-row block b
 //   group_off[a]  = first grouped slot of adapter a (optional; entry n_groups = M)
@@ -133,7 +133,7 @@ __device__ inline void route_rows_block(const int32_t* __restrict__ idx, uint32_
     if (a >= 0) {
       const int i = (int)((wave * per + it) * 64u + lane);
       src_row[p] = i;
-      dst_pos[i] = p;
+      if (dst_pos) dst_pos[i] = p;
       slot_group[p] = a;
     }
   };
@@ -168,7 +168,6 @@ __device__ inline void route_rows_block(const int32_t* __restrict__ idx, uint32_
 // skyrl/tx/layers/util.py:8-59): group g owns group_sizes[g] consecutive rows and is padded
 // to a multiple of 32 grouped slots so that a 32-row block never mixes two weights.
 //   src_row[p]   = original row of slot p, -1 for padding
-//   dst_pos[m]   = slot of row m, -1 for rows beyond sum(group_sizes) (their output is zero)
 //   blk_range[b] = g | g << 16 for the 32-row blocks in use, -1 beyond
 //   tile_tab     = number of row tiles, then first block | blocks << 32 | group << 48 of each: a group's blocks
 //                  in the fewest tiles of at most tile_blocks, of heights that differ by one at most
@@ -212,7 +211,7 @@ __device__ inline uint32_t block_prefix_capped(uint32_t v, uint32_t limit, uint3
 // sum(group_sizes) get no slot; their output rows (zero_out, bf16 [M, zero_cols], optional) are cleared here.
 __device__ inline void route_groups_block(const int32_t* __restrict__ group_sizes, uint32_t M, uint32_t n_groups,
                                           uint32_t slots, int32_t* __restrict__ src_row,
-                                          int32_t* __restrict__ dst_pos, int32_t* __restrict__ blk_range,
+                                          int32_t* __restrict__ blk_range,
                                           uint64_t* __restrict__ tile_tab, uint32_t tile_blocks, uint16_t* __restrict__ zero_out, uint32_t zero_cols,
                                           uint32_t part, uint32_t n_parts) {
   __shared__ uint32_t row_start[kMaxGroups + 1];
@@ -249,16 +248,12 @@ __device__ inline void route_groups_block(const int32_t* __restrict__ group_size
         if (slot_start[mid] <= p) lo = mid; else hi = mid;
       }
       const uint32_t i = p - slot_start[lo];
-      if (i < row_start[lo + 1u] - row_start[lo]) {
-        src = (int)(row_start[lo] + i);
-        dst_pos[src] = (int)p;
-      }
+      if (i < row_start[lo + 1u] - row_start[lo]) src = (int)(row_start[lo] + i);
       range = (int)(lo | (lo << 16));
     }
     src_row[p] = src;
     if ((p & 31u) == 0) blk_range[p >> 5] = range;
   }
-  for (uint32_t i = rows_total + part * 1024u + tid; i < M; i += stride) dst_pos[i] = -1;
   if (zero_out) {
     const size_t begin = (size_t)rows_total * zero_cols, end = (size_t)M * zero_cols;
     for (size_t i = begin + part * 1024u + tid; i < end; i += stride) zero_out[i] = 0;
@@ -267,29 +262,19 @@ __device__ inline void route_groups_block(const int32_t* __restrict__ group_size
 
 // ---------------------------------------------------------------------------------------
 // Per-token dynamic int8 quantization (skyrl/tx/kernels/quantized_lora.py:199-212 with one
-// group per row), optionally preceded by RMSNorm
-// (skyrl/tx/kernels/rocm/bf16_rms_gate_up_lora_swiglu.py:299-303).  One wave per row; the
-// row lives in registers (NCH chunks of 8 bf16 per lane).  Bit-exact rules:
+// group per row), row-major: the public row quantizer, and the rows of a grouped call that have no slot.  One
+// wave per row; the row lives in registers (NCH chunks of 8 bf16 per lane).  Bit-exact rules, of every quantizer here:
 //   scale = amax > 0 ? amax / 127 : 1         IEEE float32 division
 //   code  = clamp(rint(v / scale), -127, 127) IEEE division, round half to even
-//   RMSNorm: mean = float(sum_f64(x*x) / K), inv = 1 / sqrt(mean + eps) (IEEE), and
-//            n = bf16((x * inv) * gamma) with two separate float32 multiplications.
+//   RMSNorm (skyrl/tx/kernels/rocm/bf16_rms_gate_up_lora_swiglu.py:299-303): mean = float(sum_f64(x*x) / K),
+//            inv = 1 / sqrt(mean + eps) (IEEE), and n = bf16((x * inv) * gamma) with two separate float32
+//            multiplications.
 // ---------------------------------------------------------------------------------------
 struct QuantArgs {
   const uint16_t* x;       // bf16 [M, K]
-  const float* gamma;      // f32 [K] or null
-  float eps;
-  uint32_t M, K, K_pad, KB;
-  const int32_t* dst_pos;  // grouped slot per row or null (identity)
-  unsigned char* xq_packed;// packed codes or null
-  float* sx_slots;         // f32 per grouped slot or null
+  uint32_t M, K;
   int8_t* codes_rm;        // row-major codes [M, K] or null
   float* scales_rm;        // f32 [M] or null
-  uint16_t* xn;            // bf16 [M, K] normalized rows or null
-  uint16_t* xn_aux;        // second copy for the caller or null
-  uint16_t* zero_out;      // bf16 [M, zero_cols]: rows without a slot (dst_pos < 0) are zero-filled
-  uint32_t zero_cols;
-  uint32_t* tile_ctr;      // 256 words cleared for the GEMM launches' tile counters, or null
   // Optional gather on the way in: row m is read from x[row_map[m] / row_div] (the sorted (token,
   // choice) pairs of an expert layer read their token's row; x then has the tokens' row count,
   // row_limit, to which the source row is clamped)
@@ -303,11 +288,10 @@ __device__ inline uint32_t mapped_row(int32_t value, uint32_t div, uint32_t limi
   return r < limit ? r : limit - 1u;
 }
 
-template <int NCH, bool RMS>
+template <int NCH>
 __global__ __launch_bounds__(256) void quant_rows_kernel(QuantArgs a) {
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t m = blockIdx.x * 4u + (threadIdx.x >> 6);
-  if (a.tile_ctr && blockIdx.x == 0) a.tile_ctr[threadIdx.x] = 0u;
   if (m >= a.M) return;
   const uint32_t xrow = a.row_map ? mapped_row(a.row_map[m], a.row_div, a.row_limit) : m;
   const uint16_t* xr = a.x + (size_t)xrow * a.K;
@@ -324,37 +308,6 @@ __global__ __launch_bounds__(256) void quant_rows_kernel(QuantArgs a) {
       v[j][2 * e + 1] = __uint_as_float(w[e] & 0xffff0000u);
     }
   }
-  if (RMS) {
-    double ss = 0.0;
-#pragma unroll
-    for (int j = 0; j < NCH; ++j)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) ss += (double)v[j][e] * (double)v[j][e];
-    ss = wave_sum(ss);
-    float var = (float)(ss / (double)a.K);
-    float inv = 1.0f / sqrtf(var + a.eps);
-#pragma unroll
-    for (int j = 0; j < NCH; ++j) {
-      uint32_t k0 = (j * 64u + lane) * 8u;
-      if (k0 < a.K) {
-        float4 g0 = *reinterpret_cast<const float4*>(a.gamma + k0);
-        float4 g1 = *reinterpret_cast<const float4*>(a.gamma + k0 + 4);
-        float g[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
-        uint32_t packed[4];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          float t = v[j][e] * inv;
-          t = t * g[e];
-          uint32_t b = f32_to_bf16_bits(t);
-          v[j][e] = __uint_as_float(b << 16);
-          if (e & 1) packed[e >> 1] |= b << 16; else packed[e >> 1] = b;
-        }
-        uint4 o = make_uint4(packed[0], packed[1], packed[2], packed[3]);
-        if (a.xn) *reinterpret_cast<uint4*>(a.xn + (size_t)m * a.K + k0) = o;
-        if (a.xn_aux) *reinterpret_cast<uint4*>(a.xn_aux + (size_t)m * a.K + k0) = o;
-      }
-    }
-  }
   float amax = 0.0f;
 #pragma unroll
   for (int j = 0; j < NCH; ++j)
@@ -362,14 +315,8 @@ __global__ __launch_bounds__(256) void quant_rows_kernel(QuantArgs a) {
     for (int e = 0; e < 8; ++e) amax = fmaxf(amax, fabsf(v[j][e]));
   amax = wave_max(amax);
   const float scale = amax > 0.0f ? amax / 127.0f : 1.0f;
-  const int p = a.dst_pos ? a.dst_pos[m] : (int)m;
-  if (p < 0 && a.zero_out) {
-    for (uint32_t cidx = lane; cidx < a.zero_cols; cidx += 64u) a.zero_out[(size_t)m * a.zero_cols + cidx] = 0;
-  }
-  if (lane == 0) {
-    if (a.sx_slots && p >= 0) a.sx_slots[p] = scale;
-    if (a.scales_rm) a.scales_rm[m] = scale;
-  }
+  if (lane == 0 && a.scales_rm) a.scales_rm[m] = scale;
+  if (!a.codes_rm) return;
   // codes = rint(v / scale) with the correctly rounded quotient, as in quant_lora_kernel: v * (1 / scale)
   // with the hardware reciprocal rounds to the same integer unless the product lies within 1e-4 of a
   // tie; those cases (and scales outside the reciprocal's safe range) are redone with the division.
@@ -377,36 +324,31 @@ __global__ __launch_bounds__(256) void quant_rows_kernel(QuantArgs a) {
   const bool scale_safe = scale > 1e-30f && scale < 1e30f;
 #pragma unroll
   for (int j = 0; j < NCH; ++j) {
-    uint32_t c = j * 64u + lane;
-    uint32_t k0 = c * 8u;
-    if (k0 >= a.K_pad) continue;
+    const uint32_t k0 = (j * 64u + lane) * 8u;
+    if (k0 >= a.K) continue;
     uint32_t lo = 0, hi = 0;
-    if (k0 < a.K) {
-      float q[8];
-      float off_integer = 0.0f;
+    float q[8];
+    float off_integer = 0.0f;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float t = v[j][e] * rscale;
-        q[e] = rintf(t);
-        off_integer = fmaxf(off_integer, fabsf(t - q[e]));
-      }
-      if (!scale_safe || off_integer > 0.4999f) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) q[e] = rintf(v[j][e] / scale);
-      }
-      // q is an integer in [-127, 127] (|v| <= the row's absmax): q + 128 lands in its byte with one
-      // v_cvt_pk_u8_f32, and flipping bit 7 of every byte turns the biased value into two's complement
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        lo = __builtin_amdgcn_cvt_pk_u8_f32(q[e] + 128.0f, (uint32_t)e, lo);
-        hi = __builtin_amdgcn_cvt_pk_u8_f32(q[e + 4] + 128.0f, (uint32_t)e, hi);
-      }
-      lo ^= 0x80808080u;
-      hi ^= 0x80808080u;
-      if (a.codes_rm) *reinterpret_cast<uint2*>(a.codes_rm + (size_t)m * a.K + k0) = make_uint2(lo, hi);
+    for (int e = 0; e < 8; ++e) {
+      const float t = v[j][e] * rscale;
+      q[e] = rintf(t);
+      off_integer = fmaxf(off_integer, fabsf(t - q[e]));
     }
-    if (a.xq_packed && p >= 0)
-      *reinterpret_cast<uint2*>(a.xq_packed + packed_offset((uint32_t)p, k0, a.KB)) = make_uint2(lo, hi);
+    if (!scale_safe || off_integer > 0.4999f) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) q[e] = rintf(v[j][e] / scale);
+    }
+    // q is an integer in [-127, 127] (|v| <= the row's absmax): q + 128 lands in its byte with one
+    // v_cvt_pk_u8_f32, and flipping bit 7 of every byte turns the biased value into two's complement
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      lo = __builtin_amdgcn_cvt_pk_u8_f32(q[e] + 128.0f, (uint32_t)e, lo);
+      hi = __builtin_amdgcn_cvt_pk_u8_f32(q[e + 4] + 128.0f, (uint32_t)e, hi);
+    }
+    lo ^= 0x80808080u;
+    hi ^= 0x80808080u;
+    *reinterpret_cast<uint2*>(a.codes_rm + (size_t)m * a.K + k0) = make_uint2(lo, hi);
   }
 }
 
@@ -589,7 +531,7 @@ __global__ __launch_bounds__(256) void zero_words_kernel(uint32_t* p, uint32_t c
 
 // ---------------------------------------------------------------------------------------
 // One launch for the independent preparation jobs of a call: adapter routing (block 0
-// when `idx` is given), the rows' statistics (dense calls), LoRA A transposition and LoRA B operand packing
+// when `idx` is given), the rows' statistics (dense calls), LoRA A and LoRA B in operand order
 // (the other blocks).
 // ---------------------------------------------------------------------------------------
 struct LoraPrepArgs {
@@ -597,12 +539,12 @@ struct LoraPrepArgs {
   int32_t* src_row; int32_t* dst_pos; int32_t* slot_group; int32_t* blk_range;
   const uint16_t* lora_a;    // bf16 [n_groups, K, r]
   const uint16_t* lora_b;    // bf16 [n_groups, r, N]
-  uint16_t* at;              // bf16 [n_groups, r, K]
+  uint16_t* at;              // A in operand order
   unsigned char* bp;         // packed B operands
   uint32_t M, K, N, n_groups, r, nkk, ncb, slots, route_blocks, a_blocks;
   uint32_t route_pad;        // dense routing block: every group's first slot is a multiple of this (0 or 1: packed)
-  uint32_t a_operand_kb;     // 0: `at` is the transposed A; else K_pad / 32 and `at` takes A in MFMA operand order
-  uint32_t a_operand_steps, a_operand_rb;  // or: ceil(K / 64) and the 32-wide rank blocks of lora_a_kernel's operand order
+  uint32_t a_operand_kb;     // K_pad / 32: the quantizer's operand order (lora_a_pack_item) ...
+  uint32_t a_operand_steps, a_operand_rb;  // ... or ceil(K / 64) and the 32-wide rank blocks of lora_a_kernel's (lora_a_pack32_item)
   // grouped (ragged) call: the routing block lays the groups out from their sizes instead
   const int32_t* group_sizes;  // int32 [n_groups] or null
   uint64_t* tile_tab;          // row tiles of the grouped GEMM ...
@@ -740,7 +682,7 @@ __global__ __launch_bounds__(1024, 8) void lora_prep_kernel(LoraPrepArgs p) {
   if (b < p.route_blocks) {
     __builtin_amdgcn_s_setprio(3);  // a chain of short steps beside waves that wait for memory
     if (p.group_sizes)
-      route_groups_block(p.group_sizes, p.M, p.n_groups, p.slots, p.src_row, p.dst_pos, p.blk_range, p.tile_tab,
+      route_groups_block(p.group_sizes, p.M, p.n_groups, p.slots, p.src_row, p.blk_range, p.tile_tab,
                          p.tile_blocks, p.zero_out, p.zero_cols, b, p.route_blocks);
     else
       route_rows_block(p.idx, p.M, p.n_groups, p.slots, p.src_row, p.dst_pos, p.slot_group, p.blk_range, nullptr,
@@ -760,14 +702,12 @@ __global__ __launch_bounds__(1024, 8) void lora_prep_kernel(LoraPrepArgs p) {
     if (p.a_operand_steps)
       lora_a_pack32_item(p.lora_a, reinterpret_cast<unsigned char*>(p.at), p.n_groups, p.K, p.r, p.a_operand_steps,
                          p.a_operand_rb, (uint64_t)b * 1024u + threadIdx.x);
-    else if (p.a_operand_kb && (p.r & 3u) == 0)
+    else if ((p.r & 3u) == 0)
       lora_a_pack4_item(p.lora_a, reinterpret_cast<unsigned char*>(p.at), p.n_groups, p.K, p.r, p.a_operand_kb, p.nkk,
                         (uint64_t)b * 1024u + threadIdx.x);
-    else if (p.a_operand_kb)
+    else
       lora_a_pack_item(p.lora_a, reinterpret_cast<unsigned char*>(p.at), p.n_groups, p.K, p.r, p.a_operand_kb, p.nkk,
                        (uint64_t)b * 1024u + threadIdx.x);
-    else
-      lora_a_transpose_item(p.lora_a, p.at, p.n_groups, p.K, p.r, (uint64_t)b * 1024u + threadIdx.x);
     return;
   }
   b -= p.a_blocks;
@@ -780,11 +720,8 @@ __global__ __launch_bounds__(1024, 8) void lora_prep_kernel(LoraPrepArgs p) {
 // ---------------------------------------------------------------------------------------
 // LoRA-A projection on bf16 MFMA: z[p, :] = n[src_row[p], :] @ A[group(p)]  (float32
 // accumulation of exact bf16 products; skyrl/tx/kernels/quantized_lora.py:300-301 and
-// skyrl/tx/layers/lora.py:150).  One workgroup of 8 waves per 32-row block; the waves take
-// disjoint K ranges and are reduced through LDS in wave order.  The float32 result is split
-// into three bf16 terms (z = hi + mid + lo exactly) and stored in the MFMA operand order the
-// GEMM epilogue consumes: zp[block][kk][term][lane][8], lane = row % 32 + 32 * h holding the
-// rank columns 16 kk + 8 h + 0..7.
+// skyrl/tx/layers/lora.py:150), of the backward and of the group-scaled call.  One workgroup of 16 waves per
+// 32-row block and slice of K; the waves take disjoint K ranges and are reduced through LDS in a fixed order.
 // ---------------------------------------------------------------------------------------
 struct LoraAArgs {
   const uint16_t* xsrc;     // bf16 [M, K] (x, or the normalized rows)
@@ -793,19 +730,12 @@ struct LoraAArgs {
   const int32_t* src_row;   // or null (identity)
   const int32_t* slot_group;// or null (group 0)
   const int32_t* blk_range; // or null
-  unsigned char* zp;        // packed z fragments
-  uint32_t M, K, r, nkk, steps_per_wave, n_steps, n_blocks;
-  uint32_t nterms;          // bf16 terms carried per value: 3 (exact split of the f32 value) or 2
-  // Optional float32 copies (backward): zf = the raw projection, zsf = the projection times the
-  // row's group scale; with group_scale the packed fragments carry the scaled value.  [slot][zf_stride]
-  float* zf; float* zsf; const float* group_scale; uint32_t zf_stride;
-  // K split (backward): with n_ksplit > 1 the grid holds n_ksplit workgroups per row block, each
+  uint32_t M, K, r, steps_per_wave, n_steps, n_blocks;
+  float* zf; uint32_t zf_stride;  // the projection, [slot][zf_stride]
+  // K split: with n_ksplit > 1 the grid holds n_ksplit workgroups per row block, each
   // sums its own range of k steps and writes zf + ksplit_index * zf_slice (floats); the caller adds
   // the slices.  0 or 1: one workgroup per row block.
   uint32_t n_ksplit, zf_slice;
-  // Optional gather on the way in (see QuantArgs): source row = row_map[row] / row_div, clamped to row_limit
-  const int32_t* row_map;
-  uint32_t row_div, row_limit;
 };
 
 // STAGED (RB = 1, the transposed A; with or without the K split): the operands of a k step travel through 8 KiB of LDS
@@ -819,7 +749,6 @@ template <int RB, bool STAGED = false>  // RB: number of 32-wide rank blocks (1 
 __global__ __launch_bounds__(1024) void lora_a_kernel(LoraAArgs a) {
   static_assert(!STAGED || RB == 1, "the staged form holds one rank block");
   __shared__ float red[4][RB][16][64];
-  __shared__ float zs[32][RB * 32 + 1];
   const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
   const uint32_t nks = a.n_ksplit > 1u ? a.n_ksplit : 1u;
   const uint32_t pb = blockIdx.x / nks, ks = blockIdx.x % nks;
@@ -831,7 +760,6 @@ __global__ __launch_bounds__(1024) void lora_a_kernel(LoraAArgs a) {
   const uint32_t p = pb * 32u + i;
   int src = a.src_row ? a.src_row[p] : (int)p;
   if (src >= (int)a.M) src = -1;
-  if (a.row_map && src >= 0) src = (int)mapped_row(a.row_map[src], a.row_div, a.row_limit);
   const uint32_t rowgrp = (a.slot_group && ghi > glo) ? (uint32_t)a.slot_group[p] : glo;
   const uint16_t* xr = a.xsrc + (size_t)(src < 0 ? 0 : src) * a.K;
   v16f acc[RB];
@@ -854,7 +782,6 @@ __global__ __launch_bounds__(1024) void lora_a_kernel(LoraAArgs a) {
       const uint32_t pj = pb * 32u + 8u * j + r8;
       int sj = a.src_row ? a.src_row[pj] : (int)pj;
       if (sj >= (int)a.M) sj = -1;
-      if (a.row_map && sj >= 0) sj = (int)mapped_row(a.row_map[sj], a.row_div, a.row_limit);
       xrow[j] = a.xsrc + (size_t)(sj < 0 ? 0 : sj) * a.K;
     }
     // where lane (i, h) finds quarter t of its operand: line i, piece 4 h + t
@@ -972,39 +899,8 @@ __global__ __launch_bounds__(1024) void lora_a_kernel(LoraAArgs a) {
     float sum = red[0][b][e][l];
 #pragma unroll
     for (int w = 1; w < 4; ++w) sum += red[w][b][e][l];
-    zs[8u * (e >> 2) + 4u * (l >> 5) + (e & 3u)][b * 32u + (l & 31u)] = sum;
-  }
-  __syncthreads();
-  if (a.zf || a.group_scale) {
-    for (uint32_t q = threadIdx.x; q < 32u * RB * 32u; q += 1024u) {
-      const uint32_t row = q / (RB * 32u), col = q % (RB * 32u);
-      const float raw = zs[row][col];
-      if (a.zf) a.zf[(size_t)ks * a.zf_slice + (size_t)(pb * 32u + row) * a.zf_stride + col] = raw;
-      if (a.group_scale) {
-        const uint32_t gr = (a.slot_group && ghi > glo) ? (uint32_t)a.slot_group[pb * 32u + row] : glo;
-        const float scaled = raw * a.group_scale[gr];
-        zs[row][col] = scaled;
-        if (a.zsf) a.zsf[(size_t)(pb * 32u + row) * a.zf_stride + col] = scaled;
-      }
-    }
-    __syncthreads();
-  }
-  if (!a.zp) return;
-  for (uint32_t q = threadIdx.x; q < a.nkk * 3u * 64u; q += 1024u) {
-    const uint32_t l = q & 63u, term = (q >> 6) % 3u, kk = q / 192u;
-    const uint32_t row = l & 31u, hh = l >> 5;
-    v8us o;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float z = zs[row][16u * kk + 8u * hh + e];
-      const uint32_t b0 = f32_to_bf16_bits(z);
-      const float r1 = z - bf16_bits_to_f32(b0);
-      const uint32_t b1 = f32_to_bf16_bits(r1);
-      const float r2 = r1 - bf16_bits_to_f32(b1);
-      const uint32_t b2 = f32_to_bf16_bits(r2);
-      o[e] = (unsigned short)(term == 0 ? b0 : (term == 1 ? b1 : (a.nterms >= 3u ? b2 : 0u)));
-    }
-    *reinterpret_cast<v8us*>(a.zp + (((size_t)pb * a.nkk + kk) * 3u + term) * kBlockBytes + l * 16u) = o;
+    const uint32_t row = 8u * (e >> 2) + 4u * (l >> 5) + (e & 3u), col = b * 32u + (l & 31u);
+    a.zf[(size_t)ks * a.zf_slice + (size_t)(pb * 32u + row) * a.zf_stride + col] = sum;
   }
 }
 
@@ -1016,9 +912,9 @@ __global__ __launch_bounds__(1024) void lora_a_kernel(LoraAArgs a) {
 // uses them twice: as int8 codes written into the activation's 1 KiB fragment block, and as the A operand
 // of v_mfma_f32_16x16x32_bf16 against the LoRA A of the row's group in that instruction's operand order.
 // The waves' z tiles are added in a fixed order, split exactly into three bf16 terms and stored in the
-// operand order the GEMM epilogue reads (see lora_a_kernel).
-// Arithmetic follows quant_rows_kernel (skyrl/tx/kernels/quantized_lora.py:199-212 and the
-// RMSNorm of bf16_rms_gate_up_lora_swiglu.py:299-303) operation for operation.
+// operand order the GEMM epilogue reads: zp[block][kk][term][lane][8], lane = row % 32 + 32 * h holding the
+// rank columns 16 kk + 8 h + 0..7.
+// Arithmetic: the rules at quant_rows_kernel, operation for operation.
 // Bound by memory for long rows and by latency for few of them.  Splitting the statistics off reads x twice,
 // the second time largely from the caches, and in return nothing has to be held: rows that had to wait in the
 // LDS for their scale gave a workgroup 16 of them only up to K = 4608 and four at K = 12288, where every
