@@ -697,11 +697,15 @@ GroupedLayout make_grouped_layout(uint32_t m, uint32_t k, uint32_t n, uint32_t n
   return w;
 }
 
-// Four waves per half block once the half blocks fill the chip several times over (a wave then has more of K to itself and
-// the sum over the waves costs less), else sixteen (the pass is a chain of latencies).  Measured, 16 / 4 waves, 128 groups, rank 16:
-// 16384 gathered rows of 2048: 44 / 31 us, 8168: 25 / 20, 128 (256 half blocks at most): 8.2 / 9.8; 16384 rows of 768: 22 / 14.5.
+// Four waves per half block once more rows than 4096 come (a wave then has more of K to itself and the sum over
+// the waves costs less), else sixteen (the pass is a chain of latencies); without LoRA there is no such sum and the line lies
+// at twice the rows.  Prologue in us, 16 / 4 waves, rows x K:
+//   128 groups, rank 16: 128 x 2048 17.6 / 18.5, 2048 19.1 / 19.2, 4096 21.8 / 22.2, 4608 29.8 / 26.1, 8192 32.6 / 30.1, 16384
+//     54.8 / 46.9; 4096 x 768 14.4 / 14.6, 6144 19.3 / 17.4.  32 groups of 1024: 4096 14.3 / 14.3, 4608 18.2 / 16.3.
+//   64 groups, rank 64: 512 x 2048 22.2 / 22.9, 4096 31.7 / 31.8, 4608 39.4 / 36.6, 32768 110 / 87.
+//   128 groups, no LoRA: 128 x 2048 11.5 / 12.8, 4608 19.0 / 19.6, 8192 20.3 / 20.8, 12288 27.1 / 26.1, 16384 35.2 / 33.5.
 int launch_grouped_quant(const QuantLoraArgs& q, uint32_t nkk, hipStream_t s) {
-  const bool few_waves = q.M >= 4096u;
+  const bool few_waves = q.M > (nkk ? 4096u : 8192u);
   const dim3 grid(q.n_half_blocks);
 #define W8A8_GQL(CB)                                                                                          \
   if (few_waves) hipLaunchKernelGGL((quant_lora_kernel<CB, false, 4u>), grid, dim3(256), 0, s, q);            \
@@ -870,9 +874,11 @@ int run_grouped(const mi355_w8a8_grouped_problem* p, hipStream_t s) {
 // and not all of it (sk_wgs workgroups of sk_q stages each; 0: no split).
 struct BwdDxSplit { uint32_t direct_tiles, sk_q, sk_wgs; };
 
-// Costs in stage times (about 1.05 us): a split adds the partial tiles' way through memory, 256 KiB written
+// Costs in stage times (about 1.05 us, 1.1 in the group-scaled kernel, whose stages have as many MFMAs): a split adds the partial tiles' way through memory, 256 KiB written
 // and read again for every workgroup and split tile (about 0.11 each at 4.7 TB/s), and a launch.  Measured: 2048 x 2560,
 // N = 10240 (80 tiles of 320 stages) 339 us whole, 135 + 22 us split; 3003 x 4096, N = 24576 (192 of 768) 800 us and 657 + 29 us.
+// Group-scaled, with what goes before the pull-back, whole / split: 200 x 4096 <- 4096 150 / 57, 800 x 12288 <- 4096 (128 tiles
+// left over of 384) 285 / 230, 1536 x 12288 <- 4096 (64 of 576) 434 / 355, 1536 x 2560 <- 6144 221 / 142.
 // Calls of fewer than 64 stages (N < 2048) stay whole: little to gain, and a grouped call over the same rows
 // then gives the same bits.
 // k_blocks: k blocks of a wave's tile (2; 1 in the group-scaled kernel, whose partial tiles are half the size).

@@ -275,8 +275,10 @@ __global__ __launch_bounds__(1024) void moe_scatter_kernel(MoeSortArgs a) {
 
 // The whole sort in one launch: every chunk's workgroup counts all pairs for itself, those of earlier chunks apart.
 // Bound by the launches (three dependent ones of 3-5 us otherwise); the repeated counting grows with the square of
-// the chunks, hence the limit.  Measured, 128 groups: 128 pairs 9 -> 4.4 us, 16384 pairs (16 chunks) 14.5 -> 10.4.
-constexpr uint32_t kMoeSortChunks = 16;
+// the chunks, hence the limit, just before few groups (whose counters collide) make the two level.  One launch / three:
+//   32 groups: 1024 pairs 4.4 / 7.5 us, 16384 7.5 / 9.7, 32768 10.9 / 11.1, 65536 17.9 / 13.8;
+//   128 groups: 1024 4.8 / 8.0, 16384 7.5 / 10.5, 32768 10.1 / 12.7, 65536 15.5 / 16.4;  512 groups: 32768 11.1 / 14.2.
+constexpr uint32_t kMoeSortChunks = 32;
 __global__ __launch_bounds__(1024) void moe_sort_kernel(MoeSortArgs a) {
   __shared__ uint32_t all[kMoeMaxExperts];   // pairs per group; then first position of this chunk's pairs of a group
   __shared__ uint32_t earlier[kMoeMaxExperts];

@@ -63,6 +63,7 @@ def test_row_tiles(sizes, k, n, rank, swiglu):
 
 @pytest.mark.parametrize("m,x_rows,repeat,k,rank", [
     (40, 5, 8, 136, 16), (300, 700, 1, 512, 24), (4100, 513, 8, 320, 8), (4097, 5000, 1, 256, 0), (24, 24, 3, 1032, 40),
+    (4097, 600, 7, 256, 40), (8193, 1100, 8, 136, 0),
 ])
 def test_mapped_rows_equal_gathered_rows(m, x_rows, repeat, k, rank):
     """Rows read through a map -- fewer source rows than rows (their statistics are taken per source row) and more,

@@ -9,6 +9,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("pairs,groups,repeat", [
     (1, 1, 1), (64, 1024, 8), (1023, 128, 1), (1024, 3, 8), (1025, 128, 5), (16384, 128, 8), (16385, 1024, 1), (40000, 60, 8),
+    (32768, 2, 8), (32769, 2, 1),
 ])
 def test_sort_is_stable(pairs, groups, repeat):
     import torch
