@@ -90,3 +90,40 @@ def test_parts_that_are_not_asked_for(pkg):
     torch.cuda.synchronize()
     assert torch.equal(whole[0], only_dx[0]) and only_dx[1:] == (None, None, None)
     assert only_lora[0] is None and all(torch.equal(p, q) for p, q in zip(whole[1:], only_lora[1:]))
+
+
+@pytest.mark.parametrize("m,k,n,bits", [(70, 192, 128, 4), (300, 264, 2056, 8)])  # whole tiles, split ones
+def test_replays_under_capture(pkg, m, k, n, bits):
+    """Captured once, replayed with new operands in the same buffers and eager work between: the eager call's bits."""
+    import torch
+
+    dev = torch.device("cuda:0")
+    g = torch.Generator(device="cpu").manual_seed(m)
+    bf = lambda *shape: (torch.randn(*shape, generator=g) * 0.1).to(torch.bfloat16).to(dev)
+    w = pkg.quantized_lora.quantize_frozen_weight(torch.randn(k, n, generator=g).to(dev), bits=bits, group_size=32 if k % 64 else 64)
+    operands = [bf(m, k), bf(m, n), bf(k, 16), bf(16, n)]
+    scaling = torch.full((), 1.5, device=dev)
+    x, dy, a, b = operands
+    run = lambda: pkg.gq_linear.backward(x, dy, w, a, b, scaling)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        run()
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = run()
+    for i in range(4):
+        for t in operands:
+            t.copy_(bf(*t.shape))
+        x[0, 0] = float("inf") if i == 1 else 1.0  # the look at operands that are not finite starts anew each time
+        want = run()
+        for t in got:
+            t.fill_(7.0)
+        junk = torch.randn(512, 512, device=dev)
+        assert bool(torch.isfinite((junk @ junk).sum()))
+        graph.replay()
+        torch.cuda.synchronize()
+        for p, q in zip(got, want):
+            assert torch.equal(torch.nan_to_num(p.float(), nan=3e38), torch.nan_to_num(q.float(), nan=3e38)), i
