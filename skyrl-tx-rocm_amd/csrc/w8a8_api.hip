@@ -659,9 +659,9 @@ struct GroupedLayout {
 
 // 32-row blocks that a GEMM tile holds at most, 4 or 8; the flags force either (8 only where K has the steps it
 // needs).  8 once the groups average at least 96 rows, so that nearly every group is one tile, while those tiles
-// still fill three quarters of the CUs and the epilogue's operands fit the ring (rank <= 16; beyond it the
-// tall tile spills 60 to 210 bytes a lane, with SwiGLU 28 up to there).  Grouped call, 4 / 8, sizes rows x K x N: 48 groups of 200 x 1024 x 1024, rank 16:
-// 63 / 59 us; 32 of 256 x 1024 x 1024 (128 tall tiles): 47 / 56; 128 of 128 x 2048 x 1536, rank 64: 240 / 273;
+// still fill three quarters of the CUs and the epilogue's operands fit the ring (rank <= 16; beyond it the tall
+// tile spills 60 to 212 bytes a lane).  Grouped call, 4 / 8, sizes rows x K x N: 48 groups of 200 x 1024 x 1024,
+// rank 16: 63 / 59 us; 32 of 256 x 1024 x 1024 (128 tall tiles): 47 / 56; 128 of 128 x 2048 x 1536, rank 64: 240 / 273;
 // 128 of 64 x 2048 x 1536, rank 16: 112 / 116.
 uint32_t grouped_tile_blocks(uint32_t m, uint32_t k, uint32_t n, uint32_t n_groups, uint32_t rank, uint32_t flags) {
   if (k_padded(k) < kGroupedTallMinK) return 4u;

@@ -60,6 +60,9 @@ enum { kModeDense = 0, kModeDense128 = 1 };
 
 // Where the epilogue of one 32-row block finds its operands: in memory.  (The grouped kernel has a form that finds them in the LDS.)
 struct EpilogueFromMemory {
+  // (Formed anew, the grouped kernel's registers fell so that a load of the epilogue shares one with an operand of the k
+  // loop, which then drains its ring at every step: rank 32, 128 rows a group 97 -> 122 us.)
+  static constexpr bool kLaneAnew = false;
   const GemmArgs& g;
   uint32_t pbase, tcol0, ncb_total;
   __device__ float sx(int c) const { return g.sx[pbase + c]; }
@@ -86,7 +89,9 @@ __device__ inline __attribute__((always_inline)) void gemm_epilogue_block(const 
                                                                           const float (&sw)[4], uint32_t tcol0, bool full_n,
                                                                           uint32_t n_out) {
   constexpr bool kLora = (NKK > 0) && (EPI != kEpiAcc);
-  const int lane = threadIdx.x & 63;
+  int lane = threadIdx.x & 63;
+  // (opaque: what the epilogue derives from it is formed here and not held, or spilled, through the k loop)
+  if constexpr (Source::kLaneAnew) asm volatile("" : "+v"(lane));
   const int c = lane & 31, h = lane >> 5;
   const uint32_t ncol = tcol0 + 4u * c;
   __builtin_amdgcn_sched_barrier(0);  // keep the blocks' register lifetimes apart
