@@ -525,6 +525,52 @@ __device__ inline void bwd_dx_store_block(const BwdDxArgs& g, uint32_t pbase, ui
   }
 }
 
+// The stages of a segment through a ring of AHEAD + 1 LDS stages, LOADS direct-to-LDS loads per wave each: stage i asks for
+// stage i + AHEAD.  `first` prepares the operands of stage 0 (busy: the wave has rows); `even` / `odd` (i, more) multiply
+// stage i and, with more, prepare those of i + 1.  L is even.
+template <int AHEAD, int LOADS, class Issue, class First, class Even, class Odd>
+__device__ inline __attribute__((always_inline)) void bwd_dx_stages(int L, bool busy, Issue&& issue, First&& first, Even&& even, Odd&& odd) {
+  wait_vmcnt<0>();  // stores of the previous tile
+  lds_barrier();
+#pragma unroll
+  for (int i = 0; i < AHEAD; ++i)
+    if (i < L) issue(i);
+  wait_vmcnt<0>();
+  lds_barrier();
+  if (busy) first();
+  const int L_main = L - AHEAD;  // stages that still have loads to issue
+  int i = 0;
+  for (; i + 1 < L_main; i += 2) {
+    // stage i + 1 (and so stage i) is older than the loads of the last AHEAD - 2 stages
+    wait_vmcnt<(AHEAD - 2) * LOADS>();
+    lds_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    issue(i + AHEAD);
+    even(i, true);
+    __builtin_amdgcn_sched_barrier(0);
+    wait_vmcnt<(AHEAD - 2) * LOADS>();
+    lds_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    issue(i + 1 + AHEAD);
+    odd(i + 1, true);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  for (; i < L; i += 2) {  // drain: fewer loads in flight than the count above assumes
+    wait_vmcnt<0>();
+    lds_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    if (i + AHEAD < L) issue(i + AHEAD);
+    even(i, true);
+    __builtin_amdgcn_sched_barrier(0);
+    wait_vmcnt<0>();
+    lds_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    if (i + 1 + AHEAD < L) issue(i + 1 + AHEAD);
+    odd(i + 1, i + 2 < L);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
 // ROWS128: the tile is 128 rows x 512 k (the eight waves side by side along k, the same 128 x 64 wave
 // tile): a stage then holds half the dy panel and twice the weight blocks, the same bytes and the same
 // four loads per wave.  For grouped calls whose weights own few rows each: half the padding per weight,
@@ -704,59 +750,23 @@ __global__ __launch_bounds__(512, 1) void bwd_dx_kernel(BwdDxArgs g) {
       }
     };
 
-    // ---- main loop.  Stage i issues the loads of stage i + 5.
     v8bf bqA[2][2], bqB[2][2];
-    wait_vmcnt<0>();  // stores of the previous tile
-    lds_barrier();
+    bwd_dx_stages<kBwdAhead, kBwdLoadsPerStage>(
+        L, n_act > 0, issue,
+        [&] {  // operands of stage 0
+          NextRegs nx;
+          next_read(0, nx);
+          next_wait(nx);
+          uint32_t pk[8];
 #pragma unroll
-    for (int i = 0; i < kBwdAhead; ++i)
-      if (i < L) issue(i);
-    wait_vmcnt<0>();
-    lds_barrier();
-    if (n_act > 0) {  // operands of stage 0
-      NextRegs nx;
-      next_read(0, nx);
-      next_wait(nx);
-      uint32_t pk[8];
+          for (int cb = 0; cb < 2; ++cb) {
+            const v16i tr = transpose_block(nx.raw[cb]);
 #pragma unroll
-      for (int cb = 0; cb < 2; ++cb) {
-        const v16i tr = transpose_block(nx.raw[cb]);
-#pragma unroll
-        for (int gq = 0; gq < 4; ++gq) convert4(tr, nx.s4[gq], gq, pk);
-        to_operands(pk, bqA[cb]);
-      }
-    }
-    const int L_main = L - kBwdAhead;  // stages that still have loads to issue
-    int i = 0;
-    for (; i + 1 < L_main; i += 2) {
-      // stage i + 1 (and so stage i) is older than the loads of the last three stages
-      wait_vmcnt<(kBwdAhead - 2) * kBwdLoadsPerStage>();
-      lds_barrier();
-      __builtin_amdgcn_sched_barrier(0);
-      issue(i + kBwdAhead);
-      stage(i, bqA, bqB, true);
-      __builtin_amdgcn_sched_barrier(0);
-      wait_vmcnt<(kBwdAhead - 2) * kBwdLoadsPerStage>();
-      lds_barrier();
-      __builtin_amdgcn_sched_barrier(0);
-      issue(i + 1 + kBwdAhead);
-      stage(i + 1, bqB, bqA, true);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    for (; i < L; i += 2) {  // drain: fewer loads in flight than the count above assumes
-      wait_vmcnt<0>();
-      lds_barrier();
-      __builtin_amdgcn_sched_barrier(0);
-      if (i + kBwdAhead < L) issue(i + kBwdAhead);
-      stage(i, bqA, bqB, true);
-      __builtin_amdgcn_sched_barrier(0);
-      wait_vmcnt<0>();
-      lds_barrier();
-      __builtin_amdgcn_sched_barrier(0);
-      if (i + 1 + kBwdAhead < L) issue(i + 1 + kBwdAhead);
-      stage(i + 1, bqB, bqA, i + 2 < L);
-      __builtin_amdgcn_sched_barrier(0);
-    }
+            for (int gq = 0; gq < 4; ++gq) convert4(tr, nx.s4[gq], gq, pk);
+            to_operands(pk, bqA[cb]);
+          }
+        },
+        [&](int i, bool more) { stage(i, bqA, bqB, more); }, [&](int i, bool more) { stage(i, bqB, bqA, more); });
 
     if (whole) {
 #pragma unroll

@@ -257,55 +257,19 @@ __global__ __launch_bounds__(512, 1) void gq_bwd_dx_kernel(GqBwdDxArgs a) {
       if (convert_next) to_operands(pk, bqN);
     };
 
-    // ---- main loop.  Stage i issues the loads of stage i + 6.
     v8bf bqA[2][TERMS], bqB[2][TERMS];
-    wait_vmcnt<0>();  // stores of the previous tile
-    lds_barrier();
+    bwd_dx_stages<kGqBwdAhead, kGqBwdLoads>(
+        L, n_act > 0, issue,
+        [&] {  // operands of stage 0
+          NextRegs nx;
+          next_read(0, nx);
+          uint32_t pk[TERMS][8];
+          const v16i tr = transpose_block(nx.raw);
 #pragma unroll
-    for (int i = 0; i < kGqBwdAhead; ++i)
-      if (i < L) issue(i);
-    wait_vmcnt<0>();
-    lds_barrier();
-    if (n_act > 0) {  // operands of stage 0
-      NextRegs nx;
-      next_read(0, nx);
-      uint32_t pk[TERMS][8];
-      const v16i tr = transpose_block(nx.raw);
-#pragma unroll
-      for (int gq = 0; gq < 4; ++gq) convert4(tr, nx.s4[gq], gq, pk);
-      to_operands(pk, bqA);
-    }
-    const int L_main = L - kGqBwdAhead;  // stages that still have loads to issue
-    int i = 0;
-    for (; i + 1 < L_main; i += 2) {
-      // stage i + 1 (and so stage i) is older than the loads of the last four stages
-      wait_vmcnt<(kGqBwdAhead - 2) * kGqBwdLoads>();
-      lds_barrier();
-      __builtin_amdgcn_sched_barrier(0);
-      issue(i + kGqBwdAhead);
-      stage(i, bqA, bqB, true);
-      __builtin_amdgcn_sched_barrier(0);
-      wait_vmcnt<(kGqBwdAhead - 2) * kGqBwdLoads>();
-      lds_barrier();
-      __builtin_amdgcn_sched_barrier(0);
-      issue(i + 1 + kGqBwdAhead);
-      stage(i + 1, bqB, bqA, true);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    for (; i < L; i += 2) {  // drain: fewer loads in flight than the count above assumes
-      wait_vmcnt<0>();
-      lds_barrier();
-      __builtin_amdgcn_sched_barrier(0);
-      if (i + kGqBwdAhead < L) issue(i + kGqBwdAhead);
-      stage(i, bqA, bqB, true);
-      __builtin_amdgcn_sched_barrier(0);
-      wait_vmcnt<0>();
-      lds_barrier();
-      __builtin_amdgcn_sched_barrier(0);
-      if (i + 1 + kGqBwdAhead < L) issue(i + 1 + kGqBwdAhead);
-      stage(i + 1, bqB, bqA, i + 2 < L);
-      __builtin_amdgcn_sched_barrier(0);
-    }
+          for (int gq = 0; gq < 4; ++gq) convert4(tr, nx.s4[gq], gq, pk);
+          to_operands(pk, bqA);
+        },
+        [&](int i, bool more) { stage(i, bqA, bqB, more); }, [&](int i, bool more) { stage(i, bqB, bqA, more); });
 
     const uint32_t kbw = kb0 + (uint32_t)wcol;
     if (whole) {
