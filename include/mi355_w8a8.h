@@ -80,8 +80,8 @@ typedef enum mi355_w8a8_status {
 #define MI355_W8A8_FLAG_TILE_256X256 128u
 #define MI355_W8A8_FLAG_TILE_128X128 2048u
 #define MI355_W8A8_FLAG_TILE_256X128_PAIR 4096u
-/* row tiles of the grouped call: the first forces tiles of at most 128 rows, the second of at most 256 (K > 128;
- * shorter K keeps 128); default: by the groups' average size, the rank and how many tiles result.  The results are
+/* row tiles of the grouped call (of twice the rows that the names say): the first forces tiles of at most 128 rows,
+ * the second of at most 256 (K > 128; shorter K keeps 128); default: by the groups' average size, the rank and how many tiles result.  The results are
  * the same bits.  Pass the same flags to the workspace query. */
 #define MI355_W8A8_FLAG_GROUPED_TILE64 256u
 #define MI355_W8A8_FLAG_GROUPED_TILE128 512u
@@ -93,13 +93,14 @@ typedef enum mi355_w8a8_status {
  * adapter_indices or another tile geometry.  The caller vouches for it; calls that run as 32-row chunks
  * keep no such copies and ignore the flag. */
 /* Calls of at most 32 rows (the skinny-M kernels, with SwiGLU too) write no such copies and ignore it: a larger call
- * may not rely on one of them.  What they can keep has flags of its own, MI355_W8A8_FLAG_DECODE_B_WRITE / _KEPT. */
-/* mi355_w8a8_grouped_v1 takes the flag too: its launch that lays out the slots then leaves the transposed A
- * and the packed B of an earlier grouped call on the same workspace with the same (k, n, n_groups, rank) as
+ * may not rely on one of them, unless that one ran with MI355_W8A8_FLAG_FORCE_TILED.  What they can keep has flags of
+ * its own, MI355_W8A8_FLAG_DECODE_B_WRITE / _KEPT. */
+/* mi355_w8a8_grouped_v1 takes the flag too: its launch that lays out the slots then leaves the A and B in
+ * operand order of an earlier grouped call on the same workspace with the same (k, n, n_groups, rank) as
  * they are. */
 #define MI355_W8A8_FLAG_LORA_PACK_VALID 1024u
-/* Calls of at most 16 rows, rank at most 32, m * rank at least 256, n a multiple of 4, without SwiGLU: B regrouped per row and adapter in the
- * workspace (a loop over the same batch reads it faster than B itself).  WRITE: this call regroups B and uses it.  KEPT: the
+/* Calls of at most 16 rows, rank at most 32, m * rank above 128, n a multiple of 4, without SwiGLU: B regrouped per row
+ * and adapter in the workspace (a loop over the same batch reads it faster than B itself).  WRITE: this call regroups B and uses it.  KEPT: the
  * workspace holds what a call with WRITE left there, for the same m, k, n, n_adapters and rank and the same contents
  * of lora_b and adapter_indices, and no call of other dimensions, or with MI355_W8A8_FLAG_FORCE_TILED, has used the
  * workspace since; the caller vouches for it.  Pass the flag to the workspace query.  Other calls ignore both. */

@@ -31,10 +31,11 @@ inline bool skinny_pairs(uint32_t n, bool swiglu, bool residual) {
   return swiglu || (!residual && (n & 1u) == 0 && n_padded(n) / 128u * 4u >= 512u);
 }
 // Calls that can keep B regrouped: one slice, one row half, whole column quads, and values enough.  Per call of a loop, B
-// gathered / regrouped: 12288 x 4096, 16 rows of rank 32 20.4 / 18.9 us, 8 rows 17.9 / 17.3; 2560 x 6144, 16 rows of
-// rank 32 16.2 / 13.8; with 4 rows of rank 16 or one row level (10.8 / 11.0, 11.5 / 11.9).
+// gathered / regrouped: 12288 x 4096, 16 rows of rank 32 20.4 / 18.9 us, 8 rows 17.9 / 17.3, 9 rows of rank 16 16.5 / 15.8;
+// 2560 x 6144, 16 rows of rank 32 16.2 / 13.8, 9 rows of rank 16 11.9 / 11.3; below that, where the host bounds a call,
+// level or 0.3 slower (4096 x 2560, 4 rows of rank 16 10.0 / 10.4, 8 rows 10.3 / 10.3).
 inline bool skinny_b_can_be_kept(uint32_t m, uint32_t n, uint32_t r, bool swiglu) {
-  return !swiglu && m <= 16u && r <= 32u && m * r >= 256u && (n & 3u) == 0;
+  return !swiglu && m <= 16u && r <= 32u && m * r > 128u && (n & 3u) == 0;
 }
 
 struct SkinnyLayout {

@@ -15,7 +15,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("m,k,n,n_ad,rank,form", [
     (16, 64, 4, 1, 16, "plain"), (9, 512, 132, 2, 31, "residual"), (15, 1024, 260, 16, 18, "plain"), (8, 256, 100, 3, 32, "residual"),
     (16, 2048, 128, 64, 16, "rms"), (16, 12288, 144, 5, 17, "residual"), (13, 16384, 64, 4, 29, "plain"),
-    (17, 256, 64, 2, 32, "plain"), (12, 256, 66, 2, 32, "plain"), (12, 256, 64, 2, 33, "plain"), (16, 256, 64, 2, 32, "swiglu"),
+    (9, 256, 64, 2, 16, "plain"), (17, 256, 64, 2, 32, "plain"), (12, 256, 66, 2, 32, "plain"), (12, 256, 64, 2, 33, "plain"), (16, 256, 64, 2, 32, "swiglu"),
     (16, 256, 16384, 2, 16, "plain"), (16, 256, 16384, 2, 16, "residual"),   # two slices (never kept), one
 ])
 def test_kept_b(m, k, n, n_ad, rank, form):
