@@ -353,13 +353,13 @@ struct GqBwdPlain {
   __device__ float d_a(uint32_t k, uint32_t j) const {
     double sum = 0.0;
     for (uint32_t m = 0; m < M && !is_nan(sum); ++m)
-      sum += (double)(bf16_bits_to_f32(x[(size_t)m * K + k]) * rs[(size_t)m * kBwdRankStride + j]);
+      sum += (double)bf16_bits_to_f32(x[(size_t)m * K + k]) * (double)rs[(size_t)m * kBwdRankStride + j];
     return (float)sum;
   }
   __device__ float d_b(const float* z, uint32_t n, uint32_t j) const {
     double sum = 0.0;
     for (uint32_t m = 0; m < M && !is_nan(sum); ++m)
-      sum += (double)(z[(size_t)m * kBwdRankStride + j] * bf16_bits_to_f32(dy[(size_t)m * N + n]));
+      sum += (double)z[(size_t)m * kBwdRankStride + j] * (double)bf16_bits_to_f32(dy[(size_t)m * N + n]);
     return (float)sum;
   }
   // This thread's share of sum(dy * (z @ B)).  By rows: r . z, or the products themselves where either is infinite.

@@ -51,3 +51,23 @@ def test_classes_of_the_cotangents(place, bits, group, scale, rank):
         assert torch.equal(g.isinf(), inf) and torch.equal(g[inf], r[inf]), name
         fin = r.isfinite()  # one rounding to bf16, float32 sums (2^-23 of a few hundred terms of size below 4)
         assert ((g - r)[fin].abs() <= 2.0 ** -8 * r[fin].abs() + 2.0 ** -12).all(), name
+
+
+def test_a_product_beyond_float32_beside_an_infinity():
+    """x * rs beyond the largest float32 is finite in the sum: the infinity of another row decides."""
+    import torch
+
+    pkg = load_package()
+    m, k, n, s = 40, 64, 64, 1.0
+    gen = torch.Generator().manual_seed(9)
+    rnd = lambda *shape: (torch.randn(*shape, generator=gen) * 0.5).to(torch.bfloat16)
+    x, dy, a, b = rnd(m, k).abs() + 1, torch.zeros(m, n, dtype=torch.bfloat16), rnd(k, 8), torch.zeros(8, n, dtype=torch.bfloat16)
+    x[3] = 4.0
+    b[2, 40], dy[3, 40], dy[7, 41], b[2, 41] = 2e38, 1.0, -INF, 1.0  # rs[3] = 2e38, times 4 beyond float32; rs[7] = -inf
+    wt = pkg.quantized_lora.quantize_frozen_weight(torch.randn(k, n, generator=gen).cuda(), bits=8, group_size=32)
+    print("[case] product beyond float32 beside an infinity", flush=True)
+    da = pkg.gq_linear.backward(x.cuda(), dy.cuda(), wt, a.cuda(), b.cuda(), s)[1].double().cpu()
+    rs = (dy.double() @ b.double().T) * s
+    want = x.double().T @ rs
+    assert torch.equal(da.isnan(), want.isnan()) and torch.equal(da.isinf(), want.isinf())
+    assert torch.equal(da[want.isinf()], want[want.isinf()])
