@@ -903,7 +903,7 @@ BwdDxSplit bwd_dx_split(uint32_t tiles_m, uint32_t tiles_k, uint32_t NB, uint32_
 struct BwdLayout {
   BwdDxSplit split;
   uint64_t part;
-  uint64_t dyp, swp, at, ap, rp, z, r_raw, rs, rpart, src_row, slot_group, blk_range, group_off, partA, partB, total;
+  uint64_t dyp, swp, at, ap, rp, z, r_raw, rs, rpart, zpart, src_row, slot_group, blk_range, group_off, partA, partB, total;
   uint64_t beyond;  // group-scaled calls
   uint32_t part_blocks;
   uint32_t slots, nkk, K_pad, KB, N_pad, NB, tiles_m, tiles_k, max_chunks, R, n_slices, groups_per_slice;
@@ -911,6 +911,14 @@ struct BwdLayout {
 
 // Workgroups of the preparation that lay out A for the pull-back's epilogue.
 uint32_t bwd_ap_blocks(uint32_t n_groups, uint32_t KB, uint32_t nkk) { return (uint32_t)(((uint64_t)n_groups * KB * nkk * 64u + 1023u) / 1024u); }
+
+// K slices of z = x @ A: a call of few row blocks still fills the chip.  A slice keeps at least one 64-wide step for each of
+// the 16 waves, and the count depends on K and N only, so that a grouped call and the dense calls over its groups add in the
+// same order.
+uint32_t bwd_z_slices(uint32_t k, uint32_t n_slices) {
+  const uint32_t by_steps = (k + 63u) / 64u / 16u ? (k + 63u) / 64u / 16u : 1u;
+  return by_steps < n_slices ? by_steps : n_slices;
+}
 
 // gq_k_pad: padded K of a group-scaled weight (its own k blocks, tiles of 128 k), or 0
 BwdLayout make_bwd_layout(uint32_t m, uint32_t k, uint32_t n, uint32_t n_groups, uint32_t rank, uint32_t gq_k_pad = 0u) {
@@ -925,7 +933,7 @@ BwdLayout make_bwd_layout(uint32_t m, uint32_t k, uint32_t n, uint32_t n_groups,
   w.max_chunks = (m + kBwdChunkRows - 1u) / kBwdChunkRows + n_groups;
   {  // dy is packed (and r accumulated) by workgroups that own a slice of the 128-column groups
     const uint32_t ng = w.N_pad / 128u;
-    w.n_slices = (ng + 3u) / 4u < 8u ? (ng + 3u) / 4u : 8u;
+    w.n_slices = (ng + 3u) / 4u < kBwdMaxSlices ? (ng + 3u) / 4u : kBwdMaxSlices;
     w.groups_per_slice = (ng + w.n_slices - 1u) / w.n_slices;
   }
   const uint32_t k_blocks = gq_k_pad ? 1u : 2u;  // of a wave's tile
@@ -948,7 +956,8 @@ BwdLayout make_bwd_layout(uint32_t m, uint32_t k, uint32_t n, uint32_t n_groups,
     w.z = off; off += align256((uint64_t)w.slots * kBwdRankStride * 4u);
     w.r_raw = off; off += align256((uint64_t)w.slots * kBwdRankStride * 4u);
     w.rs = off; off += align256((uint64_t)w.slots * kBwdRankStride * 4u);
-    w.rpart = off; off += align256((uint64_t)w.n_slices * w.slots * kBwdRankStride * 4u);  // also the K slices of z
+    w.rpart = off; off += align256((uint64_t)w.n_slices * w.slots * kBwdRankStride * 4u);
+    w.zpart = off; off += align256((uint64_t)bwd_z_slices(k, w.n_slices) * w.slots * kBwdRankStride * 4u);
     w.partA = off; off += align256((uint64_t)w.max_chunks * w.R * k * 4u);
     w.partB = off; off += align256((uint64_t)w.max_chunks * w.R * n * 4u);
     w.beyond = off; off += gq_k_pad ? align256((1u + bwd_ap_blocks(n_groups, w.KB, w.nkk)) * 4u) : 0u;
@@ -1056,20 +1065,19 @@ int launch_bwd_body(const BwdBody& b, const Layout& w, unsigned char* ws, hipStr
     if ((st = launch_status())) return st;
   }
   if (b.lora && !b.skip_prologue) {
-    {
-      BwdRFinishArgs f{};
-      f.rpart = reinterpret_cast<const float*>(ws + w.rpart);
-      f.slot_group = b.slot_group;
-      f.blk_range = b.skip_range;
-      f.lora_scaling = b.lora_scaling;
-      f.r_raw = reinterpret_cast<float*>(ws + w.r_raw);
-      f.rs = reinterpret_cast<float*>(ws + w.rs);
-      f.rp = ws + w.rp;
-      f.n_slices = w.n_slices; f.slots = w.slots; f.nkk = w.nkk; f.cols = w.nkk > 2u ? 64u : 32u;
-      f.beyond = beyond;
-      hipLaunchKernelGGL(bwd_r_finish_kernel, dim3(w.slots / 32u), dim3(256), 0, s, f);
-      if ((st = launch_status())) return st;
-    }
+    BwdRFinishArgs f{};
+    f.rpart = reinterpret_cast<const float*>(ws + w.rpart);
+    f.zpart = reinterpret_cast<const float*>(ws + w.zpart);
+    f.slot_group = b.slot_group;
+    f.blk_range = b.skip_range;
+    f.lora_scaling = b.lora_scaling;
+    f.r_raw = reinterpret_cast<float*>(ws + w.r_raw);
+    f.rs = reinterpret_cast<float*>(ws + w.rs);
+    f.rp = ws + w.rp;
+    f.z = reinterpret_cast<float*>(ws + w.z);
+    f.n_blocks = w.slots / 32u;
+    f.n_slices = w.n_slices; f.slots = w.slots; f.nkk = w.nkk; f.cols = w.nkk > 2u ? 64u : 32u;
+    f.beyond = beyond;
     // z = x @ A, recomputed rather than saved by the forward (and, of a group-scaled call, looked at for x)
     if (b.d_lora_b || b.d_lora_scaling || (beyond && b.d_lora_a)) {
       LoraAArgs lz{};
@@ -1079,29 +1087,18 @@ int launch_bwd_body(const BwdBody& b, const Layout& w, unsigned char* ws, hipStr
       lz.M = b.m; lz.K = b.k; lz.r = b.rank;
       lz.n_steps = (b.k + 63u) / 64u;
       lz.n_blocks = w.slots / 32u;
-      // K is cut into slices so that a call of few row blocks still fills the chip; the slices land
-      // in the partial table (r's partials have been consumed, it holds n_slices of them) and are
-      // added in slice order.  A slice keeps at least one 64-wide step for each of the 16 waves, and
-      // the count depends on K and N only, so that a grouped call and the dense calls over its
-      // groups add in the same order.
-      const uint32_t by_steps = lz.n_steps / 16u ? lz.n_steps / 16u : 1u;
-      const uint32_t nks = by_steps < w.n_slices ? by_steps : w.n_slices;
+      const uint32_t nks = bwd_z_slices(b.k, w.n_slices);
       lz.n_ksplit = nks;
       lz.steps_per_wave = ((lz.n_steps + nks - 1u) / nks + 15u) / 16u;
-      lz.zf = reinterpret_cast<float*>(ws + w.rpart);
+      lz.zf = reinterpret_cast<float*>(ws + w.zpart);
       lz.zf_stride = kBwdRankStride;
       lz.zf_slice = w.slots * kBwdRankStride;
       const dim3 grid(lz.n_blocks * nks);
       if ((st = launch_lora_a(lz, w.nkk, grid, s))) return st;
-      BwdRFinishArgs f{};
-      f.rpart = reinterpret_cast<const float*>(ws + w.rpart);
-      f.blk_range = b.skip_range;
-      f.r_raw = reinterpret_cast<float*>(ws + w.z);
-      f.n_slices = nks; f.slots = w.slots; f.nkk = w.nkk; f.cols = w.nkk > 2u ? 64u : 32u;
-      f.beyond = beyond;
-      hipLaunchKernelGGL(bwd_r_finish_kernel, dim3(w.slots / 32u), dim3(256), 0, s, f);
-      if ((st = launch_status())) return st;
+      f.z_slices = nks;
     }
+    hipLaunchKernelGGL(bwd_r_finish_kernel, dim3(f.n_blocks * (f.z_slices ? 2u : 1u)), dim3(256), 0, s, f);
+    if ((st = launch_status())) return st;
   }
   if (!b.skip_gemm) {
     BwdDxArgs g{};
@@ -1341,7 +1338,7 @@ int run_gq_backward(const mi355_w8a8_gq_bwd_problem* p, hipStream_t s) {
 // ---------------------------------------------------------------------------------------
 struct BwdGroupedLayout {
   uint64_t dyp, swp, src_row, slot_group, blk_range, group_beg, group_end, tile_weight, chunk_tab, chunk0,
-      at, ap, rp, z, r_raw, rs, rpart, partA, partB, total;
+      at, ap, rp, z, r_raw, rs, rpart, zpart, partA, partB, total;
   uint32_t slots, nkk, K_pad, KB, N_pad, NB, tiles_m, tiles_k, max_chunks, R, n_slices, groups_per_slice, n_weights,
       gpw, sw_stride, tile_rows;
 };
@@ -1372,7 +1369,7 @@ BwdGroupedLayout make_bwd_grouped_layout(uint32_t m, uint32_t k, uint32_t n, uin
   w.max_chunks = (m + kBwdChunkRows - 1u) / kBwdChunkRows + n_groups;
   {
     const uint32_t ng = w.N_pad / 128u;
-    w.n_slices = (ng + 3u) / 4u < 8u ? (ng + 3u) / 4u : 8u;
+    w.n_slices = (ng + 3u) / 4u < kBwdMaxSlices ? (ng + 3u) / 4u : kBwdMaxSlices;
     w.groups_per_slice = (ng + w.n_slices - 1u) / w.n_slices;
   }
   w.sw_stride = w.N_pad + kBwdScalePad;
@@ -1395,6 +1392,7 @@ BwdGroupedLayout make_bwd_grouped_layout(uint32_t m, uint32_t k, uint32_t n, uin
     w.r_raw = off; off += align256((uint64_t)w.slots * kBwdRankStride * 4u);
     w.rs = off; off += align256((uint64_t)w.slots * kBwdRankStride * 4u);
     w.rpart = off; off += align256((uint64_t)w.n_slices * w.slots * kBwdRankStride * 4u);
+    w.zpart = off; off += align256((uint64_t)bwd_z_slices(k, w.n_slices) * w.slots * kBwdRankStride * 4u);
     w.partA = off; off += align256((uint64_t)w.max_chunks * w.R * k * 4u);
     w.partB = off; off += align256((uint64_t)w.max_chunks * w.R * n * 4u);
   }

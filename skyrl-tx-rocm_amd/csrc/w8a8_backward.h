@@ -137,13 +137,20 @@ __global__ __launch_bounds__(256) void bwd_pack_dy_kernel(BwdPackDyArgs a) {
   }
 }
 
-// r of a 32-row block: the slices' partial sums added in slice order; written raw (for dscaling),
-// scaled by the row's group (for dA), and the scaled value split exactly into three bf16 terms in
-// the operand order of the pull-back epilogue, rp[block][kk][term][lane][8].
+// r and z of a 32-row block: the slices' partial sums added in slice order (workgroups 0 .. n_blocks - 1 of the launch: r,
+// the ones behind them: z).  r is written raw (for dscaling), scaled by the row's group (for dA), and the scaled value split
+// exactly into three bf16 terms in the operand order of the pull-back epilogue, rp[block][kk][term][lane][8]; z is the plain
+// sum.
+// Bound by the latency of the loads: a workgroup reads 32 rows x n_slices slices, and adding as the slices arrive, a value
+// at a time, waited once per slice and value (2048 rows, rank 64, 8 slices: 21.3 us for r and 7.1 us for the 2 slices of z,
+// 64 workgroups each).  With four columns a thread and all slices' loads in flight together, both in one launch: 5.6 us
+// (3003 rows, rank 32: 11.9 + 10.4 against 4.9).
+constexpr uint32_t kBwdMaxSlices = 8;
 struct BwdRFinishArgs {
-  const float* rpart; const int32_t* slot_group; const int32_t* blk_range; const float* lora_scaling;
-  float* r_raw; float* rs; unsigned char* rp;
-  uint32_t n_slices, slots, nkk, cols;  // cols = 16 * nkk rounded up to 32
+  const float* rpart; const float* zpart;  // [slices][slots][64]
+  const int32_t* slot_group; const int32_t* blk_range; const float* lora_scaling;
+  float* r_raw; float* rs; unsigned char* rp; float* z;
+  uint32_t n_blocks, n_slices, z_slices, slots, nkk, cols;  // cols = 16 * nkk rounded up to 32
   uint32_t* beyond;  // set where a value is beyond what bf16 terms can carry, or null
 };
 
@@ -152,22 +159,41 @@ __device__ inline bool beyond_bf16_terms(float v) { return (__float_as_uint(v) &
 
 __global__ __launch_bounds__(256) void bwd_r_finish_kernel(BwdRFinishArgs a) {
   __shared__ float zs[32][kBwdRankStride + 1];
-  const uint32_t pb = blockIdx.x;
+  const bool of_z = blockIdx.x >= a.n_blocks;  // workgroup-uniform
+  const uint32_t pb = of_z ? blockIdx.x - a.n_blocks : blockIdx.x;
   if (a.blk_range && a.blk_range[pb] < 0) return;  // block without rows (grouped calls): never consumed
-  for (uint32_t q = threadIdx.x; q < 32u * a.cols; q += 256u) {
-    const uint32_t row = q / a.cols, col = q % a.cols, slot = pb * 32u + row;
-    float raw = 0.0f;
-    for (uint32_t sl = 0; sl < a.n_slices; ++sl) raw += a.rpart[((size_t)sl * a.slots + slot) * kBwdRankStride + col];
-    a.r_raw[(size_t)slot * kBwdRankStride + col] = raw;
-    if (a.beyond && beyond_bf16_terms(raw)) *a.beyond = 1u;
-    if (!a.rp) continue;  // plain sum of the slices (the z table)
-    const uint32_t gr = a.slot_group ? (uint32_t)a.slot_group[slot] : 0u;
-    const float scaled = raw * a.lora_scaling[gr];
-    if (a.beyond && beyond_bf16_terms(scaled)) *a.beyond = 1u;
-    a.rs[(size_t)slot * kBwdRankStride + col] = scaled;
-    zs[row][col] = scaled;
+  const float* part = of_z ? a.zpart : a.rpart;
+  const uint32_t n_slices = of_z ? a.z_slices : a.n_slices, quads = a.cols / 4u;
+  const size_t slice = (size_t)a.slots * kBwdRankStride;
+  for (uint32_t q = threadIdx.x; q < 32u * quads; q += 256u) {
+    const uint32_t row = q / quads, col = q % quads * 4u, slot = pb * 32u + row;
+    const float* src = part + (size_t)slot * kBwdRankStride + col;
+    float4 v[kBwdMaxSlices];
+#pragma unroll
+    for (uint32_t sl = 0; sl < kBwdMaxSlices; ++sl)
+      v[sl] = *reinterpret_cast<const float4*>(src + (sl < n_slices ? sl : 0u) * slice);
+    float raw[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (uint32_t sl = 0; sl < kBwdMaxSlices; ++sl)
+      if (sl < n_slices) { raw[0] += v[sl].x; raw[1] += v[sl].y; raw[2] += v[sl].z; raw[3] += v[sl].w; }
+    float* dst = (of_z ? a.z : a.r_raw) + (size_t)slot * kBwdRankStride + col;
+    *reinterpret_cast<float4*>(dst) = make_float4(raw[0], raw[1], raw[2], raw[3]);
+    bool bad = false;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) bad |= beyond_bf16_terms(raw[e]);
+    if (!of_z) {
+      const float sc = a.lora_scaling[a.slot_group ? (uint32_t)a.slot_group[slot] : 0u];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        raw[e] *= sc;
+        bad |= beyond_bf16_terms(raw[e]);
+        zs[row][col + e] = raw[e];
+      }
+      *reinterpret_cast<float4*>(a.rs + (size_t)slot * kBwdRankStride + col) = make_float4(raw[0], raw[1], raw[2], raw[3]);
+    }
+    if (a.beyond && bad) *a.beyond = 1u;
   }
-  if (!a.rp) return;
+  if (of_z) return;
   __syncthreads();
   for (uint32_t q = threadIdx.x; q < a.nkk * 3u * 64u; q += 256u) {
     const uint32_t l = q & 63u, term = (q >> 6) % 3u, kk = q / 192u;
