@@ -903,7 +903,7 @@ BwdDxSplit bwd_dx_split(uint32_t tiles_m, uint32_t tiles_k, uint32_t NB, uint32_
 struct BwdLayout {
   BwdDxSplit split;
   uint64_t part;
-  uint64_t dyp, swp, at, ap, rp, z, r_raw, rs, rpart, zpart, src_row, slot_group, blk_range, group_off, partA, partB, total;
+  uint64_t dyp, swp, at, ap, rp, z, r_raw, rs, rpart, zpart, row_dot, src_row, slot_group, blk_range, group_off, partA, partB, total;
   uint64_t beyond;  // group-scaled calls
   uint32_t part_blocks;
   uint32_t slots, nkk, K_pad, KB, N_pad, NB, tiles_m, tiles_k, max_chunks, R, n_slices, groups_per_slice;
@@ -958,6 +958,7 @@ BwdLayout make_bwd_layout(uint32_t m, uint32_t k, uint32_t n, uint32_t n_groups,
     w.rs = off; off += align256((uint64_t)w.slots * kBwdRankStride * 4u);
     w.rpart = off; off += align256((uint64_t)w.n_slices * w.slots * kBwdRankStride * 4u);
     w.zpart = off; off += align256((uint64_t)bwd_z_slices(k, w.n_slices) * w.slots * kBwdRankStride * 4u);
+    w.row_dot = off; off += align256((uint64_t)w.slots * 8u);
     w.partA = off; off += align256((uint64_t)w.max_chunks * w.R * k * 4u);
     w.partB = off; off += align256((uint64_t)w.max_chunks * w.R * n * 4u);
     w.beyond = off; off += gq_k_pad ? align256((1u + bwd_ap_blocks(n_groups, w.KB, w.nkk)) * 4u) : 0u;
@@ -1075,7 +1076,8 @@ int launch_bwd_body(const BwdBody& b, const Layout& w, unsigned char* ws, hipStr
     f.rs = reinterpret_cast<float*>(ws + w.rs);
     f.rp = ws + w.rp;
     f.z = reinterpret_cast<float*>(ws + w.z);
-    f.n_blocks = w.slots / 32u;
+    f.row_dot = reinterpret_cast<double*>(ws + w.row_dot);
+    f.r = b.rank;
     f.n_slices = w.n_slices; f.slots = w.slots; f.nkk = w.nkk; f.cols = w.nkk > 2u ? 64u : 32u;
     f.beyond = beyond;
     // z = x @ A, recomputed rather than saved by the forward (and, of a group-scaled call, looked at for x)
@@ -1097,7 +1099,7 @@ int launch_bwd_body(const BwdBody& b, const Layout& w, unsigned char* ws, hipStr
       if ((st = launch_lora_a(lz, w.nkk, grid, s))) return st;
       f.z_slices = nks;
     }
-    hipLaunchKernelGGL(bwd_r_finish_kernel, dim3(f.n_blocks * (f.z_slices ? 2u : 1u)), dim3(256), 0, s, f);
+    hipLaunchKernelGGL(bwd_r_finish_kernel, dim3(w.slots / 32u), dim3(256), 0, s, f);
     if ((st = launch_status())) return st;
   }
   if (!b.skip_gemm) {
@@ -1164,6 +1166,7 @@ int launch_bwd_body(const BwdBody& b, const Layout& w, unsigned char* ws, hipStr
     r.partA = d.partA; r.partB = d.partB;
     r.r_raw = reinterpret_cast<const float*>(ws + w.r_raw);
     r.z = d.z;
+    r.row_dot = reinterpret_cast<const double*>(ws + w.row_dot);
     r.lora_scaling = b.lora_scaling;
     r.group_off = b.group_off;
     r.chunk0_tab = b.chunk0; r.group_beg = b.group_beg; r.group_end = b.group_end;
@@ -1171,7 +1174,7 @@ int launch_bwd_body(const BwdBody& b, const Layout& w, unsigned char* ws, hipStr
     r.d_b = static_cast<uint16_t*>(b.d_lora_b);
     r.d_s = b.d_lora_scaling;
     r.K = b.k; r.N = b.n; r.r = b.rank; r.R = w.R; r.n_groups = b.n_groups;
-    r.blocks_a = b.d_lora_a ? (uint32_t)(((uint64_t)b.n_groups * b.rank * b.k + 255u) / 256u) : 0u;
+    r.blocks_a = b.d_lora_a ? b.n_groups * ((b.k + kBwdReduceCols - 1u) / kBwdReduceCols) : 0u;
     r.blocks_b = b.d_lora_b ? (uint32_t)(((uint64_t)b.n_groups * b.rank * b.n / 4u + 255u) / 256u) : 0u;
   }
   if (b.lora && (b.want_grads || (beyond && !b.skip_gemm))) {
@@ -1338,7 +1341,7 @@ int run_gq_backward(const mi355_w8a8_gq_bwd_problem* p, hipStream_t s) {
 // ---------------------------------------------------------------------------------------
 struct BwdGroupedLayout {
   uint64_t dyp, swp, src_row, slot_group, blk_range, group_beg, group_end, tile_weight, chunk_tab, chunk0,
-      at, ap, rp, z, r_raw, rs, rpart, zpart, partA, partB, total;
+      at, ap, rp, z, r_raw, rs, rpart, zpart, row_dot, partA, partB, total;
   uint32_t slots, nkk, K_pad, KB, N_pad, NB, tiles_m, tiles_k, max_chunks, R, n_slices, groups_per_slice, n_weights,
       gpw, sw_stride, tile_rows;
 };
@@ -1393,6 +1396,7 @@ BwdGroupedLayout make_bwd_grouped_layout(uint32_t m, uint32_t k, uint32_t n, uin
     w.rs = off; off += align256((uint64_t)w.slots * kBwdRankStride * 4u);
     w.rpart = off; off += align256((uint64_t)w.n_slices * w.slots * kBwdRankStride * 4u);
     w.zpart = off; off += align256((uint64_t)bwd_z_slices(k, w.n_slices) * w.slots * kBwdRankStride * 4u);
+    w.row_dot = off; off += align256((uint64_t)w.slots * 8u);
     w.partA = off; off += align256((uint64_t)w.max_chunks * w.R * k * 4u);
     w.partB = off; off += align256((uint64_t)w.max_chunks * w.R * n * 4u);
   }

@@ -137,10 +137,9 @@ __global__ __launch_bounds__(256) void bwd_pack_dy_kernel(BwdPackDyArgs a) {
   }
 }
 
-// r and z of a 32-row block: the slices' partial sums added in slice order (workgroups 0 .. n_blocks - 1 of the launch: r,
-// the ones behind them: z).  r is written raw (for dscaling), scaled by the row's group (for dA), and the scaled value split
-// exactly into three bf16 terms in the operand order of the pull-back epilogue, rp[block][kk][term][lane][8]; z is the plain
-// sum.
+// r and z of a 32-row block: the slices' partial sums added in slice order.  r is written raw, scaled by the row's group (for
+// dA), and the scaled value split exactly into three bf16 terms in the operand order of the pull-back epilogue,
+// rp[block][kk][term][lane][8]; z is the plain sum, and row_dot the row's r . z in double (for dscaling).
 // Bound by the latency of the loads: a workgroup reads 32 rows x n_slices slices, and adding as the slices arrive, a value
 // at a time, waited once per slice and value (2048 rows, rank 64, 8 slices: 21.3 us for r and 7.1 us for the 2 slices of z,
 // 64 workgroups each).  With four columns a thread and all slices' loads in flight together, both in one launch: 5.6 us
@@ -150,7 +149,8 @@ struct BwdRFinishArgs {
   const float* rpart; const float* zpart;  // [slices][slots][64]
   const int32_t* slot_group; const int32_t* blk_range; const float* lora_scaling;
   float* r_raw; float* rs; unsigned char* rp; float* z;
-  uint32_t n_blocks, n_slices, z_slices, slots, nkk, cols;  // cols = 16 * nkk rounded up to 32
+  double* row_dot;  // [slots]
+  uint32_t n_slices, z_slices, slots, nkk, cols, r;  // cols = 16 * nkk rounded up to 32; z_slices 0: no z
   uint32_t* beyond;  // set where a value is beyond what bf16 terms can carry, or null
 };
 
@@ -159,41 +159,50 @@ __device__ inline bool beyond_bf16_terms(float v) { return (__float_as_uint(v) &
 
 __global__ __launch_bounds__(256) void bwd_r_finish_kernel(BwdRFinishArgs a) {
   __shared__ float zs[32][kBwdRankStride + 1];
-  const bool of_z = blockIdx.x >= a.n_blocks;  // workgroup-uniform
-  const uint32_t pb = of_z ? blockIdx.x - a.n_blocks : blockIdx.x;
+  const uint32_t pb = blockIdx.x;
   if (a.blk_range && a.blk_range[pb] < 0) return;  // block without rows (grouped calls): never consumed
-  const float* part = of_z ? a.zpart : a.rpart;
-  const uint32_t n_slices = of_z ? a.z_slices : a.n_slices, quads = a.cols / 4u;
+  const uint32_t quads = a.cols / 4u;  // 8 or 16 lanes to a row
   const size_t slice = (size_t)a.slots * kBwdRankStride;
   for (uint32_t q = threadIdx.x; q < 32u * quads; q += 256u) {
     const uint32_t row = q / quads, col = q % quads * 4u, slot = pb * 32u + row;
-    const float* src = part + (size_t)slot * kBwdRankStride + col;
-    float4 v[kBwdMaxSlices];
+    const size_t at = (size_t)slot * kBwdRankStride + col;
+    float4 v[kBwdMaxSlices], u[kBwdMaxSlices];
+#pragma unroll
+    for (uint32_t sl = 0; sl < kBwdMaxSlices; ++sl) v[sl] = *reinterpret_cast<const float4*>(a.rpart + at + (sl < a.n_slices ? sl : 0u) * slice);
+    if (a.z_slices) {
+#pragma unroll
+      for (uint32_t sl = 0; sl < kBwdMaxSlices; ++sl) u[sl] = *reinterpret_cast<const float4*>(a.zpart + at + (sl < a.z_slices ? sl : 0u) * slice);
+    }
+    const float sc = a.lora_scaling[a.slot_group ? (uint32_t)a.slot_group[slot] : 0u];
+    float raw[4] = {0.0f, 0.0f, 0.0f, 0.0f}, scaled[4], z[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (uint32_t sl = 0; sl < kBwdMaxSlices; ++sl)
-      v[sl] = *reinterpret_cast<const float4*>(src + (sl < n_slices ? sl : 0u) * slice);
-    float raw[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (uint32_t sl = 0; sl < kBwdMaxSlices; ++sl)
-      if (sl < n_slices) { raw[0] += v[sl].x; raw[1] += v[sl].y; raw[2] += v[sl].z; raw[3] += v[sl].w; }
-    float* dst = (of_z ? a.z : a.r_raw) + (size_t)slot * kBwdRankStride + col;
-    *reinterpret_cast<float4*>(dst) = make_float4(raw[0], raw[1], raw[2], raw[3]);
+      if (sl < a.n_slices) { raw[0] += v[sl].x; raw[1] += v[sl].y; raw[2] += v[sl].z; raw[3] += v[sl].w; }
     bool bad = false;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) bad |= beyond_bf16_terms(raw[e]);
-    if (!of_z) {
-      const float sc = a.lora_scaling[a.slot_group ? (uint32_t)a.slot_group[slot] : 0u];
+    for (int e = 0; e < 4; ++e) {
+      scaled[e] = raw[e] * sc;
+      bad |= beyond_bf16_terms(raw[e]) || beyond_bf16_terms(scaled[e]);
+      zs[row][col + e] = scaled[e];
+    }
+    *reinterpret_cast<float4*>(a.r_raw + at) = make_float4(raw[0], raw[1], raw[2], raw[3]);
+    *reinterpret_cast<float4*>(a.rs + at) = make_float4(scaled[0], scaled[1], scaled[2], scaled[3]);
+    if (a.z_slices) {
+#pragma unroll
+      for (uint32_t sl = 0; sl < kBwdMaxSlices; ++sl)
+        if (sl < a.z_slices) { z[0] += u[sl].x; z[1] += u[sl].y; z[2] += u[sl].z; z[3] += u[sl].w; }
+      *reinterpret_cast<float4*>(a.z + at) = make_float4(z[0], z[1], z[2], z[3]);
+      double dot = 0.0;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        raw[e] *= sc;
-        bad |= beyond_bf16_terms(raw[e]);
-        zs[row][col + e] = raw[e];
+        bad |= beyond_bf16_terms(z[e]);
+        if (col + e < a.r) dot += (double)raw[e] * (double)z[e];  // (beyond the rank: x times a zero of A, no number that counts)
       }
-      *reinterpret_cast<float4*>(a.rs + (size_t)slot * kBwdRankStride + col) = make_float4(raw[0], raw[1], raw[2], raw[3]);
+      for (uint32_t o = 1; o < quads; o <<= 1) dot += __shfl_xor(dot, (int)o, 64);
+      if (col == 0) a.row_dot[slot] = dot;
     }
     if (a.beyond && bad) *a.beyond = 1u;
   }
-  if (of_z) return;
   __syncthreads();
   for (uint32_t q = threadIdx.x; q < a.nkk * 3u * 64u; q += 256u) {
     const uint32_t l = q & 63u, term = (q >> 6) % 3u, kk = q / 192u;
@@ -1082,6 +1091,7 @@ struct BwdReduceArgs {
   const float* partA; const float* partB;
   const float* r_raw;       // f32 [slots][64] unscaled dy @ B.T
   const float* z;           // f32 [slots][64]
+  const double* row_dot;    // f64 [slots] r . z
   const float* lora_scaling;
   const int32_t* group_off;
   // grouped calls: first chunk of every group (n_groups + 1) and the groups' slot ranges, in memory
@@ -1092,13 +1102,19 @@ struct BwdReduceArgs {
   uint32_t K, N, r, R, n_groups, blocks_a, blocks_b;
 };
 
+constexpr uint32_t kBwdReduceCols = 64;  // columns of dA of a workgroup
+
 struct BwdNoPlain { static constexpr bool kAny = false; };
 
+// Adds the chunks.  Bound by memory (2048 rows, rank 64: 26 MB of partials) and by the one workgroup per group that forms ds.
+// 2048 rows of rank 64 15-18 -> 7.4 us, 3003 of rank 32 34 -> 6.8 and 8.3, 1536 of one adapter 29 -> 5.6, 128 experts
+// 13 and 19 -> 9.1 and 10.6: with ds formed from bwd_r_finish_kernel's row_dot, and dA read along k and turned in the LDS.
 // Plain: what replaces the sums of the partials where an operand is not finite (group-scaled calls), or BwdNoPlain.
 template <class Plain>
 __global__ __launch_bounds__(256) void bwd_dlora_reduce_kernel(BwdReduceArgs a, Plain plain) {
   __shared__ uint32_t chunk0_lds[kMaxAdapters + 1];
   __shared__ double red[256];
+  __shared__ __attribute__((aligned(16))) uint16_t turn[kBwdReduceCols][kBwdRankStride + 8];
   const uint32_t tid = threadIdx.x;
   bool use_plain = false;  // kernel-uniform
   if constexpr (Plain::kAny) use_plain = plain.wanted();
@@ -1123,29 +1139,16 @@ __global__ __launch_bounds__(256) void bwd_dlora_reduce_kernel(BwdReduceArgs a, 
   auto reduce_ds = [&](uint32_t b) {  // one block per group
     const uint32_t o0 = (uint32_t)(a.group_beg ? a.group_beg[b] : a.group_off[b]);
     const uint32_t o1 = (uint32_t)(a.group_end ? a.group_end[b] : a.group_off[b + 1]);
-    // thread = (rank column j, one of four rows per pass); eight passes of loads are in flight at a time:
-    // one load pair per iteration left this single workgroup per group waiting out a memory latency per
-    // four rows, longer than the rest of the launch takes
     double sum = 0.0;
-    const uint32_t j = tid & 63u;
     if (use_plain) {
       if constexpr (Plain::kAny) sum = plain.d_s(a.r_raw, a.z);
-    } else if (j < a.r) {
-      uint32_t slot = o0 + (tid >> 6);
-      for (; slot + 28u < o1; slot += 32u) {
-        float rv[8], zv[8];
+    } else {
+      for (uint32_t slot = o0 + tid; slot < o1; slot += 1024u) {
+        double v[4];
 #pragma unroll
-        for (uint32_t u = 0; u < 8; ++u) {
-          const size_t off = (size_t)(slot + 4u * u) * kBwdRankStride + j;
-          rv[u] = a.r_raw[off];
-          zv[u] = a.z[off];
-        }
+        for (uint32_t u = 0; u < 4; ++u) v[u] = a.row_dot[slot + 256u * u < o1 ? slot + 256u * u : slot];
 #pragma unroll
-        for (uint32_t u = 0; u < 8; ++u) sum += (double)rv[u] * (double)zv[u];
-      }
-      for (; slot < o1; slot += 4u) {
-        const size_t off = (size_t)slot * kBwdRankStride + j;
-        sum += (double)a.r_raw[off] * (double)a.z[off];
+        for (uint32_t u = 0; u < 4; ++u) sum += slot + 256u * u < o1 ? v[u] : 0.0;
       }
     }
     red[tid] = sum;
@@ -1156,8 +1159,24 @@ __global__ __launch_bounds__(256) void bwd_dlora_reduce_kernel(BwdReduceArgs a, 
     }
     if (tid == 0) a.d_s[b] = (float)red[0];
   };
-  // The blocks of ds come first in the grid: each walks all rows of its group and takes longest, so it
-  // starts at once and runs beside the short dA / dB blocks instead of after them.
+  // four adjacent columns of rank row j, the chunks of a group added in order, four of them in flight
+  auto sum_chunks = [&](const float* part, uint32_t grp, uint32_t j, uint32_t col, uint32_t C) -> float4 {
+    float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
+    const uint32_t ce = chunk0(grp + 1u);
+    for (uint32_t ch = chunk0(grp); ch < ce; ch += 4u) {
+      float4 v[4];
+#pragma unroll
+      for (uint32_t u = 0; u < 4; ++u)
+        v[u] = *reinterpret_cast<const float4*>(part + ((size_t)(ch + u < ce ? ch + u : ch) * a.R + j) * C + col);
+#pragma unroll
+      for (uint32_t u = 0; u < 4; ++u)
+        if (ch + u < ce) { sum.x += v[u].x; sum.y += v[u].y; sum.z += v[u].z; sum.w += v[u].w; }
+    }
+    return sum;
+  };
+  // The blocks of ds come first in the grid: each walks all rows of its group (one number a row, see bwd_r_finish_kernel:
+  // over the r and z tables themselves one workgroup a group took longer than the rest of the launch), so it starts at once
+  // and runs beside the short dA / dB blocks instead of after them.
   const uint32_t blocks_s = a.d_s ? a.n_groups : 0u;
   if (blockIdx.x < blocks_s) {
     reduce_ds(blockIdx.x);
@@ -1165,33 +1184,47 @@ __global__ __launch_bounds__(256) void bwd_dlora_reduce_kernel(BwdReduceArgs a, 
   }
   uint32_t b = blockIdx.x - blocks_s;
   if (b < a.blocks_a) {
-    // dA [group][k][j]: a thread per output element, j fastest, so that the stores are contiguous
-    const uint64_t e = (uint64_t)b * 256u + tid;
-    if (e >= (uint64_t)a.n_groups * a.K * a.r || !a.d_a) return;
-    const uint32_t j = (uint32_t)(e % a.r), col = (uint32_t)((e / a.r) % a.K), grp = (uint32_t)(e / ((uint64_t)a.r * a.K));
-    float sum = 0.0f;
-    if (use_plain) {
-      if constexpr (Plain::kAny) sum = plain.d_a(col, j);
-    } else {
-      for (uint32_t ch = chunk0(grp), ce = chunk0(grp + 1u); ch < ce; ++ch) sum += a.partA[((size_t)ch * a.R + j) * a.K + col];
+    // dA [group][k][j]: a block turns 64 columns k of a group, read along k, into rows of j (their outputs are one
+    // piece of memory).  (A thread per output, j fastest, read four bytes of every line it touched, once per rank.)
+    const uint32_t strips = (a.K + kBwdReduceCols - 1u) / kBwdReduceCols, grp = b / strips, c0 = b % strips * kBwdReduceCols;
+    const uint32_t cl = (tid & 15u) * 4u, col = c0 + cl;  // (K is a multiple of 8)
+    for (uint32_t j = tid >> 4; j < a.r; j += 16u) {
+      float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (col < a.K) {
+        if (use_plain) {
+          if constexpr (Plain::kAny)
+            sum = make_float4(plain.d_a(col, j), plain.d_a(col + 1u, j), plain.d_a(col + 2u, j), plain.d_a(col + 3u, j));
+        } else {
+          sum = sum_chunks(a.partA, grp, j, col, a.K);
+        }
+      }
+      turn[cl][j] = (uint16_t)f32_to_bf16_bits(sum.x);
+      turn[cl + 1u][j] = (uint16_t)f32_to_bf16_bits(sum.y);
+      turn[cl + 2u][j] = (uint16_t)f32_to_bf16_bits(sum.z);
+      turn[cl + 3u][j] = (uint16_t)f32_to_bf16_bits(sum.w);
     }
-    a.d_a[e] = (uint16_t)f32_to_bf16_bits(sum);
+    __syncthreads();
+    const uint32_t cols = a.K - c0 < kBwdReduceCols ? a.K - c0 : kBwdReduceCols;
+    uint16_t* dst = a.d_a + ((size_t)grp * a.K + c0) * a.r;
+    if ((a.r & 7u) == 0) {
+      for (uint32_t e = tid * 8u; e < cols * a.r; e += 2048u)
+        *reinterpret_cast<v8us*>(dst + e) = *reinterpret_cast<const v8us*>(&turn[e / a.r][e % a.r]);
+    } else {
+      for (uint32_t e = tid; e < cols * a.r; e += 256u) dst[e] = turn[e / a.r][e % a.r];
+    }
     return;
   }
   if (b < a.blocks_a + a.blocks_b) {
     // dB [group][j][n]: a thread per four adjacent columns (N is a multiple of 8)
     const uint64_t e = ((uint64_t)(b - a.blocks_a) * 256u + tid) * 4u;
-    if (e >= (uint64_t)a.n_groups * a.r * a.N || !a.d_b) return;
+    if (e >= (uint64_t)a.n_groups * a.r * a.N) return;
     const uint32_t col = (uint32_t)(e % a.N), j = (uint32_t)((e / a.N) % a.r), grp = (uint32_t)(e / ((uint64_t)a.N * a.r));
     float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
     if (use_plain) {
       if constexpr (Plain::kAny)
         sum = make_float4(plain.d_b(a.z, col, j), plain.d_b(a.z, col + 1u, j), plain.d_b(a.z, col + 2u, j), plain.d_b(a.z, col + 3u, j));
     } else {
-      for (uint32_t ch = chunk0(grp), ce = chunk0(grp + 1u); ch < ce; ++ch) {
-        const float4 v = *reinterpret_cast<const float4*>(a.partB + ((size_t)ch * a.R + j) * a.N + col);
-        sum.x += v.x; sum.y += v.y; sum.z += v.z; sum.w += v.w;
-      }
+      sum = sum_chunks(a.partB, grp, j, col, a.N);
     }
     const float sc = a.lora_scaling[grp];
     *reinterpret_cast<uint2*>(a.d_b + e) = make_uint2(pack_bf16x2(sum.x * sc, sum.y * sc), pack_bf16x2(sum.z * sc, sum.w * sc));
