@@ -58,6 +58,7 @@ inline uint64_t align256(uint64_t v) { return (v + 255u) & ~uint64_t(255); }
 
 struct WsLayout {
   uint64_t xq, sx, zp, at, bp, row_scale, row_inv, src_row, slot_group, blk_range, tile_ctr, skinny, total;
+  uint64_t split_z, split_bytes;  // the last part: a call that finds no room for it does without
   uint32_t slots, nkk, K_pad, KB, n_steps, steps_per_wave;
   uint32_t rows_bound;  // the slots that can hold rows (a multiple of 32)
 };
@@ -67,16 +68,15 @@ inline uint32_t rank_chunks(uint32_t rank) { return rank == 0 ? 0u : (rank <= 16
 
 // Between the skinny-M limit and this many rows a call without SwiGLU may run the skinny-M kernels
 // on chunks of 32 rows: the weight is streamed once per chunk (the later passes from the last-level
-// cache).  A chunk costs 14-29 us, growing with the weight's bytes; the tiled call (128 x 128 tiles,
-// adapters on block boundaries) about 20 us + 7.5 us per 1024 of K whatever the rows.  Measured,
-// chunks against tiles: 4096 x 2560 at 64 rows 43 us / 57, at 96 rows 63 / 57; 12288 x 4096 at
-// 96 rows 88 / 113, at 128 rows 116 / 114; 2560 x 6144 at 33 rows 55 / 42; 1024 x 1024 at 33 rows 27 / 24.
-constexpr uint32_t kSkinnyChunkedMaxRows = 128;
+// cache).  A chunk costs 14-25 us, growing with the weight's bytes; the tiled call (K-split tiles, z in quarters) 16 us
+// + 2.7 us per 1024 of K whatever the rows.  Measured, chunks against tiles: 12288 x 4096 at 40 rows 38 us / 48, at 64 rows 46 / 50;
+// 9728 x 2560 at 64 rows 39 / 48; 4096 x 2560, rank 64 at 33 rows 28 / 30; 8192 x 8192 at 40 rows 51 / 43, at 65 rows 80 / 45 (hence
+// the line in N); 2560 x 6144 at 40 rows 50 / 28.  The upper lines are from before those tiles: at 64 rows of 4096 x 2560 the chunks
+// are now level to 20 % behind, at 96 rows of 12288 x 4096 66 us / 50.
+constexpr uint32_t kSkinnyChunkedMaxRows = 96;
 inline bool skinny_chunked_pays(uint32_t m, uint32_t k, uint32_t n) {
-  if (m > kSkinnyChunkedMaxRows || (uint64_t)k_padded(k) * n_padded(n) > (64ull << 20)) return false;
-  if (k < 4096u) return false;
-  if (k >= 8192u) return m <= 96u;
-  return m <= 64u && n_padded(n) <= 4096u;
+  if (m > kSkinnyChunkedMaxRows || n_padded(n) > 4096u || (uint64_t)k_padded(k) * n_padded(n) > (64ull << 20)) return false;
+  return k >= 8192u || (k >= 4096u && m <= 64u);
 }
 
 // Grouped slots a call of m rows and n_groups adapters can need when every adapter's rows start on a
@@ -98,6 +98,23 @@ inline bool padded_groups_fit(uint32_t m, uint32_t n, uint32_t n_groups, bool wi
   const uint64_t resident = wide_tiles ? 256u : 512u;
   return rounds((uint64_t)(round_up(rows, tile_m) / tile_m) * per_row, resident) ==
          rounds((uint64_t)(round_up(base, tile_m) / tile_m) * per_row, resident);
+}
+
+// 64 x 128 tiles of a call whose slots end at rows_bound, the waves of a workgroup splitting K (w8a8_gemm_ksplit_kernel), and
+// whether it takes them: while all are resident at once, one to a CU (up to 256) or two.  Beyond, the 128 x 128 geometry moves
+// fewer bytes.  Whole call, the other prologue in front of the 128 x 128 tiles: 4096 -> 2560, rank 64: 333 rows 34 us against 51, 700 (480 tiles)
+// 46 against 52; 2560 -> 6144, rank 64: 128 rows 29 / 42, 333 rows (480) 39 / 43; 1024 -> 3072, rank 16 19 / 25;
+// 12288 -> 4096, rank 32: 333 rows 55 / 102; SwiGLU 1024 -> 6144, 333 rows 24 / 26.  As three rounds of pairs 2560 -> 6144, 700 rows 59 / 48.
+constexpr uint32_t kKSplitMaxTiles = 512u;
+inline uint32_t ksplit_tiles_m(uint32_t rows_bound) { return (rows_bound + (uint32_t)kGemm64TileM - 1u) / (uint32_t)kGemm64TileM; }
+inline bool ksplit_fits(uint32_t rows_bound, uint32_t n) { return ksplit_tiles_m(rows_bound) * ((n + 127u) / 128u) <= kKSplitMaxTiles; }
+// Bytes of z's four quarters (quant_lora_kernel's SPLIT form) for a call that may take those tiles, or 0.  Prologue of the call,
+// quarters / sixteen waves to a half block: 333 x 4096, rank 64 14 / 22 us, 333 x 12288, rank 32 22 / 41, 1000 x 1032 10 / 12;
+// level from 2000 rows of 1024 on.
+constexpr uint32_t kSplitZMaxRows = 2048;
+inline uint64_t split_z_bytes(uint32_t m, uint32_t n, uint32_t n_groups, uint32_t rank) {
+  if (!rank || m <= (uint32_t)kSkinnyMaxRows || m > kSplitZMaxRows || !ksplit_fits(round_up(m, 32u), n)) return 0u;
+  return (uint64_t)padded_rows_bound(m, n_groups < 2u ? 1u : n_groups) * rank_chunks(rank) * 256u;
 }
 
 WsLayout make_layout(uint32_t m, uint32_t k, uint32_t n, uint32_t n_groups, uint32_t rank, bool routed,
@@ -127,6 +144,8 @@ WsLayout make_layout(uint32_t m, uint32_t k, uint32_t n, uint32_t n_groups, uint
   w.tile_ctr = off; off += 1024u;  // two sets of eight counters, 64 bytes apart
   w.zp = off; off += rank ? align256((uint64_t)(w.slots / 32u) * w.nkk * 3u * kBlockBytes) : 0u;
   w.skinny = off; off += align256(skinny_layout(k, keep_b, m, n, rank).total);
+  w.split_bytes = split_z_bytes(m, n, n_groups, rank);
+  w.split_z = off; off += w.split_bytes;
   w.total = off;
   return w;
 }
@@ -188,6 +207,28 @@ int launch_gemm(const GemmArgs& g, uint32_t nkk, hipStream_t s) {
     case 1: return launch_gemm_one<EPI, 1, MODE>(g, s);
     case 2: return launch_gemm_one<EPI, 2, MODE>(g, s);
     case 4: return launch_gemm_one<EPI, 4, MODE>(g, s);
+    default: return MI355_W8A8_ERR_UNSUPPORTED;
+  }
+}
+
+template <int EPI, int NKK, bool PAIR>
+int launch_gemm_ksplit_one(const GemmArgs& g, hipStream_t s) {
+  constexpr int lds_bytes = PAIR ? kGemm64LdsBytes / 2 : kGemm64LdsBytes;
+  if (hipFuncSetAttribute(reinterpret_cast<const void*>(&w8a8_gemm_ksplit_kernel<EPI, NKK, PAIR>),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes) != hipSuccess)
+    return MI355_W8A8_ERR_LAUNCH;
+  hipLaunchKernelGGL((w8a8_gemm_ksplit_kernel<EPI, NKK, PAIR>), dim3(round_up(g.tiles_m * g.tiles_n, 8u)), dim3(256), lds_bytes, s, g);
+  return launch_status();
+}
+
+template <int EPI>
+int launch_gemm_ksplit(const GemmArgs& g, uint32_t nkk, hipStream_t s) {
+  const bool pair = g.tiles_m * g.tiles_n > 256u;
+  switch (nkk) {
+    case 0: return pair ? launch_gemm_ksplit_one<EPI, 0, true>(g, s) : launch_gemm_ksplit_one<EPI, 0, false>(g, s);
+    case 1: return pair ? launch_gemm_ksplit_one<EPI, 1, true>(g, s) : launch_gemm_ksplit_one<EPI, 1, false>(g, s);
+    case 2: return pair ? launch_gemm_ksplit_one<EPI, 2, true>(g, s) : launch_gemm_ksplit_one<EPI, 2, false>(g, s);
+    case 4: return pair ? launch_gemm_ksplit_one<EPI, 4, true>(g, s) : launch_gemm_ksplit_one<EPI, 4, false>(g, s);
     default: return MI355_W8A8_ERR_UNSUPPORTED;
   }
 }
@@ -404,6 +445,20 @@ int launch_quant_rows(const QuantLoraRowsArgs& a, uint32_t nkk, hipStream_t s) {
   }
 }
 
+int launch_quant_split(const QuantLoraArgs& q, bool normalize, hipStream_t s) {
+  const dim3 grid(q.n_half_blocks * 4u), block(256);
+#define W8A8_QS(CB)                                                                                        \
+  if (normalize) hipLaunchKernelGGL((quant_lora_kernel<CB, true, 4, true>), grid, block, 0, s, q);         \
+  else hipLaunchKernelGGL((quant_lora_kernel<CB, false, 4, true>), grid, block, 0, s, q)
+  switch (q.nkk) {
+    case 1: W8A8_QS(1); break;
+    case 2: W8A8_QS(2); break;
+    default: W8A8_QS(4); break;
+  }
+#undef W8A8_QS
+  return launch_status();
+}
+
 // Which of the two prologues a tiled call takes: quant_lora_rows_kernel (the rows held in the LDS: no launch for their statistics,
 // and a second group among sixteen rows costs little) or quant_lora_kernel (x read twice, two workgroups per CU,
 // A fetched once per sixteen rows whatever K is).  `boundaries`: the groups follow each other without padding, so
@@ -468,7 +523,7 @@ int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
   // The workspace is always sized for the routed layout so one allocation serves every call.
   const uint64_t need = mi355_w8a8_workspace_bytes(p->m, p->k, p->n, p->n_adapters, p->rank, p->flags);
   if (!p->workspace) return MI355_W8A8_ERR_WORKSPACE;
-  if (p->workspace_bytes < need) return MI355_W8A8_ERR_WORKSPACE;
+  if (p->workspace_bytes < need - split_z_bytes(p->m, p->n, p->n_adapters, lora ? p->rank : 0u)) return MI355_W8A8_ERR_WORKSPACE;
   if (reinterpret_cast<uintptr_t>(p->workspace) & 255u) return MI355_W8A8_ERR_ALIGN;
   const int path = choose_forward_path(p->m, p->k, p->n, p->flags);
   if (path < 0) return path;
@@ -517,7 +572,10 @@ int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
   // Rows held in the LDS, or read twice behind a launch that takes their statistics (quant_lora_rows_kernel,
   // quant_lora_kernel).
   const bool pack = lora && !(p->flags & MI355_W8A8_FLAG_LORA_PACK_VALID);
-  const bool rows_in_lds = prologue_keeps_rows(w.rows_bound, p->k, rms, lora, pack, routed && !pad_groups);
+  // (neither this nor the next may depend on the measurement flags: a GEMM-only call reads what its prologue left)
+  const bool ksplit = path == MI355_W8A8_PATH_TILED_128X128 && !(p->flags & MI355_W8A8_FLAG_TILE_128X128) && ksplit_fits(w.rows_bound, p->n);
+  const bool split_z = ksplit && w.split_bytes && p->workspace_bytes >= w.split_z + w.split_bytes;
+  const bool rows_in_lds = !split_z && prologue_keeps_rows(w.rows_bound, p->k, rms, lora, pack, routed && !pad_groups);
   const bool route_inline = rows_in_lds && routed && !pack && p->m <= kInlineRouteMaxRows;
   // launch 1: adapter routing, the rows' statistics and (unless the workspace holds them) the LoRA operands
   const uint32_t route_blocks = routed && !route_inline ? 1u : 0u, stat_blocks = rows_in_lds ? 0u : (p->m + 15u) / 16u;
@@ -574,9 +632,12 @@ int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
   q.nterms = (p->flags & MI355_W8A8_FLAG_LORA_SPLIT2) ? 2u : 3u;
   q.tile_ctr = reinterpret_cast<uint32_t*>(ws + w.tile_ctr);
   q.group_pad = pad_groups ? 32u : 1u;
+  q.zpart = reinterpret_cast<float*>(ws + w.split_z); q.slots = w.rows_bound;
   if (!skip_prologue) {
     const dim3 grid(q.n_half_blocks), block(1024);
-    if (rows_in_lds) {
+    if (split_z) {
+      if ((st = launch_quant_split(q, normalize, s))) return st;
+    } else if (rows_in_lds) {
       QuantLoraRowsArgs qr{};
       qr.q = q;
       qr.eps = p->rms_eps; qr.scales_rm = p->aux_x_scales; qr.xn_aux = static_cast<uint16_t*>(p->aux_normalized);
@@ -623,7 +684,7 @@ int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
   g.blk_range = routed ? blk_range : nullptr;
   g.residual = static_cast<const uint16_t*>(p->residual);
   g.out = p->out;
-  g.M = p->m; g.N = p->n; g.K_pad = w.K_pad; g.KB = w.KB; g.slots = w.slots;
+  g.M = p->m; g.N = p->n; g.K_pad = w.K_pad; g.KB = w.KB; g.slots = split_z ? q.slots : w.slots;
   g.total_rows = w.rows_bound;
   g.groups_per_weight = 1;
   g.tiles_m = w.slots / kTileM;
@@ -647,6 +708,12 @@ int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
   }
   if (wide) return swiglu ? launch_gemm16<kEpiSwiglu>(g, w.nkk, s) : launch_gemm16<kEpiPlain>(g, w.nkk, s);
   if (pair) return swiglu ? launch_gemm16<kEpiSwiglu, 2>(g, w.nkk, s) : launch_gemm16<kEpiPlain, 2>(g, w.nkk, s);
+  if (ksplit) {
+    g.tiles_m = ksplit_tiles_m(w.rows_bound);
+    g.tiles_n = (p->n + 127u) / 128u;
+    if (split_z) { g.zpart = q.zpart; g.nterms = q.nterms; }
+    return swiglu ? launch_gemm_ksplit<kEpiSwiglu>(g, w.nkk, s) : launch_gemm_ksplit<kEpiPlain>(g, w.nkk, s);
+  }
   if (small)
     return swiglu ? launch_gemm<kEpiSwiglu, kModeDense128>(g, w.nkk, s) : launch_gemm<kEpiPlain, kModeDense128>(g, w.nkk, s);
   return swiglu ? launch_gemm<kEpiSwiglu>(g, w.nkk, s) : launch_gemm<kEpiPlain>(g, w.nkk, s);
@@ -2244,7 +2311,8 @@ int mi355_w8a8_forward_static_ws_v1(const mi355_w8a8_problem* p, void* stream) {
   // so a call must not be told to keep it.
   if (p->flags & (MI355_W8A8_FLAG_LORA_PACK_VALID | MI355_W8A8_FLAG_SKIP_PROLOGUE | MI355_W8A8_FLAG_DECODE_B_KEPT))
     return MI355_W8A8_ERR_UNSUPPORTED;
-  const uint64_t need = mi355_w8a8_workspace_bytes(p->m, p->k, p->n, p->n_adapters, p->rank, p->flags);
+  const uint64_t full = mi355_w8a8_workspace_bytes(p->m, p->k, p->n, p->n_adapters, p->rank, p->flags);
+  const uint64_t need = full ? full - split_z_bytes(p->m, p->n, p->n_adapters, p->n_adapters ? p->rank : 0u) : 0u;
   if (need == 0 || need > MI355_W8A8_STATIC_WORKSPACE_BYTES) return MI355_W8A8_ERR_WORKSPACE;
   void* ws = static_workspace();
   if (!ws) return MI355_W8A8_ERR_LAUNCH;

@@ -24,6 +24,8 @@ struct GemmArgs {
   const float* sx;           // f32 [slots]
   const float* sw;           // f32 [N]
   const unsigned char* zp;   // packed z fragments [slots/32][NKK][3][64 lanes][8 bf16] or null
+  const float* zpart;        // f32 [4][slots][16 NKK] whose sum is z, instead of zp (w8a8_gemm_ksplit_kernel), or null
+  uint32_t nterms;           // bf16 terms that z is split into there (3 or 2)
   const float* lora_scaling; // f32 [n_groups]
   const unsigned char* bp;   // LoRA B in MFMA operand order [n_groups][N_pad/32][NKK][64 lanes][8 bf16] or null
   const int32_t* src_row;    // original row of every grouped slot, or null (identity)
@@ -469,6 +471,255 @@ void w8a8_gemm_kernel(GemmArgs g) {
     };
     epilogue_block(0);
     if constexpr (kWR == 2) epilogue_block(1);
+  }
+}
+
+// ---------------------------------------------------------------------------------------
+// The same product for calls of few rows: 64 x 128 tiles, the four waves of a workgroup taking every fourth 32-wide k block
+// of the whole tile.  No two waves read the same bytes, so the operands go from the caches into registers (kRing k blocks
+// ahead) without the LDS and without barriers, which then adds the waves' integer sums: exact, so the result is
+// the 128 x 128 geometry's bit for bit.  Behind it wave (i, jp) owns row block i and columns 4 c + 2 jp, + 1: a quarter of the
+// tile's epilogue each, whose operands have been on their way since the kernel's start.
+// PAIR: two workgroups to a CU, for up to twice the tiles: half the registers, so a shorter ring, the epilogue's operands
+// fetched behind the main loop, and the sums exchanged a column block at a time.
+// Bound by what a CU takes from the caches (24 KiB for 128 of K, 64 bytes a clock: 5 us at K = 4096 for one workgroup) and by the
+// latencies before and behind that.  333 x 4096 -> 2560, rank 64: 30 us on 80 tiles of 128 x 128, whose ring of LDS stages takes
+// 12 us at the LDS's rate, now 17; 333 x 12288 -> 4096 64 / 38; 700 x 4096 -> 2560 (480 tiles, PAIR) 32 / 31.
+// ---------------------------------------------------------------------------------------
+constexpr int kGemm64TileM = 64;
+constexpr int kGemm64LdsBytes = 4 * 3 * 8192;  // to each wave from the three others: 2 column blocks x 16 registers (PAIR: one)
+
+template <int EPI, int NKK, bool PAIR>
+__global__ __launch_bounds__(256, PAIR ? 2 : 1) void w8a8_gemm_ksplit_kernel(GemmArgs g) {
+  static_assert(EPI != kEpiAcc, "accumulators are read off the other geometries");
+  constexpr int kRing = PAIR ? 3 : 6;
+  constexpr int kParts = PAIR ? 2 : 1;  // passes of the sums' exchange
+  constexpr int kKK = NKK > 0 ? NKK : 1;
+  extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
+  const int lane = threadIdx.x & 63, c = lane & 31, h = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wr = wave & 1, jp = wave >> 1;
+  // an XCD's workgroups take the row tiles of neighbouring column tiles: the weight is fetched into one L2
+  const uint32_t ntile = g.tiles_m * g.tiles_n, per_xcd = (ntile + 7u) / 8u;
+  const uint32_t t = (blockIdx.x & 7u) * per_xcd + (blockIdx.x >> 3);
+  if ((blockIdx.x >> 3) >= per_xcd || t >= ntile) return;
+  const uint32_t tn = t / g.tiles_m, tm = t - tn * g.tiles_m;
+  const uint32_t tcol0 = tn * 128u, n_out = (EPI == kEpiSwiglu) ? g.N / 2u : g.N;
+  if (tcol0 >= g.N) return;  // workgroup-uniform
+  const uint32_t lane16 = (uint32_t)lane * 16u;
+
+  // ---- what the epilogue needs of this wave's row block and columns
+  const uint32_t pbase = tm * 64u + (uint32_t)wr * 32u;
+  const bool has_rows = pbase < g.total_rows;  // (the tile's second block may lie behind the slots that can hold rows)
+  const uint32_t pblk = has_rows ? pbase : tm * 64u;
+  const float sx_lane = g.sx[pblk + c];
+  const int src_lane = g.src_row ? g.src_row[pblk + c] : (int)(pblk + c);
+  const uint32_t range = (NKK > 0 && g.blk_range) ? (uint32_t)g.blk_range[pblk / 32u] : 0u;
+  const int glo = (int)(range & 0xffffu), ghi = (int)(range >> 16);
+  const int grp_lane = (NKK > 0 && ghi > glo && g.slot_group) ? g.slot_group[pblk + c] : glo;
+  const uint32_t ncol = tcol0 + 4u * c + 2u * jp;  // the lane's two columns
+  const bool full_n = tcol0 + 128u <= g.N && (g.N & 3u) == 0;  // workgroup-uniform
+  float sw[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) sw[j] = g.sw[ncol + j < g.N ? ncol + j : g.N - 1u];
+  const uint32_t ncb_total = n_padded(g.N) / 32u;
+  // LoRA operands of chunk kk: B of group gi for the two column blocks, z as bf16 terms (of the packed form, or its quarters
+  // added in order and split as quant_lora_store_z does)
+  auto fetch_b = [&](int gi, int kk, v8us (&b)[2]) {
+    const unsigned char* bb = g.bp + (((size_t)gi * ncb_total + tcol0 / 32u + 2u * jp) * kKK + kk) * kBlockBytes + lane16;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) b[j] = *reinterpret_cast<const v8us*>(bb + j * (kKK * kBlockBytes));
+  };
+  auto fetch_z = [&](int kk, v8us (&zt)[3]) {
+    const unsigned char* zb = g.zp + ((size_t)(pblk / 32u) * kKK + kk) * 3u * kBlockBytes + lane16;
+#pragma unroll
+    for (int t3 = 0; t3 < 3; ++t3) zt[t3] = *reinterpret_cast<const v8us*>(zb + t3 * kBlockBytes);
+  };
+  auto z_from_quarters = [&](int kk, v8us (&zt)[3]) {
+    const float* zq = g.zpart + (size_t)(pblk + c) * (16u * kKK) + 16 * kk + 8u * h;
+    const size_t quarter = (size_t)g.slots * (16u * kKK);
+    v4f q4[4][2];
+#pragma unroll
+    for (int p = 0; p < 4; ++p)
+#pragma unroll
+      for (int e = 0; e < 2; ++e) q4[p][e] = *reinterpret_cast<const v4f*>(zq + p * quarter + 4 * e);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float z = ((q4[0][e >> 2][e & 3] + q4[1][e >> 2][e & 3]) + q4[2][e >> 2][e & 3]) + q4[3][e >> 2][e & 3];
+      const uint32_t b0 = f32_to_bf16_bits(z);
+      const float r1 = z - bf16_bits_to_f32(b0);
+      const uint32_t b1 = f32_to_bf16_bits(r1);
+      const float r2 = r1 - bf16_bits_to_f32(b1);
+      zt[0][e] = (unsigned short)b0;
+      zt[1][e] = (unsigned short)b1;
+      zt[2][e] = (unsigned short)(g.nterms >= 3u ? f32_to_bf16_bits(r2) : 0u);
+    }
+  };
+  v8us zf[kKK][3], bf[kKK][2];  // (!PAIR: held from here on)
+  if constexpr (NKK > 0 && !PAIR) {
+#pragma unroll
+    for (int kk = 0; kk < kKK; ++kk) {
+      fetch_b(glo, kk, bf[kk]);
+      if (!g.zpart) fetch_z(kk, zf[kk]);  // kernel-uniform
+    }
+  }
+
+  // ---- main loop: stage s is k block 4 s + wave of the tile's two row blocks and four column blocks
+  const int n_stages = (int)(g.KB / 4u);  // (K_pad is a multiple of 128)
+  const size_t rb_bytes = (size_t)g.KB * kBlockBytes;
+  const unsigned char* const Ag = g.xq + (size_t)tm * 2u * rb_bytes + (size_t)wave * kBlockBytes;
+  const unsigned char* const Bg = g.wp + (size_t)tn * 4u * rb_bytes + (size_t)wave * kBlockBytes;
+  v4i af[kRing][2], wf[kRing][4];
+  auto fetch = [&](int u, int s) {
+    const size_t off = (size_t)(s < n_stages ? s : n_stages - 1) * (4u * kBlockBytes);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) af[u][i] = *reinterpret_cast<const v4i*>(Ag + i * rb_bytes + off + lane16);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) wf[u][j] = *reinterpret_cast<const v4i*>(Bg + j * rb_bytes + off + lane16);
+  };
+  v16i acc[2][4];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0;
+#pragma unroll
+  for (int u = 0; u < kRing; ++u) {
+    fetch(u, u);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  auto mul = [&](int u) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[u][i], wf[u][j], acc[i][j], 0, 0, 0);
+  };
+  int s0 = 0;
+#pragma unroll 1
+  for (; s0 + kRing <= n_stages; s0 += kRing) {
+#pragma unroll
+    for (int u = 0; u < kRing; ++u) {
+      mul(u);
+      fetch(u, s0 + u + kRing);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < kRing - 1; ++u)
+    if (s0 + u < n_stages) mul(u);  // wave-uniform
+
+  // ---- the waves' sums: to wave d its row block and column pair from the three others
+  v16i own[2];
+#pragma unroll
+  for (int part = 0; part < kParts; ++part) {
+    constexpr int kBlocks = 2 / kParts;  // column blocks of a pass
+    if (part) __syncthreads();  // (those of the pass before are read)
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+      if (wave == d) {
+#pragma unroll
+        for (int j = 0; j < kBlocks; ++j) own[part + j] = acc[d & 1][2 * (d >> 1) + part + j];
+      } else {
+        v4i* dst = reinterpret_cast<v4i*>(lds + (d * 3 + (wave < d ? wave : wave - 1)) * (4096 * kBlocks)) + lane;
+#pragma unroll
+        for (int j = 0; j < kBlocks; ++j)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const v16i& a = acc[d & 1][2 * (d >> 1) + part + j];
+            dst[(j * 4 + e) * 64] = v4i{a[4 * e], a[4 * e + 1], a[4 * e + 2], a[4 * e + 3]};
+          }
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < 3; ++s) {
+      const v4i* src = reinterpret_cast<const v4i*>(lds + (wave * 3 + s) * (4096 * kBlocks)) + lane;
+#pragma unroll
+      for (int j = 0; j < kBlocks; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const v4i v = src[(j * 4 + e) * 64];
+#pragma unroll
+          for (int q = 0; q < 4; ++q) own[part + j][4 * e + q] += v[q];
+        }
+    }
+  }
+  if (!has_rows) return;  // wave-uniform
+
+  if constexpr (NKK > 0 && !PAIR) {
+    if (g.zpart) {
+#pragma unroll
+      for (int kk = 0; kk < kKK; ++kk) z_from_quarters(kk, zf[kk]);
+    }
+  }
+  // ---- epilogue: gemm_epilogue_block's arithmetic on one column pair
+  const bool row_ok = src_lane >= 0 && src_lane < (int)g.M;
+  const uint32_t off_lane = row_ok ? (uint32_t)src_lane * n_out : 0xffffffffu;
+  const bool fast = full_n && __builtin_amdgcn_ballot_w64(!row_ok) == 0;  // wave-uniform
+  for (int gi = glo; gi <= ghi; ++gi) {  // wave-uniform; a boundary block runs once per group
+    v16f low[2];
+    if constexpr (NKK > 0) {
+      const float sgrp = g.lora_scaling[gi];
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) low[j][e] = 0.0f;
+#pragma unroll
+      for (int kk = 0; kk < NKK; ++kk) {
+        if (PAIR || gi > glo) fetch_b(gi, kk, bf[kk]);
+        if constexpr (PAIR) {
+          if (g.zpart) z_from_quarters(kk, zf[kk]);
+          else fetch_z(kk, zf[kk]);
+        }
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int t3 = 2; t3 >= 0; --t3)
+            low[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, zf[kk][t3]), __builtin_bit_cast(v8bf, bf[kk][j]),
+                                                             low[j], 0, 0, 0);
+      }
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) low[j][e] = low[j][e] * sgrp;
+    }
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      const int src_lane_addr = 16 * h + 4 * (8 * (v >> 2) + (v & 3));
+      const uint32_t rowoff = (uint32_t)__builtin_amdgcn_ds_bpermute(src_lane_addr, (int)off_lane);
+      const float sxv = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(src_lane_addr, __builtin_bit_cast(int, sx_lane)));
+      const float t0 = (float)own[0][v] * sxv, t1 = (float)own[1][v] * sxv;
+      float y0 = t0 * sw[0], y1 = t1 * sw[1];
+      if constexpr (NKK > 0) {
+        y0 = y0 + low[0][v];
+        y1 = y1 + low[1][v];
+      }
+      bool row_valid = fast || rowoff != 0xffffffffu;
+      if (NKK > 0 && ghi > glo) row_valid = row_valid && __builtin_amdgcn_ds_bpermute(src_lane_addr, grp_lane) == gi;
+      if constexpr (EPI == kEpiSwiglu) {  // (y0, y1) = (gate, up) of product column ncol / 2
+        const uint32_t f = pack_bf16x2(y0, y1);
+        const float p = swiglu_f32(__uint_as_float(f << 16), __uint_as_float(f & 0xffff0000u));
+        if (row_valid && (ncol >> 1) < n_out) reinterpret_cast<uint16_t*>(g.out)[rowoff + (ncol >> 1)] = (uint16_t)f32_to_bf16_bits(p);
+      } else {
+        uint16_t* o = reinterpret_cast<uint16_t*>(g.out) + (size_t)rowoff + ncol;
+        if (!row_valid) continue;
+        const bool in0 = full_n || ncol < g.N, in1 = full_n || ncol + 1u < g.N;
+        if (g.residual) {
+          const uint16_t* r = g.residual + (size_t)rowoff + ncol;
+          const uint32_t rr = full_n ? *reinterpret_cast<const uint32_t*>(r) : (in0 ? r[0] : 0u) | (in1 ? (uint32_t)r[1] << 16 : 0u);
+          y0 = y0 + __uint_as_float(rr << 16);
+          y1 = y1 + __uint_as_float(rr & 0xffff0000u);
+        }
+        const uint32_t bits = pack_bf16x2(y0, y1);
+        if (full_n) {
+          *reinterpret_cast<uint32_t*>(o) = bits;
+        } else {
+          if (in0) o[0] = (uint16_t)(bits & 0xffffu);
+          if (in1) o[1] = (uint16_t)(bits >> 16);
+        }
+      }
+    }
   }
 }
 

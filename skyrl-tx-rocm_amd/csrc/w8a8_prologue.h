@@ -939,6 +939,8 @@ struct QuantLoraArgs {
   float* sx_slots;          // f32 [slots]
   const uint16_t* at;       // LoRA A in MFMA operand order [n_groups][KB][CB][64 lanes][8 bf16] (lora_a_pack_item) or null (CB == 0)
   unsigned char* zp;        // packed z fragments
+  float* zpart;             // SPLIT: f32 [4][slots][16 CB], the quarters' sums
+  uint32_t slots;
   uint32_t r, nkk, nterms;
   uint32_t* tile_ctr;       // 256 words cleared for the GEMM launches' tile counters, or null
   uint32_t group_pad;       // > 1: whole half blocks may be empty
@@ -1064,17 +1066,41 @@ __device__ inline void quant_lora_store_z(const QuantLoraArgs& a, v4f (&acc)[kCB
   }
 }
 
-template <int CB, bool RMS, uint32_t WAVES = 16>  // CB: 16-wide rank blocks (0 = no LoRA, 1, 2, 4)
-__global__ __launch_bounds__(WAVES * 64, 4) void quant_lora_kernel(QuantLoraArgs a) {
+// The sum of a quarter's four tiles (waves w, w + 4, w + 8, w + 12 of the sixteen), in quant_lora_store_z's order.
+template <int kCB>
+__device__ inline void quant_lora_store_quarter(const QuantLoraArgs& a, const v4f (&acc)[kCB], float (*red)[kCB][4][64], uint32_t hb, uint32_t part) {
+  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+#pragma unroll
+  for (int b = 0; b < kCB; ++b)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) red[wave][b][e][lane] = acc[b][e];
+  __syncthreads();
+  for (uint32_t t = tid; t < (uint32_t)kCB * 256u; t += 256u) {
+    const uint32_t l = t & 63u, e = (t >> 6) & 3u, b = t >> 8;
+    const float sum = (red[0][b][e][l] + red[2][b][e][l]) + (red[1][b][e][l] + red[3][b][e][l]);
+    a.zpart[((size_t)part * a.slots + hb * 16u + 4u * (l >> 4) + e) * (kCB * 16u) + b * 16u + (l & 15u)] = sum;
+  }
+}
+
+// SPLIT: four workgroups of four waves share the half block, for calls whose half blocks are far fewer than the CUs.  Workgroup
+// `part` plays waves part, part + 4, + 8, + 12 of the sixteen, fetches a quarter of A, and leaves the sum of its waves'
+// tiles, added as the sixteen add theirs, in zpart: the consumer adds the quarters in order and so has the same z to the last bit
+// (w8a8_gemm_ksplit_kernel).  With few rows the sixteen-wave form is a chain of operand fetches in 128 registers a lane
+// (512 KiB of A for a workgroup at K = 4096, rank 64); a quarter of it fits in flight at once.
+template <int CB, bool RMS, uint32_t WAVES = 16, bool SPLIT = false>  // CB: 16-wide rank blocks (0 = no LoRA, 1, 2, 4)
+__global__ __launch_bounds__(WAVES * 64, SPLIT ? 2 : 4) void quant_lora_kernel(QuantLoraArgs a) {
+  static_assert(!SPLIT || (WAVES == 4 && CB > 0), "four workgroups of four waves, for LoRA-A");
   constexpr int kCB = CB > 0 ? CB : 1;
-  constexpr uint32_t kRing = CB == 4 || (CB == 2 && RMS) ? 2 : 4;  // operand sets (what 128 registers per lane hold)
-  constexpr uint32_t kAhead = 4;  // k-blocks of x a wave has in flight; a multiple of kRing
+  constexpr uint32_t kStride = SPLIT ? 16 : WAVES;  // k-blocks between two of a wave's
+  constexpr uint32_t kRing = SPLIT ? (RMS ? 4 : 8) : (CB == 4 || (CB == 2 && RMS) ? 2 : 4);  // operand sets (what the registers hold)
+  constexpr uint32_t kAhead = SPLIT ? 8 : 4;  // k-blocks of x a wave has in flight; a multiple of kRing
   static_assert(WAVES == 4 || WAVES == 16, "the reduction ends in four waves");
   __shared__ float red[CB > 0 ? (WAVES == 16 ? 8 : 4) : 1][kCB][4][64];  // wave tiles on their way to waves 0..7, then 0..3
   __shared__ float zs[16][kCB * 16 + 1];
   const uint32_t tid = threadIdx.x, lane = tid & 63u;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const uint32_t hb = blockIdx.x;                    // half block: slots 16 hb .. 16 hb + 15
+  const uint32_t hb = SPLIT ? blockIdx.x >> 2 : blockIdx.x;  // half block: slots 16 hb .. 16 hb + 15
+  const uint32_t vw = SPLIT ? (blockIdx.x & 3u) + 4u * wave : wave;  // the wave of the sixteen
   if (a.tile_ctr && blockIdx.x == 0 && tid < 256u) a.tile_ctr[tid] = 0u;
   if (hb >= a.n_half_blocks) return;
   const uint32_t pb = hb >> 1, half16 = hb & 1u;
@@ -1088,7 +1114,7 @@ __global__ __launch_bounds__(WAVES * 64, 4) void quant_lora_kernel(QuantLoraArgs
   const uint32_t xrow = a.row_map ? mapped_row(a.row_map[row], a.row_div, a.row_limit) : row;
   const float scale = a.row_scale[a.scale_by_source ? xrow : row];
   const float inv = RMS ? a.row_inv[row] : 1.0f;
-  if (wave == 0 && lane < 16u) a.sx_slots[hb * 16u + i] = scale;
+  if (vw == 0 && lane < 16u) a.sx_slots[hb * 16u + i] = scale;
   const float rscale = __builtin_amdgcn_rcpf(scale);
   const unsigned char* const xr = reinterpret_cast<const unsigned char*>(a.x) + (size_t)xrow * 2u * a.K;
   const uint32_t range = (CB > 0 && a.blk_range) ? (uint32_t)a.blk_range[pb] : 0u;
@@ -1101,37 +1127,37 @@ __global__ __launch_bounds__(WAVES * 64, 4) void quant_lora_kernel(QuantLoraArgs
   unsigned char* const xq_dst =
       a.xq_packed + (size_t)pb * a.KB * kBlockBytes + (16u * half16 + i + 32u * (q >> 1)) * 16u + 8u * (q & 1u);
 
-  // The wave's j-th k-block is wave + WAVES j.  Everything beyond the last block is read as zeros without a
+  // The wave's j-th k-block is vw + kStride j.  Everything beyond the last block is read as zeros without a
   // condition: A and the norm weights through buffer resources that end with the data, x from the row's start.
   const __amdgpu_buffer_rsrc_t grsrc =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.gamma), 0, RMS ? (int)(a.K * 4u) : 0, 0x00020000);
   const uint32_t at_bytes = a.KB * (uint32_t)kCB * kBlockBytes;  // of one group
-  const uint32_t kq = wave * 32u + q * 8u;                       // the lane's k in its wave's first k-block
+  const uint32_t kq = vw * 32u + q * 8u;                         // the lane's k in its wave's first k-block
   auto fetch_x = [&](uint32_t j) -> uint4 {
-    const uint32_t k0 = kq + WAVES * 32u * j;
+    const uint32_t k0 = kq + kStride * 32u * j;
     return *reinterpret_cast<const uint4*>(xr + 2u * (k0 < a.K ? k0 : 0u));  // (beyond K: zeroed where it is used)
   };
   struct Operands { v4i w[kCB]; v4f g0, g1; };
   auto fetch_operands = [&](const __amdgpu_buffer_rsrc_t& arsrc, uint32_t j, Operands& o) {
     if constexpr (CB > 0) {  // CB consecutive 1 KiB pieces (zero beyond K and the rank)
-      const uint32_t off = (wave + WAVES * j) * (uint32_t)(kCB * kBlockBytes) + lane * 16u;
+      const uint32_t off = (vw + kStride * j) * (uint32_t)(kCB * kBlockBytes) + lane * 16u;
 #pragma unroll
       for (int b = 0; b < CB; ++b) o.w[b] = __builtin_amdgcn_raw_buffer_load_b128(arsrc, off + b * kBlockBytes, 0, 0);
     }
     if constexpr (RMS) {
-      const uint32_t off = (kq + WAVES * 32u * j) * 4u;
+      const uint32_t off = (kq + kStride * 32u * j) * 4u;
       o.g0 = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(grsrc, off, 0, 0));
       o.g1 = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(grsrc, off + 16u, 0, 0));
     }
   };
   const bool scale_safe = scale > 1e-30f && scale < 1e30f;
   auto work = [&](auto codes, bool in_group, uint32_t j, const uint4& rawx, const Operands& o) {
-    const uint32_t kb = wave + WAVES * j;
+    const uint32_t kb = vw + kStride * j;
     uint4 raw = rawx;
     if constexpr (RMS)
       raw = rms_normalize8(rawx, inv, make_float4(o.g0[0], o.g0[1], o.g0[2], o.g0[3]), make_float4(o.g1[0], o.g1[1], o.g1[2], o.g1[3]));
     if (kb * 32u + 32u > a.K) {  // wave-uniform: the last k-block of an odd K, and the padding behind it
-      const bool live = kq + WAVES * 32u * j < a.K;
+      const bool live = kq + kStride * 32u * j < a.K;
       raw.x = live ? raw.x : 0u; raw.y = live ? raw.y : 0u; raw.z = live ? raw.z : 0u; raw.w = live ? raw.w : 0u;
     }
     if constexpr (decltype(codes)::value) {
@@ -1149,7 +1175,7 @@ __global__ __launch_bounds__(WAVES * 64, 4) void quant_lora_kernel(QuantLoraArgs
   // A pass over the k-blocks, kAhead per trip: the x of kAhead k-blocks and the other operands of kRing - 1
   // are in flight beside the one at work.  (With few workgroups on the chip the loop is a chain of those
   // loads' latencies; no load or store in it is conditional, so the compiler's waits can count.)
-  const uint32_t n_j = wave < a.KB ? (a.KB - wave + WAVES - 1u) / WAVES : 0u;
+  const uint32_t n_j = vw < a.KB ? (a.KB - vw + kStride - 1u) / kStride : 0u;
   auto pass = [&](auto codes, uint32_t grp, bool in_group) {
     const __amdgpu_buffer_rsrc_t arsrc = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<uint16_t*>(a.at) + (size_t)grp * (at_bytes / 2u), 0, CB > 0 ? (int)at_bytes : 0, 0x00020000);
@@ -1183,7 +1209,8 @@ __global__ __launch_bounds__(WAVES * 64, 4) void quant_lora_kernel(QuantLoraArgs
 #pragma unroll 1
     for (uint32_t grp = glo + 1u; grp <= ghi; ++grp) pass(std::false_type{}, grp, rowgrp == grp);
   }
-  if constexpr (CB > 0) quant_lora_store_z<kCB, WAVES>(a, acc, red, zs, pb, half16);
+  if constexpr (SPLIT) quant_lora_store_quarter<kCB>(a, acc, red, hb, blockIdx.x & 3u);
+  else if constexpr (CB > 0) quant_lora_store_z<kCB, WAVES>(a, acc, red, zs, pb, half16);
 }
 
 // ---------------------------------------------------------------------------------------
