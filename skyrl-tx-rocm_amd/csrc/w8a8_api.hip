@@ -1049,10 +1049,17 @@ int launch_bwd_dx_geometry(const BwdDxArgs& g, hipStream_t s) {
   uint32_t want = ((g.direct_tiles + 7u) / 8u) * 8u;
   if (g.sk_wgs > want) want = g.sk_wgs;
   const dim3 grid(want < 256u ? want : 256u), block(512);
-  if (hipFuncSetAttribute(reinterpret_cast<const void*>(&bwd_dx_kernel<NKK, ROWS128>),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, kBwdLdsBytes) != hipSuccess)
-    return MI355_W8A8_ERR_LAUNCH;
-  hipLaunchKernelGGL((bwd_dx_kernel<NKK, ROWS128>), grid, block, kBwdLdsBytes, s, g);
+  if (ROWS128) {
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&bwd_dx_kernel<NKK, true>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, kBwdLdsBytes) != hipSuccess)
+      return MI355_W8A8_ERR_LAUNCH;
+    hipLaunchKernelGGL((bwd_dx_kernel<NKK, true>), grid, block, kBwdLdsBytes, s, g);
+  } else {
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&bwd_dx_wide_kernel<NKK>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, kBwdLdsBytes) != hipSuccess)
+      return MI355_W8A8_ERR_LAUNCH;
+    hipLaunchKernelGGL((bwd_dx_wide_kernel<NKK>), grid, dim3(256), kBwdLdsBytes, s, g);
+  }
   if (!g.sk_wgs) return launch_status();
   if (const int st = launch_status()) return st;
   const uint32_t split_tiles = g.tiles_m * g.tiles_k - g.direct_tiles;

@@ -12,6 +12,8 @@
 // sixteen n per lane, exactly the B operand of v_mfma_f32_32x32x16_bf16 once the integers are
 // scaled and rounded to bf16.  No transposed ("shadow") copy of the weight exists.
 #pragma once
+#include <type_traits>
+
 #include "w8a8_device.h"
 #include "w8a8_prologue.h"
 
@@ -606,6 +608,57 @@ __device__ inline __attribute__((always_inline)) void bwd_dx_stages(int L, bool 
   }
 }
 
+// The tiles and split stages of this workgroup in order: work(tile, first stage, stages, slot).
+template <class Work>
+__device__ inline __attribute__((always_inline)) void bwd_dx_schedule(const BwdDxArgs& g, bool may_split, Work&& work) {
+  const uint32_t ntile = g.direct_tiles;
+  const uint32_t wgs_per_xcd = gridDim.x >> 3, xcd = blockIdx.x & 7u;
+  // band-major tile order, so an XCD's workgroups share panels.  One weight:
+  // every XCD walks a contiguous range of bands.  Grouped calls: the bands are dealt round-robin to the
+  // XCDs, because the slots in use end before the last bands and a contiguous split would leave the
+  // last XCDs without work.
+  const uint32_t band_tiles = 4u * g.tiles_k, n_bands = (g.tiles_m + 3u) / 4u;
+  const uint32_t per_xcd = g.tile_weight ? ((n_bands + 7u) / 8u) * band_tiles : (ntile + 7u) / 8u;
+  uint32_t ti = blockIdx.x >> 3;
+  // behind the whole tiles: this workgroup's stages of the split tiles' joint sequence (an XCD's workgroups are
+  // neighbours)
+  const uint32_t sw8 = g.sk_wgs >> 3, sk_w = xcd * sw8 + (blockIdx.x >> 3);
+  uint32_t s0 = 0, s1 = 0;
+  if (may_split && (blockIdx.x >> 3) < sw8) {
+    const uint32_t total = (g.tiles_m * g.tiles_k - ntile) * g.NB;
+    s0 = sk_w * g.sk_q < total ? sk_w * g.sk_q : total;
+    s1 = s0 + g.sk_q < total ? s0 + g.sk_q : total;
+  }
+#pragma unroll 1
+  for (;;) {
+    uint32_t t, nb0 = 0, len = g.NB, slot = 0;
+    if (ti < per_xcd) {
+      const uint32_t pos = ti;
+      ti += wgs_per_xcd;
+      if (g.tile_weight) {
+        const uint32_t band = xcd + 8u * (pos / band_tiles), in_band = pos % band_tiles;
+        if (band >= n_bands) { ti = per_xcd; continue; }
+        const uint32_t band_rows = (g.tiles_m - band * 4u) < 4u ? (g.tiles_m - band * 4u) : 4u;
+        if (in_band >= band_rows * g.tiles_k) continue;  // a last band with fewer than 4 row tiles
+        t = band * band_tiles + in_band;
+      } else {
+        t = xcd * per_xcd + pos;
+        if (t >= ntile) { ti = per_xcd; continue; }
+      }
+    } else if (s0 < s1) {
+      const uint32_t u = s0 / g.NB;
+      nb0 = s0 - u * g.NB;
+      len = s1 - s0 < g.NB - nb0 ? s1 - s0 : g.NB - nb0;
+      t = ntile + u;
+      slot = sk_w + u;
+      s0 += len;
+    } else {
+      break;
+    }
+    work(t, (int)nb0, (int)len, slot);
+  }
+}
+
 // ROWS128: the tile is 128 rows x 512 k (the eight waves side by side along k, the same 128 x 64 wave
 // tile): a stage then holds half the dy panel and twice the weight blocks, the same bytes and the same
 // four loads per wave.  For grouped calls whose weights own few rows each: half the padding per weight,
@@ -822,54 +875,248 @@ __global__ __launch_bounds__(512, 1) void bwd_dx_kernel(BwdDxArgs g) {
     }
   };
 
-  const uint32_t ntile = g.direct_tiles;
-  const uint32_t wgs_per_xcd = gridDim.x >> 3, xcd = blockIdx.x & 7u;
-  // band-major tile order, so an XCD's workgroups share panels.  One weight:
-  // every XCD walks a contiguous range of bands.  Grouped calls: the bands are dealt round-robin to the
-  // XCDs, because the slots in use end before the last bands and a contiguous split would leave the
-  // last XCDs without work.
-  const uint32_t band_tiles = 4u * g.tiles_k, n_bands = (g.tiles_m + 3u) / 4u;
-  const uint32_t per_xcd = g.tile_weight ? ((n_bands + 7u) / 8u) * band_tiles : (ntile + 7u) / 8u;
-  uint32_t ti = blockIdx.x >> 3;
-  // behind the whole tiles: this workgroup's stages of the split tiles' joint sequence (an XCD's workgroups are
-  // neighbours)
-  const uint32_t sw8 = g.sk_wgs >> 3, sk_w = xcd * sw8 + (blockIdx.x >> 3);
-  uint32_t s0 = 0, s1 = 0;
-  if (!ROWS128 && (blockIdx.x >> 3) < sw8) {
-    const uint32_t total = (g.tiles_m * g.tiles_k - ntile) * g.NB;
-    s0 = sk_w * g.sk_q < total ? sk_w * g.sk_q : total;
-    s1 = s0 + g.sk_q < total ? s0 + g.sk_q : total;
-  }
-#pragma unroll 1
-  for (;;) {
-    uint32_t t, nb0 = 0, len = g.NB, slot = 0;
-    if (ti < per_xcd) {
-      const uint32_t pos = ti;
-      ti += wgs_per_xcd;
-      if (g.tile_weight) {
-        const uint32_t band = xcd + 8u * (pos / band_tiles), in_band = pos % band_tiles;
-        if (band >= n_bands) { ti = per_xcd; continue; }
-        const uint32_t band_rows = (g.tiles_m - band * 4u) < 4u ? (g.tiles_m - band * 4u) : 4u;
-        if (in_band >= band_rows * g.tiles_k) continue;  // a last band with fewer than 4 row tiles
-        t = band * band_tiles + in_band;
-      } else {
-        t = xcd * per_xcd + pos;
-        if (t >= ntile) { ti = per_xcd; continue; }
-      }
-    } else if (s0 < s1) {
-      const uint32_t u = s0 / g.NB;
-      nb0 = s0 - u * g.NB;
-      len = s1 - s0 < g.NB - nb0 ? s1 - s0 : g.NB - nb0;
-      t = ntile + u;
-      slot = sk_w + u;
-      s0 += len;
-    } else {
-      break;
-    }
+  bwd_dx_schedule(g, !ROWS128, [&](uint32_t t, int nb0, int len, uint32_t slot) {
     uint32_t tm, tk;
     bwd_dx_tile_at(g, t, tm, tk);
-    segment(tm, tk, (int)nb0, (int)len, len == g.NB, slot);
+    segment(tm, tk, nb0, len, len == (int)g.NB, slot);
+  });
+}
+
+// The 256 x 256 geometry: four waves, one to a SIMD, side by side along k: a wave tile of 256 rows x 64 k (8 x 2 accumulator
+// blocks, 256 registers, beside 256 others).  No two waves then convert the same weight blocks, which as eight waves of
+// 128 x 64 every two did: 2 transposing MFMAs and 80 vector instructions for 32 MFMAs instead of 16.  What a
+// second wave per SIMD hid is hidden by order: the conversion of the next stage's blocks stands between single MFMAs, the dy
+// fragments are read three pairs ahead, and a barrier comes every two stages.
+// ROWS: row blocks multiplied (8, or 4 where the tile holds no more: the others' dy is loaded from block 0 and left alone).
+// @MEASURED@
+constexpr int kBwdWideLoads = 7;  // direct-to-LDS loads per wave and stage: 4 panel chunks, 2 weight blocks, scales
+
+// The accumulator tied, as one read-write operand, in the half of the register file that is named: left to the compiler, or all
+// in one half, up to a half of the sixteen sets was moved between the halves at every pass of the loop (540 moves for 64 MFMAs).
+// The compiler does not see that an MFMA writes the sums: they are next touched by the MFMA of the other half block or
+// of the next stage, and the epilogue stands behind explicit wait states.
+template <bool HIGH>
+__device__ inline void bwd_mfma(v16f& acc, const v8bf& a, const v8bf& b) {
+  if constexpr (HIGH) asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
+  else asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "v"(b));
+}
+// The sums for the vector ALU.  (As plain values their uses behind the loop drew the sums into the other half within it.)
+template <bool HIGH>
+__device__ inline v16f bwd_sums(v16f& acc) {
+  v16f y;
+  if constexpr (HIGH) {
+#pragma unroll
+    for (int e = 0; e < 16; ++e) asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(y[e]) : "a"(acc[e]));
+  } else {
+    asm volatile("" : "+v"(acc));  // (behind the wait states, too)
+    y = acc;
   }
+  return y;
+}
+// W[n][k] of a 32 x 32 block in vector registers (the builtin's result lands in the half that the sums fill); not to be read for
+// 19 wait states.
+__device__ inline void bwd_transpose(v16i& tr, const v4i& raw, const v4i& ident) {
+  asm volatile("v_mfma_i32_32x32x32_i8 %0, %1, %2, 0" : "=&v"(tr) : "v"(raw), "v"(ident));
+}
+
+template <int NKK>
+__global__ __launch_bounds__(256, 1) void bwd_dx_wide_kernel(BwdDxArgs g) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = lane & 31, h = lane >> 5;
+  const uint32_t lane16 = (uint32_t)lane * 16u;
+  v4i ident = {0, 0, 0, 0};  // identity operand of the transposing MFMA: lane (column c, k half h) holds byte 1 at k == c
+  {
+    const int word = ((c >> 4) == h) ? (int)(1u << (8 * (c & 3))) : 0;
+    const int wi = (c & 15) >> 2;
+    ident[0] = wi == 0 ? word : 0; ident[1] = wi == 1 ? word : 0;
+    ident[2] = wi == 2 ? word : 0; ident[3] = wi == 3 ? word : 0;
+  }
+  const uint32_t lds_base = (uint32_t)(uintptr_t)(lptr_t)lds;
+
+  // stages nb0 .. nb0 + L - 1 (an even number) of a tile: all of them (whole), or partial sums for slot `slot`
+  auto segment = [&](auto rows_tag, uint32_t tm, uint32_t tk, int live_blocks, int tw, int nb0, int L, bool whole, uint32_t slot) {
+    constexpr int ROWS = decltype(rows_tag)::value;
+    const float* swp_t = g.swp + (size_t)tw * g.sw_stride;
+    // this wave's loads of a stage: dy of two row blocks (both halves), two weight blocks
+    const uint32_t rb0 = 2u * (uint32_t)wave < (uint32_t)live_blocks ? 2u * (uint32_t)wave : 0u;
+    const uint32_t rb1 = 2u * (uint32_t)wave + 1u < (uint32_t)live_blocks ? 2u * (uint32_t)wave + 1u : 0u;
+    const unsigned char* Ag0 = g.dyp + ((size_t)(tm * 8u + rb0) * g.NB) * 2048u;
+    const unsigned char* Ag1 = g.dyp + ((size_t)(tm * 8u + rb1) * g.NB) * 2048u;
+    const uint32_t kbw = tk * 8u + 2u * (uint32_t)wave;  // its two k blocks (blocks past the weight repeat the last)
+    const unsigned char* Wt = g.wp + (size_t)tw * g.w_stride;
+    const unsigned char* Bg0 = Wt + (size_t)(kbw < g.KB ? kbw : g.KB - 1u) * kBlockBytes;
+    const unsigned char* Bg1 = Wt + (size_t)(kbw + 1u < g.KB ? kbw + 1u : g.KB - 1u) * kBlockBytes;
+    const size_t nb_stride = (size_t)g.KB * kBlockBytes;
+    // Load j of the seven of stage i (behind the last stage: of that one again).  Loads the compiler keeps no books on: it
+    // would drain them before every read of the LDS.
+    auto issue = [&](int i, int j) {
+      const uint32_t st = lds_base + (i % kBwdStages) * kBwdStageBytes;
+      const int nb = nb0 + (i < L ? i : L - 1);
+      if (j < 4) lds_load_1k((j < 2 ? Ag0 : Ag1) + (size_t)nb * 2048u + 1024 * (j & 1), lane16, st + (wave * 4 + j) * kBlockBytes);
+      else if (j < 6) lds_load_1k((j == 4 ? Bg0 : Bg1) + (size_t)nb * nb_stride, lane16, st + kBwdStagePanel + (wave * 2 + j - 4) * kBlockBytes);
+      else lds_load_1k(reinterpret_cast<const unsigned char*>(swp_t + 32 * nb), lane16, st + kBwdStagePanel + kBwdStageWeight);
+    };
+    v16f acc[ROWS][2];
+#pragma unroll
+    for (int i = 0; i < ROWS; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+
+    struct NextRegs { v4i raw[2]; v4f s4[4]; };
+    // (explicit instructions: see bwd_dx_kernel)
+    auto next_read = [&](int i, NextRegs& r) {
+      const uint32_t st = lds_base + (i % kBwdStages) * kBwdStageBytes + kBwdStagePanel;
+      const uint32_t wa = st + (wave * 2) * kBlockBytes + lane16;
+      const uint32_t sa = st + kBwdStageWeight + 16 * h;
+      asm volatile("ds_read_b128 %0, %6\n\tds_read_b128 %1, %6 offset:1024\n\t"
+                   "ds_read_b128 %2, %7\n\tds_read_b128 %3, %7 offset:32\n\t"
+                   "ds_read_b128 %4, %7 offset:64\n\tds_read_b128 %5, %7 offset:96\n\t"
+                   "s_waitcnt lgkmcnt(0)"
+                   : "=&v"(r.raw[0]), "=&v"(r.raw[1]), "=&v"(r.s4[0]), "=&v"(r.s4[1]), "=&v"(r.s4[2]), "=&v"(r.s4[3])
+                   : "v"(wa), "v"(sa)
+                   : "memory");
+    };
+    // rows 8 (t / 2) + 4 h + 2 (t % 2) + 0, 1 of a transposed block: bf16(float(code) * scale), the per-element
+    // weight of the reference's pull-back
+    auto convert2 = [&](const v16i& tr, const v4f (&s4)[4], int t, uint32_t (&pk)[8]) {
+      const float f0 = (float)tr[2 * t] * s4[t >> 1][2 * (t & 1)], f1 = (float)tr[2 * t + 1] * s4[t >> 1][2 * (t & 1) + 1];
+      pk[t] = pack_bf16x2(f0, f1);
+    };
+    auto to_operands = [&](const uint32_t (&pk)[8], v8bf (&bq)[2]) {
+      bq[0] = __builtin_bit_cast(v8bf, v4i{(int)pk[0], (int)pk[1], (int)pk[2], (int)pk[3]});
+      bq[1] = __builtin_bit_cast(v8bf, v4i{(int)pk[4], (int)pk[5], (int)pk[6], (int)pk[7]});
+    };
+    constexpr int kPairs = 2 * ROWS;  // (half q, row block) of a stage
+    auto panel_frag = [&](int i, int pair) -> v8bf {
+      typedef __attribute__((address_space(3))) const v4i* lds_v4ptr;
+      const uint32_t at = lds_base + (i % kBwdStages) * kBwdStageBytes + lane16;
+      return __builtin_bit_cast(v8bf, *reinterpret_cast<lds_v4ptr>((uintptr_t)(at + ((pair % ROWS) * 2 + pair / ROWS) * kBlockBytes)));
+    };
+    // One stage: its MFMAs from the dy panel in the LDS; between them the operands of stage i + 1 are prepared.
+    // af: the fragments of the first three pairs; leaves those of stage i + 1 there where that one has landed (ahead).
+    auto stage = [&](int i, const v8bf (&bqC)[2][2], v8bf (&bqN)[2][2], bool ahead, v8bf (&af)[4]) {
+      NextRegs nx;
+      v16i tr;
+      uint32_t pk[8];
+      asm volatile("s_nop 3");  // (operands converted at the end of the stage before)
+      next_read(i + 1, nx);
+      // pairs behind which the two blocks are transposed; their conversion starts behind three more MFMAs, when the result is there
+      constexpr int kT0 = ROWS == 8 ? 1 : 0, kT1 = ROWS == 8 ? 7 : 3;
+      constexpr int kPer = ROWS == 8 ? 1 : 2;  // conversion steps (of 8 a block) in each half of a pair
+      auto convert_part = [&](int pair, int half) {
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+          const int t0 = (b ? kT1 : kT0) + 2;
+          if (pair == t0 && half == 0) asm volatile("" : "+v"(tr));  // (not read before this place)
+#pragma unroll
+          for (int u = 0; u < kPer; ++u) {
+            const int t = ((pair - t0) * 2 + half) * kPer + u;
+            if (pair >= t0 && t < 8) {
+              convert2(tr, nx.s4, t, pk);
+              if (t == 7) to_operands(pk, bqN[b]);
+            }
+          }
+        }
+      };
+#pragma unroll
+      for (int pair = 0; pair < kPairs; ++pair) {
+        const int q = pair / ROWS, rb = pair % ROWS;
+        if (rb < 4) bwd_mfma<true>(acc[rb][0], af[pair & 3], bqC[0][q]);
+        else bwd_mfma<false>(acc[rb][0], af[pair & 3], bqC[0][q]);
+        if (pair + 3 < kPairs) af[(pair + 3) & 3] = panel_frag(i, pair + 3);
+        else if (ahead) af[(pair + 3) & 3] = panel_frag(i + 1, pair + 3 - kPairs);
+        convert_part(pair, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        if (rb < 4) bwd_mfma<true>(acc[rb][1], af[pair & 3], bqC[1][q]);
+        else bwd_mfma<false>(acc[rb][1], af[pair & 3], bqC[1][q]);
+        if (pair % (ROWS / 4) == 0 && pair / (ROWS / 4) < kBwdWideLoads) issue(i + 4, pair / (ROWS / 4));
+        convert_part(pair, 1);
+        if (pair == kT0) bwd_transpose(tr, nx.raw[0], ident);
+        if (pair == kT1) bwd_transpose(tr, nx.raw[1], ident);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+
+    v8bf bqA[2][2], bqB[2][2], af[4];
+    wait_vmcnt<0>();  // stores of the previous tile
+    lds_barrier();
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < kBwdWideLoads; ++j) issue(i, j);
+    wait_vmcnt<0>();
+    lds_barrier();
+    {  // operands of stage 0
+      NextRegs nx;
+      next_read(0, nx);
+      uint32_t pk[8];
+#pragma unroll
+      for (int cb = 0; cb < 2; ++cb) {
+        v16i tr;
+        bwd_transpose(tr, nx.raw[cb], ident);
+        asm volatile("s_nop 15\n\ts_nop 15" : "+v"(tr));
+#pragma unroll
+        for (int t = 0; t < 8; ++t) convert2(tr, nx.s4, t, pk);
+        to_operands(pk, bqA[cb]);
+      }
+    }
+    // Two stages to a barrier: stages i and i + 1 and the weight of i + 2 have landed, i + 4 and i + 5 are asked for
+    // (into the slots of i - 2 and i - 1).
+    // (one loop for all stages: those behind the last are loads and a conversion that nothing reads, and a second loop made
+    // the allocator move a third of the sums at every pass of this one)
+#pragma unroll 1
+    for (int i = 0; i < L; i += 2) {
+      wait_vmcnt<kBwdWideLoads>();
+      lds_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int p = 0; p < 3; ++p) af[p] = panel_frag(i, p);
+      __builtin_amdgcn_sched_barrier(0);
+      stage(i, bqA, bqB, true, af);
+      stage(i + 1, bqB, bqA, false, af);
+    }
+    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");  // the last MFMAs, which the compiler does not know, have written their sums
+    auto sums = [&](int rb, v16f& a) -> v16f { return rb < 4 ? bwd_sums<true>(a) : bwd_sums<false>(a); };
+    if (whole) {
+#pragma unroll
+      for (int rb = 0; rb < ROWS; ++rb)
+        if (rb < live_blocks) {
+          const v16f y[2] = {sums(rb, acc[rb][0]), sums(rb, acc[rb][1])};
+          bwd_dx_store_block<NKK, 2>(g, tm * 256u + rb * 32u, kbw, y);
+        }
+    } else {
+#pragma unroll
+      for (int rb = 0; rb < ROWS; ++rb)
+        if (rb < live_blocks) {
+          float4* dst = bwd_dx_part<2>(g, slot, (uint32_t)rb, (uint32_t)wave);
+#pragma unroll
+          for (int cb = 0; cb < 2; ++cb) {
+            const v16f y = sums(rb, acc[rb][cb]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) dst[(cb * 4 + e) * 64] = make_float4(y[4 * e], y[4 * e + 1], y[4 * e + 2], y[4 * e + 3]);
+          }
+        }
+    }
+  };
+
+  bwd_dx_schedule(g, true, [&](uint32_t t, int nb0, int len, uint32_t slot) {
+    uint32_t tm, tk;
+    bwd_dx_tile_at(g, t, tm, tk);
+    int tw = 0, live = ((int)(g.M - tm * 256u) + 31) / 32;  // (the rows of a dense call fill the slots from the first)
+    if (g.tile_weight) {
+      const int tv = g.tile_weight[tm];
+      if (tv < 0) return;  // workgroup-uniform: no row lives in this tile
+      tw = tv & 0xffff;
+      live = ((tv >> 16) + 31) / 32;
+    }
+    live = __builtin_amdgcn_readfirstlane(live < 8 ? live : 8);
+    if (live > 4) segment(std::integral_constant<int, 8>{}, tm, tk, live, tw, nb0, len, len == (int)g.NB, slot);
+    else segment(std::integral_constant<int, 4>{}, tm, tk, live, tw, nb0, len, len == (int)g.NB, slot);
+  });
 }
 
 // The split tiles of a pull-back kernel: the partial sums of a tile added in the order of its stages, then the
