@@ -505,60 +505,103 @@ __device__ inline void bwd_dx_tile_at(const BwdDxArgs& g, uint32_t t, uint32_t& 
   tk = in_band / band_rows;
 }
 
-// A wave's block of dx, 32 rows x CBN k blocks: + rs @ A.T, one cast, rows back to their original positions.
-// pbase: first slot of the block's 32; kbw: first of its k blocks.
-template <int NKK, int CBN>
-__device__ inline void bwd_dx_store_block(const BwdDxArgs& g, uint32_t pbase, uint32_t kbw, const v16f (&acc)[CBN]) {
+// A wave's ROWS row blocks of dx, of CBN k blocks each: + rs @ A.T, one cast, rows back to their original positions.
+// pbase: first slot; kbw: first k block; live: row blocks that hold rows; sums(rb, cb): the sums of a block; turn: 32 rows of
+// kBwdTurnStride bytes of the LDS that are the wave's own.
+// A block's values are turned in the LDS so that eight lanes store a row's 128 bytes: from the accumulator layout a row went
+// out two bytes a lane, 32 stores a block instead of 4.  rs_lds: where in the LDS the operands of rs of the row blocks lie, one
+// behind the other (bwd_dx_fetch_rs, whose loads all waves of a tile share and wait for once), or 0: in memory.
+// With 2-byte stores and every block waiting for its own operands a whole 256 x 256 tile's epilogue took 39 us (rank 32), now 15.
+constexpr uint32_t kBwdTurnStride = 144;  // bytes of a row: 64 values and 16 more, so that rows start on different banks
+constexpr uint32_t kBwdTurnBytes = 32u * kBwdTurnStride;
+template <int NKK, int CBN, int ROWS, bool RS_LDS, class Sums>
+__device__ inline __attribute__((always_inline)) void bwd_dx_store(const BwdDxArgs& g, uint32_t pbase, uint32_t kbw, int live, uint32_t turn, uint32_t rs_lds, Sums&& sums) {
+  typedef __attribute__((address_space(3))) uint16_t* lds_u16;
+  typedef __attribute__((address_space(3))) const v4i* lds_cv4;
+  constexpr int kKK = NKK > 0 ? NKK : 1;
   int lane = threadIdx.x & 63;
   // (opaque: what the epilogue derives from it is formed here and not held in registers through the stages)
   asm volatile("" : "+v"(lane));
   const int c = lane & 31, h = lane >> 5;
-  const uint32_t blk = pbase / 32u;
-  const int src_lane = g.src_row ? g.src_row[pbase + c] : (int)(pbase + c);
-  const bool row_ok = src_lane >= 0 && src_lane < (int)g.M;
-  const uint32_t off_lane = row_ok ? (uint32_t)src_lane * g.K : 0xffffffffu;
-  if (__builtin_amdgcn_ballot_w64(row_ok) == 0) return;  // wave-uniform: no row of this block exists
-  const uint32_t range = (NKK > 0 && g.blk_range) ? (uint32_t)g.blk_range[blk] : 0u;
-  const int glo = (int)(range & 0xffffu), ghi = (int)(range >> 16);
-  const int grp_lane = (NKK > 0 && g.slot_group && ghi > glo) ? g.slot_group[pbase + c] : glo;
-  const int row_addr = 16 * h;
-  for (int gi = glo; gi <= ghi; ++gi) {  // a block at a group boundary runs once per group
+  int src[ROWS];  // original row of slot c of every block
+#pragma unroll
+  for (int rb = 0; rb < ROWS; ++rb) {
+    const uint32_t p = pbase + 32u * (uint32_t)(rb < live ? rb : 0) + (uint32_t)c;
+    src[rb] = g.src_row ? g.src_row[p] : (int)p;
+  }
+  v8us ab[CBN][kKK];
+  auto operand_r = [&](int rb, int chunk) -> v8bf {
+    if constexpr (RS_LDS) return __builtin_bit_cast(v8bf, *reinterpret_cast<lds_cv4>((uintptr_t)(rs_lds + (uint32_t)(rb * kKK * 3 + chunk) * kBlockBytes + (uint32_t)lane * 16u)));
+    return __builtin_bit_cast(v8bf, *reinterpret_cast<const v8us*>(g.rp + ((size_t)(pbase / 32u + (uint32_t)rb) * (uint32_t)(kKK * 3) + (uint32_t)chunk) * kBlockBytes + lane * 16));
+  };
+  int held = -1;  // group whose A operands are in ab
+  auto fetch_a = [&](int gi) {
 #pragma unroll
     for (int cb = 0; cb < CBN; ++cb) {
-      const uint32_t kb = kbw + cb;
-      if (kb >= g.KB) continue;  // wave-uniform
-      const uint32_t kcol = kb * 32u + c;
-      v16f y = acc[cb];
-      if constexpr (NKK > 0) {
-        const unsigned char* rb0 = g.rp + (size_t)blk * NKK * 3u * kBlockBytes + lane * 16;
-        const unsigned char* ab0 = g.ap + ((size_t)gi * g.KB + kb) * NKK * kBlockBytes + lane * 16;
-        v16f low;
+      const uint32_t kb = kbw + (uint32_t)cb < g.KB ? kbw + (uint32_t)cb : g.KB - 1u;
+      const unsigned char* a0 = g.ap + ((size_t)gi * g.KB + kb) * (uint32_t)kKK * kBlockBytes + lane * 16;
 #pragma unroll
-        for (int e = 0; e < 16; ++e) low[e] = 0.0f;
+      for (int kk = 0; kk < kKK; ++kk) ab[cb][kk] = *reinterpret_cast<const v8us*>(a0 + kk * kBlockBytes);
+    }
+    held = gi;
+  };
 #pragma unroll
-        for (int kk = 0; kk < NKK; ++kk) {
-          const v8bf ab = __builtin_bit_cast(v8bf, *reinterpret_cast<const v8us*>(ab0 + kk * kBlockBytes));
+  for (int rb = 0; rb < ROWS; ++rb) {
+    if (rb >= live) break;  // wave-uniform
+    const uint32_t blk = pbase / 32u + (uint32_t)rb;
+    const bool row_ok = src[rb] >= 0 && src[rb] < (int)g.M;
+    if (__builtin_amdgcn_ballot_w64(row_ok) == 0) continue;  // wave-uniform: no row of this block exists
+    const uint32_t range = (NKK > 0 && g.blk_range) ? (uint32_t)g.blk_range[blk] : 0u;
+    const int glo = (int)(range & 0xffffu), ghi = (int)(range >> 16);
+    const int grp = (NKK > 0 && g.slot_group && ghi > glo) ? g.slot_group[blk * 32u + (uint32_t)c] : glo;
+    for (int gi = glo; gi <= ghi; ++gi) {  // a block at a group boundary runs once per group
+      if (NKK > 0 && gi != held) fetch_a(gi);  // wave-uniform
 #pragma unroll
-          for (int t3 = 2; t3 >= 0; --t3) {
-            const v8bf rf = __builtin_bit_cast(v8bf, *reinterpret_cast<const v8us*>(rb0 + (kk * 3 + t3) * kBlockBytes));
-            low = __builtin_amdgcn_mfma_f32_32x32x16_bf16(rf, ab, low, 0, 0, 0);
-          }
+      for (int cb = 0; cb < CBN; ++cb) {
+        v16f y = sums(rb, cb);
+        if constexpr (NKK > 0) {
+          v16f low;
+#pragma unroll
+          for (int e = 0; e < 16; ++e) low[e] = 0.0f;
+#pragma unroll
+          for (int kk = 0; kk < NKK; ++kk)
+#pragma unroll
+            for (int t3 = 2; t3 >= 0; --t3)
+              low = __builtin_amdgcn_mfma_f32_32x32x16_bf16(operand_r(rb, kk * 3 + t3), __builtin_bit_cast(v8bf, ab[cb][kk]), low, 0, 0, 0);
+          asm volatile("" : "+v"(low));
+#pragma unroll
+          for (int e = 0; e < 16; ++e) y[e] = y[e] + low[e];
         }
 #pragma unroll
-        for (int e = 0; e < 16; ++e) y[e] = y[e] + low[e];
+        for (int v = 0; v < 16; ++v)
+          *reinterpret_cast<lds_u16>((uintptr_t)(turn + (uint32_t)(8 * (v >> 2) + 4 * h + (v & 3)) * kBwdTurnStride + (uint32_t)(cb * 64 + 2 * c))) =
+              (uint16_t)f32_to_bf16_bits(y[v]);
       }
+      // (a wave's LDS operations are in order, so the reads find the writes and the next block's writes come behind them)
+      constexpr int kPieces = 4 * CBN;  // of 16 bytes of a row
 #pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int src_lane_addr = row_addr + 4 * (8 * (v >> 2) + (v & 3));
-        const uint32_t rowoff = (uint32_t)__builtin_amdgcn_ds_bpermute(src_lane_addr, (int)off_lane);
-        // every lane takes part in the cross-lane reads: a lane that is switched off (a column
-        // beyond K) would hand zeros to the lanes that read from it
+      for (int t = 0; t < kPieces / 2; ++t) {
+        const int row = lane / kPieces + (64 / kPieces) * t, piece = lane % kPieces;
+        const v4i v = *reinterpret_cast<lds_cv4>((uintptr_t)(turn + (uint32_t)row * kBwdTurnStride + (uint32_t)piece * 16u));
+        const int m = __builtin_amdgcn_ds_bpermute(4 * row, src[rb]);
         int row_grp = gi;
-        if (NKK > 0 && ghi > glo) row_grp = __builtin_amdgcn_ds_bpermute(src_lane_addr, grp_lane);
-        const bool ok = (rowoff != 0xffffffffu) & (kcol < g.K) & (row_grp == gi);
-        if (ok) g.dx[(size_t)rowoff + kcol] = (uint16_t)f32_to_bf16_bits(y[v]);
+        if (NKK > 0 && ghi > glo) row_grp = __builtin_amdgcn_ds_bpermute(4 * row, grp);
+        const uint32_t k = kbw * 32u + 8u * (uint32_t)piece;  // (K is a multiple of 8)
+        if (m >= 0 && m < (int)g.M && k < g.K && row_grp == gi) *reinterpret_cast<v4i*>(g.dx + (uint32_t)m * g.K + k) = v;
       }
     }
+  }
+}
+
+// The operands of rs of a tile's row blocks into the LDS, by all its waves; waits for them.  Everybody is done with what lay there.
+template <int NKK>
+__device__ inline void bwd_dx_fetch_rs(const BwdDxArgs& g, uint32_t pbase, int blocks, uint32_t rs_lds, int wave, int waves) {
+  if constexpr (NKK > 0) {
+    const unsigned char* src = g.rp + (size_t)(pbase / 32u) * (uint32_t)(NKK * 3) * kBlockBytes;
+    for (int ch = wave; ch < blocks * NKK * 3; ch += waves)
+      lds_load_1k(src + (size_t)ch * kBlockBytes, (threadIdx.x & 63u) * 16u, rs_lds + (uint32_t)ch * kBlockBytes);
+    wait_vmcnt<0>();
+    lds_barrier();
   }
 }
 
@@ -665,7 +708,7 @@ __device__ inline __attribute__((always_inline)) void bwd_dx_schedule(const BwdD
 // and every wave has rows.
 //
 // The 256 registers that two waves per SIMD leave are the kernel's limit: the loads' addresses are a scalar base plus the
-// lane's offset (issue), and the epilogue derives its lane constants for itself (bwd_dx_store_block).  Held in vector
+// lane's offset (issue), and the epilogue derives its lane constants for itself (bwd_dx_store).  Held in vector
 // registers through the stages both cost 44 bytes of scratch per lane (16 with ROWS128).  Spilling / as it is, pull-back and
 // what goes before it: 2048 x 2560, N = 10240, rank 64 211 / 205 us; 512 x 2560, N = 6144 78.0 / 74.9; 4096 x 4096,
 // N = 24576 947 / 946 (whole tiles: the reloads stand outside the stages); 8168 rows of 128 experts, 2048 <- 1536 207 / 204.
@@ -694,20 +737,23 @@ __global__ __launch_bounds__(512, 1) void bwd_dx_kernel(BwdDxArgs g) {
   auto segment = [&](uint32_t tm, uint32_t tk, int nb0, int L, bool whole, uint32_t slot) {
     int tw = 0;
     int n_act = 4;  // 32-row blocks of this wave that hold rows: the others skip their matrix-core work
+    int live_blocks;  // ... of the tile
     // row block whose dy panel this wave fetches: both 1 KiB halves, or one half of it in a 128-row tile
     uint32_t load_rb = ROWS128 ? (uint32_t)wave >> 1 : (uint32_t)wave;
     if (g.tile_weight) {
       const int tv = g.tile_weight[tm];
       if (tv < 0) return;  // workgroup-uniform: no row lives in this tile
       tw = tv & 0xffff;
-      const int live_blocks = ((tv >> 16) + 31) / 32;
+      live_blocks = ((tv >> 16) + 31) / 32;
       const int live = live_blocks - wrow * 4;
       n_act = live < 0 ? 0 : (live > 4 ? 4 : live);
       // a block without rows is never multiplied: its slot is filled from block 0 of the tile, which
       // is in the caches anyway, instead of streaming unused memory (the load count stays the same)
       if ((int)load_rb >= live_blocks) load_rb = 0u;
     } else {  // (the rows of a dense call fill the slots from the first)
-      const int live = ((int)(g.M - tm * (uint32_t)(kRowBlocks * 32)) + 31) / 32 - wrow * 4;
+      live_blocks = ((int)(g.M - tm * (uint32_t)(kRowBlocks * 32)) + 31) / 32;
+      live_blocks = live_blocks > kRowBlocks ? kRowBlocks : live_blocks;
+      const int live = live_blocks - wrow * 4;
       n_act = live < 0 ? 0 : (live > 4 ? 4 : live);
     }
     n_act = __builtin_amdgcn_readfirstlane(n_act);
@@ -857,10 +903,12 @@ __global__ __launch_bounds__(512, 1) void bwd_dx_kernel(BwdDxArgs g) {
         [&](int i, bool more) { stage(i, bqA, bqB, more); }, [&](int i, bool more) { stage(i, bqB, bqA, more); });
 
     if (whole) {
-#pragma unroll
-      for (int rb = 0; rb < 4; ++rb)
-        if (rb < n_act)
-          bwd_dx_store_block<NKK, 2>(g, tm * (uint32_t)(kRowBlocks * 32) + (uint32_t)wrow * 128u + rb * 32u, kbw, acc[rb]);
+      lds_barrier();  // (every wave has read its last stage)
+      const uint32_t rs_lds = lds_base + 8u * kBwdTurnBytes;
+      bwd_dx_fetch_rs<NKK>(g, tm * (uint32_t)(kRowBlocks * 32), live_blocks, rs_lds, wave, 8);
+      if (n_act)
+        bwd_dx_store<NKK, 2, 4, true>(g, tm * (uint32_t)(kRowBlocks * 32) + (uint32_t)wrow * 128u, kbw, n_act, lds_base + (uint32_t)wave * kBwdTurnBytes,
+                                      rs_lds + (uint32_t)(wrow * 4 * NKK * 3) * kBlockBytes, [&](int rb, int cb) -> v16f { return acc[rb][cb]; });
     } else {
 #pragma unroll
       for (int rb = 0; rb < 4; ++rb)
@@ -888,7 +936,8 @@ __global__ __launch_bounds__(512, 1) void bwd_dx_kernel(BwdDxArgs g) {
 // second wave per SIMD hid is hidden by order: the conversion of the next stage's blocks stands between single MFMAs, the dy
 // fragments are read three pairs ahead, and a barrier comes every two stages.
 // ROWS: row blocks multiplied (8, or 4 where the tile holds no more: the others' dy is loaded from block 0 and left alone).
-// @MEASURED@
+// Power more than issue bounds it (all-zero dy runs a quarter faster).  3003 x 4096, N = 24576, rank 32: 663 us as eight waves of 128 x 64, now
+// 508 (1.19 PFLOP/s); 3003 x 12288, N = 4096 378 / 285, of which the epilogue below 45; 2048 x 2560, N = 10240, rank 64 131 / 105.
 constexpr int kBwdWideLoads = 7;  // direct-to-LDS loads per wave and stage: 4 panel chunks, 2 weight blocks, scales
 
 // The accumulator tied, as one read-write operand, in the half of the register file that is named: left to the compiler, or all
@@ -925,7 +974,6 @@ __global__ __launch_bounds__(256, 1) void bwd_dx_wide_kernel(BwdDxArgs g) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 31, h = lane >> 5;
-  const uint32_t lane16 = (uint32_t)lane * 16u;
   v4i ident = {0, 0, 0, 0};  // identity operand of the transposing MFMA: lane (column c, k half h) holds byte 1 at k == c
   {
     const int word = ((c >> 4) == h) ? (int)(1u << (8 * (c & 3))) : 0;
@@ -938,6 +986,11 @@ __global__ __launch_bounds__(256, 1) void bwd_dx_wide_kernel(BwdDxArgs g) {
   // stages nb0 .. nb0 + L - 1 (an even number) of a tile: all of them (whole), or partial sums for slot `slot`
   auto segment = [&](auto rows_tag, uint32_t tm, uint32_t tk, int live_blocks, int tw, int nb0, int L, bool whole, uint32_t slot) {
     constexpr int ROWS = decltype(rows_tag)::value;
+    // (opaque: the addresses derived from it are formed per segment.  Formed once for the kernel they were spilled, and a
+    // reload in front of the loop has the compiler drain every load at its first use in it)
+    int lane_s = lane;
+    asm volatile("" : "+v"(lane_s));
+    const uint32_t lane16 = (uint32_t)lane_s * 16u, h16 = (uint32_t)(lane_s >> 5) * 16u;
     const float* swp_t = g.swp + (size_t)tw * g.sw_stride;
     // this wave's loads of a stage: dy of two row blocks (both halves), two weight blocks
     const uint32_t rb0 = 2u * (uint32_t)wave < (uint32_t)live_blocks ? 2u * (uint32_t)wave : 0u;
@@ -971,7 +1024,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dx_wide_kernel(BwdDxArgs g) {
     auto next_read = [&](int i, NextRegs& r) {
       const uint32_t st = lds_base + (i % kBwdStages) * kBwdStageBytes + kBwdStagePanel;
       const uint32_t wa = st + (wave * 2) * kBlockBytes + lane16;
-      const uint32_t sa = st + kBwdStageWeight + 16 * h;
+      const uint32_t sa = st + kBwdStageWeight + h16;
       asm volatile("ds_read_b128 %0, %6\n\tds_read_b128 %1, %6 offset:1024\n\t"
                    "ds_read_b128 %2, %7\n\tds_read_b128 %3, %7 offset:32\n\t"
                    "ds_read_b128 %4, %7 offset:64\n\tds_read_b128 %5, %7 offset:96\n\t"
@@ -1079,15 +1132,22 @@ __global__ __launch_bounds__(256, 1) void bwd_dx_wide_kernel(BwdDxArgs g) {
       stage(i, bqA, bqB, true, af);
       stage(i + 1, bqB, bqA, false, af);
     }
+    wait_vmcnt<0>();
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");  // the last MFMAs, which the compiler does not know, have written their sums
+#pragma unroll
+    for (int rb = 0; rb < ROWS; ++rb)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        if (rb < 4) asm volatile("" : "+a"(acc[rb][j]));
+        else asm volatile("" : "+v"(acc[rb][j]));
+      }
     auto sums = [&](int rb, v16f& a) -> v16f { return rb < 4 ? bwd_sums<true>(a) : bwd_sums<false>(a); };
     if (whole) {
-#pragma unroll
-      for (int rb = 0; rb < ROWS; ++rb)
-        if (rb < live_blocks) {
-          const v16f y[2] = {sums(rb, acc[rb][0]), sums(rb, acc[rb][1])};
-          bwd_dx_store_block<NKK, 2>(g, tm * 256u + rb * 32u, kbw, y);
-        }
+      lds_barrier();  // (every wave has read its last stage, and nothing is on its way into the LDS)
+      const uint32_t rs_lds = lds_base + 4u * kBwdTurnBytes;
+      bwd_dx_fetch_rs<NKK>(g, tm * 256u, live_blocks, rs_lds, wave, 4);
+      bwd_dx_store<NKK, 2, ROWS, true>(g, tm * 256u, kbw, live_blocks, lds_base + (uint32_t)wave * kBwdTurnBytes, rs_lds,
+                                       [&](int rb, int cb) -> v16f { return sums(rb, acc[rb][cb]); });
     } else {
 #pragma unroll
       for (int rb = 0; rb < ROWS; ++rb)
@@ -1123,6 +1183,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dx_wide_kernel(BwdDxArgs g) {
 // kernel's own epilogue.  A wave per block of 32 rows x CBN k blocks (CBN: k blocks of a wave's tile).
 template <int NKK, int CBN>
 __global__ __launch_bounds__(256) void bwd_dx_finish_kernel(BwdDxArgs g) {
+  __shared__ __attribute__((aligned(16))) unsigned char turn[4 * kBwdTurnBytes];
   const uint32_t item = blockIdx.x * 4u + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t u = item >> 5, wave = (item >> 2) & 7u, rb = item & 3u;
   const uint32_t first = u * g.NB / g.sk_q, last = ((u + 1u) * g.NB - 1u) / g.sk_q;
@@ -1147,7 +1208,8 @@ __global__ __launch_bounds__(256) void bwd_dx_finish_kernel(BwdDxArgs g) {
         y[cb][4 * e] += v.x; y[cb][4 * e + 1] += v.y; y[cb][4 * e + 2] += v.z; y[cb][4 * e + 3] += v.w;
       }
   }
-  bwd_dx_store_block<NKK, CBN>(g, pbase, kbw, y);
+  bwd_dx_store<NKK, CBN, 1, false>(g, pbase, kbw, 1, (uint32_t)(uintptr_t)(lptr_t)turn + (threadIdx.x >> 6) * kBwdTurnBytes, 0u,
+                                   [&](int, int cb) -> v16f { return y[cb]; });
 }
 
 // ---------------------------------------------------------------------------------------

@@ -273,12 +273,13 @@ __global__ __launch_bounds__(512, 1) void gq_bwd_dx_kernel(GqBwdDxArgs a) {
 
     const uint32_t kbw = kb0 + (uint32_t)wcol;
     if (whole) {
-#pragma unroll
-      for (int rb = 0; rb < 4; ++rb)
-        if (rb < n_act) {
-          const v16f one[1] = {acc[rb]};
-          bwd_dx_store_block<NKK, 1>(g, tm * 256u + (uint32_t)wrow * 128u + rb * 32u, kbw, one);
-        }
+      lds_barrier();  // (every wave has read its last stage)
+      const uint32_t rs_lds = lds_base + 8u * kBwdTurnBytes;
+      const int live = ((int)(g.M - tm * 256u) + 31) / 32;
+      bwd_dx_fetch_rs<NKK>(g, tm * 256u, live < 8 ? live : 8, rs_lds, wave, 8);
+      if (n_act)
+        bwd_dx_store<NKK, 1, 4, true>(g, tm * 256u + (uint32_t)wrow * 128u, kbw, n_act, lds_base + (uint32_t)wave * kBwdTurnBytes,
+                                      rs_lds + (uint32_t)(wrow * 4 * NKK * 3) * kBlockBytes, [&](int rb, int) -> v16f { return acc[rb]; });
     } else {
 #pragma unroll
       for (int rb = 0; rb < 4; ++rb)
