@@ -1100,11 +1100,11 @@ int launch_gq_bwd_dx_one(const GqBwdDxArgs& a, hipStream_t s) {
   const BwdDxArgs& g = a.g;
   uint32_t want = ((g.direct_tiles + 7u) / 8u) * 8u;
   if (g.sk_wgs > want) want = g.sk_wgs;
-  const dim3 grid(want < 256u ? want : 256u), block(512);
-  if (hipFuncSetAttribute(reinterpret_cast<const void*>(&gq_bwd_dx_kernel<W4, TERMS, NKK>),
+  const dim3 grid(want < 256u ? want : 256u), block(256);
+  if (hipFuncSetAttribute(reinterpret_cast<const void*>(&gq_bwd_dx_wide_kernel<W4, TERMS, NKK>),
                           hipFuncAttributeMaxDynamicSharedMemorySize, kGqBwdLdsBytes) != hipSuccess)
     return MI355_W8A8_ERR_LAUNCH;
-  hipLaunchKernelGGL((gq_bwd_dx_kernel<W4, TERMS, NKK>), grid, block, kGqBwdLdsBytes, s, a);
+  hipLaunchKernelGGL((gq_bwd_dx_wide_kernel<W4, TERMS, NKK>), grid, block, kGqBwdLdsBytes, s, a);
   if (!g.sk_wgs) return launch_status();
   if (const int st = launch_status()) return st;
   hipLaunchKernelGGL((bwd_dx_finish_kernel<NKK, 1>), dim3((g.tiles_m * g.tiles_k - g.direct_tiles) * 8u), dim3(256), 0, s, g);

@@ -6,7 +6,7 @@
 //   two terms when the scales are bf16 values (a code of at most 8 bits times 8 bits), three otherwise.
 //
 //   gq_bwd_pack_dy_kernel  dy in operand order, and the partial sums of r = dy @ B.T
-//   gq_bwd_dx_kernel       the pull-back
+//   gq_bwd_dx_wide_kernel  the pull-back
 // The rest (tables, r / z finish, LoRA cotangents) is the per-channel backward's.
 #pragma once
 #include "w8a8_backward.h"
@@ -84,23 +84,22 @@ __global__ __launch_bounds__(256) void gq_bwd_pack_dy_kernel(BwdPackDyArgs a) {
 }
 
 // ---------------------------------------------------------------------------------------
-// The pull-back.  Workgroup = 8 waves (2 along rows x 4 along k), tile 256 rows x 128 k, wave tile 128 x 32
-// (4 accumulator blocks of v_mfma_f32_32x32x16_bf16), contraction in stages of one 32-wide n block.  A stage's
+// The pull-back.  Workgroup = 4 waves side by side along k, one to a SIMD, tile 256 rows x 128 k, wave tile 256 x 32
+// (8 accumulator blocks of v_mfma_f32_32x32x16_bf16), contraction in stages of one 32-wide n block.  A stage's
 // dy panel (16 KiB), its four weight blocks (4 KiB, half that in 4-bit codes) and their scales (128 bytes a block)
-// travel L2 -> LDS with direct-to-LDS loads six stages ahead, three per wave.  While the matrix core works on
+// travel L2 -> LDS with direct-to-LDS loads four stages ahead, six per wave.  While the matrix core works on
 // a stage, each wave prepares its weight block of the next: transposed by the identity MFMA, scaled in float32,
-// split into TERMS bf16 operands.  The schedule is bwd_dx_kernel's; half its k per wave leaves the registers for
-// the terms, and a stage has as many MFMAs (TERMS = 2) for half the tile.
+// split into TERMS bf16 operands.  The order of things is bwd_dx_wide_kernel's; two row blocks take turns so that the terms'
+// MFMAs on one accumulator do not follow each other.
 // Bound by the matrix core and the term arithmetic beside it: 1536 rows, K = 12288, N = 4096, 8-bit codes, groups of
-// 64: 352 us (0.88 PFLOP/s of bf16 products in two terms) where the float32 library GEMM took 1096 us and the
-// dequantization and casts before it 250.
+// 64, two terms: 277 us, 1.12 PFLOP/s of bf16 products (as eight waves of 128 x 32, every two of which converted the same blocks, 322-337 us; the float32 library
+// GEMM took 1096 us and the dequantization and casts before it 250).
 // ---------------------------------------------------------------------------------------
-constexpr int kGqBwdStages = 7;
-constexpr int kGqBwdAhead = kGqBwdStages - 1;
+constexpr int kGqBwdStages = 6;
 constexpr int kGqBwdPanel = 16384, kGqBwdWeight = 4096;
 constexpr int kGqBwdStageBytes = kGqBwdPanel + kGqBwdWeight + 1024;
 constexpr int kGqBwdLdsBytes = kGqBwdStages * kGqBwdStageBytes;
-constexpr int kGqBwdLoads = 3;  // per wave and stage: 2 panel chunks, and weight blocks or scales
+constexpr int kGqBwdLoads = 6;  // per wave and stage: 4 panel chunks, a weight chunk, scales
 
 struct GqBwdDxArgs {
   BwdDxArgs g;          // wp: packed codes; KB: k blocks (k_pad / 32); NB: n blocks of dyp (even)
@@ -109,72 +108,69 @@ struct GqBwdDxArgs {
 };
 
 template <bool W4, int TERMS, int NKK>
-__global__ __launch_bounds__(512, 1) void gq_bwd_dx_kernel(GqBwdDxArgs a) {
+__global__ __launch_bounds__(256, 1) void gq_bwd_dx_wide_kernel(GqBwdDxArgs a) {
   const BwdDxArgs& g = a.g;
   extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wrow = wave >> 2, wcol = wave & 3;
-  const int c = lane & 31, h = lane >> 5;
   const uint32_t lds_base = (uint32_t)(uintptr_t)(lptr_t)lds;
   constexpr uint32_t kBlk8 = W4 ? 512u : 1024u;  // bytes of a weight block
-
   // identity operand of the transposing MFMA: lane (column c, k half h) holds byte 1 at k == c
   v4i ident = {0, 0, 0, 0};
   {
+    const int c = lane & 31, h = lane >> 5;
     const int word = ((c >> 4) == h) ? (int)(1u << (8 * (c & 3))) : 0;
     const int wi = (c & 15) >> 2;
     ident[0] = wi == 0 ? word : 0; ident[1] = wi == 1 ? word : 0;
     ident[2] = wi == 2 ? word : 0; ident[3] = wi == 3 ? word : 0;
   }
 
-  auto segment = [&](uint32_t tm, uint32_t tk, int nb0, int L, bool whole, uint32_t slot) {
-    int n_act = ((int)(g.M - tm * 256u) + 31) / 32 - wrow * 4;  // the wave's row blocks with rows
-    n_act = __builtin_amdgcn_readfirstlane(n_act < 0 ? 0 : (n_act > 4 ? 4 : n_act));
-    const unsigned char* panel = g.dyp + ((size_t)(tm * 8u + (uint32_t)wave) * g.NB) * 2048u + lane * 16;
+  // stages nb0 .. nb0 + L - 1 (an even number) of a tile: all of them (whole), or partial sums for slot `slot`; ROWS: row blocks
+  // multiplied, at least live_blocks
+  auto segment = [&](auto rows_tag, uint32_t tm, uint32_t tk, int live_blocks, int nb0, int L, bool whole, uint32_t slot) {
+    constexpr int ROWS = decltype(rows_tag)::value;
+    int lane_s = lane;
+    asm volatile("" : "+v"(lane_s));  // (what is derived from it is formed per segment: see bwd_dx_wide_kernel)
+    const uint32_t lane16 = (uint32_t)lane_s * 16u, h = (uint32_t)lane_s >> 5;
+    const uint32_t rb0 = 2u * (uint32_t)wave < (uint32_t)live_blocks ? 2u * (uint32_t)wave : 0u;
+    const uint32_t rb1 = 2u * (uint32_t)wave + 1u < (uint32_t)live_blocks ? 2u * (uint32_t)wave + 1u : 0u;
+    const unsigned char* Ag0 = g.dyp + ((size_t)(tm * 8u + rb0) * g.NB) * 2048u;
+    const unsigned char* Ag1 = g.dyp + ((size_t)(tm * 8u + rb1) * g.NB) * 2048u;
     const uint32_t kb0 = tk * 4u;
     auto clamp_kb = [&](uint32_t kb) { return kb < g.KB ? kb : g.KB - 1u; };
-    // what this wave fetches beside the panel: waves 0..3 the weight blocks (one each, or in 4-bit codes two
-    // of 512 bytes, waves 2 and 3 repeating 0 and 1), waves 4..7 the four blocks' scales (each all of them, to
-    // the same place)
-    uint32_t w_off, w_dst;  // of waves 0..3: byte offset inside an n block's row of blocks
-    if (W4) {
-      w_off = clamp_kb(kb0 + 2u * (wave & 1) + (uint32_t)h) * 512u + (lane & 31) * 16u;
-      w_dst = (wave & 1) * 1024u;
-    } else {
-      w_off = clamp_kb(kb0 + (wave & 3)) * 1024u + lane * 16u;
-      w_dst = (wave & 3) * 1024u;
-    }
-    const uint32_t s_piece = (lane & 7) * 4u;
-    const float* s_row = a.ws + (size_t)(clamp_kb(kb0 + ((lane >> 3) & 3)) * 32u / a.group) * a.N;
-    auto issue = [&](int i) {  // stage i of the segment
-      const uint32_t nb = (uint32_t)(nb0 + i);
-      unsigned char* St = lds + (i % kGqBwdStages) * kGqBwdStageBytes;
-      load_1k_to_lds(panel + (size_t)nb * 2048u, St + (wave * 2) * kBlockBytes);
-      load_1k_to_lds(panel + (size_t)nb * 2048u + 1024u, St + (wave * 2 + 1) * kBlockBytes);
-      if (wave < 4) {
+    // its chunk of the weight blocks: one of four, or in 4-bit codes two of 512 bytes (waves 2 and 3 repeating 0 and 1)
+    const uint32_t w_off = W4 ? clamp_kb(kb0 + 2u * ((uint32_t)wave & 1u) + h) * 512u + ((uint32_t)lane_s & 31u) * 16u
+                              : clamp_kb(kb0 + (uint32_t)wave) * 1024u + lane16;
+    const uint32_t w_dst = (W4 ? (uint32_t)wave & 1u : (uint32_t)wave) * 1024u;
+    // the four blocks' scales, by each wave to the same place
+    const uint32_t s_piece = ((uint32_t)lane_s & 7u) * 4u;
+    const uint32_t s_row = clamp_kb(kb0 + (((uint32_t)lane_s >> 3) & 3u)) * 32u / a.group * a.N;
+    auto issue = [&](int i, int j) {  // load j of the six of stage i (behind the last stage: of that one again)
+      const uint32_t st = lds_base + (uint32_t)(i % kGqBwdStages) * kGqBwdStageBytes;
+      const uint32_t nb = (uint32_t)(nb0 + (i < L ? i : L - 1));
+      if (j < 4) {
+        lds_load_1k((j < 2 ? Ag0 : Ag1) + (size_t)nb * 2048u + 1024 * (j & 1), lane16, st + (uint32_t)(wave * 4 + j) * kBlockBytes);
+      } else if (j == 4) {
         const uint32_t nbw = nb < a.weight_nb ? nb : a.weight_nb - 1u;  // (dy is zero beyond the last column)
-        load_1k_to_lds(g.wp + (size_t)nbw * g.KB * kBlk8 + w_off, St + kGqBwdPanel + w_dst);
+        lds_load_1k(g.wp + (size_t)nbw * g.KB * kBlk8, w_off, st + kGqBwdPanel + w_dst);
       } else {
         const uint32_t n = nb * 32u + s_piece;
-        load_1k_to_lds(reinterpret_cast<const unsigned char*>(s_row + (n < a.N ? n : 0u)), St + kGqBwdPanel + kGqBwdWeight);
+        lds_load_1k(reinterpret_cast<const unsigned char*>(a.ws), (s_row + (n < a.N ? n : 0u)) * 4u, st + kGqBwdPanel + kGqBwdWeight);
       }
     };
-
-    v16f acc[4];
+    v16f acc[ROWS];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < ROWS; ++i)
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][e] = 0.0f;
 
-    // explicit LDS reads: a compiler-visible one of memory that direct-to-LDS loads write would drain every
-    // load in flight first; the wait stands in the same block, so no register is handed out before it is filled
+    // (the wait stands in the same block, so no register is handed out before it is filled)
     struct NextRegs { v4i raw; v4f s4[4]; };
     auto next_read = [&](int i, NextRegs& r) {
-      const uint32_t st = lds_base + (i % kGqBwdStages) * kGqBwdStageBytes + kGqBwdPanel;
-      const uint32_t sa = st + kGqBwdWeight + wcol * 128 + 16 * h;
+      const uint32_t st = lds_base + (uint32_t)(i % kGqBwdStages) * kGqBwdStageBytes + kGqBwdPanel;
+      const uint32_t sa = st + kGqBwdWeight + (uint32_t)wave * 128u + 16u * h;
       if constexpr (W4) {
-        const uint32_t wa = st + wcol * 512 + lane * 8;
+        const uint32_t wa = st + (uint32_t)wave * 512u + lane16 / 2u;
         uint2 raw;
         asm volatile("ds_read_b64 %0, %5\n\tds_read_b128 %1, %6\n\tds_read_b128 %2, %6 offset:32\n\t"
                      "ds_read_b128 %3, %6 offset:64\n\tds_read_b128 %4, %6 offset:96\n\ts_waitcnt lgkmcnt(0)"
@@ -187,36 +183,29 @@ __global__ __launch_bounds__(512, 1) void gq_bwd_dx_kernel(GqBwdDxArgs a) {
         for (int q = 0; q < 4; ++q)
 #pragma unroll
           for (int e = 0; e < 4; ++e) r.s4[q][e] = r.s4[q][e] * 0.0625f;
+        // (the transposing MFMA is assembly: without wait states behind the vector ALU's write it read the last register of the
+        // operand before it was written)
+        asm volatile("s_nop 3" : "+v"(r.raw));
       } else {
-        const uint32_t wa = st + wcol * 1024 + lane * 16;
+        const uint32_t wa = st + (uint32_t)wave * 1024u + lane16;
         asm volatile("ds_read_b128 %0, %5\n\tds_read_b128 %1, %6\n\tds_read_b128 %2, %6 offset:32\n\t"
                      "ds_read_b128 %3, %6 offset:64\n\tds_read_b128 %4, %6 offset:96\n\ts_waitcnt lgkmcnt(0)"
                      : "=&v"(r.raw), "=&v"(r.s4[0]), "=&v"(r.s4[1]), "=&v"(r.s4[2]), "=&v"(r.s4[3])
                      : "v"(wa), "v"(sa) : "memory");
       }
     };
-    auto transpose_block = [&](const v4i& rawb) -> v16i {
-      v16i z16;
+    // rows 8 (t / 2) + 4 h + 2 (t % 2) + 0, 1 of a transposed block: code * scale in float32, split into TERMS bf16 values
+    auto convert2 = [&](const v16i& tr, const v4f (&s4)[4], int t, uint32_t (&pk)[TERMS][8]) {
+      float f0 = (float)tr[2 * t] * s4[t >> 1][2 * (t & 1)], f1 = (float)tr[2 * t + 1] * s4[t >> 1][2 * (t & 1) + 1];
 #pragma unroll
-      for (int e = 0; e < 16; ++e) z16[e] = 0;
-      return __builtin_amdgcn_mfma_i32_32x32x32_i8(rawb, ident, z16, 0, 0, 0);
-    };
-    // rows 8 gq + 4 h + 0..3 of a transposed block: code * scale in float32, split into TERMS bf16 values
-    auto convert4 = [&](const v16i& tr, const v4f& s4, int gq, uint32_t (&pk)[TERMS][8]) {
-      float f[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) f[e] = (float)tr[4 * gq + e] * s4[e];
-#pragma unroll
-      for (int t = 0; t < TERMS; ++t)
-#pragma unroll
-        for (int p = 0; p < 2; ++p) {
-          const uint32_t w = pack_bf16x2(f[2 * p], f[2 * p + 1]);
-          pk[t][2 * gq + p] = w;
-          if (t + 1 < TERMS) {
-            f[2 * p] = f[2 * p] - __uint_as_float(w << 16);
-            f[2 * p + 1] = f[2 * p + 1] - __uint_as_float(w & 0xffff0000u);
-          }
+      for (int u = 0; u < TERMS; ++u) {
+        const uint32_t w = pack_bf16x2(f0, f1);
+        pk[u][t] = w;
+        if (u + 1 < TERMS) {
+          f0 = f0 - __uint_as_float(w << 16);
+          f1 = f1 - __uint_as_float(w & 0xffff0000u);
         }
+      }
     };
     auto to_operands = [&](const uint32_t (&pk)[TERMS][8], v8bf (&bq)[2][TERMS]) {
 #pragma unroll
@@ -225,106 +214,115 @@ __global__ __launch_bounds__(512, 1) void gq_bwd_dx_kernel(GqBwdDxArgs a) {
         for (int q = 0; q < 2; ++q)
           bq[q][t] = __builtin_bit_cast(v8bf, v4i{(int)pk[t][4 * q], (int)pk[t][4 * q + 1], (int)pk[t][4 * q + 2], (int)pk[t][4 * q + 3]});
     };
-    auto panel_frag = [&](int i, int pair) -> v8bf {  // pair = 4 q + row block
-      const unsigned char* St = lds + (i % kGqBwdStages) * kGqBwdStageBytes;
-      return __builtin_bit_cast(
-          v8bf, *reinterpret_cast<const v4i*>(St + ((wrow * 4 + (pair & 3)) * 2 + (pair >> 2)) * kBlockBytes + lane * 16));
+    constexpr int kPairs = 2 * ROWS;  // (half q, row block) of a stage
+    auto panel_frag = [&](int i, int pair) -> v8bf {
+      typedef __attribute__((address_space(3))) const v4i* lds_v4ptr;
+      const uint32_t at = lds_base + (uint32_t)(i % kGqBwdStages) * kGqBwdStageBytes + lane16;
+      return __builtin_bit_cast(v8bf, *reinterpret_cast<lds_v4ptr>((uintptr_t)(at + (uint32_t)((pair % ROWS) * 2 + pair / ROWS) * kBlockBytes)));
     };
-    auto stage = [&](int i, const v8bf (&bqC)[2][TERMS], v8bf (&bqN)[2][TERMS], bool convert_next) {
-      if (n_act == 0) return;  // wave-uniform: a wave without rows only feeds the pipeline
+    // One stage: its MFMAs from the dy panel in the LDS, two row blocks at a time, small terms first; between them the operands
+    // of stage i + 1 are prepared.  af: the fragments of the first two pairs; leaves those of stage i + 1 there where that one
+    // has landed (ahead).
+    auto stage = [&](int i, const v8bf (&bqC)[2][TERMS], v8bf (&bqN)[2][TERMS], bool ahead, v8bf (&af)[4]) {
+      constexpr int kSlots = kPairs * TERMS;  // MFMAs
+      constexpr int kFirst = 5, kGap = (kSlots - 6) / 8;  // where the eight conversion steps stand: four MFMAs behind the transposing one
+      static_assert(kFirst + 7 * kGap < kSlots, "the conversion ends inside the stage");
       NextRegs nx;
       v16i tr;
       uint32_t pk[TERMS][8];
-      if (convert_next) {
-        next_read(i + 1, nx);
-        tr = transpose_block(nx.raw);
-      }
-      v8bf af = panel_frag(i, 0);
+      asm volatile("s_nop 3");  // (operands converted at the end of the stage before)
+      next_read(i + 1, nx);
 #pragma unroll
-      for (int pair = 0; pair < 8; ++pair) {
-        const int q = pair >> 2, rb = pair & 3;
-        v8bf af_next = af;
-        if (pair < 7) af_next = panel_frag(i, pair + 1);
-        if (rb < n_act) {
+      for (int p = 0; p < kPairs; p += 2) {
+        const int q = p / ROWS, rb = p % ROWS;
 #pragma unroll
-          for (int t = TERMS - 1; t >= 0; --t)  // small terms first
-            acc[rb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af, bqC[q][t], acc[rb], 0, 0, 0);
-        }
-        if (convert_next && pair >= 2 && pair < 6) convert4(tr, nx.s4[pair - 2], pair - 2, pk);
-        __builtin_amdgcn_sched_barrier(0);
-        af = af_next;
+        for (int t = TERMS - 1; t >= 0; --t)
+#pragma unroll
+          for (int u = 0; u < 2; ++u) {
+            const int sl = p * TERMS + (TERMS - 1 - t) * 2 + u;
+            bwd_mfma<true>(acc[rb + u], af[(p + u) & 3], bqC[q][t]);
+            if (t == TERMS - 1) {  // the next two pairs' fragments
+              if (p + 2 < kPairs) af[(p + 2 + u) & 3] = panel_frag(i, p + 2 + u);
+              else if (ahead) af[(p + 2 + u) & 3] = panel_frag(i + 1, u);
+            }
+            if (sl == 0) bwd_transpose(tr, nx.raw, ident);
+            if (sl == kFirst) asm volatile("" : "+v"(tr));  // (not read before this place)
+            if (sl >= kFirst && (sl - kFirst) % kGap == 0 && (sl - kFirst) / kGap < 8) {
+              convert2(tr, nx.s4, (sl - kFirst) / kGap, pk);
+              if ((sl - kFirst) / kGap == 7) to_operands(pk, bqN);
+            }
+            if (sl % (kSlots / 8) == 1 && sl / (kSlots / 8) < kGqBwdLoads) issue(i + 4, sl / (kSlots / 8));
+            __builtin_amdgcn_sched_barrier(0);
+          }
       }
-      if (convert_next) to_operands(pk, bqN);
     };
 
-    v8bf bqA[2][TERMS], bqB[2][TERMS];
-    bwd_dx_stages<kGqBwdAhead, kGqBwdLoads>(
-        L, n_act > 0, issue,
-        [&] {  // operands of stage 0
-          NextRegs nx;
-          next_read(0, nx);
-          uint32_t pk[TERMS][8];
-          const v16i tr = transpose_block(nx.raw);
+    v8bf bqA[2][TERMS], bqB[2][TERMS], af[4];
+    wait_vmcnt<0>();  // stores of the previous tile
+    lds_barrier();
 #pragma unroll
-          for (int gq = 0; gq < 4; ++gq) convert4(tr, nx.s4[gq], gq, pk);
-          to_operands(pk, bqA);
-        },
-        [&](int i, bool more) { stage(i, bqA, bqB, more); }, [&](int i, bool more) { stage(i, bqB, bqA, more); });
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < kGqBwdLoads; ++j) issue(i, j);
+    wait_vmcnt<0>();
+    lds_barrier();
+    {  // operands of stage 0
+      NextRegs nx;
+      next_read(0, nx);
+      uint32_t pk[TERMS][8];
+      v16i tr;
+      bwd_transpose(tr, nx.raw, ident);
+      asm volatile("s_nop 15\n\ts_nop 15" : "+v"(tr));
+#pragma unroll
+      for (int t = 0; t < 8; ++t) convert2(tr, nx.s4, t, pk);
+      to_operands(pk, bqA);
+    }
+    // Two stages to a barrier: stages i and i + 1 and the weight of i + 2 have landed, i + 4 and i + 5 are asked for
+    // (into the slots of i - 2 and i - 1).
+#pragma unroll 1
+    for (int i = 0; i < L; i += 2) {
+      wait_vmcnt<kGqBwdLoads>();
+      lds_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int p = 0; p < 2; ++p) af[p] = panel_frag(i, p);
+      __builtin_amdgcn_sched_barrier(0);
+      stage(i, bqA, bqB, true, af);
+      stage(i + 1, bqB, bqA, false, af);
+    }
+    wait_vmcnt<0>();
+    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");  // the last MFMAs, which the compiler does not know, have written their sums
+#pragma unroll
+    for (int rb = 0; rb < ROWS; ++rb) asm volatile("" : "+a"(acc[rb]));
 
-    const uint32_t kbw = kb0 + (uint32_t)wcol;
+    const uint32_t kbw = kb0 + (uint32_t)wave;
     if (whole) {
-      lds_barrier();  // (every wave has read its last stage)
-      const uint32_t rs_lds = lds_base + 8u * kBwdTurnBytes;
-      const int live = ((int)(g.M - tm * 256u) + 31) / 32;
-      bwd_dx_fetch_rs<NKK>(g, tm * 256u, live < 8 ? live : 8, rs_lds, wave, 8);
-      if (n_act)
-        bwd_dx_store<NKK, 1, 4, true>(g, tm * 256u + (uint32_t)wrow * 128u, kbw, n_act, lds_base + (uint32_t)wave * kBwdTurnBytes,
-                                      rs_lds + (uint32_t)(wrow * 4 * NKK * 3) * kBlockBytes, [&](int rb, int) -> v16f { return acc[rb]; });
+      lds_barrier();  // (every wave has read its last stage, and nothing is on its way into the LDS)
+      const uint32_t rs_lds = lds_base + 4u * kBwdTurnBytes;
+      bwd_dx_fetch_rs<NKK>(g, tm * 256u, live_blocks, rs_lds, wave, 4);
+      bwd_dx_store<NKK, 1, ROWS, true>(g, tm * 256u, kbw, live_blocks, lds_base + (uint32_t)wave * kBwdTurnBytes, rs_lds,
+                                       [&](int rb, int) -> v16f { return bwd_sums<true>(acc[rb]); });
     } else {
 #pragma unroll
-      for (int rb = 0; rb < 4; ++rb)
-        if (rb < n_act) {
-          float4* dst = bwd_dx_part<1>(g, slot, (uint32_t)(wrow * 4 + rb), (uint32_t)wcol);
+      for (int rb = 0; rb < ROWS; ++rb)
+        if (rb < live_blocks) {
+          float4* dst = bwd_dx_part<1>(g, slot, (uint32_t)rb, (uint32_t)wave);
+          const v16f y = bwd_sums<true>(acc[rb]);
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
-            dst[e * 64] = make_float4(acc[rb][4 * e], acc[rb][4 * e + 1], acc[rb][4 * e + 2], acc[rb][4 * e + 3]);
+          for (int e = 0; e < 4; ++e) dst[e * 64] = make_float4(y[4 * e], y[4 * e + 1], y[4 * e + 2], y[4 * e + 3]);
         }
     }
   };
 
-  // ---- whole tiles (an XCD walks a contiguous range of the band-major order), then the split ones
-  const uint32_t ntile = g.direct_tiles;
-  const uint32_t wgs_per_xcd = gridDim.x >> 3, xcd = blockIdx.x & 7u;
-  const uint32_t per_xcd = (ntile + 7u) / 8u;
-  uint32_t ti = blockIdx.x >> 3;
-  const uint32_t sw8 = g.sk_wgs >> 3, sk_w = xcd * sw8 + (blockIdx.x >> 3);
-  uint32_t s0 = 0, s1 = 0;
-  if ((blockIdx.x >> 3) < sw8) {
-    const uint32_t total = (g.tiles_m * g.tiles_k - ntile) * g.NB;
-    s0 = sk_w * g.sk_q < total ? sk_w * g.sk_q : total;
-    s1 = s0 + g.sk_q < total ? s0 + g.sk_q : total;
-  }
-#pragma unroll 1
-  for (;;) {
-    uint32_t t, nb0 = 0, len = g.NB, slot = 0;
-    if (ti < per_xcd) {
-      t = xcd * per_xcd + ti;
-      ti += wgs_per_xcd;
-      if (t >= ntile) { ti = per_xcd; continue; }
-    } else if (s0 < s1) {
-      const uint32_t u = s0 / g.NB;
-      nb0 = s0 - u * g.NB;
-      len = s1 - s0 < g.NB - nb0 ? s1 - s0 : g.NB - nb0;
-      t = ntile + u;
-      slot = sk_w + u;
-      s0 += len;
-    } else {
-      break;
-    }
+  // whole tiles (an XCD walks a contiguous range of the band-major order), then the split ones
+  bwd_dx_schedule(g, true, [&](uint32_t t, int nb0, int len, uint32_t slot) {
     uint32_t tm, tk;
     bwd_dx_tile_at(g, t, tm, tk);
-    segment(tm, tk, (int)nb0, (int)len, len == g.NB, slot);
-  }
+    const int live0 = ((int)(g.M - tm * 256u) + 31) / 32;
+    const int live = __builtin_amdgcn_readfirstlane(live0 < 8 ? live0 : 8);
+    if (live > 4) segment(std::integral_constant<int, 8>{}, tm, tk, live, nb0, len, len == (int)g.NB, slot);
+    else segment(std::integral_constant<int, 4>{}, tm, tk, live, nb0, len, len == (int)g.NB, slot);
+  });
 }
 
 // ---------------------------------------------------------------------------------------

@@ -1,5 +1,6 @@
 """The assembly of the four-wave pull-back kernels (no GPU: hipcc cross-compiles).  Their MFMAs are inline assembly with tied
-accumulators, so the compiler inserts no wait states in front of a read of a result by another unit: between an MFMA and the first
+accumulators, so the compiler inserts no wait states in front of a read of a result by another unit, or of an operand that the
+vector ALU has just written (at least two): between an MFMA and the first
 read of a register it wrote there must be at least 13 (what the compiler leaves behind the same MFMA as a builtin; every instruction counts as one,
 another MFMA as the 8 for which it holds the matrix core, `s_nop n` as n + 1).  Inside the loops no accumulator is
 moved and no load is waited for but by the loop's own count: a reload or a move there is what the layout of registers avoids."""
@@ -40,6 +41,24 @@ def closest_read(lines):
     return worst
 
 
+def operand_gap(lines):
+    """Fewest wait states between a vector instruction's write and an assembly MFMA (tied or from 0) that reads it."""
+    written, n, worst = {}, 0, 99
+    for t in lines:
+        nop = re.match(r"s_nop (\d+)", t)
+        n += int(nop.group(1)) + 1 if nop else 1
+        if not t.startswith("v_"):
+            continue
+        ops = t.split(None, 1)[1].split(", ")
+        if "mfma" in t:
+            for r in regs(", ".join(ops[1:3])):
+                worst = min(worst, n - written.get(r, -99) - 1)
+        else:
+            for r in regs(ops[0]):
+                written[r] = n
+    return worst
+
+
 def kernels(asm):
     for m in re.finditer(r"^(_ZN4w8a8\d+(?:bwd_dx_wide|gq_bwd_dx_wide)_kernel\S+):(.*?)^\.Lfunc_end", asm, re.M | re.S):
         yield m.group(1), m.group(2)
@@ -51,6 +70,7 @@ def instructions(text):
 
 def test_the_count_itself():
     assert closest_read(["v_mfma_f32_32x32x16_bf16 a[0:15], v[0:3], v[4:7], a[0:15]", "s_nop 3", "v_accvgpr_read_b32 v9, a5"]) == 5
+    assert operand_gap(["v_or_b32_e32 v7, v1, v2", "s_nop 1", "v_mfma_f32_32x32x16_bf16 v[16:31], v[0:3], v[4:7], v[16:31]"]) == 2
     assert closest_read(["v_mfma_f32_32x32x16_bf16 v[0:15], v[20:23], v[24:27], v[0:15]", "v_mov_b32 v3, v40", "v_mov_b32 v41, v3"]) == 99
 
 
@@ -61,7 +81,9 @@ def test_results_are_not_read_early(tmp_path):
     except RuntimeError as e:  # pragma: no cover - the image ships hipcc
         pytest.skip(str(e))
     tu = tmp_path / "pullback.hip"
-    body = '#include "w8a8_backward.h"\nusing namespace w8a8;\n'
+    body = '#include "w8a8_gq_bwd.h"\nusing namespace w8a8;\n'
+    body += "".join(f"template __global__ void w8a8::gq_bwd_dx_wide_kernel<{f},{t},{k}>(GqBwdDxArgs);\n"
+                    for f in ("true", "false") for t, k in ((2, 1), (2, 2), (3, 4)))
     body += "".join(f"template __global__ void w8a8::bwd_dx_wide_kernel<{k}>(BwdDxArgs);\n" for k in (0, 1, 2, 4))
     tu.write_text(body)
     flags = [f for f in build.HIPCC_FLAGS if f not in ("-shared", "-fPIC") and not f.startswith("-Wl,")]
@@ -70,9 +92,10 @@ def test_results_are_not_read_early(tmp_path):
                           capture_output=True, text=True)
     assert proc.returncode == 0, proc.stderr[-2000:]
     found = list(kernels(out.read_text()))
-    assert len(found) == 4
+    assert len(found) == 10
     for name, text in found:
         assert closest_read(instructions(text)) >= 13, name
+        assert operand_gap(instructions(text)) >= 2, name
         loops = 0
         for block in re.split(r"^\.LBB\S+:", text, flags=re.M):
             ins = instructions(block)
@@ -80,5 +103,5 @@ def test_results_are_not_read_early(tmp_path):
             if sum("mfma_f32" in t for t in ins) >= 32 and any("s_barrier" in t for t in ins):
                 loops += 1
                 assert not [t for t in ins if t.startswith(("v_accvgpr", "scratch"))], name
-                assert {t for t in ins if "vmcnt" in t} <= {"s_waitcnt vmcnt(7)"}, name
+                assert {t for t in ins if "vmcnt" in t} <= {"s_waitcnt vmcnt(6)" if "gq" in name else "s_waitcnt vmcnt(7)"}, name
         assert loops >= 2, name  # tiles of eight row blocks, and of four
