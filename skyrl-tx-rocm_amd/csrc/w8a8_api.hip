@@ -2189,19 +2189,15 @@ int run_gq_linear(const mi355_w8a8_gq_problem* p, hipStream_t s) {
     return launch_status();
   }
   if (p->group_size % 64u == 0 && !(p->flags & MI355_W8A8_FLAG_GQ_DIRECT)) {
-    // groups of whole 64-wide k steps: 128 x 128 tiles staged through the LDS
-    const dim3 grid((g.n_col_blocks + 3u) / 4u, (L.m_pad / 32u + 3u) / 4u), block(256);
-    if (p->weight_bits == 4u) {
-      if (hipFuncSetAttribute(reinterpret_cast<const void*>(&gq_gemm_lds_kernel<true>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)gq_lds_bytes(true)) != hipSuccess)
-        return MI355_W8A8_ERR_LAUNCH;
-      hipLaunchKernelGGL((gq_gemm_lds_kernel<true>), grid, block, gq_lds_bytes(true), s, g);
-    } else {
-      if (hipFuncSetAttribute(reinterpret_cast<const void*>(&gq_gemm_lds_kernel<false>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)gq_lds_bytes(false)) != hipSuccess)
-        return MI355_W8A8_ERR_LAUNCH;
-      hipLaunchKernelGGL((gq_gemm_lds_kernel<false>), grid, block, gq_lds_bytes(false), s, g);
-    }
+    // groups of whole 64-wide k steps: 64 x 128 tiles staged through the LDS
+    const dim3 grid((p->n + kGqTileCols - 1u) / kGqTileCols, (L.m_pad + kGqTileRows - 1u) / kGqTileRows), block(256);
+    const bool w4 = p->weight_bits == 4u, small = p->group_size <= kGqSmallGroup;
+    const auto kernel = w4 ? (small ? &gq_gemm_lds_kernel<true, true> : &gq_gemm_lds_kernel<true, false>)
+                           : (small ? &gq_gemm_lds_kernel<false, true> : &gq_gemm_lds_kernel<false, false>);
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                            (int)gq_lds_bytes(w4)) != hipSuccess)
+      return MI355_W8A8_ERR_LAUNCH;
+    hipLaunchKernelGGL(kernel, grid, block, gq_lds_bytes(w4), s, g);
     return launch_status();
   }
   const dim3 grid((g.n_col_blocks + 7u) / 8u, (L.m_pad / 32u + 1u) / 2u), block(256);

@@ -556,118 +556,161 @@ __device__ inline void gq_store_row_block(const GqGemmArgs& a, const float (&out
   gq_finish_row_block(a, outv, lacc, lora, rb, col, two_cols, lane);
 }
 
-// The low-rank sums of a workgroup's 128 x 128 tile with B staged through the LDS (the stage ring is free by
-// then): per 16 ranks and per batch of up to eight adapters present among the tile's rows, the four waves
-// bring the adapters' B values of the tile's 128 columns in with direct-to-LDS loads (a slot of 16 ranks x
-// 256 bytes per adapter, 1 KiB per instruction), and every wave then takes its passes -- one per adapter
-// present in a row block, the rows of the other adapters zeroed -- with its operands from there.  Per output
-// the passes, their order and their operands are those of gq_store_row_block, which asks memory for the
-// same B values once per pass, row block and lane, one dependent round trip after the other.  z comes
-// straight from memory: a lane's eight values of a 16-rank step are 32 consecutive bytes.
-// Needs N % 8 == 0 and B aligned to 16 bytes (the 16-byte pieces), at most 64 adapters (the mask).
-// LDS: [0, 32 KiB) the batch, [32 KiB, + 32) the waves' adapter masks.  All four waves must call it.
-constexpr uint32_t kGqLoraLdsBytes = 32768u + 64u;
-__device__ inline bool gq_tile_lora_ok(const GqGemmArgs& a) {
-  return a.n_adapters <= 64u && (a.N & 7u) == 0 && (reinterpret_cast<uintptr_t>(a.lora_b) & 15u) == 0;
-}
-__device__ inline void gq_tile_lora_sums(const GqGemmArgs& a, unsigned char* lds, const uint32_t (&rbs)[2],
-                                         const bool (&rb_ok)[2], uint32_t cbase, uint32_t wave, uint32_t wc, uint32_t lane,
-                                         v16f (&lacc)[2][2]) {
-  typedef __attribute__((address_space(3))) const uint16_t* lds_u16ptr;
-  const uint32_t lds_addr = (uint32_t)(uintptr_t)(lptr_t)lds;
-  const uint32_t rowl = lane & 31u, kg = lane >> 5, c = lane & 31u;
-  int my_ad[2];
-  uint32_t zrow[2];
+// The end of a workgroup's 64 x 128 tile (four waves, 64 x 32 each).  Per 32-row block the scaled low-rank sums are
+// added and the values cast into the LDS, where those of a row change hands, so that sixteen lanes store 256
+// consecutive bytes instead of every lane two.  LDS: behind the batch of the low-rank sums, rows of 272 bytes (16 bytes
+// apart in the banks), then the adapters' factors of the 64 rows.
+constexpr uint32_t kGqOutStride = 272u, kGqOutOff = 16384u, kGqFactorOff = kGqOutOff + 64u * kGqOutStride;
+constexpr uint32_t kGqEpilogueBytes = kGqFactorOff + 256u;
+__device__ inline void gq_finish_values(const GqGemmArgs& a, unsigned char* lds, uint32_t i, const v16f& outv,
+                                        const v16f& lacc, bool lora, uint32_t row0, uint32_t col0, uint32_t wave, uint32_t lane) {
+  typedef __attribute__((address_space(3))) const v4f* lds_f4ptr;
+  typedef __attribute__((address_space(3))) uint16_t* lds_u16ptr;
+  typedef __attribute__((address_space(3))) unsigned char* lds_ptr;
+  const uint32_t col = wave * 32u + (lane & 31u), r0 = i * 32u + 4u * (lane >> 5);
+  const lds_ptr l = (lds_ptr)(lptr_t)lds + r0 * kGqOutStride + col * 2u;
+  if (a.aux_base && col0 + col < a.N) {
+    uint32_t row = row0 + r0;
+    float* base = a.aux_base + (size_t)row * a.N + col0 + col;
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const uint32_t rowg = rbs[i] * 32u + rowl;
-    my_ad[i] = -1;  // rows beyond M (and row blocks beyond the edge) belong to no adapter
-    zrow[i] = 0;
-    if (rb_ok[i] && rowg < a.M) {
-      const int ad = a.idx ? a.idx[rowg] : 0;
-      my_ad[i] = ad < 0 ? 0 : (ad >= (int)a.n_adapters ? (int)a.n_adapters - 1 : ad);
-      zrow[i] = a.z_slot ? (uint32_t)a.z_slot[rowg] : rowg;
+    for (uint32_t v = 0; v < 16; ++v) {
+      if (row < a.M) *base = outv[v];
+      const uint32_t step = (v & 3u) == 3u ? 5u : 1u;
+      row += step;
+      base += (size_t)step * a.N;
     }
   }
-  unsigned long long pm[2] = {0ull, 0ull};  // adapters present in the wave's row blocks (wave-uniform)
-  for (uint32_t ad = 0; ad < a.n_adapters; ++ad)
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
-      if (__builtin_amdgcn_ballot_w64(my_ad[i] == (int)ad) != 0) pm[i] |= 1ull << ad;
-  unsigned long long* const masks = reinterpret_cast<unsigned long long*>(lds + 32768u);
-  if (lane == 0) masks[wave] = pm[0] | pm[1];
+  for (uint32_t q = 0; q < 4; ++q) {  // four consecutive rows
+    v4f sg = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (lora) sg = *reinterpret_cast<lds_f4ptr>((lds_ptr)(lptr_t)lds + kGqFactorOff + (r0 + 8u * q) * 4u);
+#pragma unroll
+    for (uint32_t e = 0; e < 4; ++e) {
+      float y = outv[4 * q + e];
+      if (lora) {
+        const float low = lacc[4 * q + e] * sg[e];
+        y = y + low;
+      }
+      *reinterpret_cast<lds_u16ptr>(l + kGqOutOff + (8u * q + e) * kGqOutStride) = (uint16_t)f32_to_bf16_bits(y);
+    }
+  }
+}
+
+__device__ inline void gq_store_tile(const GqGemmArgs& a, unsigned char* lds, uint32_t row0, uint32_t col0, uint32_t wave,
+                                     uint32_t lane) {
+  typedef __attribute__((address_space(3))) unsigned char* lds_ptr;
+  typedef __attribute__((address_space(3))) const v4i* lds_i4ptr;
+  const lds_ptr l = (lds_ptr)(lptr_t)lds + kGqOutOff;
   __syncthreads();
-  const unsigned long long wg_mask = masks[0] | masks[1] | masks[2] | masks[3];
+  const bool wide = (a.N & 7u) == 0 && (reinterpret_cast<uintptr_t>(a.out) & 15u) == 0;
+#pragma unroll
+  for (uint32_t p = 0; p < 4; ++p) {  // 64 rows x 16 pieces of 8 columns
+    const uint32_t rl = p * 16u + wave * 4u + (lane >> 4), cl = (lane & 15u) * 8u;
+    const uint32_t row = row0 + rl;
+    if (row >= a.M || col0 + cl >= a.N) continue;
+    const v4i v = *reinterpret_cast<lds_i4ptr>(l + rl * kGqOutStride + cl * 2u);
+    uint16_t* const o = a.out + (size_t)row * a.N + col0 + cl;
+    if (wide) {
+      *reinterpret_cast<v4i*>(o) = v;
+    } else {
+#pragma unroll
+      for (uint32_t e = 0; e < 8; ++e)
+        if (col0 + cl + e < a.N) o[e] = (uint16_t)((uint32_t)v[e / 2u] >> (16u * (e & 1u)));
+    }
+  }
+}
+
+// The low-rank sums of one 32-row block of a workgroup's 64 x 128 tile with B staged through the LDS (the stage ring is free by
+// then): per 16 ranks and per batch of up to four adapters present among the block's rows, the four waves
+// bring the adapters' B values of the tile's 128 columns in with direct-to-LDS loads (a slot of 16 ranks x
+// 256 bytes per adapter, 1 KiB per instruction), and every wave then takes its passes -- one per adapter,
+// the rows of the other adapters zeroed -- with its operands from there.  Per output
+// the passes, their order and their operands are those of gq_store_row_block, which asks memory for the
+// same B values once per pass, row block and lane, one dependent round trip after the other.  z comes
+// straight from memory: a lane's eight values of a 16-rank step are 32 consecutive bytes.  Where N % 8 != 0 or B is
+// not aligned to 16 bytes the pieces are read value by value.  Adapters are looked for 64 at a time (the mask).
+// LDS: [0, 16 KiB) the batch.  All four waves must call it; every wave takes column block `wave`.
+constexpr uint32_t kGqLoraLdsBytes = 16384u;
+__device__ inline void gq_tile_lora_sums(const GqGemmArgs& a, unsigned char* lds, uint32_t rb, uint32_t cbase, uint32_t wave,
+                                         uint32_t lane, v16f& lacc) {
+  typedef __attribute__((address_space(3))) uint16_t* lds_u16ptr;
+  const uint32_t lds_addr = (uint32_t)(uintptr_t)(lptr_t)lds;
+  const uint32_t kg = lane >> 5, c = lane & 31u;
+  const uint32_t rowg = rb * 32u + c;
+  int my_ad = -1;  // rows beyond M belong to no adapter
+  uint32_t zrow = 0;
+  if (rowg < a.M) {
+    const int ad = a.idx ? a.idx[rowg] : 0;
+    my_ad = ad < 0 ? 0 : (ad >= (int)a.n_adapters ? (int)a.n_adapters - 1 : ad);
+    zrow = a.z_slot ? (uint32_t)a.z_slot[rowg] : rowg;
+  }
   // what this lane brings in per slot: rank 4 wave + lane / 16 of the step, columns 8 (lane % 16) .. + 7 of the tile
   const uint32_t ld_rank = 4u * wave + (lane >> 4), ld_col = cbase * 32u + (lane & 15u) * 8u;
+  const bool pieces = (a.N & 7u) == 0 && (reinterpret_cast<uintptr_t>(a.lora_b) & 15u) == 0;
   for (uint32_t r0 = 0; r0 < a.r; r0 += 16u) {
-    uint32_t term[2][3][4];
+    uint32_t term[3][4];
+    float z8[8];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      float z8[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) z8[e] = 0.0f;
-      if (my_ad[i] >= 0) {
-        const float* zp = a.z + (size_t)zrow[i] * 64u + r0 + 8u * kg;
-        float4 lo4 = *reinterpret_cast<const float4*>(zp), hi4 = *reinterpret_cast<const float4*>(zp + 4);
-        for (uint32_t sl = 1; sl < a.z_slices; ++sl) {  // the K slices of the projection, added in order
-          const float4 l2 = *reinterpret_cast<const float4*>(zp + (size_t)sl * a.z_slice_stride);
-          const float4 h2 = *reinterpret_cast<const float4*>(zp + (size_t)sl * a.z_slice_stride + 4);
-          lo4.x = lo4.x + l2.x; lo4.y = lo4.y + l2.y; lo4.z = lo4.z + l2.z; lo4.w = lo4.w + l2.w;
-          hi4.x = hi4.x + h2.x; hi4.y = hi4.y + h2.y; hi4.z = hi4.z + h2.z; hi4.w = hi4.w + h2.w;
-        }
-        const float t8[8] = {lo4.x, lo4.y, lo4.z, lo4.w, hi4.x, hi4.y, hi4.z, hi4.w};
-#pragma unroll
-        for (int e = 0; e < 8; ++e) z8[e] = r0 + 8u * kg + (uint32_t)e < a.r ? t8[e] : 0.0f;
+    for (int e = 0; e < 8; ++e) z8[e] = 0.0f;
+    if (my_ad >= 0) {
+      const float* zp = a.z + (size_t)zrow * 64u + r0 + 8u * kg;
+      float4 lo4 = *reinterpret_cast<const float4*>(zp), hi4 = *reinterpret_cast<const float4*>(zp + 4);
+#pragma unroll 1
+      for (uint32_t sl = 1; sl < a.z_slices; ++sl) {  // the K slices of the projection, added in order
+        const float4 l2 = *reinterpret_cast<const float4*>(zp + (size_t)sl * a.z_slice_stride);
+        const float4 h2 = *reinterpret_cast<const float4*>(zp + (size_t)sl * a.z_slice_stride + 4);
+        lo4.x = lo4.x + l2.x; lo4.y = lo4.y + l2.y; lo4.z = lo4.z + l2.z; lo4.w = lo4.w + l2.w;
+        hi4.x = hi4.x + h2.x; hi4.y = hi4.y + h2.y; hi4.z = hi4.z + h2.z; hi4.w = hi4.w + h2.w;
       }
+      const float t8[8] = {lo4.x, lo4.y, lo4.z, lo4.w, hi4.x, hi4.y, hi4.z, hi4.w};
 #pragma unroll
-      for (int d = 0; d < 4; ++d) {
-        float hi[2], mid[2], lo[2];
+      for (int e = 0; e < 8; ++e) z8[e] = r0 + 8u * kg + (uint32_t)e < a.r ? t8[e] : 0.0f;
+    }
 #pragma unroll
-        for (int e = 0; e < 2; ++e) {
-          const float z = z8[2 * d + e];
-          hi[e] = bf16_round_f32(z);
-          const float r1 = z - hi[e];
-          mid[e] = bf16_round_f32(r1);
-          lo[e] = bf16_round_f32(r1 - mid[e]);
-        }
-        term[i][0][d] = pack_bf16x2(hi[0], hi[1]);
-        term[i][1][d] = pack_bf16x2(mid[0], mid[1]);
-        term[i][2][d] = pack_bf16x2(lo[0], lo[1]);
+    for (int d = 0; d < 4; ++d) {
+      float hi[2], mid[2], lo[2];
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const float z = z8[2 * d + e];
+        hi[e] = bf16_round_f32(z);
+        const float r1 = z - hi[e];
+        mid[e] = bf16_round_f32(r1);
+        lo[e] = bf16_round_f32(r1 - mid[e]);
       }
+      term[0][d] = pack_bf16x2(hi[0], hi[1]);
+      term[1][d] = pack_bf16x2(mid[0], mid[1]);
+      term[2][d] = pack_bf16x2(lo[0], lo[1]);
     }
     const bool ld_on = r0 + ld_rank < a.r && ld_col < a.N;
     const uint32_t ld_off = ((r0 + ld_rank) * a.N + ld_col) * 2u;
-    unsigned long long rem = wg_mask;
-    while (rem) {  // batches of up to eight adapters, smallest first (workgroup-uniform)
-      uint32_t ads[8], nb = 0;
-#pragma unroll
-      for (int sl = 0; sl < 8; ++sl) {
-        ads[sl] = 0;
-        if (rem) {
-          ads[sl] = (uint32_t)__builtin_ctzll(rem);
-          rem &= rem - 1ull;
-          nb = (uint32_t)sl + 1u;
+    for (uint32_t first = 0; first < a.n_adapters; first += 64u) {
+      unsigned long long rem = 0ull;  // adapters of the block's rows (the same for all four waves)
+#pragma unroll 1
+      for (uint32_t ad = 0; ad < 64u && first + ad < a.n_adapters; ++ad)
+        if (__builtin_amdgcn_ballot_w64(my_ad == (int)(first + ad)) != 0) rem |= 1ull << ad;
+      while (rem) {  // batches of up to four adapters, smallest first (workgroup-uniform)
+        __syncthreads();  // the batch before has been read
+        unsigned long long batch = rem;
+        uint32_t nb = 0;
+#pragma unroll 1
+        for (; rem && nb < 4u; ++nb, rem &= rem - 1ull) {
+          const unsigned char* const b = reinterpret_cast<const unsigned char*>(a.lora_b) +
+                                         (size_t)(first + (uint32_t)__builtin_ctzll(rem)) * a.r * a.N * 2u;
+          const uint32_t dst = nb * 4096u + wave * 1024u;
+          if (pieces) {
+            if (ld_on) lds_load_1k(b, ld_off, lds_addr + dst);
+          } else if (ld_on) {
+#pragma unroll 1
+            for (uint32_t e = 0; e < 8u && ld_col + e < a.N; ++e)
+              reinterpret_cast<lds_u16ptr>((lptr_t)lds)[dst / 2u + lane * 8u + e] = *reinterpret_cast<const uint16_t*>(b + ld_off + 2u * e);
+          }
         }
-      }
-      __syncthreads();  // the batch before has been read
-#pragma unroll
-      for (uint32_t sl = 0; sl < 8; ++sl) {
-        if (sl < nb && ld_on)
-          lds_load_1k(reinterpret_cast<const unsigned char*>(a.lora_b) + (size_t)ads[sl] * a.r * a.N * 2u, ld_off,
-                      lds_addr + sl * 4096u + wave * 1024u);
-      }
-      wait_vmcnt<0>();
-      __syncthreads();
-#pragma unroll
-      for (uint32_t sl = 0; sl < 8; ++sl) {
-        if (sl >= nb) break;
-        const uint32_t ad = ads[sl];
-        if (!(((pm[0] | pm[1]) >> ad) & 1ull)) continue;  // wave-uniform
-        v4i bo[2];
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          const uint32_t lcol = (2u * wc + (uint32_t)j) * 32u + c;
+        wait_vmcnt<0>();
+        __syncthreads();
+#pragma unroll 1
+        for (uint32_t sl = 0; sl < nb; ++sl, batch &= batch - 1ull) {
+          const bool mine = my_ad == (int)(first + (uint32_t)__builtin_ctzll(batch));
+          const uint32_t lcol = wave * 32u + c;
           const bool col_ok = cbase * 32u + lcol < a.N;
           uint32_t braw[8];
 #pragma unroll
@@ -676,24 +719,16 @@ __device__ inline void gq_tile_lora_sums(const GqGemmArgs& a, unsigned char* lds
             const uint16_t v = reinterpret_cast<lds_u16ptr>((lptr_t)lds)[(sl * 16u + rank) * 128u + lcol];
             braw[e] = (col_ok && r0 + rank < a.r) ? (uint32_t)v : 0u;
           }
+          v4i bo;
 #pragma unroll
-          for (int d = 0; d < 4; ++d) bo[j][d] = (int)(braw[2 * d] | (braw[2 * d + 1] << 16));
-        }
+          for (int d = 0; d < 4; ++d) bo[d] = (int)(braw[2 * d] | (braw[2 * d + 1] << 16));
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          if (!((pm[i] >> ad) & 1ull)) continue;  // wave-uniform
-          const bool mine = my_ad[i] == (int)ad;
-          v4i za[3];
+          for (int t = 2; t >= 0; --t) {
+            v4i za;
 #pragma unroll
-          for (int t = 0; t < 3; ++t)
-#pragma unroll
-            for (int d = 0; d < 4; ++d) za[t][d] = mine ? (int)term[i][t][d] : 0;
-#pragma unroll
-          for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int t = 2; t >= 0; --t)
-              lacc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, za[t]),
-                                                                    __builtin_bit_cast(v8bf, bo[j]), lacc[i][j], 0, 0, 0);
+            for (int d = 0; d < 4; ++d) za[d] = mine ? (int)term[t][d] : 0;
+            lacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, za), __builtin_bit_cast(v8bf, bo), lacc, 0, 0, 0);
+          }
         }
       }
     }
@@ -818,191 +853,205 @@ __global__ __launch_bounds__(256, 2) void gq_gemm_kernel(GqGemmArgs a) {
 
 // ---------------------------------------------------------------------------------------
 // The same product for groups that are multiples of 64 k, staged through the LDS: a workgroup of four
-// waves (2 x 2) owns a 128 x 128 output tile; per 64-wide k step its activation fragments (8 KiB), weight
-// fragments (4 or 8 KiB) and the group's scales (128 column and 128 row scales) arrive once per workgroup by
-// direct-to-LDS loads, three steps ahead, and every wave reads the fragments of its 64 x 64 share from
+// waves owns a 64 x 128 output tile, a wave 64 x 32 of it; per 64-wide k step its activation fragments (4 KiB),
+// weight fragments (4 or 8 KiB) and the group's scales (128 column and 64 row scales) arrive once per
+// workgroup by direct-to-LDS loads, two or three steps ahead, and every wave reads its fragments from
 // there.  Per output the arithmetic and its order are those of gq_gemm_kernel (the step and the epilogue
-// are shared), so the two kernels agree bit for bit; this one asks the L2 for half the bytes and keeps
-// three steps in flight instead of one.
-constexpr uint32_t kGqLdsStages = 4;
-__host__ __device__ constexpr uint32_t gq_lds_stage_bytes(bool w4) { return 8192u + (w4 ? 4096u : 8192u) + 1024u; }
-__host__ __device__ constexpr uint32_t gq_lds_bytes(bool w4) { return kGqLdsStages * gq_lds_stage_bytes(w4); }
-static_assert(gq_lds_bytes(true) >= kGqLoraLdsBytes && gq_lds_bytes(true) >= 4u * 32u * 64u * 4u, "the epilogue reuses the ring");
+// are shared), so the two kernels agree bit for bit.
+// Bound by instruction issue: four vector operations per output and group beside group / 32 MFMAs per block.  A wave
+// alone issues one every 4.7 cycles, two waves of a SIMD two in that time where both are plain multiplications,
+// additions or logical operations: hence 64 x 32 a wave, 128 registers and four waves to a SIMD, where 64 x 64 (203
+// registers, two waves) left the ALU waiting for its own wave.  The smaller tile also fills the chip: 1536 rows x 4096
+// columns are 768 workgroups for 1024 places instead of 384 for 512.  The ring's places are unrolled (28 scalar
+// instructions a stage instead of 43).  K = 12288, N = 4096: 4096 rows, 4-bit codes in groups of 128 387 -> 350 us;
+// 1536 rows, 8-bit codes in groups of 64 214 -> 192 us.
+// Sums of at most kGqSmallGroup products leave the matrix core as float32 values: v_cvt_f32_i32 takes 4.3 cycles of a
+// SIMD with several waves, a subtraction 2.5 (399 -> 383 us at 4096 rows as above).  The accumulators start at the bit pattern of 1.5 * 2^23, a float32 whose last place is
+// one: while |s| < 2^22 (here at most 256 * 128 * 127) the pattern plus s reads as 1.5 * 2^23 + s, and one subtraction
+// returns s exactly.
+constexpr uint32_t kGqSmallGroup = 256u;
+constexpr int kGqSumOrigin = 0x4b400000;
+constexpr float kGqSumOffset = 12582912.0f;
+constexpr uint32_t kGqTileRows = 64u, kGqTileCols = 128u;
+__host__ __device__ constexpr uint32_t gq_lds_stages(bool w4) { return w4 ? 4u : 3u; }
+__host__ __device__ constexpr uint32_t gq_lds_stage_bytes(bool w4) { return 4096u + (w4 ? 4096u : 8192u) + 1024u; }
+__host__ __device__ constexpr uint32_t gq_lds_bytes(bool w4) { return gq_lds_stages(w4) * gq_lds_stage_bytes(w4); }
+static_assert(gq_lds_bytes(true) >= kGqEpilogueBytes && gq_lds_bytes(false) >= kGqEpilogueBytes && kGqLoraLdsBytes <= kGqOutOff,
+              "the epilogue reuses the ring");
+static_assert(4u * gq_lds_bytes(true) <= 160u * 1024u && 4u * gq_lds_bytes(false) <= 160u * 1024u, "four workgroups per CU");
 
-template <bool W4>
-__global__ __launch_bounds__(256, 2) void gq_gemm_lds_kernel(GqGemmArgs a) {
+template <bool W4, bool SMALL>
+__global__ __launch_bounds__(256, 4) void gq_gemm_lds_kernel(GqGemmArgs a) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char gq_lds[];  // the stage ring; the epilogue's z rows afterwards
-  constexpr uint32_t kStage = gq_lds_stage_bytes(W4), kWOff = 8192u, kSOff = 8192u + (W4 ? 4096u : 8192u);
+  constexpr uint32_t kStage = gq_lds_stage_bytes(W4), kWOff = 4096u, kSOff = kWOff + (W4 ? 4096u : 8192u);
   constexpr uint32_t kWBlk = W4 ? 512u : 1024u;      // bytes of a weight fragment (one column block, one k block)
-  constexpr uint32_t kLoads = 2u + (W4 ? 1u : 2u) + 1u;  // direct-to-LDS loads per wave and stage
-  constexpr uint32_t NS = kGqLdsStages;
+  constexpr uint32_t kLoads = 1u + (W4 ? 1u : 2u) + 1u;  // direct-to-LDS loads per wave and stage
+  constexpr uint32_t NS = gq_lds_stages(W4);
   typedef __attribute__((address_space(3))) const unsigned char* lds_cptr;
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const uint32_t wr = wave >> 1, wc = wave & 1u;
   const uint32_t c = lane & 31u, h = lane >> 5;
   const uint32_t kbs = a.K_pad / 32u, blocks_per_group = a.group / 32u;  // both even here
   const uint32_t n_stages = kbs / 2u;
   const uint32_t n_rb = a.M_pad / 32u;
-  const uint32_t rbase = blockIdx.y * 4u, cbase = blockIdx.x * 4u;
+  const uint32_t rbase = blockIdx.y * 2u, cbase = blockIdx.x * 4u;
   // blocks that hang over the edge are read from the last valid one; their results are never stored
   auto rb_of = [&](uint32_t l) { return rbase + l < n_rb ? rbase + l : n_rb - 1u; };
   auto cb_of = [&](uint32_t l) { return cbase + l < a.n_col_blocks ? cbase + l : a.n_col_blocks - 1u; };
-  const uint32_t rbs[2] = {rb_of(2u * wr), rb_of(2u * wr + 1u)};
-  const uint32_t cbs[2] = {cb_of(2u * wc), cb_of(2u * wc + 1u)};
-  const uint32_t col[2] = {cbs[0] * 32u + c, cbs[1] * 32u + c};
   const uint32_t lds0 = (uint32_t)(uintptr_t)(lptr_t)gq_lds;
-  // what this wave brings in per stage: row block `wave` (2 KiB), column block `wave` (1 or 2 KiB), 64 scales
-  const unsigned char* const a_src = reinterpret_cast<const unsigned char*>(a.codes) + (size_t)rb_of(wave) * kbs * 1024u;
-  const unsigned char* const w_src = a.wp + (size_t)cb_of(wave) * kbs * kWBlk;
-  uint32_t s_idx;  // the wave's scale of a group: a column (waves 0, 1) or a row (waves 2, 3), clamped to the last one
+  // what this wave brings in per stage: k block `wave` % 2 of row block `wave` / 2 (1 KiB), column block `wave`
+  // (1 or 2 KiB), 64 scales (columns, columns, rows, and the rows once more so that all waves count alike)
+  const unsigned char* a_src =
+      reinterpret_cast<const unsigned char*>(a.codes) + ((size_t)rb_of(wave >> 1) * kbs + (wave & 1u)) * 1024u;
+  const unsigned char* w_src = a.wp + (size_t)cb_of(wave) * kbs * kWBlk;
+  uint32_t s_idx;  // the lane's scale of a group, clamped to the last one
   if (wave < 2u) {
     const uint32_t cc = cbase * 32u + wave * 64u + lane;
     s_idx = cc < a.N ? cc : a.N - 1u;
   } else {
-    const uint32_t rr = rbase * 32u + (wave - 2u) * 64u + lane;
+    const uint32_t rr = rbase * 32u + lane;
     s_idx = rr < a.M_pad ? rr : a.M_pad - 1u;
   }
   const uint32_t stages_per_group = blocks_per_group / 2u;
-  const float* const s_src = wave < 2u ? a.ws : a.xs;     // the wave's scales: one row of them per group
+  const float* s_src = wave < 2u ? a.ws : a.xs;           // the wave's scales: one row of them per group
   const uint32_t s_stride = wave < 2u ? a.N : a.M_pad;
-  uint32_t ld_sig = 0, ld_group = 0;                      // stage inside its group and group of the next stage requested
-  auto load_stage = [&](uint32_t st) {
-    const uint32_t slot = lds0 + (st % NS) * kStage;
-    lds_load_1k(a_src + (size_t)st * 2048u, lane * 16u, slot + wave * 2048u);
-    lds_load_1k(a_src + (size_t)st * 2048u, 1024u + lane * 16u, slot + wave * 2048u + 1024u);
-    lds_load_1k(w_src + (size_t)st * 2u * kWBlk, lane * 16u, slot + kWOff + wave * 2u * kWBlk);
-    if (!W4) lds_load_1k(w_src + (size_t)st * 2u * kWBlk, 1024u + lane * 16u, slot + kWOff + wave * 2u * kWBlk + 1024u);
-    lds_gather_dword(s_src + (size_t)ld_group * s_stride, s_idx * 4u, slot + kSOff + wave * 256u);
-    if (++ld_sig == stages_per_group) { ld_sig = 0; ++ld_group; }  // (stages are requested in order)
+  uint32_t ld_left = n_stages, ld_sig = 0;                // stages not requested yet, stage inside its group of the next one
+  // the next stage into ring slot u; behind the last stage the last one again (its slot is not read any more), so
+  // that every stage waits for the same count
+  auto load_stage = [&](uint32_t u) {
+    const uint32_t slot = lds0 + u * kStage;
+    lds_load_1k(a_src, lane * 16u, slot + wave * 1024u);
+    lds_load_1k(w_src, lane * 16u, slot + kWOff + wave * 2u * kWBlk);
+    if (!W4) lds_load_1k(w_src, 1024u + lane * 16u, slot + kWOff + wave * 2u * kWBlk + 1024u);
+    lds_gather_dword(s_src, s_idx * 4u, slot + kSOff + wave * 256u);
+    if (ld_left > 1u) {
+      --ld_left;
+      a_src += 2048u;
+      w_src += 2u * kWBlk;
+      if (++ld_sig == stages_per_group) { ld_sig = 0; s_src += s_stride; }
+    }
   };
 
-  float outv[2][2][16];
+  v16f outv[2];
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) outv[i][j][v] = 0.0f;
-  v16i acc[2][2];
-  // one k block, as in gq_gemm_kernel: four MFMAs (from zero when the block opens a group) and, when it
+    for (int v = 0; v < 16; ++v) outv[i][v] = 0.0f;
+  v16i acc[2];
+  constexpr int o = SMALL ? kGqSumOrigin : 0;
+  v16i origin = {o, o, o, o, o, o, o, o, o, o, o, o, o, o, o, o};
+  if (SMALL) asm volatile("" : "+v"(origin));  // kept in registers instead of written again for every group
+  // one k block, as in gq_gemm_kernel: two MFMAs (from zero when the block opens a group) and, when it
   // closes a group, (f32(acc) * sx) * sw added in group order; for 4-bit codes sw carries the exact 1/16
   // (opens / closes: whether the k block is the first / last of its group, workgroup-uniform and kept by
-  // counting: a remainder per k block costs more instructions than the block's four MFMAs leave room for)
-  auto step = [&](bool opens, bool closes, const v4i& fa0, const v4i& fa1, const GqRawFragment<W4>& r0,
-                  const GqRawFragment<W4>& r1, lds_cptr sc) {
-    const v4i fb0 = gq_expand<W4>(r0), fb1 = gq_expand<W4>(r1);
+  // counting: a remainder per k block costs more instructions than the block's MFMAs leave room for)
+  auto step = [&](bool opens, bool closes, const v4i& fa0, const v4i& fa1, const GqRawFragment<W4>& r0, lds_cptr sc) {
+    const v4i fb = gq_expand<W4>(r0);
     if (opens) {
-      const v16i zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-      acc[0][0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa0, fb0, zero, 0, 0, 0);
-      acc[0][1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa0, fb1, zero, 0, 0, 0);
-      acc[1][0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa1, fb0, zero, 0, 0, 0);
-      acc[1][1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa1, fb1, zero, 0, 0, 0);
+      acc[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa0, fb, origin, 0, 0, 0);
+      acc[1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa1, fb, origin, 0, 0, 0);
     } else {
-      acc[0][0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa0, fb0, acc[0][0], 0, 0, 0);
-      acc[0][1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa0, fb1, acc[0][1], 0, 0, 0);
-      acc[1][0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa1, fb0, acc[1][0], 0, 0, 0);
-      acc[1][1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa1, fb1, acc[1][1], 0, 0, 0);
+      acc[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa0, fb, acc[0], 0, 0, 0);
+      acc[1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa1, fb, acc[1], 0, 0, 0);
     }
     if (closes) {
       typedef __attribute__((address_space(3))) const float* lds_fptr;
       typedef float gq_f4 __attribute__((ext_vector_type(4)));
       typedef __attribute__((address_space(3))) const gq_f4* lds_f4ptr;
-      float swl[2];
+      float swl = reinterpret_cast<lds_fptr>(sc)[wave * 32u + c];
+      if (W4) swl = swl * 0.0625f;
+      // eight sums at a time, each of the four steps for all eight before the next step (the same operations per
+      // output; output by output every instruction needs the result of the one in front of it)
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        swl[j] = reinterpret_cast<lds_fptr>(sc)[(2u * wc + (uint32_t)j) * 32u + c];
-        if (W4) swl[j] = swl[j] * 0.0625f;
-      }
-      // a fragment's sixteen sums at a time, each of the four steps for all sixteen before the next step (the
-      // same operations per output; measured 3 % faster than output by output, where every instruction
-      // needs the result of the one in front of it)
+      for (int p = 0; p < 4; ++p) {
+        const int i = p >> 1, v0 = 8 * (p & 1);
+        gq_f4 s4[2];
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        gq_f4 s4[4];
+        for (int q = 0; q < 2; ++q)
+          s4[q] = *reinterpret_cast<lds_f4ptr>(sc + 512u + ((uint32_t)i * 32u + 2u * v0 + 8u * q + 4u * h) * 4u);
+        float t[8];
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-          s4[q] = *reinterpret_cast<lds_f4ptr>(sc + 512u + ((2u * wr + (uint32_t)i) * 32u + 8u * q + 4u * h) * 4u);
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          float t[16];
-#pragma unroll
-          for (int v = 0; v < 16; ++v) t[v] = (float)acc[i][j][v];
-          __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-          for (int v = 0; v < 16; ++v) t[v] = t[v] * s4[v >> 2][v & 3];
-          __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-          for (int v = 0; v < 16; ++v) t[v] = t[v] * swl[j];
-          __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-          for (int v = 0; v < 16; ++v) outv[i][j][v] = outv[i][j][v] + t[v];
-          __builtin_amdgcn_sched_barrier(0);
+        for (int v = 0; v < 8; ++v) {
+          if (SMALL) t[v] = __int_as_float(acc[i][v0 + v]) - kGqSumOffset;
+          else t[v] = (float)acc[i][v0 + v];
         }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int v = 0; v < 8; ++v) t[v] = t[v] * s4[v >> 2][v & 3];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int v = 0; v < 8; ++v) t[v] = t[v] * swl;
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int v = 0; v < 8; ++v) outv[i][v0 + v] = outv[i][v0 + v] + t[v];
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
   };
 
-  for (uint32_t st = 0; st + 1u < NS && st < n_stages; ++st) load_stage(st);
   uint32_t sig = 0;  // stage inside its group
-  for (uint32_t st = 0; st < n_stages; ++st) {
-    // stage st has landed once at most the NS - 2 younger stages are outstanding (none are issued near the end)
-    if (st + NS - 2u < n_stages) wait_vmcnt<(NS - 2) * kLoads>();
-    else wait_vmcnt<0>();
-    lds_barrier();  // everybody's pieces of stage st; and every wave is done with stage st - 1
-    if (st + NS - 1u < n_stages) load_stage(st + NS - 1u);  // into the slot of stage st - 1
-    lds_cptr slot = reinterpret_cast<lds_cptr>((uintptr_t)(lds0 + (st % NS) * kStage));
+  auto stage = [&](uint32_t u) {
+    wait_vmcnt<(NS - 2) * kLoads>();  // the stage has landed once at most the NS - 2 younger ones are outstanding
+    lds_barrier();  // everybody's pieces of the stage; and every wave is done with the stage before
+    load_stage((u + NS - 1u) % NS);  // into the slot of the stage before
+    lds_cptr slot = reinterpret_cast<lds_cptr>((uintptr_t)(lds0 + u * kStage));
     v4i fa[2][2];
-    GqRawFragment<W4> fr[2][2];
+    GqRawFragment<W4> fr[2];
 #pragma unroll
     for (uint32_t kl = 0; kl < 2; ++kl) {
+      typedef __attribute__((address_space(3))) const v4i* lds_v4ptr;
 #pragma unroll
-      for (uint32_t i = 0; i < 2; ++i) {
-        typedef __attribute__((address_space(3))) const v4i* lds_v4ptr;
-        fa[kl][i] = *reinterpret_cast<lds_v4ptr>(slot + (2u * wr + i) * 2048u + kl * 1024u + lane * 16u);
-        lds_cptr wp = slot + kWOff + (2u * wc + i) * 2u * kWBlk + kl * kWBlk + lane * (W4 ? 8u : 16u);
-        if (W4) {
-          typedef uint32_t gq_u2 __attribute__((ext_vector_type(2)));
-          typedef __attribute__((address_space(3))) const gq_u2* lds_u2ptr;
-          const gq_u2 t = *reinterpret_cast<lds_u2ptr>(wp);
-          fr[kl][i].v = make_uint4(t[0], t[1], 0u, 0u);
-        } else {
-          typedef uint32_t gq_u4 __attribute__((ext_vector_type(4)));
-          typedef __attribute__((address_space(3))) const gq_u4* lds_u4ptr;
-          const gq_u4 t = *reinterpret_cast<lds_u4ptr>(wp);
-          fr[kl][i].v = make_uint4(t[0], t[1], t[2], t[3]);
-        }
+      for (uint32_t i = 0; i < 2; ++i)
+        fa[kl][i] = *reinterpret_cast<lds_v4ptr>(slot + i * 2048u + kl * 1024u + lane * 16u);
+      lds_cptr wp = slot + kWOff + wave * 2u * kWBlk + kl * kWBlk + lane * (W4 ? 8u : 16u);
+      if (W4) {
+        typedef uint32_t gq_u2 __attribute__((ext_vector_type(2)));
+        typedef __attribute__((address_space(3))) const gq_u2* lds_u2ptr;
+        const gq_u2 t = *reinterpret_cast<lds_u2ptr>(wp);
+        fr[kl].v = make_uint4(t[0], t[1], 0u, 0u);
+      } else {
+        typedef uint32_t gq_u4 __attribute__((ext_vector_type(4)));
+        typedef __attribute__((address_space(3))) const gq_u4* lds_u4ptr;
+        const gq_u4 t = *reinterpret_cast<lds_u4ptr>(wp);
+        fr[kl].v = make_uint4(t[0], t[1], t[2], t[3]);
       }
     }
     const bool last_of_group = sig + 1u == stages_per_group;
-    step(sig == 0u, false, fa[0][0], fa[0][1], fr[0][0], fr[0][1], slot + kSOff);
-    step(false, last_of_group, fa[1][0], fa[1][1], fr[1][0], fr[1][1], slot + kSOff);
+    step(sig == 0u, false, fa[0][0], fa[0][1], fr[0], slot + kSOff);
+    step(false, last_of_group, fa[1][0], fa[1][1], fr[1], slot + kSOff);
     sig = last_of_group ? 0u : sig + 1u;
+  };
+  for (uint32_t u = 0; u + 1u < NS; ++u) load_stage(u);
+  for (uint32_t st = 0; st < n_stages; st += NS) {
+#pragma unroll
+    for (uint32_t u = 0; u < NS; ++u) {
+      if (st + u >= n_stages) break;
+      stage(u);
+    }
   }
+  wait_vmcnt<0>();  // (repeated loads on their way into the ring)
   // ---- epilogue: LoRA term per adapter present in the tile, store (the ring is free: its last reads are done)
   lds_barrier();
-  const bool two_cols = cbase + 2u * wc + 1u < a.n_col_blocks;
-  const bool rb_ok[2] = {rbase + 2u * wr < n_rb, rbase + 2u * wr + 1u < n_rb};
-  const bool cols_ok = cbase + 2u * wc < a.n_col_blocks;
-  if (a.z && gq_tile_lora_ok(a)) {  // workgroup-uniform
-    v16f lacc[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) lacc[i][j][v] = 0.0f;
-    gq_tile_lora_sums(a, gq_lds, rbs, rb_ok, cbase, wave, wc, lane, lacc);
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-      if (rb_ok[i] && cols_ok) gq_finish_row_block(a, outv[i], lacc[i], true, rbs[i], col, two_cols, lane);
-    return;
+  const bool lora = a.z != nullptr;
+  if (lora) {
+    if (wave == 0) {
+      const uint32_t row = rbase * 32u + lane;
+      int ad = (a.idx && row < a.M) ? a.idx[row] : 0;
+      ad = ad < 0 ? 0 : (ad >= (int)a.n_adapters ? (int)a.n_adapters - 1 : ad);
+      *reinterpret_cast<__attribute__((address_space(3))) float*>((uintptr_t)(lds0 + kGqFactorOff + lane * 4u)) = a.lora_scaling[ad];
+    }
+    __syncthreads();
   }
-  float (*zs)[64] = reinterpret_cast<float (*)[64]>(gq_lds + wave * 32u * 64u * 4u);
-  if (rb_ok[0] && cols_ok) {
-    gq_store_row_block(a, outv[0], rbs[0], col, two_cols, zs, lane);
-    if (rb_ok[1]) gq_store_row_block(a, outv[1], rbs[1], col, two_cols, zs, lane);
+#pragma unroll 1
+  for (uint32_t i = 0; i < 2; ++i) {
+    v16f lacc;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) lacc[v] = 0.0f;
+    if (lora) gq_tile_lora_sums(a, gq_lds, rbase + i, cbase, wave, lane, lacc);  // workgroup-uniform
+    gq_finish_values(a, gq_lds, i, outv[0], lacc, lora, rbase * 32u, cbase * 32u, wave, lane);
+    outv[0] = outv[1];
   }
+  gq_store_tile(a, gq_lds, rbase * 32u, cbase * 32u, wave, lane);
 }
 
 // ---------------------------------------------------------------------------------------
