@@ -1235,22 +1235,33 @@ struct BwdDloraArgs {
   uint32_t M, K, N, n_groups, max_chunks, col_tiles_a, col_tiles_b;
 };
 
-// chunk id -> (group, first slot, rows); false beyond the last chunk
-__device__ inline bool bwd_find_chunk(const int32_t* group_off, uint32_t n_groups, uint32_t cid, uint32_t& grp,
+// chunk id -> (first slot, rows); rows = 0 beyond the last chunk.  The same in every lane of the wave: 64 groups
+// are looked at together (one after the other they were a chain of loads).
+__device__ inline void bwd_find_chunk(const int32_t* group_off, uint32_t n_groups, uint32_t cid, uint32_t lane,
                                       uint32_t& slot0, uint32_t& rows) {
-  uint32_t run = 0;
-  for (uint32_t gq = 0; gq < n_groups; ++gq) {
-    const uint32_t o0 = (uint32_t)group_off[gq], o1 = (uint32_t)group_off[gq + 1];
+  slot0 = rows = 0;
+  uint32_t run = 0;  // chunks of the groups before
+  for (uint32_t g0 = 0; g0 < n_groups; g0 += 64u) {
+    const uint32_t g = g0 + lane < n_groups ? g0 + lane : n_groups;
+    const uint32_t o0 = (uint32_t)group_off[g], o1 = (uint32_t)group_off[g < n_groups ? g + 1u : g];
     const uint32_t nch = (o1 - o0 + kBwdChunkRows - 1u) / kBwdChunkRows;
-    if (cid < run + nch) {
-      grp = gq;
-      slot0 = o0 + (cid - run) * kBwdChunkRows;
-      rows = o1 - slot0 < kBwdChunkRows ? o1 - slot0 : kBwdChunkRows;
-      return true;
+    uint32_t upto = nch;  // of this and the lanes below
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const uint32_t v = (uint32_t)__shfl_up((int)upto, d);
+      upto += lane >= (uint32_t)d ? v : 0u;
     }
-    run += nch;
+    const uint64_t reached = __builtin_amdgcn_ballot_w64(cid < run + upto);
+    if (reached) {
+      const int own = __builtin_ctzll(reached);
+      const uint32_t before = run + (uint32_t)__builtin_amdgcn_readlane((int)(upto - nch), own);
+      const uint32_t end = (uint32_t)__builtin_amdgcn_readlane((int)o1, own);
+      slot0 = (uint32_t)__builtin_amdgcn_readlane((int)o0, own) + (cid - before) * kBwdChunkRows;
+      rows = end - slot0 < kBwdChunkRows ? end - slot0 : kBwdChunkRows;
+      return;
+    }
+    run += (uint32_t)__builtin_amdgcn_readlane((int)upto, 63);
   }
-  return false;
 }
 
 // Matrix-core version.  out[j][c] = sum_m P[m][j] * Q[m][c] contracts over rows, so both operands
@@ -1261,27 +1272,33 @@ __device__ inline bool bwd_find_chunk(const int32_t* group_off, uint32_t n_group
 // packs into the B operands of the contraction over m.  A wave owns 64 columns (two 32-column
 // strips) and walks the chunk's 32-row blocks, eight per staging pass of P; a workgroup of four
 // waves owns 256 columns.
+// Bound by latencies: a call has few chunks, so a SIMD holds one to three waves.  Hence the ring of Q in flight beside
+// the block at work, through the staging passes too (one rank block: two blocks, so that three workgroups fit a
+// CU; with four blocks and two workgroups experts of 64 rows took 30.2 us instead of 22.5); all of a pass's P
+// requested together, with two rank blocks the second pass's while the first is multiplied; P's operands read ahead of
+// the transposition; loads without conditions (a row or column that is not there reads the tensor's first bytes and
+// is cleared where it is used), so that the waits count.  One block of Q ahead, P's pieces one after the other
+// and operands read at their MFMAs, before, us -> now: 2048 rows of rank 64, 2560 + 10240 columns 37.9 -> 29.7; 3003 rows of
+// rank 32, 12288 + 4096 40.9 -> 34.3, 4096 + 24576 60-62 both (200 MB, 3.3 TB/s); 1536 rows of one
+// adapter 27.7 -> 19.6; 128 experts of 64 rows 22 and 27 both.
 template <int RB>  // 32-wide rank blocks
-__global__ __launch_bounds__(256) void bwd_dlora_kernel(BwdDloraArgs a) {
+__global__ __launch_bounds__(256, RB == 1 ? 3 : 1) void bwd_dlora_kernel(BwdDloraArgs a) {
+  constexpr uint32_t kRing = RB == 1 ? 2 : 4;  // blocks of Q in flight
+  constexpr uint32_t kItems = 4 * RB;  // operand pieces of P that a thread stages in a pass
   // P operands: [row block 8][rank block RB][q 2][term 3][64 lanes][8 bf16]
   extern __shared__ __attribute__((aligned(1024))) unsigned char pop[];
-  __shared__ int rowsrc[kBwdStageRows];
-  __shared__ uint32_t info[3];
-  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+  __shared__ int rowsrc[kBwdChunkRows];
+  const uint32_t tid = threadIdx.x, lane = tid & 63u;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint32_t per_chunk = a.col_tiles_a + a.col_tiles_b;
   const uint32_t cid = blockIdx.x / per_chunk, ct = blockIdx.x % per_chunk;
-  if (tid == 0) {
-    uint32_t grp = 0, slot0 = 0, rows = 0;
-    if (a.chunk_tab) {
-      grp = (uint32_t)a.chunk_tab[3u * cid]; slot0 = (uint32_t)a.chunk_tab[3u * cid + 1u];
-      rows = (uint32_t)a.chunk_tab[3u * cid + 2u];
-    } else if (!bwd_find_chunk(a.group_off, a.n_groups, cid, grp, slot0, rows)) {
-      rows = 0;
-    }
-    info[0] = grp; info[1] = slot0; info[2] = rows;
+  uint32_t slot0, rows;
+  if (a.chunk_tab) {
+    slot0 = (uint32_t)a.chunk_tab[3u * cid + 1u];
+    rows = (uint32_t)a.chunk_tab[3u * cid + 2u];
+  } else {
+    bwd_find_chunk(a.group_off, a.n_groups, cid, lane, slot0, rows);
   }
-  __syncthreads();
-  const uint32_t slot0 = info[1], rows = info[2];
   if (rows == 0) return;  // workgroup-uniform
   const bool job_a = ct < a.col_tiles_a;
   const float* psrc = job_a ? a.rs : a.z;
@@ -1291,6 +1308,58 @@ __global__ __launch_bounds__(256) void bwd_dlora_kernel(BwdDloraArgs a) {
   const uint32_t c = lane & 31u, h = lane >> 5;
   const uint32_t col0 = ((job_a ? ct : ct - a.col_tiles_a) * 4u + wave) * 64u;  // first column of the wave
   const bool active = col0 < C;
+  const uint32_t n_blocks = (rows + 31u) / 32u;
+
+  // item i of a thread = (row block, rank block, q, lane); element e is row 16 q + 8 (e / 4) + 4 h + e % 4
+  const uint32_t pq = wave & 1u;
+  auto item_block = [&](uint32_t i) { return (4u * i + wave) / (2u * RB); };
+  auto item_rank = [&](uint32_t i) { return (4u * i + wave) / 2u % RB; };
+  auto load_p = [&](uint32_t base, float (&praw)[kItems][8]) {
+#pragma unroll
+    for (uint32_t i = 0; i < kItems; ++i)
+      if (base + item_block(i) * 32u < rows) {  // wave-uniform
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          uint32_t m = base + item_block(i) * 32u + 16u * pq + 8u * (e >> 2) + 4u * h + (e & 3);
+          m = m < rows ? m : rows - 1u;
+          praw[i][e] = psrc[(size_t)(slot0 + m) * kBwdRankStride + item_rank(i) * 32u + c];
+        }
+      }
+  };
+  auto stage_p = [&](uint32_t base, const float (&praw)[kItems][8]) {
+#pragma unroll
+    for (uint32_t i = 0; i < kItems; ++i)
+      if (base + item_block(i) * 32u < rows) {
+        v8us t0, t1, t2;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const uint32_t m = base + item_block(i) * 32u + 16u * pq + 8u * (e >> 2) + 4u * h + (e & 3);
+          const float v = m < rows ? praw[i][e] : 0.0f;
+          const uint32_t b0 = f32_to_bf16_bits(v);
+          const float r1 = v - bf16_bits_to_f32(b0);
+          const uint32_t b1 = f32_to_bf16_bits(r1);
+          const float r2 = r1 - bf16_bits_to_f32(b1);
+          t0[e] = (unsigned short)b0; t1[e] = (unsigned short)b1; t2[e] = (unsigned short)f32_to_bf16_bits(r2);
+        }
+        unsigned char* dst = pop + (((size_t)item_block(i) * RB + item_rank(i)) * 2u + pq) * 3u * kBlockBytes + lane * 16u;
+        *reinterpret_cast<v8us*>(dst) = t0;
+        *reinterpret_cast<v8us*>(dst + kBlockBytes) = t1;
+        *reinterpret_cast<v8us*>(dst + 2 * kBlockBytes) = t2;
+      }
+  };
+  // (the rows' sources first: Q waits for them)
+  int src[kBwdChunkRows / 256u];
+#pragma unroll
+  for (uint32_t i = 0; i < kBwdChunkRows / 256u; ++i) {
+    const uint32_t m = i * 256u + tid < rows ? i * 256u + tid : rows - 1u;
+    src[i] = a.src_row ? a.src_row[slot0 + m] : (int)(slot0 + m);
+  }
+  float praw[kItems][8];
+  load_p(0, praw);
+#pragma unroll
+  for (uint32_t i = 0; i < kBwdChunkRows / 256u; ++i) rowsrc[i * 256u + tid] = i * 256u + tid < rows ? src[i] : -1;
+  lds_barrier();
+
   // identity halves: lane (column c, half h) element e is 1 where the contraction slot 8 h + e is column c
   v8us id0 = {0, 0, 0, 0, 0, 0, 0, 0}, id1 = {0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
@@ -1305,79 +1374,88 @@ __global__ __launch_bounds__(256) void bwd_dlora_kernel(BwdDloraArgs a) {
     for (int b = 0; b < RB; ++b)
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[st][b][e] = 0.0f;
-  const v8us zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
-  auto load_q = [&](uint32_t bi, v8us (&dst)[2][2]) {  // [strip][column half]: row c of the block, 8 columns
-    const int srow = rowsrc[bi * 32u + c];
+  v4i qf[kRing][2][2];  // [strip][column half]: row c of the block, 8 columns
+  bool row_ok[kRing];
+  auto load_q = [&](uint32_t bi, uint32_t u) {
+    const int srow = rowsrc[(bi < n_blocks ? bi : n_blocks - 1u) * 32u + c];
+    row_ok[u] = srow >= 0;
 #pragma unroll
     for (int st = 0; st < 2; ++st)
 #pragma unroll
       for (int hc = 0; hc < 2; ++hc) {
         const uint32_t col = col0 + 32u * st + 16u * hc + 8u * h;
-        dst[st][hc] = (srow >= 0 && col + 8u <= C) ? *reinterpret_cast<const v8us*>(Q + (size_t)srow * C + col) : zero8;
+        qf[u][st][hc] = *reinterpret_cast<const v4i*>(Q + (row_ok[u] && col + 8u <= C ? (size_t)srow * C + col : 0));
       }
   };
-  for (uint32_t base = 0; base < rows; base += kBwdStageRows) {
-    const uint32_t cnt = rows - base < kBwdStageRows ? rows - base : kBwdStageRows;
-    const uint32_t n_blocks = (cnt + 31u) / 32u;
-    __syncthreads();  // the previous pass's operands are no longer read
-    // stage P: item = (row block, rank block, q, lane); element e is row 16 q + 8 (e / 4) + 4 h + e % 4
-    for (uint32_t it = tid; it < n_blocks * RB * 2u * 64u; it += 256u) {
-      const uint32_t l = it & 63u, q = (it >> 6) & 1u, jb = (it >> 7) % RB, bi = (it >> 7) / RB;
-      const uint32_t j = jb * 32u + (l & 31u), hh = l >> 5;
-      v8us t0, t1, t2;
+  auto multiply = [&](uint32_t bi, uint32_t u) {  // bi: the block in the staging pass
+    v8us pf[RB][2][3];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const uint32_t m = bi * 32u + 16u * q + 8u * (e >> 2) + 4u * hh + (e & 3);
-        const float v = m < cnt ? psrc[(size_t)(slot0 + base + m) * kBwdRankStride + j] : 0.0f;
-        const uint32_t b0 = f32_to_bf16_bits(v);
-        const float r1 = v - bf16_bits_to_f32(b0);
-        const uint32_t b1 = f32_to_bf16_bits(r1);
-        const float r2 = r1 - bf16_bits_to_f32(b1);
-        t0[e] = (unsigned short)b0; t1[e] = (unsigned short)b1; t2[e] = (unsigned short)f32_to_bf16_bits(r2);
+    for (int b = 0; b < RB; ++b)
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+#pragma unroll
+        for (int t3 = 0; t3 < 3; ++t3)
+          pf[b][q][t3] = *reinterpret_cast<const v8us*>(pop + ((((size_t)bi * RB + b) * 2u + q) * 3u + t3) * kBlockBytes + lane * 16u);
+    // (they arrive behind the transposition; read one by one each makes its MFMAs wait)
+    if constexpr (RB == 2) __builtin_amdgcn_sched_barrier(0);
+    v4i bq[2][2];
+#pragma unroll
+    for (int st = 0; st < 2; ++st) {
+      v16f tr;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) tr[e] = 0.0f;
+#pragma unroll
+      for (int hc = 0; hc < 2; ++hc) {
+        const bool ok = row_ok[u] && col0 + 32u * st + 16u * hc + 8u * h + 8u <= C;
+        v4i f;
+#pragma unroll
+        for (int d = 0; d < 4; ++d) f[d] = ok ? qf[u][st][hc][d] : 0;
+        tr = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, f), __builtin_bit_cast(v8bf, hc ? id1 : id0), tr, 0, 0, 0);
       }
-      unsigned char* dst = pop + ((((size_t)bi * RB + jb) * 2u + q) * 3u) * kBlockBytes + l * 16u;
-      *reinterpret_cast<v8us*>(dst) = t0;
-      *reinterpret_cast<v8us*>(dst + kBlockBytes) = t1;
-      *reinterpret_cast<v8us*>(dst + 2 * kBlockBytes) = t2;
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) bq[st][q][e] = (int)pack_bf16x2(tr[8 * q + 2 * e], tr[8 * q + 2 * e + 1]);
     }
-    for (uint32_t i = tid; i < kBwdStageRows; i += 256u)
-      rowsrc[i] = i < cnt ? (a.src_row ? a.src_row[slot0 + base + i] : (int)(slot0 + base + i)) : -1;
-    __syncthreads();
+#pragma unroll
+    for (int b = 0; b < RB; ++b)
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+#pragma unroll
+        for (int t3 = 2; t3 >= 0; --t3)
+#pragma unroll
+          for (int st = 0; st < 2; ++st)
+            acc[st][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, pf[b][q][t3]),
+                                                                 __builtin_bit_cast(v8bf, bq[st][q]), acc[st][b], 0, 0, 0);
+  };
+  constexpr uint32_t kPassBlocks = kBwdStageRows / 32u;
+  static_assert(kBwdChunkRows == 2u * kBwdStageRows, "a chunk is two passes");
+  static_assert(kPassBlocks % kRing == 0, "a pass holds whole turns of the ring");
+  if (active) {
+#pragma unroll
+    for (uint32_t u = 0; u < kRing; ++u) load_q(u, u);
+  }
+  stage_p(0, praw);
+  lds_barrier();
+  if constexpr (RB == 2) load_p(kBwdStageRows, praw);
+  for (uint32_t b0 = 0; b0 < n_blocks; b0 += kRing) {
+    if (b0 && b0 % kPassBlocks == 0) {
+      lds_barrier();  // the pass before is no longer read
+      if constexpr (RB == 1) {
+        float pn[kItems][8];
+        load_p(b0 * 32u, pn);
+        stage_p(b0 * 32u, pn);
+      } else {
+        stage_p(b0 * 32u, praw);
+      }
+      lds_barrier();
+    }
     if (!active) continue;
-    v8us qf[2][2];
-    load_q(0, qf);
-    for (uint32_t bi = 0; bi < n_blocks; ++bi) {
-      v8us qn[2][2];
-      if (bi + 1u < n_blocks) load_q(bi + 1u, qn);
+    // (one body: with a second one for the last blocks the allocator copied and spilled the accumulators where they meet)
 #pragma unroll
-      for (int st = 0; st < 2; ++st) {
-        v16f tr;
-#pragma unroll
-        for (int e = 0; e < 16; ++e) tr[e] = 0.0f;
-        tr = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, qf[st][0]), __builtin_bit_cast(v8bf, id0), tr, 0, 0, 0);
-        tr = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, qf[st][1]), __builtin_bit_cast(v8bf, id1), tr, 0, 0, 0);
-        v4i bq[2];
-#pragma unroll
-        for (int q = 0; q < 2; ++q)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) bq[q][e] = (int)pack_bf16x2(tr[8 * q + 2 * e], tr[8 * q + 2 * e + 1]);
-#pragma unroll
-        for (int b = 0; b < RB; ++b)
-#pragma unroll
-          for (int q = 0; q < 2; ++q)
-#pragma unroll
-            for (int t3 = 2; t3 >= 0; --t3) {
-              const v8bf pf = __builtin_bit_cast(
-                  v8bf, *reinterpret_cast<const v8us*>(pop + ((((size_t)bi * RB + b) * 2u + q) * 3u + t3) * kBlockBytes + lane * 16u));
-              acc[st][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pf, __builtin_bit_cast(v8bf, bq[q]), acc[st][b], 0, 0, 0);
-            }
-      }
-      if (bi + 1u < n_blocks) {
-#pragma unroll
-        for (int st = 0; st < 2; ++st)
-#pragma unroll
-          for (int hc = 0; hc < 2; ++hc) qf[st][hc] = qn[st][hc];
-      }
+    for (uint32_t u = 0; u < kRing; ++u) {
+      if (u == 0 || b0 + u < n_blocks) multiply(b0 % kPassBlocks + u, u);
+      load_q(b0 + u + kRing, u);  // behind the last block: its lines again
     }
   }
   if (!active) return;
