@@ -2073,8 +2073,15 @@ int run_gq_linear(const mi355_w8a8_gq_problem* p, hipStream_t s) {
   q.codes_rm = p->aux_x_codes; q.scales_rm = p->aux_x_scales;
   q.M = p->m; q.M_pad = L.m_pad; q.K = p->k; q.K_pad = p->k_pad; q.group = p->group_size; q.G = L.G;
   q.qmax = p->activation_bits == 4u ? 7.0f : 127.0f;
-  // few rows: a row's groups are dealt to several waves so that the launch still fills the chip
-  const uint32_t q_slices = L.m_pad >= 1024u ? 1u : (L.G < 16u ? L.G : 16u);
+  // A row's groups are dealt to several waves: with few rows so that the launch fills the chip (2816 waves), with many so that
+  // a wave that waits for its 3072 values has others beside it.  More waves than that only find less to do each.
+  // One slice from 1024 rows on and 16 below, before, us -> now: K = 12288, groups of 128: 333 rows 13.8 -> 9.5,
+  // 992 23.0 -> 17.5, 1536 30.3 -> 22.3, 4096 54.3 -> 51.8; K = 4096, groups of 64: 700 rows 12.9 -> 7.4, 2048 13.9 -> 13.2;
+  // K = 1024: 992 rows 14.8 -> 5.2, 1536 and more the same single slice (two: 4096 rows 10.5 -> 12.0).
+  uint32_t q_slices = 2816u / L.m_pad;
+  if (q_slices < (p->k + 3071u) / 3072u) q_slices = (p->k + 3071u) / 3072u;
+  if (q_slices > 16u) q_slices = 16u;
+  if (q_slices > L.G) q_slices = L.G;
   q.groups_per_slice = (L.G + q_slices - 1u) / q_slices;
   const uint32_t q_grid_y = (L.G + q.groups_per_slice - 1u) / q.groups_per_slice;
   const bool decode = L.m_pad == 32u;  // few rows: z in K slices instead of row blocks
