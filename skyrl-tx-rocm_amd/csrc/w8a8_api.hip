@@ -212,7 +212,7 @@ int launch_gemm(const GemmArgs& g, uint32_t nkk, hipStream_t s) {
 }
 
 template <int EPI, int NKK, bool PAIR>
-int launch_gemm_ksplit_one(const GemmArgs& g, hipStream_t s) {
+int launch_gemm_ksplit_one(const GemmKSplitArgs& g, hipStream_t s) {
   constexpr int lds_bytes = PAIR ? kGemm64LdsBytes / 2 : kGemm64LdsBytes;
   if (hipFuncSetAttribute(reinterpret_cast<const void*>(&w8a8_gemm_ksplit_kernel<EPI, NKK, PAIR>),
                           hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes) != hipSuccess)
@@ -222,7 +222,7 @@ int launch_gemm_ksplit_one(const GemmArgs& g, hipStream_t s) {
 }
 
 template <int EPI>
-int launch_gemm_ksplit(const GemmArgs& g, uint32_t nkk, hipStream_t s) {
+int launch_gemm_ksplit(const GemmKSplitArgs& g, uint32_t nkk, hipStream_t s) {
   const bool pair = g.tiles_m * g.tiles_n > 256u;
   switch (nkk) {
     case 0: return pair ? launch_gemm_ksplit_one<EPI, 0, true>(g, s) : launch_gemm_ksplit_one<EPI, 0, false>(g, s);
@@ -445,7 +445,7 @@ int launch_quant_rows(const QuantLoraRowsArgs& a, uint32_t nkk, hipStream_t s) {
   }
 }
 
-int launch_quant_split(const QuantLoraArgs& q, bool normalize, hipStream_t s) {
+int launch_quant_split(const QuantLoraSplitArgs& q, bool normalize, hipStream_t s) {
   const dim3 grid(q.n_half_blocks * 4u), block(256);
 #define W8A8_QS(CB)                                                                                        \
   if (normalize) hipLaunchKernelGGL((quant_lora_kernel<CB, true, 4, true>), grid, block, 0, s, q);         \
@@ -632,11 +632,11 @@ int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
   q.nterms = (p->flags & MI355_W8A8_FLAG_LORA_SPLIT2) ? 2u : 3u;
   q.tile_ctr = reinterpret_cast<uint32_t*>(ws + w.tile_ctr);
   q.group_pad = pad_groups ? 32u : 1u;
-  q.zpart = reinterpret_cast<float*>(ws + w.split_z); q.slots = w.rows_bound;
   if (!skip_prologue) {
     const dim3 grid(q.n_half_blocks), block(1024);
     if (split_z) {
-      if ((st = launch_quant_split(q, normalize, s))) return st;
+      QuantLoraSplitArgs qs{q, reinterpret_cast<float*>(ws + w.split_z), w.rows_bound};
+      if ((st = launch_quant_split(qs, normalize, s))) return st;
     } else if (rows_in_lds) {
       QuantLoraRowsArgs qr{};
       qr.q = q;
@@ -684,7 +684,7 @@ int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
   g.blk_range = routed ? blk_range : nullptr;
   g.residual = static_cast<const uint16_t*>(p->residual);
   g.out = p->out;
-  g.M = p->m; g.N = p->n; g.K_pad = w.K_pad; g.KB = w.KB; g.slots = split_z ? q.slots : w.slots;
+  g.M = p->m; g.N = p->n; g.K_pad = w.K_pad; g.KB = w.KB; g.slots = w.slots;
   g.total_rows = w.rows_bound;
   g.groups_per_weight = 1;
   g.tiles_m = w.slots / kTileM;
@@ -709,10 +709,10 @@ int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
   if (wide) return swiglu ? launch_gemm16<kEpiSwiglu>(g, w.nkk, s) : launch_gemm16<kEpiPlain>(g, w.nkk, s);
   if (pair) return swiglu ? launch_gemm16<kEpiSwiglu, 2>(g, w.nkk, s) : launch_gemm16<kEpiPlain, 2>(g, w.nkk, s);
   if (ksplit) {
-    g.tiles_m = ksplit_tiles_m(w.rows_bound);
-    g.tiles_n = (p->n + 127u) / 128u;
-    if (split_z) { g.zpart = q.zpart; g.nterms = q.nterms; }
-    return swiglu ? launch_gemm_ksplit<kEpiSwiglu>(g, w.nkk, s) : launch_gemm_ksplit<kEpiPlain>(g, w.nkk, s);
+    GemmKSplitArgs gk{g, split_z ? reinterpret_cast<const float*>(ws + w.split_z) : nullptr, w.rows_bound, q.nterms};
+    gk.tiles_m = ksplit_tiles_m(w.rows_bound);
+    gk.tiles_n = (p->n + 127u) / 128u;
+    return swiglu ? launch_gemm_ksplit<kEpiSwiglu>(gk, w.nkk, s) : launch_gemm_ksplit<kEpiPlain>(gk, w.nkk, s);
   }
   if (small)
     return swiglu ? launch_gemm<kEpiSwiglu, kModeDense128>(g, w.nkk, s) : launch_gemm<kEpiPlain, kModeDense128>(g, w.nkk, s);

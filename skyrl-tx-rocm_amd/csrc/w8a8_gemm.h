@@ -24,8 +24,6 @@ struct GemmArgs {
   const float* sx;           // f32 [slots]
   const float* sw;           // f32 [N]
   const unsigned char* zp;   // packed z fragments [slots/32][NKK][3][64 lanes][8 bf16] or null
-  const float* zpart;        // f32 [4][slots][16 NKK] whose sum is z, instead of zp (w8a8_gemm_ksplit_kernel), or null
-  uint32_t nterms;           // bf16 terms that z is split into there (3 or 2)
   const float* lora_scaling; // f32 [n_groups]
   const unsigned char* bp;   // LoRA B in MFMA operand order [n_groups][N_pad/32][NKK][64 lanes][8 bf16] or null
   const int32_t* src_row;    // original row of every grouped slot, or null (identity)
@@ -489,8 +487,16 @@ void w8a8_gemm_kernel(GemmArgs g) {
 constexpr int kGemm64TileM = 64;
 constexpr int kGemm64LdsBytes = 4 * 3 * 8192;  // to each wave from the three others: 2 column blocks x 16 registers (PAIR: one)
 
+// What this kernel alone is handed stands behind the arguments of all.  (Amid them it moved what every GEMM kernel reads, whose scalar
+// loads then fell apart: the 128 x 128 geometry took 1 to 2 % longer.)
+struct GemmKSplitArgs : GemmArgs {
+  const float* zpart;  // f32 [4][z_slots][16 NKK] whose sum is z, instead of zp, or null
+  uint32_t z_slots;
+  uint32_t nterms;     // bf16 terms that z is split into (3 or 2)
+};
+
 template <int EPI, int NKK, bool PAIR>
-__global__ __launch_bounds__(256, PAIR ? 2 : 1) void w8a8_gemm_ksplit_kernel(GemmArgs g) {
+__global__ __launch_bounds__(256, PAIR ? 2 : 1) void w8a8_gemm_ksplit_kernel(GemmKSplitArgs g) {
   static_assert(EPI != kEpiAcc, "accumulators are read off the other geometries");
   constexpr int kRing = PAIR ? 3 : 6;
   constexpr int kParts = PAIR ? 2 : 1;  // passes of the sums' exchange
@@ -537,7 +543,7 @@ __global__ __launch_bounds__(256, PAIR ? 2 : 1) void w8a8_gemm_ksplit_kernel(Gem
   };
   auto z_from_quarters = [&](int kk, v8us (&zt)[3]) {
     const float* zq = g.zpart + (size_t)(pblk + c) * (16u * kKK) + 16 * kk + 8u * h;
-    const size_t quarter = (size_t)g.slots * (16u * kKK);
+    const size_t quarter = (size_t)g.z_slots * (16u * kKK);
     v4f q4[4][2];
 #pragma unroll
     for (int p = 0; p < 4; ++p)

@@ -939,8 +939,6 @@ struct QuantLoraArgs {
   float* sx_slots;          // f32 [slots]
   const uint16_t* at;       // LoRA A in MFMA operand order [n_groups][KB][CB][64 lanes][8 bf16] (lora_a_pack_item) or null (CB == 0)
   unsigned char* zp;        // packed z fragments
-  float* zpart;             // SPLIT: f32 [4][slots][16 CB], the quarters' sums
-  uint32_t slots;
   uint32_t r, nkk, nterms;
   uint32_t* tile_ctr;       // 256 words cleared for the GEMM launches' tile counters, or null
   uint32_t group_pad;       // > 1: whole half blocks may be empty
@@ -948,6 +946,11 @@ struct QuantLoraArgs {
   // row_scale then holds a value per source row (scale_by_source) or per row
   const int32_t* row_map;
   uint32_t row_div, row_limit, scale_by_source;
+};
+// the form that leaves z in quarters
+struct QuantLoraSplitArgs : QuantLoraArgs {
+  float* zpart;             // f32 [4][slots][16 CB], the quarters' sums
+  uint32_t slots;
 };
 
 // Row-major copies of the packed codes and of the slots' scales for a caller that asks for them (one workgroup per slot;
@@ -1068,7 +1071,7 @@ __device__ inline void quant_lora_store_z(const QuantLoraArgs& a, v4f (&acc)[kCB
 
 // The sum of a quarter's four tiles (waves w, w + 4, w + 8, w + 12 of the sixteen), in quant_lora_store_z's order.
 template <int kCB>
-__device__ inline void quant_lora_store_quarter(const QuantLoraArgs& a, const v4f (&acc)[kCB], float (*red)[kCB][4][64], uint32_t hb, uint32_t part) {
+__device__ inline void quant_lora_store_quarter(const QuantLoraSplitArgs& a, const v4f (&acc)[kCB], float (*red)[kCB][4][64], uint32_t hb, uint32_t part) {
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
 #pragma unroll
   for (int b = 0; b < kCB; ++b)
@@ -1088,7 +1091,7 @@ __device__ inline void quant_lora_store_quarter(const QuantLoraArgs& a, const v4
 // (w8a8_gemm_ksplit_kernel).  With few rows the sixteen-wave form is a chain of operand fetches in 128 registers a lane
 // (512 KiB of A for a workgroup at K = 4096, rank 64); a quarter of it fits in flight at once.
 template <int CB, bool RMS, uint32_t WAVES = 16, bool SPLIT = false>  // CB: 16-wide rank blocks (0 = no LoRA, 1, 2, 4)
-__global__ __launch_bounds__(WAVES * 64, SPLIT ? 2 : 4) void quant_lora_kernel(QuantLoraArgs a) {
+__global__ __launch_bounds__(WAVES * 64, SPLIT ? 2 : 4) void quant_lora_kernel(std::conditional_t<SPLIT, QuantLoraSplitArgs, QuantLoraArgs> a) {
   static_assert(!SPLIT || (WAVES == 4 && CB > 0), "four workgroups of four waves, for LoRA-A");
   constexpr int kCB = CB > 0 ? CB : 1;
   constexpr uint32_t kStride = SPLIT ? 16 : WAVES;  // k-blocks between two of a wave's
