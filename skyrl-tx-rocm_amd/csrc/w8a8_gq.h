@@ -558,10 +558,11 @@ __device__ inline void gq_store_row_block(const GqGemmArgs& a, const float (&out
 
 // The end of a workgroup's 64 x 128 tile (four waves, 64 x 32 each).  Per 32-row block the scaled low-rank sums are
 // added and the values cast into the LDS, where those of a row change hands, so that sixteen lanes store 256
-// consecutive bytes instead of every lane two.  LDS: behind the batch of the low-rank sums, rows of 272 bytes (16 bytes
-// apart in the banks), then the adapters' factors of the 64 rows.
-constexpr uint32_t kGqOutStride = 272u, kGqOutOff = 16384u, kGqFactorOff = kGqOutOff + 64u * kGqOutStride;
+// consecutive bytes instead of every lane two.  LDS: the batch of the low-rank sums and, once that is read, rows of 272 bytes
+// (16 bytes apart in the banks); behind both z's terms of a step and the adapters' factors of the 64 rows.
+constexpr uint32_t kGqBatchBytes = 32768u, kGqOutStride = 272u, kGqTermOff = kGqBatchBytes, kGqFactorOff = kGqTermOff + 2u * 3u * 1024u;
 constexpr uint32_t kGqEpilogueBytes = kGqFactorOff + 256u;
+static_assert(64u * kGqOutStride <= kGqBatchBytes, "the values take the place of the batch");
 __device__ inline void gq_finish_values(const GqGemmArgs& a, unsigned char* lds, uint32_t i, const v16f& outv,
                                         const v16f& lacc, bool lora, uint32_t row0, uint32_t col0, uint32_t wave, uint32_t lane) {
   typedef __attribute__((address_space(3))) const v4f* lds_f4ptr;
@@ -591,7 +592,7 @@ __device__ inline void gq_finish_values(const GqGemmArgs& a, unsigned char* lds,
         const float low = lacc[4 * q + e] * sg[e];
         y = y + low;
       }
-      *reinterpret_cast<lds_u16ptr>(l + kGqOutOff + (8u * q + e) * kGqOutStride) = (uint16_t)f32_to_bf16_bits(y);
+      *reinterpret_cast<lds_u16ptr>(l + (8u * q + e) * kGqOutStride) = (uint16_t)f32_to_bf16_bits(y);
     }
   }
 }
@@ -600,7 +601,7 @@ __device__ inline void gq_store_tile(const GqGemmArgs& a, unsigned char* lds, ui
                                      uint32_t lane) {
   typedef __attribute__((address_space(3))) unsigned char* lds_ptr;
   typedef __attribute__((address_space(3))) const v4i* lds_i4ptr;
-  const lds_ptr l = (lds_ptr)(lptr_t)lds + kGqOutOff;
+  const lds_ptr l = (lds_ptr)(lptr_t)lds;
   __syncthreads();
   const bool wide = (a.N & 7u) == 0 && (reinterpret_cast<uintptr_t>(a.out) & 15u) == 0;
 #pragma unroll
@@ -620,80 +621,68 @@ __device__ inline void gq_store_tile(const GqGemmArgs& a, unsigned char* lds, ui
   }
 }
 
-// The low-rank sums of one 32-row block of a workgroup's 64 x 128 tile with B staged through the LDS (the stage ring is free by
-// then): per 16 ranks and per batch of up to four adapters present among the block's rows, the four waves
+// The low-rank sums of a workgroup's 64 x 128 tile with B staged through the LDS (the stage ring is free by
+// then): per 16 ranks and per batch of up to eight adapters present among the tile's rows, the four waves
 // bring the adapters' B values of the tile's 128 columns in with direct-to-LDS loads (a slot of 16 ranks x
-// 256 bytes per adapter, 1 KiB per instruction), and every wave then takes its passes -- one per adapter,
-// the rows of the other adapters zeroed -- with its operands from there.  Per output
+// 256 bytes per adapter, 1 KiB per instruction), and every wave then takes its passes -- one per row block and adapter present
+// in it, the rows of the other adapters zeroed -- with its operands from there.  Per output
 // the passes, their order and their operands are those of gq_store_row_block, which asks memory for the
-// same B values once per pass, row block and lane, one dependent round trip after the other.  z comes
-// straight from memory: a lane's eight values of a 16-rank step are 32 consecutive bytes.  Where N % 8 != 0 or B is
-// not aligned to 16 bytes the pieces are read value by value.  Adapters are looked for 64 at a time (the mask).
-// LDS: [0, 16 KiB) the batch.  All four waves must call it; every wave takes column block `wave`.
-constexpr uint32_t kGqLoraLdsBytes = 16384u;
-__device__ inline void gq_tile_lora_sums(const GqGemmArgs& a, unsigned char* lds, uint32_t rb, uint32_t cbase, uint32_t wave,
-                                         uint32_t lane, v16f& lacc) {
+// same B values once per pass, row block and lane, one dependent round trip after the other.  z is on its way
+// with the first batch of a step, and waves 0 and 1 split it into the operands of all four.  Where N % 8 != 0
+// or B is not aligned to 16 bytes the pieces are read value by value.  Adapters are looked for 64 at a time (the masks), once
+// for all ranks.
+// A batch costs its round trip, so both row blocks share it and it holds eight.  The call in batches of four for one row block at a
+// time, z in front of them, us -> now: 4096 x 4096 -> 6144, 4-bit codes in groups of 128, eight adapters of rank 64 310 -> 270, one 226 -> 207;
+// 2300 x 1024 -> 3072, eight of rank 64 83 -> 65.
+// LDS: [0, 32 KiB) the batch, then the operands of z.  All four waves must call it; every wave takes column block `wave` of row blocks rb0, rb0 + 1.
+__device__ inline void gq_tile_lora_sums(const GqGemmArgs& a, unsigned char* lds, uint32_t rb0, uint32_t cbase, uint32_t wave,
+                                         uint32_t lane, v16f (&lacc)[2]) {
   typedef __attribute__((address_space(3))) uint16_t* lds_u16ptr;
   const uint32_t lds_addr = (uint32_t)(uintptr_t)(lptr_t)lds;
   const uint32_t kg = lane >> 5, c = lane & 31u;
-  const uint32_t rowg = rb * 32u + c;
-  int my_ad = -1;  // rows beyond M belong to no adapter
-  uint32_t zrow = 0;
-  if (rowg < a.M) {
-    const int ad = a.idx ? a.idx[rowg] : 0;
-    my_ad = ad < 0 ? 0 : (ad >= (int)a.n_adapters ? (int)a.n_adapters - 1 : ad);
-    zrow = a.z_slot ? (uint32_t)a.z_slot[rowg] : rowg;
+  typedef __attribute__((address_space(3))) v4i* lds_i4ptr;
+  int my_ad[2];
+#pragma unroll
+  for (uint32_t i = 0; i < 2; ++i) {
+    const uint32_t rowg = (rb0 + i) * 32u + c;
+    my_ad[i] = -1;  // rows beyond M belong to no adapter
+    if (rowg < a.M) {
+      const int ad = a.idx ? a.idx[rowg] : 0;
+      my_ad[i] = ad < 0 ? 0 : (ad >= (int)a.n_adapters ? (int)a.n_adapters - 1 : ad);
+    }
   }
+  const uint32_t zrowg = (rb0 + (wave & 1u)) * 32u + c;  // the row whose z the lane splits (waves 0 and 1)
+  const bool z_on = zrowg < a.M;
+  const uint32_t zrow = z_on && a.z_slot ? (uint32_t)a.z_slot[zrowg] : zrowg;
+  const lds_i4ptr terms = reinterpret_cast<lds_i4ptr>((uintptr_t)(lds_addr + kGqTermOff)) + lane;  // [row block][term][lane]
   // what this lane brings in per slot: rank 4 wave + lane / 16 of the step, columns 8 (lane % 16) .. + 7 of the tile
   const uint32_t ld_rank = 4u * wave + (lane >> 4), ld_col = cbase * 32u + (lane & 15u) * 8u;
   const bool pieces = (a.N & 7u) == 0 && (reinterpret_cast<uintptr_t>(a.lora_b) & 15u) == 0;
-  for (uint32_t r0 = 0; r0 < a.r; r0 += 16u) {
-    uint32_t term[3][4];
-    float z8[8];
+  for (uint32_t first = 0; first < a.n_adapters; first += 64u) {
+    unsigned long long present[2] = {0ull, 0ull};  // adapters of the row blocks (the same for all four waves)
 #pragma unroll
-    for (int e = 0; e < 8; ++e) z8[e] = 0.0f;
-    if (my_ad >= 0) {
-      const float* zp = a.z + (size_t)zrow * 64u + r0 + 8u * kg;
-      float4 lo4 = *reinterpret_cast<const float4*>(zp), hi4 = *reinterpret_cast<const float4*>(zp + 4);
+    for (int i = 0; i < 2; ++i) {
+      unsigned long long todo = __builtin_amdgcn_ballot_w64(my_ad[i] >= (int)first && my_ad[i] < (int)(first + 64u));
 #pragma unroll 1
-      for (uint32_t sl = 1; sl < a.z_slices; ++sl) {  // the K slices of the projection, added in order
-        const float4 l2 = *reinterpret_cast<const float4*>(zp + (size_t)sl * a.z_slice_stride);
-        const float4 h2 = *reinterpret_cast<const float4*>(zp + (size_t)sl * a.z_slice_stride + 4);
-        lo4.x = lo4.x + l2.x; lo4.y = lo4.y + l2.y; lo4.z = lo4.z + l2.z; lo4.w = lo4.w + l2.w;
-        hi4.x = hi4.x + h2.x; hi4.y = hi4.y + h2.y; hi4.z = hi4.z + h2.z; hi4.w = hi4.w + h2.w;
+      while (todo) {
+        const int ad = __builtin_amdgcn_readlane(my_ad[i], __builtin_ctzll(todo));
+        present[i] |= 1ull << ((uint32_t)ad - first);
+        todo &= ~__builtin_amdgcn_ballot_w64(my_ad[i] == ad);
       }
-      const float t8[8] = {lo4.x, lo4.y, lo4.z, lo4.w, hi4.x, hi4.y, hi4.z, hi4.w};
-#pragma unroll
-      for (int e = 0; e < 8; ++e) z8[e] = r0 + 8u * kg + (uint32_t)e < a.r ? t8[e] : 0.0f;
     }
-#pragma unroll
-    for (int d = 0; d < 4; ++d) {
-      float hi[2], mid[2], lo[2];
-#pragma unroll
-      for (int e = 0; e < 2; ++e) {
-        const float z = z8[2 * d + e];
-        hi[e] = bf16_round_f32(z);
-        const float r1 = z - hi[e];
-        mid[e] = bf16_round_f32(r1);
-        lo[e] = bf16_round_f32(r1 - mid[e]);
-      }
-      term[0][d] = pack_bf16x2(hi[0], hi[1]);
-      term[1][d] = pack_bf16x2(mid[0], mid[1]);
-      term[2][d] = pack_bf16x2(lo[0], lo[1]);
-    }
-    const bool ld_on = r0 + ld_rank < a.r && ld_col < a.N;
-    const uint32_t ld_off = ((r0 + ld_rank) * a.N + ld_col) * 2u;
-    for (uint32_t first = 0; first < a.n_adapters; first += 64u) {
-      unsigned long long rem = 0ull;  // adapters of the block's rows (the same for all four waves)
 #pragma unroll 1
-      for (uint32_t ad = 0; ad < 64u && first + ad < a.n_adapters; ++ad)
-        if (__builtin_amdgcn_ballot_w64(my_ad == (int)(first + ad)) != 0) rem |= 1ull << ad;
-      while (rem) {  // batches of up to four adapters, smallest first (workgroup-uniform)
+    for (uint32_t r0 = 0; r0 < a.r; r0 += 16u) {
+      const bool ld_on = r0 + ld_rank < a.r && ld_col < a.N;
+      const uint32_t ld_off = ((r0 + ld_rank) * a.N + ld_col) * 2u;
+      unsigned long long rem = present[0] | present[1];
+      bool fresh = true;  // z of this step is not here yet
+#pragma unroll 1
+      while (rem) {  // batches of up to eight adapters, smallest first (workgroup-uniform)
         __syncthreads();  // the batch before has been read
         unsigned long long batch = rem;
         uint32_t nb = 0;
 #pragma unroll 1
-        for (; rem && nb < 4u; ++nb, rem &= rem - 1ull) {
+        for (; rem && nb < 8u; ++nb, rem &= rem - 1ull) {
           const unsigned char* const b = reinterpret_cast<const unsigned char*>(a.lora_b) +
                                          (size_t)(first + (uint32_t)__builtin_ctzll(rem)) * a.r * a.N * 2u;
           const uint32_t dst = nb * 4096u + wave * 1024u;
@@ -705,11 +694,49 @@ __device__ inline void gq_tile_lora_sums(const GqGemmArgs& a, unsigned char* lds
               reinterpret_cast<lds_u16ptr>((lptr_t)lds)[dst / 2u + lane * 8u + e] = *reinterpret_cast<const uint16_t*>(b + ld_off + 2u * e);
           }
         }
+        if (fresh && wave < 2u) {
+          float z8[8];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) z8[e] = 0.0f;
+          if (z_on) {
+            const float* zp = a.z + (size_t)zrow * 64u + r0 + 8u * kg;
+            float4 lo4 = *reinterpret_cast<const float4*>(zp), hi4 = *reinterpret_cast<const float4*>(zp + 4);
+#pragma unroll 1
+            for (uint32_t sl = 1; sl < a.z_slices; ++sl) {  // the K slices of the projection, added in order
+              const float4 l2 = *reinterpret_cast<const float4*>(zp + (size_t)sl * a.z_slice_stride);
+              const float4 h2 = *reinterpret_cast<const float4*>(zp + (size_t)sl * a.z_slice_stride + 4);
+              lo4.x = lo4.x + l2.x; lo4.y = lo4.y + l2.y; lo4.z = lo4.z + l2.z; lo4.w = lo4.w + l2.w;
+              hi4.x = hi4.x + h2.x; hi4.y = hi4.y + h2.y; hi4.z = hi4.z + h2.z; hi4.w = hi4.w + h2.w;
+            }
+            const float t8[8] = {lo4.x, lo4.y, lo4.z, lo4.w, hi4.x, hi4.y, hi4.z, hi4.w};
+#pragma unroll
+            for (int e = 0; e < 8; ++e) z8[e] = r0 + 8u * kg + (uint32_t)e < a.r ? t8[e] : 0.0f;
+          }
+          v4i term[3];
+#pragma unroll
+          for (int d = 0; d < 4; ++d) {
+            float hi[2], mid[2], lo[2];
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+              const float z = z8[2 * d + e];
+              hi[e] = bf16_round_f32(z);
+              const float r1 = z - hi[e];
+              mid[e] = bf16_round_f32(r1);
+              lo[e] = bf16_round_f32(r1 - mid[e]);
+            }
+            term[0][d] = (int)pack_bf16x2(hi[0], hi[1]);
+            term[1][d] = (int)pack_bf16x2(mid[0], mid[1]);
+            term[2][d] = (int)pack_bf16x2(lo[0], lo[1]);
+          }
+#pragma unroll
+          for (uint32_t t = 0; t < 3; ++t) terms[(wave * 3u + t) * 64u] = term[t];
+        }
+        fresh = false;
         wait_vmcnt<0>();
         __syncthreads();
 #pragma unroll 1
         for (uint32_t sl = 0; sl < nb; ++sl, batch &= batch - 1ull) {
-          const bool mine = my_ad == (int)(first + (uint32_t)__builtin_ctzll(batch));
+          const uint32_t ad = (uint32_t)__builtin_ctzll(batch);
           const uint32_t lcol = wave * 32u + c;
           const bool col_ok = cbase * 32u + lcol < a.N;
           uint32_t braw[8];
@@ -723,11 +750,16 @@ __device__ inline void gq_tile_lora_sums(const GqGemmArgs& a, unsigned char* lds
 #pragma unroll
           for (int d = 0; d < 4; ++d) bo[d] = (int)(braw[2 * d] | (braw[2 * d + 1] << 16));
 #pragma unroll
-          for (int t = 2; t >= 0; --t) {
-            v4i za;
+          for (int i = 0; i < 2; ++i) {
+            if (!((present[i] >> ad) & 1ull)) continue;  // wave-uniform
+            const bool mine = my_ad[i] == (int)(first + ad);
 #pragma unroll
-            for (int d = 0; d < 4; ++d) za[d] = mine ? (int)term[t][d] : 0;
-            lacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, za), __builtin_bit_cast(v8bf, bo), lacc, 0, 0, 0);
+            for (int t = 2; t >= 0; --t) {
+              v4i za = terms[(i * 3 + t) * 64];
+#pragma unroll
+              for (int d = 0; d < 4; ++d) za[d] = mine ? za[d] : 0;
+              lacc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, za), __builtin_bit_cast(v8bf, bo), lacc[i], 0, 0, 0);
+            }
           }
         }
       }
@@ -875,14 +907,14 @@ constexpr float kGqSumOffset = 12582912.0f;
 constexpr uint32_t kGqTileRows = 64u, kGqTileCols = 128u;
 __host__ __device__ constexpr uint32_t gq_lds_stages(bool w4) { return w4 ? 4u : 3u; }
 __host__ __device__ constexpr uint32_t gq_lds_stage_bytes(bool w4) { return 4096u + (w4 ? 4096u : 8192u) + 1024u; }
-__host__ __device__ constexpr uint32_t gq_lds_bytes(bool w4) { return gq_lds_stages(w4) * gq_lds_stage_bytes(w4); }
-static_assert(gq_lds_bytes(true) >= kGqEpilogueBytes && gq_lds_bytes(false) >= kGqEpilogueBytes && kGqLoraLdsBytes <= kGqOutOff,
-              "the epilogue reuses the ring");
+__host__ __device__ constexpr uint32_t gq_lds_bytes(bool w4) {  // the ring, then the epilogue
+  return gq_lds_stages(w4) * gq_lds_stage_bytes(w4) > kGqEpilogueBytes ? gq_lds_stages(w4) * gq_lds_stage_bytes(w4) : kGqEpilogueBytes;
+}
 static_assert(4u * gq_lds_bytes(true) <= 160u * 1024u && 4u * gq_lds_bytes(false) <= 160u * 1024u, "four workgroups per CU");
 
 template <bool W4, bool SMALL>
 __global__ __launch_bounds__(256, 4) void gq_gemm_lds_kernel(GqGemmArgs a) {
-  extern __shared__ __attribute__((aligned(1024))) unsigned char gq_lds[];  // the stage ring; the epilogue's z rows afterwards
+  extern __shared__ __attribute__((aligned(1024))) unsigned char gq_lds[];  // the stage ring; the epilogue's batches of B and values afterwards
   constexpr uint32_t kStage = gq_lds_stage_bytes(W4), kWOff = 4096u, kSOff = kWOff + (W4 ? 4096u : 8192u);
   constexpr uint32_t kWBlk = W4 ? 512u : 1024u;      // bytes of a weight fragment (one column block, one k block)
   constexpr uint32_t kLoads = 1u + (W4 ? 1u : 2u) + 1u;  // direct-to-LDS loads per wave and stage
@@ -1042,15 +1074,17 @@ __global__ __launch_bounds__(256, 4) void gq_gemm_lds_kernel(GqGemmArgs a) {
     }
     __syncthreads();
   }
-#pragma unroll 1
-  for (uint32_t i = 0; i < 2; ++i) {
-    v16f lacc;
+  v16f lacc[2];
 #pragma unroll
-    for (int v = 0; v < 16; ++v) lacc[v] = 0.0f;
-    if (lora) gq_tile_lora_sums(a, gq_lds, rbase + i, cbase, wave, lane, lacc);  // workgroup-uniform
-    gq_finish_values(a, gq_lds, i, outv[0], lacc, lora, rbase * 32u, cbase * 32u, wave, lane);
-    outv[0] = outv[1];
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) lacc[i][v] = 0.0f;
+  if (lora) {  // workgroup-uniform
+    gq_tile_lora_sums(a, gq_lds, rbase, cbase, wave, lane, lacc);
+    __syncthreads();  // the last batch has been read
   }
+#pragma unroll
+  for (uint32_t i = 0; i < 2; ++i) gq_finish_values(a, gq_lds, i, outv[i], lacc[i], lora, rbase * 32u, cbase * 32u, wave, lane);
   gq_store_tile(a, gq_lds, rbase * 32u, cbase * 32u, wave, lane);
 }
 
