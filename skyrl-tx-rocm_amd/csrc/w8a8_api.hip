@@ -2034,6 +2034,19 @@ int run_gq_pack(const void* codes, void* packed, uint32_t k_pad, uint32_t n, uin
   return launch_status();
 }
 
+// Whether the staged group-scaled product of 8-bit codes in groups beyond kGqSmallGroup takes 128 x 128 tiles (512 places) instead of
+// 64 x 128 (1024): with little scaling between the MFMAs the operands' way from the L2 counts, 17 KiB a stage for twice
+// the outputs instead of 13, and a long K repays the taller tile's longer fill and end.  Where the places of a first round are nearly all taken,
+// or beyond one and a half.  Whole call, 64 x 128 / 128 x 128, one adapter of rank 32: 12288 -> 4096, groups of 1024: 1536 rows (768 tiles of 64 x 128) 141 us / 138,
+// 2048 180 / 163, 2560 228 / 251, 3072 269 / 267, 4096 338 / 307, 8192 686 / 629, groups of 512 347 / 322 and 697 / 651; 12288 -> 2560, 3072 rows
+// (960) 200 / 181, 4096 (1280) 247 / 267; 8192 -> 2048, 4096 rows 153 / 143; 6144 -> 4096, 4096 rows 184 / 173; 4096 -> 12288, groups of 512, 3072 rows
+// 262 / 272; 2048 -> 8192, 4096 rows 137 / 145.  Groups of 256 7 % better at 12288 and 1 to 5 % worse at 4096 and below, of 128 level or worse.
+constexpr uint32_t kGqTallMinK = 6144u;
+inline bool gq_tall_tiles_pay(uint32_t m, uint32_t k_pad, uint32_t n) {
+  const uint64_t tiles = (uint64_t)((m + 63u) / 64u) * ((n + kGqTileCols - 1u) / kGqTileCols);
+  return k_pad >= kGqTallMinK && ((tiles > 896u && tiles <= 1024u) || tiles > 1600u);
+}
+
 int run_gq_linear(const mi355_w8a8_gq_problem* p, hipStream_t s) {
   if (!p) return MI355_W8A8_ERR_NULL;
   if (p->struct_size != sizeof(mi355_w8a8_gq_problem)) return MI355_W8A8_ERR_STRUCT;
@@ -2196,15 +2209,18 @@ int run_gq_linear(const mi355_w8a8_gq_problem* p, hipStream_t s) {
     return launch_status();
   }
   if (p->group_size % 64u == 0 && !(p->flags & MI355_W8A8_FLAG_GQ_DIRECT)) {
-    // groups of whole 64-wide k steps: 64 x 128 tiles staged through the LDS
-    const dim3 grid((p->n + kGqTileCols - 1u) / kGqTileCols, (L.m_pad + kGqTileRows - 1u) / kGqTileRows), block(256);
+    // groups of whole 64-wide k steps: tiles of 64 or 128 rows x 128 columns staged through the LDS
     const bool w4 = p->weight_bits == 4u, small = p->group_size <= kGqSmallGroup;
-    const auto kernel = w4 ? (small ? &gq_gemm_lds_kernel<true, true> : &gq_gemm_lds_kernel<true, false>)
-                           : (small ? &gq_gemm_lds_kernel<false, true> : &gq_gemm_lds_kernel<false, false>);
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                            (int)gq_lds_bytes(w4)) != hipSuccess)
+    const bool tall = !w4 && !small && gq_tall_tiles_pay(p->m, p->k_pad, p->n);
+    const uint32_t rb = tall ? 4u : 2u;
+    const dim3 grid((p->n + kGqTileCols - 1u) / kGqTileCols, (L.m_pad + rb * 32u - 1u) / (rb * 32u)), block(256);
+    const auto kernel = tall ? &gq_gemm_lds_kernel<false, false, 4>
+                        : w4 ? (small ? &gq_gemm_lds_kernel<true, true, 2> : &gq_gemm_lds_kernel<true, false, 2>)
+                             : (small ? &gq_gemm_lds_kernel<false, true, 2> : &gq_gemm_lds_kernel<false, false, 2>);
+    const uint32_t lds_bytes = gq_lds_bytes(w4, rb);
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes) != hipSuccess)
       return MI355_W8A8_ERR_LAUNCH;
-    hipLaunchKernelGGL(kernel, grid, block, gq_lds_bytes(w4), s, g);
+    hipLaunchKernelGGL(kernel, grid, block, lds_bytes, s, g);
     return launch_status();
   }
   const dim3 grid((g.n_col_blocks + 7u) / 8u, (L.m_pad / 32u + 1u) / 2u), block(256);

@@ -556,13 +556,15 @@ __device__ inline void gq_store_row_block(const GqGemmArgs& a, const float (&out
   gq_finish_row_block(a, outv, lacc, lora, rb, col, two_cols, lane);
 }
 
-// The end of a workgroup's 64 x 128 tile (four waves, 64 x 32 each).  Per 32-row block the scaled low-rank sums are
+// The end of a workgroup's tile of RB row blocks x 128 columns (four waves, 32 columns each).  Per 32-row block the scaled low-rank sums are
 // added and the values cast into the LDS, where those of a row change hands, so that sixteen lanes store 256
-// consecutive bytes instead of every lane two.  LDS: the batch of the low-rank sums and, once that is read, rows of 272 bytes
-// (16 bytes apart in the banks); behind both z's terms of a step and the adapters' factors of the 64 rows.
-constexpr uint32_t kGqBatchBytes = 32768u, kGqOutStride = 272u, kGqTermOff = kGqBatchBytes, kGqFactorOff = kGqTermOff + 2u * 3u * 1024u;
-constexpr uint32_t kGqEpilogueBytes = kGqFactorOff + 256u;
-static_assert(64u * kGqOutStride <= kGqBatchBytes, "the values take the place of the batch");
+// consecutive bytes instead of every lane two.  LDS: the batch of the low-rank sums and z's terms of a step; once they are
+// read, rows of 272 bytes (16 bytes apart in the banks); behind both the adapters' factors of the tile's rows.
+constexpr uint32_t kGqBatchBytes = 32768u, kGqOutStride = 272u, kGqTermOff = kGqBatchBytes;
+__host__ __device__ constexpr uint32_t gq_factor_off(uint32_t rb) { return kGqTermOff + rb * 3u * 1024u; }
+__host__ __device__ constexpr uint32_t gq_epilogue_bytes(uint32_t rb) { return gq_factor_off(rb) + rb * 128u; }
+static_assert(2u * 32u * kGqOutStride <= gq_factor_off(2) && 4u * 32u * kGqOutStride <= gq_factor_off(4), "the values take the place of the batch");
+template <int RB>
 __device__ inline void gq_finish_values(const GqGemmArgs& a, unsigned char* lds, uint32_t i, const v16f& outv,
                                         const v16f& lacc, bool lora, uint32_t row0, uint32_t col0, uint32_t wave, uint32_t lane) {
   typedef __attribute__((address_space(3))) const v4f* lds_f4ptr;
@@ -584,7 +586,7 @@ __device__ inline void gq_finish_values(const GqGemmArgs& a, unsigned char* lds,
 #pragma unroll
   for (uint32_t q = 0; q < 4; ++q) {  // four consecutive rows
     v4f sg = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (lora) sg = *reinterpret_cast<lds_f4ptr>((lds_ptr)(lptr_t)lds + kGqFactorOff + (r0 + 8u * q) * 4u);
+    if (lora) sg = *reinterpret_cast<lds_f4ptr>((lds_ptr)(lptr_t)lds + gq_factor_off(RB) + (r0 + 8u * q) * 4u);
 #pragma unroll
     for (uint32_t e = 0; e < 4; ++e) {
       float y = outv[4 * q + e];
@@ -597,6 +599,7 @@ __device__ inline void gq_finish_values(const GqGemmArgs& a, unsigned char* lds,
   }
 }
 
+template <int RB>
 __device__ inline void gq_store_tile(const GqGemmArgs& a, unsigned char* lds, uint32_t row0, uint32_t col0, uint32_t wave,
                                      uint32_t lane) {
   typedef __attribute__((address_space(3))) unsigned char* lds_ptr;
@@ -605,7 +608,7 @@ __device__ inline void gq_store_tile(const GqGemmArgs& a, unsigned char* lds, ui
   __syncthreads();
   const bool wide = (a.N & 7u) == 0 && (reinterpret_cast<uintptr_t>(a.out) & 15u) == 0;
 #pragma unroll
-  for (uint32_t p = 0; p < 4; ++p) {  // 64 rows x 16 pieces of 8 columns
+  for (uint32_t p = 0; p < 2u * RB; ++p) {  // rows x 16 pieces of 8 columns
     const uint32_t rl = p * 16u + wave * 4u + (lane >> 4), cl = (lane & 15u) * 8u;
     const uint32_t row = row0 + rl;
     if (row >= a.M || col0 + cl >= a.N) continue;
@@ -621,29 +624,30 @@ __device__ inline void gq_store_tile(const GqGemmArgs& a, unsigned char* lds, ui
   }
 }
 
-// The low-rank sums of a workgroup's 64 x 128 tile with B staged through the LDS (the stage ring is free by
+// The low-rank sums of a workgroup's tile with B staged through the LDS (the stage ring is free by
 // then): per 16 ranks and per batch of up to eight adapters present among the tile's rows, the four waves
 // bring the adapters' B values of the tile's 128 columns in with direct-to-LDS loads (a slot of 16 ranks x
 // 256 bytes per adapter, 1 KiB per instruction), and every wave then takes its passes -- one per row block and adapter present
 // in it, the rows of the other adapters zeroed -- with its operands from there.  Per output
 // the passes, their order and their operands are those of gq_store_row_block, which asks memory for the
 // same B values once per pass, row block and lane, one dependent round trip after the other.  z is on its way
-// with the first batch of a step, and waves 0 and 1 split it into the operands of all four.  Where N % 8 != 0
+// with the first batch of a step, and a wave splits a row block's into the operands of all four.  Where N % 8 != 0
 // or B is not aligned to 16 bytes the pieces are read value by value.  Adapters are looked for 64 at a time (the masks), once
 // for all ranks.
-// A batch costs its round trip, so both row blocks share it and it holds eight.  The call in batches of four for one row block at a
+// A batch costs its round trip, so the row blocks share it and it holds eight.  The call in batches of four for one row block at a
 // time, z in front of them, us -> now: 4096 x 4096 -> 6144, 4-bit codes in groups of 128, eight adapters of rank 64 310 -> 270, one 226 -> 207;
 // 2300 x 1024 -> 3072, eight of rank 64 83 -> 65.
-// LDS: [0, 32 KiB) the batch, then the operands of z.  All four waves must call it; every wave takes column block `wave` of row blocks rb0, rb0 + 1.
+// LDS: [0, 32 KiB) the batch, then the operands of z.  All four waves must call it; every wave takes column block `wave` of row blocks rb0 ..
+template <int RB>
 __device__ inline void gq_tile_lora_sums(const GqGemmArgs& a, unsigned char* lds, uint32_t rb0, uint32_t cbase, uint32_t wave,
-                                         uint32_t lane, v16f (&lacc)[2]) {
+                                         uint32_t lane, v16f (&lacc)[RB]) {
   typedef __attribute__((address_space(3))) uint16_t* lds_u16ptr;
   const uint32_t lds_addr = (uint32_t)(uintptr_t)(lptr_t)lds;
   const uint32_t kg = lane >> 5, c = lane & 31u;
   typedef __attribute__((address_space(3))) v4i* lds_i4ptr;
-  int my_ad[2];
+  int my_ad[RB];
 #pragma unroll
-  for (uint32_t i = 0; i < 2; ++i) {
+  for (uint32_t i = 0; i < RB; ++i) {
     const uint32_t rowg = (rb0 + i) * 32u + c;
     my_ad[i] = -1;  // rows beyond M belong to no adapter
     if (rowg < a.M) {
@@ -651,7 +655,7 @@ __device__ inline void gq_tile_lora_sums(const GqGemmArgs& a, unsigned char* lds
       my_ad[i] = ad < 0 ? 0 : (ad >= (int)a.n_adapters ? (int)a.n_adapters - 1 : ad);
     }
   }
-  const uint32_t zrowg = (rb0 + (wave & 1u)) * 32u + c;  // the row whose z the lane splits (waves 0 and 1)
+  const uint32_t zrowg = (rb0 + wave % RB) * 32u + c;  // the row whose z the lane splits (waves below RB)
   const bool z_on = zrowg < a.M;
   const uint32_t zrow = z_on && a.z_slot ? (uint32_t)a.z_slot[zrowg] : zrowg;
   const lds_i4ptr terms = reinterpret_cast<lds_i4ptr>((uintptr_t)(lds_addr + kGqTermOff)) + lane;  // [row block][term][lane]
@@ -659,9 +663,10 @@ __device__ inline void gq_tile_lora_sums(const GqGemmArgs& a, unsigned char* lds
   const uint32_t ld_rank = 4u * wave + (lane >> 4), ld_col = cbase * 32u + (lane & 15u) * 8u;
   const bool pieces = (a.N & 7u) == 0 && (reinterpret_cast<uintptr_t>(a.lora_b) & 15u) == 0;
   for (uint32_t first = 0; first < a.n_adapters; first += 64u) {
-    unsigned long long present[2] = {0ull, 0ull};  // adapters of the row blocks (the same for all four waves)
+    unsigned long long present[RB], all = 0ull;  // adapters of the row blocks (the same for all four waves)
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < RB; ++i) {
+      present[i] = 0ull;
       unsigned long long todo = __builtin_amdgcn_ballot_w64(my_ad[i] >= (int)first && my_ad[i] < (int)(first + 64u));
 #pragma unroll 1
       while (todo) {
@@ -669,12 +674,13 @@ __device__ inline void gq_tile_lora_sums(const GqGemmArgs& a, unsigned char* lds
         present[i] |= 1ull << ((uint32_t)ad - first);
         todo &= ~__builtin_amdgcn_ballot_w64(my_ad[i] == ad);
       }
+      all |= present[i];
     }
 #pragma unroll 1
     for (uint32_t r0 = 0; r0 < a.r; r0 += 16u) {
       const bool ld_on = r0 + ld_rank < a.r && ld_col < a.N;
       const uint32_t ld_off = ((r0 + ld_rank) * a.N + ld_col) * 2u;
-      unsigned long long rem = present[0] | present[1];
+      unsigned long long rem = all;
       bool fresh = true;  // z of this step is not here yet
 #pragma unroll 1
       while (rem) {  // batches of up to eight adapters, smallest first (workgroup-uniform)
@@ -694,7 +700,7 @@ __device__ inline void gq_tile_lora_sums(const GqGemmArgs& a, unsigned char* lds
               reinterpret_cast<lds_u16ptr>((lptr_t)lds)[dst / 2u + lane * 8u + e] = *reinterpret_cast<const uint16_t*>(b + ld_off + 2u * e);
           }
         }
-        if (fresh && wave < 2u) {
+        if (fresh && wave < (uint32_t)RB) {
           float z8[8];
 #pragma unroll
           for (int e = 0; e < 8; ++e) z8[e] = 0.0f;
@@ -750,7 +756,7 @@ __device__ inline void gq_tile_lora_sums(const GqGemmArgs& a, unsigned char* lds
 #pragma unroll
           for (int d = 0; d < 4; ++d) bo[d] = (int)(braw[2 * d] | (braw[2 * d + 1] << 16));
 #pragma unroll
-          for (int i = 0; i < 2; ++i) {
+          for (int i = 0; i < RB; ++i) {
             if (!((present[i] >> ad) & 1ull)) continue;  // wave-uniform
             const bool mine = my_ad[i] == (int)(first + ad);
 #pragma unroll
@@ -885,9 +891,9 @@ __global__ __launch_bounds__(256, 2) void gq_gemm_kernel(GqGemmArgs a) {
 
 // ---------------------------------------------------------------------------------------
 // The same product for groups that are multiples of 64 k, staged through the LDS: a workgroup of four
-// waves owns a 64 x 128 output tile, a wave 64 x 32 of it; per 64-wide k step its activation fragments (4 KiB),
-// weight fragments (4 or 8 KiB) and the group's scales (128 column and 64 row scales) arrive once per
-// workgroup by direct-to-LDS loads, two or three steps ahead, and every wave reads its fragments from
+// waves owns an output tile of RB row blocks x 128 columns, 64 x 128 or 128 x 128, a wave all its rows x 32; per 64-wide k step its
+// activation fragments (2 KiB a row block), weight fragments (4 or 8 KiB) and the group's scales (128 column and 64 or 128 row
+// scales) arrive once per workgroup by direct-to-LDS loads, two or three steps ahead, and every wave reads its fragments from
 // there.  Per output the arithmetic and its order are those of gq_gemm_kernel (the step and the epilogue
 // are shared), so the two kernels agree bit for bit.
 // Bound by instruction issue: four vector operations per output and group beside group / 32 MFMAs per block.  A wave
@@ -897,6 +903,7 @@ __global__ __launch_bounds__(256, 2) void gq_gemm_kernel(GqGemmArgs a) {
 // columns are 768 workgroups for 1024 places instead of 384 for 512.  The ring's places are unrolled (28 scalar
 // instructions a stage instead of 43).  K = 12288, N = 4096: 4096 rows, 4-bit codes in groups of 128 387 -> 350 us;
 // 1536 rows, 8-bit codes in groups of 64 214 -> 192 us.
+// In long groups little of that is left and the operands' way bounds it: 128 x 128 where gq_tall_tiles_pay says so.
 // Sums of at most kGqSmallGroup products leave the matrix core as float32 values: v_cvt_f32_i32 takes 4.3 cycles of a
 // SIMD with several waves, a subtraction 2.5 (399 -> 383 us at 4096 rows as above).  The accumulators start at the bit pattern of 1.5 * 2^23, a float32 whose last place is
 // one: while |s| < 2^22 (here at most 256 * 128 * 127) the pattern plus s reads as 1.5 * 2^23 + s, and one subtraction
@@ -904,21 +911,24 @@ __global__ __launch_bounds__(256, 2) void gq_gemm_kernel(GqGemmArgs a) {
 constexpr uint32_t kGqSmallGroup = 256u;
 constexpr int kGqSumOrigin = 0x4b400000;
 constexpr float kGqSumOffset = 12582912.0f;
-constexpr uint32_t kGqTileRows = 64u, kGqTileCols = 128u;
-__host__ __device__ constexpr uint32_t gq_lds_stages(bool w4) { return w4 ? 4u : 3u; }
-__host__ __device__ constexpr uint32_t gq_lds_stage_bytes(bool w4) { return 4096u + (w4 ? 4096u : 8192u) + 1024u; }
-__host__ __device__ constexpr uint32_t gq_lds_bytes(bool w4) {  // the ring, then the epilogue
-  return gq_lds_stages(w4) * gq_lds_stage_bytes(w4) > kGqEpilogueBytes ? gq_lds_stages(w4) * gq_lds_stage_bytes(w4) : kGqEpilogueBytes;
+constexpr uint32_t kGqTileCols = 128u;
+// (rb: row blocks of a tile)
+__host__ __device__ constexpr uint32_t gq_lds_stages(bool w4, uint32_t rb) { return w4 || rb == 4u ? 4u : 3u; }
+__host__ __device__ constexpr uint32_t gq_lds_stage_bytes(bool w4, uint32_t rb) { return rb * 2048u + (w4 ? 4096u : 8192u) + 1024u; }
+__host__ __device__ constexpr uint32_t gq_lds_bytes(bool w4, uint32_t rb) {  // the ring, then the epilogue
+  const uint32_t ring = gq_lds_stages(w4, rb) * gq_lds_stage_bytes(w4, rb);
+  return ring > gq_epilogue_bytes(rb) ? ring : gq_epilogue_bytes(rb);
 }
-static_assert(4u * gq_lds_bytes(true) <= 160u * 1024u && 4u * gq_lds_bytes(false) <= 160u * 1024u, "four workgroups per CU");
+static_assert(4u * gq_lds_bytes(true, 2) <= 160u * 1024u && 4u * gq_lds_bytes(false, 2) <= 160u * 1024u, "four workgroups per CU");
+static_assert(2u * gq_lds_bytes(false, 4) <= 160u * 1024u, "two workgroups per CU");
 
-template <bool W4, bool SMALL>
-__global__ __launch_bounds__(256, 4) void gq_gemm_lds_kernel(GqGemmArgs a) {
+template <bool W4, bool SMALL, int RB>
+__global__ __launch_bounds__(256, RB == 2 ? 4 : 2) void gq_gemm_lds_kernel(GqGemmArgs a) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char gq_lds[];  // the stage ring; the epilogue's batches of B and values afterwards
-  constexpr uint32_t kStage = gq_lds_stage_bytes(W4), kWOff = 4096u, kSOff = kWOff + (W4 ? 4096u : 8192u);
+  constexpr uint32_t kStage = gq_lds_stage_bytes(W4, RB), kWOff = RB * 2048u, kSOff = kWOff + (W4 ? 4096u : 8192u);
   constexpr uint32_t kWBlk = W4 ? 512u : 1024u;      // bytes of a weight fragment (one column block, one k block)
-  constexpr uint32_t kLoads = 1u + (W4 ? 1u : 2u) + 1u;  // direct-to-LDS loads per wave and stage
-  constexpr uint32_t NS = gq_lds_stages(W4);
+  constexpr uint32_t kLoads = RB / 2u + (W4 ? 1u : 2u) + 1u;  // direct-to-LDS loads per wave and stage
+  constexpr uint32_t NS = gq_lds_stages(W4, RB);
   typedef __attribute__((address_space(3))) const unsigned char* lds_cptr;
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -926,22 +936,22 @@ __global__ __launch_bounds__(256, 4) void gq_gemm_lds_kernel(GqGemmArgs a) {
   const uint32_t kbs = a.K_pad / 32u, blocks_per_group = a.group / 32u;  // both even here
   const uint32_t n_stages = kbs / 2u;
   const uint32_t n_rb = a.M_pad / 32u;
-  const uint32_t rbase = blockIdx.y * 2u, cbase = blockIdx.x * 4u;
+  const uint32_t rbase = blockIdx.y * RB, cbase = blockIdx.x * 4u;
   // blocks that hang over the edge are read from the last valid one; their results are never stored
   auto rb_of = [&](uint32_t l) { return rbase + l < n_rb ? rbase + l : n_rb - 1u; };
   auto cb_of = [&](uint32_t l) { return cbase + l < a.n_col_blocks ? cbase + l : a.n_col_blocks - 1u; };
   const uint32_t lds0 = (uint32_t)(uintptr_t)(lptr_t)gq_lds;
   // what this wave brings in per stage: k block `wave` % 2 of row block `wave` / 2 (1 KiB), column block `wave`
   // (1 or 2 KiB), 64 scales (columns, columns, rows, and the rows once more so that all waves count alike)
-  const unsigned char* a_src =
-      reinterpret_cast<const unsigned char*>(a.codes) + ((size_t)rb_of(wave >> 1) * kbs + (wave & 1u)) * 1024u;
+  const unsigned char* a_src = reinterpret_cast<const unsigned char*>(a.codes) +
+                               (RB == 2 ? (size_t)rb_of(wave >> 1) * kbs + (wave & 1u) : (size_t)rb_of(wave) * kbs) * 1024u;
   const unsigned char* w_src = a.wp + (size_t)cb_of(wave) * kbs * kWBlk;
   uint32_t s_idx;  // the lane's scale of a group, clamped to the last one
   if (wave < 2u) {
     const uint32_t cc = cbase * 32u + wave * 64u + lane;
     s_idx = cc < a.N ? cc : a.N - 1u;
   } else {
-    const uint32_t rr = rbase * 32u + lane;
+    const uint32_t rr = rbase * 32u + (RB == 4 ? (wave - 2u) * 64u : 0u) + lane;
     s_idx = rr < a.M_pad ? rr : a.M_pad - 1u;
   }
   const uint32_t stages_per_group = blocks_per_group / 2u;
@@ -952,7 +962,8 @@ __global__ __launch_bounds__(256, 4) void gq_gemm_lds_kernel(GqGemmArgs a) {
   // that every stage waits for the same count
   auto load_stage = [&](uint32_t u) {
     const uint32_t slot = lds0 + u * kStage;
-    lds_load_1k(a_src, lane * 16u, slot + wave * 1024u);
+    lds_load_1k(a_src, lane * 16u, slot + wave * (RB * 512u));
+    if (RB == 4) lds_load_1k(a_src, 1024u + lane * 16u, slot + wave * 2048u + 1024u);
     lds_load_1k(w_src, lane * 16u, slot + kWOff + wave * 2u * kWBlk);
     if (!W4) lds_load_1k(w_src, 1024u + lane * 16u, slot + kWOff + wave * 2u * kWBlk + 1024u);
     lds_gather_dword(s_src, s_idx * 4u, slot + kSOff + wave * 256u);
@@ -964,12 +975,12 @@ __global__ __launch_bounds__(256, 4) void gq_gemm_lds_kernel(GqGemmArgs a) {
     }
   };
 
-  v16f outv[2];
+  v16f outv[RB];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < RB; ++i)
 #pragma unroll
     for (int v = 0; v < 16; ++v) outv[i][v] = 0.0f;
-  v16i acc[2];
+  v16i acc[RB];
   constexpr int o = SMALL ? kGqSumOrigin : 0;
   v16i origin = {o, o, o, o, o, o, o, o, o, o, o, o, o, o, o, o};
   if (SMALL) asm volatile("" : "+v"(origin));  // kept in registers instead of written again for every group
@@ -977,14 +988,14 @@ __global__ __launch_bounds__(256, 4) void gq_gemm_lds_kernel(GqGemmArgs a) {
   // closes a group, (f32(acc) * sx) * sw added in group order; for 4-bit codes sw carries the exact 1/16
   // (opens / closes: whether the k block is the first / last of its group, workgroup-uniform and kept by
   // counting: a remainder per k block costs more instructions than the block's MFMAs leave room for)
-  auto step = [&](bool opens, bool closes, const v4i& fa0, const v4i& fa1, const GqRawFragment<W4>& r0, lds_cptr sc) {
+  auto step = [&](bool opens, bool closes, const v4i (&fa)[RB], const GqRawFragment<W4>& r0, lds_cptr sc) {
     const v4i fb = gq_expand<W4>(r0);
     if (opens) {
-      acc[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa0, fb, origin, 0, 0, 0);
-      acc[1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa1, fb, origin, 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < RB; ++i) acc[i] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[i], fb, origin, 0, 0, 0);
     } else {
-      acc[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa0, fb, acc[0], 0, 0, 0);
-      acc[1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa1, fb, acc[1], 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < RB; ++i) acc[i] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[i], fb, acc[i], 0, 0, 0);
     }
     if (closes) {
       typedef __attribute__((address_space(3))) const float* lds_fptr;
@@ -995,7 +1006,7 @@ __global__ __launch_bounds__(256, 4) void gq_gemm_lds_kernel(GqGemmArgs a) {
       // eight sums at a time, each of the four steps for all eight before the next step (the same operations per
       // output; output by output every instruction needs the result of the one in front of it)
 #pragma unroll
-      for (int p = 0; p < 4; ++p) {
+      for (int p = 0; p < 2 * RB; ++p) {
         const int i = p >> 1, v0 = 8 * (p & 1);
         gq_f4 s4[2];
 #pragma unroll
@@ -1027,13 +1038,13 @@ __global__ __launch_bounds__(256, 4) void gq_gemm_lds_kernel(GqGemmArgs a) {
     lds_barrier();  // everybody's pieces of the stage; and every wave is done with the stage before
     load_stage((u + NS - 1u) % NS);  // into the slot of the stage before
     lds_cptr slot = reinterpret_cast<lds_cptr>((uintptr_t)(lds0 + u * kStage));
-    v4i fa[2][2];
+    v4i fa[2][RB];
     GqRawFragment<W4> fr[2];
 #pragma unroll
     for (uint32_t kl = 0; kl < 2; ++kl) {
       typedef __attribute__((address_space(3))) const v4i* lds_v4ptr;
 #pragma unroll
-      for (uint32_t i = 0; i < 2; ++i)
+      for (uint32_t i = 0; i < RB; ++i)
         fa[kl][i] = *reinterpret_cast<lds_v4ptr>(slot + i * 2048u + kl * 1024u + lane * 16u);
       lds_cptr wp = slot + kWOff + wave * 2u * kWBlk + kl * kWBlk + lane * (W4 ? 8u : 16u);
       if (W4) {
@@ -1049,8 +1060,8 @@ __global__ __launch_bounds__(256, 4) void gq_gemm_lds_kernel(GqGemmArgs a) {
       }
     }
     const bool last_of_group = sig + 1u == stages_per_group;
-    step(sig == 0u, false, fa[0][0], fa[0][1], fr[0], slot + kSOff);
-    step(false, last_of_group, fa[1][0], fa[1][1], fr[1], slot + kSOff);
+    step(sig == 0u, false, fa[0], fr[0], slot + kSOff);
+    step(false, last_of_group, fa[1], fr[1], slot + kSOff);
     sig = last_of_group ? 0u : sig + 1u;
   };
   for (uint32_t u = 0; u + 1u < NS; ++u) load_stage(u);
@@ -1066,26 +1077,26 @@ __global__ __launch_bounds__(256, 4) void gq_gemm_lds_kernel(GqGemmArgs a) {
   lds_barrier();
   const bool lora = a.z != nullptr;
   if (lora) {
-    if (wave == 0) {
-      const uint32_t row = rbase * 32u + lane;
+    if (wave < RB / 2u) {
+      const uint32_t row = rbase * 32u + wave * 64u + lane;
       int ad = (a.idx && row < a.M) ? a.idx[row] : 0;
       ad = ad < 0 ? 0 : (ad >= (int)a.n_adapters ? (int)a.n_adapters - 1 : ad);
-      *reinterpret_cast<__attribute__((address_space(3))) float*>((uintptr_t)(lds0 + kGqFactorOff + lane * 4u)) = a.lora_scaling[ad];
+      *reinterpret_cast<__attribute__((address_space(3))) float*>((uintptr_t)(lds0 + gq_factor_off(RB) + (wave * 64u + lane) * 4u)) = a.lora_scaling[ad];
     }
     __syncthreads();
   }
-  v16f lacc[2];
+  v16f lacc[RB];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < RB; ++i)
 #pragma unroll
     for (int v = 0; v < 16; ++v) lacc[i][v] = 0.0f;
   if (lora) {  // workgroup-uniform
-    gq_tile_lora_sums(a, gq_lds, rbase, cbase, wave, lane, lacc);
+    gq_tile_lora_sums<RB>(a, gq_lds, rbase, cbase, wave, lane, lacc);
     __syncthreads();  // the last batch has been read
   }
 #pragma unroll
-  for (uint32_t i = 0; i < 2; ++i) gq_finish_values(a, gq_lds, i, outv[i], lacc[i], lora, rbase * 32u, cbase * 32u, wave, lane);
-  gq_store_tile(a, gq_lds, rbase * 32u, cbase * 32u, wave, lane);
+  for (uint32_t i = 0; i < RB; ++i) gq_finish_values<RB>(a, gq_lds, i, outv[i], lacc[i], lora, rbase * 32u, cbase * 32u, wave, lane);
+  gq_store_tile<RB>(a, gq_lds, rbase * 32u, cbase * 32u, wave, lane);
 }
 
 // ---------------------------------------------------------------------------------------
