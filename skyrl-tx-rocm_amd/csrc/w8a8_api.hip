@@ -108,9 +108,20 @@ inline bool padded_groups_fit(uint32_t m, uint32_t n, uint32_t n_groups, bool wi
 constexpr uint32_t kKSplitMaxTiles = 512u;
 inline uint32_t ksplit_tiles_m(uint32_t rows_bound) { return (rows_bound + (uint32_t)kGemm64TileM - 1u) / (uint32_t)kGemm64TileM; }
 inline bool ksplit_fits(uint32_t rows_bound, uint32_t n) { return ksplit_tiles_m(rows_bound) * ((n + 127u) / 128u) <= kKSplitMaxTiles; }
-// Bytes of z's four quarters (quant_lora_kernel's SPLIT form) for a call that may take those tiles, or 0.  Prologue of the call,
-// quarters / sixteen waves to a half block: 333 x 4096, rank 64 14 / 22 us, 333 x 12288, rank 32 22 / 41, 1000 x 1032 10 / 12;
-// level from 2000 rows of 1024 on.
+inline uint32_t ksplit_tiles(uint32_t rows_bound, uint32_t n) { return ksplit_tiles_m(rows_bound) * ((n + 127u) / 128u); }
+// Whether such a call's prologue leaves z in quarters (quant_lora_kernel's SPLIT form) instead of packed.  The prologue is a chain over K
+// that four workgroups to a half block shorten: 333 x 4096, rank 64 14 us / 22 packed, 333 x 12288, rank 32 22 / 41, 1000 x 1032 10 / 12.  But every tile then
+// reads four floats where it reads three bf16 terms and splits them itself, in pairs behind its main loop.  Whole call, quarters / packed: rank 16
+// 256 -> 4096, 1024 rows (512 tiles) 16.6 us / 17.7, 4096 -> 2560, 1400 rows 42 / 45; rank 32 256 -> 4096, 768 rows (384) 4 % slower, 1024 -> 3072, 1024 rows (384) 2 %,
+// 2048 -> 2048, 1024 rows 8 % faster, 1024 -> 1024, 1400 rows 4 % slower; rank 64 256 -> 4096, 768 rows 24.0 / 19.6, 512 -> 2048, 2000 rows 31.0 / 24.0, 1024 -> 3072, 1024 rows 29.0 / 25.4,
+// 520 rows (216) 4 % slower, 2048 -> 2048, 1400 rows (352) 36.7 / 33.7, 640 rows level, 4096 -> 2560, 1400 rows (440) 50.7 / 47.9, 768 rows 10 % faster, 8192 -> 8192, 400 rows (448) 60.8 / 69.2.
+constexpr uint32_t kSplitZMinKRank64 = 2048u;
+inline bool split_z_pays(uint32_t m, uint32_t k, uint32_t nkk, uint32_t tiles) {
+  if (nkk <= 1u) return true;
+  if (nkk > 2u && k < kSplitZMinKRank64) return false;
+  return k >= m * (nkk / 2u) * (tiles > 256u ? 2u : 1u);
+}
+// Bytes of z's four quarters for a call that may leave them, or 0.
 constexpr uint32_t kSplitZMaxRows = 2048;
 inline uint64_t split_z_bytes(uint32_t m, uint32_t n, uint32_t n_groups, uint32_t rank) {
   if (!rank || m <= (uint32_t)kSkinnyMaxRows || m > kSplitZMaxRows || !ksplit_fits(round_up(m, 32u), n)) return 0u;
@@ -574,7 +585,7 @@ int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
   const bool pack = lora && !(p->flags & MI355_W8A8_FLAG_LORA_PACK_VALID);
   // (neither this nor the next may depend on the measurement flags: a GEMM-only call reads what its prologue left)
   const bool ksplit = path == MI355_W8A8_PATH_TILED_128X128 && !(p->flags & MI355_W8A8_FLAG_TILE_128X128) && ksplit_fits(w.rows_bound, p->n);
-  const bool split_z = ksplit && w.split_bytes && p->workspace_bytes >= w.split_z + w.split_bytes;
+  const bool split_z = ksplit && w.split_bytes && split_z_pays(p->m, p->k, w.nkk, ksplit_tiles(w.rows_bound, p->n)) && p->workspace_bytes >= w.split_z + w.split_bytes;
   const bool rows_in_lds = !split_z && prologue_keeps_rows(w.rows_bound, p->k, rms, lora, pack, routed && !pad_groups);
   const bool route_inline = rows_in_lds && routed && !pack && p->m <= kInlineRouteMaxRows;
   // launch 1: adapter routing, the rows' statistics and (unless the workspace holds them) the LoRA operands
