@@ -90,8 +90,8 @@ typedef enum mi355_w8a8_status {
  * lora_a / lora_b contents and the same (k, n, n_adapters, rank): this call does not write them again
  * (adapters that do not change between calls, as in serving).  They sit at the start of the workspace, at
  * places that depend on (k, n, n_adapters, rank) only, so the earlier call may have had another m, other
- * adapter_indices or another tile geometry.  The caller vouches for it; calls that run as 32-row chunks
- * keep no such copies and ignore the flag. */
+ * adapter_indices or another tile geometry.  The caller vouches for it; calls for which mi355_w8a8_forward_path
+ * says 32-row chunks keep no such copies and ignore the flag (whatever they run on: see there). */
 /* Calls of at most 32 rows (the skinny-M kernels, with SwiGLU too) write no such copies and ignore it: a larger call
  * may not rely on one of them, unless that one ran with MI355_W8A8_FLAG_FORCE_TILED.  What they can keep has flags of
  * its own, MI355_W8A8_FLAG_DECODE_B_WRITE / _KEPT. */
@@ -562,10 +562,11 @@ int mi355_w8a8_gq_linear_v1(const mi355_w8a8_gq_problem* problem, void* stream);
 /*
  * Which kernels mi355_w8a8_forward_v1 and its three named forms run for these dimensions and flags
  * (no counterpart in the reference; for benchmarks and logs).  Returns an MI355_W8A8_PATH_* value or
- * a negative status.
+ * a negative status.  A call for which this says 32-row chunks may run on tiles all the same: its adapters, which are no argument
+ * here, decide too.  It keeps no LoRA operands for later calls either way and takes no FLAG_SKIP_PROLOGUE / _SKIP_GEMM.
  */
 #define MI355_W8A8_PATH_SKINNY 1         /* m <= 32 (SwiGLU included): row quantizer + weight-streaming kernel */
-#define MI355_W8A8_PATH_SKINNY_CHUNKS 2  /* 33..128 rows: the same two kernels per chunk of 32 rows */
+#define MI355_W8A8_PATH_SKINNY_CHUNKS 2  /* 33..96 rows: the same two kernels per chunk of 32 rows */
 #define MI355_W8A8_PATH_TILED_256X128 3  /* prologue + 256 x 128 tiles, two workgroups per CU */
 #define MI355_W8A8_PATH_TILED_256X256 4  /* prologue + 256 x 256 tiles, one workgroup per CU */
 #define MI355_W8A8_PATH_TILED_128X128 5  /* prologue + 128 x 128 tiles, two workgroups per CU */

@@ -68,15 +68,12 @@ inline uint32_t rank_chunks(uint32_t rank) { return rank == 0 ? 0u : (rank <= 16
 
 // Between the skinny-M limit and this many rows a call without SwiGLU may run the skinny-M kernels
 // on chunks of 32 rows: the weight is streamed once per chunk (the later passes from the last-level
-// cache).  A chunk costs 14-25 us, growing with the weight's bytes; the tiled call (K-split tiles, z in quarters) 16 us
-// + 2.7 us per 1024 of K whatever the rows.  Measured, chunks against tiles: 12288 x 4096 at 40 rows 38 us / 48, at 64 rows 46 / 50;
-// 9728 x 2560 at 64 rows 39 / 48; 4096 x 2560, rank 64 at 33 rows 28 / 30; 8192 x 8192 at 40 rows 51 / 43, at 65 rows 80 / 45 (hence
-// the line in N); 2560 x 6144 at 40 rows 50 / 28.  The upper lines are from before those tiles: at 64 rows of 4096 x 2560 the chunks
-// are now level to 20 % behind, at 96 rows of 12288 x 4096 66 us / 50.
+// cache), whatever the adapters.  Where it may is what mi355_w8a8_forward_path reports and what callers go by;
+// whether it does is chunks_pay's choice.
 constexpr uint32_t kSkinnyChunkedMaxRows = 96;
-inline bool skinny_chunked_pays(uint32_t m, uint32_t k, uint32_t n) {
-  if (m > kSkinnyChunkedMaxRows || n_padded(n) > 4096u || (uint64_t)k_padded(k) * n_padded(n) > (64ull << 20)) return false;
-  return k >= 8192u || (k >= 4096u && m <= 64u);
+inline bool skinny_chunks_possible(uint32_t m, uint32_t k, uint32_t n) {
+  if (m > kSkinnyChunkedMaxRows || k < 4096u || (uint64_t)k_padded(k) * n_padded(n) > (64ull << 20)) return false;
+  return k >= 8192u || (m <= 64u && n_padded(n) <= 4096u);
 }
 
 // Grouped slots a call of m rows and n_groups adapters can need when every adapter's rows start on a
@@ -109,6 +106,28 @@ constexpr uint32_t kKSplitMaxTiles = 512u;
 inline uint32_t ksplit_tiles_m(uint32_t rows_bound) { return (rows_bound + (uint32_t)kGemm64TileM - 1u) / (uint32_t)kGemm64TileM; }
 inline bool ksplit_fits(uint32_t rows_bound, uint32_t n) { return ksplit_tiles_m(rows_bound) * ((n + 127u) / 128u) <= kKSplitMaxTiles; }
 inline uint32_t ksplit_tiles(uint32_t rows_bound, uint32_t n) { return ksplit_tiles_m(rows_bound) * ((n + 127u) / 128u); }
+// Chunks or 128 x 128 tiles where a call may run on chunks.  Tiles run one to a CU, two (1.5 times as long) or behind each other, by
+// the slots of the call's groups on block boundaries, and bring every adapter's A and B into operand order first; a chunk takes 11 to 30 us
+// whatever the adapters.  Chunks / tiles in us.  No adapters: 12288 x 4096 at 64 rows 33 / 50-64, at 96 49 / 63; 8192 x 1024 at 96 34 / 42; 4096 x 2560 at 64
+// 17 / 25; 8192 x 8192 at 40 40 / 36-43, at 65 62 / 43.  One to a CU: 12288 x 4096, rank 16 at 64 45 / 48, at 72 60 / 46, rank 64 at 48 50 / 54, at 64 58 / 54; 6144 x 4096, rank 16
+// at 64 30 / 31, rank 64 at 56 41 / 37; 4096 x 2560, rank 16 at 48 24 / 24, at 64 27 / 24, sixteen adapters 27 / 28, rank 64 at 48 33 / 31, at 64 39 / 32; 8192 x 1024, rank 64, 16 adapters
+// at 56 45 / 48, 48 at 64 49 / 69, at 96 75 / 70; 8192 x 8192, rank 64 at 33 64 / 42.  In pairs: 12288 x 4096, 16 adapters of rank 16 at 96 69 / 74; 9728 x 2560, 24 of rank 16 at 96
+// 62 / 63; 6144 x 4096, 16 of rank 64 at 64 49 / 57; 8192 x 8192, 8 of rank 64 at 33 66 / 63; 8192 x 6144, 16 of rank 16 at 33 48 / 56, of rank 64 at 48 70 / 69, at 64 84 / 72; 12288 x
+// 5120, 16 of rank 64 at 64 94 / 94.  Behind each other: 8192 x 8192, 16 of rank 16 at 64 61 / 87, at 72 83 / 88, 48 of rank 16 at 33 53 / 252, at 96 94 / 119; 12288 x 5120, 24 of
+// rank 16 at 96 104 / 121.
+inline bool chunks_pay(uint32_t m, uint32_t k, uint32_t n, uint32_t slots, uint32_t groups, uint32_t nkk) {
+  const bool narrow = n_padded(n) <= 4096u;
+  if (!nkk) return narrow;
+  const uint32_t tiles = ksplit_tiles(slots, n);
+  if (tiles <= 256u) {
+    if (!narrow) return false;
+    if (nkk <= 2u) return m <= (k >= 6144u || groups > 8u ? 64u : 48u);
+    return m <= (k >= 8192u && groups > 8u ? (groups > 32u ? 80u : 64u) : 48u);
+  }
+  if (narrow) return true;
+  if (tiles <= kKSplitMaxTiles) return groups > 8u && m <= 64u && m <= k / 170u;
+  return groups > 16u || m <= 64u;
+}
 // Whether such a call's prologue leaves z in quarters (quant_lora_kernel's SPLIT form) instead of packed.  The prologue is a chain over K
 // that four workgroups to a half block shorten: 333 x 4096, rank 64 14 us / 22 packed, 333 x 12288, rank 32 22 / 41, 1000 x 1032 10 / 12.  But every tile then
 // reads four floats where it reads three bf16 terms and splits them itself, in pairs behind its main loop.  Whole call, quarters / packed: rank 16
@@ -409,7 +428,7 @@ int choose_forward_path(uint32_t m, uint32_t k, uint32_t n, uint32_t flags) {
     skinny = true;
   }
   if (skinny) return MI355_W8A8_PATH_SKINNY;
-  if (!swiglu && skinny_chunked_pays(m, k, n) &&
+  if (!swiglu && skinny_chunks_possible(m, k, n) &&
       !(flags & (MI355_W8A8_FLAG_FORCE_TILED | MI355_W8A8_FLAG_TILE_256X128 | MI355_W8A8_FLAG_TILE_256X256 |
                  MI355_W8A8_FLAG_TILE_128X128 | MI355_W8A8_FLAG_TILE_256X128_PAIR)))
     return MI355_W8A8_PATH_SKINNY_CHUNKS;
@@ -536,8 +555,14 @@ int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
   if (!p->workspace) return MI355_W8A8_ERR_WORKSPACE;
   if (p->workspace_bytes < need - split_z_bytes(p->m, p->n, p->n_adapters, lora ? p->rank : 0u)) return MI355_W8A8_ERR_WORKSPACE;
   if (reinterpret_cast<uintptr_t>(p->workspace) & 255u) return MI355_W8A8_ERR_ALIGN;
-  const int path = choose_forward_path(p->m, p->k, p->n, p->flags);
-  if (path < 0) return path;
+  const int reported = choose_forward_path(p->m, p->k, p->n, p->flags);
+  if (reported < 0) return reported;
+  int path = reported;
+  if (path == MI355_W8A8_PATH_SKINNY_CHUNKS) {
+    const uint32_t groups = routed ? p->n_adapters : 1u, slots = groups > 1u ? padded_rows_bound(p->m, groups) : round_up(p->m, 32u);
+    if (!chunks_pay(p->m, p->k, p->n, slots, groups, lora ? rank_chunks(p->rank) : 0u))
+      path = choose_forward_path(p->m, p->k, p->n, p->flags | MI355_W8A8_FLAG_FORCE_TILED);
+  }
   // groups on block boundaries: only where the empty slots cost no round on the chip
   const bool pad_groups =
       routed && ((path == MI355_W8A8_PATH_TILED_128X128 && padded_groups_fit(p->m, p->n, p->n_adapters)) ||
@@ -554,11 +579,13 @@ int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
   if (skinny) {
     return launch_skinny(p, ws + w.xq, reinterpret_cast<float*>(ws + w.sx), ws + w.skinny, w.K_pad, w.KB, s);
   }
-  if (path == MI355_W8A8_PATH_SKINNY_CHUNKS) {
+  if (reported == MI355_W8A8_PATH_SKINNY_CHUNKS) {
     // The chunks overwrite each other's prologue results, so there is no GEMM-only or prologue-only
-    // rerun of such a call; the choice of path must not depend on those flags either (a GEMM-only
-    // tiled call would read tables no tiled prologue has written).
+    // rerun of such a call (nor of one that takes tiles in their place); the choice of path must not depend on those flags either
+    // (a GEMM-only tiled call would read tables no tiled prologue has written).
     if (p->flags & (MI355_W8A8_FLAG_SKIP_PROLOGUE | MI355_W8A8_FLAG_SKIP_GEMM)) return MI355_W8A8_ERR_UNSUPPORTED;
+  }
+  if (path == MI355_W8A8_PATH_SKINNY_CHUNKS) {
     for (uint32_t row0 = 0; row0 < p->m; row0 += (uint32_t)kSkinnyMaxRows) {
       mi355_w8a8_problem sub = *p;
       sub.m = p->m - row0 < (uint32_t)kSkinnyMaxRows ? p->m - row0 : (uint32_t)kSkinnyMaxRows;
@@ -582,8 +609,9 @@ int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
   const bool skip_gemm = (p->flags & MI355_W8A8_FLAG_SKIP_GEMM) != 0;
   // Rows held in the LDS, or read twice behind a launch that takes their statistics (quant_lora_rows_kernel,
   // quant_lora_kernel).
-  const bool pack = lora && !(p->flags & MI355_W8A8_FLAG_LORA_PACK_VALID);
-  // (neither this nor the next may depend on the measurement flags: a GEMM-only call reads what its prologue left)
+  // (tiles in the place of chunks, which keep no packed operands and ignore what a caller vouches for, always pack)
+  const bool pack = lora && (!(p->flags & MI355_W8A8_FLAG_LORA_PACK_VALID) || reported == MI355_W8A8_PATH_SKINNY_CHUNKS);
+  // (neither the next two may depend on the measurement flags: a GEMM-only call reads what its prologue left)
   const bool ksplit = path == MI355_W8A8_PATH_TILED_128X128 && !(p->flags & MI355_W8A8_FLAG_TILE_128X128) && ksplit_fits(w.rows_bound, p->n);
   const bool split_z = ksplit && w.split_bytes && split_z_pays(p->m, p->k, w.nkk, ksplit_tiles(w.rows_bound, p->n)) && p->workspace_bytes >= w.split_z + w.split_bytes;
   const bool rows_in_lds = !split_z && prologue_keeps_rows(w.rows_bound, p->k, rms, lora, pack, routed && !pad_groups);
