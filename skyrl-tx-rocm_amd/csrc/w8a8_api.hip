@@ -106,6 +106,24 @@ constexpr uint32_t kKSplitMaxTiles = 512u;
 inline uint32_t ksplit_tiles_m(uint32_t rows_bound) { return (rows_bound + (uint32_t)kGemm64TileM - 1u) / (uint32_t)kGemm64TileM; }
 inline bool ksplit_fits(uint32_t rows_bound, uint32_t n) { return ksplit_tiles_m(rows_bound) * ((n + 127u) / 128u) <= kKSplitMaxTiles; }
 inline uint32_t ksplit_tiles(uint32_t rows_bound, uint32_t n) { return ksplit_tiles_m(rows_bound) * ((n + 127u) / 128u); }
+// Whether a routed call that the K-split tiles fit without padding puts its groups on block boundaries all the same.  A block of several groups runs its
+// epilogue and its LoRA-A once for each, a matter of the rank and of how many groups share 32 rows; the empty slots cost tiles, which
+// matters where those then run two to a CU, or no longer on these kernels at all, and the more the longer K is.
+// Whole call, packed / on boundaries.  Same number to a CU: 2560 -> 6144, 4 adapters of rank 64, 333 rows 38 us / 37 and up.  From one to two: 8192 -> 8192, 8 adapters
+// of rank 16, 64 rows 60 / 52, rank 64, 97 rows 68 / 62, 256 53 / 62; 2560 -> 6144, 8 of rank 16, 160 rows 31 / 27, of rank 32, 256 31 / 33; 4096 -> 2560, 8 of rank 64, 768 rows 42 / 46; 1024 -> 3072, 4 of rank
+// 64, 520 rows 28 / 25.  From one to behind each other: 4096 -> 24576, 4 of rank 64, 33 rows 59 / 63; 4096 -> 4096, 24 of rank 16, 300 rows 40 / 53.  From two: 8192 -> 8192, 8 of rank 16, 400 rows
+// 79 / 91; 2048 -> 10960 SwiGLU, 8 adapters, 200 rows, rank 64 54 / 45, rank 32 42 / 39, at 160 rows rank 16 32 / 37; 4096 -> 4096, 4 of rank 32, 1024 rows 52 / 55; 256 -> 4096 level.  Many rows of rank
+// 64: 4096 -> 2560, 4 adapters, 1600 rows 62 / 58, 2560 -> 1024, 2000 rows 41 / 38.
+inline bool ksplit_padding_pays(uint32_t m, uint32_t k, uint32_t n, uint32_t groups, uint32_t nkk) {
+  const uint32_t packed = ksplit_tiles(round_up(m, 32u), n), padded = ksplit_tiles(padded_rows_bound(m, groups), n);
+  if (padded <= 256u || (packed > 256u && padded <= kKSplitMaxTiles)) return true;
+  if (nkk > 2u && m >= 1280u) return true;
+  const uint64_t group_work = ((uint64_t)m * k / groups) >> 10;
+  if (padded <= kKSplitMaxTiles) return k <= 1536u || group_work <= (nkk > 1u ? 100u : 80u);
+  if (k <= 512u) return true;
+  if (packed <= 256u) return group_work <= (nkk > 2u ? 24u : 16u);
+  return group_work <= (nkk > 2u ? (k <= 2048u ? 140u : 70u) : (nkk == 2u && k <= 2048u ? 70u : 16u));
+}
 // Chunks or 128 x 128 tiles where a call may run on chunks.  Tiles run one to a CU, two (1.5 times as long) or behind each other, by
 // the slots of the call's groups on block boundaries, and bring every adapter's A and B into operand order first; a chunk takes 11 to 30 us
 // whatever the adapters.  Chunks / tiles in us.  No adapters: 12288 x 4096 at 64 rows 33 / 50-64, at 96 49 / 63; 8192 x 1024 at 96 34 / 42; 4096 x 2560 at 64
@@ -563,9 +581,12 @@ int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
     if (!chunks_pay(p->m, p->k, p->n, slots, groups, lora ? rank_chunks(p->rank) : 0u))
       path = choose_forward_path(p->m, p->k, p->n, p->flags | MI355_W8A8_FLAG_FORCE_TILED);
   }
-  // groups on block boundaries: only where the empty slots cost no round on the chip
+  // groups on block boundaries: only where the empty slots cost no round on the chip, or less than they save
+  const bool may_ksplit = path == MI355_W8A8_PATH_TILED_128X128 && !(p->flags & MI355_W8A8_FLAG_TILE_128X128);
   const bool pad_groups =
-      routed && ((path == MI355_W8A8_PATH_TILED_128X128 && padded_groups_fit(p->m, p->n, p->n_adapters)) ||
+      routed && ((path == MI355_W8A8_PATH_TILED_128X128 && padded_groups_fit(p->m, p->n, p->n_adapters) &&
+                  (!may_ksplit || !ksplit_fits(round_up(p->m, 32u), p->n) ||
+                   ksplit_padding_pays(p->m, p->k, p->n, p->n_adapters, rank_chunks(p->rank)))) ||
                  (path == MI355_W8A8_PATH_TILED_256X256 && padded_groups_fit(p->m, p->n, p->n_adapters, true)));
   const WsLayout w = make_layout(p->m, p->k, p->n, p->n_adapters, lora ? p->rank : 0u, routed, pad_groups);
   unsigned char* ws = static_cast<unsigned char*>(p->workspace);
@@ -612,7 +633,7 @@ int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
   // (tiles in the place of chunks, which keep no packed operands and ignore what a caller vouches for, always pack)
   const bool pack = lora && (!(p->flags & MI355_W8A8_FLAG_LORA_PACK_VALID) || reported == MI355_W8A8_PATH_SKINNY_CHUNKS);
   // (neither the next two may depend on the measurement flags: a GEMM-only call reads what its prologue left)
-  const bool ksplit = path == MI355_W8A8_PATH_TILED_128X128 && !(p->flags & MI355_W8A8_FLAG_TILE_128X128) && ksplit_fits(w.rows_bound, p->n);
+  const bool ksplit = may_ksplit && ksplit_fits(w.rows_bound, p->n);
   const bool split_z = ksplit && w.split_bytes && split_z_pays(p->m, p->k, w.nkk, ksplit_tiles(w.rows_bound, p->n)) && p->workspace_bytes >= w.split_z + w.split_bytes;
   const bool rows_in_lds = !split_z && prologue_keeps_rows(w.rows_bound, p->k, rms, lora, pack, routed && !pad_groups);
   const bool route_inline = rows_in_lds && routed && !pack && p->m <= kInlineRouteMaxRows;
