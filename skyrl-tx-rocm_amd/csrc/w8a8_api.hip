@@ -1104,32 +1104,20 @@ int validate_bwd_dims(uint32_t m, uint32_t k, uint32_t n, uint32_t n_adapters, u
   return MI355_W8A8_OK;
 }
 
-template <int NKK, bool ROWS128>
-int launch_bwd_dx_geometry(const BwdDxArgs& g, hipStream_t s) {
+template <int NKK>
+int launch_bwd_dx(const BwdDxArgs& g, bool rows128, hipStream_t s) {
   uint32_t want = ((g.direct_tiles + 7u) / 8u) * 8u;
   if (g.sk_wgs > want) want = g.sk_wgs;
-  const dim3 grid(want < 256u ? want : 256u), block(512);
-  if (ROWS128) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&bwd_dx_kernel<NKK, true>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, kBwdLdsBytes) != hipSuccess)
-      return MI355_W8A8_ERR_LAUNCH;
-    hipLaunchKernelGGL((bwd_dx_kernel<NKK, true>), grid, block, kBwdLdsBytes, s, g);
-  } else {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&bwd_dx_wide_kernel<NKK>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, kBwdLdsBytes) != hipSuccess)
-      return MI355_W8A8_ERR_LAUNCH;
-    hipLaunchKernelGGL((bwd_dx_wide_kernel<NKK>), grid, dim3(256), kBwdLdsBytes, s, g);
-  }
+  const dim3 grid(want < 256u ? want : 256u);
+  const auto kernel = rows128 ? &bwd_dx_kernel<NKK> : &bwd_dx_wide_kernel<NKK>;
+  if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kBwdLdsBytes) != hipSuccess)
+    return MI355_W8A8_ERR_LAUNCH;
+  hipLaunchKernelGGL(kernel, grid, dim3(rows128 ? 512 : 256), kBwdLdsBytes, s, g);
   if (!g.sk_wgs) return launch_status();
   if (const int st = launch_status()) return st;
   const uint32_t split_tiles = g.tiles_m * g.tiles_k - g.direct_tiles;
   hipLaunchKernelGGL((bwd_dx_finish_kernel<NKK, 2>), dim3(split_tiles * 8u), dim3(256), 0, s, g);
   return launch_status();
-}
-
-template <int NKK>
-int launch_bwd_dx(const BwdDxArgs& g, bool rows128, hipStream_t s) {
-  return rows128 ? launch_bwd_dx_geometry<NKK, true>(g, s) : launch_bwd_dx_geometry<NKK, false>(g, s);
 }
 
 // The stages of a backward call behind its routing tables: dy into operand order (with the partial

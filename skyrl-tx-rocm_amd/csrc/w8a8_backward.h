@@ -450,21 +450,18 @@ __global__ __launch_bounds__(1024) void bwd_grouped_prep_kernel(BwdGroupedPrepAr
 }
 
 // ---------------------------------------------------------------------------------------
-// dx = dyp @ bf16(W * sw).T (+ rs @ A.T), one bf16 cast.
-// Workgroup = 8 waves (2 along rows x 4 along k), tile 256 rows x 256 k, wave tile 128 x 64
-// (4 x 2 accumulator blocks of v_mfma_f32_32x32x16_bf16).  The contraction runs over n in stages
-// of one 32-wide n block.  A stage's dy panel (16 KiB), weight blocks (8 KiB) and scales travel
-// HBM/L2 -> LDS with direct-to-LDS loads five stages ahead.  While the matrix core works on stage
+// dx = dyp @ bf16(W * sw).T (+ rs @ A.T), one bf16 cast, on tiles of 256 rows x 256 k (bwd_dx_wide_kernel: dense calls, and grouped ones whose weights
+// own many rows) or of 128 rows x 512 k (bwd_dx_kernel: grouped calls whose weights own few).
+// The contraction runs over n in stages of one 32-wide n block.  A stage's dy panel, weight blocks (24 KiB together) and scales travel
+// HBM/L2 -> LDS with direct-to-LDS loads four or five stages ahead.  While the matrix core works on stage
 // nb, the vector ALU prepares the weight operands of stage nb + 1: each wave transposes its two
 // blocks with the identity MFMA, scales, rounds to bf16 and keeps them in registers.
 // ---------------------------------------------------------------------------------------
 constexpr int kBwdStages = 6;
-constexpr int kBwdAhead = kBwdStages - 1;  // stages between a load and its use
 constexpr int kBwdStagePanel = 16384;      // dy: 8 row blocks x 2 halves
 constexpr int kBwdStageWeight = 8192;      // 8 k blocks of the n block
 constexpr int kBwdStageBytes = kBwdStagePanel + kBwdStageWeight + 1024;  // + a 1 KiB chunk of scales (the stage's 32 lead it)
 constexpr int kBwdLdsBytes = kBwdStages * kBwdStageBytes;
-constexpr int kBwdLoadsPerStage = 4;  // direct-to-LDS loads per wave per stage: 2 panel chunks, 1 weight block, scales
 constexpr int kBwdScalePad = 256;     // floats readable past the last stage's scales
 
 struct BwdDxArgs {
@@ -605,7 +602,7 @@ __device__ inline void bwd_dx_fetch_rs(const BwdDxArgs& g, uint32_t pbase, int b
   }
 }
 
-// The stages of a segment through a ring of AHEAD + 1 LDS stages, LOADS direct-to-LDS loads per wave each: stage i asks for
+// The stages of a tile through a ring of AHEAD + 1 LDS stages, LOADS direct-to-LDS loads per wave each: stage i asks for
 // stage i + AHEAD.  `first` prepares the operands of stage 0 (busy: the wave has rows); `even` / `odd` (i, more) multiply
 // stage i and, with more, prepare those of i + 1.  L is even.
 template <int AHEAD, int LOADS, class Issue, class First, class Even, class Odd>
@@ -702,25 +699,22 @@ __device__ inline __attribute__((always_inline)) void bwd_dx_schedule(const BwdD
   }
 }
 
-// ROWS128: the tile is 128 rows x 512 k (the eight waves side by side along k, the same 128 x 64 wave
-// tile): a stage then holds half the dy panel and twice the weight blocks, the same bytes and the same
-// four loads per wave.  For grouped calls whose weights own few rows each: half the padding per weight,
-// and every wave has rows.
+// The 128 x 512 geometry: eight waves side by side along k, a wave tile of 128 rows x 64 k (4 x 2 accumulator blocks of
+// v_mfma_f32_32x32x16_bf16).  A stage holds half the dy panel of the 256 x 256 tile and twice the weight blocks, the same
+// bytes.  For grouped calls whose weights own few rows each: half the padding per weight, and every wave has rows.
 //
 // The 256 registers that two waves per SIMD leave are the kernel's limit: the loads' addresses are a scalar base plus the
 // lane's offset (issue), and the epilogue derives its lane constants for itself (bwd_dx_store).  Held in vector
-// registers through the stages both cost 44 bytes of scratch per lane (16 with ROWS128).  Spilling / as it is, pull-back and
-// what goes before it: 2048 x 2560, N = 10240, rank 64 211 / 205 us; 512 x 2560, N = 6144 78.0 / 74.9; 4096 x 4096,
-// N = 24576 947 / 946 (whole tiles: the reloads stand outside the stages); 8168 rows of 128 experts, 2048 <- 1536 207 / 204.
-template <int NKK, bool ROWS128 = false>
+// registers through the stages both cost 16 bytes of scratch per lane; 8168 rows of 128 experts, 2048 <- 1536, spilling / as it is 207 / 204 us.
+constexpr int kBwdPanel128 = 8192, kBwdWeight512 = 16384;  // 4 row blocks x 2 halves; 16 k blocks
+static_assert(kBwdPanel128 + kBwdWeight512 + 1024 == kBwdStageBytes, "a stage keeps its size in both geometries");
+constexpr int kBwdAhead = kBwdStages - 1;  // stages between a load and its use
+constexpr int kBwdLoadsPerStage = 4;       // direct-to-LDS loads per wave and stage: a panel chunk, 2 weight blocks, scales
+template <int NKK>
 __global__ __launch_bounds__(512, 1) void bwd_dx_kernel(BwdDxArgs g) {
-  constexpr int kRowBlocks = ROWS128 ? 4 : 8, kKBlocks = ROWS128 ? 16 : 8;  // of a tile
-  constexpr int kPanel = kRowBlocks * 2048, kWeight = kKBlocks * kBlockBytes;
-  static_assert(kPanel + kWeight + 1024 == kBwdStageBytes, "a stage keeps its size in both geometries");
   extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wrow = ROWS128 ? 0 : wave >> 2, wcol = ROWS128 ? wave : wave & 3;
   const int c = lane & 31, h = lane >> 5;
   const uint32_t lane16 = (uint32_t)lane * 16u;
 
@@ -733,60 +727,32 @@ __global__ __launch_bounds__(512, 1) void bwd_dx_kernel(BwdDxArgs g) {
     ident[2] = wi == 2 ? word : 0; ident[3] = wi == 3 ? word : 0;
   }
 
-  // One tile, or the stages nb0 .. nb0 + L - 1 (an even number) of one whose partial sums go to slot `slot`.
-  auto segment = [&](uint32_t tm, uint32_t tk, int nb0, int L, bool whole, uint32_t slot) {
-    int tw = 0;
-    int n_act = 4;  // 32-row blocks of this wave that hold rows: the others skip their matrix-core work
-    int live_blocks;  // ... of the tile
-    // row block whose dy panel this wave fetches: both 1 KiB halves, or one half of it in a 128-row tile
-    uint32_t load_rb = ROWS128 ? (uint32_t)wave >> 1 : (uint32_t)wave;
-    if (g.tile_weight) {
-      const int tv = g.tile_weight[tm];
-      if (tv < 0) return;  // workgroup-uniform: no row lives in this tile
-      tw = tv & 0xffff;
-      live_blocks = ((tv >> 16) + 31) / 32;
-      const int live = live_blocks - wrow * 4;
-      n_act = live < 0 ? 0 : (live > 4 ? 4 : live);
-      // a block without rows is never multiplied: its slot is filled from block 0 of the tile, which
-      // is in the caches anyway, instead of streaming unused memory (the load count stays the same)
-      if ((int)load_rb >= live_blocks) load_rb = 0u;
-    } else {  // (the rows of a dense call fill the slots from the first)
-      live_blocks = ((int)(g.M - tm * (uint32_t)(kRowBlocks * 32)) + 31) / 32;
-      live_blocks = live_blocks > kRowBlocks ? kRowBlocks : live_blocks;
-      const int live = live_blocks - wrow * 4;
-      n_act = live < 0 ? 0 : (live > 4 ? 4 : live);
-    }
-    n_act = __builtin_amdgcn_readfirstlane(n_act);
+  auto tile = [&](uint32_t tm, uint32_t tk) {
+    const int tv = g.tile_weight[tm];
+    if (tv < 0) return;  // workgroup-uniform: no row lives in this tile
+    const int tw = tv & 0xffff, live_blocks = ((tv >> 16) + 31) / 32;
+    // 32-row blocks that hold rows: the others skip their matrix-core work
+    const int n_act = __builtin_amdgcn_readfirstlane(live_blocks < 0 ? 0 : (live_blocks > 4 ? 4 : live_blocks));
+    // row block of whose dy panel this wave fetches a half.  A block without rows is never multiplied: its slot is filled from block 0
+    // of the tile, which is in the caches anyway, instead of streaming unused memory (the load count stays the same)
+    const uint32_t load_rb = (wave >> 1) < live_blocks ? (uint32_t)wave >> 1 : 0u;
     const float* swp_t = g.swp + (size_t)tw * g.sw_stride;
-
-    // this wave's two panel chunks of a stage (row block = wave, halves q = 0, 1) and its weight block
-    const unsigned char* Ag = g.dyp + ((size_t)(tm * (uint32_t)kRowBlocks + load_rb) * g.NB) * 2048u +
-                              (ROWS128 ? (wave & 1) * 1024 : 0);
-    const uint32_t kbw = tk * (uint32_t)kKBlocks + (uint32_t)wcol * 2u;  // first of the two k blocks this wave multiplies
-    // the block(s) it loads: one of eight, or its own two of sixteen; blocks past the weight repeat the last
-    const uint32_t kbl0 = tk * (uint32_t)kKBlocks + (ROWS128 ? 2u * (uint32_t)wave : (uint32_t)wave);
-    const uint32_t kbl = kbl0 < g.KB ? kbl0 : g.KB - 1u;
-    const uint32_t kbl1 = kbl0 + 1u < g.KB ? kbl0 + 1u : g.KB - 1u;
+    const unsigned char* Ag = g.dyp + ((size_t)(tm * 4u + load_rb) * g.NB) * 2048u + (wave & 1) * 1024;
+    const uint32_t kbw = tk * 16u + (uint32_t)wave * 2u;  // its two k blocks (blocks past the weight repeat the last)
+    const uint32_t kbl = kbw < g.KB ? kbw : g.KB - 1u;
+    const uint32_t kbl1 = kbw + 1u < g.KB ? kbw + 1u : g.KB - 1u;
     const unsigned char* Bg = g.wp + (size_t)tw * g.w_stride + (size_t)kbl * kBlockBytes;
     const unsigned char* Bg1 = g.wp + (size_t)tw * g.w_stride + (size_t)kbl1 * kBlockBytes;
     const size_t nb_stride = (size_t)g.KB * kBlockBytes;
 
-    auto issue = [&](int i) {  // stage i of the segment
-      unsigned char* St = lds + (i % kBwdStages) * kBwdStageBytes;
-      const int nb = nb0 + i;
-      const unsigned char* src = Ag + (size_t)nb * 2048u + lane16;
-      if constexpr (ROWS128) {
-        load_1k_to_lds(src, St + wave * kBlockBytes);
-        // (few rows per weight: most of its bytes are read by one workgroup only)
-        load_1k_to_lds_once(Bg + (size_t)nb * nb_stride + lane16, St + kPanel + (wave * 2) * kBlockBytes);
-        load_1k_to_lds_once(Bg1 + (size_t)nb * nb_stride + lane16, St + kPanel + (wave * 2 + 1) * kBlockBytes);
-      } else {
-        load_1k_to_lds(src, St + (wave * 2) * kBlockBytes);
-        load_1k_to_lds(src + 1024, St + (wave * 2 + 1) * kBlockBytes);
-        load_1k_to_lds(Bg + (size_t)nb * nb_stride + lane16, St + kPanel + wave * kBlockBytes);
-      }
+    auto issue = [&](int nb) {
+      unsigned char* St = lds + (nb % kBwdStages) * kBwdStageBytes;
+      load_1k_to_lds(Ag + (size_t)nb * 2048u + lane16, St + wave * kBlockBytes);
+      // (few rows per weight: most of its bytes are read by one workgroup only)
+      load_1k_to_lds_once(Bg + (size_t)nb * nb_stride + lane16, St + kBwdPanel128 + (wave * 2) * kBlockBytes);
+      load_1k_to_lds_once(Bg1 + (size_t)nb * nb_stride + lane16, St + kBwdPanel128 + (wave * 2 + 1) * kBlockBytes);
       // every wave fetches the same 1 KiB of scales (the stage's 32 lead it) to the same place
-      load_1k_to_lds(reinterpret_cast<const unsigned char*>(swp_t + 32 * nb) + lane16, St + kPanel + kWeight);
+      load_1k_to_lds(reinterpret_cast<const unsigned char*>(swp_t + 32 * nb) + lane16, St + kBwdPanel128 + kBwdWeight512);
     };
 
     v16f acc[4][2];
@@ -818,7 +784,7 @@ __global__ __launch_bounds__(512, 1) void bwd_dx_kernel(BwdDxArgs g) {
     auto panel_frag = [&](int nb, int pair) -> v8bf {  // pair = 4 q + row block
       const unsigned char* St = lds + (nb % kBwdStages) * kBwdStageBytes;
       return __builtin_bit_cast(
-          v8bf, *reinterpret_cast<const v4i*>(St + ((wrow * 4 + (pair & 3)) * 2 + (pair >> 2)) * kBlockBytes + lane * 16));
+          v8bf, *reinterpret_cast<const v4i*>(St + ((pair & 3) * 2 + (pair >> 2)) * kBlockBytes + lane * 16));
     };
     // The weight blocks and scales of the next stage are read from LDS with explicit instructions:
     // a compiler-visible read of memory that direct-to-LDS loads write makes the compiler drain
@@ -827,9 +793,9 @@ __global__ __launch_bounds__(512, 1) void bwd_dx_kernel(BwdDxArgs g) {
     const uint32_t lds_base = (uint32_t)(uintptr_t)(lptr_t)lds;
     struct NextRegs { v4i raw[2]; v4f s4[4]; };
     auto next_read = [&](int nb1, NextRegs& r) {
-      const uint32_t st = lds_base + (nb1 % kBwdStages) * kBwdStageBytes + kPanel;
-      const uint32_t wa = st + (wcol * 2) * kBlockBytes + lane * 16;
-      const uint32_t sa = st + kWeight + 16 * h;
+      const uint32_t st = lds_base + (nb1 % kBwdStages) * kBwdStageBytes + kBwdPanel128;
+      const uint32_t wa = st + (wave * 2) * kBlockBytes + lane * 16;
+      const uint32_t sa = st + kBwdWeight512 + 16 * h;
       asm volatile("ds_read_b128 %0, %6\n\tds_read_b128 %1, %6 offset:1024\n\t"
                    "ds_read_b128 %2, %7\n\tds_read_b128 %3, %7 offset:32\n\t"
                    "ds_read_b128 %4, %7 offset:64\n\tds_read_b128 %5, %7 offset:96"
@@ -886,7 +852,7 @@ __global__ __launch_bounds__(512, 1) void bwd_dx_kernel(BwdDxArgs g) {
 
     v8bf bqA[2][2], bqB[2][2];
     bwd_dx_stages<kBwdAhead, kBwdLoadsPerStage>(
-        L, n_act > 0, issue,
+        (int)g.NB, n_act > 0, issue,
         [&] {  // operands of stage 0
           NextRegs nx;
           next_read(0, nx);
@@ -902,31 +868,18 @@ __global__ __launch_bounds__(512, 1) void bwd_dx_kernel(BwdDxArgs g) {
         },
         [&](int i, bool more) { stage(i, bqA, bqB, more); }, [&](int i, bool more) { stage(i, bqB, bqA, more); });
 
-    if (whole) {
-      lds_barrier();  // (every wave has read its last stage)
-      const uint32_t rs_lds = lds_base + 8u * kBwdTurnBytes;
-      bwd_dx_fetch_rs<NKK>(g, tm * (uint32_t)(kRowBlocks * 32), live_blocks, rs_lds, wave, 8);
-      if (n_act)
-        bwd_dx_store<NKK, 2, 4, true>(g, tm * (uint32_t)(kRowBlocks * 32) + (uint32_t)wrow * 128u, kbw, n_act, lds_base + (uint32_t)wave * kBwdTurnBytes,
-                                      rs_lds + (uint32_t)(wrow * 4 * NKK * 3) * kBlockBytes, [&](int rb, int cb) -> v16f { return acc[rb][cb]; });
-    } else {
-#pragma unroll
-      for (int rb = 0; rb < 4; ++rb)
-        if (rb < n_act) {
-          float4* dst = bwd_dx_part<2>(g, slot, (uint32_t)(wrow * 4 + rb), (uint32_t)wcol);
-#pragma unroll
-          for (int cb = 0; cb < 2; ++cb)
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-              dst[(cb * 4 + e) * 64] = make_float4(acc[rb][cb][4 * e], acc[rb][cb][4 * e + 1], acc[rb][cb][4 * e + 2], acc[rb][cb][4 * e + 3]);
-        }
-    }
+    lds_barrier();  // (every wave has read its last stage)
+    const uint32_t rs_lds = lds_base + 8u * kBwdTurnBytes;
+    bwd_dx_fetch_rs<NKK>(g, tm * 128u, live_blocks, rs_lds, wave, 8);
+    if (n_act)
+      bwd_dx_store<NKK, 2, 4, true>(g, tm * 128u, kbw, n_act, lds_base + (uint32_t)wave * kBwdTurnBytes, rs_lds,
+                                    [&](int rb, int cb) -> v16f { return acc[rb][cb]; });
   };
 
-  bwd_dx_schedule(g, !ROWS128, [&](uint32_t t, int nb0, int len, uint32_t slot) {
+  bwd_dx_schedule(g, false, [&](uint32_t t, int, int, uint32_t) {
     uint32_t tm, tk;
     bwd_dx_tile_at(g, t, tm, tk);
-    segment(tm, tk, nb0, len, len == (int)g.NB, slot);
+    tile(tm, tk);
   });
 }
 
@@ -963,7 +916,7 @@ __device__ inline v16f bwd_sums(v16f& acc) {
   return y;
 }
 // W[n][k] of a 32 x 32 block in vector registers (the builtin's result lands in the half that the sums fill); not to be read for
-// 19 wait states.
+// 13 wait states (what the compiler leaves behind the builtin; the calls here leave three MFMAs or 32 of s_nop).
 __device__ inline void bwd_transpose(v16i& tr, const v4i& raw, const v4i& ident) {
   asm volatile("v_mfma_i32_32x32x32_i8 %0, %1, %2, 0" : "=&v"(tr) : "v"(raw), "v"(ident));
 }
