@@ -169,7 +169,7 @@ def test_gq_linear_matches_oracle(dev, pkg, m, k, n, wb, ab, group, rank, n_ad):
     (130, 128, 132, 8, 8, 64, 8, 3),       # N not a multiple of 8
 ])
 def test_gq_lds_staged_and_direct_kernels_agree_bitwise(dev, pkg, m, k, n, wb, ab, group, rank, n_ad):
-    """Groups of whole 64-wide k steps run on the LDS-staged 128 x 128 tiles; the kernel that feeds its wave
+    """Groups of whole 64-wide k steps run on the LDS-staged tiles; the kernel that feeds its wave
     tiles from the L2 (FLAG_GQ_DIRECT) gives the same float32 base and the same output, bit for bit."""
     import torch
 

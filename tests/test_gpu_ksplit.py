@@ -1,6 +1,5 @@
-"""64 x 128 tiles whose waves split K, behind a prologue that leaves z in quarters: the bits of the 128 x 128 geometry (which takes
-the other prologue) at the edges of tiles, k blocks, ranks and columns, one workgroup to a CU and two, and where the
-workspace has no room for the quarters."""
+"""64 x 128 tiles whose waves split K: the bits of the 128 x 128 geometry at the edges of tiles, k blocks, ranks and columns, one
+workgroup to a CU and two, and beyond the rows whose prologue may leave z in quarters."""
 
 import pytest
 
