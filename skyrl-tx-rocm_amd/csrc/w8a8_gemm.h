@@ -663,7 +663,8 @@ __global__ __launch_bounds__(256, PAIR ? 2 : 1) void w8a8_gemm_ksplit_kernel(Gem
   const bool row_ok = src_lane >= 0 && src_lane < (int)g.M;
   const uint32_t off_lane = row_ok ? (uint32_t)src_lane * n_out : 0xffffffffu;
   const bool fast = full_n && __builtin_amdgcn_ballot_w64(!row_ok) == 0;  // wave-uniform
-  for (int gi = glo; gi <= ghi; ++gi) {  // wave-uniform; a boundary block runs once per group
+  for (int gi = glo; gi <= ghi; ++gi) {  // wave-uniform; a boundary block runs once per group that has rows in it
+    if (NKK > 0 && ghi > glo && __builtin_amdgcn_ballot_w64(grp_lane == gi) == 0) continue;
     v16f low[2];
     if constexpr (NKK > 0) {
       const float sgrp = g.lora_scaling[gi];

@@ -1210,7 +1210,8 @@ __global__ __launch_bounds__(WAVES * 64, SPLIT ? 2 : 4) void quant_lora_kernel(s
   pass(std::true_type{}, glo, ghi == glo || rowgrp == glo);
   if constexpr (CB > 0) {
 #pragma unroll 1
-    for (uint32_t grp = glo + 1u; grp <= ghi; ++grp) pass(std::false_type{}, grp, rowgrp == grp);
+    for (uint32_t grp = glo + 1u; grp <= ghi; ++grp)
+      if (__builtin_amdgcn_ballot_w64(rowgrp == grp) != 0) pass(std::false_type{}, grp, rowgrp == grp);  // workgroup-uniform
   }
   if constexpr (SPLIT) quant_lora_store_quarter<kCB>(a, acc, red, hb, blockIdx.x & 3u);
   else if constexpr (CB > 0) quant_lora_store_z<kCB, WAVES>(a, acc, red, zs, pb, half16);
@@ -1536,6 +1537,7 @@ __global__ __launch_bounds__(1024) void quant_lora_rows_kernel(QuantLoraRowsArgs
 #pragma unroll 1
   for (uint32_t grp = glo; grp <= ghi; ++grp) {  // workgroup-uniform: one trip except at a group boundary
     const bool first = grp == glo;
+    if (CB > 0 && !first && __builtin_amdgcn_ballot_w64(rowgrp == grp) == 0) continue;
     const bool in_group = ghi == glo || rowgrp == grp;
     v4i wa[kCB], wb2[kCB];
     uint4 ra, rb;
