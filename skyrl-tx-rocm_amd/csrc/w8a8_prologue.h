@@ -1085,6 +1085,18 @@ __device__ inline void quant_lora_store_quarter(const QuantLoraSplitArgs& a, con
   }
 }
 
+// At a group boundary: the rows of group grp (rowgrp: a lane's slot row lane % 16) keep this pass's sums, the others what they have (`first`: nothing
+// yet).  Zeroing the other groups' rows of x instead leaves them 0 x infinity where the group's A is not finite.
+template <int kCB>
+__device__ inline void keep_group_rows(v4f (&z)[kCB], const v4f (&acc)[kCB], uint32_t rowgrp, uint32_t grp, bool first) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const bool own = (uint32_t)__shfl((int)rowgrp, (int)(4u * ((threadIdx.x & 63u) >> 4)) + e, 64) == grp;
+#pragma unroll
+    for (int b = 0; b < kCB; ++b) z[b][e] = own ? acc[b][e] : (first ? 0.0f : z[b][e]);
+  }
+}
+
 // SPLIT: four workgroups of four waves share the half block, for calls whose half blocks are far fewer than the CUs.  Workgroup
 // `part` plays waves part, part + 4, + 8, + 12 of the sixteen, fetches a quarter of A, and leaves the sum of its waves'
 // tiles, added as the sixteen add theirs, in zpart: the consumer adds the quarters in order and so has the same z to the last bit
@@ -1154,7 +1166,7 @@ __global__ __launch_bounds__(WAVES * 64, SPLIT ? 2 : 4) void quant_lora_kernel(s
     }
   };
   const bool scale_safe = scale > 1e-30f && scale < 1e30f;
-  auto work = [&](auto codes, bool in_group, uint32_t j, const uint4& rawx, const Operands& o) {
+  auto work = [&](auto codes, uint32_t j, const uint4& rawx, const Operands& o) {
     const uint32_t kb = vw + kStride * j;
     uint4 raw = rawx;
     if constexpr (RMS)
@@ -1167,8 +1179,7 @@ __global__ __launch_bounds__(WAVES * 64, SPLIT ? 2 : 4) void quant_lora_kernel(s
       *reinterpret_cast<uint2*>(xq_dst + (size_t)kb * kBlockBytes) = quant_codes8(raw, scale, rscale, scale_safe);
     }
     if constexpr (CB > 0) {
-      // (zeros where the lane has no value; at a group boundary the rows of the other groups are zeroed)
-      const v4i xa = in_group ? v4i{(int)raw.x, (int)raw.y, (int)raw.z, (int)raw.w} : v4i{0, 0, 0, 0};
+      const v4i xa = {(int)raw.x, (int)raw.y, (int)raw.z, (int)raw.w};
 #pragma unroll
       for (int b = 0; b < CB; ++b)
         acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, xa), __builtin_bit_cast(v8bf, o.w[b]),
@@ -1179,7 +1190,7 @@ __global__ __launch_bounds__(WAVES * 64, SPLIT ? 2 : 4) void quant_lora_kernel(s
   // are in flight beside the one at work.  (With few workgroups on the chip the loop is a chain of those
   // loads' latencies; no load or store in it is conditional, so the compiler's waits can count.)
   const uint32_t n_j = vw < a.KB ? (a.KB - vw + kStride - 1u) / kStride : 0u;
-  auto pass = [&](auto codes, uint32_t grp, bool in_group) {
+  auto pass = [&](auto codes, uint32_t grp) {
     const __amdgpu_buffer_rsrc_t arsrc = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<uint16_t*>(a.at) + (size_t)grp * (at_bytes / 2u), 0, CB > 0 ? (int)at_bytes : 0, 0x00020000);
     uint4 xc[kAhead];
@@ -1194,7 +1205,7 @@ __global__ __launch_bounds__(WAVES * 64, SPLIT ? 2 : 4) void quant_lora_kernel(s
 #pragma unroll
       for (uint32_t u = 0; u < kAhead; ++u) {
         fetch_operands(arsrc, j + u + kRing - 1u, o[(u + kRing - 1u) % kRing]);
-        work(codes, in_group, j + u, xc[u], o[u % kRing]);
+        work(codes, j + u, xc[u], o[u % kRing]);
         xc[u] = fetch_x(j + u + kAhead);
       }
     }
@@ -1202,16 +1213,25 @@ __global__ __launch_bounds__(WAVES * 64, SPLIT ? 2 : 4) void quant_lora_kernel(s
     for (uint32_t u = 0; u + 1u < kAhead; ++u) {  // the rest, fewer than kAhead
       if (j + u >= n_j) break;  // wave-uniform
       fetch_operands(arsrc, j + u + kRing - 1u, o[(u + kRing - 1u) % kRing]);
-      work(codes, in_group, j + u, xc[u], o[u % kRing]);
+      work(codes, j + u, xc[u], o[u % kRing]);
     }
   };
   // one pass per group present among the slots (one, except at a group boundary): the first also forms the
-  // codes, a later one only adds the rows of its group to z
-  pass(std::true_type{}, glo, ghi == glo || rowgrp == glo);
-  if constexpr (CB > 0) {
+  // codes, a later one only z, and every row keeps the sums of its own group's pass
+  pass(std::true_type{}, glo);
+  if (CB > 0 && ghi > glo) {  // workgroup-uniform
+    v4f z[kCB];
+    keep_group_rows<kCB>(z, acc, rowgrp, glo, true);
 #pragma unroll 1
-    for (uint32_t grp = glo + 1u; grp <= ghi; ++grp)
-      if (__builtin_amdgcn_ballot_w64(rowgrp == grp) != 0) pass(std::false_type{}, grp, rowgrp == grp);  // workgroup-uniform
+    for (uint32_t grp = glo + 1u; grp <= ghi; ++grp) {
+      if (__builtin_amdgcn_ballot_w64(rowgrp == grp) == 0) continue;
+#pragma unroll
+      for (int b = 0; b < kCB; ++b) acc[b] = v4f{0.f, 0.f, 0.f, 0.f};
+      pass(std::false_type{}, grp);
+      keep_group_rows<kCB>(z, acc, rowgrp, grp, false);
+    }
+#pragma unroll
+    for (int b = 0; b < kCB; ++b) acc[b] = z[b];
   }
   if constexpr (SPLIT) quant_lora_store_quarter<kCB>(a, acc, red, hb, blockIdx.x & 3u);
   else if constexpr (CB > 0) quant_lora_store_z<kCB, WAVES>(a, acc, red, zs, pb, half16);
@@ -1507,7 +1527,7 @@ __global__ __launch_bounds__(1024) void quant_lora_rows_kernel(QuantLoraRowsArgs
   unsigned char* const xq_dst =
       a.xq_packed + (size_t)pb * a.KB * kBlockBytes + (16u * half16 + i + 32u * (q >> 1)) * 16u + 8u * (q & 1u);
   // One pass over the k-blocks per group present among the slots (one, except at a group boundary): the
-  // first pass also forms the codes; a later pass only adds the rows of its group to z.  The loop is kept rolled, two
+  // first pass also forms the codes; a later pass only z.  The loop is kept rolled, two
   // k-blocks per trip with their operands requested one trip ahead and no load inside the work on a
   // k-block, so that the compiler's waits count loads instead of draining them.
   auto request = [&](uint32_t grp, uint32_t kb, v4i (&w)[kCB], uint4& raw) {
@@ -1520,40 +1540,48 @@ __global__ __launch_bounds__(1024) void quant_lora_rows_kernel(QuantLoraRowsArgs
     const uint32_t k0 = kb * 32u + q * 8u;
     raw = (kb < a.KB && k0 < a.K && src >= 0) ? *reinterpret_cast<const uint4*>(rowl + 2u * k0) : make_uint4(0, 0, 0, 0);
   };
-  auto work = [&](bool first, bool in_group, uint32_t kb, const v4i (&w)[kCB], const uint4& raw) {
+  auto work = [&](bool first, uint32_t kb, const v4i (&w)[kCB], const uint4& raw) {
     if (first) {  // wave-uniform
       const uint2 codes = quant_codes8(raw, scale, rscale, scale_safe);
       if (mine_row) *reinterpret_cast<uint2*>(xq_dst + (size_t)kb * kBlockBytes) = codes;
     }
     if constexpr (CB > 0) {
-      // (zeros where the lane has no value; at a group boundary the rows of the other groups are zeroed)
-      const v4i xa = in_group ? v4i{(int)raw.x, (int)raw.y, (int)raw.z, (int)raw.w} : v4i{0, 0, 0, 0};
+      const v4i xa = {(int)raw.x, (int)raw.y, (int)raw.z, (int)raw.w};  // (zeros where the lane has no value)
 #pragma unroll
       for (int b = 0; b < CB; ++b)
         acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, xa), __builtin_bit_cast(v8bf, w[b]),
                                                          acc[b], 0, 0, 0);
     }
   };
+  v4f z[kCB];  // (at a group boundary: every row the sums of its own group's pass)
 #pragma unroll 1
   for (uint32_t grp = glo; grp <= ghi; ++grp) {  // workgroup-uniform: one trip except at a group boundary
     const bool first = grp == glo;
-    if (CB > 0 && !first && __builtin_amdgcn_ballot_w64(rowgrp == grp) == 0) continue;
-    const bool in_group = ghi == glo || rowgrp == grp;
+    if (CB > 0 && !first) {
+      if (__builtin_amdgcn_ballot_w64(rowgrp == grp) == 0) continue;
+#pragma unroll
+      for (int b = 0; b < kCB; ++b) acc[b] = v4f{0.f, 0.f, 0.f, 0.f};
+    }
     v4i wa[kCB], wb2[kCB];
     uint4 ra, rb;
     request(grp, wave, wa, ra);
     request(grp, wave + 16u, wb2, rb);
 #pragma unroll 1
     for (uint32_t kb = wave; kb < a.KB; kb += 32u) {
-      work(first, in_group, kb, wa, ra);
+      work(first, kb, wa, ra);
       request(grp, kb + 32u, wa, ra);
       if (kb + 16u >= a.KB) break;  // wave-uniform
-      work(first, in_group, kb + 16u, wb2, rb);
+      work(first, kb + 16u, wb2, rb);
       request(grp, kb + 48u, wb2, rb);
     }
     if constexpr (CB == 0) break;
+    if (ghi > glo) keep_group_rows<kCB>(z, acc, rowgrp, grp, first);
   }
   if constexpr (CB > 0) {
+    if (ghi > glo) {
+#pragma unroll
+      for (int b = 0; b < kCB; ++b) acc[b] = z[b];
+    }
     __syncthreads();  // the rows are spent: their bytes take the wave tiles
     quant_lora_store_z<kCB, 16u>(a, acc, reinterpret_cast<float (*)[kCB][4][64]>(ql_lds), zs, pb, half16, r0, r0 + R);
   }

@@ -45,3 +45,18 @@ def test_an_adapter_without_rows(m, k, n, n_ad, rank):
     plain, inf, nan = both(case, spoil)
     assert torch.equal(plain.view(torch.int16), inf.view(torch.int16))
     assert torch.equal(plain.view(torch.int16), nan.view(torch.int16))
+
+
+@pytest.mark.parametrize("m,k,n,n_ad,rank", CASES)
+@pytest.mark.parametrize("rms", [False, True])
+def test_the_other_rows_of_a_block(m, k, n, n_ad, rank, rms):
+    import torch
+
+    case = wc.make_case(m, k, n, n_adapters=n_ad, rank=rank, seed=m + n, rms=rms)
+    spoil = n_ad // 2
+    print(f"[case] other rows {m}x{k}x{n} adapters={n_ad} rank={rank} rms={rms}", flush=True)
+    plain, inf, nan = both(case, spoil)
+    others = torch.from_numpy(case["idx"] != spoil).to(plain.device)
+    assert torch.equal(plain[others].view(torch.int16), inf[others].view(torch.int16))
+    assert torch.equal(plain[others].view(torch.int16), nan[others].view(torch.int16))
+    assert not torch.isfinite(inf[~others]).any() and not torch.isfinite(nan[~others]).any()
