@@ -93,13 +93,14 @@ PROFILE_TRAFFIC = {
     "qwen3-8b-gate_up-m4096": ("w8a8_gemm16_kernel__qwen3-8b-gate_up-m4096.txt", [r"w8a8_gemm16_kernel<1, 2, 4>"]),
     "qwen3-8b-down-m16-decode": ("skinny_stream_kernel__qwen3-8b-down-m16-decode.txt",
                                  [r"skinny_quant_kernel<", r"skinny_stream_kernel<"]),
-    "qwen3-8b-gate_up-m4096-backward": ("bwd_dx_kernel__qwen3-8b-gate_up-m4096-backward.txt", [r"bwd_dx_kernel<"]),
+    "qwen3-8b-gate_up-m4096-backward": ("bwd_dx_kernel__qwen3-8b-gate_up-m4096-backward.txt",
+                                        [r"bwd_dx_wide_kernel<"]),
     "qwen3-30b-a3b-moe-mlp-t2048": ("w8a8_grouped_kernel__qwen3-30b-a3b-moe-mlp-t2048.txt",
                                     [r"w8a8_grouped_kernel<1, 1, "]),  # grouped gate/up with the SwiGLU epilogue
     "qwen3-30b-a3b-moe-experts-t2048-backward": ("bwd_dx_kernel_grouped__qwen3-30b-a3b-moe-experts-t2048-backward.txt",
-                                                 [r"bwd_pack_dy_kernel<0>", r"bwd_dx_kernel<0, true>"]),
+                                                 [r"bwd_pack_dy_kernel<0>", r"bwd_dx_kernel<0>"]),
     "qwen3-8b-gate_up-m4096-fused-backward": ("swiglu_bwd_kernel__qwen3-8b-gate_up-m4096-fused-backward.txt",
-                                              [r"bwd_dx_kernel<"]),
+                                              [r"bwd_dx_wide_kernel<"]),
     "qwen3-8b-down-m4096-w4a8-g128": ("gq_gemm_kernel__qwen3-8b-down-m4096-w4a8-g128.txt", [r"gq_gemm_(lds_)?kernel<"]),
     "qwen3-30b-a3b-moe-routing-t4096": ("moe_spread_kernel__qwen3-30b-a3b-moe-routing-t4096.txt",
                                         [r"moe_hist_kernel", r"moe_scan_kernel", r"moe_scatter_kernel",
@@ -318,7 +319,7 @@ def cpu_baseline(case, cfg, sample_rows):
 
 def bench_backward(args, cfg, pkg, dev):
     """One step = one backward call (tables, dy packing + r, z, dx pull-back, dA / dB / dscaling).
-    ``value`` counts the pull-back's 2*M*K*N only; the roofline prices bwd_dx_kernel alone
+    ``value`` counts the pull-back's 2*M*K*N only; the roofline prices bwd_dx_wide_kernel alone
     (bf16 MFMA) from HIP events around launches of that kernel."""
     import torch
 
@@ -366,7 +367,7 @@ def bench_backward(args, cfg, pkg, dev):
         "config": {"workload": args.workload, **{kk: v for kk, v in cfg.items() if kk != "seed"}},
         "roofline": {"bound": "mfma", "achieved": achieved, "peak": BF16_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved / BF16_PEAK_TFLOPS, "traffic": measured_traffic_bytes(args.workload),
-                     "kernel": "bwd_dx_kernel",
+                     "kernel": "bwd_dx_wide_kernel",
                      "kernel_avg_ms": float(k_ms.mean()), "kernel_min_ms": float(k_ms.min()),
                      "algorithmic_flops": flops,
                      # dy once, int8 weight once, dx once (the kernel reads dy re-laid-out by the packing pass)
@@ -399,7 +400,7 @@ def bench_fused_backward(args, cfg, pkg, dev):
     """One step = one backward of the fused RMSNorm -> gate/up -> SwiGLU call: the forward
     recomputation (projection + normalized rows), the SwiGLU pull-back, the linear backward and the
     RMSNorm pull-back.  ``value`` counts the pull-back's 2*M*K*N only; the roofline prices
-    bwd_dx_kernel (bf16 MFMA) as in the plain backward, and ``stages`` gives the two memory-bound
+    bwd_dx_wide_kernel (bf16 MFMA) as in the plain backward, and ``stages`` gives the two memory-bound
     pull-back kernels against HBM."""
     import torch
 
@@ -474,7 +475,7 @@ def bench_fused_backward(args, cfg, pkg, dev):
         "vs_baseline": None, "dtype": "bf16", "data": "synthetic",
         "config": {"workload": args.workload, **{kk: v for kk, v in cfg.items() if kk != "seed"}},
         "roofline": {"bound": "mfma", "achieved": achieved, "peak": BF16_PEAK_TFLOPS, "unit": "TFLOP/s",
-                     "frac": achieved / BF16_PEAK_TFLOPS, "traffic": measured_traffic_bytes(args.workload), "kernel": "bwd_dx_kernel",
+                     "frac": achieved / BF16_PEAK_TFLOPS, "traffic": measured_traffic_bytes(args.workload), "kernel": "bwd_dx_wide_kernel",
                      "kernel_avg_ms": float(k_ms.mean()), "kernel_min_ms": float(k_ms.min()),
                      "algorithmic_flops": flops, "algorithmic_bytes": 2 * m * n + k * n + 2 * m * k},
         "stages": {
