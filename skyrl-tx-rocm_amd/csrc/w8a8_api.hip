@@ -114,13 +114,16 @@ inline uint32_t ksplit_tiles(uint32_t rows_bound, uint32_t n) { return ksplit_ti
 // 64, 520 rows 28 / 25.  From one to behind each other: 4096 -> 24576, 4 of rank 64, 33 rows 59 / 63; 4096 -> 4096, 24 of rank 16, 300 rows 40 / 53.  From two: 8192 -> 8192, 8 of rank 16, 400 rows
 // 79 / 91; 2048 -> 10960 SwiGLU, 8 adapters, 200 rows, rank 64 54 / 45, rank 32 42 / 39, at 160 rows rank 16 32 / 37; 4096 -> 4096, 4 of rank 32, 1024 rows 52 / 55; 256 -> 4096 level.  Many rows of rank
 // 64: 4096 -> 2560, 4 adapters, 1600 rows 62 / 58, 2560 -> 1024, 2000 rows 41 / 38.
+// Many groups of rank 64, rows dealt at random: 12288 -> 6144, 24 adapters, 54 rows 187 / 143; 4096 -> 5120, 24, 155 rows 74 / 68; 4096 -> 6144, 16, 323 rows 71 / 68;
+// 6144 -> 2048, 64, 1124 rows 128 / 105; 8192 -> 1024, 64, 1271 rows 125 / 115 (1000 rows 115 / 111, 700 rows 106 / 108).
 inline bool ksplit_padding_pays(uint32_t m, uint32_t k, uint32_t n, uint32_t groups, uint32_t nkk) {
   const uint32_t packed = ksplit_tiles(round_up(m, 32u), n), padded = ksplit_tiles(padded_rows_bound(m, groups), n);
   if (padded <= 256u || (packed > 256u && padded <= kKSplitMaxTiles)) return true;
-  if (nkk > 2u && m >= 1280u) return true;
+  if (nkk > 2u && (m >= 1280u || (groups > 32u && m >= 960u))) return true;
   const uint64_t group_work = ((uint64_t)m * k / groups) >> 10;
-  if (padded <= kKSplitMaxTiles) return k <= 1536u || group_work <= (nkk > 1u ? 100u : 80u);
+  if (padded <= kKSplitMaxTiles) return k <= 1536u || group_work <= (nkk > 2u ? 100u : 70u);
   if (k <= 512u) return true;
+  if (nkk > 2u && m / groups <= (packed <= 256u ? (k <= 4096u ? 8u : 4u) : (k <= 4096u ? 32u : 16u))) return true;
   if (packed <= 256u) return group_work <= (nkk > 2u ? 24u : 16u);
   return group_work <= (nkk > 2u ? (k <= 2048u ? 140u : 70u) : (nkk == 2u && k <= 2048u ? 70u : 16u));
 }

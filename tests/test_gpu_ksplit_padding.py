@@ -16,6 +16,9 @@ pytestmark = pytest.mark.gpu
     (170, 2048, 10960, 8, 32), (170, 2048, 10960, 8, 8),  # behind each other on boundaries, packed in pairs
     (333, 4096, 2560, 40, 8),   # packed, eight rows to a group
     (50, 640, 3000, 64, 16),    # fewer rows than adapters
+    (155, 4096, 5120, 24, 64), (240, 4096, 5120, 24, 64),  # rank 64, six rows to a group: on boundaries; ten: packed
+    (323, 4096, 6144, 16, 64),  # twenty rows to a group where packed tiles run in pairs: on boundaries
+    (1000, 2560, 2048, 40, 64),  # many groups and rows: on boundaries
 ])
 def test_same_bits_as_128x128(m, k, n, n_ad, rank):
     import torch
