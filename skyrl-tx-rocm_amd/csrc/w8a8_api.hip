@@ -262,24 +262,24 @@ int launch_gemm(const GemmArgs& g, uint32_t nkk, hipStream_t s) {
   }
 }
 
-template <int EPI, int NKK, bool PAIR>
+template <int EPI, int NKK, bool PAIR, bool CHUNKS>
 int launch_gemm_ksplit_one(const GemmKSplitArgs& g, hipStream_t s) {
   constexpr int lds_bytes = PAIR ? kGemm64LdsBytes / 2 : kGemm64LdsBytes;
-  if (hipFuncSetAttribute(reinterpret_cast<const void*>(&w8a8_gemm_ksplit_kernel<EPI, NKK, PAIR>),
+  if (hipFuncSetAttribute(reinterpret_cast<const void*>(&w8a8_gemm_ksplit_kernel<EPI, NKK, PAIR, CHUNKS>),
                           hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes) != hipSuccess)
     return MI355_W8A8_ERR_LAUNCH;
-  hipLaunchKernelGGL((w8a8_gemm_ksplit_kernel<EPI, NKK, PAIR>), dim3(round_up(g.tiles_m * g.tiles_n, 8u)), dim3(256), lds_bytes, s, g);
+  hipLaunchKernelGGL((w8a8_gemm_ksplit_kernel<EPI, NKK, PAIR, CHUNKS>), dim3(round_up(g.tiles_m * g.tiles_n, 8u)), dim3(256), lds_bytes, s, g);
   return launch_status();
 }
 
-template <int EPI>
+template <int EPI, bool CHUNKS = false>
 int launch_gemm_ksplit(const GemmKSplitArgs& g, uint32_t nkk, hipStream_t s) {
   const bool pair = g.tiles_m * g.tiles_n > 256u;
   switch (nkk) {
-    case 0: return pair ? launch_gemm_ksplit_one<EPI, 0, true>(g, s) : launch_gemm_ksplit_one<EPI, 0, false>(g, s);
-    case 1: return pair ? launch_gemm_ksplit_one<EPI, 1, true>(g, s) : launch_gemm_ksplit_one<EPI, 1, false>(g, s);
-    case 2: return pair ? launch_gemm_ksplit_one<EPI, 2, true>(g, s) : launch_gemm_ksplit_one<EPI, 2, false>(g, s);
-    case 4: return pair ? launch_gemm_ksplit_one<EPI, 4, true>(g, s) : launch_gemm_ksplit_one<EPI, 4, false>(g, s);
+    case 0: return pair ? launch_gemm_ksplit_one<EPI, 0, true, false>(g, s) : launch_gemm_ksplit_one<EPI, 0, false, false>(g, s);
+    case 1: return pair ? launch_gemm_ksplit_one<EPI, 1, true, CHUNKS>(g, s) : launch_gemm_ksplit_one<EPI, 1, false, CHUNKS>(g, s);
+    case 2: return pair ? launch_gemm_ksplit_one<EPI, 2, true, CHUNKS>(g, s) : launch_gemm_ksplit_one<EPI, 2, false, CHUNKS>(g, s);
+    case 4: return pair ? launch_gemm_ksplit_one<EPI, 4, true, CHUNKS>(g, s) : launch_gemm_ksplit_one<EPI, 4, false, CHUNKS>(g, s);
     default: return MI355_W8A8_ERR_UNSUPPORTED;
   }
 }
@@ -589,7 +589,9 @@ int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
   const bool pad_groups =
       routed && ((path == MI355_W8A8_PATH_TILED_128X128 && padded_groups_fit(p->m, p->n, p->n_adapters) &&
                   (!may_ksplit || !ksplit_fits(round_up(p->m, 32u), p->n) ||
-                   ksplit_padding_pays(p->m, p->k, p->n, p->n_adapters, rank_chunks(p->rank)))) ||
+                   ksplit_padding_pays(p->m, p->k, p->n, p->n_adapters, rank_chunks(p->rank))) &&
+                  // (in the place of chunks on the K-split tiles only, which they fit unpadded: sums_again)
+                  (reported != MI355_W8A8_PATH_SKINNY_CHUNKS || ksplit_fits(padded_rows_bound(p->m, p->n_adapters), p->n))) ||
                  (path == MI355_W8A8_PATH_TILED_256X256 && padded_groups_fit(p->m, p->n, p->n_adapters, true)));
   const WsLayout w = make_layout(p->m, p->k, p->n, p->n_adapters, lora ? p->rank : 0u, routed, pad_groups);
   unsigned char* ws = static_cast<unsigned char*>(p->workspace);
@@ -775,6 +777,7 @@ int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
     GemmKSplitArgs gk{g, split_z ? reinterpret_cast<const float*>(ws + w.split_z) : nullptr, w.rows_bound, q.nterms};
     gk.tiles_m = ksplit_tiles_m(w.rows_bound);
     gk.tiles_n = (p->n + 127u) / 128u;
+    if (reported == MI355_W8A8_PATH_SKINNY_CHUNKS) return launch_gemm_ksplit<kEpiPlain, true>(gk, w.nkk, s);  // (never SwiGLU)
     return swiglu ? launch_gemm_ksplit<kEpiSwiglu>(gk, w.nkk, s) : launch_gemm_ksplit<kEpiPlain>(gk, w.nkk, s);
   }
   if (small)

@@ -495,7 +495,8 @@ struct GemmKSplitArgs : GemmArgs {
   uint32_t nterms;     // bf16 terms that z is split into (3 or 2)
 };
 
-template <int EPI, int NKK, bool PAIR>
+// CHUNKS: the call stands in for 32-row chunks (sums_again).
+template <int EPI, int NKK, bool PAIR, bool CHUNKS>
 __global__ __launch_bounds__(256, PAIR ? 2 : 1) void w8a8_gemm_ksplit_kernel(GemmKSplitArgs g) {
   static_assert(EPI != kEpiAcc, "accumulators are read off the other geometries");
   constexpr int kRing = PAIR ? 3 : 6;
@@ -559,6 +560,39 @@ __global__ __launch_bounds__(256, PAIR ? 2 : 1) void w8a8_gemm_ksplit_kernel(Gem
       zt[0][e] = (unsigned short)b0;
       zt[1][e] = (unsigned short)b1;
       zt[2][e] = (unsigned short)(g.nterms >= 3u ? f32_to_bf16_bits(r2) : 0u);
+    }
+  };
+  // The low-rank sums of a call in the place of chunks where they are not finite: an infinite z has one term (the rest is inf - inf), and an
+  // infinite B meets z's first term alone (terms of both signs would cancel to NaN).  z @ B is then infinite where it is in float32, as
+  // in the chunks.  (In every call the look at the sums would cost 0.1 us a pass: 0.6 % over 440 calls, 5 % with 48 adapters among few rows.  An instance
+  // of its own: compiled into all it cost them 0.2 %.)
+  auto sums_again = [&](int gi, v16f (&low)[2]) {
+    auto odd = [](unsigned short v) { return (v & 0x7f80u) == 0x7f80u; };
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) low[j][e] = 0.0f;
+#pragma unroll 1
+    for (int kk = 0; kk < kKK; ++kk) {
+      v8us z[3], b[2];
+      fetch_b(gi, kk, b);
+      if (g.zpart) z_from_quarters(kk, z);
+      else fetch_z(kk, z);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        z[1][e] = odd(z[0][e]) ? (unsigned short)0 : z[1][e];
+        z[2][e] = odd(z[0][e]) ? (unsigned short)0 : z[2][e];
+      }
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        v8us fin = b[j];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) fin[e] = odd(fin[e]) ? (unsigned short)0 : fin[e];
+#pragma unroll
+        for (int t3 = 2; t3 >= 0; --t3)
+          low[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, z[t3]), __builtin_bit_cast(v8bf, t3 ? fin : b[j]),
+                                                           low[j], 0, 0, 0);
+      }
     }
   };
   v8us zf[kKK][3], bf[kKK][2];  // (!PAIR: held from here on)
@@ -685,6 +719,17 @@ __global__ __launch_bounds__(256, PAIR ? 2 : 1) void w8a8_gemm_ksplit_kernel(Gem
           for (int t3 = 2; t3 >= 0; --t3)
             low[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, zf[kk][t3]), __builtin_bit_cast(v8bf, bf[kk][j]),
                                                              low[j], 0, 0, 0);
+      }
+      if constexpr (CHUNKS) {
+        // of the rows of the group (bit 8 (e / 4) + e % 4: the lane's value e): slots without a row may hold anything
+        const uint32_t rows = (uint32_t)__builtin_amdgcn_ballot_w64(row_ok && grp_lane == gi) >> (4 * h);
+        bool again = false;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const float probe = __builtin_fmaf(low[0][e], 0.0f, low[1][e] * 0.0f);  // NaN where one is not finite
+          again |= !(probe == 0.0f) && ((rows >> (8 * (e >> 2) + (e & 3))) & 1u) != 0;
+        }
+        if (__builtin_amdgcn_ballot_w64(again) != 0) sums_again(gi, low);  // wave-uniform
       }
 #pragma unroll
       for (int j = 0; j < 2; ++j)
