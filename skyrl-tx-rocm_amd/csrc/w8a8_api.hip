@@ -132,8 +132,8 @@ inline bool ksplit_padding_pays(uint32_t m, uint32_t k, uint32_t n, uint32_t gro
 // whatever the adapters.  Chunks / tiles in us.  No adapters: 12288 x 4096 at 64 rows 33 / 50-64, at 96 49 / 63; 8192 x 1024 at 96 34 / 42; 4096 x 2560 at 64
 // 17 / 25; 8192 x 8192 at 40 40 / 36-43, at 65 62 / 43.  One to a CU: 12288 x 4096, rank 16 at 64 45 / 48, at 72 60 / 46, rank 64 at 48 50 / 54, at 64 58 / 54; 6144 x 4096, rank 16
 // at 64 30 / 31, rank 64 at 56 41 / 37; 4096 x 2560, rank 16 at 48 24 / 24, at 64 27 / 24, sixteen adapters 27 / 28, rank 64 at 48 33 / 31, at 64 39 / 32; 8192 x 1024, rank 64, 16 adapters
-// at 56 45 / 48, 48 at 64 49 / 69, at 96 75 / 70; 8192 x 8192, rank 64 at 33 64 / 42.  In pairs: 12288 x 4096, 16 adapters of rank 16 at 96 69 / 74; 9728 x 2560, 24 of rank 16 at 96
-// 62 / 63; 6144 x 4096, 16 of rank 64 at 64 49 / 57; 8192 x 8192, 8 of rank 64 at 33 66 / 63; 8192 x 6144, 16 of rank 16 at 33 48 / 56, of rank 64 at 48 70 / 69, at 64 84 / 72; 12288 x
+// at 56 45 / 48, 48 at 64 49 / 69, at 96 75 / 70, 48 of rank 32 at 67 53 / 57; 8192 x 8192, rank 64 at 33 64 / 42.  In pairs: 12288 x 4096, 16 adapters of rank 16 at 96 69 / 74; 9728 x 2560, 24 of rank 16 at 96
+// 62 / 63; 6144 x 4096, 16 of rank 64 at 64 49 / 57; 8192 x 8192, 8 of rank 64 at 33 66 / 63, of rank 8 at 40 53 / 57, of rank 32 at 37 57 / 61; 8192 x 6144, 16 of rank 16 at 33 48 / 56, of rank 64 at 48 70 / 69, at 64 84 / 72; 12288 x
 // 5120, 16 of rank 64 at 64 94 / 94.  Behind each other: 8192 x 8192, 16 of rank 16 at 64 61 / 87, at 72 83 / 88, 48 of rank 16 at 33 53 / 252, at 96 94 / 119; 12288 x 5120, 24 of
 // rank 16 at 96 104 / 121.
 inline bool chunks_pay(uint32_t m, uint32_t k, uint32_t n, uint32_t slots, uint32_t groups, uint32_t nkk) {
@@ -142,11 +142,11 @@ inline bool chunks_pay(uint32_t m, uint32_t k, uint32_t n, uint32_t slots, uint3
   const uint32_t tiles = ksplit_tiles(slots, n);
   if (tiles <= 256u) {
     if (!narrow) return false;
-    if (nkk <= 2u) return m <= (k >= 6144u || groups > 8u ? 64u : 48u);
+    if (nkk <= 2u) return m <= (groups > 32u ? 80u : (k >= 6144u || groups > 8u ? 64u : 48u));
     return m <= (k >= 8192u && groups > 8u ? (groups > 32u ? 80u : 64u) : 48u);
   }
   if (narrow) return true;
-  if (tiles <= kKSplitMaxTiles) return groups > 8u && m <= 64u && m <= k / 170u;
+  if (tiles <= kKSplitMaxTiles) return groups > (nkk > 2u ? 8u : 7u) && m <= 64u && m <= k / 170u;
   return groups > 16u || m <= 64u;
 }
 // Whether such a call's prologue leaves z in quarters (quant_lora_kernel's SPLIT form) instead of packed.  The prologue is a chain over K

@@ -16,7 +16,9 @@ CASES = [(65, 8192, 136, 3, 16),    # tiles: a third chunk
          (40, 8192, 4104, 16, 16),  # chunks: the same of a wider weight
          (40, 8192, 4104, 8, 16),   # tiles
          (70, 8192, 4104, 40, 8),   # chunks: tiles would run behind each other
-         (33, 8200, 4104, 0, 0)]    # tiles: no adapters, a wide weight
+         (33, 8200, 4104, 0, 0),    # tiles: no adapters, a wide weight
+         (40, 8192, 7944, 8, 16),   # chunks: eight groups whose tiles would run in pairs
+         (67, 8192, 136, 40, 16)]   # chunks: many groups of few rows
 
 
 @pytest.mark.parametrize("m,k,n,n_ad,rank", CASES)
