@@ -1087,13 +1087,14 @@ __device__ inline void quant_lora_store_quarter(const QuantLoraSplitArgs& a, con
 
 // At a group boundary: the rows of group grp (rowgrp: a lane's slot row lane % 16) keep this pass's sums, the others what they have (`first`: nothing
 // yet).  Zeroing the other groups' rows of x instead leaves them 0 x infinity where the group's A is not finite.
-template <int kCB>
-__device__ inline void keep_group_rows(v4f (&z)[kCB], const v4f (&acc)[kCB], uint32_t rowgrp, uint32_t grp, bool first) {
+template <int kCB, class Keep>
+__device__ inline void keep_group_rows(const v4f (&acc)[kCB], uint32_t rowgrp, uint32_t grp, bool first, Keep&& keep) {
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     const bool own = (uint32_t)__shfl((int)rowgrp, (int)(4u * ((threadIdx.x & 63u) >> 4)) + e, 64) == grp;
 #pragma unroll
-    for (int b = 0; b < kCB; ++b) z[b][e] = own ? acc[b][e] : (first ? 0.0f : z[b][e]);
+    for (int b = 0; b < kCB; ++b)
+      if (own || first) keep(b, e, own ? acc[b][e] : 0.0f);
   }
 }
 
@@ -1221,17 +1222,23 @@ __global__ __launch_bounds__(WAVES * 64, SPLIT ? 2 : 4) void quant_lora_kernel(s
   pass(std::true_type{}, glo);
   if (CB > 0 && ghi > glo) {  // workgroup-uniform
     v4f z[kCB];
-    keep_group_rows<kCB>(z, acc, rowgrp, glo, true);
+    auto keep = [&](int b, int e, float v) {
+      if constexpr (SPLIT) red[wave][b][e][lane] = v;  // (its registers are all taken)
+      else z[b][e] = v;
+    };
+    keep_group_rows<kCB>(acc, rowgrp, glo, true, keep);
 #pragma unroll 1
     for (uint32_t grp = glo + 1u; grp <= ghi; ++grp) {
       if (__builtin_amdgcn_ballot_w64(rowgrp == grp) == 0) continue;
 #pragma unroll
       for (int b = 0; b < kCB; ++b) acc[b] = v4f{0.f, 0.f, 0.f, 0.f};
       pass(std::false_type{}, grp);
-      keep_group_rows<kCB>(z, acc, rowgrp, grp, false);
+      keep_group_rows<kCB>(acc, rowgrp, grp, false, keep);
     }
 #pragma unroll
-    for (int b = 0; b < kCB; ++b) acc[b] = z[b];
+    for (int b = 0; b < kCB; ++b)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[b][e] = SPLIT ? red[wave][b][e][lane] : z[b][e];
   }
   if constexpr (SPLIT) quant_lora_store_quarter<kCB>(a, acc, red, hb, blockIdx.x & 3u);
   else if constexpr (CB > 0) quant_lora_store_z<kCB, WAVES>(a, acc, red, zs, pb, half16);
@@ -1575,7 +1582,7 @@ __global__ __launch_bounds__(1024) void quant_lora_rows_kernel(QuantLoraRowsArgs
       request(grp, kb + 48u, wb2, rb);
     }
     if constexpr (CB == 0) break;
-    if (ghi > glo) keep_group_rows<kCB>(z, acc, rowgrp, grp, first);
+    if (ghi > glo) keep_group_rows<kCB>(acc, rowgrp, grp, first, [&](int b, int e, float v) { z[b][e] = v; });
   }
   if constexpr (CB > 0) {
     if (ghi > glo) {
