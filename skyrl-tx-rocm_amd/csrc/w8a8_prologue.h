@@ -676,8 +676,10 @@ __device__ inline void row_stats(const LoraPrepArgs& p, uint32_t m) {
 
 // (Two workgroups per CU: 4096 rows are 256 blocks of statistics, and the routing block beside them must not
 // put one of them into a second round.)
+// (Aligned so that its 20 KB of instructions lie within 64 KiB: across such a line the launch took 6.4 us instead of 5.95 at 333 rows, 4096 -> 2560, 4
+// adapters of rank 64, in the same code.)
 template <int STATS>  // 0: no row statistics, 1: of x, 2: of the normalized rows
-__global__ __launch_bounds__(1024, 8) void lora_prep_kernel(LoraPrepArgs p) {
+__global__ __launch_bounds__(1024, 8) __attribute__((aligned(32768))) void lora_prep_kernel(LoraPrepArgs p) {
   uint32_t b = blockIdx.x;
   if (b < p.route_blocks) {
     __builtin_amdgcn_s_setprio(3);  // a chain of short steps beside waves that wait for memory
