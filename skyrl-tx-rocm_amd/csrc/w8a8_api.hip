@@ -2140,11 +2140,9 @@ int run_gq_linear(const mi355_w8a8_gq_problem* p, hipStream_t s) {
   q.codes_rm = p->aux_x_codes; q.scales_rm = p->aux_x_scales;
   q.M = p->m; q.M_pad = L.m_pad; q.K = p->k; q.K_pad = p->k_pad; q.group = p->group_size; q.G = L.G;
   q.qmax = p->activation_bits == 4u ? 7.0f : 127.0f;
-  // A row's groups are dealt to several waves: with few rows so that the launch fills the chip (2816 waves), with many so that
-  // a wave that waits for its 3072 values has others beside it.  More waves than that only find less to do each.
-  // One slice from 1024 rows on and 16 below, before, us -> now: K = 12288, groups of 128: 333 rows 13.8 -> 9.5,
-  // 992 23.0 -> 17.5, 1536 30.3 -> 22.3, 4096 54.3 -> 51.8; K = 4096, groups of 64: 700 rows 12.9 -> 7.4, 2048 13.9 -> 13.2;
-  // K = 1024: 992 rows 14.8 -> 5.2, 1536 and more the same single slice (two: 4096 rows 10.5 -> 12.0).
+  // gq_quant_kernel (groups that gq_quant_tile_kernel does not take, and decode): a row's groups are dealt to several
+  // waves, with few rows so that the launch fills the chip (2816 waves), with many so that a wave that waits for its 3072
+  // values has others beside it.  More waves than that only find less to do each.
   uint32_t q_slices = 2816u / L.m_pad;
   if (q_slices < (p->k + 3071u) / 3072u) q_slices = (p->k + 3071u) / 3072u;
   if (q_slices > 16u) q_slices = 16u;
@@ -2155,7 +2153,14 @@ int run_gq_linear(const mi355_w8a8_gq_problem* p, hipStream_t s) {
   // one adapter's z shares the quantizer's launch (rows of 16-byte pieces; several adapters: a wave per row)
   const bool decode_z = decode && p->n_adapters == 1u && (p->k & 7u) == 0 && aligned16(p->x);
   if (!decode_z) {
-    hipLaunchKernelGGL(gq_quant_kernel, dim3(L.m_pad / 4u, q_grid_y), dim3(256), 0, s, q);
+    if (!decode && (p->k & 7u) == 0 && (p->group_size == 32u || p->group_size == 64u || p->group_size == 128u)) {
+      const dim3 qgrid(L.m_pad / 16u, (p->k_pad + 511u) / 512u);
+      if (p->group_size == 32u) hipLaunchKernelGGL((gq_quant_tile_kernel<1>), qgrid, dim3(256), 0, s, q);
+      else if (p->group_size == 64u) hipLaunchKernelGGL((gq_quant_tile_kernel<2>), qgrid, dim3(256), 0, s, q);
+      else hipLaunchKernelGGL((gq_quant_tile_kernel<4>), qgrid, dim3(256), 0, s, q);
+    } else {
+      hipLaunchKernelGGL(gq_quant_kernel, dim3(L.m_pad / 4u, q_grid_y), dim3(256), 0, s, q);
+    }
     if ((st = launch_status())) return st;
   }
 

@@ -64,6 +64,42 @@ __device__ inline uint32_t pack_bf16x2(float lo, float hi) {
 __device__ inline uint32_t f32_to_bf16_bits(float f) { return pack_bf16x2(f, 0.0f) & 0xffffu; }
 __device__ inline float bf16_round_f32(float f) { return bf16_bits_to_f32(f32_to_bf16_bits(f)); }
 
+// Largest |value| of eight bf16 values against a running maximum of pairs: |bf16| compares like its 15
+// magnitude bits as an integer (a NaN ends above every number and the scale then falls back to 1, as the
+// reference's comparison amax > 0 does).
+__device__ inline uint32_t bf16_absmax_pairs(uint32_t amax_bits, const uint4& raw) {
+  typedef unsigned short us2 __attribute__((ext_vector_type(2)));
+  us2 mx = __builtin_bit_cast(us2, amax_bits);
+  mx = __builtin_elementwise_max(mx, __builtin_bit_cast(us2, raw.x & 0x7fff7fffu));
+  mx = __builtin_elementwise_max(mx, __builtin_bit_cast(us2, raw.y & 0x7fff7fffu));
+  mx = __builtin_elementwise_max(mx, __builtin_bit_cast(us2, raw.z & 0x7fff7fffu));
+  mx = __builtin_elementwise_max(mx, __builtin_bit_cast(us2, raw.w & 0x7fff7fffu));
+  return __builtin_bit_cast(uint32_t, mx);
+}
+
+// ---- int8 codes of bf16 values: code = rint(v / scale), the quotient correctly rounded, with scale = amax / qmax for
+// the largest |v|.  q0 = v * r (r: the hardware reciprocal) is corrected by its remainder v - q0 * scale, which a fused
+// multiply-add forms exactly: three operations, no division and no look at how near a tie the quotient lies.  (Ties are
+// common here: v and amax are bf16 values, and 127 v / amax is a half integer for every third value or so of a row whose
+// amax is a power of two.  The form before, one product and a division for the 512 values of a wave where one of them lay
+// near a tie, took that division for every other piece: 28 vector operations a value, now 7.)  That the codes are those
+// of the division was checked for every pair of bf16 significands and every reciprocal within two units of the last place;
+// powers of two drop out while scale and r are ordinary numbers (tests/test_quotient.py).
+__device__ inline float code_quotient(float v, float scale, float r) {
+  const float q0 = v * r;
+  return __builtin_fmaf(__builtin_fmaf(-q0, scale, v), r, q0);
+}
+// The codes of four quotients of at most 127.5, byte e the e-th: 1.5 * 2^23 has a last place of one, so the sum's low byte
+// is the quotient rounded to nearest even in two's complement.
+__device__ inline uint32_t code_bytes4(const float (&q)[4]) {
+  uint32_t m[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) m[e] = __float_as_uint(q[e] + 12582912.0f);
+  const uint32_t lo = __builtin_amdgcn_perm(m[1], m[0], 0x0c0c0400u), hi = __builtin_amdgcn_perm(m[3], m[2], 0x0c0c0400u);
+  return __builtin_amdgcn_perm(hi, lo, 0x05040100u);
+}
+__device__ inline bool code_scale_ordinary(float scale) { return scale > 1e-30f && scale < 1e30f; }
+
 __device__ inline float wave_max(float v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));

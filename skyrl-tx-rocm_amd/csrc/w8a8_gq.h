@@ -99,6 +99,27 @@ __device__ inline void gq_load_piece(const GqQuantArgs& a, const uint16_t* xr, b
   }
 }
 
+// The codes of eight values of a group: code_quotient, or for a group whose scale is not an ordinary number or whose
+// maximum is a NaN (rscale < 0) the division and the clip.
+__device__ inline float gq_rscale(float amax, float scale) {
+  return amax == amax && code_scale_ordinary(scale) ? __builtin_amdgcn_rcpf(scale) : -1.0f;
+}
+__device__ inline uint2 gq_codes8(const float (&v)[8], float scale, float rscale, float qmax) {
+  if (__builtin_amdgcn_ballot_w64(rscale < 0.0f) != 0) {  // wave-uniform
+    uint32_t w[2] = {0, 0};
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {  // biased by 128 into its byte; flipping bit 7 makes it two's complement
+      const float q = fminf(fmaxf(__builtin_rintf(v[j] / scale), -qmax), qmax);
+      w[j >> 2] = __builtin_amdgcn_cvt_pk_u8_f32(q + 128.0f, (uint32_t)j & 3u, w[j >> 2]);
+    }
+    return make_uint2(w[0] ^ 0x80808080u, w[1] ^ 0x80808080u);
+  }
+  float q[2][4];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) q[j >> 2][j & 3] = code_quotient(v[j], scale, rscale);
+  return make_uint2(code_bytes4(q[0]), code_bytes4(q[1]));
+}
+
 __device__ inline void gq_quant_rows(const GqQuantArgs& a, uint32_t row_quad, uint32_t slice) {
   __shared__ float piece_max[4][kGqMaxPieces];
   __shared__ float group_scale[4][kGqMaxGroups];
@@ -123,50 +144,18 @@ __device__ inline void gq_quant_rows(const GqQuantArgs& a, uint32_t row_quad, ui
       for (uint32_t p = 0; p < pieces_per_group; ++p) amax = fmaxf(amax, piece_max[wave][gl * pieces_per_group + p]);
       const float scale = amax > 0.0f ? amax / a.qmax : 1.0f;
       group_scale[wave][gl] = scale;
-      group_rscale[wave][gl] = (amax == amax && scale > 1e-30f && scale < 1e30f) ? __builtin_amdgcn_rcpf(scale) : -1.0f;
+      group_rscale[wave][gl] = gq_rscale(amax, scale);
       a.scales[(size_t)g * a.M_pad + row] = scale;
       if (a.scales_rm && live) a.scales_rm[(size_t)row * a.G + g] = scale;
     }
     __builtin_amdgcn_s_waitcnt(0xc07f);
     __builtin_amdgcn_wave_barrier();
   };
-  // codes = clip(rint(v / scale)) with the correctly rounded quotient.  v * (1 / scale) with the hardware
-  // reciprocal is within 3 * 2^-24 * 128 < 2.3e-5 of it (|quotient| <= qmax <= 127), and forming it biased by
-  // 128 in one fused step adds at most 2^-17: both round to the same integer unless the product lies within
-  // 4e-5 of a tie.  Those pieces, and groups whose scale is not an ordinary number (rscale < 0), are redone
-  // with the division.  |v| <= the group's maximum, so the clip only ever acts in the redone cases.  The
-  // biased value lands in its byte with one v_cvt_pk_u8_f32; flipping bit 7 makes it two's complement.
   auto quantize_piece = [&](uint32_t p, const float (&v)[8]) {
     const uint32_t k = (p_lo + p) * 8u;
-    const float scale = group_scale[wave][p / pieces_per_group];
-    const float rscale = group_rscale[wave][p / pieces_per_group];
-    float c[8];
-    float off_integer = 0.0f;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const float t = __builtin_fmaf(v[j], rscale, 128.0f);
-      c[j] = rintf(t);
-      off_integer = fmaxf(off_integer, fabsf(t - c[j]));
-    }
-    const bool redo = rscale < 0.0f || off_integer > 0.49996f;
-    if (__builtin_amdgcn_ballot_w64(redo) != 0) {  // wave-uniform
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        float q = __builtin_rintf(v[j] / scale);
-        q = fminf(fmaxf(q, -a.qmax), a.qmax);
-        c[j] = q + 128.0f;
-      }
-    }
-    uint32_t w[2] = {0, 0};
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      w[0] = __builtin_amdgcn_cvt_pk_u8_f32(c[j], (uint32_t)j, w[0]);
-      w[1] = __builtin_amdgcn_cvt_pk_u8_f32(c[j + 4], (uint32_t)j, w[1]);
-    }
-    w[0] ^= 0x80808080u;
-    w[1] ^= 0x80808080u;
-    *reinterpret_cast<uint2*>(cblk + (size_t)(k >> 5) * 1024u + ((k >> 4) & 1u) * 512u + (k & 15u)) = make_uint2(w[0], w[1]);
-    if (a.codes_rm && live) *reinterpret_cast<uint2*>(a.codes_rm + (size_t)row * a.K_pad + k) = make_uint2(w[0], w[1]);
+    const uint2 w = gq_codes8(v, group_scale[wave][p / pieces_per_group], group_rscale[wave][p / pieces_per_group], a.qmax);
+    *reinterpret_cast<uint2*>(cblk + (size_t)(k >> 5) * 1024u + ((k >> 4) & 1u) * 512u + (k & 15u)) = w;
+    if (a.codes_rm && live) *reinterpret_cast<uint2*>(a.codes_rm + (size_t)row * a.K_pad + k) = w;
   };
   if ((a.K & 7u) == 0) {
     // rows of 16-byte pieces: the wave's share of the row (at most 2048 pieces, 32 per lane) stays in registers
@@ -223,6 +212,70 @@ __device__ inline void gq_quant_rows(const GqQuantArgs& a, uint32_t row_quad, ui
 }
 
 __global__ __launch_bounds__(256) void gq_quant_kernel(GqQuantArgs a) { gq_quant_rows(a, blockIdx.x, blockIdx.y); }
+
+// The same for groups of 32, 64 or 128 and rows of 16-byte pieces, nothing through the LDS: a wave takes 16 rows x 128 k,
+// lane (i = l % 16, q = l / 16) the k 32 b + 8 q + 0..7 of row i for b = 0..3, so that a group lies in GB of a lane's
+// pieces and the row's four lanes, and the codes of a block go out as 16 rows x 16 consecutive bytes.
+// Bound by HBM where rows are many, else by the launch: 4096 x 12288, groups of 128 (150 MB) 55 -> 32.4 us, 1536 rows 22.0 -> 10.6,
+// 333 8.6 -> 4.7; 4096 x 1024 8.7 -> 4.0.  The kernel above spent most of that in its vector operations, 130 KB of
+// unrolled instructions and 49 KB of LDS a workgroup.  Several chunks of 128 k to a wave, the next on its way: 32.4 -> 32.7 (two)
+// and 34.2 (four), and 10.6 -> 13.0 (four) at 1536 rows.
+template <int GB>  // 32-wide k blocks of a group: 1, 2, 4
+__global__ __launch_bounds__(256) void gq_quant_tile_kernel(GqQuantArgs a) {
+  constexpr uint32_t NG = 4u / GB;  // groups of 128 k
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t c = blockIdx.y * 4u + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // the wave's 128 k
+  const uint32_t kbs = a.K_pad / 32u;
+  if (c * 4u >= kbs) return;
+  const uint32_t i = lane & 15u, q = lane >> 4;
+  const uint32_t row = blockIdx.x * 16u + i;
+  const bool live = row < a.M;
+  const uint16_t* const xr = a.x + (size_t)(live ? row : 0u) * a.K;
+  uint4 r[4];
+#pragma unroll
+  for (uint32_t b = 0; b < 4; ++b) {  // (beyond the matrix: a value that is there, and zeros in its place)
+    const uint32_t k = c * 128u + b * 32u + q * 8u;
+    r[b] = *reinterpret_cast<const uint4*>(xr + (k < a.K ? k : 0u));
+  }
+  if (c * 128u + 128u > a.K || blockIdx.x * 16u + 16u > a.M) {  // wave-uniform
+#pragma unroll
+    for (uint32_t b = 0; b < 4; ++b)
+      if (!live || c * 128u + b * 32u + q * 8u >= a.K) r[b] = make_uint4(0u, 0u, 0u, 0u);
+  }
+  unsigned char* const dst = reinterpret_cast<unsigned char*>(a.codes) + ((size_t)(blockIdx.x >> 1) * kbs + c * 4u) * 1024u +
+                             (16u * (blockIdx.x & 1u) + i + 32u * (q >> 1)) * 16u + 8u * (q & 1u);
+#pragma unroll
+  for (uint32_t g = 0; g < NG; ++g) {
+    uint32_t top2 = 0u;
+#pragma unroll
+    for (uint32_t b = 0; b < (uint32_t)GB; ++b) top2 = bf16_absmax_pairs(top2, r[g * GB + b]);
+    uint32_t top = (top2 >> 16) > (top2 & 0xffffu) ? top2 >> 16 : top2 & 0xffffu;
+    const auto s16 = __builtin_amdgcn_permlane16_swap(top, top, false, false);  // with the other lanes of the row
+    top = s16[0] > s16[1] ? s16[0] : s16[1];
+    const auto s32 = __builtin_amdgcn_permlane32_swap(top, top, false, false);
+    top = s32[0] > s32[1] ? s32[0] : s32[1];
+    const float amax = __uint_as_float(top << 16);
+    const float scale = amax > 0.0f ? amax / a.qmax : 1.0f;
+    const float rscale = gq_rscale(amax, scale);
+    const uint32_t gi = c * NG + g;
+    if (q == 0 && gi < a.G) {
+      a.scales[(size_t)gi * a.M_pad + row] = scale;
+      if (a.scales_rm && live) a.scales_rm[(size_t)row * a.G + gi] = scale;
+    }
+#pragma unroll
+    for (uint32_t b = g * GB; b < (g + 1u) * GB; ++b) {
+      const uint32_t w[4] = {r[b].x, r[b].y, r[b].z, r[b].w};
+      float v[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] = (j & 1) ? __uint_as_float(w[j >> 1] & 0xffff0000u) : __uint_as_float(w[j >> 1] << 16);
+      const uint2 codes = gq_codes8(v, scale, rscale, a.qmax);
+      if (c * 4u + b < kbs) {  // wave-uniform
+        *reinterpret_cast<uint2*>(dst + b * 1024u) = codes;
+        if (a.codes_rm && live) *reinterpret_cast<uint2*>(a.codes_rm + (size_t)row * a.K_pad + c * 128u + b * 32u + q * 8u) = codes;
+      }
+    }
+  }
+}
 
 // ---------------------------------------------------------------------------------------
 struct GqLoraZArgs {

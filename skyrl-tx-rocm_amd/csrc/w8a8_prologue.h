@@ -564,18 +564,6 @@ struct LoraPrepArgs {
   uint16_t* xn_aux;            // bf16 [M, K] normalized rows for the caller, or null (STATS == 2)
 };
 
-// Largest |value| of eight bf16 values against a running maximum of pairs: |bf16| compares like its 15
-// magnitude bits as an integer (a NaN ends above every number and the scale then falls back to 1, as the
-// reference's comparison amax > 0 does).
-__device__ inline uint32_t bf16_absmax_pairs(uint32_t amax_bits, const uint4& raw) {
-  typedef unsigned short us2 __attribute__((ext_vector_type(2)));
-  us2 mx = __builtin_bit_cast(us2, amax_bits);
-  mx = __builtin_elementwise_max(mx, __builtin_bit_cast(us2, raw.x & 0x7fff7fffu));
-  mx = __builtin_elementwise_max(mx, __builtin_bit_cast(us2, raw.y & 0x7fff7fffu));
-  mx = __builtin_elementwise_max(mx, __builtin_bit_cast(us2, raw.z & 0x7fff7fffu));
-  mx = __builtin_elementwise_max(mx, __builtin_bit_cast(us2, raw.w & 0x7fff7fffu));
-  return __builtin_bit_cast(uint32_t, mx);
-}
 // (x * inv) * gamma, one bf16 rounding, of eight values
 __device__ inline uint4 rms_normalize8(const uint4& raw, float inv, const float4& g0, const float4& g1) {
   const float g[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
@@ -971,43 +959,36 @@ __global__ __launch_bounds__(256) void codes_row_major_kernel(const unsigned cha
 
 constexpr uint32_t kPaddedRouteMaxRows = 8192;  // groups start on block boundaries up to here (padded_groups_fit)
 
+// How a wave's rows are quantized: 0 by code_quotient; 1 the same, but a scale of one may stand for a row with a NaN, whose
+// other values then need the clip; 2 a scale is not an ordinary number.  Wave-uniform.
+__device__ inline uint32_t quant_mode(float scale) {
+  if (__builtin_amdgcn_ballot_w64(!code_scale_ordinary(scale)) != 0) return 2u;
+  return __builtin_amdgcn_ballot_w64(scale == 1.0f) != 0 ? 1u : 0u;
+}
 // The int8 codes of eight (normalized) bf16 values.
-__device__ inline uint2 quant_codes8(const uint4& raw, float scale, float rscale, bool scale_safe) {
+__device__ inline uint2 quant_codes8(const uint4& raw, float scale, float rscale, uint32_t mode) {
   const uint32_t nb[4] = {raw.x, raw.y, raw.z, raw.w};  // the (normalized) values as bf16 pairs
   float v[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e)
     v[e] = (e & 1) ? __uint_as_float(nb[e >> 1] & 0xffff0000u) : __uint_as_float(nb[e >> 1] << 16);
-  // codes = rint(v / scale) with the correctly rounded quotient.  v * (1 / scale) with the
-  // hardware reciprocal is within 3 * 2^-24 * 128 < 2.3e-5 of it, so both round to the same
-  // integer unless the product lies that close to a tie; those cases (and scales outside the
-  // reciprocal's safe range) are redone with the division.
-  // The codes are formed biased by 128 (the fused v * (1 / scale) + 128 adds at most another 2^-17 to
-  // the distance above, still far inside the tie margin): c is then an integer in [1, 255] (|v| <= the
-  // row's absmax, so the clip of the reference never acts), lands in its byte with one
-  // v_cvt_pk_u8_f32, and flipping bit 7 of every byte turns the biased value into two's complement.
-  float c[8];
-  float off_integer = 0.0f;  // largest distance of a quotient from its rounded value
+  if (mode != 0u) {
+    const uint32_t top = bf16_absmax_pairs(0u, raw);  // beyond 127.5, as no value of a row of scale one without a NaN is
+    if (mode == 2u || __builtin_amdgcn_ballot_w64(scale == 1.0f && ((top >> 16) > 0x42ffu || (top & 0xffffu) > 0x42ffu)) != 0) {
+      // biased by 128 the code lands in its byte, clipped, with one v_cvt_pk_u8_f32; flipping bit 7 makes it two's complement
+      uint32_t lo = 0, hi = 0;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    const float t = __builtin_fmaf(v[e], rscale, 128.0f);
-    c[e] = rintf(t);
-    off_integer = fmaxf(off_integer, fabsf(t - c[e]));
+      for (int e = 0; e < 4; ++e) {
+        lo = __builtin_amdgcn_cvt_pk_u8_f32(rintf(v[e] / scale) + 128.0f, (uint32_t)e, lo);
+        hi = __builtin_amdgcn_cvt_pk_u8_f32(rintf(v[e + 4] / scale) + 128.0f, (uint32_t)e, hi);
+      }
+      return make_uint2(lo ^ 0x80808080u, hi ^ 0x80808080u);
+    }
   }
-  const bool redo = !scale_safe || off_integer > 0.49996f;  // margin 4e-5 > 2.3e-5 + 2^-17
-  if (__builtin_amdgcn_ballot_w64(redo) != 0) {  // wave-uniform
+  float q[2][4];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) c[e] = rintf(v[e] / scale) + 128.0f;
-  }
-  uint32_t lo = 0, hi = 0;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    lo = __builtin_amdgcn_cvt_pk_u8_f32(c[e], (uint32_t)e, lo);
-    hi = __builtin_amdgcn_cvt_pk_u8_f32(c[e + 4], (uint32_t)e, hi);
-  }
-  lo ^= 0x80808080u;  // (a lane without a value holds zeros: 0 -> 128 -> code 0)
-  hi ^= 0x80808080u;
-  return make_uint2(lo, hi);
+  for (int e = 0; e < 8; ++e) q[e >> 2][e & 3] = code_quotient(v[e], scale, rscale);
+  return make_uint2(code_bytes4(q[0]), code_bytes4(q[1]));
 }
 
 // z of a half block: the waves' tiles added in a fixed order, split into three bf16 terms and stored as the GEMM
@@ -1168,7 +1149,7 @@ __global__ __launch_bounds__(WAVES * 64, SPLIT ? 2 : 4) void quant_lora_kernel(s
       o.g1 = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(grsrc, off + 16u, 0, 0));
     }
   };
-  const bool scale_safe = scale > 1e-30f && scale < 1e30f;
+  const uint32_t mode = quant_mode(scale);
   auto work = [&](auto codes, uint32_t j, const uint4& rawx, const Operands& o) {
     const uint32_t kb = vw + kStride * j;
     uint4 raw = rawx;
@@ -1179,7 +1160,7 @@ __global__ __launch_bounds__(WAVES * 64, SPLIT ? 2 : 4) void quant_lora_kernel(s
       raw.x = live ? raw.x : 0u; raw.y = live ? raw.y : 0u; raw.z = live ? raw.z : 0u; raw.w = live ? raw.w : 0u;
     }
     if constexpr (decltype(codes)::value) {
-      *reinterpret_cast<uint2*>(xq_dst + (size_t)kb * kBlockBytes) = quant_codes8(raw, scale, rscale, scale_safe);
+      *reinterpret_cast<uint2*>(xq_dst + (size_t)kb * kBlockBytes) = quant_codes8(raw, scale, rscale, mode);
     }
     if constexpr (CB > 0) {
       const v4i xa = {(int)raw.x, (int)raw.y, (int)raw.z, (int)raw.w};
@@ -1523,7 +1504,7 @@ __global__ __launch_bounds__(1024) void quant_lora_rows_kernel(QuantLoraRowsArgs
   const int src = mine_row ? row_src[i] : -1;
   const float scale = mine_row ? row_scale[i] : 1.0f;
   const float rscale = __builtin_amdgcn_rcpf(scale);
-  const bool scale_safe = scale > 1e-30f && scale < 1e30f;
+  const uint32_t mode = quant_mode(scale);
   const unsigned char* const rowl = ql_lds + (mine_row ? i - r0 : 0u) * p.row_stride;
   const uint32_t range = CB == 0 ? 0u : (route_here ? route_range : (a.blk_range ? (uint32_t)a.blk_range[pb] : 0u));
   const uint32_t glo = range & 0xffffu, ghi = range >> 16;
@@ -1551,7 +1532,7 @@ __global__ __launch_bounds__(1024) void quant_lora_rows_kernel(QuantLoraRowsArgs
   };
   auto work = [&](bool first, uint32_t kb, const v4i (&w)[kCB], const uint4& raw) {
     if (first) {  // wave-uniform
-      const uint2 codes = quant_codes8(raw, scale, rscale, scale_safe);
+      const uint2 codes = quant_codes8(raw, scale, rscale, mode);
       if (mine_row) *reinterpret_cast<uint2*>(xq_dst + (size_t)kb * kBlockBytes) = codes;
     }
     if constexpr (CB > 0) {
