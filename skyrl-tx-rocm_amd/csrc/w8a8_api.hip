@@ -97,6 +97,23 @@ inline bool padded_groups_fit(uint32_t m, uint32_t n, uint32_t n_groups, bool wi
          rounds((uint64_t)(round_up(base, tile_m) / tile_m) * per_row, resident);
 }
 
+// Tiles of 192 x 256 instead of 256 x 256 where they fill the chip's rounds of 256 tiles better.  A round of them takes 0.79 of
+// the time; beside the rounds the tiles themselves count, since a partly filled round runs at a higher clock.  The GEMM, 256 / 192
+// rows, us: 2560 -> 6144, rank 64, 1536 rows (144 / 192 tiles) 42.1 / 33.5, 1900 (192 / 240) 46.3 / 35.1, 2800 (264 / 360) 80.9 / 63.1, 3900 (384 /
+// 504) 88.2 / 67.1; 2560 -> 10240, rank 64, 2048 (320 / 440) 83.3 / 67.6; 12288 -> 4096, rank 32, 3003 (192 / 256) 134.5 / 120.3; 4096 -> 24576, rank
+// 32, 1281 (576 / 672) 154.9 / 135.3, 3003 (1152 / 1536) 278 / 269, 2300 (864 / 1152) 213 / 224, 2800 (1056 / 1440) 263 / 275.
+inline uint64_t gemm16_tiles(uint32_t rows_bound, uint32_t n, uint32_t tile_rows) {
+  return (uint64_t)((rows_bound + tile_rows - 1u) / tile_rows) * (n_padded(n) / (uint32_t)kG16TileN);
+}
+inline bool gemm16_short_tiles(uint32_t rows_bound, uint32_t n, uint32_t flags) {
+  const uint64_t t6 = gemm16_tiles(rows_bound, n, 192u), t8 = gemm16_tiles(rows_bound, n, 256u);
+  return !(flags & MI355_W8A8_FLAG_TILE_256X256) && ((t6 + 255u) / 256u * 256u + t6) * 79u < ((t8 + 255u) / 256u * 256u + t8) * 100u;
+}
+// the rounds of such a call, in hundredths of one of 256 x 256 tiles
+inline uint64_t gemm16_rounds(uint32_t rows_bound, uint32_t n, uint32_t flags) {
+  return gemm16_short_tiles(rows_bound, n, flags) ? (gemm16_tiles(rows_bound, n, 192u) + 255u) / 256u * 79u : (gemm16_tiles(rows_bound, n, 256u) + 255u) / 256u * 100u;
+}
+
 // 64 x 128 tiles of a call whose slots end at rows_bound, the waves of a workgroup splitting K (w8a8_gemm_ksplit_kernel), and
 // whether it takes them: while all are resident at once, one to a CU (up to 256) or two.  Beyond, the 128 x 128 geometry moves
 // fewer bytes.  Whole call, the other prologue in front of the 128 x 128 tiles: 4096 -> 2560, rank 64: 333 rows 34 us against 51, 700 (480 tiles)
@@ -307,28 +324,28 @@ int launch_grouped(const GemmArgs& g, uint32_t nkk, hipStream_t s) {
   }
 }
 
-template <int EPI, int NKK, int NW = 4>
+template <int EPI, int NKK, int NW = 4, int MF = 8>
 int launch_gemm16_one(const GemmArgs& g, hipStream_t s) {
   // persistent grid: one workgroup per CU (two in the 256 x 128 geometry), a multiple of 8 so that every
   // XCD gets the same share
-  using Geo = G16Geo<NW>;
+  using Geo = G16Geo<NW, MF>;
   const uint32_t ntile = g.tiles_m * g.tiles_n;
   const uint32_t want = ((ntile + 7u) / 8u) * 8u;
   const dim3 grid(want < (uint32_t)Geo::kResident ? want : (uint32_t)Geo::kResident), block(Geo::kThreads);
-  if (hipFuncSetAttribute(reinterpret_cast<const void*>(&w8a8_gemm16_kernel<EPI, NKK, NW>),
+  if (hipFuncSetAttribute(reinterpret_cast<const void*>(&w8a8_gemm16_kernel<EPI, NKK, NW, MF>),
                           hipFuncAttributeMaxDynamicSharedMemorySize, Geo::kLdsBytes) != hipSuccess)
     return MI355_W8A8_ERR_LAUNCH;
-  hipLaunchKernelGGL((w8a8_gemm16_kernel<EPI, NKK, NW>), grid, block, Geo::kLdsBytes, s, g);
+  hipLaunchKernelGGL((w8a8_gemm16_kernel<EPI, NKK, NW, MF>), grid, block, Geo::kLdsBytes, s, g);
   return launch_status();
 }
 
-template <int EPI, int NW = 4>
+template <int EPI, int NW = 4, int MF = 8>
 int launch_gemm16(const GemmArgs& g, uint32_t nkk, hipStream_t s) {
   switch (nkk) {
-    case 0: return launch_gemm16_one<EPI, 0, NW>(g, s);
-    case 1: return launch_gemm16_one<EPI, 1, NW>(g, s);
-    case 2: return launch_gemm16_one<EPI, 2, NW>(g, s);
-    case 4: return launch_gemm16_one<EPI, 4, NW>(g, s);
+    case 0: return launch_gemm16_one<EPI, 0, NW, MF>(g, s);
+    case 1: return launch_gemm16_one<EPI, 1, NW, MF>(g, s);
+    case 2: return launch_gemm16_one<EPI, 2, NW, MF>(g, s);
+    case 4: return launch_gemm16_one<EPI, 4, NW, MF>(g, s);
     default: return MI355_W8A8_ERR_UNSUPPORTED;
   }
 }
@@ -592,7 +609,8 @@ int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
                    ksplit_padding_pays(p->m, p->k, p->n, p->n_adapters, rank_chunks(p->rank))) &&
                   // (in the place of chunks on the K-split tiles only, which they fit unpadded: sums_again)
                   (reported != MI355_W8A8_PATH_SKINNY_CHUNKS || ksplit_fits(padded_rows_bound(p->m, p->n_adapters), p->n))) ||
-                 (path == MI355_W8A8_PATH_TILED_256X256 && padded_groups_fit(p->m, p->n, p->n_adapters, true)));
+                 (path == MI355_W8A8_PATH_TILED_256X256 && padded_groups_fit(p->m, p->n, p->n_adapters, true) &&
+                  gemm16_rounds(padded_rows_bound(p->m, p->n_adapters), p->n, p->flags) <= gemm16_rounds(round_up(p->m, 32u), p->n, p->flags)));
   const WsLayout w = make_layout(p->m, p->k, p->n, p->n_adapters, lora ? p->rank : 0u, routed, pad_groups);
   unsigned char* ws = static_cast<unsigned char*>(p->workspace);
   int32_t* src_row = reinterpret_cast<int32_t*>(ws + w.src_row);
@@ -770,6 +788,10 @@ int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
                            : (small ? launch_gemm_one<kEpiAcc, 0, kModeDense128>(ga, s) : launch_gemm_one<kEpiAcc, 0, kModeDense>(ga, s)))))
       return st;
     g.tile_ctr += 128;  // the second counter set
+  }
+  if (wide && gemm16_short_tiles(w.rows_bound, p->n, p->flags)) {
+    g.tiles_m = (w.rows_bound + 191u) / 192u;
+    return swiglu ? launch_gemm16<kEpiSwiglu, 4, 6>(g, w.nkk, s) : launch_gemm16<kEpiPlain, 4, 6>(g, w.nkk, s);
   }
   if (wide) return swiglu ? launch_gemm16<kEpiSwiglu>(g, w.nkk, s) : launch_gemm16<kEpiPlain>(g, w.nkk, s);
   if (pair) return swiglu ? launch_gemm16<kEpiSwiglu, 2>(g, w.nkk, s) : launch_gemm16<kEpiPlain, 2>(g, w.nkk, s);

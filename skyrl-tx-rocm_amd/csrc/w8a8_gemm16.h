@@ -52,15 +52,20 @@ constexpr uint32_t kG16MinKPad = 384;               // at least six stages: the 
 //           three 24 KiB stages each: while one workgroup runs its epilogue on the vector ALU the other's
 //           main loop has the matrix core to itself.
 // The wave tile (128 x 64), its fragment reads and its epilogue are the same in both.
-template <int NW>
+// MF, the 16-row fragments of a wave: 8, or 6 for tiles of 192 rows (NW = 4) where those fill the chip's rounds better
+// (gemm16_fragments).  A stage is then 28 KiB, brought in by seven of the eight waves.
+template <int NW, int MF = 8>
 struct G16Geo {
+  static constexpr int kTileM = 32 * MF;
   static constexpr int kTileN = 64 * NW;
   static constexpr int kStages = NW == 4 ? 4 : 3;
-  static constexpr int kStageBytes = 16384 + 4096 * NW;  // A: 8 row blocks x 2 k blocks, then B: 2 NW column blocks x 2 k blocks
+  static constexpr int kStageABytes = 2048 * MF;                   // A: MF row blocks x 2 k blocks
+  static constexpr int kStageBytes = kStageABytes + 4096 * NW;     // then B: 2 NW column blocks x 2 k blocks
   static constexpr int kRingBytes = kStages * kStageBytes;
   static constexpr int kWaves = 2 * NW;
   static constexpr int kLdsBytes = kRingBytes + kWaves * 1024 + (NW == 4 ? 0 : 64);  // + per wave 128 row scales and 128 row positions (+ the next tile's position)
-  static constexpr int kLoads = kStageBytes / 1024 / kWaves;     // direct-to-LDS loads per wave and stage (4 or 6)
+  static constexpr int kLoads = NW == 4 ? 4 : 6;                 // direct-to-LDS loads per wave and stage
+  static constexpr int kLoadWaves = kStageBytes / 1024 / kLoads; // waves that have any
   static constexpr int kThreads = 64 * kWaves;
   static constexpr int kResident = NW == 4 ? 256 : 512;          // workgroups the chip holds at once
 };
@@ -92,12 +97,13 @@ template <int OFF>
 __device__ inline void g16_load_1k_m0(const unsigned char* base_uniform, uint32_t voff) {  // M0 set before
   asm volatile("global_load_lds_dwordx4 %0, %1 offset:%2" :: "v"(voff), "s"(base_uniform), "n"(OFF) : "memory", "m0");
 }
-// One wave copies 128 dwords: lane l moves global[base + 4 l] and global[base + 256 + 4 l] to the same
-// offsets behind lds_addr.
-__device__ inline void g16_load_128_dwords(const void* base_uniform, uint32_t lane4, uint32_t lds_addr_uniform) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1\n\t"
-               "global_load_lds_dword %0, %1 offset:256"
-               :: "v"(lane4), "s"(base_uniform), "s"(lds_addr_uniform) : "memory", "m0");
+// One wave copies 128 dwords: lane l moves global[base + voff0] and global[base + voff1] to lds_addr + 4 l and + 256 + 4 l
+// (base1: base - 256, since the instruction offset applies to both addresses).
+__device__ inline void g16_load_128_dwords(const void* base_uniform, const void* base1_uniform, uint32_t voff0, uint32_t voff1,
+                                           uint32_t lds_addr_uniform) {
+  asm volatile("s_mov_b32 m0, %4\n\ts_nop 0\n\tglobal_load_lds_dword %0, %2\n\t"
+               "global_load_lds_dword %1, %3 offset:256"
+               :: "v"(voff0), "v"(voff1), "s"(base_uniform), "s"(base1_uniform), "s"(lds_addr_uniform) : "memory", "m0");
 }
 // LDS fragment read.  These are ordinary loads the compiler keeps its books on: it places the waits
 // (precisely, since it never sees the direct-to-LDS loads) and may spill or move the values safely.
@@ -131,10 +137,11 @@ __device__ inline void g16_mfma_first(v4i& acc, const v4i& a, const v4i& b) {
 constexpr int g16_frag_off(int f) { return (f >> 1) * 2048 + (f & 1) * 256; }  // activation fragment f of a wave's four row blocks
 constexpr int g16_bfrag_off(int j) { return j * 2048; }                        // weight fragment j: the wave's half of column block j
 
-template <int EPI, int NKK, int NW = 4>
+template <int EPI, int NKK, int NW = 4, int MF = 8>
 __global__ __launch_bounds__(G16Geo<NW>::kThreads, NW == 4 ? 1 : 2)
 void w8a8_gemm16_kernel(GemmArgs g) {
-  using Geo = G16Geo<NW>;
+  using Geo = G16Geo<NW, MF>;
+  static_assert(MF == 8 || (MF == 6 && NW == 4), "");
   constexpr int kS = Geo::kStages;
   constexpr int kLoads = Geo::kLoads;
   constexpr uint32_t kSB = Geo::kStageBytes;
@@ -146,7 +153,7 @@ void w8a8_gemm16_kernel(GemmArgs g) {
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wrow = wave / NW, wcol = wave % NW;  // wave tile: rows 128 wrow, columns 64 wcol of the tile
+  const int wrow = wave / NW, wcol = wave % NW;  // wave tile: rows 16 MF wrow, columns 64 wcol of the tile
   const int cgrp = wcol >> 1, chalf = wcol & 1;  // its 128-column group inside the tile and its half of every block
   const uint32_t c16 = lane & 15, q = lane >> 4;
   // byte offset of the lane's 16 bytes inside a pair of k blocks (lower 16 rows of the block)
@@ -173,32 +180,34 @@ void w8a8_gemm16_kernel(GemmArgs g) {
     const uint32_t in_band = t - band * GM * g.tiles_n;
     T.tm = band * GM + in_band % band_rows;
     T.tn = in_band / band_rows;
-    T.Ag = g.xq + (size_t)T.tm * 8u * g.KB * kBlockBytes;
+    T.Ag = g.xq;
     T.Bg = g.wp;
     T.swp = g.sw;
     T.valid = true;
     return T;
   };
-  // chunk ch = kLoads wave + i of a stage: 0..15 activations (row block ch / 2, k block ch % 2), 16..
+  // chunk ch = kLoads wave + i of a stage: 0 .. 2 MF - 1 activations (row block ch / 2, k block ch % 2), then the
   // weights; stage kt of a chunk lies 2 KiB * kt behind its base.  Returned: base - 1024 (i % 4), see
   // g16_load_4k.
   auto chunk_base = [&](const GemmTile& Tx, int i) -> const unsigned char* {
     const int ch = wave * kLoads + i;
-    const bool isA = ch < 16;
-    uint32_t rb = isA ? (uint32_t)(ch >> 1) : Tx.tn * (uint32_t)(2 * NW) + (uint32_t)((ch - 16) >> 1);
-    if (!isA && rb >= ncb_total) rb = ncb_total - 1u;  // keep every wave's load count equal
+    const bool isA = ch < 2 * MF;
+    uint32_t rb = isA ? Tx.tm * (uint32_t)MF + (uint32_t)(ch >> 1) : Tx.tn * (uint32_t)(2 * NW) + (uint32_t)((ch - 2 * MF) >> 1);
+    const uint32_t last = isA ? g.slots / 32u - 1u : ncb_total - 1u;
+    if (rb > last) rb = last;  // keep every wave's load count equal
     return (isA ? Tx.Ag : Tx.Bg) + ((size_t)rb * g.KB + (uint32_t)(ch & 1)) * kBlockBytes - (size_t)(i & 3) * 1024u;
   };
   // the wave's loads of one stage: lane offset voff inside the chunks, LDS address of its first chunk
   auto load_stage = [&](const unsigned char* const* cb, uint32_t voff, uint32_t dst) {
     if constexpr (kS != 4) dst = __builtin_amdgcn_readfirstlane(dst);  // (the ring position modulo 3 is formed on the vector ALU)
+    if (Geo::kLoadWaves < Geo::kWaves && wave >= Geo::kLoadWaves) return;
     g16_load_4k(cb[0], cb[1], cb[2], cb[3], voff, dst);
     if constexpr (kLoads == 6) g16_load_2k(cb[4], cb[5], voff, dst + 4096u);
   };
 
   const uint32_t lds_addr = (uint32_t)(uintptr_t)(lptr_t)lds;
-  const uint32_t a0 = lds_addr + (uint32_t)wrow * 8192u + lane_off;           // activation fragments, ring slot 0
-  const uint32_t b0 = lds_addr + 16384u + (uint32_t)cgrp * 8192u + (uint32_t)chalf * 256u + lane_off;  // weight fragments, ring slot 0
+  const uint32_t a0 = lds_addr + (uint32_t)wrow * (Geo::kStageABytes / 2) + lane_off;  // activation fragments, ring slot 0
+  const uint32_t b0 = lds_addr + Geo::kStageABytes + (uint32_t)cgrp * 8192u + (uint32_t)chalf * 256u + lane_off;  // weight fragments, ring slot 0
   const uint32_t dma0 = lds_addr + (uint32_t)wave * (kLoads * kBlockBytes);  // the wave's chunks, ring slot 0
   // per wave: f32 sx[128] then int32 src_row[128] of its rows, behind the stage ring
   unsigned char* const rowdata = lds + Geo::kRingBytes + wave * 1024;  // (the waves of a row half hold the same data)
@@ -243,9 +252,9 @@ void w8a8_gemm16_kernel(GemmArgs g) {
 #pragma unroll
     for (int i = 0; i < kLoads; ++i) cbase[i] = chunk_base(T, i);
 
-    v4i acc[8][4];
+    v4i acc[MF][4];
     v4i bf[2][4];  // weight fragments of the current / next stage
-    v4i af[4];     // activation fragments, three ahead of the MFMAs
+    v4i af[4];     // activation fragments, three ahead of the MFMAs: fragment f of a stage of parity P in af[(f + MF P) % 4]
     if (!prefetched) {
 #pragma unroll
       for (int st = 0; st < kS; ++st) {
@@ -295,28 +304,24 @@ void w8a8_gemm16_kernel(GemmArgs g) {
       const uint32_t sa = a0s + slot * kSB;
       const uint32_t san = a0s + slot_n * kSB;
       const uint32_t sbn = b0s + slot_n * kSB;
+      constexpr int o = P ? MF & 3 : 0, on = P ? 0 : MF & 3;  // af's place of fragment 0, here and of the next stage
       auto mfma_row = [&](auto BI) {
         constexpr int bi = decltype(BI)::value;
 #pragma unroll
         for (int bj = 0; bj < 4; ++bj) {
-          if constexpr (first) g16_mfma_first(acc[bi][bj], af[bi & 3], bf[P][bj]);
-          else g16_mfma(acc[bi][bj], af[bi & 3], bf[P][bj]);
+          if constexpr (first) g16_mfma_first(acc[bi][bj], af[(bi + o) & 3], bf[P][bj]);
+          else g16_mfma(acc[bi][bj], af[(bi + o) & 3], bf[P][bj]);
         }
         __builtin_amdgcn_sched_barrier(0);
       };
       using std::integral_constant;
       // in flight here, oldest first: B0..B3, A0, A1, A2 of this stage
-      af[3] = g16_ds_read<g16_frag_off(3)>(sa);
-      mfma_row(integral_constant<int, 0>{});
-      af[0] = g16_ds_read<g16_frag_off(4)>(sa);
-      mfma_row(integral_constant<int, 1>{});
-      af[1] = g16_ds_read<g16_frag_off(5)>(sa);
-      mfma_row(integral_constant<int, 2>{});
-      af[2] = g16_ds_read<g16_frag_off(6)>(sa);
-      mfma_row(integral_constant<int, 3>{});
-      af[3] = g16_ds_read<g16_frag_off(7)>(sa);
-      mfma_row(integral_constant<int, 4>{});
-      mfma_row(integral_constant<int, 5>{});
+      g16_for<0, MF - 3>([&](auto BI) {
+        constexpr int bi = decltype(BI)::value;
+        af[(bi + 3 + o) & 3] = g16_ds_read<g16_frag_off(bi + 3)>(sa);
+        mfma_row(BI);
+      });
+      mfma_row(integral_constant<int, MF - 3>{});
       // The next stage must have landed: own loads first, then everybody's; the barrier also ends every
       // wave's reads of this stage's buffer.  Three stages are in the queue behind this one as long as
       // the tile or a next tile provides them.
@@ -334,12 +339,12 @@ void w8a8_gemm16_kernel(GemmArgs g) {
       auto one = [&](auto BI, auto BJ) {
         constexpr int bi = decltype(BI)::value, bj = decltype(BJ)::value;
         __builtin_amdgcn_sched_barrier(0);
-        if constexpr (first) g16_mfma_first(acc[bi][bj], af[bi & 3], bf[P][bj]);
-        else g16_mfma(acc[bi][bj], af[bi & 3], bf[P][bj]);
+        if constexpr (first) g16_mfma_first(acc[bi][bj], af[(bi + o) & 3], bf[P][bj]);
+        else g16_mfma(acc[bi][bj], af[(bi + o) & 3], bf[P][bj]);
         __builtin_amdgcn_sched_barrier(0);
       };
-      using C6 = integral_constant<int, 6>;
-      using C7 = integral_constant<int, 7>;
+      using C6 = integral_constant<int, MF - 2>;
+      using C7 = integral_constant<int, MF - 1>;
       one(C6{}, integral_constant<int, 0>{});
       if constexpr (REM >= 1) {
         bf[1 - P][0] = g16_ds_read<g16_bfrag_off(0)>(sbn);
@@ -352,12 +357,12 @@ void w8a8_gemm16_kernel(GemmArgs g) {
       }
       one(C6{}, integral_constant<int, 2>{});
       if constexpr (REM >= 1) {
-        af[0] = g16_ds_read<g16_frag_off(0)>(san);
-        af[1] = g16_ds_read<g16_frag_off(1)>(san);
+        af[on] = g16_ds_read<g16_frag_off(0)>(san);
+        af[(1 + on) & 3] = g16_ds_read<g16_frag_off(1)>(san);
       }
       one(C6{}, integral_constant<int, 3>{});
       one(C7{}, integral_constant<int, 0>{});
-      if constexpr (REM >= 1) af[2] = g16_ds_read<g16_frag_off(2)>(san);
+      if constexpr (REM >= 1) af[(2 + on) & 3] = g16_ds_read<g16_frag_off(2)>(san);
       if (REM >= kS || (REM >= 1 && has_next)) {  // compile-time facts but has_next; the last stage issues none
         const uint32_t voff4 = (uint32_t)(REM >= kS ? kt + kS : kt + kS - KT) * 2048u + (uint32_t)lane * 16u;
         if constexpr (REM >= kS) load_stage(cbase, voff4, dma0 + slot * kSB);
@@ -386,12 +391,24 @@ void w8a8_gemm16_kernel(GemmArgs g) {
     // adapters present in the wave's four 32-row blocks: one scalar load (the compiler would
     // fetch them through the vector memory path and wait vmcnt(0))
     v4i range4 = {0, 0, 0, 0};
-    if (kLora && g.blk_range)
-      asm volatile("s_load_dwordx4 %0, %1, 0x0\n\ts_waitcnt lgkmcnt(0)"
-                   : "=s"(range4) : "s"(g.blk_range + (T.tm * 256u + wrow * 128u) / 32u) : "memory");
+    if (kLora && g.blk_range) {
+      if constexpr (MF == 8) {
+        asm volatile("s_load_dwordx4 %0, %1, 0x0\n\ts_waitcnt lgkmcnt(0)"
+                     : "=s"(range4) : "s"(g.blk_range + (T.tm * 256u + wrow * 128u) / 32u) : "memory");
+      } else {  // (three blocks, of which the last tile may lack some: the last existing one in their place)
+        const uint32_t blk = (T.tm * (uint32_t)Geo::kTileM + wrow * (16u * MF)) / 32u, last = g.slots / 32u - 1u;
+        const int32_t* const r0 = g.blk_range + (blk < last ? blk : last);
+        const int32_t* const r1 = g.blk_range + (blk + 1u < last ? blk + 1u : last);
+        const int32_t* const r2 = g.blk_range + (blk + 2u < last ? blk + 2u : last);
+        int v0, v1, v2;
+        asm volatile("s_load_dword %0, %3, 0x0\n\ts_load_dword %1, %4, 0x0\n\ts_load_dword %2, %5, 0x0\n\ts_waitcnt lgkmcnt(0)"
+                     : "=&s"(v0), "=&s"(v1), "=&s"(v2) : "s"(r0), "s"(r1), "s"(r2) : "memory");
+        range4 = v4i{v0, v1, v2, v2};
+      }
+    }
     // ---- What the epilogue works with is set up here, behind the main loop's bulk, so that none of it
     // is live (or spilled) across the loop; preload() requests what it starts from.
-    const uint32_t m0 = T.tm * 256u + wrow * 128u;     // first slot of the wave
+    const uint32_t m0 = T.tm * (uint32_t)Geo::kTileM + wrow * (16u * MF);  // first slot of the wave
     const uint32_t tgrp0 = T.tn * (uint32_t)Geo::kTileN + cgrp * 128u;  // first column of the wave's group of 128
     const uint32_t tcol0 = tgrp0 + chalf * 64u;        // first of the wave's 64 columns
     const bool wave_live = tcol0 < g.N;                // wave-uniform; a dead wave only feeds the loads
@@ -428,7 +445,9 @@ void w8a8_gemm16_kernel(GemmArgs g) {
       blane[ks] = kk * kBlockBytes + lora_lane;
     }
     auto z_soff = [&](int bi, int t3) -> uint32_t {
-      return ((m0 / 32u + (uint32_t)(bi >> 1)) * kNkk * 3u + (uint32_t)t3) * kBlockBytes + (uint32_t)(bi & 1) * 256u;
+      uint32_t blk = m0 / 32u + (uint32_t)(bi >> 1);
+      if (MF != 8 && blk >= g.slots / 32u) blk = g.slots / 32u - 1u;
+      return (blk * kNkk * 3u + (uint32_t)t3) * kBlockBytes + (uint32_t)(bi & 1) * 256u;
     };
     auto b_soff = [&](int gi, int bj) -> uint32_t {
       return (((uint32_t)gi * ncb_total + tgrp0 / 32u + (uint32_t)bj) * kNkk) * kBlockBytes + (uint32_t)chalf * 256u;
@@ -457,8 +476,14 @@ void w8a8_gemm16_kernel(GemmArgs g) {
     uint32_t grabbed = 0;  // the position after next of a dynamic schedule, requested with the epilogue's operands
     auto preload = [&]() {
       if (kDyn && tid == 0) grabbed = atomicAdd(ctr, 1u);
-      if (EPI != kEpiAcc) g16_load_128_dwords(g.sx + m0, (uint32_t)lane * 4u, lds_addr + Geo::kRingBytes + wave * 1024);
-      if (g.src_row) g16_load_128_dwords(g.src_row + m0, (uint32_t)lane * 4u, lds_addr + Geo::kRingBytes + wave * 1024 + 512);
+      // (a tile of 192 rows may end behind the tables: their last entry in the place of what they lack)
+      uint32_t s0 = m0 + (uint32_t)lane, s1 = s0 + 64u;
+      if constexpr (MF != 8) {
+        s0 = s0 < g.slots ? s0 : g.slots - 1u;
+        s1 = s1 < g.slots ? s1 : g.slots - 1u;
+      }
+      if (EPI != kEpiAcc) g16_load_128_dwords(g.sx, g.sx - 64, s0 * 4u, s1 * 4u, lds_addr + Geo::kRingBytes + wave * 1024);
+      if (g.src_row) g16_load_128_dwords(g.src_row, g.src_row - 64, s0 * 4u, s1 * 4u, lds_addr + Geo::kRingBytes + wave * 1024 + 512);
       if (!wave_live) return;
       if (EPI != kEpiAcc && full_n) swr = *reinterpret_cast<const v4i*>(T.swp + tcol0 + 4u * c16);
       if constexpr (kLora) {
@@ -490,15 +515,15 @@ void w8a8_gemm16_kernel(GemmArgs g) {
     // consecutive original columns tcol0 + 4 c16 + j held by the accumulator blocks j.
     if (!wave_live) continue;  // wave beyond the last column; it still takes part in the next tile
     if constexpr (kLora) load_z(1, 1);
-    // Does every one of the wave's 128 slots hold a row of the output, and every lane four columns?
+    // Does every one of the wave's 16 MF slots hold a row of the output, and every lane four columns?
     // (wave-uniform; true for all but the tiles at the end of an adapter's rows or of the matrix)
-    bool tile_plain = out_small && full_n && m0 + 128u <= total_rows;
+    bool tile_plain = out_small && full_n && m0 + 16u * MF <= total_rows;
     if (g.src_row) {
       const int2 s2 = *reinterpret_cast<const int2*>(rowdata + 512u + (uint32_t)lane * 8u);
-      const bool both = (uint32_t)s2.x < g.M && (uint32_t)s2.y < g.M;
+      const bool both = ((uint32_t)s2.x < g.M && (uint32_t)s2.y < g.M) || (MF != 8 && lane >= 8 * MF);
       tile_plain = tile_plain && (__builtin_amdgcn_ballot_w64(!both) == 0);
     } else {
-      tile_plain = tile_plain && m0 + 128u <= g.M;
+      tile_plain = tile_plain && m0 + 16u * MF <= g.M;
     }
     const uint32_t ncol = tcol0 + 4u * c16;  // the lane's four consecutive columns
     float sw[4];
@@ -509,7 +534,7 @@ void w8a8_gemm16_kernel(GemmArgs g) {
       for (int j = 0; j < 4; ++j)
         if (ncol + j < g.N) sw[j] = T.swp[ncol + j];
     }
-    g16_for<0, 8>([&](auto BI) {
+    g16_for<0, MF>([&](auto BI) {
       constexpr int bi = decltype(BI)::value;
       const uint32_t pbase = m0 + bi * 16u;  // first slot of the 16-row fragment
       if (pbase >= total_rows) return;       // wave-uniform
@@ -683,7 +708,7 @@ void w8a8_gemm16_kernel(GemmArgs g) {
           else rows(std::integral_constant<int, 2>{});
         }  // groups of the fragment
         // this fragment's z operands are spent: their ring slot takes the fragment two ahead
-        if constexpr (kLora && bi + 2 < 8) load_z(bi & 1, bi + 2);
+        if constexpr (kLora && bi + 2 < MF) load_z(bi & 1, bi + 2);
       }
     });
   }
