@@ -25,8 +25,8 @@ namespace w8a8 {
 //   32 nb + 16 q + 8 (e / 4) + 4 h + e % 4,
 // the n that the transposing MFMA leaves in contraction slot 8 h + e of its q-th half.  Rows are
 // in grouped (adapter-sorted) slot order; slots without a row and columns beyond N are zero.
-// A wave takes a row block and a 128-column group at a time: a lane reads 4 x 16 consecutive
-// original columns of its row and owns the pieces of the eight packed blocks (q, j = column % 4)
+// A wave takes a row block and a 128-column group at a time: a lane owns 4 x 16 consecutive
+// original columns of its row, the pieces of the eight packed blocks (q, j = column % 4)
 // that interleave them.
 // The same pass computes r = dy @ B[group].T on bf16 MFMAs (the 8-value pieces a lane has loaded
 // are A operands as they are; the matching pieces of B are 16-byte loads), so dy is read once:
@@ -48,11 +48,16 @@ struct BwdPackDyArgs {
   uint32_t M, N, NB, n_row_blocks, n_col_groups, n_slices, groups_per_slice, r, slots;
 };
 
+// dy arrives in whole lines, 4 rows x 256 bytes a load and the next group's under this one's work, and changes hands through the
+// LDS, piece p of row r in place p ^ (r % 16), so that neither side has bank conflicts.  Asked for as it is consumed (32 rows x two
+// pieces of 16 bytes a load, each under a condition and so with a wait of its own) it took, us before -> now: 3003 x 24576, rank 32
+// 84.5 -> 67.2 (298 MB); 2048 x 10240, rank 64 24.8 -> 22.2; 333 x 6144, rank 64 12.5 -> 8.2; 8168 x 2048, rank 16 15.0 -> 13.9.
 template <int RB>  // 32-wide rank blocks (0 = packing only)
-__global__ __launch_bounds__(256) void bwd_pack_dy_kernel(BwdPackDyArgs a) {
+__global__ __launch_bounds__(256, 3) void bwd_pack_dy_kernel(BwdPackDyArgs a) {
   constexpr int kRB = RB > 0 ? RB : 1;
-  __shared__ float red[4][kRB][16][64];
-  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[4][8192];  // a tile of 32 rows x 128 columns per wave; later the waves' sums of r
+  static_assert(sizeof(lds) >= 4u * kRB * 16u * 64u * 4u, "");
+  const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t mb = blockIdx.x / a.n_slices, sl = blockIdx.x % a.n_slices;
   if (mb >= a.n_row_blocks) return;
   if (a.blk_range && a.blk_range[mb] < 0) return;  // block without rows (grouped calls): never consumed
@@ -64,67 +69,111 @@ __global__ __launch_bounds__(256) void bwd_pack_dy_kernel(BwdPackDyArgs a) {
   const uint32_t range = (RB > 0 && a.blk_range) ? (uint32_t)a.blk_range[mb] : 0u;
   const uint32_t glo = range & 0xffffu, ghi = range >> 16;
   const uint32_t rowgrp = (RB > 0 && a.slot_group && ghi > glo) ? (uint32_t)a.slot_group[p] : glo;
-  const bool vec = (a.N & 7u) == 0;
   v16f acc[kRB];
 #pragma unroll
   for (int b = 0; b < kRB; ++b)
 #pragma unroll
     for (int e = 0; e < 16; ++e) acc[b][e] = 0.0f;
-  const uint32_t g_end = (sl + 1u) * a.groups_per_slice < a.n_col_groups ? (sl + 1u) * a.groups_per_slice : a.n_col_groups;
-  for (uint32_t G = sl * a.groups_per_slice + wave; G < g_end; G += 4u) {
-    // piece t = 4 q + 2 ch + part: the 8 columns 128 G + 64 q + 32 ch + 16 h + 8 part .. + 7 of the lane's row
-    v8us pc[8];
+  // load u of a group: piece lane % 16 (8 columns) of row 4 u + lane / 16
+  const uint32_t lp = lane & 15u, lr = lane >> 4;
+  uint32_t row_off[8];
+  uint32_t rows_on = 0u;
 #pragma unroll
-    for (int t = 0; t < 8; ++t) {
-      const uint32_t col = 128u * G + 64u * (t >> 2) + 32u * ((t >> 1) & 1) + 16u * h + 8u * (t & 1);
-      if (src >= 0 && vec && col + 8u <= a.N) {
-        pc[t] = *reinterpret_cast<const v8us*>(a.dy + (size_t)src * a.N + col);
-      } else {
+  for (uint32_t u = 0; u < 8; ++u) {
+    const int r = __shfl(src, (int)(4u * u + lr), 64);
+    row_off[u] = r < 0 ? 0u : (uint32_t)r * a.N;
+    rows_on |= r < 0 ? 0u : 1u << u;
+  }
+  auto fetch = [&](uint32_t G, v4i (&d)[8]) {  // (a row or column that is not there: the tensor's first bytes, cleared where they are used)
+    const uint32_t col = 128u * G + 8u * lp < a.N ? 128u * G + 8u * lp : 0u;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) pc[t][e] = (src >= 0 && col + e < a.N) ? a.dy[(size_t)src * a.N + col + e] : (uint16_t)0;
-      }
+    for (uint32_t u = 0; u < 8; ++u) {
+      uint32_t off = row_off[u];
+      asm volatile("" : "+v"(off));  // (eight 64-bit addresses kept across the loop would spill)
+      d[u] = *reinterpret_cast<const v4i*>(a.dy + ((size_t)off + col));
     }
+  };
+  // B of a group: rows of ranks beyond r end behind the resource and read as zeros
+  const uint32_t b_off = (i * a.N + 16u * h) * 2u;
+  typedef __attribute__((address_space(3))) v4i* lds_v4ptr;
+  const uint32_t tile = (uint32_t)(uintptr_t)(lptr_t)lds + wave * 8192u;
+  const uint32_t g_end = (sl + 1u) * a.groups_per_slice < a.n_col_groups ? (sl + 1u) * a.groups_per_slice : a.n_col_groups;
+  v4i d[8];
+  uint32_t G = sl * a.groups_per_slice + wave;
+  if (G < g_end) fetch(G, d);
+#pragma unroll 1
+  for (; G < g_end; G += 4u) {
+    const bool cols_on = 128u * G + 8u * lp < a.N;
 #pragma unroll
-    for (int q = 0; q < 2; ++q)
+    for (uint32_t u = 0; u < 8; ++u) {
+      const v4i zero = {0, 0, 0, 0};
+      *reinterpret_cast<lds_v4ptr>((uintptr_t)(tile + (4u * u + lr) * 256u + (lp ^ ((4u * u + lr) & 15u)) * 16u)) =
+          (rows_on >> u) & 1u && cols_on ? d[u] : zero;
+    }
+    // piece 4 q + t, t = 2 ch + part: the 8 columns 128 G + 64 q + 32 ch + 16 h + 8 part .. + 7 of the lane's row
+    auto piece_of = [&](int q, int t) { return 8u * q + 4u * (t >> 1) + 2u * h + (t & 1); };
+    v8us wb[kRB][4];
+    auto fetch_b = [&](uint32_t grp, int q) {
+      const __amdgpu_buffer_rsrc_t brsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(a.lora_b) + (size_t)grp * a.r * a.N, 0,
+                                                                             (int)(a.r * a.N * 2u), 0x00020000);
+#pragma unroll
+      for (int b = 0; b < RB; ++b)
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+          wb[b][t] = __builtin_bit_cast(v8us, __builtin_amdgcn_raw_buffer_load_b128(brsrc, b_off + (t >> 1) * 64u + (t & 1) * 16u,
+                                                                                    (128u * G + 64u * q + 32u * b * a.N) * 2u, 0));
+      if (128u * G + 128u > a.N) {  // (columns beyond N are another rank's)
+#pragma unroll
+        for (int b = 0; b < RB; ++b)
+#pragma unroll
+          for (int t = 0; t < 4; ++t)
+            if (128u * G + 8u * piece_of(q, t) >= a.N) wb[b][t] = v8us{0, 0, 0, 0, 0, 0, 0, 0};
+      }
+    };
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      if constexpr (RB > 0) fetch_b(glo, q);
+      v8us pc[4];
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+        pc[t] = __builtin_bit_cast(v8us, *reinterpret_cast<lds_v4ptr>((uintptr_t)(tile + i * 256u + (piece_of(q, t) ^ (i & 15u)) * 16u)));
+      __builtin_amdgcn_wave_barrier();
+      if (q == 1 && G + 4u < g_end) fetch(G + 4u, d);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         // element e < 4 of packed block j: column 4 e + j of the first 16, e >= 4: of the second 16
         v8us o;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          o[e] = pc[4 * q + ((4 * e + j) >> 3)][(4 * e + j) & 7];
-          o[4 + e] = pc[4 * q + 2 + ((4 * e + j) >> 3)][(4 * e + j) & 7];
+          o[e] = pc[(4 * e + j) >> 3][(4 * e + j) & 7];
+          o[4 + e] = pc[2 + ((4 * e + j) >> 3)][(4 * e + j) & 7];
         }
         const size_t off = ((((size_t)mb * a.NB + 4u * G + j) * 2u + q) * 64u + lane) * 16u;
         *reinterpret_cast<v8us*>(a.dyp + off) = o;
       }
-    if constexpr (RB > 0) {
-      // a block at a group boundary runs once per group with the other groups' rows zeroed
-      for (uint32_t grp = glo; grp <= ghi; ++grp) {
-        const bool mine = src >= 0 && rowgrp == grp;
-        const uint16_t* bg = a.lora_b + (size_t)grp * a.r * a.N;
-        v8us wb[RB][8];
+      if constexpr (RB > 0) {
+        // a block at a group boundary runs once per group with the other groups' rows zeroed
+#pragma unroll 1
+        for (uint32_t grp = glo;;) {
+          const bool mine = src >= 0 && rowgrp == grp;
 #pragma unroll
-        for (int b = 0; b < RB; ++b)
-#pragma unroll
-          for (int t = 0; t < 8; ++t) {
-            const uint32_t col = 128u * G + 64u * (t >> 2) + 32u * ((t >> 1) & 1) + 16u * h + 8u * (t & 1);
-            const uint32_t j = b * 32u + i;
+          for (int t = 0; t < 4; ++t) {
             const v8us zero = {0, 0, 0, 0, 0, 0, 0, 0};
-            wb[b][t] = (j < a.r && col + 8u <= a.N) ? *reinterpret_cast<const v8us*>(bg + (size_t)j * a.N + col) : zero;
+            const v8bf xa = __builtin_bit_cast(v8bf, mine ? pc[t] : zero);
+#pragma unroll
+            for (int b = 0; b < RB; ++b)
+              acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa, __builtin_bit_cast(v8bf, wb[b][t]), acc[b], 0, 0, 0);
           }
-#pragma unroll
-        for (int t = 0; t < 8; ++t) {
-          const v8us zero = {0, 0, 0, 0, 0, 0, 0, 0};
-          const v8bf xa = __builtin_bit_cast(v8bf, mine ? pc[t] : zero);
-#pragma unroll
-          for (int b = 0; b < RB; ++b)
-            acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa, __builtin_bit_cast(v8bf, wb[b][t]), acc[b], 0, 0, 0);
+          if (++grp > ghi) break;
+          fetch_b(grp, q);
         }
       }
     }
   }
   if constexpr (RB > 0) {
+    float (*const red)[kRB][16][64] = reinterpret_cast<float (*)[kRB][16][64]>(&lds[0][0]);
+    __syncthreads();  // everybody's tiles are spent
 #pragma unroll
     for (int b = 0; b < RB; ++b)
 #pragma unroll
