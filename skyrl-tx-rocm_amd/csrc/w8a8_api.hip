@@ -1297,7 +1297,10 @@ int launch_bwd_body(const BwdBody& b, const Layout& w, unsigned char* ws, hipStr
     d.chunk_tab = b.chunk_tab;
     d.partA = reinterpret_cast<float*>(ws + w.partA);
     d.partB = reinterpret_cast<float*>(ws + w.partB);
-    d.M = b.m; d.K = b.k; d.N = b.n; d.n_groups = b.n_groups; d.max_chunks = w.max_chunks;
+    d.chunk0_tab = b.chunk0;
+    d.d_a = static_cast<uint16_t*>(b.d_lora_a); d.d_b = static_cast<uint16_t*>(b.d_lora_b);
+    d.lora_scaling = b.lora_scaling;
+    d.M = b.m; d.K = b.k; d.N = b.n; d.r = b.rank; d.n_groups = b.n_groups; d.max_chunks = w.max_chunks;
     d.col_tiles_a = b.d_lora_a ? (b.k + 255u) / 256u : 0u;
     d.col_tiles_b = b.d_lora_b ? (b.n + 255u) / 256u : 0u;
     if (d.col_tiles_a + d.col_tiles_b) {
