@@ -217,7 +217,7 @@ typedef struct mi355_w8a8_bwd_problem {
  * beyond sum(group_sizes) are zero.
  */
 typedef struct mi355_w8a8_grouped_bwd_problem {
-  uint32_t struct_size;     /* sizeof(mi355_w8a8_grouped_bwd_problem) */
+  uint32_t struct_size;     /* sizeof(mi355_w8a8_grouped_bwd_problem), or the offset of x_row_map: no map */
   uint32_t flags;           /* 0 */
   uint32_t m;               /* total rows */
   uint32_t k;               /* multiple of 8 */
@@ -239,6 +239,10 @@ typedef struct mi355_w8a8_grouped_bwd_problem {
   float* d_lora_scaling;    /* f32 [n_groups] or NULL */
   void* workspace;          /* >= mi355_w8a8_grouped_bwd_workspace_bytes(...), 256-byte aligned */
   uint64_t workspace_bytes;
+  /* Optional gather of x as in mi355_w8a8_grouped_problem: row i of the call is x[x_row_map[i] / x_row_repeat] */
+  const int32_t* x_row_map; /* int32 [m] or NULL */
+  uint32_t x_row_repeat;    /* >= 1 with a map */
+  uint32_t x_rows;          /* rows of x with a map; 0 = ceil(m / x_row_repeat) */
 } mi355_w8a8_grouped_bwd_problem;
 
 /*

@@ -111,6 +111,7 @@ class GroupedBwdProblem(ctypes.Structure):
         ("x", _vp), ("dy", _vp), ("w_packed", _vp), ("w_scales", _vp), ("lora_a", _vp), ("lora_b", _vp),
         ("lora_scaling", _vp), ("group_sizes", _vp), ("dx", _vp), ("d_lora_a", _vp), ("d_lora_b", _vp),
         ("d_lora_scaling", _vp), ("workspace", _vp), ("workspace_bytes", _u64),
+        ("x_row_map", _vp), ("x_row_repeat", _u32), ("x_rows", _u32),
     ]
 
 

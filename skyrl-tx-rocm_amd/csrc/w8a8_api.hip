@@ -5,6 +5,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <cstddef>
+#include <cstring>
 #include <mutex>
 
 #include "w8a8_device.h"
@@ -1160,6 +1162,7 @@ struct BwdBody {
   // tables (null: identity routing, everything in group 0)
   const int32_t* src_row; const int32_t* slot_group; const int32_t* blk_range; const int32_t* group_off;
   // grouped calls only
+  const int32_t* x_row; uint32_t x_rows;  // src_row and the rows of x where x is gathered, or null
   const int32_t* skip_range;  // blk_range again when blocks without rows are to be skipped
   const int32_t* tile_weight; const int32_t* chunk_tab; const int32_t* chunk0; const int32_t* group_beg;
   const int32_t* group_end;
@@ -1235,8 +1238,8 @@ int launch_bwd_body(const BwdBody& b, const Layout& w, unsigned char* ws, hipStr
       LoraAArgs lz{};
       lz.xsrc = static_cast<const uint16_t*>(b.x);
       lz.at = reinterpret_cast<const uint16_t*>(ws + w.at);
-      lz.src_row = b.src_row; lz.slot_group = b.slot_group; lz.blk_range = b.blk_range;
-      lz.M = b.m; lz.K = b.k; lz.r = b.rank;
+      lz.src_row = b.x_row ? b.x_row : b.src_row; lz.slot_group = b.slot_group; lz.blk_range = b.blk_range;
+      lz.M = b.x_row ? b.x_rows : b.m; lz.K = b.k; lz.r = b.rank;
       lz.n_steps = (b.k + 63u) / 64u;
       lz.n_blocks = w.slots / 32u;
       const uint32_t nks = bwd_z_slices(b.k, w.n_slices);
@@ -1293,6 +1296,7 @@ int launch_bwd_body(const BwdBody& b, const Layout& w, unsigned char* ws, hipStr
     d.rs = reinterpret_cast<const float*>(ws + w.rs);
     d.z = reinterpret_cast<const float*>(ws + w.z);
     d.src_row = b.src_row;
+    d.x_row = b.x_row ? b.x_row : b.src_row;
     d.group_off = b.group_off;
     d.chunk_tab = b.chunk_tab;
     d.partA = reinterpret_cast<float*>(ws + w.partA);
@@ -1494,7 +1498,7 @@ int run_gq_backward(const mi355_w8a8_gq_bwd_problem* p, hipStream_t s) {
 // ---------------------------------------------------------------------------------------
 struct BwdGroupedLayout {
   uint64_t dyp, swp, src_row, slot_group, blk_range, group_beg, group_end, tile_weight, chunk_tab, chunk0,
-      at, ap, rp, z, r_raw, rs, rpart, zpart, row_dot, partA, partB, total;
+      at, ap, rp, z, r_raw, rs, rpart, zpart, row_dot, partA, partB, x_row, total;
   uint32_t slots, nkk, K_pad, KB, N_pad, NB, tiles_m, tiles_k, max_chunks, R, n_slices, groups_per_slice, n_weights,
       gpw, sw_stride, tile_rows;
 };
@@ -1553,6 +1557,7 @@ BwdGroupedLayout make_bwd_grouped_layout(uint32_t m, uint32_t k, uint32_t n, uin
     w.partA = off; off += align256((uint64_t)w.max_chunks * w.R * k * 4u);
     w.partB = off; off += align256((uint64_t)w.max_chunks * w.R * n * 4u);
   }
+  w.x_row = off; off += rank ? align256((uint64_t)w.slots * 4u) : 0u;
   w.total = off;
   return w;
 }
@@ -1571,9 +1576,13 @@ int validate_bwd_grouped_dims(uint32_t m, uint32_t k, uint32_t n, uint32_t n_gro
   return MI355_W8A8_OK;
 }
 
-int run_grouped_backward(const mi355_w8a8_grouped_bwd_problem* p, hipStream_t s) {
-  if (!p) return MI355_W8A8_ERR_NULL;
-  if (p->struct_size != sizeof(mi355_w8a8_grouped_bwd_problem)) return MI355_W8A8_ERR_STRUCT;
+int run_grouped_backward(const mi355_w8a8_grouped_bwd_problem* given, hipStream_t s) {
+  if (!given) return MI355_W8A8_ERR_NULL;
+  constexpr uint32_t kWithoutMap = offsetof(mi355_w8a8_grouped_bwd_problem, x_row_map);
+  if (given->struct_size != sizeof(mi355_w8a8_grouped_bwd_problem) && given->struct_size != kWithoutMap) return MI355_W8A8_ERR_STRUCT;
+  mi355_w8a8_grouped_bwd_problem problem{};
+  memcpy(&problem, given, given->struct_size);
+  const mi355_w8a8_grouped_bwd_problem* const p = &problem;
   if (p->flags) return MI355_W8A8_ERR_SHAPE;
   int st = validate_bwd_grouped_dims(p->m, p->k, p->n, p->n_groups, p->rank, p->groups_per_weight);
   if (st) return st;
@@ -1590,9 +1599,14 @@ int run_grouped_backward(const mi355_w8a8_grouped_bwd_problem* p, hipStream_t s)
       !aligned16(p->lora_a) || !aligned16(p->lora_b) || !aligned16(p->dx) || !aligned16(p->d_lora_a) ||
       !aligned16(p->d_lora_b) || (reinterpret_cast<uintptr_t>(p->group_sizes) & 3u))
     return MI355_W8A8_ERR_ALIGN;
-  const uint64_t dx_bytes = (uint64_t)p->m * p->k * 2u, dy_bytes = (uint64_t)p->m * p->n * 2u;
+  const uint32_t x_repeat = p->x_row_map ? p->x_row_repeat : 1u;
+  if (p->x_row_map && (x_repeat == 0 || (reinterpret_cast<uintptr_t>(p->x_row_map) & 3u))) return MI355_W8A8_ERR_SHAPE;
+  const uint32_t x_rows = (p->x_row_map && p->x_rows) ? p->x_rows : (p->m + x_repeat - 1u) / x_repeat;
+  if ((uint64_t)x_rows * p->k >= (1ull << 32) - (1ull << 20)) return MI355_W8A8_ERR_UNSUPPORTED;
+  const uint64_t dx_bytes = (uint64_t)p->m * p->k * 2u, dy_bytes = (uint64_t)p->m * p->n * 2u, x_bytes = (uint64_t)x_rows * p->k * 2u;
   const uint64_t a_bytes = (uint64_t)p->n_groups * p->rank * p->k * 2u, b_bytes = (uint64_t)p->n_groups * p->rank * p->n * 2u;
-  if (overlaps(p->dx, dx_bytes, p->dy, dy_bytes) || overlaps(p->dx, dx_bytes, p->x, dx_bytes) ||
+  if (overlaps(p->dx, dx_bytes, p->dy, dy_bytes) || overlaps(p->dx, dx_bytes, p->x, x_bytes) ||
+      overlaps(p->dx, dx_bytes, p->x_row_map, (uint64_t)p->m * 4u) ||
       overlaps(p->dx, dx_bytes, p->workspace, p->workspace_bytes) ||
       overlaps(p->d_lora_a, a_bytes, p->lora_a, a_bytes) || overlaps(p->d_lora_b, b_bytes, p->lora_b, b_bytes) ||
       overlaps(p->d_lora_a, a_bytes, p->workspace, p->workspace_bytes) ||
@@ -1600,10 +1614,15 @@ int run_grouped_backward(const mi355_w8a8_grouped_bwd_problem* p, hipStream_t s)
       overlaps(p->d_lora_a, a_bytes, p->dx, dx_bytes) || overlaps(p->d_lora_b, b_bytes, p->dx, dx_bytes))
     return MI355_W8A8_ERR_ALIAS;
   const BwdGroupedLayout w = make_bwd_grouped_layout(p->m, p->k, p->n, p->n_groups, p->rank, p->groups_per_weight);
-  if (!p->workspace || p->workspace_bytes < w.total) return MI355_W8A8_ERR_WORKSPACE;
+  // (the table of gathered rows lies at the end: a call without a map does without it)
+  if (!p->workspace || p->workspace_bytes < (p->x_row_map ? w.total : w.x_row)) return MI355_W8A8_ERR_WORKSPACE;
   if (reinterpret_cast<uintptr_t>(p->workspace) & 255u) return MI355_W8A8_ERR_ALIGN;
   unsigned char* ws = static_cast<unsigned char*>(p->workspace);
   BwdGroupTables tab{};
+  if (p->x_row_map && lora) {
+    tab.x_row = reinterpret_cast<int32_t*>(ws + w.x_row);
+    tab.x_map = p->x_row_map; tab.x_div = x_repeat; tab.x_rows = x_rows;
+  }
   tab.src_row = reinterpret_cast<int32_t*>(ws + w.src_row);
   tab.slot_group = reinterpret_cast<int32_t*>(ws + w.slot_group);
   tab.blk_range = reinterpret_cast<int32_t*>(ws + w.blk_range);
@@ -1641,6 +1660,7 @@ int run_grouped_backward(const mi355_w8a8_grouped_bwd_problem* p, hipStream_t s)
   b.dx = p->dx; b.d_lora_a = p->d_lora_a; b.d_lora_b = p->d_lora_b; b.d_lora_scaling = p->d_lora_scaling;
   b.lora = lora; b.want_grads = want_grads;
   b.src_row = tab.src_row; b.slot_group = tab.slot_group; b.blk_range = tab.blk_range; b.skip_range = tab.blk_range;
+  b.x_row = tab.x_row; b.x_rows = x_rows;
   b.tile_weight = tab.tile_weight; b.chunk_tab = tab.chunk_tab; b.chunk0 = tab.chunk0;
   b.group_beg = tab.group_beg; b.group_end = tab.group_end;
   b.w_stride = (size_t)mi355_w8a8_packed_weight_bytes(p->k, p->n);

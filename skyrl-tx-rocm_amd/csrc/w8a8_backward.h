@@ -376,6 +376,8 @@ __global__ __launch_bounds__(1024) void bwd_prep_kernel(BwdPrepArgs p) {
 struct BwdGroupTables {
   int32_t* src_row; int32_t* slot_group; int32_t* blk_range;
   int32_t* group_beg; int32_t* group_end; int32_t* tile_weight; int32_t* chunk_tab; int32_t* chunk0;
+  // rows of x gathered through a map: x_row[slot] is the row of x that src_row[slot] stands for
+  int32_t* x_row; const int32_t* x_map; uint32_t x_div, x_rows;
 };
 
 __device__ inline void route_weight_groups_block(const int32_t* __restrict__ group_sizes, uint32_t M, uint32_t n_groups,
@@ -448,6 +450,7 @@ __device__ inline void route_weight_groups_block(const int32_t* __restrict__ gro
       }
     }
     t.src_row[p] = src;
+    if (t.x_row) t.x_row[p] = src < 0 ? -1 : (int)mapped_row(t.x_map[src], t.x_div, t.x_rows);
     t.slot_group[p] = grp;
     if ((p & 31u) == 0) t.blk_range[p >> 5] = range;
     if (p % tile_rows == 0) t.tile_weight[p / tile_rows] = tile;  // (a weight's tiles start at its first slot)
@@ -1230,6 +1233,7 @@ struct BwdDloraArgs {
   const float* rs;          // f32 [slots][64]  (dy @ B.T) * s
   const float* z;           // f32 [slots][64]  x @ A
   const int32_t* src_row;   // or null
+  const int32_t* x_row;     // src_row for x
   const int32_t* group_off; // [n_groups + 1]
   const int32_t* chunk_tab; // grouped calls: (group, first slot, rows) per chunk instead of group_off
   const int32_t* chunk0_tab; // grouped calls: first chunk of every group
@@ -1365,7 +1369,8 @@ __global__ __launch_bounds__(256, RB == 1 ? 3 : 1) void bwd_dlora_kernel(BwdDlor
 #pragma unroll
   for (uint32_t i = 0; i < kBwdChunkRows / 256u; ++i) {
     const uint32_t m = i * 256u + tid < rows ? i * 256u + tid : rows - 1u;
-    src[i] = a.src_row ? a.src_row[slot0 + m] : (int)(slot0 + m);
+    const int32_t* const rows_of = job_a ? a.x_row : a.src_row;
+    src[i] = rows_of ? rows_of[slot0 + m] : (int)(slot0 + m);
   }
   float praw[kItems][8];
   load_p(0, praw);

@@ -983,11 +983,13 @@ def grouped_forward(x: torch.Tensor, group_sizes: torch.Tensor, weight: PackedGr
 
 class GroupedBackwardPlan:
     """Validated arguments, outputs, workspace and the C struct of one grouped backward call;
-    ``run()`` is a single C call on torch's current stream.  Nothing is read back to the host."""
+    ``run()`` is a single C call on torch's current stream.  Nothing is read back to the host.  With ``row_map``
+    (int32 [rows]) row i of x is ``x[row_map[i] // row_repeat]``, as in ``GroupedForwardPlan``."""
 
     def __init__(self, x: torch.Tensor | None, dy: torch.Tensor, group_sizes: torch.Tensor,
                  weight: PackedGroupedW8Weight, lora_a=None, lora_b=None, lora_scaling=None, *,
-                 groups_per_weight: int = 1, need_lora_grads: bool = True):
+                 groups_per_weight: int = 1, need_lora_grads: bool = True, row_map: torch.Tensor | None = None,
+                 row_repeat: int = 1):
         if dy.ndim != 2 or dy.dtype != torch.bfloat16:
             raise TypeError("dy must be a BF16 matrix [rows, N]")
         _require_cuda(dy, "dy")
@@ -1019,11 +1021,20 @@ class GroupedBackwardPlan:
             if tuple(s1.shape) != (n_groups,):
                 raise ValueError(f"lora_scaling must be a scalar or have shape ({n_groups},)")
         want = bool(r) and need_lora_grads
+        rmap = None
         if want:
             if x is None:
                 raise ValueError("x is needed for the LoRA cotangents")
-            if x.dtype != torch.bfloat16 or tuple(x.shape) != (m, k):
-                raise ValueError(f"x must be BF16 [{m}, {k}], got {x.dtype} {tuple(x.shape)}")
+            rows = m
+            if row_map is not None:
+                if isinstance(row_repeat, bool) or not isinstance(row_repeat, int) or row_repeat < 1:
+                    raise ValueError(f"row_repeat must be a positive integer, got {row_repeat!r}")
+                rmap = row_map.reshape(-1).to(device=dev, dtype=torch.int32).contiguous()
+                rows = x.shape[0]
+                if rmap.numel() != m or m > rows * row_repeat:
+                    raise ValueError(f"row_map with {rmap.numel()} entries does not fit {m} rows of {rows} x {row_repeat}")
+            if x.dtype != torch.bfloat16 or tuple(x.shape) != (rows, k):
+                raise ValueError(f"x must be BF16 [{rows}, {k}], got {x.dtype} {tuple(x.shape)}")
             _require_cuda(x, "x")
             xf = x.detach().contiguous()
         lib = _native.load()
@@ -1050,12 +1061,14 @@ class GroupedBackwardPlan:
         p.d_lora_b = self.d_lora_b.data_ptr() if want else None
         p.d_lora_scaling = self.d_lora_scaling.data_ptr() if want else None
         p.workspace, p.workspace_bytes = ws.data_ptr(), ws_bytes
+        if rmap is not None:
+            p.x_row_map, p.x_row_repeat, p.x_rows = rmap.data_ptr(), row_repeat, xf.shape[0]
         self.problem = p
         self.device = dev
         self.dims = {"m": m, "k": k, "n": n, "n_groups": n_groups, "rank": r}
         self.group_sizes = gs   # the int32 tensor the call reads: rewrite it in place to route the next run differently
         self._fn = lib.mi355_w8a8_grouped_bwd_v1
-        self._keep = (xf, dyf, gs, weight, a3, b3, s1, ws)
+        self._keep = (xf, dyf, gs, weight, a3, b3, s1, ws, rmap)
 
     def run(self):
         """Enqueue the call; returns ``(dx, d_lora_a, d_lora_b, d_lora_scaling)`` (reused tensors)."""
@@ -1067,13 +1080,15 @@ class GroupedBackwardPlan:
 
 def grouped_backward(x: torch.Tensor | None, dy: torch.Tensor, group_sizes: torch.Tensor,
                      weight: PackedGroupedW8Weight, lora_a=None, lora_b=None, lora_scaling=None, *,
-                     groups_per_weight: int = 1, need_lora_grads: bool = True):
+                     groups_per_weight: int = 1, need_lora_grads: bool = True, row_map: torch.Tensor | None = None,
+                     row_repeat: int = 1):
     """Cotangents of ``grouped_forward`` (plain epilogue): ``(dx, d_lora_a, d_lora_b, d_lora_scaling)``,
     one native call for all groups (the derivative of ``LoRAExpert.__call__``, skyrl/tx/layers/lora.py:
     394-444, under the rule of ``backward``).  Rows beyond ``sum(group_sizes)`` get a zero ``dx``;
     groups without rows get zero cotangents."""
     return GroupedBackwardPlan(x, dy, group_sizes, weight, lora_a, lora_b, lora_scaling,
-                               groups_per_weight=groups_per_weight, need_lora_grads=need_lora_grads).run()
+                               groups_per_weight=groups_per_weight, need_lora_grads=need_lora_grads, row_map=row_map,
+                               row_repeat=row_repeat).run()
 
 
 def grouped_backward_per_weight(x: torch.Tensor | None, dy: torch.Tensor, group_sizes: torch.Tensor,
@@ -1230,10 +1245,13 @@ class _MoeRouteFunction(torch.autograd.Function):
         ctx.save_for_backward(router_logits, selected)
         ctx.norm = norm_topk_prob
         ctx.mark_non_differentiable(selected)
+        ctx.set_materialize_grads(False)  # (else zeros are made for the indices)
         return weights, selected
 
     @staticmethod
     def backward(ctx, d_weights, _d_selected):
+        if d_weights is None:
+            return None, None, None
         router_logits, selected = ctx.saved_tensors
         d_logits = moe_route_backward(router_logits, selected, d_weights.contiguous(), ctx.norm)
         return d_logits.reshape(router_logits.shape).to(router_logits.dtype), None, None
@@ -1387,20 +1405,24 @@ class _MoeExpertMlpFunction(torch.autograd.Function):
     def forward(ctx, hidden, weights, gate_up_a, gate_up_b, down_a, down_b, lora_scaling, selected, gate_up_weight,
                 down_weight, top_k):
         n_experts = gate_up_weight.n_weights
+        factors = None  # one vector of the experts' factors for all four projections' calls
+        if gate_up_a is not None or down_a is not None:
+            factors = _scaling_vector(lora_scaling.detach() if isinstance(lora_scaling, torch.Tensor) else lora_scaling,
+                                      n_experts, hidden.device)
         _, group_sizes, sort_indices, unsort, _ = moe_dispatch(None, selected, n_experts, repeat=top_k)
-        fused = grouped_forward(hidden, group_sizes, gate_up_weight, gate_up_a, gate_up_b, lora_scaling,
+        fused = grouped_forward(hidden, group_sizes, gate_up_weight, gate_up_a, gate_up_b, factors,
                                 row_map=sort_indices, row_repeat=top_k)
         act = swiglu(fused)
-        down = grouped_forward(act, group_sizes, down_weight, down_a, down_b, lora_scaling)
+        down = grouped_forward(act, group_sizes, down_weight, down_a, down_b, factors)
         ctx.save_for_backward(hidden, weights, gate_up_a, gate_up_b, down_a, down_b, lora_scaling, group_sizes,
-                              sort_indices, unsort, fused, act, down)
-        ctx.gate_up_weight, ctx.down_weight, ctx.top_k, ctx.selected = gate_up_weight, down_weight, top_k, selected
+                              sort_indices, unsort, fused, act, down, factors)
+        ctx.gate_up_weight, ctx.down_weight, ctx.top_k = gate_up_weight, down_weight, top_k
         return moe_combine(down, unsort, weights)
 
     @staticmethod
     def backward(ctx, d_out):
         (hidden, weights, gate_up_a, gate_up_b, down_a, down_b, lora_scaling, group_sizes, sort_indices, unsort, fused,
-         act, down) = ctx.saved_tensors
+         act, down, factors) = ctx.saved_tensors
         top_k = ctx.top_k
         lora = gate_up_a is not None
         need_lora = lora and any(ctx.needs_input_grad[2:7])
@@ -1408,13 +1430,12 @@ class _MoeExpertMlpFunction(torch.autograd.Function):
         d_down, d_w = moe_combine_backward(d_out.contiguous(), down if need_w else None, sort_indices, weights,
                                            need_weight_grads=need_w)
         d_act, d_da, d_db, ds_dn = grouped_backward(act, d_down, group_sizes, ctx.down_weight, down_a, down_b,
-                                                    lora_scaling, need_lora_grads=need_lora)
+                                                    factors, need_lora_grads=need_lora)
         d_fused = swiglu_backward(fused, d_act)
-        x_sorted = None
-        if need_lora:  # the LoRA cotangents of gate/up contract over the sorted hidden rows
-            x_sorted = moe_dispatch(hidden, ctx.selected, ctx.gate_up_weight.n_weights, repeat=top_k)[0]
-        d_xs, d_ga, d_gb, ds_gu = grouped_backward(x_sorted, d_fused, group_sizes, ctx.gate_up_weight, gate_up_a,
-                                                   gate_up_b, lora_scaling, need_lora_grads=need_lora)
+        # (the LoRA cotangents of gate/up contract over the sorted hidden rows, read through the sort)
+        d_xs, d_ga, d_gb, ds_gu = grouped_backward(hidden if need_lora else None, d_fused, group_sizes, ctx.gate_up_weight,
+                                                   gate_up_a, gate_up_b, factors, need_lora_grads=need_lora,
+                                                   row_map=sort_indices, row_repeat=top_k)
         d_hidden = None
         if ctx.needs_input_grad[0]:
             d_hidden = moe_combine(d_xs, unsort, torch.ones_like(weights))
@@ -1513,7 +1534,7 @@ def moe_expert_mlp(hidden, router_logits, top_k: int, gate_up_weight, down_weigh
         return plan.run(h2, selected, weights).reshape(hidden.shape)
     scaling = lora_scaling
     if gate_up_a is not None and not isinstance(scaling, torch.Tensor):
-        scaling = _scaling_scalar(scaling, hidden.device)
+        scaling = _scaling_vector(scaling, n_experts, hidden.device)
     out = _MoeExpertMlpFunction.apply(h2, weights, gate_up_a, gate_up_b, down_a, down_b, scaling, selected,
                                       gate_up_weight, down_weight, top_k)
     return out.reshape(hidden.shape)
