@@ -540,13 +540,13 @@ class _LoraLinearFunction(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, lora_a, lora_b, lora_scaling, weight, adapter_indices, residual):
-        out = forward(x, weight, lora_a, lora_b, lora_scaling, adapter_indices=adapter_indices,
-                      residual=residual, entry="linear" if residual is None else "residual")
+        plan = ForwardPlan(x, weight, lora_a, lora_b, lora_scaling, adapter_indices=adapter_indices,
+                           residual=residual, entry="linear" if residual is None else "residual", keep_lora_pack=False)
         ctx.save_for_backward(x, lora_a, lora_b, lora_scaling)
         ctx.weight = weight
-        ctx.adapter_indices = adapter_indices
+        ctx.adapter_indices = plan.adapter_indices  # (one per row: expanded once for both directions)
         ctx.has_residual = residual is not None
-        return out
+        return plan.run()
 
     @staticmethod
     def backward(ctx, dy):
@@ -746,6 +746,7 @@ class _RmsGateUpFunction(torch.autograd.Function):
                                rms_gamma=gamma, eps=eps, want_normalized=True,
                                flags=0 if rows <= SKINNY_MAX_ROWS else _native.FLAG_FORCE_TILED)
             fused = plan.run()
+            ctx.adapter_indices = plan.adapter_indices  # (one per row: expanded once for both directions)
             ctx.save_for_backward(x, lora_a, lora_b, lora_scaling, gamma, fused, plan.aux["normalized"])
             return swiglu(fused)
         ctx.save_for_backward(x, lora_a, lora_b, lora_scaling, gamma)
@@ -759,12 +760,9 @@ class _RmsGateUpFunction(torch.autograd.Function):
         if ctx.saved_projection:
             fused, normalized = ctx.saved_tensors[5:]
             d_fused = swiglu_backward(fused, d_product.contiguous().reshape(*fused.shape[:-1], -1))
-            idx = ctx.adapter_indices
             rows = normalized.shape[0]
-            if idx is not None and idx.numel() != rows:
-                idx = idx.reshape(-1).repeat_interleave(rows // idx.numel())
             dn, da, db, ds = backward(normalized, d_fused.reshape(rows, -1), ctx.weight, lora_a, lora_b, lora_scaling,
-                                      adapter_indices=idx, need_lora_grads=need)
+                                      adapter_indices=ctx.adapter_indices, need_lora_grads=need)
             dx = rms_norm_backward(x.reshape(rows, -1), gamma, dn, eps=ctx.eps, in_place=True).reshape(x.shape)
         else:
             dx, da, db, ds = rms_gate_up_swiglu_backward(x, gamma, ctx.weight, lora_a, lora_b, lora_scaling,
@@ -1913,25 +1911,27 @@ class _QkvStageFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, hidden, input_norm_weight, q_norm_weight, k_norm_weight, lora_a, lora_b, lora_scaling, weight,
                 positions, config, adapter_indices, save_projection):
-        ctx.weight, ctx.config, ctx.adapter_indices = weight, config, adapter_indices
+        ctx.weight, ctx.config = weight, config
         ctx.saved_projection = bool(save_projection)
-        gamma = 1.0 + input_norm_weight.detach().to(torch.float32)
+        gamma = _one_plus(input_norm_weight)
         plan = ForwardPlan(hidden, weight, lora_a, lora_b, lora_scaling, adapter_indices=adapter_indices,
                            rms_gamma=gamma, eps=config.rms_norm_eps, want_normalized=ctx.saved_projection)
         fused = plan.run()
+        ctx.adapter_indices = plan.adapter_indices  # (one per row; like the float32 norm weights made once for both directions)
         keep = (fused, plan.aux["normalized"]) if ctx.saved_projection else ()
-        ctx.save_for_backward(hidden, input_norm_weight, q_norm_weight, k_norm_weight, lora_a, lora_b, lora_scaling,
-                              positions, *keep)
-        q, k, v, gate = qkv_split_norm_rope(fused, q_norm_weight, k_norm_weight, positions, config)
+        q_w, k_w = (w.detach().to(device=hidden.device, dtype=torch.float32) for w in (q_norm_weight, k_norm_weight))
+        # (the weights themselves are saved too: written between the two directions they are refused)
+        ctx.save_for_backward(hidden, input_norm_weight, q_norm_weight, k_norm_weight, plan.gamma, q_w, k_w, lora_a, lora_b,
+                              lora_scaling, positions, *keep)
+        q, k, v, gate = qkv_split_norm_rope(fused, q_w, k_w, positions, config)
         return q, k, v, gate
 
     @staticmethod
     def backward(ctx, d_q, d_k, d_v, d_gate):
-        hidden, in_w, q_w, k_w, lora_a, lora_b, lora_scaling, positions = ctx.saved_tensors[:8]
+        hidden, in_w, q_norm, k_norm, gamma, q_w, k_w, lora_a, lora_b, lora_scaling, positions = ctx.saved_tensors[:11]
         config = ctx.config
-        gamma = 1.0 + in_w.detach().to(torch.float32)
         if ctx.saved_projection:
-            fused, normalized = ctx.saved_tensors[8:]
+            fused, normalized = ctx.saved_tensors[11:]
         else:
             plan = ForwardPlan(hidden, ctx.weight, lora_a, lora_b, lora_scaling, adapter_indices=ctx.adapter_indices,
                                rms_gamma=gamma, eps=config.rms_norm_eps, want_normalized=True)
@@ -1943,11 +1943,8 @@ class _QkvStageFunction(torch.autograd.Function):
         d_fused, dqw, dkw = qkv_split_norm_rope_backward(fused, q_w, k_w, positions, config, d_q, d_k, d_v, d_gate,
                                                          need_norm_weight_grads=need_head)
         rows = normalized.shape[0]
-        idx = ctx.adapter_indices
-        if idx is not None and idx.numel() != rows:
-            idx = idx.reshape(-1).repeat_interleave(rows // idx.numel())
         dn, da, db, ds = backward(normalized, d_fused.reshape(rows, -1), ctx.weight, lora_a, lora_b, lora_scaling,
-                                  adapter_indices=idx, need_lora_grads=need_lora)
+                                  adapter_indices=ctx.adapter_indices, need_lora_grads=need_lora)
         dh, dinw = delta_rms_norm_backward(hidden.reshape(rows, -1), gamma, dn, eps=config.rms_norm_eps,
                                            need_weight_grad=need_in, in_place=not need_in)
         if need_lora:
@@ -1957,9 +1954,17 @@ class _QkvStageFunction(torch.autograd.Function):
         else:
             da = db = ds = None
         dinw = dinw.to(in_w.dtype) if need_in else None
-        dqw = dqw.to(q_w.dtype) if ctx.needs_input_grad[2] else None
-        dkw = dkw.to(k_w.dtype) if ctx.needs_input_grad[3] else None
+        dqw = dqw.to(q_norm.dtype) if ctx.needs_input_grad[2] else None
+        dkw = dkw.to(k_norm.dtype) if ctx.needs_input_grad[3] else None
         return dh.reshape(hidden.shape), dinw, dqw, dkw, da, db, ds, None, None, None, None, None
+
+
+def _one_plus(weight: torch.Tensor) -> torch.Tensor:
+    """float32 ``1 + weight`` of a norm weight in delta form, in one launch where torch promotes to float32 by itself."""
+    w = weight.detach()
+    if w.is_cuda and w.ndim == 1 and w.dtype in (torch.bfloat16, torch.float16, torch.float32):
+        return _constant_scaling(1.0, 1, str(w.device)) + w
+    return 1.0 + w.to(torch.float32)
 
 
 def qkv_lora_rope(hidden, input_norm_weight, q_norm_weight, k_norm_weight, weight, lora_a, lora_b, lora_scaling,
@@ -1970,7 +1975,7 @@ def qkv_lora_rope(hidden, input_norm_weight, q_norm_weight, k_norm_weight, weigh
     tensors = [t for t in (hidden, input_norm_weight, q_norm_weight, k_norm_weight, lora_a, lora_b, lora_scaling)
                if isinstance(t, torch.Tensor)]
     if not (torch.is_grad_enabled() and any(t.requires_grad for t in tensors)):
-        gamma = 1.0 + input_norm_weight.to(torch.float32)
+        gamma = _one_plus(input_norm_weight)
         fused = forward(hidden, weight, lora_a, lora_b, lora_scaling, adapter_indices=adapter_indices,
                         rms_gamma=gamma, eps=config.rms_norm_eps)
         return qkv_split_norm_rope(fused, q_norm_weight, k_norm_weight, positions, config)
