@@ -1476,45 +1476,75 @@ __global__ __launch_bounds__(256, RB == 1 ? 3 : 1) void bwd_dlora_kernel(BwdDlor
       load_q(b0 + u + kRing, u);  // behind the last block: its lines again
     }
   }
-  if (!active) return;
-  // lane (c, h) holds column col0 + 32 st + c, rank rows 32 b + 8 (v / 4) + 4 h + v % 4.  A group of one chunk is done here: its
-  // sums with the second kernel's operations (added to zero, dB scaled, cast).  128 experts of 64 rows, rank 16, 2048 -> 1536 and 768 -> 2048: this
-  // kernel 26.5 + 22.9 -> 25.9 + 21.8 us, the second 10.4 + 9.0 -> 5.0 + 4.7.
-  const float sc = only && !job_a ? a.lora_scaling[group] : 1.0f;
+  // lane (c, h) holds column col0 + 32 st + c, rank rows 32 b + 8 (v / 4) + 4 h + v % 4
+  if (!only) {  // workgroup-uniform
+    if (!active) return;
 #pragma unroll
-  for (int st = 0; st < 2; ++st) {
-    const uint32_t col = col0 + 32u * st + c;
-    if (col >= C) continue;
+    for (int st = 0; st < 2; ++st) {
+      const uint32_t col = col0 + 32u * st + c;
+      if (col >= C) continue;
 #pragma unroll
-    for (int b = 0; b < RB; ++b)
+      for (int b = 0; b < RB; ++b)
 #pragma unroll
-      for (int v4 = 0; v4 < 4; ++v4) {
-        const uint32_t j = b * 32u + 8u * v4 + 4u * h;  // four consecutive rank rows
-        float y[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) y[e] = acc[st][b][4 * v4 + e];
-        if (!only) {  // workgroup-uniform
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (j + e < a.r) part[((size_t)cid * (RB * 32u) + j + e) * C + col] = y[e];
-        } else if (job_a) {
-          uint16_t* const o = a.d_a + ((size_t)group * a.K + col) * a.r + j;
-          const uint32_t lo = pack_bf16x2(0.0f + y[0], 0.0f + y[1]), hi = pack_bf16x2(0.0f + y[2], 0.0f + y[3]);
-          if ((a.r & 3u) == 0) {
-            if (j < a.r) *reinterpret_cast<uint2*>(o) = make_uint2(lo, hi);
-          } else {
-            if (j < a.r) o[0] = (uint16_t)lo;
-            if (j + 1u < a.r) o[1] = (uint16_t)(lo >> 16);
-            if (j + 2u < a.r) o[2] = (uint16_t)hi;
-            if (j + 3u < a.r) o[3] = (uint16_t)(hi >> 16);
-          }
-        } else {
-          uint16_t* const o = a.d_b + ((size_t)group * a.r + j) * a.N + col;
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (j + e < a.r) o[(size_t)e * a.N] = (uint16_t)f32_to_bf16_bits((0.0f + y[e]) * sc);
+        for (int v = 0; v < 16; ++v) {
+          if (b * 32u + 8u * (v >> 2) >= a.r) continue;  // (uniform; rank rows beyond r are not read)
+          const uint32_t j = b * 32u + 8u * (v >> 2) + 4u * h + (v & 3);
+          part[((size_t)cid * (RB * 32u) + j) * C + col] = acc[st][b][v];
         }
-      }
+    }
+    return;
+  }
+  // A group of one chunk is done here, its sums with the second kernel's operations (added to zero, dB scaled, cast).  The values change
+  // hands in the LDS (P is spent): dA's lie r to a column there, so that a wave's 64 columns are one piece of memory, dB's 64
+  // columns to a rank row.  Both kernels, us, before -> now: 128 experts of 64 rows, rank 16, 2048 -> 1536 and 768 -> 2048 68.8 -> 53.7; 2048 rows of
+  // rank 64, 512 to an adapter, 2560 + 10240 columns 35.1 -> 33.0 (straight from the registers 38.6).
+  lds_barrier();
+  if (!active) return;
+  typedef __attribute__((address_space(3))) unsigned char* lds_ptr;
+  typedef __attribute__((address_space(3))) const v4i* lds_v4ptr;
+  typedef uint32_t v2u __attribute__((ext_vector_type(2)));
+  const uint32_t cols = C - col0 < 64u ? C - col0 : 64u;
+  if (job_a) {
+    constexpr uint32_t kStride = RB * 64u + 16u;  // bytes of a column
+    static_assert(4u * 64u * kStride <= (kBwdStageRows / 32u) * RB * 6u * (uint32_t)kBlockBytes, "P's place");
+    const lds_ptr turn = (lds_ptr)(lptr_t)pop + wave * (64u * kStride);
+#pragma unroll
+    for (int st = 0; st < 2; ++st)
+#pragma unroll
+      for (int b = 0; b < RB; ++b)
+#pragma unroll
+        for (int v = 0; v < 16; v += 4)
+          *reinterpret_cast<__attribute__((address_space(3))) v2u*>(turn + (32u * st + c) * kStride + (b * 32u + 2u * v + 4u * h) * 2u) =
+              v2u{pack_bf16x2(0.0f + acc[st][b][v], 0.0f + acc[st][b][v + 1]), pack_bf16x2(0.0f + acc[st][b][v + 2], 0.0f + acc[st][b][v + 3])};
+    __builtin_amdgcn_wave_barrier();  // (a wave reads what it has written itself)
+    uint16_t* const o = a.d_a + ((size_t)group * a.K + col0) * a.r;
+    if ((a.r & 7u) == 0) {
+      const uint32_t pieces = a.r / 8u;
+      for (uint32_t e = lane; e < cols * pieces; e += 64u)
+        *reinterpret_cast<v4i*>(o + e * 8u) = *reinterpret_cast<lds_v4ptr>(turn + (e / pieces) * kStride + (e % pieces) * 16u);
+    } else {
+      for (uint32_t e = lane; e < cols * a.r; e += 64u)
+        o[e] = *reinterpret_cast<__attribute__((address_space(3))) const uint16_t*>(turn + (e / a.r) * kStride + (e % a.r) * 2u);
+    }
+  } else {
+    constexpr uint32_t kStride = 144u;  // bytes of a rank row
+    static_assert(4u * RB * 32u * kStride <= (kBwdStageRows / 32u) * RB * 6u * (uint32_t)kBlockBytes, "P's place");
+    const lds_ptr turn = (lds_ptr)(lptr_t)pop + wave * (RB * 32u * kStride);
+    const float sc = a.lora_scaling[group];
+#pragma unroll
+    for (int st = 0; st < 2; ++st)
+#pragma unroll
+      for (int b = 0; b < RB; ++b)
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+          *reinterpret_cast<__attribute__((address_space(3))) uint16_t*>(turn + (b * 32u + 8u * (v >> 2) + 4u * h + (v & 3)) * kStride + (32u * st + c) * 2u) =
+              (uint16_t)f32_to_bf16_bits((0.0f + acc[st][b][v]) * sc);
+    __builtin_amdgcn_wave_barrier();
+    uint16_t* const o = a.d_b + (size_t)group * a.r * a.N + col0;
+    const uint32_t cl = (lane & 7u) * 8u;  // (N is a multiple of 8)
+    if (cl < cols)
+      for (uint32_t j = lane >> 3; j < a.r; j += 8u)
+        *reinterpret_cast<v4i*>(o + (size_t)j * a.N + cl) = *reinterpret_cast<lds_v4ptr>(turn + j * kStride + cl * 2u);
   }
 }
 
