@@ -7,10 +7,13 @@ the library is missing, or a launch is refused, the caller gets an exception.
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import threading
 from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().parent / "lib" / "libmi355_w8a8.so"
+HOST_PATH = LIB_PATH.with_name("mi355_w8a8_host.so")
 
 ABI_VERSION = 1
 FLAG_SWIGLU = 1
@@ -290,6 +293,31 @@ def load() -> ctypes.CDLL:
                 raise RuntimeError("libmi355_w8a8.so ABI version mismatch")
             _lib = lib
         return _lib
+
+
+_host = None
+entry_address: dict = {}  # of the entry points that the host module calls
+
+
+def host():
+    """Load (once) and return the module with the host side of a forward call; raises if it was not built."""
+    global _host
+    if _host is not None:
+        return _host
+    lib = load()
+    with _lock:
+        if _host is None:
+            if not HOST_PATH.exists():
+                raise RuntimeError(f"{HOST_PATH} is missing: build it with skyrl-tx-rocm_amd/build.py")
+            loader = importlib.machinery.ExtensionFileLoader("mi355_w8a8_host", str(HOST_PATH))
+            module = importlib.util.module_from_spec(importlib.util.spec_from_loader("mi355_w8a8_host", loader))
+            loader.exec_module(module)
+            for name, fn in (("forward", "forward_v1"), ("linear", "lora_linear_v1"), ("gateup", "rms_gateup_swiglu_v1"),
+                             ("residual", "lora_residual_v1"), ("workspace_bytes", "workspace_bytes"),
+                             ("gq_linear", "gq_linear_v1"), ("gq_workspace_bytes", "gq_workspace_bytes")):
+                entry_address[name] = ctypes.cast(getattr(lib, f"mi355_w8a8_{fn}"), ctypes.c_void_p).value
+            _host = module
+        return _host
 
 
 def check(fn: str, status: int) -> None:

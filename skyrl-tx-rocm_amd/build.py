@@ -1,6 +1,7 @@
 """Builds the gfx950 shared library of the W8A8 LoRA linear path with hipcc.
 
-``python build.py`` compiles ``csrc/w8a8_api.hip`` into ``lib/libmi355_w8a8.so``.
+``python build.py`` compiles ``csrc/w8a8_api.hip`` into ``lib/libmi355_w8a8.so`` and, with g++,
+``csrc/w8a8_host_call.cc`` into the Python module ``lib/mi355_w8a8_host.so``.
 hipcc cross-compiles without a GPU.  Flags: ``-ffp-contract=off -fno-fast-math`` keep
 the quantizer and the float32 epilogue bit-exact (no fused multiply-add, IEEE
 division and square root); packed FP32 instructions are disabled.
@@ -18,6 +19,7 @@ HERE = Path(__file__).resolve().parent
 CSRC = HERE / "csrc"
 LIB_DIR = HERE / "lib"
 LIB_PATH = LIB_DIR / "libmi355_w8a8.so"
+HOST_PATH = LIB_DIR / "mi355_w8a8_host.so"
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",
@@ -69,6 +71,29 @@ def build_ffi(verbose: bool = False) -> Path | None:
     return out
 
 
+def build_host(verbose: bool = False) -> Path:
+    """The host side of a forward call on torch tensors (no GPU code), against the installed torch."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    tmp = LIB_DIR / "mi355_w8a8_host.so.tmp"
+    lib_dir = Path(torch.__file__).resolve().parent / "lib"
+    include = [f"-I{p}" for p in cpp_extension.include_paths()]
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}", *include,
+           f"-I{sysconfig.get_paths()['include']}", str(CSRC / "w8a8_host_call.cc"), f"-L{lib_dir}", "-lc10", "-ltorch_cpu",
+           "-ltorch_python", "-o", str(tmp)]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"g++ failed on the host module ({proc.returncode}):\n{proc.stderr}")
+    if verbose and proc.stderr.strip():
+        print(proc.stderr, file=sys.stderr)
+    os.replace(tmp, HOST_PATH)
+    return HOST_PATH
+
+
 def build(verbose: bool = False) -> Path:
     LIB_DIR.mkdir(parents=True, exist_ok=True)
     tmp = LIB_DIR / "libmi355_w8a8.so.tmp"
@@ -81,6 +106,7 @@ def build(verbose: bool = False) -> Path:
     if verbose and err.strip():
         print(err, file=sys.stderr)
     os.replace(tmp, LIB_PATH)
+    build_host(verbose)
     build_ffi(verbose)
     return LIB_PATH
 

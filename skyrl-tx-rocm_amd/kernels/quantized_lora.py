@@ -204,22 +204,33 @@ class _GroupScaledLoraFunction(torch.autograd.Function):
         return dx, da, db, ds, None, None
 
 
-def quantized_frozen_linear(x: torch.Tensor, weight: GroupQuantizedWeight, *, activation_bits: int = 8):
-    from .rocm import gq_linear, w8a8_lora
+_rocm_modules = None
 
+
+def _rocm():
+    """``(gq_linear, w8a8_lora)``, which import this module (an import statement at every call takes a microsecond)."""
+    global _rocm_modules
+    if _rocm_modules is None:
+        from .rocm import gq_linear, w8a8_lora
+
+        _rocm_modules = (gq_linear, w8a8_lora)
+    return _rocm_modules
+
+
+def quantized_frozen_linear(x: torch.Tensor, weight: GroupQuantizedWeight, *, activation_bits: int = 8):
+    gq_linear, w8a8_lora = _rocm()
     per_channel = _is_per_channel_w8a8(weight, activation_bits)
     if not x.dtype.is_floating_point:
         raise TypeError(f"activations must be floating point, got {x.dtype}")
     if per_channel:
         return w8a8_lora.w8a8_frozen_linear(x, weight, enabled=True)
-    return gq_linear.forward(x, weight, activation_bits=activation_bits)
+    return gq_linear._forward(x, weight, gq_linear._pack_valid, None, None, None, activation_bits)
 
 
 def quantized_lora_linear(x: torch.Tensor, weight: GroupQuantizedWeight, lora_a: torch.Tensor,
                           lora_b: torch.Tensor, lora_scaling, *, activation_bits: int = 8) -> torch.Tensor:
     """Frozen W8A8 linear plus LoRA: bf16(base_f32 + ((x @ A) @ B) * s), one cast."""
-    from .rocm import gq_linear, w8a8_lora
-
+    gq_linear, w8a8_lora = _rocm()
     per_channel = _is_per_channel_w8a8(weight, activation_bits)
     if x.ndim < 1:
         raise ValueError(f"activations must have at least one dimension, got {tuple(x.shape)}")
@@ -249,4 +260,4 @@ def quantized_lora_linear(x: torch.Tensor, weight: GroupQuantizedWeight, lora_a:
         else:
             s_arg = lora_scaling if isinstance(lora_scaling, torch.Tensor) and lora_scaling.requires_grad else scaling
         return _GroupScaledLoraFunction.apply(x, lora_a, lora_b, s_arg, weight, activation_bits)
-    return gq_linear.forward(x, weight, lora_a, lora_b, scaling, activation_bits=activation_bits)
+    return gq_linear._forward(x, weight, gq_linear._pack_valid, lora_a, lora_b, scaling, activation_bits)

@@ -49,6 +49,11 @@ def prepare_group_weight(weight) -> PackedGroupWeight:
     if isinstance(weight, PackedGroupWeight):
         return weight
     ql.validate_quantized_weight(weight)
+    return _pack_valid(weight)
+
+
+def _pack_valid(weight) -> PackedGroupWeight:
+    """``prepare_group_weight`` of a weight that the caller has just validated."""
     codes = weight.codes
     _require_cuda(codes, "weight codes")
     key = (codes.data_ptr(), weight.scales.data_ptr(), weight.padded_in_features, codes.shape[1], weight.bits,
@@ -98,16 +103,33 @@ def forward(x: torch.Tensor, weight, lora_a=None, lora_b=None, lora_scaling=None
     quantized_lora.py:215-254.  ``lora_a`` / ``lora_b`` are [K, r] / [r, N] with a scalar scaling, or
     stacked [n, K, r] / [n, r, N] with ``lora_scaling`` [n] and one adapter index per row.
     ``flags``: 0, or ``_native.FLAG_GQ_DIRECT`` for the kernel without LDS staging (same bits)."""
+    return _forward(x, weight, prepare_group_weight, lora_a, lora_b, lora_scaling, activation_bits, adapter_indices, return_aux,
+                    flags)
+
+
+def _forward(x, weight, pack, lora_a, lora_b, lora_scaling, activation_bits, adapter_indices=None, return_aux=False, flags=0):
     if activation_bits not in (4, 8):
         raise ValueError(f"bits must be 4 or 8, got {activation_bits}")
     if x.dtype != torch.bfloat16:
         raise TypeError(f"x must be BF16, got {x.dtype}")
     _require_cuda(x, "x")
-    pw = prepare_group_weight(weight)
+    pw = pack(weight)
     k, n = pw.in_features, pw.out_features
     if x.ndim < 1 or x.shape[-1] != k or x.numel() == 0:
         raise ValueError(f"activation K={x.shape[-1] if x.ndim else None} does not match weight K={k}")
     dev = x.device
+    if not (return_aux or flags or adapter_indices is not None or pw.source_group_size):
+        # an ordinary call goes through the host module; for any other it returns None
+        scaling = lora_scaling
+        if lora_a is not None and isinstance(scaling, (int, float)) and lora_a.ndim in (2, 3):
+            scaling = _scaling_vector(scaling, lora_a.shape[0] if lora_a.ndim == 3 else 1, dev)
+        result = _native.host().group_scaled(
+            x, pw.packed, pw.scales, k, pw.padded_in_features, n, pw.group_size, pw.bits, activation_bits, lora_a, lora_b,
+            scaling, _native.entry_address["gq_linear"], _native.entry_address["gq_workspace_bytes"], _stream_ptr(dev))
+        if type(result) is int:
+            _native.check("mi355_w8a8_gq_linear_v1", result)
+        elif result is not None:
+            return result
     flat = x.reshape(-1, k).contiguous()
     m = flat.shape[0]
 
