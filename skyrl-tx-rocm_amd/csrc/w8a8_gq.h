@@ -329,9 +329,7 @@ __global__ __launch_bounds__(256) void gq_lora_z_kernel(GqLoraZArgs a) {
   }
 #pragma unroll
   for (uint32_t j = 0; j < RB * 8u; ++j) {
-    float v = acc[j];
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
+    const float v = wave_sum(acc[j]);
     if (lane == 0 && j < a.r) zout[j] = v;
   }
 }
@@ -572,12 +570,7 @@ __device__ inline void gq_store_row_block(const GqGemmArgs& a, const float (&out
       }
       int done_below = -1;
       for (;;) {  // adapters present among the block's rows, smallest first (wave-uniform)
-        int cand = my_ad > done_below ? my_ad : 0x7fffffff;
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) {
-          const int o = __shfl_xor(cand, off);
-          cand = o < cand ? o : cand;
-        }
+        const int cand = __builtin_amdgcn_readfirstlane(wave_min(my_ad > done_below ? my_ad : 0x7fffffff));
         if (cand == 0x7fffffff) break;
         done_below = cand;
         const bool mine = my_ad == cand;

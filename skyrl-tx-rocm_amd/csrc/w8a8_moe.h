@@ -56,8 +56,7 @@ __global__ __launch_bounds__(256) void moe_route_kernel(MoeRouteArgs a) {
     v[j] = e < a.E ? expf(v[j] - mx) : 0.0f;
     sum += v[j];
   }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
+  sum = wave_sum(sum);
 #pragma unroll
   for (uint32_t j = 0; j < NV; ++j) {
     const uint32_t e = j * 64u + lane;
@@ -71,12 +70,9 @@ __global__ __launch_bounds__(256) void moe_route_kernel(MoeRouteArgs a) {
 #pragma unroll
     for (uint32_t j = 0; j < NV; ++j)
       if (v[j] > best) { best = v[j]; bi = (int)(j * 64u + lane); }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-      const float ob = __shfl_xor(best, off);
-      const int oi = __shfl_xor(bi, off);
-      if (ob > best || (ob == best && oi < bi)) { best = ob; bi = oi; }
-    }
+    const float top = wave_max(best);
+    bi = __builtin_amdgcn_readfirstlane(wave_min(best == top ? bi : 0x7fffffff));  // of equal ones the lowest
+    best = top;
     if (lane == ((uint32_t)bi & 63u)) {
 #pragma unroll
       for (uint32_t j = 0; j < NV; ++j)
@@ -87,7 +83,7 @@ __global__ __launch_bounds__(256) void moe_route_kernel(MoeRouteArgs a) {
   if (a.norm) {
     float s = 0.0f;
     for (uint32_t j = 0; j < a.top_k; ++j) {
-      const float wj = __shfl(my_w, (int)j);
+      const float wj = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(my_w), j));
       s = j == 0 ? wj : s + wj;
     }
     my_w = my_w / s;
@@ -133,8 +129,7 @@ __global__ __launch_bounds__(256) void moe_route_bwd_kernel(MoeRouteBwdArgs a) {
     v[j] = e < a.E ? expf(v[j] - mx) : 0.0f;
     sum += v[j];
   }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
+  sum = wave_sum(sum);
 #pragma unroll
   for (uint32_t j = 0; j < NV; ++j) {
     const uint32_t e = j * 64u + lane;
@@ -152,16 +147,13 @@ __global__ __launch_bounds__(256) void moe_route_bwd_kernel(MoeRouteBwdArgs a) {
   float dps = dw;
   if (a.norm) {
     float tot = ps, dot = 0.0f;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) tot += __shfl_xor(tot, off);
+    tot = wave_sum(tot);
     dot = dw * (ps / tot);
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) dot += __shfl_xor(dot, off);
+    dot = wave_sum(dot);
     dps = (dw - dot) / tot;
   }
   float s = own ? ps * dps : 0.0f;
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
+  s = wave_sum(s);
   __builtin_amdgcn_wave_barrier();  // every lane has read its probability
 #pragma unroll
   for (uint32_t j = 0; j < NV; ++j) {
@@ -430,8 +422,7 @@ __global__ __launch_bounds__(256) void moe_combine_bwd_kernel(MoeCombineBwdArgs 
           make_uint4(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]), pack_bf16x2(o[4], o[5]), pack_bf16x2(o[6], o[7]));
     }
     if (a.d_weights) {
-#pragma unroll
-      for (int off = 32; off > 0; off >>= 1) dot += __shfl_xor(dot, off);
+      dot = wave_sum(dot);
       if (lane == 0) a.d_weights[pair] = dot;
     }
   }

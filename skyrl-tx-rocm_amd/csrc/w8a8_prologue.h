@@ -581,11 +581,7 @@ __device__ inline uint4 rms_normalize8(const uint4& raw, float inv, const float4
 // The scale of a row from its wave's running maxima.
 __device__ inline float row_scale_of(uint32_t amax_bits) {
   uint32_t top = (amax_bits >> 16) > (amax_bits & 0xffffu) ? (amax_bits >> 16) : (amax_bits & 0xffffu);
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    const uint32_t other = (uint32_t)__shfl_xor((int)top, o, 64);
-    top = other > top ? other : top;
-  }
+  top = wave_fold(top, [](uint32_t a, uint32_t b) { return a > b ? a : b; });
   const float amax = __uint_as_float(top << 16);
   return amax > 0.0f ? amax / 127.0f : 1.0f;
 }

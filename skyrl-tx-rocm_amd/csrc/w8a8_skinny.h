@@ -200,9 +200,15 @@ __device__ inline void skinny_lora_a_unit(const uint16_t* __restrict__ xsrc, con
       }
     }
   }
-  for (uint32_t off = rch2; off < 64u; off <<= 1) {
+  const auto add = [](float x, float y) { return x + y; };
 #pragma unroll
-    for (int e = 0; e < 8; ++e) accz[e] += __shfl_xor(accz[e], (int)off, 64);
+  for (int e = 0; e < 8; ++e) {  // the steps rch2, 2 rch2, .., 32
+    if (rch2 < 2u) accz[e] = lane_step<1>(accz[e], add);
+    if (rch2 < 4u) accz[e] = lane_step<2>(accz[e], add);
+    if (rch2 < 8u) accz[e] = lane_step<4>(accz[e], add);
+    accz[e] = lane_step<8>(accz[e], add);
+    accz[e] = lane_step<16>(accz[e], add);
+    accz[e] = lane_step<32>(accz[e], add);
   }
   if (lane < rch2) {
 #pragma unroll
@@ -277,7 +283,8 @@ __global__ __launch_bounds__(1024) void skinny_quant_kernel(SkinnyQuantArgs a) {
   amax = 0.0f;
 #pragma unroll
   for (int w = 0; w < 16; ++w) amax = fmaxf(amax, red_max[w]);
-  const float scale = amax > 0.0f ? amax / 127.0f : 1.0f;
+  const float scale = amax > 0.0f ? amax / 127.0f : 1.0f, rscale = __builtin_amdgcn_rcpf(scale);
+  const bool ordinary = code_scale_ordinary(scale);
   if (tid == 0) {
     a.sx[m] = scale;
     if (a.scales_rm) a.scales_rm[m] = scale;
@@ -293,13 +300,16 @@ __global__ __launch_bounds__(1024) void skinny_quant_kernel(SkinnyQuantArgs a) {
     if (k0 >= a.K_pad) continue;
     uint32_t lo = 0, hi = 0;
     if (k0 < a.K) {
+      float q[2][4];
+      if (ordinary) {  // workgroup-uniform; a NaN (which the row's maximum passes over) takes the lower limit either way
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        float q = rintf(v[j][e] / scale);
-        q = fminf(fmaxf(q, -127.0f), 127.0f);
-        const uint32_t b = (uint32_t)(int)q & 0xffu;
-        if (e < 4) lo |= b << (8 * e); else hi |= b << (8 * (e - 4));
+        for (int e = 0; e < 8; ++e) q[e >> 2][e & 3] = fmaxf(code_quotient(v[j][e], scale, rscale), -127.0f);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) q[e >> 2][e & 3] = fminf(fmaxf(v[j][e] / scale, -127.0f), 127.0f);
       }
+      lo = code_bytes4(q[0]);
+      hi = code_bytes4(q[1]);
       if (a.codes_rm) *reinterpret_cast<uint2*>(a.codes_rm + (size_t)m * a.K + k0) = make_uint2(lo, hi);
     }
     *reinterpret_cast<uint2*>(a.xq + packed_offset(m, k0, a.KB)) = make_uint2(lo, hi);
