@@ -654,52 +654,6 @@ __device__ inline void bwd_dx_fetch_rs(const BwdDxArgs& g, uint32_t pbase, int b
   }
 }
 
-// The stages of a tile through a ring of AHEAD + 1 LDS stages, LOADS direct-to-LDS loads per wave each: stage i asks for
-// stage i + AHEAD.  `first` prepares the operands of stage 0 (busy: the wave has rows); `even` / `odd` (i, more) multiply
-// stage i and, with more, prepare those of i + 1.  L is even.
-template <int AHEAD, int LOADS, class Issue, class First, class Even, class Odd>
-__device__ inline __attribute__((always_inline)) void bwd_dx_stages(int L, bool busy, Issue&& issue, First&& first, Even&& even, Odd&& odd) {
-  wait_vmcnt<0>();  // stores of the previous tile
-  lds_barrier();
-#pragma unroll
-  for (int i = 0; i < AHEAD; ++i)
-    if (i < L) issue(i);
-  wait_vmcnt<0>();
-  lds_barrier();
-  if (busy) first();
-  const int L_main = L - AHEAD;  // stages that still have loads to issue
-  int i = 0;
-  for (; i + 1 < L_main; i += 2) {
-    // stage i + 1 (and so stage i) is older than the loads of the last AHEAD - 2 stages
-    wait_vmcnt<(AHEAD - 2) * LOADS>();
-    lds_barrier();
-    __builtin_amdgcn_sched_barrier(0);
-    issue(i + AHEAD);
-    even(i, true);
-    __builtin_amdgcn_sched_barrier(0);
-    wait_vmcnt<(AHEAD - 2) * LOADS>();
-    lds_barrier();
-    __builtin_amdgcn_sched_barrier(0);
-    issue(i + 1 + AHEAD);
-    odd(i + 1, true);
-    __builtin_amdgcn_sched_barrier(0);
-  }
-  for (; i < L; i += 2) {  // drain: fewer loads in flight than the count above assumes
-    wait_vmcnt<0>();
-    lds_barrier();
-    __builtin_amdgcn_sched_barrier(0);
-    if (i + AHEAD < L) issue(i + AHEAD);
-    even(i, true);
-    __builtin_amdgcn_sched_barrier(0);
-    wait_vmcnt<0>();
-    lds_barrier();
-    __builtin_amdgcn_sched_barrier(0);
-    if (i + 1 + AHEAD < L) issue(i + 1 + AHEAD);
-    odd(i + 1, i + 2 < L);
-    __builtin_amdgcn_sched_barrier(0);
-  }
-}
-
 // The tiles and split stages of this workgroup in order: work(tile, first stage, stages, slot).
 template <class Work>
 __device__ inline __attribute__((always_inline)) void bwd_dx_schedule(const BwdDxArgs& g, bool may_split, Work&& work) {
@@ -751,13 +705,47 @@ __device__ inline __attribute__((always_inline)) void bwd_dx_schedule(const BwdD
   }
 }
 
-// The 128 x 512 geometry: eight waves side by side along k, a wave tile of 128 rows x 64 k (4 x 2 accumulator blocks of
-// v_mfma_f32_32x32x16_bf16).  A stage holds half the dy panel of the 256 x 256 tile and twice the weight blocks, the same
+// The operands of v_mfma_f32_16x16x32_bf16 from blocks packed for 32x32x16.  Lane (column c, half h) of a transposed weight
+// block holds the chunks q = 0 (lo) and 1 (hi) of its column; the operand of 16 columns wants the chunks of a column in its four
+// rows of lanes, (q, h) = (row % 2, row / 2): one swap leaves that of columns 0..15 in lo and of 16..31 in hi.
+__device__ inline void bwd_operand_rows(uint32_t& lo, uint32_t& hi) {
+  const auto s = __builtin_amdgcn_permlane16_swap(lo, hi, false, false);
+  lo = s[0]; hi = s[1];
+}
+// ... and where the lane finds its part of dy's rows 0..15 in the two 1 KiB chunks of a row block (rows 16..31: 256 bytes on)
+__device__ inline uint32_t bwd_frag_offset(uint32_t lane) {
+  return ((lane >> 4) & 1u) * (uint32_t)kBlockBytes + (lane >> 5) * 512u + (lane & 15u) * 16u;
+}
+// row block p of 16 of the panel
+__device__ inline v8bf bwd_panel_frag(uint32_t panel, int p) {
+  typedef __attribute__((address_space(3))) const v4i* lds_v4ptr;
+  return __builtin_bit_cast(v8bf, *reinterpret_cast<lds_v4ptr>((uintptr_t)(panel + (uint32_t)((p >> 1) * 2048 + (p & 1) * 256))));
+}
+// Four 16 x 16 blocks, [row half][column half], as the 32 x 32 block that the epilogue and the partial tiles know: a lane's
+// rows 4 (lane / 16) + i of a half become rows 8 j + 4 (lane / 32) + i, the column's bit 4 the lane's.
+__device__ inline v16f bwd_block32(const v4f (&b)[2][2]) {
+  v16f y;
+#pragma unroll
+  for (int rh = 0; rh < 2; ++rh)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(b[rh][0][i]), __float_as_uint(b[rh][1][i]), false, false);
+      const auto t = __builtin_amdgcn_permlane32_swap(s[0], s[1], false, false);
+      y[8 * rh + i] = __uint_as_float(t[0]);
+      y[8 * rh + 4 + i] = __uint_as_float(t[1]);
+    }
+  return y;
+}
+
+// The 128 x 512 geometry: eight waves side by side along k, a wave tile of 128 rows x 64 k (8 x 4 accumulator blocks of
+// v_mfma_f32_16x16x32_bf16).  A stage holds half the dy panel of the 256 x 256 tile and twice the weight blocks, the same
 // bytes.  For grouped calls whose weights own few rows each: half the padding per weight, and every wave has rows.
 //
-// The 256 registers that two waves per SIMD leave are the kernel's limit: the loads' addresses are a scalar base plus the
-// lane's offset (issue), and the epilogue derives its lane constants for itself (bwd_dx_store).  Held in vector
-// registers through the stages both cost 16 bytes of scratch per lane; 8168 rows of 128 experts, 2048 <- 1536, spilling / as it is 207 / 204 us.
+// Bound by HBM (the weights are read once) and by what stands in line behind it in a stage.  The 256 registers that two waves
+// per SIMD leave are the kernel's limit: the loads' addresses are a scalar base plus the lane's offset (issue), and the epilogue
+// derives its lane constants for itself (bwd_dx_store).  1021 tokens to 8 of 128 experts, 2048 <- 1536 and 768 <- 2048 (600 MB of
+// weights): 197 us together with the row blocks skipped by a branch each, behind which the compiler read every fragment at its
+// use, and the loads' addresses formed anew for every stage; one loop for each number of row blocks 174.
 constexpr int kBwdPanel128 = 8192, kBwdWeight512 = 16384;  // 4 row blocks x 2 halves; 16 k blocks
 static_assert(kBwdPanel128 + kBwdWeight512 + 1024 == kBwdStageBytes, "a stage keeps its size in both geometries");
 constexpr int kBwdAhead = kBwdStages - 1;  // stages between a load and its use
@@ -768,7 +756,7 @@ __global__ __launch_bounds__(512, 1) void bwd_dx_kernel(BwdDxArgs g) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 31, h = lane >> 5;
-  const uint32_t lane16 = (uint32_t)lane * 16u;
+  const uint32_t lane16 = (uint32_t)lane * 16u, lds_base = (uint32_t)(uintptr_t)(lptr_t)lds;
 
   // identity operand of the transposing MFMA: lane (column c, k half h) holds byte 1 at k == c
   v4i ident = {0, 0, 0, 0};
@@ -779,170 +767,185 @@ __global__ __launch_bounds__(512, 1) void bwd_dx_kernel(BwdDxArgs g) {
     ident[2] = wi == 2 ? word : 0; ident[3] = wi == 3 ? word : 0;
   }
 
-  auto tile = [&](uint32_t tm, uint32_t tk) {
-    const int tv = g.tile_weight[tm];
-    if (tv < 0) return;  // workgroup-uniform: no row lives in this tile
-    const int tw = tv & 0xffff, live_blocks = ((tv >> 16) + 31) / 32;
-    // 32-row blocks that hold rows: the others skip their matrix-core work
-    const int n_act = __builtin_amdgcn_readfirstlane(live_blocks < 0 ? 0 : (live_blocks > 4 ? 4 : live_blocks));
+  // ROWS: the tile's 32-row blocks that hold rows; the others are not multiplied
+  auto tile = [&](auto rows_tag, uint32_t tm, uint32_t tk, int tw) {
+    constexpr int ROWS = decltype(rows_tag)::value, kRows16 = 2 * ROWS;
+    const int L = (int)g.NB;  // (even)
     // row block of whose dy panel this wave fetches a half.  A block without rows is never multiplied: its slot is filled from block 0
     // of the tile, which is in the caches anyway, instead of streaming unused memory (the load count stays the same)
-    const uint32_t load_rb = (wave >> 1) < live_blocks ? (uint32_t)wave >> 1 : 0u;
-    const float* swp_t = g.swp + (size_t)tw * g.sw_stride;
-    const unsigned char* Ag = g.dyp + ((size_t)(tm * 4u + load_rb) * g.NB) * 2048u + (wave & 1) * 1024;
+    const uint32_t load_rb = (wave >> 1) < ROWS ? (uint32_t)wave >> 1 : 0u;
+    const unsigned char* const Ag = g.dyp + ((size_t)(tm * 4u + load_rb) * g.NB) * 2048u + (wave & 1) * 1024;
     const uint32_t kbw = tk * 16u + (uint32_t)wave * 2u;  // its two k blocks (blocks past the weight repeat the last)
-    const uint32_t kbl = kbw < g.KB ? kbw : g.KB - 1u;
-    const uint32_t kbl1 = kbw + 1u < g.KB ? kbw + 1u : g.KB - 1u;
-    const unsigned char* Bg = g.wp + (size_t)tw * g.w_stride + (size_t)kbl * kBlockBytes;
-    const unsigned char* Bg1 = g.wp + (size_t)tw * g.w_stride + (size_t)kbl1 * kBlockBytes;
     const size_t nb_stride = (size_t)g.KB * kBlockBytes;
-
-    auto issue = [&](int nb) {
-      unsigned char* St = lds + (nb % kBwdStages) * kBwdStageBytes;
-      load_1k_to_lds(Ag + (size_t)nb * 2048u + lane16, St + wave * kBlockBytes);
+    const unsigned char* Bg0 = g.wp + (size_t)tw * g.w_stride + (size_t)(kbw < g.KB ? kbw : g.KB - 1u) * kBlockBytes;
+    const unsigned char* Bg1 = kbw + 1u < g.KB ? Bg0 : Bg0 - kBlockBytes;  // (lds_load_2k: 1 KiB further)
+    const unsigned char* const swp_t = reinterpret_cast<const unsigned char*>(g.swp + (size_t)tw * g.sw_stride);
+    uint32_t a_off = lane16, s_off = lane16;
+    auto issue = [&](uint32_t st) {  // the next stage's loads, into the stage buffer at st
+      lds_load_1k(Ag, a_off, st + (uint32_t)wave * kBlockBytes);
       // (few rows per weight: most of its bytes are read by one workgroup only)
-      load_1k_to_lds_once(Bg + (size_t)nb * nb_stride + lane16, St + kBwdPanel128 + (wave * 2) * kBlockBytes);
-      load_1k_to_lds_once(Bg1 + (size_t)nb * nb_stride + lane16, St + kBwdPanel128 + (wave * 2 + 1) * kBlockBytes);
+      lds_load_2k<true>(Bg0, Bg1, lane16, st + kBwdPanel128 + (uint32_t)wave * 2048u);
       // every wave fetches the same 1 KiB of scales (the stage's 32 lead it) to the same place
-      load_1k_to_lds(reinterpret_cast<const unsigned char*>(swp_t + 32 * nb) + lane16, St + kBwdPanel128 + kBwdWeight512);
+      lds_load_1k(swp_t, s_off, st + kBwdPanel128 + kBwdWeight512);
+      a_off += 2048u;
+      s_off += 128u;
+      Bg0 += nb_stride;
+      Bg1 += nb_stride;
     };
 
-    v16f acc[4][2];
+    v4f acc[kRows16][4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < kRows16; ++i)
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
+      for (int j = 0; j < 4; ++j)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+        for (int e = 0; e < 4; ++e) acc[i][j][e] = 0.0f;
 
+    typedef __attribute__((address_space(3))) const v4i* lds_v4ptr;
+    const uint32_t frag_off = bwd_frag_offset((uint32_t)lane), weight_off = (uint32_t)wave * 2048u + lane16, scale_off = 16u * (uint32_t)h;
+    struct NextRegs { v4i raw[2]; v4f s4[4]; };
+    auto next_read = [&](uint32_t st, NextRegs& r) {  // the wave's weight blocks and the scales of the stage at st
+      uint32_t wa = st + weight_off, sa = st + scale_off;
+      asm volatile("" : "+v"(wa), "+v"(sa));  // (opaque: constants are the instructions')
+#pragma unroll
+      for (int b = 0; b < 2; ++b) r.raw[b] = *reinterpret_cast<lds_v4ptr>((uintptr_t)(wa + kBwdPanel128 + b * kBlockBytes));
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        r.s4[q] = __builtin_bit_cast(v4f, *reinterpret_cast<lds_v4ptr>((uintptr_t)(sa + kBwdPanel128 + kBwdWeight512 + 32 * q)));
+    };
     auto transpose_block = [&](const v4i& rawb) -> v16i {
       v16i z16;
 #pragma unroll
       for (int e = 0; e < 16; ++e) z16[e] = 0;
       return __builtin_amdgcn_mfma_i32_32x32x32_i8(rawb, ident, z16, 0, 0, 0);
     };
-    // rows 8 gq + 4 h + 0..3 of a transposed block: bf16(float(code) * scale), the per-element
+    // rows 8 (t / 2) + 4 h + 2 (t % 2) + 0, 1 of a transposed block: bf16(float(code) * scale), the per-element
     // weight of the reference's pull-back
-    auto convert4 = [&](const v16i& tr, const v4f& s4, int gq, uint32_t (&pk)[8]) {
-      const float f0 = (float)tr[4 * gq + 0] * s4[0], f1 = (float)tr[4 * gq + 1] * s4[1];
-      const float f2 = (float)tr[4 * gq + 2] * s4[2], f3 = (float)tr[4 * gq + 3] * s4[3];
-      pk[2 * gq] = pack_bf16x2(f0, f1);
-      pk[2 * gq + 1] = pack_bf16x2(f2, f3);
+    auto convert2 = [&](const v16i& tr, const v4f (&s4)[4], int t, uint32_t (&pk)[8]) {
+      const float f0 = (float)tr[2 * t] * s4[t >> 1][2 * (t & 1)], f1 = (float)tr[2 * t + 1] * s4[t >> 1][2 * (t & 1) + 1];
+      pk[t] = pack_bf16x2(f0, f1);
     };
-    auto to_operands = [&](const uint32_t (&pk)[8], v8bf (&bq)[2]) {
+    auto to_operands = [&](uint32_t (&pk)[8], v8bf (&bq)[2]) {
+#pragma unroll
+      for (int t = 0; t < 4; ++t) bwd_operand_rows(pk[t], pk[4 + t]);
       bq[0] = __builtin_bit_cast(v8bf, v4i{(int)pk[0], (int)pk[1], (int)pk[2], (int)pk[3]});
       bq[1] = __builtin_bit_cast(v8bf, v4i{(int)pk[4], (int)pk[5], (int)pk[6], (int)pk[7]});
     };
-    auto panel_frag = [&](int nb, int pair) -> v8bf {  // pair = 4 q + row block
-      const unsigned char* St = lds + (nb % kBwdStages) * kBwdStageBytes;
-      return __builtin_bit_cast(
-          v8bf, *reinterpret_cast<const v4i*>(St + ((pair & 3) * 2 + (pair >> 2)) * kBlockBytes + lane * 16));
-    };
-    // The weight blocks and scales of the next stage are read from LDS with explicit instructions:
-    // a compiler-visible read of memory that direct-to-LDS loads write makes the compiler drain
-    // every outstanding load first (it cannot tell the stages apart), which would serialize the
-    // pipeline.  The six values are valid after next_wait().
-    const uint32_t lds_base = (uint32_t)(uintptr_t)(lptr_t)lds;
-    struct NextRegs { v4i raw[2]; v4f s4[4]; };
-    auto next_read = [&](int nb1, NextRegs& r) {
-      const uint32_t st = lds_base + (nb1 % kBwdStages) * kBwdStageBytes + kBwdPanel128;
-      const uint32_t wa = st + (wave * 2) * kBlockBytes + lane * 16;
-      const uint32_t sa = st + kBwdWeight512 + 16 * h;
-      asm volatile("ds_read_b128 %0, %6\n\tds_read_b128 %1, %6 offset:1024\n\t"
-                   "ds_read_b128 %2, %7\n\tds_read_b128 %3, %7 offset:32\n\t"
-                   "ds_read_b128 %4, %7 offset:64\n\tds_read_b128 %5, %7 offset:96"
-                   : "=&v"(r.raw[0]), "=&v"(r.raw[1]), "=&v"(r.s4[0]), "=&v"(r.s4[1]), "=&v"(r.s4[2]), "=&v"(r.s4[3])
-                   : "v"(wa), "v"(sa)
-                   : "memory");
-    };
-    auto next_wait = [&](NextRegs& r) {
-      asm volatile("s_waitcnt lgkmcnt(0)"
-                   : "+v"(r.raw[0]), "+v"(r.raw[1]), "+v"(r.s4[0]), "+v"(r.s4[1]), "+v"(r.s4[2]), "+v"(r.s4[3])
-                   :
-                   : "memory");
+    auto panel_at = [&](uint32_t st) -> uint32_t {
+      uint32_t at = st + frag_off;
+      asm volatile("" : "+v"(at));
+      return at;
     };
 
-    // One stage: 16 MFMAs of stage nb against the dy panel in LDS; between them the operands of
-    // stage nb + 1 are prepared (vector ALU work under the matrix core's shadow).
-    auto stage = [&](int nb, const v8bf (&bqC)[2][2], v8bf (&bqN)[2][2], bool convert_next) {
-      if (n_act == 0) return;  // wave-uniform: a wave without rows only feeds the pipeline
+    // One stage, at st: its MFMAs against the dy panel in the LDS; between them the operands of the stage at st_next are
+    // prepared, a block of the two in each half of the row blocks.  af: the first row block's fragment; leaves the next stage's.
+    auto stage = [&](uint32_t st, uint32_t st_next, const v8bf (&bqC)[2][2], v8bf (&bqN)[2][2], v8bf& af) {
       NextRegs nx;
       v16i tr;
       uint32_t pk[8];
-      if (convert_next) next_read(nb + 1, nx);
-      v8bf af = panel_frag(nb, 0);
+      const uint32_t panel = panel_at(st), panel_next = panel_at(st_next);
+      next_read(st_next, nx);
 #pragma unroll
-      for (int pair = 0; pair < 8; ++pair) {
-        const int q = pair >> 2, rb = pair & 3;
-        v8bf af_next = af;
-        if (pair < 7) af_next = panel_frag(nb, pair + 1);
-        if (rb < n_act) {
-          acc[rb][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af, bqC[0][q], acc[rb][0], 0, 0, 0);
-          acc[rb][1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af, bqC[1][q], acc[rb][1], 0, 0, 0);
-        }
-        if (convert_next) {
-          if (pair == 0) {
-            next_wait(nx);
-            tr = transpose_block(nx.raw[0]);
-          } else {
-            const int cstep = pair - 1;  // conversion step: k block cstep / 4, rows 8 (cstep % 4) + ...
-            convert4(tr, nx.s4[cstep & 3], cstep & 3, pk);
-            if (cstep == 3) {
-              to_operands(pk, bqN[0]);
-              tr = transpose_block(nx.raw[1]);
-            }
-          }
+      for (int p = 0; p < kRows16; ++p) {
+        const v8bf af_next = p + 1 < kRows16 ? bwd_panel_frag(panel, p + 1) : bwd_panel_frag(panel_next, 0);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          acc[p][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af, bqC[j >> 1][j & 1], acc[p][j], 0, 0, 0);
+        const int b = p / ROWS, at = p % ROWS;  // weight block, place in its half
+        if (at == 0) tr = transpose_block(nx.raw[b]);
+        constexpr int kParts = ROWS > 1 ? ROWS - 1 : 1;
+        if (ROWS == 1 || at > 0) {
+          const int part = ROWS > 1 ? at - 1 : 0;
+#pragma unroll
+          for (int t = 8 * part / kParts; t < 8 * (part + 1) / kParts; ++t) convert2(tr, nx.s4, t, pk);
+          if (part == kParts - 1) to_operands(pk, bqN[b]);
         }
         __builtin_amdgcn_sched_barrier(0);
         af = af_next;
       }
-      if (convert_next) {
-        convert4(tr, nx.s4[3], 3, pk);
-        to_operands(pk, bqN[1]);
-      }
     };
 
-    v8bf bqA[2][2], bqB[2][2];
-    bwd_dx_stages<kBwdAhead, kBwdLoadsPerStage>(
-        (int)g.NB, n_act > 0, issue,
-        [&] {  // operands of stage 0
-          NextRegs nx;
-          next_read(0, nx);
-          next_wait(nx);
-          uint32_t pk[8];
+    v8bf bqA[2][2], bqB[2][2], af;
+    wait_vmcnt<0>();  // stores of the previous tile
+    lds_barrier();
 #pragma unroll
-          for (int cb = 0; cb < 2; ++cb) {
-            const v16i tr = transpose_block(nx.raw[cb]);
+    for (int i = 0; i < kBwdAhead; ++i)
+      if (i < L) issue(lds_base + (uint32_t)i * kBwdStageBytes);
+    if (L >= kBwdAhead) wait_vmcnt<(kBwdAhead - 1) * kBwdLoadsPerStage>();  // stage 0 has landed
+    else wait_vmcnt<0>();
+    lds_barrier();
+    {  // operands of stage 0
+      NextRegs nx;
+      next_read(lds_base, nx);
+      uint32_t pk[8];
 #pragma unroll
-            for (int gq = 0; gq < 4; ++gq) convert4(tr, nx.s4[gq], gq, pk);
-            to_operands(pk, bqA[cb]);
-          }
-        },
-        [&](int i, bool more) { stage(i, bqA, bqB, more); }, [&](int i, bool more) { stage(i, bqB, bqA, more); });
+      for (int cb = 0; cb < 2; ++cb) {
+        const v16i tr = transpose_block(nx.raw[cb]);
+#pragma unroll
+        for (int t = 0; t < 8; ++t) convert2(tr, nx.s4, t, pk);
+        to_operands(pk, bqA[cb]);
+      }
+    }
+    af = bwd_panel_frag(panel_at(lds_base), 0);
+    uint32_t st = lds_base;  // of stage i; the loads go into the buffer in front of it
+    // stages i and i + 1 have landed, i + 2 .. i + 4 are on their way and i + 5 is asked for.  (Behind the last stage nothing reads
+    // the operands that are prepared.)
+    auto step = [&](int i, const v8bf (&bqC)[2][2], v8bf (&bqN)[2][2]) {
+      const uint32_t last = lds_base + (uint32_t)(kBwdStages - 1) * kBwdStageBytes;
+      const uint32_t st_next = st == last ? lds_base : st + kBwdStageBytes, st_load = st == lds_base ? last : st - kBwdStageBytes;
+      if (i + kBwdAhead < L) {
+        wait_vmcnt<(kBwdAhead - 2) * kBwdLoadsPerStage>();
+        lds_barrier();
+        issue(st_load);
+      } else {  // fewer loads in flight than that count assumes
+        wait_vmcnt<0>();
+        lds_barrier();
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      stage(st, st_next, bqC, bqN, af);
+      st = st_next;
+    };
+#pragma unroll 1
+    for (int i = 0; i < L; i += 2) {
+      step(i, bqA, bqB);
+      step(i + 1, bqB, bqA);
+    }
 
     lds_barrier();  // (every wave has read its last stage)
     const uint32_t rs_lds = lds_base + 8u * kBwdTurnBytes;
-    bwd_dx_fetch_rs<NKK>(g, tm * 128u, live_blocks, rs_lds, wave, 8);
-    if (n_act)
-      bwd_dx_store<NKK, 2, 4, true>(g, tm * 128u, kbw, n_act, lds_base + (uint32_t)wave * kBwdTurnBytes, rs_lds,
-                                    [&](int rb, int cb) -> v16f { return acc[rb][cb]; });
+    bwd_dx_fetch_rs<NKK>(g, tm * 128u, ROWS, rs_lds, wave, 8);
+    bwd_dx_store<NKK, 2, ROWS, true>(g, tm * 128u, kbw, ROWS, lds_base + (uint32_t)wave * kBwdTurnBytes, rs_lds,
+                                     [&](int rb, int cb) -> v16f {
+      const v4f b[2][2] = {{acc[2 * rb][2 * cb], acc[2 * rb][2 * cb + 1]}, {acc[2 * rb + 1][2 * cb], acc[2 * rb + 1][2 * cb + 1]}};
+      return bwd_block32(b);
+    });
   };
 
   bwd_dx_schedule(g, false, [&](uint32_t t, int, int, uint32_t) {
     uint32_t tm, tk;
     bwd_dx_tile_at(g, t, tm, tk);
-    tile(tm, tk);
+    const int tv = g.tile_weight[tm];
+    if (tv < 0) return;  // workgroup-uniform: no row lives in this tile
+    const int tw = tv & 0xffff, blocks = __builtin_amdgcn_readfirstlane(((tv >> 16) + 31) / 32);
+    if (blocks <= 1) tile(std::integral_constant<int, 1>{}, tm, tk, tw);
+    else if (blocks == 2) tile(std::integral_constant<int, 2>{}, tm, tk, tw);
+    else if (blocks == 3) tile(std::integral_constant<int, 3>{}, tm, tk, tw);
+    else tile(std::integral_constant<int, 4>{}, tm, tk, tw);
   });
 }
 
-// The 256 x 256 geometry: four waves, one to a SIMD, side by side along k: a wave tile of 256 rows x 64 k (8 x 2 accumulator
+// The 256 x 256 geometry: four waves, one to a SIMD, side by side along k: a wave tile of 256 rows x 64 k (16 x 4 accumulator
 // blocks, 256 registers, beside 256 others).  No two waves then convert the same weight blocks, which as eight waves of
-// 128 x 64 every two did: 2 transposing MFMAs and 80 vector instructions for 32 MFMAs instead of 16.  What a
+// 128 x 64 every two did: 2 transposing MFMAs and 88 vector instructions for 64 MFMAs instead of 32.  What a
 // second wave per SIMD hid is hidden by order: the conversion of the next stage's blocks stands between single MFMAs, the dy
-// fragments are read three pairs ahead, and a barrier comes every two stages.
-// ROWS: row blocks multiplied (8, or 4 where the tile holds no more: the others' dy is loaded from block 0 and left alone).
-// Power more than issue bounds it (all-zero dy runs a quarter faster).  3003 x 4096, N = 24576, rank 32: 663 us as eight waves of 128 x 64, now
-// 508 (1.19 PFLOP/s); 3003 x 12288, N = 4096 378 / 285, of which the epilogue below 45; 2048 x 2560, N = 10240, rank 64 131 / 105.
+// fragments are read three row blocks ahead, also across the barrier, which comes every two stages.
+// ROWS: row blocks of 32 multiplied (8, or 4 where the tile holds no more: the others' dy is loaded from block 0 and left alone).
+// Power bounds it (all-zero dy runs a quarter faster), and the one wave's issue slots: 128 MFMAs hold the matrix core for 2048
+// clocks, 512 slots.  v_mfma_f32_16x16x32_bf16 carries half the sums per product of 32x32x16: from registers alone
+// 2045 TFLOP/s against 1750 to 1790.  An MLP's two pull-backs, 3003 rows, 4096 <- 24576 and 12288 <- 4096: 837 us with 32x32x16
+// and 464 instructions to two stages (the weight's reads waited for where they stood), 789 now (1.15 PFLOP/s; 472).  With
+// 16x16x32 but 549 instructions it was 2 % slower than before.  2048 x 2560, N = 10240, rank 64: 110 / 107.
 constexpr int kBwdWideLoads = 7;  // direct-to-LDS loads per wave and stage: 4 panel chunks, 2 weight blocks, scales
 
 // The accumulator tied, as one read-write operand, in the half of the register file that is named: left to the compiler, or all
@@ -950,17 +953,17 @@ constexpr int kBwdWideLoads = 7;  // direct-to-LDS loads per wave and stage: 4 p
 // The compiler does not see that an MFMA writes the sums: they are next touched by the MFMA of the other half block or
 // of the next stage, and the epilogue stands behind explicit wait states.
 template <bool HIGH>
-__device__ inline void bwd_mfma(v16f& acc, const v8bf& a, const v8bf& b) {
-  if constexpr (HIGH) asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
-  else asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "v"(b));
+__device__ inline void bwd_mfma(v4f& acc, const v8bf& a, const v8bf& b) {
+  if constexpr (HIGH) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
+  else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "v"(b));
 }
 // The sums for the vector ALU.  (As plain values their uses behind the loop drew the sums into the other half within it.)
 template <bool HIGH>
-__device__ inline v16f bwd_sums(v16f& acc) {
-  v16f y;
+__device__ inline v4f bwd_sums(v4f& acc) {
+  v4f y;
   if constexpr (HIGH) {
 #pragma unroll
-    for (int e = 0; e < 16; ++e) asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(y[e]) : "a"(acc[e]));
+    for (int e = 0; e < 4; ++e) asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(y[e]) : "a"(acc[e]));
   } else {
     asm volatile("" : "+v"(acc));  // (behind the wait states, too)
     y = acc;
@@ -996,106 +999,125 @@ __global__ __launch_bounds__(256, 1) void bwd_dx_wide_kernel(BwdDxArgs g) {
     int lane_s = lane;
     asm volatile("" : "+v"(lane_s));
     const uint32_t lane16 = (uint32_t)lane_s * 16u, h16 = (uint32_t)(lane_s >> 5) * 16u;
-    const float* swp_t = g.swp + (size_t)tw * g.sw_stride;
     // this wave's loads of a stage: dy of two row blocks (both halves), two weight blocks
     const uint32_t rb0 = 2u * (uint32_t)wave < (uint32_t)live_blocks ? 2u * (uint32_t)wave : 0u;
     const uint32_t rb1 = 2u * (uint32_t)wave + 1u < (uint32_t)live_blocks ? 2u * (uint32_t)wave + 1u : 0u;
-    const unsigned char* Ag0 = g.dyp + ((size_t)(tm * 8u + rb0) * g.NB) * 2048u;
-    const unsigned char* Ag1 = g.dyp + ((size_t)(tm * 8u + rb1) * g.NB) * 2048u;
+    const unsigned char* const Ag0 = g.dyp + ((size_t)(tm * 8u + rb0) * g.NB + (uint32_t)nb0) * 2048u;
+    const unsigned char* const Ag1 = g.dyp + ((size_t)(tm * 8u + rb1) * g.NB + (uint32_t)nb0) * 2048u;
     const uint32_t kbw = tk * 8u + 2u * (uint32_t)wave;  // its two k blocks (blocks past the weight repeat the last)
-    const unsigned char* Wt = g.wp + (size_t)tw * g.w_stride;
-    const unsigned char* Bg0 = Wt + (size_t)(kbw < g.KB ? kbw : g.KB - 1u) * kBlockBytes;
-    const unsigned char* Bg1 = Wt + (size_t)(kbw + 1u < g.KB ? kbw + 1u : g.KB - 1u) * kBlockBytes;
     const size_t nb_stride = (size_t)g.KB * kBlockBytes;
-    // Load j of the seven of stage i (behind the last stage: of that one again).  Loads the compiler keeps no books on: it
-    // would drain them before every read of the LDS.
-    auto issue = [&](int i, int j) {
-      const uint32_t st = lds_base + (i % kBwdStages) * kBwdStageBytes;
-      const int nb = nb0 + (i < L ? i : L - 1);
-      if (j < 4) lds_load_1k((j < 2 ? Ag0 : Ag1) + (size_t)nb * 2048u + 1024 * (j & 1), lane16, st + (wave * 4 + j) * kBlockBytes);
-      else if (j < 6) lds_load_1k((j == 4 ? Bg0 : Bg1) + (size_t)nb * nb_stride, lane16, st + kBwdStagePanel + (wave * 2 + j - 4) * kBlockBytes);
-      else lds_load_1k(reinterpret_cast<const unsigned char*>(swp_t + 32 * nb), lane16, st + kBwdStagePanel + kBwdStageWeight);
+    const unsigned char* Bg0 = g.wp + (size_t)tw * g.w_stride + (size_t)nb0 * nb_stride + (size_t)(kbw < g.KB ? kbw : g.KB - 1u) * kBlockBytes;
+    const unsigned char* Bg1 = kbw + 1u < g.KB ? Bg0 : Bg0 - kBlockBytes;  // (lds_load_2k: 1 KiB further)
+    const unsigned char* const swp_t = reinterpret_cast<const unsigned char*>(g.swp + (size_t)tw * g.sw_stride + 32 * nb0);
+    uint32_t a_off = lane16, s_off = lane16;
+    int stages_left = L - 1;
+    // Part j of four of the loads of the next stage to be asked for, into the stage buffer at st (behind the last stage: of that
+    // one again).  Loads the compiler keeps no books on: it would drain them before every read of the LDS.  The addresses go
+    // on from stage to stage: a loop of 128 MFMAs leaves 400 issue slots for all else, and formed anew they took 100.
+    auto issue = [&](uint32_t st, int j) {
+      if (j == 0) lds_load_2k(Ag0, a_off, st + (uint32_t)wave * 4096u);
+      else if (j == 1) lds_load_2k(Ag1, a_off, st + (uint32_t)wave * 4096u + 2048u);
+      else if (j == 2) lds_load_2k<false>(Bg0, Bg1, lane16, st + kBwdStagePanel + (uint32_t)wave * 2048u);
+      else {
+        lds_load_1k(swp_t, s_off, st + kBwdStagePanel + kBwdStageWeight);
+        const bool more = stages_left > 0;
+        --stages_left;
+        a_off += more ? 2048u : 0u;
+        s_off += more ? 128u : 0u;
+        Bg0 += more ? nb_stride : 0;
+        Bg1 += more ? nb_stride : 0;
+      }
     };
-    v16f acc[ROWS][2];
+    constexpr int kRows16 = 2 * ROWS;  // row blocks of 16
+    v4f acc[kRows16][4];
 #pragma unroll
-    for (int i = 0; i < ROWS; ++i)
+    for (int i = 0; i < kRows16; ++i)
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
+      for (int j = 0; j < 4; ++j)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+        for (int e = 0; e < 4; ++e) acc[i][j][e] = 0.0f;
 
     struct NextRegs { v4i raw[2]; v4f s4[4]; };
-    // (explicit instructions: see bwd_dx_kernel)
-    auto next_read = [&](int i, NextRegs& r) {
-      const uint32_t st = lds_base + (i % kBwdStages) * kBwdStageBytes + kBwdStagePanel;
-      const uint32_t wa = st + (wave * 2) * kBlockBytes + lane16;
-      const uint32_t sa = st + kBwdStageWeight + h16;
-      asm volatile("ds_read_b128 %0, %6\n\tds_read_b128 %1, %6 offset:1024\n\t"
-                   "ds_read_b128 %2, %7\n\tds_read_b128 %3, %7 offset:32\n\t"
-                   "ds_read_b128 %4, %7 offset:64\n\tds_read_b128 %5, %7 offset:96\n\t"
-                   "s_waitcnt lgkmcnt(0)"
-                   : "=&v"(r.raw[0]), "=&v"(r.raw[1]), "=&v"(r.s4[0]), "=&v"(r.s4[1]), "=&v"(r.s4[2]), "=&v"(r.s4[3])
-                   : "v"(wa), "v"(sa)
-                   : "memory");
+    const uint32_t weight_off = (uint32_t)wave * 2048u + lane16;
+    // The weight blocks and scales of the stage at st, in three parts.  (Reads that the compiler waits for where they are used.)
+    auto next_read = [&](uint32_t st, int part, NextRegs& r) {
+      typedef __attribute__((address_space(3))) const v4i* lds_v4ptr;
+      if (part == 0) {
+        uint32_t wa = st + weight_off;
+        asm volatile("" : "+v"(wa));
+        r.raw[0] = *reinterpret_cast<lds_v4ptr>((uintptr_t)(wa + kBwdStagePanel));
+        r.raw[1] = *reinterpret_cast<lds_v4ptr>((uintptr_t)(wa + kBwdStagePanel + kBlockBytes));
+      } else {
+        uint32_t sa = st + h16;
+        asm volatile("" : "+v"(sa));
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+          r.s4[2 * part - 2 + q] = __builtin_bit_cast(v4f, *reinterpret_cast<lds_v4ptr>((uintptr_t)(sa + kBwdStagePanel + kBwdStageWeight + 32 * (2 * part - 2 + q))));
+      }
     };
     // rows 8 (t / 2) + 4 h + 2 (t % 2) + 0, 1 of a transposed block: bf16(float(code) * scale), the per-element
     // weight of the reference's pull-back
-    auto convert2 = [&](const v16i& tr, const v4f (&s4)[4], int t, uint32_t (&pk)[8]) {
-      const float f0 = (float)tr[2 * t] * s4[t >> 1][2 * (t & 1)], f1 = (float)tr[2 * t + 1] * s4[t >> 1][2 * (t & 1) + 1];
-      pk[t] = pack_bf16x2(f0, f1);
+    auto convert_first = [&](const v16i& tr, int t, float (&f)[2]) { f[0] = (float)tr[2 * t]; f[1] = (float)tr[2 * t + 1]; };
+    auto convert_second = [&](const v4f (&s4)[4], int t, const float (&f)[2], uint32_t (&pk)[8]) {
+      pk[t] = pack_bf16x2(f[0] * s4[t >> 1][2 * (t & 1)], f[1] * s4[t >> 1][2 * (t & 1) + 1]);
     };
     auto to_operands = [&](const uint32_t (&pk)[8], v8bf (&bq)[2]) {
       bq[0] = __builtin_bit_cast(v8bf, v4i{(int)pk[0], (int)pk[1], (int)pk[2], (int)pk[3]});
       bq[1] = __builtin_bit_cast(v8bf, v4i{(int)pk[4], (int)pk[5], (int)pk[6], (int)pk[7]});
     };
-    constexpr int kPairs = 2 * ROWS;  // (half q, row block) of a stage
-    auto panel_frag = [&](int i, int pair) -> v8bf {
-      typedef __attribute__((address_space(3))) const v4i* lds_v4ptr;
-      const uint32_t at = lds_base + (i % kBwdStages) * kBwdStageBytes + lane16;
-      return __builtin_bit_cast(v8bf, *reinterpret_cast<lds_v4ptr>((uintptr_t)(at + ((pair % ROWS) * 2 + pair / ROWS) * kBlockBytes)));
+    const uint32_t frag_off = bwd_frag_offset((uint32_t)lane_s);
+    auto panel_at = [&](uint32_t st) -> uint32_t {
+      uint32_t at = st + frag_off;
+      asm volatile("" : "+v"(at));  // (opaque: the rows' offsets are the instructions', not sixteen registers)
+      return at;
     };
-    // One stage: its MFMAs from the dy panel in the LDS; between them the operands of stage i + 1 are prepared.
-    // af: the fragments of the first three pairs; leaves those of stage i + 1 there where that one has landed (ahead).
-    auto stage = [&](int i, const v8bf (&bqC)[2][2], v8bf (&bqN)[2][2], bool ahead, v8bf (&af)[4]) {
+    // One stage, at st: its MFMAs from the dy panel in the LDS; between them the operands of the stage at st_next are prepared
+    // and the loads of the one at st_load are issued.  af: the fragments of the first three row blocks; leaves the next stage's.
+    auto stage = [&](uint32_t st, uint32_t st_next, uint32_t st_load, const v8bf (&bqC)[2][2], v8bf (&bqN)[2][2], v8bf (&af)[4]) {
       NextRegs nx;
       v16i tr;
       uint32_t pk[8];
+      float part[2];
       asm volatile("s_nop 3");  // (operands converted at the end of the stage before)
-      next_read(i + 1, nx);
-      // pairs behind which the two blocks are transposed; their conversion starts behind three more MFMAs, when the result is there
-      constexpr int kT0 = ROWS == 8 ? 1 : 0, kT1 = ROWS == 8 ? 7 : 3;
-      constexpr int kPer = ROWS == 8 ? 1 : 2;  // conversion steps (of 8 a block) in each half of a pair
-      auto convert_part = [&](int pair, int half) {
+      const uint32_t panel = panel_at(st), panel_next = panel_at(st_next);
+      // row blocks behind which the two weight blocks are transposed; their conversion starts behind five more MFMAs, when
+      // the result is there
+      constexpr int kT0 = ROWS == 8 ? 2 : 0, kT1 = ROWS == 8 ? 8 : 3;
+      constexpr int kPer = ROWS == 8 ? 1 : 2;  // conversion steps (of 8 a block) in each half of a row block's MFMAs
+      auto convert_part = [&](int p, int quarter) {  // (a step in two quarters; two steps a half: one to a quarter)
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
           const int t0 = (b ? kT1 : kT0) + 2;
-          if (pair == t0 && half == 0) asm volatile("" : "+v"(tr));  // (not read before this place)
-#pragma unroll
-          for (int u = 0; u < kPer; ++u) {
-            const int t = ((pair - t0) * 2 + half) * kPer + u;
-            if (pair >= t0 && t < 8) {
-              convert2(tr, nx.s4, t, pk);
-              if (t == 7) to_operands(pk, bqN[b]);
-            }
+          if (p == t0 && quarter == 0) asm volatile("" : "+v"(tr));  // (not read before this place)
+          const int t = kPer == 1 ? (p - t0) * 2 + (quarter >> 1) : (p - t0) * 4 + quarter;
+          const bool opens = kPer == 2 || (quarter & 1) == 0;
+          if (p >= t0 && t > 4 && t <= 8 && opens) {  // (of the step before: the swap waits two states for its operands)
+            bwd_operand_rows(pk[t - 5], pk[t - 1]);
+            if (t == 8) to_operands(pk, bqN[b]);
+          }
+          if (p >= t0 && t < 8) {
+            if (opens) convert_first(tr, t, part);
+            if (kPer == 2 || (quarter & 1) == 1) convert_second(nx.s4, t, part, pk);
           }
         }
       };
 #pragma unroll
-      for (int pair = 0; pair < kPairs; ++pair) {
-        const int q = pair / ROWS, rb = pair % ROWS;
-        if (rb < 4) bwd_mfma<true>(acc[rb][0], af[pair & 3], bqC[0][q]);
-        else bwd_mfma<false>(acc[rb][0], af[pair & 3], bqC[0][q]);
-        if (pair + 3 < kPairs) af[(pair + 3) & 3] = panel_frag(i, pair + 3);
-        else if (ahead) af[(pair + 3) & 3] = panel_frag(i + 1, pair + 3 - kPairs);
-        convert_part(pair, 0);
-        __builtin_amdgcn_sched_barrier(0);
-        if (rb < 4) bwd_mfma<true>(acc[rb][1], af[pair & 3], bqC[1][q]);
-        else bwd_mfma<false>(acc[rb][1], af[pair & 3], bqC[1][q]);
-        if (pair % (ROWS / 4) == 0 && pair / (ROWS / 4) < kBwdWideLoads) issue(i + 4, pair / (ROWS / 4));
-        convert_part(pair, 1);
-        if (pair == kT0) bwd_transpose(tr, nx.raw[0], ident);
-        if (pair == kT1) bwd_transpose(tr, nx.raw[1], ident);
-        __builtin_amdgcn_sched_barrier(0);
+      for (int p = 0; p < kRows16; ++p) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          if (p < 8) bwd_mfma<true>(acc[p][j], af[p & 3], bqC[j >> 1][j & 1]);
+          else bwd_mfma<false>(acc[p][j], af[p & 3], bqC[j >> 1][j & 1]);
+          if (j == 0) {
+            if (p + 3 < kRows16) af[(p + 3) & 3] = bwd_panel_frag(panel, p + 3);
+            else af[(p + 3) & 3] = bwd_panel_frag(panel_next, p + 3 - kRows16);
+          }
+          if (p == 0 && j > 0) next_read(st_next, j - 1, nx);
+          if (j == 2 && p % (ROWS / 2) == ROWS / 4 && p / (ROWS / 2) < 4) issue(st_load, p / (ROWS / 2));
+          convert_part(p, j);
+          if (j == 3 && p == kT0) bwd_transpose(tr, nx.raw[0], ident);
+          if (j == 3 && p == kT1) bwd_transpose(tr, nx.raw[1], ident);
+          __builtin_amdgcn_sched_barrier(0);
+        }
       }
     };
 
@@ -1105,12 +1127,13 @@ __global__ __launch_bounds__(256, 1) void bwd_dx_wide_kernel(BwdDxArgs g) {
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int j = 0; j < kBwdWideLoads; ++j) issue(i, j);
+      for (int j = 0; j < 4; ++j) issue(lds_base + (uint32_t)i * kBwdStageBytes, j);
     wait_vmcnt<0>();
     lds_barrier();
     {  // operands of stage 0
       NextRegs nx;
-      next_read(0, nx);
+#pragma unroll
+      for (int part = 0; part < 3; ++part) next_read(lds_base, part, nx);
       uint32_t pk[8];
 #pragma unroll
       for (int cb = 0; cb < 2; ++cb) {
@@ -1118,41 +1141,59 @@ __global__ __launch_bounds__(256, 1) void bwd_dx_wide_kernel(BwdDxArgs g) {
         bwd_transpose(tr, nx.raw[cb], ident);
         asm volatile("s_nop 15\n\ts_nop 15" : "+v"(tr));
 #pragma unroll
-        for (int t = 0; t < 8; ++t) convert2(tr, nx.s4, t, pk);
+        for (int t = 0; t < 8; ++t) {
+          float part[2];
+          convert_first(tr, t, part);
+          convert_second(nx.s4, t, part, pk);
+          if (t >= 4) bwd_operand_rows(pk[t - 4], pk[t]);
+        }
         to_operands(pk, bqA[cb]);
       }
     }
-    // Two stages to a barrier: stages i and i + 1 and the weight of i + 2 have landed, i + 4 and i + 5 are asked for
-    // (into the slots of i - 2 and i - 1).
+    // Two stages to a barrier: stages i, i + 1 and i + 2 have landed, i + 4 and i + 5 are asked for (into the buffers of i - 2
+    // and i - 1).
     // (one loop for all stages: those behind the last are loads and a conversion that nothing reads, and a second loop made
     // the allocator move a third of the sums at every pass of this one)
+#pragma unroll
+    for (int p = 0; p < 3; ++p) af[p] = bwd_panel_frag(panel_at(lds_base), p);
+    uint32_t st_load = lds_base + 4u * kBwdStageBytes, st = lds_base, st_next = lds_base + 2u * kBwdStageBytes;
 #pragma unroll 1
     for (int i = 0; i < L; i += 2) {
       wait_vmcnt<kBwdWideLoads>();
-      lds_barrier();
+      // (the reads in flight are of stage i, whose buffer is filled again two barriers on)
+      asm volatile("s_barrier" ::: "memory");
       __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int p = 0; p < 3; ++p) af[p] = panel_frag(i, p);
-      __builtin_amdgcn_sched_barrier(0);
-      stage(i, bqA, bqB, true, af);
-      stage(i + 1, bqB, bqA, false, af);
+      stage(st, st + kBwdStageBytes, st_load, bqA, bqB, af);
+      stage(st + kBwdStageBytes, st_next, st_load + kBwdStageBytes, bqB, bqA, af);
+      const uint32_t before = st_load;
+      st_load = st; st = st_next; st_next = before;
     }
     wait_vmcnt<0>();
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");  // the last MFMAs, which the compiler does not know, have written their sums
 #pragma unroll
-    for (int rb = 0; rb < ROWS; ++rb)
+    for (int p = 0; p < kRows16; ++p)
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        if (rb < 4) asm volatile("" : "+a"(acc[rb][j]));
-        else asm volatile("" : "+v"(acc[rb][j]));
+      for (int j = 0; j < 4; ++j) {
+        if (p < 8) asm volatile("" : "+a"(acc[p][j]));
+        else asm volatile("" : "+v"(acc[p][j]));
       }
-    auto sums = [&](int rb, v16f& a) -> v16f { return rb < 4 ? bwd_sums<true>(a) : bwd_sums<false>(a); };
+    auto sums = [&](int rb, int cb) -> v16f {
+      v4f b[2][2];
+#pragma unroll
+      for (int rh = 0; rh < 2; ++rh)
+#pragma unroll
+        for (int ch = 0; ch < 2; ++ch) {
+          v4f& a = acc[2 * rb + rh][2 * cb + ch];
+          b[rh][ch] = rb < 4 ? bwd_sums<true>(a) : bwd_sums<false>(a);
+        }
+      return bwd_block32(b);
+    };
     if (whole) {
       lds_barrier();  // (every wave has read its last stage, and nothing is on its way into the LDS)
       const uint32_t rs_lds = lds_base + 4u * kBwdTurnBytes;
       bwd_dx_fetch_rs<NKK>(g, tm * 256u, live_blocks, rs_lds, wave, 4);
       bwd_dx_store<NKK, 2, ROWS, true>(g, tm * 256u, kbw, live_blocks, lds_base + (uint32_t)wave * kBwdTurnBytes, rs_lds,
-                                       [&](int rb, int cb) -> v16f { return sums(rb, acc[rb][cb]); });
+                                       sums);
     } else {
 #pragma unroll
       for (int rb = 0; rb < ROWS; ++rb)
@@ -1160,7 +1201,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dx_wide_kernel(BwdDxArgs g) {
           float4* dst = bwd_dx_part<2>(g, slot, (uint32_t)rb, (uint32_t)wave);
 #pragma unroll
           for (int cb = 0; cb < 2; ++cb) {
-            const v16f y = sums(rb, acc[rb][cb]);
+            const v16f y = sums(rb, cb);
 #pragma unroll
             for (int e = 0; e < 4; ++e) dst[(cb * 4 + e) * 64] = make_float4(y[4 * e], y[4 * e + 1], y[4 * e + 2], y[4 * e + 3]);
           }

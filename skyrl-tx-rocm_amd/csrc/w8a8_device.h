@@ -100,6 +100,12 @@ __device__ inline uint32_t code_bytes4(const float (&q)[4]) {
 }
 __device__ inline bool code_scale_ordinary(float scale) { return scale > 1e-30f && scale < 1e30f; }
 
+// f(integral_constant 0), f(1), ..: an unrolled loop whose index is a constant expression.
+template <class F, int... S>
+__device__ inline __attribute__((always_inline)) void each_of(F&& f, std::integer_sequence<int, S...>) {
+  (f(std::integral_constant<int, S>{}), ...);
+}
+
 // One step of a butterfly over the wave: op(v, the value of lane ^ O) for an op that commutes, without the LDS.  Rows of 16
 // and halves of 32 change places by the permlane swaps, which leave both operands in every lane; below that the data
 // parallel moves carry the value (lane ^ 4 as reversed quads in a reversed half row).  __shfl_xor goes through the LDS pipe,
@@ -174,10 +180,6 @@ typedef __attribute__((address_space(3))) void* lptr_t;
 __device__ inline void load_1k_to_lds(const unsigned char* src_lane, unsigned char* lds_dst_uniform) {
   __builtin_amdgcn_global_load_lds((gptr_t)src_lane, (lptr_t)lds_dst_uniform, 16, 0, 0);
 }
-// ... for data that is read once (non-temporal)
-__device__ inline void load_1k_to_lds_once(const unsigned char* src_lane, unsigned char* lds_dst_uniform) {
-  __builtin_amdgcn_global_load_lds((gptr_t)src_lane, (lptr_t)lds_dst_uniform, 16, 0, 2);
-}
 // A gather of 64 dwords by one wave: lane l moves 4 bytes global[base + voff] (voff a multiple of 4, any
 // place) -> LDS[lds_addr_uniform + 4 l].
 __device__ inline void lds_gather_dword(const void* base_uniform, uint32_t voff, uint32_t lds_addr_uniform) {
@@ -191,6 +193,21 @@ __device__ inline void lds_gather_dword(const void* base_uniform, uint32_t voff,
 __device__ inline void lds_load_1k(const unsigned char* base_uniform, uint32_t voff, uint32_t lds_addr_uniform) {
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
                :: "v"(voff), "s"(base_uniform), "s"(lds_addr_uniform) : "memory", "m0");
+}
+// two KiB, one behind the other at both ends (an instruction's offset counts for the LDS as well) ...
+__device__ inline void lds_load_2k(const unsigned char* base_uniform, uint32_t voff, uint32_t lds_addr_uniform) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1\n\tglobal_load_lds_dwordx4 %0, %1 offset:1024"
+               :: "v"(voff), "s"(base_uniform), "s"(lds_addr_uniform) : "memory", "m0");
+}
+// ... the second from second_uniform + 1024; for data that is read once (non-temporal)
+template <bool ONCE>
+__device__ inline void lds_load_2k(const unsigned char* base_uniform, const unsigned char* second_uniform, uint32_t voff, uint32_t lds_addr_uniform) {
+  if constexpr (ONCE)
+    asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt\n\tglobal_load_lds_dwordx4 %0, %2 offset:1024 nt"
+                 :: "v"(voff), "s"(base_uniform), "s"(second_uniform), "s"(lds_addr_uniform) : "memory", "m0");
+  else
+    asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1\n\tglobal_load_lds_dwordx4 %0, %2 offset:1024"
+                 :: "v"(voff), "s"(base_uniform), "s"(second_uniform), "s"(lds_addr_uniform) : "memory", "m0");
 }
 __device__ inline void lds_load_1k_once(const unsigned char* base_uniform, uint32_t voff, uint32_t lds_addr_uniform) {
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt"

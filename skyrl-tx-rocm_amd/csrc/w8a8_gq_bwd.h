@@ -85,14 +85,14 @@ __global__ __launch_bounds__(256) void gq_bwd_pack_dy_kernel(BwdPackDyArgs a) {
 
 // ---------------------------------------------------------------------------------------
 // The pull-back.  Workgroup = 4 waves side by side along k, one to a SIMD, tile 256 rows x 128 k, wave tile 256 x 32
-// (8 accumulator blocks of v_mfma_f32_32x32x16_bf16), contraction in stages of one 32-wide n block.  A stage's
+// (16 x 2 accumulator blocks of v_mfma_f32_16x16x32_bf16), contraction in stages of one 32-wide n block.  A stage's
 // dy panel (16 KiB), its four weight blocks (4 KiB, half that in 4-bit codes) and their scales (128 bytes a block)
 // travel L2 -> LDS with direct-to-LDS loads four stages ahead, six per wave.  While the matrix core works on
 // a stage, each wave prepares its weight block of the next: transposed by the identity MFMA, scaled in float32,
 // split into TERMS bf16 operands.  The order of things is bwd_dx_wide_kernel's; two row blocks take turns so that the terms'
 // MFMAs on one accumulator do not follow each other.
 // Bound by the matrix core and the term arithmetic beside it: 1536 rows, K = 12288, N = 4096, 8-bit codes, groups of
-// 64, two terms: 277 us, 1.12 PFLOP/s of bf16 products (as eight waves of 128 x 32, every two of which converted the same blocks, 322-337 us; the float32 library
+// 64, two terms: 276 us, 1.12 PFLOP/s of bf16 products (282 with 32x32x16 and the loads' addresses formed anew for every stage; as eight waves of 128 x 32, every two of which converted the same blocks, 322-337 us; the float32 library
 // GEMM took 1096 us and the dequantization and casts before it 250).
 // ---------------------------------------------------------------------------------------
 constexpr int kGqBwdStages = 6;
@@ -134,8 +134,8 @@ __global__ __launch_bounds__(256, 1) void gq_bwd_dx_wide_kernel(GqBwdDxArgs a) {
     const uint32_t lane16 = (uint32_t)lane_s * 16u, h = (uint32_t)lane_s >> 5;
     const uint32_t rb0 = 2u * (uint32_t)wave < (uint32_t)live_blocks ? 2u * (uint32_t)wave : 0u;
     const uint32_t rb1 = 2u * (uint32_t)wave + 1u < (uint32_t)live_blocks ? 2u * (uint32_t)wave + 1u : 0u;
-    const unsigned char* Ag0 = g.dyp + ((size_t)(tm * 8u + rb0) * g.NB) * 2048u;
-    const unsigned char* Ag1 = g.dyp + ((size_t)(tm * 8u + rb1) * g.NB) * 2048u;
+    const unsigned char* const Ag0 = g.dyp + ((size_t)(tm * 8u + rb0) * g.NB + (uint32_t)nb0) * 2048u;
+    const unsigned char* const Ag1 = g.dyp + ((size_t)(tm * 8u + rb1) * g.NB + (uint32_t)nb0) * 2048u;
     const uint32_t kb0 = tk * 4u;
     auto clamp_kb = [&](uint32_t kb) { return kb < g.KB ? kb : g.KB - 1u; };
     // its chunk of the weight blocks: one of four, or in 4-bit codes two of 512 bytes (waves 2 and 3 repeating 0 and 1)
@@ -145,116 +145,147 @@ __global__ __launch_bounds__(256, 1) void gq_bwd_dx_wide_kernel(GqBwdDxArgs a) {
     // the four blocks' scales, by each wave to the same place
     const uint32_t s_piece = ((uint32_t)lane_s & 7u) * 4u;
     const uint32_t s_row = clamp_kb(kb0 + (((uint32_t)lane_s >> 3) & 3u)) * 32u / a.group * a.N;
-    auto issue = [&](int i, int j) {  // load j of the six of stage i (behind the last stage: of that one again)
-      const uint32_t st = lds_base + (uint32_t)(i % kGqBwdStages) * kGqBwdStageBytes;
-      const uint32_t nb = (uint32_t)(nb0 + (i < L ? i : L - 1));
-      if (j < 4) {
-        lds_load_1k((j < 2 ? Ag0 : Ag1) + (size_t)nb * 2048u + 1024 * (j & 1), lane16, st + (uint32_t)(wave * 4 + j) * kBlockBytes);
-      } else if (j == 4) {
-        const uint32_t nbw = nb < a.weight_nb ? nb : a.weight_nb - 1u;  // (dy is zero beyond the last column)
-        lds_load_1k(g.wp + (size_t)nbw * g.KB * kBlk8, w_off, st + kGqBwdPanel + w_dst);
-      } else {
-        const uint32_t n = nb * 32u + s_piece;
-        lds_load_1k(reinterpret_cast<const unsigned char*>(a.ws), (s_row + (n < a.N ? n : 0u)) * 4u, st + kGqBwdPanel + kGqBwdWeight);
+    const size_t w_stride = (size_t)g.KB * kBlk8;
+    const unsigned char* Wg = g.wp + (size_t)nb0 * w_stride;
+    uint32_t a_off = lane16, s_col = (uint32_t)nb0 * 32u + s_piece;
+    int nb_load = nb0;
+    // Part j of four of the loads of the next stage to be asked for, into the stage buffer at st (behind the last stage: of that
+    // one again).  The addresses go on from stage to stage: see bwd_dx_wide_kernel.
+    auto issue = [&](uint32_t st, int j) {
+      if (j == 0) lds_load_2k(Ag0, a_off, st + (uint32_t)wave * 4096u);
+      else if (j == 1) lds_load_2k(Ag1, a_off, st + (uint32_t)wave * 4096u + 2048u);
+      else if (j == 2) lds_load_1k(Wg, w_off, st + kGqBwdPanel + w_dst);
+      else {
+        lds_load_1k(reinterpret_cast<const unsigned char*>(a.ws), (s_row + (s_col < a.N ? s_col : 0u)) * 4u, st + kGqBwdPanel + kGqBwdWeight);
+        const bool more = nb_load + 1 < nb0 + L;
+        nb_load += more ? 1 : 0;
+        a_off += more ? 2048u : 0u;
+        s_col += more ? 32u : 0u;
+        // (the weight's last block again beyond it: dy is zero there)
+        Wg += more && (uint32_t)nb_load < a.weight_nb ? w_stride : 0;
       }
     };
-    v16f acc[ROWS];
+    constexpr int kRows16 = 2 * ROWS;  // row blocks of 16
+    v4f acc[kRows16][2];
 #pragma unroll
-    for (int i = 0; i < ROWS; ++i)
+    for (int i = 0; i < kRows16; ++i)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][e] = 0.0f;
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[i][j][e] = 0.0f;
 
-    // (the wait stands in the same block, so no register is handed out before it is filled)
     struct NextRegs { v4i raw; v4f s4[4]; };
-    auto next_read = [&](int i, NextRegs& r) {
-      const uint32_t st = lds_base + (uint32_t)(i % kGqBwdStages) * kGqBwdStageBytes + kGqBwdPanel;
-      const uint32_t sa = st + kGqBwdWeight + (uint32_t)wave * 128u + 16u * h;
+    const uint32_t weight_off = W4 ? (uint32_t)wave * 512u + lane16 / 2u : (uint32_t)wave * 1024u + lane16;
+    // The weight block and scales of the stage at st, in three parts.  (Reads that the compiler waits for where they are used.)
+    auto next_read = [&](uint32_t st, int part, NextRegs& r) {
+      if (part == 0) {
+        uint32_t wa = st + weight_off;
+        asm volatile("" : "+v"(wa));
+        if constexpr (W4) {
+          typedef int v2i __attribute__((ext_vector_type(2)));
+          typedef __attribute__((address_space(3))) const v2i* lds_v2ptr;
+          const v2i raw = *reinterpret_cast<lds_v2ptr>((uintptr_t)(wa + kGqBwdPanel));
+          r.raw[0] = raw[0]; r.raw[1] = raw[1];
+        } else {
+          typedef __attribute__((address_space(3))) const v4i* lds_v4ptr;
+          r.raw = *reinterpret_cast<lds_v4ptr>((uintptr_t)(wa + kGqBwdPanel));
+        }
+      } else {
+        typedef __attribute__((address_space(3))) const v4i* lds_v4ptr;
+        uint32_t sa = st + (uint32_t)wave * 128u + 16u * h;
+        asm volatile("" : "+v"(sa));
+#pragma unroll
+        for (int q = 2 * part - 2; q < 2 * part; ++q)
+          r.s4[q] = __builtin_bit_cast(v4f, *reinterpret_cast<lds_v4ptr>((uintptr_t)(sa + kGqBwdPanel + kGqBwdWeight + 32 * q)));
+      }
+    };
+    auto next_expand = [&](NextRegs& r) {  // 4-bit codes to 16 * code; the scale takes the exact 1 / 16 (convert_part)
       if constexpr (W4) {
-        const uint32_t wa = st + (uint32_t)wave * 512u + lane16 / 2u;
-        uint2 raw;
-        asm volatile("ds_read_b64 %0, %5\n\tds_read_b128 %1, %6\n\tds_read_b128 %2, %6 offset:32\n\t"
-                     "ds_read_b128 %3, %6 offset:64\n\tds_read_b128 %4, %6 offset:96\n\ts_waitcnt lgkmcnt(0)"
-                     : "=&v"(raw), "=&v"(r.s4[0]), "=&v"(r.s4[1]), "=&v"(r.s4[2]), "=&v"(r.s4[3])
-                     : "v"(wa), "v"(sa) : "memory");
         GqRawFragment<true> f;
-        f.v = make_uint4(raw.x, raw.y, 0u, 0u);
-        r.raw = gq_expand<true>(f);  // 16 * code; the scale takes the exact 1 / 16
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) r.s4[q][e] = r.s4[q][e] * 0.0625f;
+        f.v = make_uint4((uint32_t)r.raw[0], (uint32_t)r.raw[1], 0u, 0u);
+        r.raw = gq_expand<true>(f);
         // (the transposing MFMA is assembly: without wait states behind the vector ALU's write it read the last register of the
         // operand before it was written)
         asm volatile("s_nop 3" : "+v"(r.raw));
-      } else {
-        const uint32_t wa = st + (uint32_t)wave * 1024u + lane16;
-        asm volatile("ds_read_b128 %0, %5\n\tds_read_b128 %1, %6\n\tds_read_b128 %2, %6 offset:32\n\t"
-                     "ds_read_b128 %3, %6 offset:64\n\tds_read_b128 %4, %6 offset:96\n\ts_waitcnt lgkmcnt(0)"
-                     : "=&v"(r.raw), "=&v"(r.s4[0]), "=&v"(r.s4[1]), "=&v"(r.s4[2]), "=&v"(r.s4[3])
-                     : "v"(wa), "v"(sa) : "memory");
       }
     };
     // rows 8 (t / 2) + 4 h + 2 (t % 2) + 0, 1 of a transposed block: code * scale in float32, split into TERMS bf16 values
-    auto convert2 = [&](const v16i& tr, const v4f (&s4)[4], int t, uint32_t (&pk)[TERMS][8]) {
-      float f0 = (float)tr[2 * t] * s4[t >> 1][2 * (t & 1)], f1 = (float)tr[2 * t + 1] * s4[t >> 1][2 * (t & 1) + 1];
-#pragma unroll
-      for (int u = 0; u < TERMS; ++u) {
-        const uint32_t w = pack_bf16x2(f0, f1);
-        pk[u][t] = w;
-        if (u + 1 < TERMS) {
-          f0 = f0 - __uint_as_float(w << 16);
-          f1 = f1 - __uint_as_float(w & 0xffff0000u);
-        }
+    // (step t in 3 * TERMS parts, which stand between different MFMAs)
+    constexpr int kParts = 3 * TERMS;
+    auto convert_part = [&](const v16i& tr, const v4f (&s4)[4], int t, int part, float (&f)[2], uint32_t (&pk)[TERMS][8]) {
+      const int u = part / 3;
+      if (part == 0) {
+        f[0] = (float)tr[2 * t]; f[1] = (float)tr[2 * t + 1];
+      } else if (part == 1) {
+        constexpr float kUnit = W4 ? 0.0625f : 1.0f;
+        f[0] = f[0] * (s4[t >> 1][2 * (t & 1)] * kUnit); f[1] = f[1] * (s4[t >> 1][2 * (t & 1) + 1] * kUnit);
+      } else if (part % 3 == 0) {
+        f[0] = f[0] - __uint_as_float(pk[u - 1][t] << 16);
+      } else if (part % 3 == 1) {
+        f[1] = f[1] - __uint_as_float(pk[u - 1][t] & 0xffff0000u);
+      } else {
+        pk[u][t] = pack_bf16x2(f[0], f[1]);
       }
+    };
+    auto operand_rows = [&](int t, uint32_t (&pk)[TERMS][8]) {  // behind step t >= 4
+#pragma unroll
+      for (int v = 0; v < TERMS; ++v) bwd_operand_rows(pk[v][t - 4], pk[v][t]);
     };
     auto to_operands = [&](const uint32_t (&pk)[TERMS][8], v8bf (&bq)[2][TERMS]) {
 #pragma unroll
       for (int t = 0; t < TERMS; ++t)
 #pragma unroll
-        for (int q = 0; q < 2; ++q)
-          bq[q][t] = __builtin_bit_cast(v8bf, v4i{(int)pk[t][4 * q], (int)pk[t][4 * q + 1], (int)pk[t][4 * q + 2], (int)pk[t][4 * q + 3]});
+        for (int j = 0; j < 2; ++j)
+          bq[j][t] = __builtin_bit_cast(v8bf, v4i{(int)pk[t][4 * j], (int)pk[t][4 * j + 1], (int)pk[t][4 * j + 2], (int)pk[t][4 * j + 3]});
     };
-    constexpr int kPairs = 2 * ROWS;  // (half q, row block) of a stage
-    auto panel_frag = [&](int i, int pair) -> v8bf {
-      typedef __attribute__((address_space(3))) const v4i* lds_v4ptr;
-      const uint32_t at = lds_base + (uint32_t)(i % kGqBwdStages) * kGqBwdStageBytes + lane16;
-      return __builtin_bit_cast(v8bf, *reinterpret_cast<lds_v4ptr>((uintptr_t)(at + (uint32_t)((pair % ROWS) * 2 + pair / ROWS) * kBlockBytes)));
+    const uint32_t frag_off = bwd_frag_offset((uint32_t)lane_s);
+    auto panel_at = [&](uint32_t st) -> uint32_t {
+      uint32_t at = st + frag_off;
+      asm volatile("" : "+v"(at));  // (opaque: the rows' offsets are the instructions', not sixteen registers)
+      return at;
     };
-    // One stage: its MFMAs from the dy panel in the LDS, two row blocks at a time, small terms first; between them the operands
-    // of stage i + 1 are prepared.  af: the fragments of the first two pairs; leaves those of stage i + 1 there where that one
-    // has landed (ahead).
-    auto stage = [&](int i, const v8bf (&bqC)[2][TERMS], v8bf (&bqN)[2][TERMS], bool ahead, v8bf (&af)[4]) {
-      constexpr int kSlots = kPairs * TERMS;  // MFMAs
-      constexpr int kFirst = 5, kGap = (kSlots - 6) / 8;  // where the eight conversion steps stand: four MFMAs behind the transposing one
-      static_assert(kFirst + 7 * kGap < kSlots, "the conversion ends inside the stage");
+    // One stage, at st: its MFMAs from the dy panel in the LDS, two blocks of 16 rows at a time, small terms first; between them
+    // the operands of the stage at st_next are prepared and the loads of the one at st_load are issued.  af: the fragments of
+    // the first two blocks; leaves the next stage's.
+    auto stage = [&](uint32_t st, uint32_t st_next, uint32_t st_load, const v8bf (&bqC)[2][TERMS], v8bf (&bqN)[2][TERMS], v8bf (&af)[4]) {
+      constexpr int kSlots = kRows16 * TERMS * 2;  // MFMAs
+      // the transposing one stands behind kTurn, where its operand has come from the LDS; from kFirst on, five behind it, the
+      // eight conversion steps
+      constexpr int kTurn = ROWS == 8 ? 7 : 3, kFirst = kTurn + 5, kGap = (kSlots - kFirst - 1) / 8;
+      static_assert(kGap > 0 && kFirst + 8 * kGap < kSlots, "the conversion ends inside the stage");
       NextRegs nx;
       v16i tr;
       uint32_t pk[TERMS][8];
+      float cf[2];
       asm volatile("s_nop 3");  // (operands converted at the end of the stage before)
-      next_read(i + 1, nx);
+      const uint32_t panel = panel_at(st), panel_next = panel_at(st_next);
+      auto slot = [&](auto at_slot) __attribute__((always_inline)) {
+        constexpr int sl = decltype(at_slot)::value;
+        constexpr int p = sl / (4 * TERMS) * 2, t = TERMS - 1 - sl / 4 % TERMS, u = sl / 2 % 2, j = sl % 2;
+        bwd_mfma<true>(acc[p + u][j], af[(p + u) & 3], bqC[j][t]);
+        if constexpr (t == TERMS - 1 && j == 0) {  // the next two blocks' fragments
+          if constexpr (p + 2 < kRows16) af[(p + 2 + u) & 3] = bwd_panel_frag(panel, p + 2 + u);
+          else af[(p + 2 + u) & 3] = bwd_panel_frag(panel_next, u);
+        }
+        if constexpr (sl == 1 || sl == 2 || sl == 3) next_read(st_next, sl - 1, nx);
+        if constexpr (sl == kTurn) {
+          next_expand(nx);
+          bwd_transpose(tr, nx.raw, ident);
+        }
+        if constexpr (sl == kFirst) asm volatile("" : "+v"(tr));  // (not read before this place)
+        if constexpr (sl >= kFirst && (sl - kFirst) % kGap == 0 && (sl - kFirst) / kGap > 4 && (sl - kFirst) / kGap <= 8) {
+          operand_rows((sl - kFirst) / kGap - 1, pk);
+          if constexpr ((sl - kFirst) / kGap == 8) to_operands(pk, bqN);
+        }
+        if constexpr (sl >= kFirst && sl < kFirst + 8 * kGap) {
+          constexpr int step = (sl - kFirst) / kGap, at = (sl - kFirst) % kGap;
 #pragma unroll
-      for (int p = 0; p < kPairs; p += 2) {
-        const int q = p / ROWS, rb = p % ROWS;
-#pragma unroll
-        for (int t = TERMS - 1; t >= 0; --t)
-#pragma unroll
-          for (int u = 0; u < 2; ++u) {
-            const int sl = p * TERMS + (TERMS - 1 - t) * 2 + u;
-            bwd_mfma<true>(acc[rb + u], af[(p + u) & 3], bqC[q][t]);
-            if (t == TERMS - 1) {  // the next two pairs' fragments
-              if (p + 2 < kPairs) af[(p + 2 + u) & 3] = panel_frag(i, p + 2 + u);
-              else if (ahead) af[(p + 2 + u) & 3] = panel_frag(i + 1, u);
-            }
-            if (sl == 0) bwd_transpose(tr, nx.raw, ident);
-            if (sl == kFirst) asm volatile("" : "+v"(tr));  // (not read before this place)
-            if (sl >= kFirst && (sl - kFirst) % kGap == 0 && (sl - kFirst) / kGap < 8) {
-              convert2(tr, nx.s4, (sl - kFirst) / kGap, pk);
-              if ((sl - kFirst) / kGap == 7) to_operands(pk, bqN);
-            }
-            if (sl % (kSlots / 8) == 1 && sl / (kSlots / 8) < kGqBwdLoads) issue(i + 4, sl / (kSlots / 8));
-            __builtin_amdgcn_sched_barrier(0);
-          }
-      }
+          for (int part = at * kParts / kGap; part < (at + 1) * kParts / kGap; ++part) convert_part(tr, nx.s4, step, part, cf, pk);
+        }
+        if constexpr (sl % (kSlots / 4) == kSlots / 8 && sl / (kSlots / 4) < 4) issue(st_load, sl / (kSlots / 4));
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      each_of(slot, std::make_integer_sequence<int, kSlots>{});
     };
 
     v8bf bqA[2][TERMS], bqB[2][TERMS], af[4];
@@ -263,37 +294,57 @@ __global__ __launch_bounds__(256, 1) void gq_bwd_dx_wide_kernel(GqBwdDxArgs a) {
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int j = 0; j < kGqBwdLoads; ++j) issue(i, j);
+      for (int j = 0; j < 4; ++j) issue(lds_base + (uint32_t)i * kGqBwdStageBytes, j);
     wait_vmcnt<0>();
     lds_barrier();
     {  // operands of stage 0
       NextRegs nx;
-      next_read(0, nx);
+#pragma unroll
+      for (int part = 0; part < 3; ++part) next_read(lds_base, part, nx);
+      next_expand(nx);
       uint32_t pk[TERMS][8];
       v16i tr;
       bwd_transpose(tr, nx.raw, ident);
       asm volatile("s_nop 15\n\ts_nop 15" : "+v"(tr));
 #pragma unroll
-      for (int t = 0; t < 8; ++t) convert2(tr, nx.s4, t, pk);
+      for (int t = 0; t < 8; ++t) {
+        float cf[2];
+#pragma unroll
+        for (int part = 0; part < kParts; ++part) convert_part(tr, nx.s4, t, part, cf, pk);
+        if (t >= 4) operand_rows(t, pk);
+      }
       to_operands(pk, bqA);
     }
-    // Two stages to a barrier: stages i and i + 1 and the weight of i + 2 have landed, i + 4 and i + 5 are asked for
-    // (into the slots of i - 2 and i - 1).
+    // Two stages to a barrier: stages i, i + 1 and i + 2 have landed, i + 4 and i + 5 are asked for (into the buffers of i - 2
+    // and i - 1).
+#pragma unroll
+    for (int p = 0; p < 2; ++p) af[p] = bwd_panel_frag(panel_at(lds_base), p);
+    uint32_t st_load = lds_base + 4u * kGqBwdStageBytes, st = lds_base, st_next = lds_base + 2u * kGqBwdStageBytes;
 #pragma unroll 1
     for (int i = 0; i < L; i += 2) {
       wait_vmcnt<kGqBwdLoads>();
-      lds_barrier();
+      // (the reads in flight are of stage i, whose buffer is filled again two barriers on)
+      asm volatile("s_barrier" ::: "memory");
       __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int p = 0; p < 2; ++p) af[p] = panel_frag(i, p);
-      __builtin_amdgcn_sched_barrier(0);
-      stage(i, bqA, bqB, true, af);
-      stage(i + 1, bqB, bqA, false, af);
+      stage(st, st + kGqBwdStageBytes, st_load, bqA, bqB, af);
+      stage(st + kGqBwdStageBytes, st_next, st_load + kGqBwdStageBytes, bqB, bqA, af);
+      const uint32_t before = st_load;
+      st_load = st; st = st_next; st_next = before;
     }
     wait_vmcnt<0>();
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");  // the last MFMAs, which the compiler does not know, have written their sums
 #pragma unroll
-    for (int rb = 0; rb < ROWS; ++rb) asm volatile("" : "+a"(acc[rb]));
+    for (int p = 0; p < kRows16; ++p)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) asm volatile("" : "+a"(acc[p][j]));
+    auto sums = [&](int rb, int) -> v16f {
+      v4f b[2][2];
+#pragma unroll
+      for (int rh = 0; rh < 2; ++rh)
+#pragma unroll
+        for (int ch = 0; ch < 2; ++ch) b[rh][ch] = bwd_sums<true>(acc[2 * rb + rh][ch]);
+      return bwd_block32(b);
+    };
 
     const uint32_t kbw = kb0 + (uint32_t)wave;
     if (whole) {
@@ -301,13 +352,13 @@ __global__ __launch_bounds__(256, 1) void gq_bwd_dx_wide_kernel(GqBwdDxArgs a) {
       const uint32_t rs_lds = lds_base + 4u * kBwdTurnBytes;
       bwd_dx_fetch_rs<NKK>(g, tm * 256u, live_blocks, rs_lds, wave, 4);
       bwd_dx_store<NKK, 1, ROWS, true>(g, tm * 256u, kbw, live_blocks, lds_base + (uint32_t)wave * kBwdTurnBytes, rs_lds,
-                                       [&](int rb, int) -> v16f { return bwd_sums<true>(acc[rb]); });
+                                       sums);
     } else {
 #pragma unroll
       for (int rb = 0; rb < ROWS; ++rb)
         if (rb < live_blocks) {
           float4* dst = bwd_dx_part<1>(g, slot, (uint32_t)rb, (uint32_t)wave);
-          const v16f y = bwd_sums<true>(acc[rb]);
+          const v16f y = sums(rb, 0);
 #pragma unroll
           for (int e = 0; e < 4; ++e) dst[e * 64] = make_float4(y[4 * e], y[4 * e + 1], y[4 * e + 2], y[4 * e + 3]);
         }
