@@ -391,8 +391,9 @@ __device__ inline void route_weight_groups_block(const int32_t* __restrict__ gro
   const uint32_t tid = threadIdx.x;
   int32_t sz = tid < n_groups ? group_sizes[tid] : 0;
   if (sz < 0) sz = 0;
-  uint32_t rows_total, slots_total, chunks_total;
-  const uint32_t r0 = block_prefix_capped((uint32_t)sz, M, &rows_total);
+  uint32_t row[1] = {(uint32_t)sz}, rows_of_all[1];
+  block_prefix_capped(row, M, rows_of_all);
+  const uint32_t r0 = row[0], rows_total = rows_of_all[0];
   const uint32_t r1 = (uint64_t)r0 + (uint32_t)sz > M ? M : r0 + (uint32_t)sz;
   const uint32_t rows = r1 - r0;
   if (tid < n_groups) { row_start[tid] = r0; last_group[tid] = (int)tid; }
@@ -401,11 +402,13 @@ __device__ inline void route_weight_groups_block(const int32_t* __restrict__ gro
   const uint32_t g0 = tid / gpw * gpw;  // first group of this one's weight
   const bool heads = tid < n_groups && g0 == tid;
   const uint32_t weight_rows = heads ? row_start[tid + gpw] - r0 : 0u;
-  const uint32_t wbeg = block_prefix_capped((weight_rows + tile_rows - 1u) / tile_rows * tile_rows, 0xffffffffu, &slots_total);
-  if (heads) weight_slot[tid] = wbeg;
-  if (tid < n_groups && rows) atomicMax(&last_group[g0], (int)tid);
   const uint32_t n_chunks = (rows + kBwdChunkRows - 1u) / kBwdChunkRows;
-  const uint32_t c0 = block_prefix_capped(n_chunks, 0xffffffffu, &chunks_total);  // (its barriers stand behind the tables above)
+  uint32_t place[2] = {(weight_rows + tile_rows - 1u) / tile_rows * tile_rows, n_chunks}, all[2];
+  block_prefix_capped(place, 0xffffffffu, all);
+  const uint32_t slots_total = all[0], c0 = place[1], chunks_total = all[1];
+  if (heads) weight_slot[tid] = place[0];
+  if (tid < n_groups && rows) atomicMax(&last_group[g0], (int)tid);
+  __syncthreads();
   const uint32_t p0 = tid < n_groups ? weight_slot[g0] + (r0 - row_start[g0]) : 0u;
   if (tid < n_groups) slot_beg[tid] = p0;
   __syncthreads();
@@ -1298,12 +1301,7 @@ __device__ inline void bwd_find_chunk(const int32_t* group_off, uint32_t n_group
     const uint32_t g = g0 + lane < n_groups ? g0 + lane : n_groups;
     const uint32_t o0 = (uint32_t)group_off[g], o1 = (uint32_t)group_off[g < n_groups ? g + 1u : g];
     const uint32_t nch = (o1 - o0 + kBwdChunkRows - 1u) / kBwdChunkRows;
-    uint32_t upto = nch;  // of this and the lanes below
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const uint32_t v = (uint32_t)__shfl_up((int)upto, d);
-      upto += lane >= (uint32_t)d ? v : 0u;
-    }
+    const uint32_t upto = wave_scan(nch);  // of this and the lanes below
     const uint64_t reached = __builtin_amdgcn_ballot_w64(cid < run + upto);
     if (reached) {
       const int own = __builtin_ctzll(reached);
@@ -1628,11 +1626,7 @@ __global__ __launch_bounds__(256) void bwd_dlora_reduce_kernel(BwdReduceArgs a, 
     uint32_t cnt = 0;
     if (tid < a.n_groups)
       cnt = ((uint32_t)(a.group_off[tid + 1] - a.group_off[tid]) + kBwdChunkRows - 1u) / kBwdChunkRows;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const uint32_t up = (uint32_t)__shfl_up((int)cnt, o, 64);
-      if ((int)tid >= o) cnt += up;
-    }
+    cnt = wave_scan(cnt);
     if (tid < a.n_groups) chunk0_lds[tid + 1u] = cnt;  // inclusive sums
     if (tid == 0) chunk0_lds[0] = 0u;
   }

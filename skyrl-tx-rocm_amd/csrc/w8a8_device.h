@@ -159,6 +159,21 @@ __device__ inline int wave_min(int v) { return wave_fold(v, [](int a, int b) { r
 template <typename T>
 __device__ inline T wave_sum(T v) { return wave_fold(v, [](T a, T b) { return a + b; }); }
 
+// Inclusive scan of values with identity 0 over the wave, in data parallel moves as above: inside the rows of 16, then the last
+// lane of a row to the next, then lane 31 to the upper half.
+template <typename Op>
+__device__ inline uint32_t wave_scan(uint32_t v, Op op) {
+  v = op(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false));  // row_shr:1, 2, 4, 8
+  v = op(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false));
+  v = op(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false));
+  v = op(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false));
+  v = op(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false));  // row_bcast:15
+  return op(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false));  // row_bcast:31
+}
+__device__ inline uint32_t wave_scan(uint32_t v) { return wave_scan(v, [](uint32_t a, uint32_t b) { return a + b; }); }
+// the value of the lane before, 0 in lane 0
+__device__ inline uint32_t lane_before(uint32_t v) { return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x138, 0xf, 0xf, false); }
+
 // s_waitcnt vmcnt(N) only (gfx9 encoding: vmcnt[3:0]|[15:14], expcnt[6:4], lgkmcnt[11:8])
 template <int N>
 __device__ inline void wait_vmcnt() {

@@ -252,7 +252,11 @@ __device__ inline void moe_scatter_chunk(const MoeSortArgs& a, uint32_t chunk, F
   __syncthreads();
   if (valid) {
     uint32_t before = 0;
-    for (uint32_t w = 0; w < wave; ++w) before += wave_cnt[w][g];
+#pragma unroll
+    for (uint32_t w = 0; w < 16; ++w) {  // (all reads at once)
+      const uint32_t n = wave_cnt[w][g];
+      before += w < wave ? n : 0u;
+    }
     const int pos = first_of(g) + (int)before + (int)rank;
     a.sort_indices[pos] = (int)p;
     a.unsort_indices[p] = pos;
@@ -288,10 +292,10 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(MoeSortArgs a) {
   }
   __syncthreads();
   const uint32_t n = all[tid];
-  uint32_t total;
-  const uint32_t start = block_prefix_capped(n, 0xffffffffu, &total);
+  uint32_t start[1] = {n}, total[1];
+  block_prefix_capped(start, 0xffffffffu, total);
   if (chunk == 0 && tid < a.G) a.group_sizes[tid] = (int)n;
-  all[tid] = start + earlier[tid];  // (read again behind a barrier)
+  all[tid] = start[0] + earlier[tid];  // (read again behind a barrier)
   moe_scatter_chunk(a, chunk, [&](uint32_t g) { return (int)all[g]; });
 }
 
