@@ -138,6 +138,12 @@ typedef struct mi355_w8a8_problem {
   int32_t* aux_acc;         /* int32 [m, n] raw integer accumulators */
   void* aux_normalized;     /* bf16 [m, k] RMSNorm output (only with rms_gamma) */
 } mi355_w8a8_problem;
+/* The same call with struct_size = sizeof of this: it leaves x @ A[idx], which the backward contracts with dy.  Taken where
+ * mi355_w8a8_forward_keeps_z says so. */
+typedef struct mi355_w8a8_problem_z {
+  mi355_w8a8_problem call;
+  float* z;                 /* f32 [m, rank] */
+} mi355_w8a8_problem_z;
 
 /*
  * Grouped (ragged) call: rows of x are already sorted by group (expert); group g owns
@@ -177,6 +183,10 @@ typedef struct mi355_w8a8_grouped_problem {
   uint32_t x_row_repeat;    /* >= 1 with a map */
   uint32_t x_rows;          /* rows of x with a map; 0 = ceil(m / x_row_repeat), one row per token */
 } mi355_w8a8_grouped_problem;
+typedef struct mi355_w8a8_grouped_problem_z { /* as mi355_w8a8_problem_z; every call with LoRA */
+  mi355_w8a8_grouped_problem call;
+  float* z;                 /* f32 [m, rank], rows as sorted; rows beyond sum(group_sizes) are not written */
+} mi355_w8a8_grouped_problem_z;
 
 /*
  * Backward of the plain W8A8 LoRA linear (no RMSNorm / SwiGLU / residual stage):
@@ -209,6 +219,10 @@ typedef struct mi355_w8a8_bwd_problem {
   void* workspace;          /* >= mi355_w8a8_bwd_workspace_bytes(...) bytes, 256-byte aligned */
   uint64_t workspace_bytes;
 } mi355_w8a8_bwd_problem;
+typedef struct mi355_w8a8_bwd_problem_z { /* the same call with the forward's x @ A[idx], which it otherwise forms again */
+  mi355_w8a8_bwd_problem call;
+  const float* z;           /* f32 [m, rank] */
+} mi355_w8a8_bwd_problem_z;
 
 /*
  * Backward of the grouped call (plain epilogue): rows of x and dy are sorted by group as in the
@@ -244,6 +258,10 @@ typedef struct mi355_w8a8_grouped_bwd_problem {
   uint32_t x_row_repeat;    /* >= 1 with a map */
   uint32_t x_rows;          /* rows of x with a map; 0 = ceil(m / x_row_repeat) */
 } mi355_w8a8_grouped_bwd_problem;
+typedef struct mi355_w8a8_grouped_bwd_problem_z {
+  mi355_w8a8_grouped_bwd_problem call;
+  const float* z;           /* f32 [m, rank], rows as sorted */
+} mi355_w8a8_grouped_bwd_problem_z;
 
 /*
  * Qwen3.5 attention input stage behind the fused QKV projection: split of the interleaved
@@ -362,6 +380,9 @@ int mi355_w8a8_forward_static_ws_v1(const mi355_w8a8_problem* problem, void* str
 uint64_t mi355_w8a8_bwd_workspace_bytes(uint32_t m, uint32_t k, uint32_t n, uint32_t n_adapters,
                                         uint32_t rank, uint32_t flags);
 int mi355_w8a8_lora_linear_bwd_v1(const mi355_w8a8_bwd_problem* problem, void* stream);
+
+/* 1 where a forward call of these sizes and flags takes a mi355_w8a8_problem_z (tiled paths that do not leave z in parts), else 0. */
+int mi355_w8a8_forward_keeps_z(uint32_t m, uint32_t k, uint32_t n, uint32_t n_adapters, uint32_t rank, uint32_t flags);
 
 /*
  * Backward of mi355_w8a8_grouped_v1 without FLAG_SWIGLU: the derivative of LoRAExpert.__call__

@@ -47,7 +47,7 @@ EXPORTS = (
     "mi355_w8a8_pack_weight_v1", "mi355_w8a8_unpack_weight_v1", "mi355_w8a8_quantize_rows_v1",
     "mi355_w8a8_workspace_bytes", "mi355_w8a8_grouped_workspace_bytes",
     "mi355_w8a8_lora_linear_v1", "mi355_w8a8_rms_gateup_swiglu_v1", "mi355_w8a8_lora_residual_v1",
-    "mi355_w8a8_forward_v1", "mi355_w8a8_forward_static_ws_v1", "mi355_w8a8_grouped_v1",
+    "mi355_w8a8_forward_v1", "mi355_w8a8_forward_static_ws_v1", "mi355_w8a8_forward_keeps_z", "mi355_w8a8_grouped_v1",
     "mi355_w8a8_bwd_workspace_bytes", "mi355_w8a8_lora_linear_bwd_v1",
     "mi355_w8a8_grouped_bwd_workspace_bytes", "mi355_w8a8_grouped_bwd_v1",
     "mi355_w8a8_qkv_split_norm_rope_v1",
@@ -116,6 +116,42 @@ class GroupedBwdProblem(ctypes.Structure):
         ("d_lora_scaling", _vp), ("workspace", _vp), ("workspace_bytes", _u64),
         ("x_row_map", _vp), ("x_row_repeat", _u32), ("x_rows", _u32),
     ]
+
+
+class ProblemZ(ctypes.Structure):
+    """struct mi355_w8a8_problem_z"""
+
+    _fields_ = [("call", Problem), ("z", _vp)]
+
+
+class GroupedProblemZ(ctypes.Structure):
+    """struct mi355_w8a8_grouped_problem_z"""
+
+    _fields_ = [("call", GroupedProblem), ("z", _vp)]
+
+
+class BwdProblemZ(ctypes.Structure):
+    """struct mi355_w8a8_bwd_problem_z"""
+
+    _fields_ = [("call", BwdProblem), ("z", _vp)]
+
+
+class GroupedBwdProblemZ(ctypes.Structure):
+    """struct mi355_w8a8_grouped_bwd_problem_z"""
+
+    _fields_ = [("call", GroupedBwdProblem), ("z", _vp)]
+
+
+def problem_struct(plain, with_z, z):
+    """A zeroed ``plain`` whose ``struct_size`` is set; with a tensor ``z`` the head of a ``with_z`` that names it."""
+    if z is None:
+        p = plain()
+        p.struct_size = ctypes.sizeof(plain)
+        return p
+    whole = with_z()
+    whole.z = z.data_ptr()
+    whole.call.struct_size = ctypes.sizeof(with_z)
+    return whole.call  # (keeps the whole alive and starts where it does)
 
 
 class QkvPostProblem(ctypes.Structure):
@@ -215,6 +251,8 @@ def _bind(lib: ctypes.CDLL) -> None:
     lib.mi355_w8a8_grouped_v1.argtypes = (ctypes.POINTER(GroupedProblem), _vp)
     lib.mi355_w8a8_lora_linear_bwd_v1.restype = ctypes.c_int
     lib.mi355_w8a8_lora_linear_bwd_v1.argtypes = (ctypes.POINTER(BwdProblem), _vp)
+    lib.mi355_w8a8_forward_keeps_z.restype = ctypes.c_int
+    lib.mi355_w8a8_forward_keeps_z.argtypes = (_u32, _u32, _u32, _u32, _u32, _u32)
     lib.mi355_w8a8_grouped_bwd_workspace_bytes.restype = _u64
     lib.mi355_w8a8_grouped_bwd_workspace_bytes.argtypes = (_u32, _u32, _u32, _u32, _u32, _u32)
     lib.mi355_w8a8_grouped_bwd_v1.restype = ctypes.c_int

@@ -551,11 +551,23 @@ bool prologue_keeps_rows(uint32_t rows_bound, uint32_t k, bool rms, bool lora, b
   return !pack && (wgs <= 256u || k <= 2304u);  // (two workgroups of up to 2304 k share a CU)
 }
 
+// Whether a call's LoRA-A projection passes through quant_lora_store_z whatever its routing: the tiled paths, but not where the K-split
+// tiles, which may take it in quarters, could fit (they fit fewer rows first: the unpadded count decides).
+bool forward_keeps_z(uint32_t m, uint32_t k, uint32_t n, uint32_t n_adapters, uint32_t rank, uint32_t flags) {
+  if (!n_adapters || !rank || rank > (uint32_t)kMaxRank || validate_common(m, k, n)) return false;
+  const int path = choose_forward_path(m, k, n, flags);
+  if (path < 0 || path == MI355_W8A8_PATH_SKINNY || path == MI355_W8A8_PATH_SKINNY_CHUNKS) return false;
+  return path != MI355_W8A8_PATH_TILED_128X128 || !ksplit_fits(round_up(m, 32u), n);
+}
+
 int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
   if (!p) return MI355_W8A8_ERR_NULL;
-  if (p->struct_size != sizeof(mi355_w8a8_problem)) return MI355_W8A8_ERR_STRUCT;
+  float* z_rows = nullptr;
+  if (p->struct_size == sizeof(mi355_w8a8_problem_z)) z_rows = reinterpret_cast<const mi355_w8a8_problem_z*>(p)->z;
+  else if (p->struct_size != sizeof(mi355_w8a8_problem)) return MI355_W8A8_ERR_STRUCT;
   int st = validate_common(p->m, p->k, p->n);
   if (st) return st;
+  if (z_rows && !forward_keeps_z(p->m, p->k, p->n, p->n_adapters, p->rank, p->flags)) return MI355_W8A8_ERR_UNSUPPORTED;
   if (!p->x || !p->w_packed || !p->w_scales || !p->out) return MI355_W8A8_ERR_NULL;
   const bool swiglu = (p->flags & MI355_W8A8_FLAG_SWIGLU) != 0;
   const bool rms = p->rms_gamma != nullptr;
@@ -580,9 +592,11 @@ int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
   const uint64_t x_bytes = (uint64_t)p->m * p->k * 2u;
   if (!aligned16(p->x) || !aligned16(p->w_packed) || !aligned16(p->out) || !aligned16(p->w_scales) ||
       !aligned16(p->lora_a) || !aligned16(p->lora_b) || !aligned16(p->residual) ||
-      !aligned16(p->rms_gamma) || !aligned16(p->adapter_indices))
+      !aligned16(p->rms_gamma) || !aligned16(p->adapter_indices) || !aligned16(z_rows))
     return MI355_W8A8_ERR_ALIGN;
-  if (overlaps(p->out, out_bytes, p->x, x_bytes) || overlaps(p->out, out_bytes, p->residual, out_bytes) ||
+  const uint64_t z_bytes = (uint64_t)p->m * p->rank * 4u;
+  if (overlaps(z_rows, z_bytes, p->out, out_bytes) || overlaps(z_rows, z_bytes, p->x, x_bytes) ||
+      overlaps(z_rows, z_bytes, p->workspace, p->workspace_bytes) || overlaps(p->out, out_bytes, p->x, x_bytes) || overlaps(p->out, out_bytes, p->residual, out_bytes) ||
       overlaps(p->out, out_bytes, p->w_packed, mi355_w8a8_packed_weight_bytes(p->k, p->n)) ||
       overlaps(p->out, out_bytes, p->lora_b, (uint64_t)p->n_adapters * p->rank * p->n * 2u) ||
       overlaps(p->out, out_bytes, p->lora_a, (uint64_t)p->n_adapters * p->rank * p->k * 2u) ||
@@ -717,6 +731,7 @@ int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
   q.nterms = (p->flags & MI355_W8A8_FLAG_LORA_SPLIT2) ? 2u : 3u;
   q.tile_ctr = reinterpret_cast<uint32_t*>(ws + w.tile_ctr);
   q.group_pad = pad_groups ? 32u : 1u;
+  q.z_rows = z_rows;
   if (!skip_prologue) {
     const dim3 grid(q.n_half_blocks), block(1024);
     if (split_z) {
@@ -879,7 +894,9 @@ int launch_grouped_quant(const QuantLoraArgs& q, uint32_t nkk, hipStream_t s) {
 
 int run_grouped(const mi355_w8a8_grouped_problem* p, hipStream_t s) {
   if (!p) return MI355_W8A8_ERR_NULL;
-  if (p->struct_size != sizeof(mi355_w8a8_grouped_problem)) return MI355_W8A8_ERR_STRUCT;
+  float* z_rows = nullptr;
+  if (p->struct_size == sizeof(mi355_w8a8_grouped_problem_z)) z_rows = reinterpret_cast<const mi355_w8a8_grouped_problem_z*>(p)->z;
+  else if (p->struct_size != sizeof(mi355_w8a8_grouped_problem)) return MI355_W8A8_ERR_STRUCT;
   int st = validate_common(p->m, p->k, p->n);
   if (st) return st;
   if (p->n_groups == 0) return MI355_W8A8_ERR_SHAPE;
@@ -897,17 +914,20 @@ int run_grouped(const mi355_w8a8_grouped_problem* p, hipStream_t s) {
   const uint32_t n_out = swiglu ? p->n / 2u : p->n;
   const uint64_t out_bytes = (uint64_t)p->m * n_out * 2u;
   if (!aligned16(p->x) || !aligned16(p->w_packed) || !aligned16(p->out) || !aligned16(p->w_scales) ||
-      !aligned16(p->lora_a) || !aligned16(p->lora_b) || (reinterpret_cast<uintptr_t>(p->group_sizes) & 3u))
+      !aligned16(p->lora_a) || !aligned16(p->lora_b) || !aligned16(z_rows) || (reinterpret_cast<uintptr_t>(p->group_sizes) & 3u))
     return MI355_W8A8_ERR_ALIGN;
+  if (z_rows && !lora) return MI355_W8A8_ERR_SHAPE;
   const uint32_t x_repeat = p->x_row_map ? p->x_row_repeat : 1u;
   if (p->x_row_map && (x_repeat == 0 || (reinterpret_cast<uintptr_t>(p->x_row_map) & 3u)))
     return x_repeat == 0 ? MI355_W8A8_ERR_SHAPE : MI355_W8A8_ERR_ALIGN;
   // with a row map x holds one row per token unless the caller says otherwise; gathered reads are
   // clamped to these rows
   const uint32_t x_rows = (p->x_row_map && p->x_rows) ? p->x_rows : (p->m + x_repeat - 1u) / x_repeat;
+  const uint64_t z_bytes = (uint64_t)p->m * p->rank * 4u;
   if (overlaps(p->out, out_bytes, p->x, (uint64_t)x_rows * p->k * 2u) ||
       overlaps(p->out, out_bytes, p->x_row_map, (uint64_t)p->m * 4u) ||
-      overlaps(p->out, out_bytes, p->workspace, p->workspace_bytes))
+      overlaps(p->out, out_bytes, p->workspace, p->workspace_bytes) || overlaps(z_rows, z_bytes, p->out, out_bytes) ||
+      overlaps(z_rows, z_bytes, p->x, (uint64_t)x_rows * p->k * 2u) || overlaps(z_rows, z_bytes, p->workspace, p->workspace_bytes))
     return MI355_W8A8_ERR_ALIAS;
   if ((p->flags & MI355_W8A8_FLAG_GROUPED_TILE64) && (p->flags & MI355_W8A8_FLAG_GROUPED_TILE128))
     return MI355_W8A8_ERR_SHAPE;
@@ -976,6 +996,7 @@ int run_grouped(const mi355_w8a8_grouped_problem* p, hipStream_t s) {
     q.nterms = (p->flags & MI355_W8A8_FLAG_LORA_SPLIT2) ? 2u : 3u;
     q.group_pad = 32u;
     q.row_map = p->x_row_map; q.row_div = x_repeat; q.row_limit = x_rows; q.scale_by_source = by_source ? 1u : 0u;
+    q.z_rows = z_rows;
     if ((st = launch_grouped_quant(q, lora ? w.nkk : 0u, s))) return st;
     if (p->aux_x_codes || p->aux_x_scales) {  // the caller's copies: of every row (some have no slot), then what the GEMM reads
       QuantArgs c{};
@@ -1172,6 +1193,7 @@ struct BwdBody {
   // group-scaled weights: their format (weight_bits 0: per-channel), A itself and the notes of non-finite operands
   uint32_t weight_bits, group, terms; const float* w_scales;
   const void* lora_a; uint64_t beyond;
+  const float* z_rows;  // x @ A[idx] as the forward left it, or null
 };
 
 template <bool W4, int TERMS, int NKK>
@@ -1233,8 +1255,11 @@ int launch_bwd_body(const BwdBody& b, const Layout& w, unsigned char* ws, hipStr
     f.r = b.rank;
     f.n_slices = w.n_slices; f.slots = w.slots; f.nkk = w.nkk; f.cols = w.nkk > 2u ? 64u : 32u;
     f.beyond = beyond;
-    // z = x @ A, recomputed rather than saved by the forward (and, of a group-scaled call, looked at for x)
-    if (b.d_lora_b || b.d_lora_scaling || (beyond && b.d_lora_a)) {
+    // z = x @ A, as the forward left it or formed again (and, of a group-scaled call, looked at for x).  Formed again it is a launch over all
+    // of x and one for A transposed: 42 us of an MLP's step at 3003 rows, 32 of an expert layer's at 1021 tokens.
+    if (b.z_rows && (b.d_lora_b || b.d_lora_scaling)) {
+      f.z_rows = b.z_rows; f.src_row = b.src_row; f.M = b.m;
+    } else if (b.d_lora_b || b.d_lora_scaling || (beyond && b.d_lora_a)) {
       LoraAArgs lz{};
       lz.xsrc = static_cast<const uint16_t*>(b.x);
       lz.at = reinterpret_cast<const uint16_t*>(ws + w.at);
@@ -1356,7 +1381,9 @@ int launch_bwd_body(const BwdBody& b, const Layout& w, unsigned char* ws, hipStr
 
 int run_backward(const mi355_w8a8_bwd_problem* p, hipStream_t s) {
   if (!p) return MI355_W8A8_ERR_NULL;
-  if (p->struct_size != sizeof(mi355_w8a8_bwd_problem)) return MI355_W8A8_ERR_STRUCT;
+  const float* z_rows = nullptr;
+  if (p->struct_size == sizeof(mi355_w8a8_bwd_problem_z)) z_rows = reinterpret_cast<const mi355_w8a8_bwd_problem_z*>(p)->z;
+  else if (p->struct_size != sizeof(mi355_w8a8_bwd_problem)) return MI355_W8A8_ERR_STRUCT;
   int st = validate_bwd_dims(p->m, p->k, p->n, p->n_adapters, p->rank);
   if (st) return st;
   if (p->flags & ~(MI355_W8A8_FLAG_SKIP_PROLOGUE | MI355_W8A8_FLAG_SKIP_GEMM)) return MI355_W8A8_ERR_SHAPE;
@@ -1373,11 +1400,12 @@ int run_backward(const mi355_w8a8_bwd_problem* p, hipStream_t s) {
   }
   if (!aligned16(p->x) || !aligned16(p->dy) || !aligned16(p->w_packed) || !aligned16(p->w_scales) ||
       !aligned16(p->lora_a) || !aligned16(p->lora_b) || !aligned16(p->dx) || !aligned16(p->d_lora_a) ||
-      !aligned16(p->d_lora_b) || !aligned16(p->adapter_indices))
+      !aligned16(p->d_lora_b) || !aligned16(p->adapter_indices) || !aligned16(z_rows))
     return MI355_W8A8_ERR_ALIGN;
+  if (z_rows && !lora) return MI355_W8A8_ERR_SHAPE;
   const uint64_t dx_bytes = (uint64_t)p->m * p->k * 2u, dy_bytes = (uint64_t)p->m * p->n * 2u;
   const uint64_t a_bytes = (uint64_t)p->n_adapters * p->rank * p->k * 2u, b_bytes = (uint64_t)p->n_adapters * p->rank * p->n * 2u;
-  if (overlaps(p->dx, dx_bytes, p->dy, dy_bytes) || overlaps(p->dx, dx_bytes, p->x, dx_bytes) ||
+  if (overlaps(z_rows, (uint64_t)p->m * p->rank * 4u, p->dx, dx_bytes) || overlaps(p->dx, dx_bytes, p->dy, dy_bytes) || overlaps(p->dx, dx_bytes, p->x, dx_bytes) ||
       overlaps(p->dx, dx_bytes, p->workspace, p->workspace_bytes) ||
       overlaps(p->d_lora_a, a_bytes, p->lora_a, a_bytes) || overlaps(p->d_lora_b, b_bytes, p->lora_b, b_bytes) ||
       overlaps(p->d_lora_a, a_bytes, p->workspace, p->workspace_bytes) ||
@@ -1407,7 +1435,7 @@ int run_backward(const mi355_w8a8_bwd_problem* p, hipStream_t s) {
     pa.M = p->m; pa.K = p->k; pa.N = p->n; pa.N_pad = w.N_pad; pa.n_groups = p->n_adapters; pa.r = p->rank;
     pa.nkk = w.nkk; pa.kb32 = w.KB; pa.slots = w.slots;
     pa.route_blocks = lora ? 1u : 0u;
-    pa.a_blocks = lora ? (uint32_t)(((uint64_t)p->n_adapters * p->k * ((p->rank + 7u) / 8u) + 1023u) / 1024u) : 0u;
+    pa.a_blocks = lora && !z_rows ? (uint32_t)(((uint64_t)p->n_adapters * p->k * ((p->rank + 7u) / 8u) + 1023u) / 1024u) : 0u;
     pa.ap_blocks = lora ? bwd_ap_blocks(p->n_adapters, w.KB, w.nkk) : 0u;
     const uint32_t sw_blocks = (w.N_pad + 1023u) / 1024u;
     hipLaunchKernelGGL(bwd_prep_kernel, dim3(pa.route_blocks + pa.a_blocks + pa.ap_blocks + sw_blocks), dim3(1024), 0, s, pa);
@@ -1418,6 +1446,7 @@ int run_backward(const mi355_w8a8_bwd_problem* p, hipStream_t s) {
   b.x = p->x; b.dy = p->dy; b.w_packed = p->w_packed; b.lora_b = p->lora_b; b.lora_scaling = p->lora_scaling;
   b.dx = p->dx; b.d_lora_a = p->d_lora_a; b.d_lora_b = p->d_lora_b; b.d_lora_scaling = p->d_lora_scaling;
   b.lora = lora; b.want_grads = want_grads; b.skip_prologue = skip_prologue; b.skip_gemm = skip_gemm;
+  b.z_rows = z_rows;
   b.src_row = routed ? src_row : nullptr;
   b.slot_group = routed ? slot_group : nullptr;
   b.blk_range = routed ? blk_range : nullptr;
@@ -1579,9 +1608,11 @@ int validate_bwd_grouped_dims(uint32_t m, uint32_t k, uint32_t n, uint32_t n_gro
 int run_grouped_backward(const mi355_w8a8_grouped_bwd_problem* given, hipStream_t s) {
   if (!given) return MI355_W8A8_ERR_NULL;
   constexpr uint32_t kWithoutMap = offsetof(mi355_w8a8_grouped_bwd_problem, x_row_map);
-  if (given->struct_size != sizeof(mi355_w8a8_grouped_bwd_problem) && given->struct_size != kWithoutMap) return MI355_W8A8_ERR_STRUCT;
+  const bool with_z = given->struct_size == sizeof(mi355_w8a8_grouped_bwd_problem_z);
+  if (!with_z && given->struct_size != sizeof(mi355_w8a8_grouped_bwd_problem) && given->struct_size != kWithoutMap) return MI355_W8A8_ERR_STRUCT;
+  const float* const z_rows = with_z ? reinterpret_cast<const mi355_w8a8_grouped_bwd_problem_z*>(given)->z : nullptr;
   mi355_w8a8_grouped_bwd_problem problem{};
-  memcpy(&problem, given, given->struct_size);
+  memcpy(&problem, given, with_z ? sizeof(problem) : given->struct_size);
   const mi355_w8a8_grouped_bwd_problem* const p = &problem;
   if (p->flags) return MI355_W8A8_ERR_SHAPE;
   int st = validate_bwd_grouped_dims(p->m, p->k, p->n, p->n_groups, p->rank, p->groups_per_weight);
@@ -1597,15 +1628,17 @@ int run_grouped_backward(const mi355_w8a8_grouped_bwd_problem* given, hipStream_
   }
   if (!aligned16(p->x) || !aligned16(p->dy) || !aligned16(p->w_packed) || !aligned16(p->w_scales) ||
       !aligned16(p->lora_a) || !aligned16(p->lora_b) || !aligned16(p->dx) || !aligned16(p->d_lora_a) ||
-      !aligned16(p->d_lora_b) || (reinterpret_cast<uintptr_t>(p->group_sizes) & 3u))
+      !aligned16(p->d_lora_b) || !aligned16(z_rows) || (reinterpret_cast<uintptr_t>(p->group_sizes) & 3u))
     return MI355_W8A8_ERR_ALIGN;
+  if (z_rows && !lora) return MI355_W8A8_ERR_SHAPE;
   const uint32_t x_repeat = p->x_row_map ? p->x_row_repeat : 1u;
   if (p->x_row_map && (x_repeat == 0 || (reinterpret_cast<uintptr_t>(p->x_row_map) & 3u))) return MI355_W8A8_ERR_SHAPE;
   const uint32_t x_rows = (p->x_row_map && p->x_rows) ? p->x_rows : (p->m + x_repeat - 1u) / x_repeat;
   if ((uint64_t)x_rows * p->k >= (1ull << 32) - (1ull << 20)) return MI355_W8A8_ERR_UNSUPPORTED;
   const uint64_t dx_bytes = (uint64_t)p->m * p->k * 2u, dy_bytes = (uint64_t)p->m * p->n * 2u, x_bytes = (uint64_t)x_rows * p->k * 2u;
   const uint64_t a_bytes = (uint64_t)p->n_groups * p->rank * p->k * 2u, b_bytes = (uint64_t)p->n_groups * p->rank * p->n * 2u;
-  if (overlaps(p->dx, dx_bytes, p->dy, dy_bytes) || overlaps(p->dx, dx_bytes, p->x, x_bytes) ||
+  if (overlaps(z_rows, (uint64_t)p->m * p->rank * 4u, p->dx, dx_bytes) ||
+      overlaps(p->dx, dx_bytes, p->dy, dy_bytes) || overlaps(p->dx, dx_bytes, p->x, x_bytes) ||
       overlaps(p->dx, dx_bytes, p->x_row_map, (uint64_t)p->m * 4u) ||
       overlaps(p->dx, dx_bytes, p->workspace, p->workspace_bytes) ||
       overlaps(p->d_lora_a, a_bytes, p->lora_a, a_bytes) || overlaps(p->d_lora_b, b_bytes, p->lora_b, b_bytes) ||
@@ -1645,7 +1678,7 @@ int run_grouped_backward(const mi355_w8a8_grouped_bwd_problem* given, hipStream_
     pa.M = p->m; pa.K = p->k; pa.N = p->n; pa.N_pad = w.N_pad; pa.n_groups = p->n_groups; pa.gpw = w.gpw;
     pa.n_weights = w.n_weights; pa.r = p->rank; pa.nkk = w.nkk; pa.kb32 = w.KB; pa.slots = w.slots;
     pa.max_chunks = w.max_chunks; pa.sw_stride = w.sw_stride; pa.tile_rows = w.tile_rows;
-    pa.a_blocks = lora ? (uint32_t)(((uint64_t)p->n_groups * p->k * ((p->rank + 7u) / 8u) + 1023u) / 1024u) : 0u;
+    pa.a_blocks = lora && !z_rows ? (uint32_t)(((uint64_t)p->n_groups * p->k * ((p->rank + 7u) / 8u) + 1023u) / 1024u) : 0u;
     pa.ap_blocks = lora ? bwd_ap_blocks(p->n_groups, w.KB, w.nkk) : 0u;
     pa.sw_blocks_per_weight = (w.N_pad + 1023u) / 1024u;
     // (the tables are filled slot by slot: a few workgroups, each with the prefix sums of its own)
@@ -1660,7 +1693,7 @@ int run_grouped_backward(const mi355_w8a8_grouped_bwd_problem* given, hipStream_
   b.dx = p->dx; b.d_lora_a = p->d_lora_a; b.d_lora_b = p->d_lora_b; b.d_lora_scaling = p->d_lora_scaling;
   b.lora = lora; b.want_grads = want_grads;
   b.src_row = tab.src_row; b.slot_group = tab.slot_group; b.blk_range = tab.blk_range; b.skip_range = tab.blk_range;
-  b.x_row = tab.x_row; b.x_rows = x_rows;
+  b.x_row = tab.x_row; b.x_rows = x_rows; b.z_rows = z_rows;
   b.tile_weight = tab.tile_weight; b.chunk_tab = tab.chunk_tab; b.chunk0 = tab.chunk0;
   b.group_beg = tab.group_beg; b.group_end = tab.group_end;
   b.w_stride = (size_t)mi355_w8a8_packed_weight_bytes(p->k, p->n);
@@ -2427,6 +2460,9 @@ int mi355_w8a8_rms_gateup_swiglu_v1(const mi355_w8a8_problem* p, void* stream) {
 }
 int mi355_w8a8_lora_residual_v1(const mi355_w8a8_problem* p, void* stream) {
   return run_forward(p, static_cast<hipStream_t>(stream), kReqResidual);
+}
+int mi355_w8a8_forward_keeps_z(uint32_t m, uint32_t k, uint32_t n, uint32_t n_adapters, uint32_t rank, uint32_t flags) {
+  return forward_keeps_z(m, k, n, n_adapters, rank, flags) ? 1 : 0;
 }
 int mi355_w8a8_forward_v1(const mi355_w8a8_problem* p, void* stream) {
   return run_forward(p, static_cast<hipStream_t>(stream), kReqNone);

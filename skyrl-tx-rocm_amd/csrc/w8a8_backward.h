@@ -203,6 +203,9 @@ struct BwdRFinishArgs {
   double* row_dot;  // [slots]
   uint32_t n_slices, z_slices, slots, nkk, cols, r;  // cols = 16 * nkk rounded up to 32; z_slices 0: no z
   uint32_t* beyond;  // set where a value is beyond what bf16 terms can carry, or null
+  // z of every row as the forward left it, f32 [M, r], in the place of zpart, and the row of a slot (null: its own); or null
+  const float* z_rows; const int32_t* src_row;
+  uint32_t M;
 };
 
 // A float32 value that is no sum of bf16 terms: not finite, or rounded to infinity by the first of them.
@@ -238,7 +241,14 @@ __global__ __launch_bounds__(256) void bwd_r_finish_kernel(BwdRFinishArgs a) {
     }
     *reinterpret_cast<float4*>(a.r_raw + at) = make_float4(raw[0], raw[1], raw[2], raw[3]);
     *reinterpret_cast<float4*>(a.rs + at) = make_float4(scaled[0], scaled[1], scaled[2], scaled[3]);
-    if (a.z_slices) {
+    if (a.z_slices || a.z_rows) {
+      if (a.z_rows) {  // kernel-uniform
+        const int src = a.src_row ? a.src_row[slot] : (int)slot;
+        const bool row_ok = src >= 0 && src < (int)a.M;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (row_ok && col + e < a.r) z[e] = a.z_rows[(size_t)src * a.r + col + e];
+      }
 #pragma unroll
       for (uint32_t sl = 0; sl < kBwdMaxSlices; ++sl)
         if (sl < a.z_slices) { z[0] += u[sl].x; z[1] += u[sl].y; z[2] += u[sl].z; z[3] += u[sl].w; }

@@ -932,6 +932,7 @@ struct QuantLoraArgs {
   // row_scale then holds a value per source row (scale_by_source) or per row
   const int32_t* row_map;
   uint32_t row_div, row_limit, scale_by_source;
+  float* z_rows;            // f32 [M, r]: z of every row for the backward, or null
 };
 // the form that leaves z in quarters
 struct QuantLoraSplitArgs : QuantLoraArgs {
@@ -990,9 +991,10 @@ __device__ inline uint2 quant_codes8(const uint4& raw, float scale, float rscale
 // z of a half block: the waves' tiles added in a fixed order, split into three bf16 terms and stored as the GEMM
 // epilogue reads them (its rows first_row .. end_row - 1).  red: a wave tile each for waves 0..7 (of 16) or 0..3; zs: the
 // sixteen rows of z.
-template <int kCB, uint32_t WAVES>
+// src_of(row): the row of x in it, or -1.
+template <int kCB, uint32_t WAVES, class SrcOf>
 __device__ inline void quant_lora_store_z(const QuantLoraArgs& a, v4f (&acc)[kCB], float (*red)[kCB][4][64], float (*zs)[kCB * 16 + 1],
-                                          uint32_t pb, uint32_t half16, uint32_t first_row = 0u, uint32_t end_row = 16u) {
+                                          uint32_t pb, uint32_t half16, SrcOf&& src_of, uint32_t first_row = 0u, uint32_t end_row = 16u) {
   const uint32_t tid = threadIdx.x, lane = tid & 63u;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // of 16 waves, 8..15 onto 0..7, 4..7 onto 0..3; then 0+1+2+3
@@ -1027,6 +1029,14 @@ __device__ inline void quant_lora_store_z(const QuantLoraArgs& a, v4f (&acc)[kCB
     zs[4u * (l >> 4) + e][b * 16u + (l & 15u)] = sum;
   }
   __syncthreads();
+  if (a.z_rows) {  // kernel-uniform
+    for (uint32_t t = tid; t < 16u * a.r; t += WAVES * 64u) {
+      const uint32_t row = t / a.r, col = t % a.r;
+      if (row < first_row || row >= end_row) continue;
+      const int src = src_of(row);
+      if (src >= 0 && src < (int)a.M) a.z_rows[(size_t)src * a.r + col] = zs[row][col];
+    }
+  }
   // zp[pb][kk][term][lane64][8]: lane = row % 32 + 32 * hh holds rank columns 16 kk + 8 hh + 0..7
   for (uint32_t t = tid; t < a.nkk * 3u * 32u; t += WAVES * 64u) {
     const uint32_t row = t & 15u, hh = (t >> 4) & 1u, term = (t >> 5) % 3u, kk = t / 96u;
@@ -1220,7 +1230,8 @@ __global__ __launch_bounds__(WAVES * 64, SPLIT ? 2 : 4) void quant_lora_kernel(s
       for (int e = 0; e < 4; ++e) acc[b][e] = SPLIT ? red[wave][b][e][lane] : z[b][e];
   }
   if constexpr (SPLIT) quant_lora_store_quarter<kCB>(a, acc, red, hb, blockIdx.x & 3u);
-  else if constexpr (CB > 0) quant_lora_store_z<kCB, WAVES>(a, acc, red, zs, pb, half16);
+  else if constexpr (CB > 0)
+    quant_lora_store_z<kCB, WAVES>(a, acc, red, zs, pb, half16, [&](uint32_t r) -> int { return a.src_row ? a.src_row[hb * 16u + r] : (int)(hb * 16u + r); });
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1558,7 +1569,8 @@ __global__ __launch_bounds__(1024) void quant_lora_rows_kernel(QuantLoraRowsArgs
       for (int b = 0; b < kCB; ++b) acc[b] = z[b];
     }
     __syncthreads();  // the rows are spent: their bytes take the wave tiles
-    quant_lora_store_z<kCB, 16u>(a, acc, reinterpret_cast<float (*)[kCB][4][64]>(ql_lds), zs, pb, half16, r0, r0 + R);
+    quant_lora_store_z<kCB, 16u>(a, acc, reinterpret_cast<float (*)[kCB][4][64]>(ql_lds), zs, pb, half16,
+                                   [&](uint32_t r) -> int { return row_src[r]; }, r0, r0 + R);
   }
 }
 

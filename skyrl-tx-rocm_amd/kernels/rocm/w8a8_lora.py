@@ -280,7 +280,7 @@ class ForwardPlan:
                  adapter_indices: torch.Tensor | None = None, rms_gamma: torch.Tensor | None = None,
                  eps: float = 1e-6, residual: torch.Tensor | None = None, swiglu: bool = False,
                  flags: int = 0, return_aux: bool = False, entry: str = "forward",
-                 want_normalized: bool = False, keep_lora_pack: bool = True):
+                 want_normalized: bool = False, keep_lora_pack: bool = True, want_z: bool = False):
         if x.dtype != torch.bfloat16:
             raise TypeError(f"x must be BF16, got {x.dtype}")
         if x.ndim < 2 or math.prod(x.shape[:-1]) <= 0:
@@ -341,8 +341,11 @@ class ForwardPlan:
         if (return_aux or want_normalized) and gamma is not None:
             aux["normalized"] = torch.empty((m, k), dtype=torch.bfloat16, device=dev)
 
-        p = _native.Problem()
-        p.struct_size = ctypes.sizeof(_native.Problem)
+        # x @ A of every row, for a backward: float32 [m, r], or None where the call's path has no place for it
+        self.z = None
+        if want_z and n_ad and lib.mi355_w8a8_forward_keeps_z(m, k, n, n_ad, r, flags):
+            self.z = torch.empty((m, r), dtype=torch.float32, device=dev)
+        p = _native.problem_struct(_native.Problem, _native.ProblemZ, self.z)
         p.flags = flags
         p.m, p.k, p.n, p.n_adapters, p.rank = m, k, n, n_ad, r
         p.rms_eps = float(eps)
@@ -455,7 +458,8 @@ class BackwardPlan:
     a single C call on torch's current stream (see ``ForwardPlan``)."""
 
     def __init__(self, x: torch.Tensor | None, dy: torch.Tensor, weight, lora_a=None, lora_b=None,
-                 lora_scaling=None, *, adapter_indices: torch.Tensor | None = None, need_lora_grads: bool = True):
+                 lora_scaling=None, *, adapter_indices: torch.Tensor | None = None, need_lora_grads: bool = True,
+                 z: torch.Tensor | None = None):
         if dy.dtype != torch.bfloat16:
             raise TypeError(f"dy must be BF16, got {dy.dtype}")
         if dy.ndim < 2 or math.prod(dy.shape[:-1]) <= 0:
@@ -500,8 +504,11 @@ class BackwardPlan:
         self.d_lora_a = torch.empty((n_ad, k, r), dtype=torch.bfloat16, device=dev) if want else None
         self.d_lora_b = torch.empty((n_ad, r, n), dtype=torch.bfloat16, device=dev) if want else None
         self.d_lora_scaling = torch.empty((n_ad,), dtype=torch.float32, device=dev) if want else None
-        p = _native.BwdProblem()
-        p.struct_size = ctypes.sizeof(_native.BwdProblem)
+        if z is not None:  # the forward's x @ A (ForwardPlan.z)
+            if not want or z.dtype != torch.float32 or tuple(z.shape) != (m, r) or z.device != dev:
+                raise ValueError(f"z must be float32 [{m}, {r}] on {dev}, beside LoRA cotangents")
+            z = z.contiguous()
+        p = _native.problem_struct(_native.BwdProblem, _native.BwdProblemZ, z)
         p.m, p.k, p.n, p.n_adapters, p.rank = m, k, n, n_ad, r
         p.x = xf.data_ptr() if xf is not None else None
         p.dy = dyf.data_ptr()
@@ -522,7 +529,7 @@ class BackwardPlan:
         self.dx_shape = (*dy.shape[:-1], k)
         self.dims = {"m": m, "k": k, "n": n, "n_adapters": n_ad, "rank": r}
         self._fn = lib.mi355_w8a8_lora_linear_bwd_v1
-        self._keep = (xf, dyf, pw, a3, b3, s1, idx, ws)
+        self._keep = (xf, dyf, pw, a3, b3, s1, idx, ws, z)
 
     def run(self, flags: int = 0):
         """Enqueue the call; returns ``(dx, d_lora_a, d_lora_b, d_lora_scaling)`` (reused tensors)."""
@@ -555,8 +562,9 @@ class _LoraLinearFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, lora_a, lora_b, lora_scaling, weight, adapter_indices, residual):
         plan = ForwardPlan(x, weight, lora_a, lora_b, lora_scaling, adapter_indices=adapter_indices,
-                           residual=residual, entry="linear" if residual is None else "residual", keep_lora_pack=False)
-        ctx.save_for_backward(x, lora_a, lora_b, lora_scaling)
+                           residual=residual, entry="linear" if residual is None else "residual", keep_lora_pack=False,
+                           want_z=lora_a is not None and any(ctx.needs_input_grad[1:4]))
+        ctx.save_for_backward(x, lora_a, lora_b, lora_scaling, plan.z)
         ctx.weight = weight
         ctx.adapter_indices = plan.adapter_indices  # (one per row: expanded once for both directions)
         ctx.has_residual = residual is not None
@@ -564,10 +572,10 @@ class _LoraLinearFunction(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dy):
-        x, lora_a, lora_b, lora_scaling = ctx.saved_tensors
+        x, lora_a, lora_b, lora_scaling, z = ctx.saved_tensors
         need = lora_a is not None and any(ctx.needs_input_grad[1:4])
-        dx, da, db, ds = backward(x, dy.contiguous(), ctx.weight, lora_a, lora_b, lora_scaling,
-                                  adapter_indices=ctx.adapter_indices, need_lora_grads=need)
+        dx, da, db, ds = BackwardPlan(x, dy.contiguous(), ctx.weight, lora_a, lora_b, lora_scaling,
+                                      adapter_indices=ctx.adapter_indices, need_lora_grads=need, z=z if need else None).run()
         if need:
             if lora_a.ndim == 2:
                 da, db = da[0], db[0]
@@ -660,7 +668,7 @@ class FusedBackwardPlan:
         if not isinstance(eps, float) or not eps > 0.0:
             raise ValueError(f"eps must be a positive float, got {eps!r}")
         self.fwd = ForwardPlan(x, weight, lora_a, lora_b, lora_scaling, adapter_indices=adapter_indices,
-                               rms_gamma=gamma, eps=eps, want_normalized=True)
+                               rms_gamma=gamma, eps=eps, want_normalized=True, want_z=lora_a is not None and need_lora_grads)
         d = self.fwd.dims
         m, k, n = d["m"], d["k"], d["n"]
         if n % 8:
@@ -677,7 +685,7 @@ class FusedBackwardPlan:
         idx = self.fwd.adapter_indices
         # fwd.out doubles as the projection and, after the in-place pull-back, as its cotangent
         self.bwd = BackwardPlan(self.fwd.aux["normalized"], self.fwd.out, weight, lora_a, lora_b, lora_scaling,
-                                adapter_indices=idx, need_lora_grads=need_lora_grads)
+                                adapter_indices=idx, need_lora_grads=need_lora_grads, z=self.fwd.z)
         self.device = x.device
         self.dx_shape = tuple(x.shape)
         self.dims = d
@@ -758,10 +766,11 @@ class _RmsGateUpFunction(torch.autograd.Function):
             rows = math.prod(x.shape[:-1])
             plan = ForwardPlan(x, weight, lora_a, lora_b, lora_scaling, adapter_indices=adapter_indices,
                                rms_gamma=gamma, eps=eps, want_normalized=True,
+                               want_z=lora_a is not None and any(ctx.needs_input_grad[1:4]),
                                flags=0 if rows <= SKINNY_MAX_ROWS else _native.FLAG_FORCE_TILED)
             fused = plan.run()
             ctx.adapter_indices = plan.adapter_indices  # (one per row: expanded once for both directions)
-            ctx.save_for_backward(x, lora_a, lora_b, lora_scaling, gamma, fused, plan.aux["normalized"])
+            ctx.save_for_backward(x, lora_a, lora_b, lora_scaling, gamma, fused, plan.aux["normalized"], plan.z)
             return swiglu(fused)
         ctx.save_for_backward(x, lora_a, lora_b, lora_scaling, gamma)
         return forward(x, weight, lora_a, lora_b, lora_scaling, adapter_indices=adapter_indices,
@@ -772,11 +781,11 @@ class _RmsGateUpFunction(torch.autograd.Function):
         x, lora_a, lora_b, lora_scaling, gamma = ctx.saved_tensors[:5]
         need = lora_a is not None and any(ctx.needs_input_grad[1:4])
         if ctx.saved_projection:
-            fused, normalized = ctx.saved_tensors[5:]
+            fused, normalized, z = ctx.saved_tensors[5:]
             d_fused = swiglu_backward(fused, d_product.contiguous().reshape(*fused.shape[:-1], -1))
             rows = normalized.shape[0]
-            dn, da, db, ds = backward(normalized, d_fused.reshape(rows, -1), ctx.weight, lora_a, lora_b, lora_scaling,
-                                      adapter_indices=ctx.adapter_indices, need_lora_grads=need)
+            dn, da, db, ds = BackwardPlan(normalized, d_fused.reshape(rows, -1), ctx.weight, lora_a, lora_b, lora_scaling,
+                                          adapter_indices=ctx.adapter_indices, need_lora_grads=need, z=z if need else None).run()
             dx = rms_norm_backward(x.reshape(rows, -1), gamma, dn, eps=ctx.eps, in_place=True).reshape(x.shape)
         else:
             dx, da, db, ds = rms_gate_up_swiglu_backward(x, gamma, ctx.weight, lora_a, lora_b, lora_scaling,
@@ -861,7 +870,7 @@ class GroupedForwardPlan:
     def __init__(self, x: torch.Tensor, group_sizes: torch.Tensor, weight: PackedGroupedW8Weight, lora_a=None,
                  lora_b=None, lora_scaling=None, *, swiglu: bool = False, groups_per_weight: int = 1,
                  flags: int = 0, return_aux: bool = False, row_map: torch.Tensor | None = None,
-                 row_repeat: int = 1):
+                 row_repeat: int = 1, want_z: bool = False):
         if x.dtype != torch.bfloat16:
             raise TypeError(f"x must be BF16, got {x.dtype}")
         if x.ndim != 2 or x.shape[0] <= 0:
@@ -920,8 +929,8 @@ class GroupedForwardPlan:
             self.aux["acc"] = torch.zeros((m, n), dtype=torch.int32, device=dev)
         self.x_flat, self.group_sizes, self.row_map, self.weight = flat, gs, rmap, weight
         self._keep = (a3, b3, s1)
-        p = _native.GroupedProblem()
-        p.struct_size = ctypes.sizeof(_native.GroupedProblem)
+        self.z = torch.empty((m, r), dtype=torch.float32, device=dev) if want_z and r else None  # x @ A, for a backward
+        p = _native.problem_struct(_native.GroupedProblem, _native.GroupedProblemZ, self.z)
         p.flags = flags
         p.m, p.k, p.n, p.n_groups, p.rank, p.groups_per_weight = m, k, n, n_groups, r, groups_per_weight
         p.x = flat.data_ptr()
@@ -1001,7 +1010,7 @@ class GroupedBackwardPlan:
     def __init__(self, x: torch.Tensor | None, dy: torch.Tensor, group_sizes: torch.Tensor,
                  weight: PackedGroupedW8Weight, lora_a=None, lora_b=None, lora_scaling=None, *,
                  groups_per_weight: int = 1, need_lora_grads: bool = True, row_map: torch.Tensor | None = None,
-                 row_repeat: int = 1):
+                 row_repeat: int = 1, z: torch.Tensor | None = None):
         if dy.ndim != 2 or dy.dtype != torch.bfloat16:
             raise TypeError("dy must be a BF16 matrix [rows, N]")
         _require_cuda(dy, "dy")
@@ -1058,8 +1067,11 @@ class GroupedBackwardPlan:
         self.d_lora_a = torch.empty((n_groups, k, r), dtype=torch.bfloat16, device=dev) if want else None
         self.d_lora_b = torch.empty((n_groups, r, n), dtype=torch.bfloat16, device=dev) if want else None
         self.d_lora_scaling = torch.empty((n_groups,), dtype=torch.float32, device=dev) if want else None
-        p = _native.GroupedBwdProblem()
-        p.struct_size = ctypes.sizeof(_native.GroupedBwdProblem)
+        if z is not None:  # the forward's x @ A (GroupedForwardPlan.z)
+            if not want or z.dtype != torch.float32 or tuple(z.shape) != (m, r) or z.device != dev:
+                raise ValueError(f"z must be float32 [{m}, {r}] on {dev}, beside LoRA cotangents")
+            z = z.contiguous()
+        p = _native.problem_struct(_native.GroupedBwdProblem, _native.GroupedBwdProblemZ, z)
         p.m, p.k, p.n, p.n_groups, p.rank, p.groups_per_weight = m, k, n, n_groups, r, gpw
         p.x = xf.data_ptr() if xf is not None else None
         p.dy = dyf.data_ptr()
@@ -1080,7 +1092,7 @@ class GroupedBackwardPlan:
         self.dims = {"m": m, "k": k, "n": n, "n_groups": n_groups, "rank": r}
         self.group_sizes = gs   # the int32 tensor the call reads: rewrite it in place to route the next run differently
         self._fn = lib.mi355_w8a8_grouped_bwd_v1
-        self._keep = (xf, dyf, gs, weight, a3, b3, s1, ws, rmap)
+        self._keep = (xf, dyf, gs, weight, a3, b3, s1, ws, rmap, z)
 
     def run(self):
         """Enqueue the call; returns ``(dx, d_lora_a, d_lora_b, d_lora_scaling)`` (reused tensors)."""
@@ -1162,19 +1174,20 @@ class _GroupedLinearFunction(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, lora_a, lora_b, lora_scaling, weight, group_sizes, groups_per_weight):
-        out = grouped_forward(x, group_sizes, weight, lora_a, lora_b, lora_scaling,
-                              groups_per_weight=groups_per_weight)
-        ctx.save_for_backward(x, lora_a, lora_b, lora_scaling, group_sizes)
+        plan = GroupedForwardPlan(x, group_sizes, weight, lora_a, lora_b, lora_scaling, groups_per_weight=groups_per_weight,
+                                  want_z=any(ctx.needs_input_grad[1:4]))
+        out = plan.run()
+        ctx.save_for_backward(x, lora_a, lora_b, lora_scaling, group_sizes, plan.z)
         ctx.weight = weight
         ctx.gpw = groups_per_weight
         return out
 
     @staticmethod
     def backward(ctx, dy):
-        x, lora_a, lora_b, lora_scaling, group_sizes = ctx.saved_tensors
+        x, lora_a, lora_b, lora_scaling, group_sizes, z = ctx.saved_tensors
         need = lora_a is not None and any(ctx.needs_input_grad[1:4])
-        dx, da, db, ds = grouped_backward(x, dy.contiguous(), group_sizes, ctx.weight, lora_a, lora_b,
-                                          lora_scaling, groups_per_weight=ctx.gpw, need_lora_grads=need)
+        dx, da, db, ds = GroupedBackwardPlan(x, dy.contiguous(), group_sizes, ctx.weight, lora_a, lora_b, lora_scaling,
+                                             groups_per_weight=ctx.gpw, need_lora_grads=need, z=z if need else None).run()
         if need:
             ds = ds.reshape(lora_scaling.shape).to(lora_scaling.dtype) if lora_scaling.ndim else ds.sum()
         return dx, da, db, ds, None, None, None
@@ -1422,32 +1435,35 @@ class _MoeExpertMlpFunction(torch.autograd.Function):
             factors = _scaling_vector(lora_scaling.detach() if isinstance(lora_scaling, torch.Tensor) else lora_scaling,
                                       n_experts, hidden.device)
         _, group_sizes, sort_indices, unsort, _ = moe_dispatch(None, selected, n_experts, repeat=top_k)
-        fused = grouped_forward(hidden, group_sizes, gate_up_weight, gate_up_a, gate_up_b, factors,
-                                row_map=sort_indices, row_repeat=top_k)
+        want_z = any(ctx.needs_input_grad[2:7])
+        gate_up = GroupedForwardPlan(hidden, group_sizes, gate_up_weight, gate_up_a, gate_up_b, factors,
+                                     row_map=sort_indices, row_repeat=top_k, want_z=want_z)
+        fused = gate_up.run()
         act = swiglu(fused)
-        down = grouped_forward(act, group_sizes, down_weight, down_a, down_b, factors)
+        down_plan = GroupedForwardPlan(act, group_sizes, down_weight, down_a, down_b, factors, want_z=want_z)
+        down = down_plan.run()
         ctx.save_for_backward(hidden, weights, gate_up_a, gate_up_b, down_a, down_b, lora_scaling, group_sizes,
-                              sort_indices, unsort, fused, act, down, factors)
+                              sort_indices, unsort, fused, act, down, factors, gate_up.z, down_plan.z)
         ctx.gate_up_weight, ctx.down_weight, ctx.top_k = gate_up_weight, down_weight, top_k
         return moe_combine(down, unsort, weights)
 
     @staticmethod
     def backward(ctx, d_out):
         (hidden, weights, gate_up_a, gate_up_b, down_a, down_b, lora_scaling, group_sizes, sort_indices, unsort, fused,
-         act, down, factors) = ctx.saved_tensors
+         act, down, factors, z_gate_up, z_down) = ctx.saved_tensors
         top_k = ctx.top_k
         lora = gate_up_a is not None
         need_lora = lora and any(ctx.needs_input_grad[2:7])
         need_w = ctx.needs_input_grad[1]
         d_down, d_w = moe_combine_backward(d_out.contiguous(), down if need_w else None, sort_indices, weights,
                                            need_weight_grads=need_w)
-        d_act, d_da, d_db, ds_dn = grouped_backward(act, d_down, group_sizes, ctx.down_weight, down_a, down_b,
-                                                    factors, need_lora_grads=need_lora)
+        d_act, d_da, d_db, ds_dn = GroupedBackwardPlan(act, d_down, group_sizes, ctx.down_weight, down_a, down_b, factors,
+                                                       need_lora_grads=need_lora, z=z_down if need_lora else None).run()
         d_fused = swiglu_backward(fused, d_act)
         # (the LoRA cotangents of gate/up contract over the sorted hidden rows, read through the sort)
-        d_xs, d_ga, d_gb, ds_gu = grouped_backward(hidden if need_lora else None, d_fused, group_sizes, ctx.gate_up_weight,
-                                                   gate_up_a, gate_up_b, factors, need_lora_grads=need_lora,
-                                                   row_map=sort_indices, row_repeat=top_k)
+        d_xs, d_ga, d_gb, ds_gu = GroupedBackwardPlan(hidden if need_lora else None, d_fused, group_sizes, ctx.gate_up_weight,
+                                                      gate_up_a, gate_up_b, factors, need_lora_grads=need_lora, row_map=sort_indices,
+                                                      row_repeat=top_k, z=z_gate_up if need_lora else None).run()
         d_hidden = None
         if ctx.needs_input_grad[0]:
             d_hidden = moe_combine(d_xs, unsort, torch.ones_like(weights))
@@ -1929,10 +1945,11 @@ class _QkvStageFunction(torch.autograd.Function):
         ctx.saved_projection = bool(save_projection)
         gamma = _one_plus(input_norm_weight)
         plan = ForwardPlan(hidden, weight, lora_a, lora_b, lora_scaling, adapter_indices=adapter_indices,
-                           rms_gamma=gamma, eps=config.rms_norm_eps, want_normalized=ctx.saved_projection)
+                           rms_gamma=gamma, eps=config.rms_norm_eps, want_normalized=ctx.saved_projection,
+                           want_z=ctx.saved_projection and lora_a is not None and any(ctx.needs_input_grad[4:7]))
         fused = plan.run()
         ctx.adapter_indices = plan.adapter_indices  # (one per row; like the float32 norm weights made once for both directions)
-        keep = (fused, plan.aux["normalized"]) if ctx.saved_projection else ()
+        keep = (fused, plan.aux["normalized"], plan.z) if ctx.saved_projection else ()
         q_w, k_w = (w.detach().to(device=hidden.device, dtype=torch.float32) for w in (q_norm_weight, k_norm_weight))
         # (the weights themselves are saved too: written between the two directions they are refused)
         ctx.save_for_backward(hidden, input_norm_weight, q_norm_weight, k_norm_weight, plan.gamma, q_w, k_w, lora_a, lora_b,
@@ -1944,21 +1961,22 @@ class _QkvStageFunction(torch.autograd.Function):
     def backward(ctx, d_q, d_k, d_v, d_gate):
         hidden, in_w, q_norm, k_norm, gamma, q_w, k_w, lora_a, lora_b, lora_scaling, positions = ctx.saved_tensors[:11]
         config = ctx.config
+        need_lora = lora_a is not None and any(ctx.needs_input_grad[4:7])
         if ctx.saved_projection:
-            fused, normalized = ctx.saved_tensors[11:]
+            fused, normalized, z = ctx.saved_tensors[11:]
         else:
             plan = ForwardPlan(hidden, ctx.weight, lora_a, lora_b, lora_scaling, adapter_indices=ctx.adapter_indices,
-                               rms_gamma=gamma, eps=config.rms_norm_eps, want_normalized=True)
+                               rms_gamma=gamma, eps=config.rms_norm_eps, want_normalized=True, want_z=need_lora)
             fused = plan.run()
-            normalized = plan.aux["normalized"]
-        need_lora = lora_a is not None and any(ctx.needs_input_grad[4:7])
+            normalized, z = plan.aux["normalized"], plan.z
         need_head = ctx.needs_input_grad[2] or ctx.needs_input_grad[3]
         need_in = ctx.needs_input_grad[1]
         d_fused, dqw, dkw = qkv_split_norm_rope_backward(fused, q_w, k_w, positions, config, d_q, d_k, d_v, d_gate,
                                                          need_norm_weight_grads=need_head)
         rows = normalized.shape[0]
-        dn, da, db, ds = backward(normalized, d_fused.reshape(rows, -1), ctx.weight, lora_a, lora_b, lora_scaling,
-                                  adapter_indices=ctx.adapter_indices, need_lora_grads=need_lora)
+        dn, da, db, ds = BackwardPlan(normalized, d_fused.reshape(rows, -1), ctx.weight, lora_a, lora_b, lora_scaling,
+                                      adapter_indices=ctx.adapter_indices, need_lora_grads=need_lora,
+                                      z=z if need_lora else None).run()
         dh, dinw = delta_rms_norm_backward(hidden.reshape(rows, -1), gamma, dn, eps=config.rms_norm_eps,
                                            need_weight_grad=need_in, in_place=not need_in)
         if need_lora:
