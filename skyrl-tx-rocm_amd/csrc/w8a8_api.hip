@@ -1735,7 +1735,8 @@ int run_qkv_post(const mi355_w8a8_qkv_post_problem* p, hipStream_t s) {
   a.M = p->m; a.Hq = p->num_query_heads; a.Hkv = p->num_kv_heads; a.D = p->head_dim; a.rot = p->rotary_dim;
   a.width = (uint32_t)width; a.theta = p->rope_theta; a.eps = p->rms_eps;
   (void)hipGetLastError();
-  hipLaunchKernelGGL(qkv_post_kernel, dim3(p->m), dim3(256), 0, s, a);
+  if (p->head_dim <= 256u) hipLaunchKernelGGL((qkv_post_kernel<1>), dim3(p->m), dim3(256), 0, s, a);
+  else hipLaunchKernelGGL((qkv_post_kernel<2>), dim3(p->m), dim3(256), 0, s, a);
   return launch_status();
 }
 
@@ -1796,7 +1797,8 @@ int run_qkv_post_bwd(const mi355_w8a8_qkv_post_bwd_problem* p, hipStream_t s) {
   const bool vec4 = (p->head_dim & 3u) == 0;
   (void)hipGetLastError();
   if (wgrad) {
-    if (vec4) hipLaunchKernelGGL((qkv_post_bwd_kernel<4, true>), dim3(parts), dim3(256), 0, s, a);
+    if (vec4 && p->head_dim <= 256u) hipLaunchKernelGGL((qkv_post_bwd_kernel<4, true, 1>), dim3(parts), dim3(256), 0, s, a);
+    else if (vec4) hipLaunchKernelGGL((qkv_post_bwd_kernel<4, true>), dim3(parts), dim3(256), 0, s, a);
     else hipLaunchKernelGGL((qkv_post_bwd_kernel<1, true>), dim3(parts), dim3(256), 0, s, a);
     int st;
     if ((st = launch_status())) return st;
@@ -1807,7 +1809,8 @@ int run_qkv_post_bwd(const mi355_w8a8_qkv_post_bwd_problem* p, hipStream_t s) {
     c.out = p->d_k_norm_weight; c.col0 = p->head_dim;
     hipLaunchKernelGGL(column_sum_kernel, dim3((p->head_dim + 15u) / 16u), dim3(256), 0, s, c);
   } else {
-    if (vec4) hipLaunchKernelGGL((qkv_post_bwd_kernel<4, false>), dim3(p->m), dim3(256), 0, s, a);
+    if (vec4 && p->head_dim <= 256u) hipLaunchKernelGGL((qkv_post_bwd_kernel<4, false, 1>), dim3(p->m), dim3(256), 0, s, a);
+    else if (vec4) hipLaunchKernelGGL((qkv_post_bwd_kernel<4, false>), dim3(p->m), dim3(256), 0, s, a);
     else hipLaunchKernelGGL((qkv_post_bwd_kernel<1, false>), dim3(p->m), dim3(256), 0, s, a);
   }
   return launch_status();

@@ -245,9 +245,15 @@ __global__ __launch_bounds__(256) void bwd_r_finish_kernel(BwdRFinishArgs a) {
       if (a.z_rows) {  // kernel-uniform
         const int src = a.src_row ? a.src_row[slot] : (int)slot;
         const bool row_ok = src >= 0 && src < (int)a.M;
+        const float* zr = a.z_rows + (row_ok && col < a.r ? (size_t)src * a.r + col : 0u);
+        if ((a.r & 3u) == 0) {  // kernel-uniform
+          const float4 v4 = *reinterpret_cast<const float4*>(zr);
+          if (row_ok && col < a.r) { z[0] = v4.x; z[1] = v4.y; z[2] = v4.z; z[3] = v4.w; }
+        } else {
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (row_ok && col + e < a.r) z[e] = a.z_rows[(size_t)src * a.r + col + e];
+          for (int e = 0; e < 4; ++e)
+            if (row_ok && col + e < a.r) z[e] = zr[e];
+        }
       }
 #pragma unroll
       for (uint32_t sl = 0; sl < kBwdMaxSlices; ++sl)

@@ -51,3 +51,36 @@ def test_route_of_equal_and_missing_probabilities(t, e, k):
     torch.testing.assert_close(selected.cpu().long(), order, rtol=0, atol=0)
     # both softmaxes round the exponential, a sum of at most e terms and the quotient
     torch.testing.assert_close(weights.cpu(), torch.gather(prob, 1, order), rtol=(e + 4) * 2.0 ** -24, atol=0)
+
+
+@pytest.mark.parametrize("m,k", [(33, 64), (130, 2560), (600, 8224)])
+def test_codes_of_every_kind_of_row_on_tiles(m, k):
+    """The tiled prologues: a NaN takes the row's scale to 1, its own code and a value's below -128 are -128, above 127 127."""
+    import torch
+
+    pkg = load_package()
+    case = wc.make_case(m, k, 64, n_adapters=3, rank=8, seed=m + k)
+    x = torch.from_numpy(np.random.default_rng(k).standard_normal((m, k)).astype(np.float32)).to(torch.bfloat16)
+    for row in range(m):
+        kind = (row * 5) % 8
+        if kind == 1: x[row] *= 2.0 ** -120
+        elif kind == 2: x[row] *= 2.0 ** 110
+        elif kind == 3: x[row] = (torch.arange(k) % 255 - 127) * 0.5
+        elif kind == 4: x[row] = 0.0
+        elif kind == 5: x[row] *= 100.0; x[row, k // 3] = float("nan")
+        elif kind == 6: x[row, k // 2] = float("inf")
+        elif kind == 7: x[row] = torch.where(torch.arange(k) % 2 == 0, 64.0, -0.25 * (torch.arange(k) % 256))
+    t = wc.to_torch(case, "cuda:0")
+    v = x.float().numpy()
+    nan = np.isnan(v).any(axis=1)
+    amax = np.nanmax(np.abs(v), axis=1)
+    scale = np.where(nan | (amax == 0), np.float32(1), amax / np.float32(127)).astype(np.float32)
+    with np.errstate(invalid="ignore"):
+        q = (v / scale[:, None]).astype(np.float32)
+    codes = np.clip(np.rint(np.where(np.isnan(q), np.float32(-128), q)), -128, 127).astype(np.int8)
+    for lora in (False, True):
+        args = (t["a"], t["b"], t["s"]) if lora else ()
+        _, aux = pkg.w8a8_lora.forward(x.cuda(), t["weight"], *args, adapter_indices=t["idx"] if lora else None, return_aux=True,
+                                       flags=pkg._native.FLAG_FORCE_TILED)
+        np.testing.assert_array_equal(aux["x_scales"].cpu().numpy(), scale)
+        np.testing.assert_array_equal(aux["x_codes"].cpu().numpy(), codes)
