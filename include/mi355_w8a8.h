@@ -263,6 +263,8 @@ typedef struct mi355_w8a8_grouped_bwd_problem_z {
   const float* z;           /* f32 [m, rank], rows as sorted */
 } mi355_w8a8_grouped_bwd_problem_z;
 
+/* The two head-norm weights of a stage call are bf16 (16-byte aligned as else), read as their float32 values. */
+#define MI355_W8A8_FLAG_QKV_WEIGHTS_BF16 1u
 /*
  * Qwen3.5 attention input stage behind the fused QKV projection: split of the interleaved
  * projection (per kv head: queries_per_kv (q, gate) chunk pairs, then k, then v), RMSNorm with
@@ -270,7 +272,7 @@ typedef struct mi355_w8a8_grouped_bwd_problem_z {
  */
 typedef struct mi355_w8a8_qkv_post_problem {
   uint32_t struct_size;     /* sizeof(mi355_w8a8_qkv_post_problem) */
-  uint32_t flags;           /* 0 */
+  uint32_t flags;           /* 0 or MI355_W8A8_FLAG_QKV_WEIGHTS_BF16 */
   uint32_t m;               /* rows (batch * sequence) */
   uint32_t num_query_heads;
   uint32_t num_kv_heads;    /* divides num_query_heads */
@@ -296,7 +298,7 @@ typedef struct mi355_w8a8_qkv_post_problem {
  */
 typedef struct mi355_w8a8_qkv_post_bwd_problem {
   uint32_t struct_size;     /* sizeof(mi355_w8a8_qkv_post_bwd_problem) */
-  uint32_t flags;           /* 0 */
+  uint32_t flags;           /* 0 or MI355_W8A8_FLAG_QKV_WEIGHTS_BF16 */
   uint32_t m;
   uint32_t num_query_heads;
   uint32_t num_kv_heads;

@@ -31,6 +31,7 @@ FLAG_TILE_128X128 = 2048
 FLAG_TILE_256X128_PAIR = 4096
 FLAG_DECODE_B_WRITE = 8192
 FLAG_DECODE_B_KEPT = 16384
+FLAG_QKV_WEIGHTS_BF16 = 1  # of the two QKV stage problems
 FLAG_GQ_DIRECT = 1  # mi355_w8a8_gq_problem.flags
 FLAG_GQ_BF16_SCALES = 2  # mi355_w8a8_gq_bwd_problem.flags
 STATIC_WORKSPACE_BYTES = 32 << 20

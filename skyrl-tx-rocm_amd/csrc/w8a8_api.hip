@@ -1705,7 +1705,7 @@ int run_grouped_backward(const mi355_w8a8_grouped_bwd_problem* given, hipStream_
 int run_qkv_post(const mi355_w8a8_qkv_post_problem* p, hipStream_t s) {
   if (!p) return MI355_W8A8_ERR_NULL;
   if (p->struct_size != sizeof(mi355_w8a8_qkv_post_problem)) return MI355_W8A8_ERR_STRUCT;
-  if (p->flags) return MI355_W8A8_ERR_SHAPE;
+  if (p->flags & ~MI355_W8A8_FLAG_QKV_WEIGHTS_BF16) return MI355_W8A8_ERR_SHAPE;
   if (p->m == 0 || p->num_query_heads == 0 || p->num_kv_heads == 0 || p->head_dim == 0) return MI355_W8A8_ERR_SHAPE;
   if (p->num_query_heads % p->num_kv_heads) return MI355_W8A8_ERR_SHAPE;
   if ((p->head_dim & 1u) || (p->rotary_dim & 1u) || p->rotary_dim > p->head_dim) return MI355_W8A8_ERR_SHAPE;
@@ -1730,6 +1730,7 @@ int run_qkv_post(const mi355_w8a8_qkv_post_problem* p, hipStream_t s) {
   QkvPostArgs a{};
   a.fused = static_cast<const uint16_t*>(p->fused);
   a.q_w = p->q_norm_weight; a.k_w = p->k_norm_weight; a.pos = p->positions;
+  a.w_bf16 = p->flags & MI355_W8A8_FLAG_QKV_WEIGHTS_BF16 ? 1u : 0u;
   a.q = static_cast<uint16_t*>(p->q); a.k = static_cast<uint16_t*>(p->k);
   a.v = static_cast<uint16_t*>(p->v); a.gate = static_cast<uint16_t*>(p->gate);
   a.M = p->m; a.Hq = p->num_query_heads; a.Hkv = p->num_kv_heads; a.D = p->head_dim; a.rot = p->rotary_dim;
@@ -1749,7 +1750,7 @@ inline uint64_t qkv_bwd_workspace_bytes(uint32_t m, uint32_t head_dim) {
 int run_qkv_post_bwd(const mi355_w8a8_qkv_post_bwd_problem* p, hipStream_t s) {
   if (!p) return MI355_W8A8_ERR_NULL;
   if (p->struct_size != sizeof(mi355_w8a8_qkv_post_bwd_problem)) return MI355_W8A8_ERR_STRUCT;
-  if (p->flags) return MI355_W8A8_ERR_SHAPE;
+  if (p->flags & ~MI355_W8A8_FLAG_QKV_WEIGHTS_BF16) return MI355_W8A8_ERR_SHAPE;
   if (p->m == 0 || p->num_query_heads == 0 || p->num_kv_heads == 0 || p->head_dim == 0) return MI355_W8A8_ERR_SHAPE;
   if (p->num_query_heads % p->num_kv_heads) return MI355_W8A8_ERR_SHAPE;
   if ((p->head_dim & 1u) || (p->rotary_dim & 1u) || p->rotary_dim > p->head_dim) return MI355_W8A8_ERR_SHAPE;
@@ -1788,6 +1789,7 @@ int run_qkv_post_bwd(const mi355_w8a8_qkv_post_bwd_problem* p, hipStream_t s) {
   QkvPostBwdArgs a{};
   a.fused = static_cast<const uint16_t*>(p->fused);
   a.q_w = p->q_norm_weight; a.k_w = p->k_norm_weight; a.pos = p->positions;
+  a.w_bf16 = p->flags & MI355_W8A8_FLAG_QKV_WEIGHTS_BF16 ? 1u : 0u;
   a.dq = static_cast<const uint16_t*>(p->d_q); a.dk = static_cast<const uint16_t*>(p->d_k);
   a.dv = static_cast<const uint16_t*>(p->d_v); a.dgate = static_cast<const uint16_t*>(p->d_gate);
   a.dfused = static_cast<uint16_t*>(p->d_fused);

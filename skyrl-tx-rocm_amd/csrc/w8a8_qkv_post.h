@@ -35,20 +35,32 @@ __device__ inline void qkv_fetch(QkvPieces<NP>& t, const uint16_t* a, const uint
     }
   }
 }
+// Norm weight i as float32: the tensor may be bf16 (the model's own; converted by the caller it took a launch of 2 us for each).
+__device__ inline float qkv_weight(const float* w, uint32_t i, bool bf16) {
+  return bf16 ? bf16_bits_to_f32(reinterpret_cast<const uint16_t*>(w)[i]) : w[i];  // (kernel-uniform)
+}
 // 1 + weight of the lane's elements
 template <uint32_t NP>
-__device__ inline void qkv_weights(float4 (&w)[NP], const float* src, uint32_t D, uint32_t lane) {
+__device__ inline void qkv_weights(float4 (&w)[NP], const float* src, bool bf16, uint32_t D, uint32_t lane) {
 #pragma unroll
   for (uint32_t j = 0; j < NP; ++j) {
     const uint32_t i = 4u * lane + 256u * j;
-    const float4 v = i < D ? *reinterpret_cast<const float4*>(src + i) : make_float4(0.f, 0.f, 0.f, 0.f);
+    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (i < D) {
+      if (bf16) {
+        const uint2 r = *reinterpret_cast<const uint2*>(reinterpret_cast<const uint16_t*>(src) + i);
+        v = make_float4(__uint_as_float(r.x << 16), __uint_as_float(r.x & 0xffff0000u), __uint_as_float(r.y << 16), __uint_as_float(r.y & 0xffff0000u));
+      } else {
+        v = *reinterpret_cast<const float4*>(src + i);
+      }
+    }
     w[j] = make_float4(1.0f + v.x, 1.0f + v.y, 1.0f + v.z, 1.0f + v.w);
   }
 }
 
 struct QkvPostArgs {
   const uint16_t* fused;   // bf16 [M, width]
-  const float* q_w;        // f32 [D] delta weights of the Q norm
+  const float* q_w;        // f32 [D] delta weights of the Q norm (w_bf16: bf16, like k_w)
   const float* k_w;        // f32 [D]
   const int32_t* pos;      // int32 [M]
   uint16_t* q;             // bf16 [M, Hq, D]
@@ -57,6 +69,7 @@ struct QkvPostArgs {
   uint16_t* gate;          // bf16 [M, Hq * D]
   uint32_t M, Hq, Hkv, D, rot, width;
   float theta, eps;
+  uint32_t w_bf16;
 };
 
 template <uint32_t NP>
@@ -79,8 +92,8 @@ __global__ __launch_bounds__(256) void qkv_post_kernel(QkvPostArgs a) {
   float4 wq[NP], wk[NP];
   if (vec4) {
     if (wave < units) qkv_fetch(next, chunk(wave), chunk(wave) + a.D, a.D, lane);
-    qkv_weights(wq, a.q_w, a.D, lane);
-    qkv_weights(wk, a.k_w, a.D, lane);
+    qkv_weights(wq, a.q_w, a.w_bf16 != 0u, a.D, lane);
+    qkv_weights(wk, a.k_w, a.w_bf16 != 0u, a.D, lane);
   }
   // angle[i] = position / theta^(2 i / rot), all float32 (qwen3_5_qkv_lora.py:119-127)
   const float position = (float)a.pos[row];
@@ -184,7 +197,7 @@ __global__ __launch_bounds__(256) void qkv_post_kernel(QkvPostArgs a) {
     for (uint32_t i = lane; i < a.D; i += 64u) {
       const float x = bf16_bits_to_f32(frow[off + i]);
       float t = x * inv;
-      t = t * (1.0f + w[i]);
+      t = t * (1.0f + qkv_weight(w, i, a.w_bf16 != 0u));
       buf[wave][i] = bf16_round_f32(t);
     }
     __builtin_amdgcn_s_waitcnt(0xc07f);
@@ -225,6 +238,7 @@ struct QkvPostBwdArgs {
   float* partial;          // f32 [gridDim.x][2][D] when the weight cotangents are wanted
   uint32_t M, Hq, Hkv, D, rot, width;
   float theta, eps;
+  uint32_t w_bf16;
 };
 
 // V consecutive elements per lane and piece (V = 4: 8-byte accesses; V = 1: any geometry); a head
@@ -247,8 +261,8 @@ __global__ __launch_bounds__(256) void qkv_post_bwd_kernel(QkvPostBwdArgs a) {
   uint2 next_copy[NP];
   float4 one_q[NP], one_k[NP];
   if constexpr (V == 4) {
-    qkv_weights(one_q, a.q_w, a.D, lane);
-    qkv_weights(one_k, a.k_w, a.D, lane);
+    qkv_weights(one_q, a.q_w, a.w_bf16 != 0u, a.D, lane);
+    qkv_weights(one_k, a.k_w, a.w_bf16 != 0u, a.D, lane);
   }
   auto unit_off = [&](uint32_t u) -> uint32_t {
     return u < a.Hq ? u / qpk * group_width + (u % qpk) * 2u * a.D : (u - a.Hq) * group_width + qpk * 2u * a.D;
@@ -347,7 +361,7 @@ __global__ __launch_bounds__(256) void qkv_post_bwd_kernel(QkvPostBwdArgs a) {
               const float4 o4 = is_q ? one_q[j] : one_k[j];
               one = e == 0 ? o4.x : e == 1 ? o4.y : e == 2 ? o4.z : o4.w;
             } else {
-              one = 1.0f + w[c];
+              one = 1.0f + qkv_weight(w, c, a.w_bf16 != 0u);
             }
             p[V * j + e] = uo * one;
             sp += (double)(p[V * j + e] * n[V * j + e]);

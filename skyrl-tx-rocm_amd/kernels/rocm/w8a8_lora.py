@@ -1691,12 +1691,21 @@ class Qwen35QKVStageConfig:
         return self.q_projection_width + 2 * self.kv_projection_width
 
 
+def _head_norm_weights(q_w: torch.Tensor, k_w: torch.Tensor, dev, as_they_are: bool):
+    """The two head-norm weights as a stage call takes them, and its flags: float32, or (for a call that runs at once) the
+    model's own bf16 tensors, whose conversion is a launch each."""
+    q_w, k_w = q_w.detach(), k_w.detach()
+    if as_they_are and all(w.dtype == torch.bfloat16 and w.device == dev and w.is_contiguous() and w.data_ptr() % 16 == 0 for w in (q_w, k_w)):
+        return q_w, k_w, _native.FLAG_QKV_WEIGHTS_BF16
+    return *(w.to(device=dev, dtype=torch.float32).contiguous() for w in (q_w, k_w)), 0
+
+
 class QkvPostPlan:
     """Outputs and the C struct of one split / Q-K norm / partial-RoPE call; ``run()`` is a single
     C call on torch's current stream (see ``ForwardPlan``)."""
 
     def __init__(self, fused: torch.Tensor, q_norm_weight: torch.Tensor, k_norm_weight: torch.Tensor,
-                 positions: torch.Tensor, config: Qwen35QKVStageConfig):
+                 positions: torch.Tensor, config: Qwen35QKVStageConfig, *, run_once: bool = False):
         if fused.dtype != torch.bfloat16:
             raise TypeError(f"fused must be BF16, got {fused.dtype}")
         _require_cuda(fused, "fused")
@@ -1711,8 +1720,8 @@ class QkvPostPlan:
         dev = fused.device
         flat = fused.reshape(-1, config.fused_width).contiguous()
         m = flat.shape[0]
-        qw = q_norm_weight.to(device=dev, dtype=torch.float32).contiguous()
-        kw = k_norm_weight.to(device=dev, dtype=torch.float32).contiguous()
+        # (a plan that is kept holds the weights as they are now)
+        qw, kw, flags = _head_norm_weights(q_norm_weight, k_norm_weight, dev, run_once)
         pos = positions.reshape(-1).to(device=dev, dtype=torch.int32).contiguous()
         self.q = torch.empty((m, config.num_query_heads, d), dtype=torch.bfloat16, device=dev)
         self.k = torch.empty((m, config.num_kv_heads, d), dtype=torch.bfloat16, device=dev)
@@ -1720,6 +1729,7 @@ class QkvPostPlan:
         self.gate = torch.empty((m, config.num_query_heads * d), dtype=torch.bfloat16, device=dev)
         p = _native.QkvPostProblem()
         p.struct_size = ctypes.sizeof(_native.QkvPostProblem)
+        p.flags = flags
         p.m, p.num_query_heads, p.num_kv_heads = m, config.num_query_heads, config.num_kv_heads
         p.head_dim, p.rotary_dim = d, config.rotary_dim
         p.rope_theta, p.rms_eps = float(config.rope_theta), float(config.rms_norm_eps)
@@ -1747,7 +1757,7 @@ def qkv_split_norm_rope(fused: torch.Tensor, q_norm_weight: torch.Tensor, k_norm
     """Split of the interleaved projection, Q/K RMSNorm with ``1 + weight``, partial RoPE
     (qwen3_5_qkv_lora.py:266-286).  ``fused`` is bf16 [..., fused_width], ``positions`` int [...].
     Returns q [..., Hq, D], k [..., Hkv, D], v [..., Hkv, D], gate [..., Hq * D]."""
-    return QkvPostPlan(fused, q_norm_weight, k_norm_weight, positions, config).run()
+    return QkvPostPlan(fused, q_norm_weight, k_norm_weight, positions, config, run_once=True).run()
 
 
 def qkv_split_norm_rope_backward(fused: torch.Tensor, q_norm_weight: torch.Tensor, k_norm_weight: torch.Tensor,
@@ -1782,13 +1792,13 @@ def qkv_split_norm_rope_backward(fused: torch.Tensor, q_norm_weight: torch.Tenso
 
     dq, dk = cot(d_q, hq * d, "d_q"), cot(d_k, hkv * d, "d_k")
     dv, dg = cot(d_v, hkv * d, "d_v"), cot(d_gate, hq * d, "d_gate")
-    qw = q_norm_weight.to(device=dev, dtype=torch.float32).contiguous()
-    kw = k_norm_weight.to(device=dev, dtype=torch.float32).contiguous()
+    qw, kw, flags = _head_norm_weights(q_norm_weight, k_norm_weight, dev, True)
     pos = positions.reshape(-1).to(device=dev, dtype=torch.int32).contiguous()
     d_fused = torch.empty_like(flat)
     lib = _native.load()
     p = _native.QkvPostBwdProblem()
     p.struct_size = ctypes.sizeof(_native.QkvPostBwdProblem)
+    p.flags = flags
     p.m, p.num_query_heads, p.num_kv_heads, p.head_dim, p.rotary_dim = m, hq, hkv, d, config.rotary_dim
     p.rope_theta, p.rms_eps = float(config.rope_theta), float(config.rms_norm_eps)
     p.fused, p.q_norm_weight, p.k_norm_weight, p.positions = flat.data_ptr(), qw.data_ptr(), kw.data_ptr(), pos.data_ptr()
@@ -1950,7 +1960,7 @@ class _QkvStageFunction(torch.autograd.Function):
         fused = plan.run()
         ctx.adapter_indices = plan.adapter_indices  # (one per row; like the float32 norm weights made once for both directions)
         keep = (fused, plan.aux["normalized"], plan.z) if ctx.saved_projection else ()
-        q_w, k_w = (w.detach().to(device=hidden.device, dtype=torch.float32) for w in (q_norm_weight, k_norm_weight))
+        q_w, k_w, _ = _head_norm_weights(q_norm_weight, k_norm_weight, hidden.device, True)
         # (the weights themselves are saved too: written between the two directions they are refused)
         ctx.save_for_backward(hidden, input_norm_weight, q_norm_weight, k_norm_weight, plan.gamma, q_w, k_w, lora_a, lora_b,
                               lora_scaling, positions, *keep)
