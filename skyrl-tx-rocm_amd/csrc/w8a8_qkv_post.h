@@ -19,8 +19,10 @@ __device__ inline float qkv_mean(double sum, uint32_t D) {
   return (float)((D & (D - 1u)) == 0u ? sum * (1.0 / (double)D) : sum / (double)D);  // (kernel-uniform; 1 / D is formed once)
 }
 // Four elements a lane and piece of the two chunks of a unit.  A wave asks for the next unit's before it works on one, and for its
-// first before the rotation's table is formed: one after the other the units were a chain of loads and of two sums over the
-// wave each.  2048 rows of 16 + 4 heads of 256: forward 22.6 us, now 21.1 (84 MB, 4.0 TB/s); backward 40.8, now 31.5 (126 MB).
+// first before the rotation's table is formed; the norm weights stay in registers.  Instructions bound it as much as memory
+// (40960 heads of 300 each, float64 sums and two divisions among them: the loads ahead alone gave the pull-back 0.2 us; the rest
+// is the mean as a product and the weights held).  2048 rows of 16 + 4 heads of 256: forward 22.6 us, now 21.1 (84 MB, 4.0 TB/s);
+// backward 40.8, now 31.5 (126 MB).
 // NP: pieces, one for heads of up to 256.
 template <uint32_t NP> struct QkvPieces { uint2 a[NP], b[NP]; };
 template <uint32_t NP>
