@@ -138,11 +138,15 @@ typedef struct mi355_w8a8_problem {
   int32_t* aux_acc;         /* int32 [m, n] raw integer accumulators */
   void* aux_normalized;     /* bf16 [m, k] RMSNorm output (only with rms_gamma) */
 } mi355_w8a8_problem;
-/* The same call with struct_size = sizeof of this: it leaves x @ A[idx], which the backward contracts with dy.  Taken where
- * mi355_w8a8_forward_keeps_z says so. */
+/* The same call with struct_size = sizeof of this.  With z it leaves x @ A[idx], which the backward contracts with dy: taken where
+ * mi355_w8a8_forward_keeps_z says so.  With rows_per_index > 1, a divisor of m, adapter_indices holds one entry for as many rows that
+ * follow each other, m / rows_per_index in all: not taken by the two decode paths of
+ * mi355_w8a8_forward_path. */
 typedef struct mi355_w8a8_problem_z {
   mi355_w8a8_problem call;
-  float* z;                 /* f32 [m, rank] */
+  float* z;                 /* f32 [m, rank] or NULL */
+  uint32_t rows_per_index;  /* 0 or 1: an entry per row */
+  uint32_t reserved;
 } mi355_w8a8_problem_z;
 
 /*

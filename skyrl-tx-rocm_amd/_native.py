@@ -122,7 +122,7 @@ class GroupedBwdProblem(ctypes.Structure):
 class ProblemZ(ctypes.Structure):
     """struct mi355_w8a8_problem_z"""
 
-    _fields_ = [("call", Problem), ("z", _vp)]
+    _fields_ = [("call", Problem), ("z", _vp), ("rows_per_index", _u32), ("reserved", _u32)]
 
 
 class GroupedProblemZ(ctypes.Structure):
@@ -352,7 +352,7 @@ def host():
             module = importlib.util.module_from_spec(importlib.util.spec_from_loader("mi355_w8a8_host", loader))
             loader.exec_module(module)
             for name, fn in (("forward", "forward_v1"), ("linear", "lora_linear_v1"), ("gateup", "rms_gateup_swiglu_v1"),
-                             ("residual", "lora_residual_v1"), ("workspace_bytes", "workspace_bytes"),
+                             ("residual", "lora_residual_v1"), ("workspace_bytes", "workspace_bytes"), ("forward_path", "forward_path"),
                              ("gq_linear", "gq_linear_v1"), ("gq_workspace_bytes", "gq_workspace_bytes")):
                 entry_address[name] = ctypes.cast(getattr(lib, f"mi355_w8a8_{fn}"), ctypes.c_void_p).value
             _host = module

@@ -563,8 +563,12 @@ bool forward_keeps_z(uint32_t m, uint32_t k, uint32_t n, uint32_t n_adapters, ui
 int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
   if (!p) return MI355_W8A8_ERR_NULL;
   float* z_rows = nullptr;
-  if (p->struct_size == sizeof(mi355_w8a8_problem_z)) z_rows = reinterpret_cast<const mi355_w8a8_problem_z*>(p)->z;
-  else if (p->struct_size != sizeof(mi355_w8a8_problem)) return MI355_W8A8_ERR_STRUCT;
+  uint32_t rows_per_index = 1;
+  if (p->struct_size == sizeof(mi355_w8a8_problem_z)) {
+    const mi355_w8a8_problem_z* const whole = reinterpret_cast<const mi355_w8a8_problem_z*>(p);
+    z_rows = whole->z;
+    rows_per_index = whole->rows_per_index > 1u ? whole->rows_per_index : 1u;
+  } else if (p->struct_size != sizeof(mi355_w8a8_problem)) return MI355_W8A8_ERR_STRUCT;
   int st = validate_common(p->m, p->k, p->n);
   if (st) return st;
   if (z_rows && !forward_keeps_z(p->m, p->k, p->n, p->n_adapters, p->rank, p->flags)) return MI355_W8A8_ERR_UNSUPPORTED;
@@ -586,6 +590,7 @@ int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
   } else if (p->adapter_indices) {
     return MI355_W8A8_ERR_SHAPE;
   }
+  if (rows_per_index > 1u && (!p->adapter_indices || p->m % rows_per_index)) return MI355_W8A8_ERR_SHAPE;
   if (p->aux_normalized && !rms) return MI355_W8A8_ERR_SHAPE;
   const uint32_t n_out = swiglu ? p->n / 2u : p->n;
   const uint64_t out_bytes = (uint64_t)p->m * n_out * 2u;
@@ -611,6 +616,7 @@ int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
   if (reinterpret_cast<uintptr_t>(p->workspace) & 255u) return MI355_W8A8_ERR_ALIGN;
   const int reported = choose_forward_path(p->m, p->k, p->n, p->flags);
   if (reported < 0) return reported;
+  if (rows_per_index > 1u && (reported == MI355_W8A8_PATH_SKINNY || reported == MI355_W8A8_PATH_SKINNY_CHUNKS)) return MI355_W8A8_ERR_UNSUPPORTED;
   int path = reported;
   if (path == MI355_W8A8_PATH_SKINNY_CHUNKS) {
     const uint32_t groups = routed ? p->n_adapters : 1u, slots = groups > 1u ? padded_rows_bound(p->m, groups) : round_up(p->m, 32u);
@@ -675,7 +681,7 @@ int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
   const bool ksplit = may_ksplit && ksplit_fits(w.rows_bound, p->n);
   const bool split_z = ksplit && w.split_bytes && split_z_pays(p->m, p->k, w.nkk, ksplit_tiles(w.rows_bound, p->n)) && p->workspace_bytes >= w.split_z + w.split_bytes;
   const bool rows_in_lds = !split_z && prologue_keeps_rows(w.rows_bound, p->k, rms, lora, pack, routed && !pad_groups);
-  const bool route_inline = rows_in_lds && routed && !pack && p->m <= kInlineRouteMaxRows;
+  const bool route_inline = rows_in_lds && routed && !pack && p->m <= kInlineRouteMaxRows && rows_per_index == 1u;
   // launch 1: adapter routing, the rows' statistics and (unless the workspace holds them) the LoRA operands
   const uint32_t route_blocks = routed && !route_inline ? 1u : 0u, stat_blocks = rows_in_lds ? 0u : (p->m + 15u) / 16u;
   if (!skip_prologue && (route_blocks || stat_blocks || pack)) {
@@ -689,6 +695,7 @@ int run_forward(const mi355_w8a8_problem* p, hipStream_t s, Required req) {
     pa.M = p->m; pa.K = p->k; pa.N = p->n; pa.n_groups = p->n_adapters; pa.r = p->rank; pa.nkk = w.nkk;
     pa.ncb = n_padded(p->n) / 32u; pa.slots = w.slots;
     pa.route_blocks = route_blocks;
+    pa.rows_per_index = rows_per_index;
     pa.route_pad = pad_groups ? 32u : 1u;
     pa.a_operand_kb = w.KB;  // the quantizer reads A in MFMA operand order
     pa.stat_blocks = stat_blocks;

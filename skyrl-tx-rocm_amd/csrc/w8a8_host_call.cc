@@ -85,9 +85,10 @@ PyObject* finish(at::Tensor&& out, int status) {
   return status == 0 ? THPVariable_Wrap(std::move(out)) : PyLong_FromLong(status);
 }
 
-// dense(x, packed, scales, k, n, a, b, scaling, adapter_indices, gamma, residual, flags, eps, entry, workspace_bytes, stream)
+// dense(x, packed, scales, k, n, a, b, scaling, adapter_indices, gamma, residual, flags, eps, entry, workspace_bytes, forward_path,
+// stream)
 PyObject* dense(PyObject*, PyObject* const* argv, Py_ssize_t argc) {
-  if (argc != 16) { PyErr_SetString(PyExc_TypeError, "dense takes 16 arguments"); return nullptr; }
+  if (argc != 17) { PyErr_SetString(PyExc_TypeError, "dense takes 17 arguments"); return nullptr; }
   HANDLE_TH_ERRORS
   Args arg{argv};
   const at::Tensor *x = arg.tensor(0), *packed = arg.tensor(1), *scales = arg.tensor(2), *a = arg.tensor(5), *b = arg.tensor(6),
@@ -96,8 +97,9 @@ PyObject* dense(PyObject*, PyObject* const* argv, Py_ssize_t argc) {
   const double eps = PyFloat_Check(argv[12]) ? PyFloat_AS_DOUBLE(argv[12]) : -1.0;
   const auto entry = reinterpret_cast<int (*)(const mi355_w8a8_problem*, void*)>(arg.address(13));
   const auto bytes_of = reinterpret_cast<uint64_t (*)(uint32_t, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t)>(arg.address(14));
-  void* const stream = arg.address(15);
-  if (!arg.ok || !entry || !bytes_of || !packed || !scales || n <= 0 || eps < 0.0) Py_RETURN_NONE;
+  const auto path_of = reinterpret_cast<int (*)(uint32_t, uint32_t, uint32_t, uint32_t)>(arg.address(15));
+  void* const stream = arg.address(16);
+  if (!arg.ok || !entry || !bytes_of || !path_of || !packed || !scales || n <= 0 || eps < 0.0) Py_RETURN_NONE;
   const int64_t m = rows_of(x, k, 2);
   if (m == 0) Py_RETURN_NONE;
   const c10::Device device = x->device();
@@ -117,13 +119,27 @@ PyObject* dense(PyObject*, PyObject* const* argv, Py_ssize_t argc) {
   int status;
   {
     const WithoutGil released;
-    // (one index per example: its rows follow each other)
+    // One index per example, whose rows follow each other: the routing launch of the tiled paths reads it as it is (the decode
+    // kernels take an index per row, and every path an aligned array).
     at::Tensor rows_idx;
-    if (idx) rows_idx = idx->numel() == m ? *idx : idx->reshape({-1, 1}).expand({idx->numel(), m / idx->numel()}).contiguous();
+    uint32_t per = 1;
+    if (idx) {
+      rows_idx = *idx;
+      const int64_t rows = m / idx->numel();
+      if (rows > 1) {
+        const int path = path_of((uint32_t)m, (uint32_t)k, (uint32_t)n, (uint32_t)flags);
+        if (path == MI355_W8A8_PATH_SKINNY || path == MI355_W8A8_PATH_SKINNY_CHUNKS || (reinterpret_cast<uintptr_t>(idx->const_data_ptr()) & 15u))
+          rows_idx = idx->reshape({-1, 1}).expand({idx->numel(), rows}).contiguous();
+        else
+          per = (uint32_t)rows;
+      }
+    }
     out = at::empty(shape, x->options().requires_grad(false));
     const at::Tensor ws = at::empty({(int64_t)bytes}, packed->options().requires_grad(false));
-    mi355_w8a8_problem p{};
-    p.struct_size = sizeof(p);
+    mi355_w8a8_problem_z whole{};
+    whole.rows_per_index = per;
+    mi355_w8a8_problem& p = whole.call;
+    p.struct_size = sizeof(whole);
     p.flags = (uint32_t)flags;
     p.m = (uint32_t)m; p.k = (uint32_t)k; p.n = (uint32_t)n;
     p.n_adapters = (uint32_t)lora.adapters; p.rank = (uint32_t)lora.rank;

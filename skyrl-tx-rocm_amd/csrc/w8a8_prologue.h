@@ -60,6 +60,8 @@ __global__ __launch_bounds__(256) void unpack_weight_kernel(const unsigned char*
 // One workgroup of sixteen waves, each with a contiguous range of the rows: a wave counts its rows per group
 // (lanes with the same group find each other with one ballot per bit of the index, so a group costs a wave one
 // LDS atomic per 64 rows), wave 0 turns the counts into first slots, and the waves place their rows in order.
+// rows_per_index > 1: an index serves that many rows that follow each other.  (Written out per row by a launch in front,
+// 333 rows of nine sequences, 4096 -> 2560, took 34.3 us a call, now 31.8.)
 // Rows so keep their order inside a group: reductions over a group's rows have a fixed order.  Bound by the
 // latency of its few steps: 14 us for
 // 4096 rows with an atomic per row and a search per slot.
@@ -67,7 +69,7 @@ __device__ inline void route_rows_block(const int32_t* __restrict__ idx, uint32_
                                         uint32_t slots, int32_t* __restrict__ src_row,
                                         int32_t* __restrict__ dst_pos, int32_t* __restrict__ slot_group,
                                         int32_t* __restrict__ blk_range, int32_t* __restrict__ group_off = nullptr,
-                                        uint32_t group_pad = 1u) {
+                                        uint32_t group_pad = 1u, uint32_t rows_per_index = 1u) {
   static_assert(kMaxAdapters == 64, "a lane per group");
   __shared__ int wcnt[16][kMaxAdapters];  // rows of group g in wave w; then the wave's next slot in the group
   __shared__ int cnt[kMaxAdapters];
@@ -78,7 +80,8 @@ __device__ inline void route_rows_block(const int32_t* __restrict__ idx, uint32_
   const uint32_t per = (M + 1024u - 1u) / (1024u);  // 64-row steps of a wave
   auto group_at = [&](uint32_t it) -> int {
     const uint32_t i = (wave * per + it) * 64u + lane;
-    const int a = idx[i < M ? i : M - 1u];
+    const uint32_t row = i < M ? i : M - 1u;
+    const int a = idx[rows_per_index > 1u ? row / rows_per_index : row];
     return i < M ? (a < 0 ? 0 : (a >= (int)n_groups ? (int)n_groups - 1 : a)) : -1;
   };
   auto peers_of = [&](int a) -> unsigned long long {  // lanes with this lane's group
@@ -542,6 +545,7 @@ struct LoraPrepArgs {
   uint16_t* at;              // A in operand order
   unsigned char* bp;         // packed B operands
   uint32_t M, K, N, n_groups, r, nkk, ncb, slots, route_blocks, a_blocks;
+  uint32_t rows_per_index;   // rows that an entry of idx serves (0 or 1: one)
   uint32_t route_pad;        // dense routing block: every group's first slot is a multiple of this (0 or 1: packed)
   uint32_t a_operand_kb;     // K_pad / 32: the quantizer's operand order (lora_a_pack_item) ...
   uint32_t a_operand_steps, a_operand_rb;  // ... or ceil(K / 64) and the 32-wide rank blocks of lora_a_kernel's (lora_a_pack32_item)
@@ -672,7 +676,7 @@ __global__ __launch_bounds__(1024, 8) __attribute__((aligned(32768))) void lora_
                          p.tile_blocks, p.zero_out, p.zero_cols, b, p.route_blocks);
     else
       route_rows_block(p.idx, p.M, p.n_groups, p.slots, p.src_row, p.dst_pos, p.slot_group, p.blk_range, nullptr,
-                       p.route_pad > 1u ? p.route_pad : 1u);
+                       p.route_pad > 1u ? p.route_pad : 1u, p.rows_per_index);
     return;
   }
   b -= p.route_blocks;

@@ -435,7 +435,7 @@ def forward(x: torch.Tensor, weight, lora_a=None, lora_b=None, lora_scaling=None
         result = _native.host().dense(
             x, pw.packed, pw.scales, pw.in_features, pw.out_features, lora_a, lora_b, scaling, adapter_indices, rms_gamma,
             residual, flags | _native.FLAG_SWIGLU if swiglu else flags, eps, _native.entry_address[entry],
-            _native.entry_address["workspace_bytes"], _stream_ptr(x.device))
+            _native.entry_address["workspace_bytes"], _native.entry_address["forward_path"], _stream_ptr(x.device))
         if type(result) is int:
             _native.check(f"mi355_w8a8_{entry}", result)
         elif result is not None:

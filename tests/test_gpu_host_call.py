@@ -91,3 +91,44 @@ def test_group_scaled_calls(m, k, n, bits, group, rank):
     assert torch.equal(got.view(torch.int16), want.view(torch.int16))
     assert tuple(gq.forward(x[0], w, a, b, 0.5).shape) == (n,)
     assert torch.equal(gq.forward(x.t().contiguous().t(), w, a, b, torch.tensor(0.5, device="cuda:0")).view(torch.int16), want.view(torch.int16))
+
+
+@pytest.mark.parametrize("examples,rows,k,n,n_ad,rank,rms", [
+    (3, 7, 256, 384, 3, 16, False), (2, 48, 4096, 256, 4, 32, False), (5, 13, 256, 520, 5, 8, True), (9, 37, 4096, 2560, 4, 64, False),
+    (64, 17, 128, 256, 64, 16, True), (3, 700, 512, 4096, 2, 16, True), (1, 300, 256, 256, 1, 8, False),
+])
+def test_an_index_per_example(examples, rows, k, n, n_ad, rank, rms):
+    """Decode, 32-row chunks, K-split, padded and packed groups: the bits of a call with the index written out per row, out-of-range
+    indices among them, from an array that is 16-byte aligned and from one that is not."""
+    import torch
+
+    pkg = load_package()
+    w8 = pkg.w8a8_lora
+    m = examples * rows
+    print(f"[case] index per example {examples}x{rows}x{k}x{n} adapters={n_ad} rank={rank}", flush=True)
+    t = wc.to_torch(wc.make_case(m, k, n, n_adapters=n_ad, rank=rank, seed=m, rms=rms), "cuda:0")
+    args = (t["x"], t["weight"], t["a"], t["b"], t["s"])
+    g = torch.Generator(device="cuda:0").manual_seed(m)
+    store = torch.randint(-2, n_ad + 2, (examples + 1,), generator=g, device="cuda:0", dtype=torch.int32)
+    for per in (store[:examples], store[1:]):
+        got = w8.forward(*args, adapter_indices=per, rms_gamma=t.get("gamma"))
+        want = _plan(w8, *args, adapter_indices=per.repeat_interleave(rows), rms_gamma=t.get("gamma"))
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
+def test_rows_per_index_that_does_not_fit_is_refused():
+    """The C call: a count that does not divide the rows, one without indices, one on the decode path."""
+    import ctypes
+    import torch
+
+    pkg = load_package()
+    w8, native = pkg.w8a8_lora, pkg._native
+    for m, per, indices, status in ((40, 3, True, -2), (40, 8, False, -2), (32, 8, True, -7)):  # (-2 SHAPE, -7 UNSUPPORTED)
+        t = wc.to_torch(wc.make_case(m, 128, 256, n_adapters=2, rank=8, seed=m), "cuda:0")
+        plan = w8.ForwardPlan(t["x"], t["weight"], t["a"], t["b"], t["s"], adapter_indices=t["idx"])
+        whole = native.ProblemZ(call=plan.problem, rows_per_index=per)
+        whole.call.struct_size = ctypes.sizeof(native.ProblemZ)
+        if not indices:
+            whole.call.adapter_indices = None
+        got = native.load().mi355_w8a8_forward_v1(ctypes.byref(whole.call), torch.cuda.current_stream().cuda_stream)
+        assert got == status
