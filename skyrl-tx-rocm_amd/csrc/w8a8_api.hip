@@ -2242,30 +2242,44 @@ int run_gq_linear(const mi355_w8a8_gq_problem* p, hipStream_t s) {
   const bool decode = L.m_pad == 32u;  // few rows: z in K slices instead of row blocks
   // one adapter's z shares the quantizer's launch (rows of 16-byte pieces; several adapters: a wave per row)
   const bool decode_z = decode && p->n_adapters == 1u && (p->k & 7u) == 0 && aligned16(p->x);
+  // z = x @ A[idx]: rows routed by adapter and multiplied on the matrix core (the kernels of the
+  // per-channel path) when the adapter count and K allow it, else one wave per row
+  const bool fast_z = lora && !decode && p->n_adapters <= (uint32_t)kMaxAdapters && (p->k & 7u) == 0 &&
+                      aligned16(p->x) && aligned16(p->lora_a);
+  const bool routed = fast_z && p->adapter_indices && p->n_adapters > 1u;
+  // A in lora_a_kernel's operand order
+  const uint32_t a_steps = (p->k + 63u) / 64u, a_rb = rank_chunks(p->rank) > 2u ? 2u : 1u;
+  const uint64_t a_items = (uint64_t)p->n_adapters * a_steps * a_rb * 256u;
+  uint16_t* const at = reinterpret_cast<uint16_t*>(ws + L.at);
+  // the quantizer's launch packs it where there is no routing launch to do it beside
+  const bool quant_tiles = !decode && (p->k & 7u) == 0 && (p->group_size == 32u || p->group_size == 64u || p->group_size == 128u);
+  const bool quant_packs = quant_tiles && fast_z && !routed;
   if (!decode_z) {
-    if (!decode && (p->k & 7u) == 0 && (p->group_size == 32u || p->group_size == 64u || p->group_size == 128u)) {
-      const dim3 qgrid(L.m_pad / 16u, (p->k_pad + 511u) / 512u);
-      if (p->group_size == 32u) hipLaunchKernelGGL((gq_quant_tile_kernel<1>), qgrid, dim3(256), 0, s, q);
-      else if (p->group_size == 64u) hipLaunchKernelGGL((gq_quant_tile_kernel<2>), qgrid, dim3(256), 0, s, q);
-      else hipLaunchKernelGGL((gq_quant_tile_kernel<4>), qgrid, dim3(256), 0, s, q);
+    if (quant_tiles) {
+      const uint32_t halves = L.m_pad / 16u;
+      GqQuantTileArgs t{};
+      t.q = q;
+      if (quant_packs) {
+        t.lora_a = static_cast<const uint16_t*>(p->lora_a); t.at = at;
+        t.n_groups = p->n_adapters; t.r = p->rank; t.steps = a_steps; t.rb = a_rb;
+        t.pack_y = (uint32_t)((a_items / 256u + halves - 1u) / halves);
+      }
+      const dim3 qgrid(halves, t.pack_y + (p->k_pad + 511u) / 512u);
+      if (p->group_size == 32u) hipLaunchKernelGGL((gq_quant_tile_kernel<1>), qgrid, dim3(256), 0, s, t);
+      else if (p->group_size == 64u) hipLaunchKernelGGL((gq_quant_tile_kernel<2>), qgrid, dim3(256), 0, s, t);
+      else hipLaunchKernelGGL((gq_quant_tile_kernel<4>), qgrid, dim3(256), 0, s, t);
     } else {
       hipLaunchKernelGGL(gq_quant_kernel, dim3(L.m_pad / 4u, q_grid_y), dim3(256), 0, s, q);
     }
     if ((st = launch_status())) return st;
   }
 
-  // z = x @ A[idx]: rows routed by adapter and multiplied on the matrix core (the kernels of the
-  // per-channel path) when the adapter count and K allow it, else one wave per row
-  const bool fast_z = lora && !decode && p->n_adapters <= (uint32_t)kMaxAdapters && (p->k & 7u) == 0 &&
-                      aligned16(p->x) && aligned16(p->lora_a);
-  const bool routed = fast_z && p->adapter_indices && p->n_adapters > 1u;
   int32_t* dst_pos = reinterpret_cast<int32_t*>(ws + L.dst_pos);
   uint32_t z_slices = 1u, z_slice_stride = p->m * 64u;
   if (fast_z) {
     int32_t* src_row = reinterpret_cast<int32_t*>(ws + L.src_row);
     int32_t* slot_group = reinterpret_cast<int32_t*>(ws + L.slot_group);
     int32_t* blk_range = reinterpret_cast<int32_t*>(ws + L.blk_range);
-    uint16_t* at = reinterpret_cast<uint16_t*>(ws + L.at);
     LoraPrepArgs pa{};
     pa.idx = routed ? p->adapter_indices : nullptr;
     pa.src_row = src_row; pa.dst_pos = dst_pos; pa.slot_group = slot_group; pa.blk_range = blk_range;
@@ -2274,11 +2288,12 @@ int run_gq_linear(const mi355_w8a8_gq_problem* p, hipStream_t s) {
     pa.M = p->m; pa.K = p->k; pa.N = p->n; pa.n_groups = p->n_adapters; pa.r = p->rank;
     pa.slots = L.m_pad;
     pa.route_blocks = routed ? 1u : 0u;
-    pa.a_operand_steps = (p->k + 63u) / 64u; pa.a_operand_rb = rank_chunks(p->rank) > 2u ? 2u : 1u;  // lora_a_kernel's operand order
-    const uint64_t a_items = (uint64_t)p->n_adapters * pa.a_operand_steps * pa.a_operand_rb * 256u;
+    pa.a_operand_steps = a_steps; pa.a_operand_rb = a_rb;
     pa.a_blocks = (uint32_t)((a_items + 1023u) / 1024u);
-    hipLaunchKernelGGL((lora_prep_kernel<0>), dim3(pa.route_blocks + pa.a_blocks), dim3(1024), 0, s, pa);
-    if ((st = launch_status())) return st;
+    if (!quant_packs) {
+      hipLaunchKernelGGL((lora_prep_kernel<0>), dim3(pa.route_blocks + pa.a_blocks), dim3(1024), 0, s, pa);
+      if ((st = launch_status())) return st;
+    }
     LoraAArgs la{};
     la.xsrc = q.x;
     la.at = at;

@@ -19,6 +19,7 @@
 //   gq_decode_prologue_kernel  up to 32 rows, one adapter: the quantizer and z in one launch
 #pragma once
 #include "w8a8_device.h"
+#include "w8a8_prologue.h"
 
 namespace w8a8 {
 
@@ -220,11 +221,26 @@ __global__ __launch_bounds__(256) void gq_quant_kernel(GqQuantArgs a) { gq_quant
 // 333 8.6 -> 4.7; 4096 x 1024 8.7 -> 4.0.  The kernel above spent most of that in its vector operations, 130 KB of
 // unrolled instructions and 49 KB of LDS a workgroup.  Several chunks of 128 k to a wave, the next on its way: 32.4 -> 32.7 (two)
 // and 34.2 (four), and 10.6 -> 13.0 (four) at 1536 rows.
+// The first rows of the grid put one adapter's A into lora_a_kernel's operand order, 256 operands a workgroup, which a launch of its own did in
+// 5 us behind this one: a call of 4096 rows, 12288 -> 4096, 343.3 -> 340.1 us.
+struct GqQuantTileArgs {
+  GqQuantArgs q;
+  const uint16_t* lora_a;  // bf16 [n_groups, K, r]
+  uint16_t* at;
+  uint32_t n_groups, r, steps, rb;  // as in LoraPrepArgs
+  uint32_t pack_y;         // rows of the grid that pack (0: none)
+};
 template <int GB>  // 32-wide k blocks of a group: 1, 2, 4
-__global__ __launch_bounds__(256) void gq_quant_tile_kernel(GqQuantArgs a) {
+__global__ __launch_bounds__(256) void gq_quant_tile_kernel(GqQuantTileArgs t) {
   constexpr uint32_t NG = 4u / GB;  // groups of 128 k
+  const GqQuantArgs& a = t.q;
+  if (blockIdx.y < t.pack_y) {
+    lora_a_pack32_item(t.lora_a, reinterpret_cast<unsigned char*>(t.at), t.n_groups, a.K, t.r, t.steps, t.rb,
+                       ((uint64_t)blockIdx.y * gridDim.x + blockIdx.x) * 256u + threadIdx.x);
+    return;
+  }
   const uint32_t lane = threadIdx.x & 63u;
-  const uint32_t c = blockIdx.y * 4u + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // the wave's 128 k
+  const uint32_t c = (blockIdx.y - t.pack_y) * 4u + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // the wave's 128 k
   const uint32_t kbs = a.K_pad / 32u;
   if (c * 4u >= kbs) return;
   const uint32_t i = lane & 15u, q = lane >> 4;
