@@ -2,6 +2,7 @@
 // carving and kernel launches.  Nothing here synchronises, allocates or keeps state.
 #include "../../include/mi355_w8a8.h"
 #include "w8a8_gq_bwd_api.h"
+#include "w8a8_bwd_split.h"
 
 #include <hip/hip_runtime.h>
 
@@ -1054,37 +1055,6 @@ int run_grouped(const mi355_w8a8_grouped_problem* p, hipStream_t s) {
 // ---------------------------------------------------------------------------------------
 // backward
 // ---------------------------------------------------------------------------------------
-// How the pull-back's tiles of 256 x 256 are spread over the chip: whole tiles while they come in full rounds of
-// 256 workgroups, the rest split along the contraction so that the last round takes its share of the time
-// and not all of it (sk_wgs workgroups of sk_q stages each; 0: no split).
-struct BwdDxSplit { uint32_t direct_tiles, sk_q, sk_wgs; };
-
-// Costs in stage times (about 1.05 us, 1.1 in the group-scaled kernel, whose stages have as many MFMAs): a split adds the partial tiles' way through memory, 256 KiB written
-// and read again for every workgroup and split tile (about 0.11 each at 4.7 TB/s), and a launch.  Measured: 2048 x 2560,
-// N = 10240 (80 tiles of 320 stages) 339 us whole, 135 + 22 us split; 3003 x 4096, N = 24576 (192 of 768) 800 us and 657 + 29 us.
-// Group-scaled, with what goes before the pull-back, whole / split: 200 x 4096 <- 4096 150 / 57, 800 x 12288 <- 4096 (128 tiles
-// left over of 384) 285 / 230, 1536 x 12288 <- 4096 (64 of 576) 434 / 355, 1536 x 2560 <- 6144 221 / 142.
-// Calls of fewer than 64 stages (N < 2048) stay whole: little to gain, and a grouped call over the same rows
-// then gives the same bits.
-// k_blocks: k blocks of a wave's tile (2; 1 in the group-scaled kernel, whose partial tiles are half the size).
-BwdDxSplit bwd_dx_split(uint32_t tiles_m, uint32_t tiles_k, uint32_t NB, uint32_t k_blocks = 2u) {
-  const uint32_t ntile = tiles_m * tiles_k, rem = ntile % 256u;
-  BwdDxSplit best{ntile, 0u, 0u};
-  if (rem == 0u || NB < 64u) return best;
-  double cost = 0.9 * NB;
-  for (uint32_t wgs = 64u; wgs <= 256u; wgs += 64u) {
-    uint32_t q = (rem * NB + wgs - 1u) / wgs;
-    q = round_up(q < 16u ? 16u : q, 2u);
-    const double c = q + 0.055 * k_blocks * (wgs + rem) + 8.0;
-    if (c < cost) {
-      cost = c;
-      best.direct_tiles = ntile - rem; best.sk_q = q;
-      best.sk_wgs = round_up((rem * NB + q - 1u) / q, 8u);
-    }
-  }
-  return best;
-}
-
 struct BwdLayout {
   BwdDxSplit split;
   uint64_t part;

@@ -10,6 +10,7 @@
 // The rest (tables, r / z finish, LoRA cotangents) is the per-channel backward's.
 #pragma once
 #include "w8a8_backward.h"
+#include "w8a8_bwd_split.h"
 #include "w8a8_gq.h"
 
 namespace w8a8 {
@@ -146,7 +147,7 @@ __global__ __launch_bounds__(256, 1) void gq_bwd_dx_wide_kernel(GqBwdDxArgs a) {
     const uint32_t s_piece = ((uint32_t)lane_s & 7u) * 4u;
     const uint32_t s_row = clamp_kb(kb0 + (((uint32_t)lane_s >> 3) & 3u)) * 32u / a.group * a.N;
     const size_t w_stride = (size_t)g.KB * kBlk8;
-    const unsigned char* Wg = g.wp + (size_t)nb0 * w_stride;
+    const unsigned char* Wg = g.wp + (size_t)gq_bwd_first_block((uint32_t)nb0, a.weight_nb) * w_stride;
     uint32_t a_off = lane16, s_col = (uint32_t)nb0 * 32u + s_piece;
     int nb_load = nb0;
     // Part j of four of the loads of the next stage to be asked for, into the stage buffer at st (behind the last stage: of that
@@ -161,8 +162,7 @@ __global__ __launch_bounds__(256, 1) void gq_bwd_dx_wide_kernel(GqBwdDxArgs a) {
         nb_load += more ? 1 : 0;
         a_off += more ? 2048u : 0u;
         s_col += more ? 32u : 0u;
-        // (the weight's last block again beyond it: dy is zero there)
-        Wg += more && (uint32_t)nb_load < a.weight_nb ? w_stride : 0;
+        Wg += more && gq_bwd_next_block((uint32_t)nb_load, a.weight_nb) ? w_stride : 0;
       }
     };
     constexpr int kRows16 = 2 * ROWS;  // row blocks of 16
