@@ -93,7 +93,8 @@ __global__ __launch_bounds__(256, 3) void bwd_pack_dy_kernel(BwdPackDyArgs a) {
       d[u] = *reinterpret_cast<const v4i*>(a.dy + ((size_t)off + col));
     }
   };
-  // B of a group: rows of ranks beyond r end behind the resource and read as zeros
+  // B of a group: rows of ranks beyond r lie behind the resource and read as zeros.  The whole offset is the lane's: the check takes a
+  // scalar offset off the resource's size, and the columns behind the matrix would take more than there is.
   const uint32_t b_off = (i * a.N + 16u * h) * 2u;
   typedef __attribute__((address_space(3))) v4i* lds_v4ptr;
   const uint32_t tile = (uint32_t)(uintptr_t)(lptr_t)lds + wave * 8192u;
@@ -116,12 +117,12 @@ __global__ __launch_bounds__(256, 3) void bwd_pack_dy_kernel(BwdPackDyArgs a) {
     auto fetch_b = [&](uint32_t grp, int q) {
       const __amdgpu_buffer_rsrc_t brsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(a.lora_b) + (size_t)grp * a.r * a.N, 0,
                                                                              (int)(a.r * a.N * 2u), 0x00020000);
+      const uint32_t off = b_off + (128u * G + 64u * q) * 2u;
 #pragma unroll
       for (int b = 0; b < RB; ++b)
 #pragma unroll
         for (int t = 0; t < 4; ++t)
-          wb[b][t] = __builtin_bit_cast(v8us, __builtin_amdgcn_raw_buffer_load_b128(brsrc, b_off + (t >> 1) * 64u + (t & 1) * 16u,
-                                                                                    (128u * G + 64u * q + 32u * b * a.N) * 2u, 0));
+          wb[b][t] = __builtin_bit_cast(v8us, __builtin_amdgcn_raw_buffer_load_b128(brsrc, off + 64u * b * a.N + (t >> 1) * 64u + (t & 1) * 16u, 0, 0));
       if (128u * G + 128u > a.N) {  // (columns beyond N are another rank's)
 #pragma unroll
         for (int b = 0; b < RB; ++b)
