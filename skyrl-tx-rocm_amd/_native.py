@@ -10,6 +10,7 @@ import ctypes
 import importlib.machinery
 import importlib.util
 import threading
+import warnings
 from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().parent / "lib" / "libmi355_w8a8.so"
@@ -335,27 +336,41 @@ def load() -> ctypes.CDLL:
 
 
 _host = None
+_host_tried = False
 entry_address: dict = {}  # of the entry points that the host module calls
 
 
+def _load_host():
+    """The module at ``HOST_PATH``; raises where it is missing, does not load or was built against another torch."""
+    import torch
+
+    loader = importlib.machinery.ExtensionFileLoader("mi355_w8a8_host", str(HOST_PATH))
+    module = importlib.util.module_from_spec(importlib.util.spec_from_loader("mi355_w8a8_host", loader))
+    loader.exec_module(module)
+    if getattr(module, "torch_version", None) != torch.__version__:
+        raise ImportError(f"built against torch {getattr(module, 'torch_version', None)}, this is {torch.__version__}")
+    return module
+
+
 def host():
-    """Load (once) and return the module with the host side of a forward call; raises if it was not built."""
-    global _host
-    if _host is not None:
+    """The module with the host side of a forward call (loaded once), or None where this torch cannot use it: callers then take the
+    general way, which makes the same call from Python, some 10 us slower."""
+    global _host, _host_tried
+    if _host_tried:
         return _host
     lib = load()
     with _lock:
-        if _host is None:
-            if not HOST_PATH.exists():
-                raise RuntimeError(f"{HOST_PATH} is missing: build it with skyrl-tx-rocm_amd/build.py")
-            loader = importlib.machinery.ExtensionFileLoader("mi355_w8a8_host", str(HOST_PATH))
-            module = importlib.util.module_from_spec(importlib.util.spec_from_loader("mi355_w8a8_host", loader))
-            loader.exec_module(module)
-            for name, fn in (("forward", "forward_v1"), ("linear", "lora_linear_v1"), ("gateup", "rms_gateup_swiglu_v1"),
-                             ("residual", "lora_residual_v1"), ("workspace_bytes", "workspace_bytes"), ("forward_path", "forward_path"),
-                             ("gq_linear", "gq_linear_v1"), ("gq_workspace_bytes", "gq_workspace_bytes")):
-                entry_address[name] = ctypes.cast(getattr(lib, f"mi355_w8a8_{fn}"), ctypes.c_void_p).value
-            _host = module
+        if not _host_tried:
+            try:
+                module = _load_host()
+                for name, fn in (("forward", "forward_v1"), ("linear", "lora_linear_v1"), ("gateup", "rms_gateup_swiglu_v1"),
+                                 ("residual", "lora_residual_v1"), ("workspace_bytes", "workspace_bytes"), ("forward_path", "forward_path"),
+                                 ("gq_linear", "gq_linear_v1"), ("gq_workspace_bytes", "gq_workspace_bytes")):
+                    entry_address[name] = ctypes.cast(getattr(lib, f"mi355_w8a8_{fn}"), ctypes.c_void_p).value
+                _host = module
+            except (ImportError, OSError) as e:
+                warnings.warn(f"{HOST_PATH.name} is not used ({e}): build it with skyrl-tx-rocm_amd/build.py", RuntimeWarning, stacklevel=2)
+            _host_tried = True
         return _host
 
 

@@ -82,7 +82,7 @@ def build_host(verbose: bool = False) -> Path:
     lib_dir = Path(torch.__file__).resolve().parent / "lib"
     include = [f"-I{p}" for p in cpp_extension.include_paths()]
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall",
-           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}", *include,
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}", f'-DMI355_TORCH_VERSION="{torch.__version__}"', *include,
            f"-I{sysconfig.get_paths()['include']}", str(CSRC / "w8a8_host_call.cc"), f"-L{lib_dir}", "-lc10", "-ltorch_cpu",
            "-ltorch_python", "-o", str(tmp)]
     proc = subprocess.run(cmd, capture_output=True, text=True)
@@ -106,7 +106,11 @@ def build(verbose: bool = False) -> Path:
     if verbose and err.strip():
         print(err, file=sys.stderr)
     os.replace(tmp, LIB_PATH)
-    build_host(verbose)
+    try:
+        build_host(verbose)
+    except (ImportError, OSError, RuntimeError) as e:  # (the C library serves without it; calls from torch then go the general way)
+        HOST_PATH.unlink(missing_ok=True)
+        print(f"{HOST_PATH.name} was not built: {e}", file=sys.stderr)
     build_ffi(verbose)
     return LIB_PATH
 

@@ -215,4 +215,11 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "mi355_w8a8_host", nullptr, -1, met
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit_mi355_w8a8_host() { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit_mi355_w8a8_host() {
+  PyObject* const m = PyModule_Create(&module);
+  if (m && PyModule_AddStringConstant(m, "torch_version", MI355_TORCH_VERSION) != 0) {  // (its C++ ABI is this one's: _native.host)
+    Py_DECREF(m);
+    return nullptr;
+  }
+  return m;
+}

@@ -118,12 +118,13 @@ def _forward(x, weight, pack, lora_a, lora_b, lora_scaling, activation_bits, ada
     if x.ndim < 1 or x.shape[-1] != k or x.numel() == 0:
         raise ValueError(f"activation K={x.shape[-1] if x.ndim else None} does not match weight K={k}")
     dev = x.device
-    if not (return_aux or flags or adapter_indices is not None or pw.source_group_size):
+    host = None if return_aux or flags or adapter_indices is not None or pw.source_group_size else _native.host()
+    if host is not None:
         # an ordinary call goes through the host module; for any other it returns None
         scaling = lora_scaling
         if lora_a is not None and isinstance(scaling, (int, float)) and lora_a.ndim in (2, 3):
             scaling = _scaling_vector(scaling, lora_a.shape[0] if lora_a.ndim == 3 else 1, dev)
-        result = _native.host().group_scaled(
+        result = host.group_scaled(
             x, pw.packed, pw.scales, k, pw.padded_in_features, n, pw.group_size, pw.bits, activation_bits, lora_a, lora_b,
             scaling, _native.entry_address["gq_linear"], _native.entry_address["gq_workspace_bytes"], _stream_ptr(dev))
         if type(result) is int:

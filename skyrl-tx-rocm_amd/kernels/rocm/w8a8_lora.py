@@ -426,13 +426,14 @@ def forward(x: torch.Tensor, weight, lora_a=None, lora_b=None, lora_scaling=None
             eps: float = 1e-6, residual: torch.Tensor | None = None, swiglu: bool = False,
             flags: int = 0, return_aux: bool = False, entry: str = "forward"):
     """One W8A8 forward through the C ABI.  Returns bf16 [..., n_out] (and aux tensors)."""
-    if not return_aux and isinstance(x, torch.Tensor) and x.is_cuda and x.dtype == torch.bfloat16 and x.ndim >= 2:
+    host = _native.host() if not return_aux and isinstance(x, torch.Tensor) and x.is_cuda and x.dtype == torch.bfloat16 and x.ndim >= 2 else None
+    if host is not None:
         # an ordinary call goes through the host module; for any other it returns None
         pw = prepare_weight(weight)
         scaling = lora_scaling
         if lora_a is not None and isinstance(scaling, (int, float)) and lora_a.ndim in (2, 3):
             scaling = _scaling_vector(scaling, lora_a.shape[0] if lora_a.ndim == 3 else 1, x.device)
-        result = _native.host().dense(
+        result = host.dense(
             x, pw.packed, pw.scales, pw.in_features, pw.out_features, lora_a, lora_b, scaling, adapter_indices, rms_gamma,
             residual, flags | _native.FLAG_SWIGLU if swiglu else flags, eps, _native.entry_address[entry],
             _native.entry_address["workspace_bytes"], _native.entry_address["forward_path"], _stream_ptr(x.device))
