@@ -89,7 +89,7 @@ __device__ inline float code_quotient(float v, float scale, float r) {
   const float q0 = v * r;
   return __builtin_fmaf(__builtin_fmaf(-q0, scale, v), r, q0);
 }
-// The codes of four quotients of at most 127.5, byte e the e-th: 1.5 * 2^23 has a last place of one, so the sum's low byte
+// The codes of four quotients q, -128.5 <= q < 127.5, byte e the e-th: 1.5 * 2^23 has a last place of one, so the sum's low byte
 // is the quotient rounded to nearest even in two's complement.
 __device__ inline uint32_t code_bytes4(const float (&q)[4]) {
   uint32_t m[4];

@@ -971,8 +971,8 @@ __device__ inline uint32_t quant_mode(float scale) {
 // (93 rows of 7680, rank 16: 9.7 us, 7.9 in the loop).
 __device__ inline uint2 quant_codes8(const uint4& raw, float scale, float rscale, uint32_t mode) {
   if (mode != 0u) {
-    const uint32_t top = bf16_absmax_pairs(0u, raw);  // beyond 127.5, as no value of a row of scale one without a NaN is
-    if (mode == 2u || __builtin_amdgcn_ballot_w64(scale == 1.0f && ((top >> 16) > 0x42ffu || (top & 0xffffu) > 0x42ffu)) != 0) {
+    const uint32_t top = bf16_absmax_pairs(0u, raw);  // 127.5 or more, as no value of a row of scale one without a NaN is
+    if (mode == 2u || __builtin_amdgcn_ballot_w64(scale == 1.0f && ((top >> 16) >= 0x42ffu || (top & 0xffffu) >= 0x42ffu)) != 0) {
       // biased by 128 the code lands in its byte, clipped, with one v_cvt_pk_u8_f32; flipping bit 7 makes it two's complement
       uint32_t r[4] = {raw.x, raw.y, raw.z, raw.w}, lo = 0, hi = 0;
 #pragma unroll 1

@@ -102,3 +102,27 @@ def test_per_channel_codes_of_every_pair(flags):
     _, aux = pkg.w8a8_lora.forward(x, weight, None, None, None, flags=value, return_aux=True)
     np.testing.assert_array_equal(aux["x_codes"].cpu().numpy(), want)
     np.testing.assert_array_equal(aux["x_scales"].cpu().numpy().reshape(-1), scales.reshape(-1))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,k", [(33, 512), (4400, 2560)])  # rows kept in the LDS, and read again
+def test_codes_beside_a_nan(m, k):
+    """A row with a NaN has scale one.  Its other values are clipped as int8, whatever else the wave holds: 127.5 is a bf16 value
+    that rounds to 128."""
+    import torch
+
+    pkg = load_package()
+    print(f"[case] codes beside a NaN {m}x{k}", flush=True)
+    rows = np.zeros((m, k), F)
+    rows[:, 1::4] = np.array([127.5, -127.5, 127.0, 126.5, -126.5, 0.5, 1.5, -0.5], F)[np.arange(k // 4) % 8]
+    rows[3, 64:96:2] = 300.0  # (beyond the range, in one piece of the row only)
+    rows[5, 96:128:2] = -300.0
+    nan = [0, 3, 5, 18, m - 1]
+    rows[nan, 0] = np.nan
+    x = torch.from_numpy(rows).to("cuda:0", torch.bfloat16)
+    w = pkg.quantized_lora.GroupQuantizedWeight(torch.ones((k, 64), dtype=torch.int8, device="cuda:0"), torch.ones((1, 64), device="cuda:0"),
+                                                k, k, 8, k)
+    _, aux = pkg.w8a8_lora.forward(x, w, None, None, None, flags=pkg._native.FLAG_FORCE_TILED, return_aux=True)
+    want = np.clip(np.rint(np.where(np.isnan(rows[nan]), F(-128), rows[nan])), -128, 127).astype(np.int8)
+    np.testing.assert_array_equal(aux["x_codes"][nan].cpu().numpy(), want)
+    assert (aux["x_scales"].reshape(-1)[nan] == 1.0).all()
