@@ -9,11 +9,14 @@ namespace w8a8 {
 // and not all of it (sk_wgs workgroups of sk_q stages each; 0: no split).
 struct BwdDxSplit { uint32_t direct_tiles, sk_q, sk_wgs; };
 
-// Costs in stage times (about 1.05 us, 1.1 in the group-scaled kernel, whose stages have as many MFMAs): a split adds the partial tiles' way through memory, 256 KiB written
-// and read again for every workgroup and split tile (about 0.11 each at 4.7 TB/s), and a launch.  Measured: 2048 x 2560,
-// N = 10240 (80 tiles of 320 stages) 339 us whole, 135 + 22 us split; 3003 x 4096, N = 24576 (192 of 768) 800 us and 657 + 29 us.
-// Group-scaled, with what goes before the pull-back, whole / split: 200 x 4096 <- 4096 150 / 57, 800 x 12288 <- 4096 (128 tiles
-// left over of 384) 285 / 230, 1536 x 12288 <- 4096 (64 of 576) 434 / 355, 1536 x 2560 <- 6144 221 / 142.
+// Costs in stage times (0.98 us: 256 whole tiles of 128 stages 125 us in either kernel, of 768 754; the group-scaled one's stages have
+// as many MFMAs): a split adds the partial tiles' way through memory, 256 KiB written and read again for every workgroup and split tile
+// (about 0.11 each at 4.7 TB/s), and a launch.  The weights were taken with kernels of eight waves, 1.05 and 1.1 us a stage.
+// Pull-back + finish, us, those kernels whole / split, and split as it is now: 2048 x 2560, N = 10240 (80 tiles of 320
+// stages) 339 / 135 + 22, 105 + 15; 3003 x 4096, N = 24576 (192 of 768) 800 / 657 + 29, 535 + 22; 3003 x 12288, N = 4096 (64 of 576
+// left over) 278 + 13 now.  Group-scaled, with what goes before the pull-back, whole / split, and the two alone now: 200 x 4096 <- 4096
+// 150 / 57, 23 + 7; 800 x 12288 <- 4096 (128 tiles left over of 384) 285 / 230, 172 + 8; 1536 x 12288 <- 4096 (64 of 576) 434 / 355,
+// 272 + 8; 1536 x 2560 <- 6144 221 / 142, 86 + 11.
 // Calls of fewer than 64 stages (N < 2048) stay whole: little to gain, and a grouped call over the same rows
 // then gives the same bits.
 // k_blocks: k blocks of a wave's tile (2; 1 in the group-scaled kernel, whose partial tiles are half the size).

@@ -53,7 +53,7 @@ constexpr uint32_t kG16MinKPad = 384;               // at least six stages: the 
 //           main loop has the matrix core to itself.
 // The wave tile (128 x 64), its fragment reads and its epilogue are the same in both.
 // MF, the 16-row fragments of a wave: 8, or 6 for tiles of 192 rows (NW = 4) where those fill the chip's rounds better
-// (gemm16_fragments).  A stage is then 28 KiB, brought in by seven of the eight waves.
+// (gemm16_short_tiles).  A stage is then 28 KiB, brought in by seven of the eight waves.
 template <int NW, int MF = 8>
 struct G16Geo {
   static constexpr int kTileM = 32 * MF;
